@@ -15,8 +15,8 @@ import sys
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ["capi.hip", "tile_offsets.hip", "quant.hip", "permute.hip", "gemm.hip"]
-PROBE_SOURCES = ["capi.hip", "tile_offsets.hip", "gemm.hip", "probe.hip"]  # compiled with -DAAMD_TUNING
+SOURCES = ["capi.hip", "quant.hip", "permute.hip", "gemm.hip"]
+PROBE_SOURCES = ["capi.hip", "gemm.hip", "probe.hip"]  # compiled with -DAAMD_TUNING
 LIB = os.path.join(HERE, "libatorch_amd_fp8.so")
 PROBES_LIB = os.path.join(HERE, "libatorch_amd_probes.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

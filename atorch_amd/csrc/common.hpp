@@ -195,18 +195,64 @@ __device__ __forceinline__ float amax8(const float* v) {
   return m;
 }
 
-// Which group does padded tile `t` belong to?  tile_off[E+1] is an exclusive prefix of
-// per-group tile counts.  All threads of the block take part; returns the same g in every
-// thread (E+1 if t is beyond the last tile).  `slot` is one int of shared memory.
-__device__ __forceinline__ int find_group(const int32_t* __restrict__ tile_off, int E, int t, int* slot) {
-  if (threadIdx.x == 0) *slot = E + 1;
-  __syncthreads();
-  for (int e = threadIdx.x; e < E; e += blockDim.x) {
-    int lo = tile_off[e], hi = tile_off[e + 1];
-    if (t >= lo && t < hi) *slot = e;
+// Ragged groups.  goff[E + 1] is the exclusive prefix of the groups' rows in device memory; a group of n rows owns
+// ceil(n / tile) consecutive tiles, and the groups' tiles follow each other.  Every wave turns the offsets into tile
+// ranges by itself, 64 groups at a time: lane l fetches the rows of group base + l (one trip to memory) and six DPP
+// adds make the prefix of the tile counts.  A kernel that writes the prefix to memory ahead of every launch cost
+// 2 to 5 us of a stream's time per grouped launch, ten times in a training step; this costs a workgroup about 0.1 us.
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1 .. 8: inside the rows of 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ int64_t readlane_i64(int64_t v, int lane) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)v, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)((uint64_t)v >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+// Lane l's group base + l: its rows [r_lo, r_hi) and its tiles [t_lo, t_hi) (empty past E), and the tiles of all
+// groups up to base + 63.  `carry`: the tiles of the groups before base.  All 64 lanes must be active.
+struct GroupRanges {
+  int64_t r_lo, r_hi;
+  int t_lo, t_hi, total;
+};
+template <int TILE>
+__device__ __forceinline__ GroupRanges group_ranges(const int64_t* __restrict__ goff, int E, int base, int carry) {
+  GroupRanges r;
+  const int e = base + ((int)threadIdx.x & 63);
+  r.r_lo = r.r_hi = 0;
+  if (e < E) {
+    r.r_lo = goff[e];
+    r.r_hi = goff[e + 1];
   }
-  __syncthreads();
-  return *slot;
+  const int n = (int)((r.r_hi - r.r_lo + (TILE - 1)) / TILE);
+  r.t_hi = carry + wave_inclusive_sum(n);
+  r.t_lo = r.t_hi - n;
+  r.total = __builtin_amdgcn_readlane(r.t_hi, 63);
+  return r;
+}
+// The group that holds tile t, its first tile and its rows, the same in every lane; g == E if t is past the last tile.
+struct GroupOfTile {
+  int g, t_lo;
+  int64_t r_lo, r_hi;
+};
+template <int TILE>
+__device__ __forceinline__ GroupOfTile find_group(const int64_t* __restrict__ goff, int E, int t) {
+  int carry = 0;
+  for (int base = 0; base < E; base += 64) {
+    const GroupRanges r = group_ranges<TILE>(goff, E, base, carry);
+    const unsigned long long hit = __ballot(t >= r.t_lo && t < r.t_hi);  // empty groups hold no tile
+    if (hit != 0) {
+      const int src = __builtin_ctzll(hit);
+      return {base + src, __builtin_amdgcn_readlane(r.t_lo, src), readlane_i64(r.r_lo, src), readlane_i64(r.r_hi, src)};
+    }
+    carry = r.total;
+  }
+  return {E, 0, 0, 0};
 }
 
 }  // namespace aamd

@@ -25,11 +25,6 @@
 // requested two steps ahead).  Rows are 128 bytes; the 16-byte chunks of a row
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
-#include <stdlib.h>
-#include <string.h>
-
-#include <atomic>
-
 #include "common.hpp"
 #ifdef AAMD_TUNING
 #include "../../include/atorch_amd_probes.h"
@@ -55,7 +50,6 @@ struct GemmParams {
   void* C;
   const void* bias;
   const int64_t* goff;      // [E+1] rows per group prefix (device); nullptr: one group [0, Lrows)
-  const int32_t* tile_off;  // [E+1] tile prefix (device)
   int64_t ldl, ldr;                          // row strides of L and R (bytes)
   int64_t l_kb_stride, r_kb_stride;          // bytes between consecutive 128-wide contraction blocks of a row
   int64_t r_group_stride;                    // bytes between the R matrices of consecutive groups
@@ -174,21 +168,14 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   // the 8 XCDs; every XCD gets one contiguous range of tile ids so that tiles sharing operand
   // panels meet in the same L2.
   // Row-ragged launches look their group up in the device-side offsets.  Every wave does it on its
-  // own, without LDS or barriers: lane e fetches the tile range and the row range of group e (all
-  // loads go out before the first wait: one trip to memory instead of three dependent ones, tile
-  // count -> tile index -> matching group -> its row offsets), the lane whose group holds the tile
-  // is found with a ballot and its values are broadcast with readlane.
+  // own, without LDS or barriers: lane e computes the tile range of group e (group_ranges), the lane whose group
+  // holds the tile is found with a ballot and its values are broadcast with readlane.
   int total_lt;
-  int t_lo = 0, t_hi = 0;
-  int64_t r_lo = 0, r_hi = 0;
+  GroupRanges gr = {};
   if (MODE == kRaggedRows && p.goff != nullptr) {
-    if (lane < p.E) {
-      t_lo = p.tile_off[lane];
-      t_hi = p.tile_off[lane + 1];
-      r_lo = p.goff[lane];
-      r_hi = p.goff[lane + 1];
-    }
-    total_lt = p.tile_off[p.E];
+    gr = group_ranges<BM>(p.goff, p.E, 0, 0);
+    total_lt = gr.total;
+    for (int base = 64; base < p.E; base += 64) total_lt = group_ranges<BM>(p.goff, p.E, base, total_lt).total;
   } else {
     total_lt = MODE == kRaggedRows ? (int)((p.Lrows + BM - 1) / BM) : p.nLt * p.E;
   }
@@ -238,16 +225,8 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
       l0 = 0;
       lvalid = 0;
       for (int base = 0; base < p.E; base += 64) {
-        if (base > 0) {  // more than 64 groups: the next 64
-          const int e = base + lane;
-          t_lo = t_hi = 0;
-          if (e < p.E) {
-            t_lo = p.tile_off[e];
-            t_hi = p.tile_off[e + 1];
-            r_lo = p.goff[e];
-            r_hi = p.goff[e + 1];
-          }
-        }
+        if (base > 0) gr = group_ranges<BM>(p.goff, p.E, base, gr.total);  // more than 64 groups: the next 64
+        const int t_lo = gr.t_lo, t_hi = gr.t_hi;
         int my_lt = lt, my_rt = 0;
         bool mine = lt >= t_lo && lt < t_hi;  // empty groups (and lanes past E) hold no tile
         if (by_group) {
@@ -264,11 +243,10 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
         const unsigned long long hit = __ballot(mine);
         if (hit != 0) {  // exactly one group holds the tile
           const int src = __builtin_ctzll(hit);
-          const int64_t first = r_lo + (int64_t)(my_lt - t_lo) * BM, left = r_hi - first;
+          const int64_t first = gr.r_lo + (int64_t)(my_lt - t_lo) * BM, left = gr.r_hi - first;
           const int lv = left < BM ? (int)left : BM;
           g = base + src;
-          l0 = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)((uint64_t)first >> 32), src) << 32) |
-                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)first, src));
+          l0 = readlane_i64(first, src);
           lvalid = __builtin_amdgcn_readlane(lv, src);
           if (by_group) rt = __builtin_amdgcn_readlane(my_rt, src);
           break;
@@ -289,8 +267,16 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     l0 = (int64_t)lt * BM;
     const int64_t left = p.Lrows - l0;
     lvalid = left < BM ? (int)left : BM;
-    kb0 = p.tile_off[g];
-    nkb = p.tile_off[g + 1] - kb0;
+    kb0 = nkb = 0;
+    for (int base = 0, carry = 0; base < p.E; base += 64) {  // the padded contraction blocks of group g
+      gr = group_ranges<kBK>(p.goff, p.E, base, carry);
+      if (g - base < 64) {
+        kb0 = __builtin_amdgcn_readlane(gr.t_lo, g - base);
+        nkb = __builtin_amdgcn_readlane(gr.t_hi, g - base) - kb0;
+        break;
+      }
+      carry = gr.total;
+    }
     // Operand buffers too short for the padded token count (ld_t below the device-side total): never
     // read past them, and make the failure visible: the group's gradient tile is written as NaN.
     if (kb0 + nkb > p.max_kb) {
@@ -962,8 +948,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   }
 }
 
-int launch_group_tile_offsets(const int64_t* goff, int E, int tile, int32_t* tile_off, hipStream_t st);
-
 // Launch choices a caller of the measurement build may pin per call (-1 = the library chooses, which is
 // all the product entry points ever pass).
 struct GemmOptions {
@@ -1016,8 +1000,8 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 using namespace aamd;
 
 static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
-                        int b_tile_scaled, const int64_t* group_offsets, int E, int32_t* tile_ws, int64_t M, int64_t N,
-                        int64_t K, void* c, int c_dtype, int64_t ldc, const void* bias, int bias_dtype, void* stream,
+                        int b_tile_scaled, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
+                        int c_dtype, int64_t ldc, const void* bias, int bias_dtype, void* stream,
                         const GemmOptions& g_opt = GemmOptions()) {
   AAMD_REQUIRE(c_dtype == AAMD_BF16 || c_dtype == AAMD_F32, "grouped_gemm_nt: unsupported output dtype %d", c_dtype);
   AAMD_REQUIRE(M >= 0 && N >= 0 && K >= 0, "grouped_gemm_nt: negative size");
@@ -1025,7 +1009,6 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                (long long)K, (long long)N);
   AAMD_REQUIRE(E >= 1, "grouped_gemm_nt: E must be >= 1");
   AAMD_REQUIRE(group_offsets != nullptr || E == 1, "grouped_gemm_nt: group_offsets required when E > 1");
-  AAMD_REQUIRE(group_offsets == nullptr || tile_ws != nullptr, "grouped_gemm_nt: tile_ws required");
   AAMD_REQUIRE(bias == nullptr || bias_dtype == AAMD_BF16 || bias_dtype == AAMD_F32, "grouped_gemm_nt: bad bias dtype");
   if (M == 0 || N == 0) return AAMD_OK;
   AAMD_REQUIRE(a && a_s && b && b_s && c, "grouped_gemm_nt: null pointer");
@@ -1044,10 +1027,6 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                      (b_tile_scaled || batches);
   const int BM = large ? CfgLarge::BM : CfgSmall::BM;
   const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : CfgLarge::BN) : CfgSmall::BN;
-  if (group_offsets) {
-    int rc = launch_group_tile_offsets(group_offsets, E, BM, tile_ws, st);
-    if (rc) return rc;
-  }
   GemmParams p = {};
   p.L = a; p.ldl = lda; p.Ls = a_s; p.ls_row_stride = K / kBK; p.ls_blk_stride = 1;
   p.l_kb_stride = p.r_kb_stride = kBK;
@@ -1059,7 +1038,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   p.rs_group_stride = b_tile_scaled ? N * (K / kBK) : (N / kTile) * (K / kBK);
   p.C = c; p.ldc = ldc; p.c_group_stride = 0;
   p.bias = bias; p.bias_dtype = bias_dtype; p.bias_group_stride = N;
-  p.goff = group_offsets; p.tile_off = tile_ws;
+  p.goff = group_offsets;
   p.Lrows = M; p.Rrows = N; p.nkb = (int)(K / kBK); p.E = E; p.nRt = (int)((N + BN - 1) / BN); p.nLt = 0;
   p.accumulate = 0;
   const int64_t max_lt = group_offsets ? M / BM + E : (M + BM - 1) / BM;
@@ -1074,63 +1053,33 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
 #ifndef AAMD_TUNING
 extern "C" int aamd_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b,
                                         const float* b_s, int b_tile_scaled, const int64_t* group_offsets, int E,
-                                        int32_t* tile_ws, int64_t M, int64_t N, int64_t K, void* c, int c_dtype,
+                                        int32_t* /*tile_ws*/, int64_t M, int64_t N, int64_t K, void* c, int c_dtype,
                                         int64_t ldc, const void* bias, int bias_dtype, void* stream) {
-  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, tile_ws, M, N, K, c, c_dtype, ldc, bias,
-                      bias_dtype, stream);
+  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
+                      stream);
 }
 
-// The same GEMM for callers that cannot allocate: the tile prefix lives in a file-scope device
-// array, one copy per GPU, whose address is looked up once per device.
-namespace aamd {
-constexpr int kStaticMaxGroups = AAMD_STATIC_MAX_GROUPS;
-static __device__ __align__(256) int32_t scratch[kStaticMaxGroups + 1];
-constexpr int kMaxDevices = 64;
-static std::atomic<int32_t*> g_scratch_ptr[kMaxDevices];
-
-// Device address of this GPU's copy of `scratch` (the array's name is only a host-side handle).
-static int scratch_of_current_device(int32_t** out) {
-  int dev = -1;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-  AAMD_REQUIRE(dev >= 0 && dev < kMaxDevices, "grouped_gemm_nt_static: device index %d out of range", dev);
-  int32_t* ptr = g_scratch_ptr[dev].load(std::memory_order_acquire);
-  if (ptr == nullptr) {
-    e = hipGetSymbolAddress(reinterpret_cast<void**>(&ptr), HIP_SYMBOL(scratch));
-    if (e != hipSuccess) return hip_fail(e, "hipGetSymbolAddress(scratch)");
-    AAMD_REQUIRE(ptr != nullptr, "grouped_gemm_nt_static: no device address for the scratch array");
-    g_scratch_ptr[dev].store(ptr, std::memory_order_release);  // every thread finds the same address
-  }
-  *out = ptr;
-  return AAMD_OK;
-}
-}  // namespace aamd
-
+// The same GEMM without a workspace argument.  (Neither form uses one: the kernels find their group in the offsets
+// themselves.  The limit on the groups is the entry point's contract.)
 extern "C" int aamd_grouped_gemm_fp8_nt_static(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b,
                                                const float* b_s, int b_tile_scaled, const int64_t* group_offsets,
                                                int E, int64_t M, int64_t N, int64_t K, void* c, int c_dtype,
                                                int64_t ldc, const void* bias, int bias_dtype, void* stream) {
-  AAMD_REQUIRE(E >= 1 && E <= kStaticMaxGroups, "grouped_gemm_nt_static: E=%d exceeds the %d groups the static scratch holds",
-               E, kStaticMaxGroups);
-  int32_t* ws = nullptr;
-  if (group_offsets != nullptr) {
-    const int rc = scratch_of_current_device(&ws);
-    if (rc) return rc;
-  }
-  // the tile prefix is rewritten in full (E + 1 entries) by the first kernel of every call
-  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, ws, M, N, K, c, c_dtype, ldc, bias,
-                      bias_dtype, stream);
+  AAMD_REQUIRE(E >= 1 && E <= AAMD_STATIC_MAX_GROUPS, "grouped_gemm_nt_static: E=%d exceeds the %d groups the static scratch holds",
+               E, AAMD_STATIC_MAX_GROUPS);
+  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
+                      stream);
 }
 #endif  // !AAMD_TUNING
 
 static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, const float* sxt, int64_t ld_t,
-                      int q_t_layout, const int64_t* group_offsets, int E, int32_t* tile_ws, int64_t N, int64_t K, void* dw,
+                      int q_t_layout, const int64_t* group_offsets, int E, int64_t N, int64_t K, void* dw,
                       int dw_dtype, int64_t expert_stride, int accumulate, void* stream,
                       const GemmOptions& g_opt = GemmOptions()) {
   AAMD_REQUIRE(dw_dtype == AAMD_BF16 || dw_dtype == AAMD_F32, "grouped_gemm_wgrad: unsupported output dtype %d", dw_dtype);
   AAMD_REQUIRE(N >= 0 && K >= 0 && N % kTile == 0 && K % kTile == 0,
                "grouped_gemm_wgrad: N=%lld and K=%lld must be multiples of 128", (long long)N, (long long)K);
-  AAMD_REQUIRE(E >= 1 && group_offsets && tile_ws, "grouped_gemm_wgrad: group_offsets / tile_ws required");
+  AAMD_REQUIRE(E >= 1 && group_offsets, "grouped_gemm_wgrad: group_offsets required");
   AAMD_REQUIRE(ld_t >= 0 && ld_t % kBK == 0, "grouped_gemm_wgrad: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE(ld_t < (1LL << 23), "grouped_gemm_wgrad: ld_t too large");
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "grouped_gemm_wgrad: unknown operand layout %d", q_t_layout);
@@ -1139,8 +1088,6 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   AAMD_REQUIRE(aligned16(dyt) && aligned16(xt) && aligned16(dw), "grouped_gemm_wgrad: pointers must be 16-byte aligned");
   AAMD_REQUIRE(expert_stride >= N * K && expert_stride % 4 == 0, "grouped_gemm_wgrad: bad expert stride");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_group_tile_offsets(group_offsets, E, kBK, tile_ws, st);
-  if (rc) return rc;
   GemmParams p = {};
   p.L = dyt; p.Ls = sdyt; p.ls_row_stride = 1; p.ls_blk_stride = N;
   p.R = xt; p.r_group_stride = 0;
@@ -1154,7 +1101,7 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   p.Rs = sxt; p.rs_row_stride = 1; p.rs_blk_stride = K; p.rs_group_stride = 0;
   p.C = dw; p.ldc = K; p.c_group_stride = expert_stride;
   p.bias = nullptr; p.bias_dtype = AAMD_NONE; p.bias_group_stride = 0;
-  p.goff = group_offsets; p.tile_off = tile_ws;
+  p.goff = group_offsets;
   // per-row scales on both operands: the 128x128 configuration measured faster for wgrad
   // (measurement build: tile 1 = 256 x 128)
   const int cfg = g_opt.tile > 0 ? 1 : 0;
@@ -1173,10 +1120,10 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
 #ifndef AAMD_TUNING
 extern "C" int aamd_grouped_gemm_fp8_wgrad(const uint8_t* dyt, const float* sdyt, const uint8_t* xt,
                                            const float* sxt, int64_t ld_t, int q_t_layout,
-                                           const int64_t* group_offsets, int E, int32_t* tile_ws, int64_t N,
+                                           const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, int64_t N,
                                            int64_t K, void* dw, int dw_dtype, int64_t expert_stride, int accumulate,
                                            void* stream) {
-  return wgrad_impl(dyt, sdyt, xt, sxt, ld_t, q_t_layout, group_offsets, E, tile_ws, N, K, dw, dw_dtype, expert_stride, accumulate,
+  return wgrad_impl(dyt, sdyt, xt, sxt, ld_t, q_t_layout, group_offsets, E, N, K, dw, dw_dtype, expert_stride, accumulate,
                     stream);
 }
 #else
@@ -1184,24 +1131,24 @@ extern "C" int aamd_grouped_gemm_fp8_wgrad(const uint8_t* dyt, const float* sdyt
 // opts = {tile, group_r, gl, ls_batch}, -1 = the library's own choice.
 extern "C" int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b,
                                                const float* b_s, int b_tile_scaled, const int64_t* group_offsets,
-                                               int E, int32_t* tile_ws, int64_t M, int64_t N, int64_t K, void* c,
+                                               int E, int32_t* /*tile_ws*/, int64_t M, int64_t N, int64_t K, void* c,
                                                int c_dtype, int64_t ldc, const void* bias, int bias_dtype,
                                                const int* opts, void* stream) {
   AAMD_REQUIRE(opts != nullptr, "tuning_grouped_gemm_nt: null options");
   GemmOptions o;
   o.tile = opts[0]; o.group_r = opts[1]; o.gl = opts[2]; o.ls_batch = opts[3];
-  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, tile_ws, M, N, K, c, c_dtype, ldc, bias,
-                      bias_dtype, stream, o);
+  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
+                      stream, o);
 }
 extern "C" int aamd_tuning_grouped_gemm_fp8_wgrad(const uint8_t* dyt, const float* sdyt, const uint8_t* xt,
                                                   const float* sxt, int64_t ld_t, int q_t_layout,
-                                                  const int64_t* group_offsets, int E, int32_t* tile_ws, int64_t N,
+                                                  const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, int64_t N,
                                                   int64_t K, void* dw, int dw_dtype, int64_t expert_stride,
                                                   int accumulate, const int* opts, void* stream) {
   AAMD_REQUIRE(opts != nullptr, "tuning_grouped_gemm_wgrad: null options");
   GemmOptions o;
   o.tile = opts[0]; o.group_r = opts[1]; o.gl = opts[2]; o.ls_batch = opts[3];
-  return wgrad_impl(dyt, sdyt, xt, sxt, ld_t, q_t_layout, group_offsets, E, tile_ws, N, K, dw, dw_dtype, expert_stride,
+  return wgrad_impl(dyt, sdyt, xt, sxt, ld_t, q_t_layout, group_offsets, E, N, K, dw, dw_dtype, expert_stride,
                     accumulate, stream, o);
 }
 #endif

@@ -578,16 +578,14 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
 template <typename IN>
 __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ goff,
-    const int32_t* __restrict__ tile_off, int E, uint8_t* __restrict__ q, float* __restrict__ s,
+    int E, uint8_t* __restrict__ q, float* __restrict__ s,
     uint8_t* __restrict__ q_t, float* __restrict__ s_t, int64_t ld_t, int blocked, float eps, int64_t gate_off,
     u16* __restrict__ h_out) {
   // the per-row-group column maxima are dead before the transposed codes are staged: one region
   __shared__ __attribute__((aligned(16))) uint8_t tile_t[kTile * kTLd];
   static_assert(sizeof(float) * 16 * kTile <= sizeof(tile_t), "the column maxima fit in the staging region");
   __shared__ Divider cdiv[kTile];  // scale and divider of every column of the tile
-  __shared__ int slot;
-  // the activation's table (GELU forms only), copied from the library's array; find_group's barriers order the
-  // copy before the tile's reads
+  // the activation's table (GELU forms only), copied from the library's array
   __shared__ __attribute__((aligned(16))) uint8_t lut_s[kLutBytes<IN> ? kLutBytes<IN> : 16];
   if constexpr (kLutBytes<IN> != 0) {
     const v4i* const src = reinterpret_cast<const v4i*>(std::is_same<IN, GELU>::value ? (const void*)g_gelu_lut : (const void*)g_gelub_lut);
@@ -609,11 +607,12 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
     }
   }
   const int pt = (int)by, kc = (int)bx;
-  const int g = __builtin_amdgcn_readfirstlane(find_group(tile_off, E, pt, &slot));
-  if (g >= E) return;
-  const int64_t m0 = goff[g] + (int64_t)(pt - tile_off[g]) * kTile;
-  const int64_t left = goff[g + 1] - m0;
+  const GroupOfTile at = find_group<kTile>(goff, E, pt);
+  if (at.g >= E) return;
+  const int64_t m0 = at.r_lo + (int64_t)(pt - at.t_lo) * kTile;
+  const int64_t left = at.r_hi - m0;
   const int mvalid = left < kTile ? (int)left : kTile;
+  if constexpr (kLutBytes<IN> != 0) __syncthreads();  // the copy of the table
   if (mvalid == kTile)
     dual_tile<IN, true>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, gate_off, h_out, tile_t, cdiv, nullptr, lut_s);
   else
@@ -629,13 +628,12 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
 template <typename IN>
 __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ sorted_idx,
-    uint32_t magic, int sh, uint32_t T, const int64_t* __restrict__ goff, const int32_t* __restrict__ tile_off, int E,
+    uint32_t magic, int sh, uint32_t T, const int64_t* __restrict__ goff, int E,
     uint8_t* __restrict__ q, float* __restrict__ s, uint8_t* __restrict__ q_t, float* __restrict__ s_t, int64_t ld_t,
     int blocked, float eps) {
   __shared__ __attribute__((aligned(16))) uint8_t tile_t[kTile * kTLd];
   __shared__ Divider cdiv[kTile];
   __shared__ uint32_t src_row[kTile];
-  __shared__ int slot;
   uint32_t bx = blockIdx.x, by = blockIdx.y;  // eight column tiles of a token tile on one XCD: see quant_dual_grouped_kernel
   {
     const uint32_t ntx = gridDim.x, per_row = ntx >> 3;
@@ -647,10 +645,10 @@ __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     }
   }
   const int pt = (int)by, kc = (int)bx;
-  const int g = __builtin_amdgcn_readfirstlane(find_group(tile_off, E, pt, &slot));
-  if (g >= E) return;
-  const int64_t m0 = goff[g] + (int64_t)(pt - tile_off[g]) * kTile;
-  const int64_t left = goff[g + 1] - m0;
+  const GroupOfTile at = find_group<kTile>(goff, E, pt);
+  if (at.g >= E) return;
+  const int64_t m0 = at.r_lo + (int64_t)(pt - at.t_lo) * kTile;
+  const int64_t left = at.r_hi - m0;
   const int mvalid = left < kTile ? (int)left : kTile;
   if ((int)threadIdx.x < mvalid) {
     const uint32_t flat = (uint32_t)sorted_idx[m0 + (int)threadIdx.x];
@@ -853,14 +851,13 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
 __global__ __launch_bounds__(512, 4) void swiglu_bwd_dual_kernel(const u16* __restrict__ fc1, int64_t ld, int64_t gate_off,
                                                               const u16* __restrict__ dh, int64_t ld_dh, int nt,
                                                               const int64_t* __restrict__ goff,
-                                                              const int32_t* __restrict__ tile_off, int E,
+                                                              int E,
                                                               uint8_t* __restrict__ q, float* __restrict__ s,
                                                               uint8_t* __restrict__ q_t, float* __restrict__ s_t,
                                                               int64_t ld_t, int blocked, u16* __restrict__ g_out) {
   __shared__ __attribute__((aligned(16))) uint8_t tile_ts[2][kTile * kTLd];
   __shared__ Divider cdivs[2][kTile];
-  __shared__ int slot;
-  __shared__ __attribute__((aligned(16))) float sig_s[2 * kSigN];  // find_group's barriers order the copy before its reads
+  __shared__ __attribute__((aligned(16))) float sig_s[2 * kSigN];
   for (uint32_t i = threadIdx.x; i < 2 * kSigN / 4; i += 512)
     reinterpret_cast<v4i*>(sig_s)[i] = reinterpret_cast<const v4i*>(g_sigmoid_lut)[i];
   // consecutive workgroups of one XCD take the eight consecutive feature tiles of a scale sector
@@ -876,13 +873,14 @@ __global__ __launch_bounds__(512, 4) void swiglu_bwd_dual_kernel(const u16* __re
     }
   }
   const int pt = (int)by, f = (int)bx;
-  const int g = __builtin_amdgcn_readfirstlane(find_group(tile_off, E, pt, &slot));
-  if (g >= E) return;
-  const int64_t m0 = goff[g] + (int64_t)(pt - tile_off[g]) * kTile;
-  const int64_t left = goff[g + 1] - m0;
+  const GroupOfTile at = find_group<kTile>(goff, E, pt);
+  if (at.g >= E) return;
+  const int64_t m0 = at.r_lo + (int64_t)(pt - at.t_lo) * kTile;
+  const int64_t left = at.r_hi - m0;
   const int mvalid = left < kTile ? (int)left : kTile;
   const u16* const xa = fc1 + m0 * ld + (int64_t)f * kTile;
   const u16* const xd = dh + m0 * ld_dh + (int64_t)f * kTile;
+  __syncthreads();  // the copy of the table
   if (mvalid == kTile)
     swiglu_bwd_dual_tile<true>(xa, (uint32_t)ld, gate_off, xd, (uint32_t)ld_dh, nt, m0, mvalid, pt, f, q, s, q_t, s_t,
                                (uint32_t)ld_t, blocked, g_out, tile_ts, cdivs, sig_s);
@@ -997,8 +995,6 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
   }
 }
 
-int launch_group_tile_offsets(const int64_t* goff, int E, int tile, int32_t* tile_off, hipStream_t st);
-
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace aamd
@@ -1051,7 +1047,7 @@ extern "C" int aamd_permute_quant_1x128(const void* x, int x_dtype, int64_t T, i
 }
 
 extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t M, int64_t cols, int64_t ldx,
-                                             const int64_t* group_offsets, int E, int32_t* tile_ws, uint8_t* q,
+                                             const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, uint8_t* q,
                                              float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
                                              float eps, void* stream) {
   AAMD_REQUIRE(x_dtype == AAMD_BF16 || x_dtype == AAMD_F32 || x_dtype == AAMD_F16, "quant_dual: unsupported dtype %d", x_dtype);
@@ -1060,7 +1056,7 @@ extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t
                (long long)cols);
   AAMD_REQUIRE(ldx >= cols && ldx % 8 == 0 && ldx < kMaxTileLd, "quant_dual: bad ldx=%lld", (long long)ldx);
   AAMD_REQUIRE(ld_t < kMaxTileLd, "quant_dual: ld_t=%lld too large", (long long)ld_t);
-  AAMD_REQUIRE(E >= 1 && group_offsets && tile_ws, "quant_dual: group_offsets / tile_ws required");
+  AAMD_REQUIRE(E >= 1 && group_offsets, "quant_dual: group_offsets required");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "quant_dual: q_t / s_t required");
@@ -1074,23 +1070,21 @@ extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t
   AAMD_REQUIRE(aligned16(x) && aligned16(q_t) && (!q || aligned16(q)), "quant_dual: pointers must be 16-byte aligned");
   AAMD_REQUIRE(grid_tiles <= 65535, "quant_dual: more than 65535 token tiles");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_group_tile_offsets(group_offsets, E, kTile, tile_ws, st);
-  if (rc) return rc;
   dim3 grid((unsigned)(cols / kTile), (unsigned)grid_tiles), block(256);
   const int nt = (int)(cols / kTile);
   if (x_dtype == AAMD_BF16)
-    quant_dual_grouped_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, tile_ws, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
+    quant_dual_grouped_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   else if (x_dtype == AAMD_F16)
-    quant_dual_grouped_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, tile_ws, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
+    quant_dual_grouped_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   else
-    quant_dual_grouped_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, group_offsets, tile_ws, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
+    quant_dual_grouped_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   AAMD_LAUNCH_CHECK("quant_dual_grouped");
   return AAMD_OK;
 }
 
 extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t T, int64_t cols, int64_t ldx,
                                                      const int64_t* sorted_idx, int topk, int64_t M,
-                                                     const int64_t* group_offsets, int E, int32_t* tile_ws, uint8_t* q,
+                                                     const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, uint8_t* q,
                                                      float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
                                                      float eps, void* stream) {
   AAMD_REQUIRE(x_dtype == AAMD_BF16 || x_dtype == AAMD_F32 || x_dtype == AAMD_F16, "permute_quant_dual: unsupported dtype %d", x_dtype);
@@ -1101,7 +1095,7 @@ extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype,
   AAMD_REQUIRE(topk >= 1 && topk <= 32768, "permute_quant_dual: topk=%d out of range", topk);
   AAMD_REQUIRE(T * topk < ((int64_t)1 << 31) && M <= T * topk, "permute_quant_dual: T * topk must stay below 2^31 and M within it");
   AAMD_REQUIRE(ld_t < kMaxTileLd && cols < kMaxTileLd, "permute_quant_dual: ld_t=%lld too large", (long long)ld_t);
-  AAMD_REQUIRE(E >= 1 && group_offsets && tile_ws, "permute_quant_dual: group_offsets / tile_ws required");
+  AAMD_REQUIRE(E >= 1 && group_offsets, "permute_quant_dual: group_offsets required");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "permute_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "permute_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "permute_quant_dual: q_t / s_t required");
@@ -1118,16 +1112,14 @@ extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype,
   const int sh = 31 + l;
   const uint32_t magic = (uint32_t)((((uint64_t)1 << sh) / (uint64_t)topk) + 1);
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_group_tile_offsets(group_offsets, E, kTile, tile_ws, st);
-  if (rc) return rc;
   dim3 grid((unsigned)(cols / kTile), (unsigned)grid_tiles), block(256);
   const int nt = (int)(cols / kTile);
   if (x_dtype == AAMD_BF16)
-    quant_dual_gather_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, tile_ws, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+    quant_dual_gather_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
   else if (x_dtype == AAMD_F16)
-    quant_dual_gather_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, tile_ws, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+    quant_dual_gather_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
   else
-    quant_dual_gather_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, tile_ws, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+    quant_dual_gather_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
   AAMD_LAUNCH_CHECK("permute_quant_dual_grouped");
   return AAMD_OK;
 }
@@ -1155,13 +1147,13 @@ extern "C" int aamd_swiglu_quant_1x128(const void* fc1, int64_t rows, int64_t F,
 }
 
 extern "C" int aamd_swiglu_quant_1x128_dual_grouped(const void* fc1, int64_t M, int64_t F, int64_t ld,
-                                                    const int64_t* group_offsets, int E, int32_t* tile_ws,
+                                                    const int64_t* group_offsets, int E, int32_t* /*tile_ws*/,
                                                     void* h_out, uint8_t* q, float* s, uint8_t* q_t, float* s_t,
                                                     int64_t ld_t, int q_t_layout, void* stream) {
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "swiglu_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && F >= 0 && F % kTile == 0, "swiglu_quant_dual: F=%lld must be a multiple of 128", (long long)F);
   AAMD_REQUIRE(ld >= 2 * F && ld % 8 == 0 && ld < kMaxTileLd && ld_t < kMaxTileLd, "swiglu_quant_dual: bad ld=%lld", (long long)ld);
-  AAMD_REQUIRE(E >= 1 && group_offsets && tile_ws, "swiglu_quant_dual: group_offsets / tile_ws required");
+  AAMD_REQUIRE(E >= 1 && group_offsets, "swiglu_quant_dual: group_offsets required");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "swiglu_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "swiglu_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "swiglu_quant_dual: q_t / s_t required");
@@ -1173,10 +1165,8 @@ extern "C" int aamd_swiglu_quant_1x128_dual_grouped(const void* fc1, int64_t M, 
                "swiglu_quant_dual: pointers must be 16-byte aligned");
   AAMD_REQUIRE(grid_tiles <= 65535, "swiglu_quant_dual: more than 65535 token tiles");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_group_tile_offsets(group_offsets, E, kTile, tile_ws, st);
-  if (rc) return rc;
   dim3 grid((unsigned)(F / kTile), (unsigned)grid_tiles), block(256);
-  quant_dual_grouped_kernel<GLU><<<grid, block, 0, st>>>((const u16*)fc1, ld, (int)(F / kTile), group_offsets, tile_ws, E,
+  quant_dual_grouped_kernel<GLU><<<grid, block, 0, st>>>((const u16*)fc1, ld, (int)(F / kTile), group_offsets, E,
                                                          q, s, q_t, s_t, ld_t, q_t_layout, 0.f, F, (u16*)h_out);
   AAMD_LAUNCH_CHECK("swiglu_quant_dual_grouped");
   return AAMD_OK;
@@ -1204,13 +1194,13 @@ extern "C" int aamd_gelu_quant_1x128(const void* x, int64_t rows, int64_t F, int
 
 // dh == nullptr: forward (h = gelu(x)); else backward (g = dh * gelu'(x)), dh dense with the row stride of x
 extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh, int64_t M, int64_t F, int64_t ld,
-                                                  const int64_t* group_offsets, int E, int32_t* tile_ws, void* h_out,
+                                                  const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, void* h_out,
                                                   uint8_t* q, float* s, uint8_t* q_t, float* s_t, int64_t ld_t,
                                                   int q_t_layout, void* stream) {
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "gelu_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && F >= 0 && F % kTile == 0, "gelu_quant_dual: F=%lld must be a multiple of 128", (long long)F);
   AAMD_REQUIRE(ld >= F && ld % 8 == 0 && ld < kMaxTileLd && ld_t < kMaxTileLd, "gelu_quant_dual: bad ld=%lld", (long long)ld);
-  AAMD_REQUIRE(E >= 1 && group_offsets && tile_ws, "gelu_quant_dual: group_offsets / tile_ws required");
+  AAMD_REQUIRE(E >= 1 && group_offsets, "gelu_quant_dual: group_offsets required");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "gelu_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "gelu_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "gelu_quant_dual: q_t / s_t required");
@@ -1223,16 +1213,14 @@ extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh,
                "gelu_quant_dual: pointers must be 16-byte aligned");
   AAMD_REQUIRE(grid_tiles <= 65535, "gelu_quant_dual: more than 65535 token tiles");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_group_tile_offsets(group_offsets, E, kTile, tile_ws, st);
-  if (rc) return rc;
   dim3 grid((unsigned)(F / kTile), (unsigned)grid_tiles), block(256);
   gelu_lut_kernel<<<dim3((2 * kLutN + 255) / 256), dim3(256), 0, st>>>();
   if (dh == nullptr) {
-    quant_dual_grouped_kernel<GELU><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, tile_ws, E, q, s,
+    quant_dual_grouped_kernel<GELU><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, q, s,
                                                             q_t, s_t, ld_t, q_t_layout, 0.f, 0, (u16*)h_out);
   } else {
     const int64_t dh_off = (const u16*)dh - (const u16*)x;  // elements; the loader reads dh at x + dh_off
-    quant_dual_grouped_kernel<GELUB><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, tile_ws, E, q, s,
+    quant_dual_grouped_kernel<GELUB><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, q, s,
                                                              q_t, s_t, ld_t, q_t_layout, 0.f, dh_off, (u16*)h_out);
   }
   AAMD_LAUNCH_CHECK("gelu_quant_dual_grouped");
@@ -1241,7 +1229,7 @@ extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh,
 
 extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t ld_dh, const void* fc1, int64_t ld,
                                                         int64_t M, int64_t F, const int64_t* group_offsets, int E,
-                                                        int32_t* tile_ws, void* g_out, uint8_t* q, float* s,
+                                                        int32_t* /*tile_ws*/, void* g_out, uint8_t* q, float* s,
                                                         uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
                                                         void* stream) {
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "swiglu_bwd_quant_dual: unknown q_t layout %d", q_t_layout);
@@ -1249,7 +1237,7 @@ extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t 
   AAMD_REQUIRE(ld >= 2 * F && ld % 8 == 0 && ld_dh >= F && ld_dh % 8 == 0 && ld < kMaxTileLd && ld_dh < kMaxTileLd && ld_t < kMaxTileLd,
                "swiglu_bwd_quant_dual: bad ld=%lld / ld_dh=%lld",
                (long long)ld, (long long)ld_dh);
-  AAMD_REQUIRE(E >= 1 && group_offsets && tile_ws, "swiglu_bwd_quant_dual: group_offsets / tile_ws required");
+  AAMD_REQUIRE(E >= 1 && group_offsets, "swiglu_bwd_quant_dual: group_offsets required");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "swiglu_bwd_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "swiglu_bwd_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "swiglu_bwd_quant_dual: q_t / s_t required");
@@ -1262,12 +1250,10 @@ extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t 
                "swiglu_bwd_quant_dual: pointers must be 16-byte aligned");
   AAMD_REQUIRE(grid_tiles <= 65535, "swiglu_bwd_quant_dual: more than 65535 token tiles");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_group_tile_offsets(group_offsets, E, kTile, tile_ws, st);
-  if (rc) return rc;
   const int nt = (int)(2 * F / kTile);
   dim3 grid((unsigned)(nt / 2), (unsigned)grid_tiles), block(512);  // two teams: the da and the db tile of a feature tile
   sigmoid_lut_kernel<<<dim3((2 * kSigN + 255) / 256), dim3(256), 0, st>>>();
-  swiglu_bwd_dual_kernel<<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, tile_ws, E,
+  swiglu_bwd_dual_kernel<<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, E,
                                                  q, s, q_t, s_t, ld_t, q_t_layout, (u16*)g_out);
   AAMD_LAUNCH_CHECK("swiglu_bwd_quant_dual_grouped");
   return AAMD_OK;

@@ -212,10 +212,9 @@ def tile_quant_dual_grouped(
     s = torch.empty((M, cols // TILE), dtype=torch.float32, device=dev) if rowwise else None
     q_t = _alloc_qt(cols, ld_t, blocked, dev)
     s_t = torch.empty((ld_t // TILE, cols), dtype=torch.float32, device=dev)
-    ws = torch.empty(num_groups + 1, dtype=torch.int32, device=dev)
     check(
         lib().aamd_quant_1x128_dual_grouped(
-            ptr(x), dtype_code(x.dtype, True), M, cols, cols, ptr(group_offsets), num_groups, ptr(ws),
+            ptr(x), dtype_code(x.dtype, True), M, cols, cols, ptr(group_offsets), num_groups, None,
             ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), eps, stream(),
         )
     )  # fmt: skip
@@ -250,11 +249,10 @@ def permute_tile_quant_dual_grouped(
     s = torch.empty((M, cols // TILE), dtype=torch.float32, device=dev) if rowwise else None
     q_t = _alloc_qt(cols, ld_t, blocked, dev)
     s_t = torch.empty((ld_t // TILE, cols), dtype=torch.float32, device=dev)
-    ws = torch.empty(num_groups + 1, dtype=torch.int32, device=dev)
     check(
         lib().aamd_permute_quant_1x128_dual_grouped(
             ptr(x), dtype_code(x.dtype, True), T, cols, cols, ptr(sorted_idx), topk, M, ptr(group_offsets), num_groups,
-            ptr(ws), ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), eps, stream(),
+            None, ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), eps, stream(),
         )
     )  # fmt: skip
     return q, s, q_t, s_t
@@ -302,10 +300,9 @@ def swiglu_tile_quant_dual_grouped(
     q_t = _alloc_qt(F, ld_t, blocked, dev)
     s_t = torch.empty((ld_t // TILE, F), dtype=torch.float32, device=dev)
     h = torch.empty((M, F), dtype=torch.bfloat16, device=dev) if return_activation else None
-    ws = torch.empty(num_groups + 1, dtype=torch.int32, device=dev)
     check(
         lib().aamd_swiglu_quant_1x128_dual_grouped(
-            ptr(fc1), M, F, two_f, ptr(group_offsets), num_groups, ptr(ws), ptr(h),
+            ptr(fc1), M, F, two_f, ptr(group_offsets), num_groups, None, ptr(h),
             ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), stream(),
         )
     )  # fmt: skip
@@ -342,10 +339,9 @@ def swiglu_bwd_tile_quant_dual_grouped(
     q_t = _alloc_qt(two_f, ld_t, blocked, dev)
     s_t = torch.empty((ld_t // TILE, two_f), dtype=torch.float32, device=dev)
     g = torch.empty((M, two_f), dtype=torch.bfloat16, device=dev) if return_grad else None
-    ws = torch.empty(num_groups + 1, dtype=torch.int32, device=dev)
     check(
         lib().aamd_swiglu_bwd_quant_1x128_dual_grouped(
-            ptr(dh), F, ptr(fc1), two_f, M, F, ptr(group_offsets), num_groups, ptr(ws), ptr(g),
+            ptr(dh), F, ptr(fc1), two_f, M, F, ptr(group_offsets), num_groups, None, ptr(g),
             ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), stream(),
         )
     )  # fmt: skip
@@ -395,10 +391,9 @@ def gelu_tile_quant_dual_grouped(
     q_t = _alloc_qt(F, ld_t, blocked, dev)
     s_t = torch.empty((ld_t // TILE, F), dtype=torch.float32, device=dev)
     h = torch.empty((M, F), dtype=torch.bfloat16, device=dev) if return_activation else None
-    ws = torch.empty(num_groups + 1, dtype=torch.int32, device=dev)
     check(
         lib().aamd_gelu_quant_1x128_dual_grouped(
-            ptr(x), ptr(dh), M, F, F, ptr(group_offsets), num_groups, ptr(ws), ptr(h),
+            ptr(x), ptr(dh), M, F, F, ptr(group_offsets), num_groups, None, ptr(h),
             ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), stream(),
         )
     )  # fmt: skip
@@ -444,10 +439,9 @@ def grouped_gemm_nt(
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
     assert out.shape == (M, N) and out.stride(1) == 1
     b_tile_scaled = b_s.size(1) == N
-    ws = torch.empty(E + 1, dtype=torch.int32, device=a.device)
     if bias is not None:
         assert bias.shape == (E, N) and bias.is_contiguous()
-    args = (ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), int(b_tile_scaled), ptr(group_offsets), E, ptr(ws),
+    args = (ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), int(b_tile_scaled), ptr(group_offsets), E, None,
             M, N, K, ptr(out), dtype_code(out.dtype), out.stride(0),
             ptr(bias), dtype_code(bias.dtype) if bias is not None else _lib.NONE)  # fmt: skip
     pinned = _pinned_options()
@@ -485,9 +479,8 @@ def grouped_gemm_wgrad(
         assert not accumulate
         out = torch.empty((E, N, K), dtype=out_dtype, device=dy_t.device)
     assert out.shape == (E, N, K) and out.stride(2) == 1 and out.stride(1) == K
-    ws = torch.empty(E + 1, dtype=torch.int32, device=dy_t.device)
     estride = out.stride(0) if E > 1 else N * K
-    args = (ptr(dy_t), ptr(sdy_t), ptr(x_t), ptr(sx_t), ld_t, int(blocked), ptr(group_offsets), E, ptr(ws), N, K,
+    args = (ptr(dy_t), ptr(sdy_t), ptr(x_t), ptr(sx_t), ld_t, int(blocked), ptr(group_offsets), E, None, N, K,
             ptr(out), dtype_code(out.dtype), estride, int(accumulate))  # fmt: skip
     pinned = _pinned_options()
     if pinned:

@@ -379,10 +379,9 @@ class HipQuantizeOp:
         bias_dt = dtype_code(bias_t.dtype) if bias_t is not None else _lib.NONE
         if fused:
             goff = self.group_offsets(m_splits, dev)
-            ws = torch.empty(E + 1, dtype=torch.int32, device=dev)
             check(
                 lib().aamd_grouped_gemm_fp8_nt(
-                    a[0], a[1], sa[0], b[0], sb[0], 0, goff.data_ptr(), E, ws.data_ptr(), M, N, K,
+                    a[0], a[1], sa[0], b[0], sb[0], 0, goff.data_ptr(), E, None, M, N, K,
                     c[0], out_dt, c[1], bias_t.data_ptr() if bias_t is not None else None, bias_dt, stream(),
                 )
             )  # fmt: skip
@@ -450,17 +449,15 @@ class HipQuantizeOp:
         oc = _base_of_stack(list(out_list))
         if la is not None and lb is not None and oc is not None and la[1] == lb[1]:
             goff = self.group_offsets(m_splits, dev)
-            ws = torch.empty(E + 1, dtype=torch.int32, device=dev)
             check(
                 lib().aamd_grouped_gemm_fp8_wgrad(
-                    la[0], la[2], lb[0], lb[2], la[1], _lib.QT_ROWS, goff.data_ptr(), E, ws.data_ptr(), N, K,
+                    la[0], la[2], lb[0], lb[2], la[1], _lib.QT_ROWS, goff.data_ptr(), E, None, N, K,
                     oc[0], out_dt, oc[1], int(accumulate), stream(),
                 )
             )  # fmt: skip
             return
         # generic path: one launch per group on densely re-laid operands
         pairs = torch.tensor([[0, m] for m in m_splits], dtype=torch.int64, device=dev)
-        ws = torch.empty(2, dtype=torch.int32, device=dev)
         for e in range(E):
             o = out_list[e]
             assert o.is_contiguous()
@@ -477,7 +474,7 @@ class HipQuantizeOp:
             check(
                 lib().aamd_grouped_gemm_fp8_wgrad(
                     dyt.data_ptr(), sdyt.data_ptr(), xt.data_ptr(), sxt.data_ptr(), ld, _lib.QT_ROWS, pairs[e].data_ptr(), 1,
-                    ws.data_ptr(), N, K, o.data_ptr(), out_dt, N * K, int(accumulate), stream(),
+                    None, N, K, o.data_ptr(), out_dt, N * K, int(accumulate), stream(),
                 )
             )  # fmt: skip
 

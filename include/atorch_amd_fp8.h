@@ -98,7 +98,7 @@ int aamd_permute_rows(const void *x, int x_dtype, int64_t T, int64_t cols, const
  *       poff_g = sum_{j<g} ceil(M_j/128)*128; pad tokens of a group are written 0
  *   s_t [ld_t/128, cols]: s_t[poff_g/128 + m/128, c]
  *   ld_t % 128 == 0 and ld_t >= poff_E (M + 127*E rounded up to 128 always suffices)
- *   tile_ws: E+1 int32 of scratch.
+ *   tile_ws: not used (the kernels find their group in group_offsets themselves); may be NULL.
  */
 int aamd_quant_1x128_dual_grouped(const void *x, int x_dtype, int64_t M, int64_t cols, int64_t ldx,
                                   const int64_t *group_offsets, int E, int32_t *tile_ws, uint8_t *q, float *s,
@@ -208,7 +208,7 @@ int aamd_gelu_quant_1x128_dual_grouped(const void *x, const void *dh, int64_t M,
  *   b [E, N, K] codes dense, b_s [E, N/128, K/128] (b_tile_scaled == 0) or [E, N, K/128] (!= 0)
  *   group_offsets [E+1] int64 device, or NULL for a single group [0, M] (then E must be 1)
  *   c [M, N] of c_dtype (row stride ldc elements, rows 16-byte aligned); rows of empty groups are not touched
- *   bias [E, N] of bias_dtype or NULL (AAMD_NONE); tile_ws: E+1 int32 scratch.
+ *   bias [E, N] of bias_dtype or NULL (AAMD_NONE); tile_ws: not used; may be NULL.
  *   K % 128 == 0, N % 128 == 0.
  */
 int aamd_grouped_gemm_fp8_nt(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b, const float *b_s,
@@ -219,10 +219,8 @@ int aamd_grouped_gemm_fp8_nt(const uint8_t *a, int64_t lda, const float *a_s, co
 /*
  * aamd_grouped_gemm_fp8_nt for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): the same arguments without
- * tile_ws.  No counterpart in the reference.  The E+1 ints of scratch live in a static device array
- * of the library (AAMD_STATIC_MAX_GROUPS + 1 ints per GPU, held until the process ends); the call
- * allocates and frees nothing.  E > AAMD_STATIC_MAX_GROUPS is rejected with AAMD_ERR_ARG.  All calls
- * on one GPU share that array: calls that may overlap on one GPU (different streams) race on it.
+ * tile_ws.  No counterpart in the reference.  The call allocates and
+ * frees nothing; E > AAMD_STATIC_MAX_GROUPS is rejected with AAMD_ERR_ARG.
  */
 #define AAMD_STATIC_MAX_GROUPS 4096
 int aamd_grouped_gemm_fp8_nt_static(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b,
