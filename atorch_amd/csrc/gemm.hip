@@ -177,38 +177,81 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     total_lt = gr.total;
     for (int base = 64; base < p.E; base += 64) total_lt = group_ranges<BM>(p.goff, p.E, base, total_lt).total;
   } else {
-    total_lt = MODE == kRaggedRows ? (int)((p.Lrows + BM - 1) / BM) : p.nLt * p.E;
+    total_lt = (int)((p.Lrows + BM - 1) / BM);  // kRaggedRows without groups
   }
-  const int64_t ntot = (int64_t)total_lt * p.nRt;
   const int64_t bid = blockIdx.x;
-  if (bid >= ntot) return;
-  int g, lt, rt;
-  const int64_t per = ntot / 8, rem = ntot % 8;
   const int64_t xcd = bid % 8, idx = bid / 8;
-  const int64_t pid = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
   const int GL = p.gl;
-  const bool by_group = MODE == kRaggedRows && p.goff != nullptr && p.group_r;  // tile order per group, below
-  {
-    // inside the range: groups of GL L tiles, R tile index outer, L tile inner
-    if (MODE == kRaggedK && p.group_r) {
-      // wgrad with more R tiles than L tiles: groups of GL R tiles, all L tiles of the expert inside
-      const int64_t per_e = (int64_t)p.nLt * p.nRt;
-      const int e = (int)(pid / per_e);
-      const int64_t pe = pid - e * per_e;
-      const int64_t width = (int64_t)GL * p.nLt;
-      const int first = (int)(pe / width) * GL;
-      const int gsz = p.nRt - first < GL ? p.nRt - first : GL;
-      const int in_grp = (int)(pe % width);
-      rt = first + in_grp % gsz;
-      lt = e * p.nLt + in_grp / gsz;
+  int g, lt, rt;
+  int kb_lo = 0, kb_hi = 0;  // kRaggedK: the contraction blocks of group g
+  int64_t pid = 0;
+  bool by_group = false;
+  if constexpr (MODE == kRaggedK) {
+    // The length of the contraction, and with it the time of a tile, differs from group to group, so every XCD takes
+    // an eighth of the tiles of every group (one range of tiles over all groups left the XCD that owned the busiest
+    // groups working alone: 16001 rows Zipf-distributed over 60 groups, 2816 x 2048 fp32 outputs, 800 us against 295 us), and
+    // the groups that are longer than average go first, so that the launch ends on short tiles.
+    const int per_g = p.nLt * p.nRt;  // tiles of a group
+    const int per_x = (per_g + 7) >> 3;
+    const int turn = __builtin_amdgcn_readfirstlane((int)((uint32_t)idx / (uint32_t)per_x));
+    const int pos = (int)idx - turn * per_x;
+    g = turn;
+    if (turn >= p.E) return;
+    if (p.E <= 64) {
+      gr = group_ranges<kBK>(p.goff, p.E, 0, 0);
+      const int n = gr.t_hi - gr.t_lo;
+      const bool live = lane < p.E;
+      const unsigned long long big = __ballot(live && (int64_t)n * p.E > 2 * (int64_t)gr.total);
+      const unsigned long long mid = __ballot(live && (int64_t)n * p.E > (int64_t)gr.total) & ~big;
+      const unsigned long long low = ((p.E == 64 ? 0ull : 1ull << p.E) - 1ull) & ~(big | mid);
+      // this lane's group is the r-th of the order: all of `big`, then all of `mid`, then the rest
+      const unsigned long long below = (1ull << lane) - 1ull;
+      const int nbig = __popcll(big), nmid = __popcll(mid);
+      const int r = (big >> lane) & 1 ? __popcll(big & below)
+                    : (mid >> lane) & 1 ? nbig + __popcll(mid & below) : nbig + nmid + __popcll(low & below);
+      g = __builtin_ctzll(__ballot(live && r == turn));
+      kb_lo = __builtin_amdgcn_readlane(gr.t_lo, g);
+      kb_hi = __builtin_amdgcn_readlane(gr.t_hi, g);
     } else {
-      const int64_t width = (int64_t)GL * p.nRt;
-      const int first = (int)(pid / width) * GL;
-      const int gsz = total_lt - first < GL ? total_lt - first : GL;
-      const int in_grp = (int)(pid % width);
+      for (int base = 0, carry = 0; base < p.E; base += 64) {
+        gr = group_ranges<kBK>(p.goff, p.E, base, carry);
+        if (g - base < 64) {
+          kb_lo = __builtin_amdgcn_readlane(gr.t_lo, g - base);
+          kb_hi = __builtin_amdgcn_readlane(gr.t_hi, g - base);
+          break;
+        }
+        carry = gr.total;
+      }
+    }
+    // this XCD's eighth; which one rotates with the group, so that remainders spread over the XCDs
+    const int part = (int)(xcd + turn) & 7, size = per_g >> 3, rem = per_g & 7;
+    if (pos >= size + (part < rem ? 1 : 0)) return;
+    const int pe = part * size + (part < rem ? part : rem) + pos;
+    // groups of GL tiles of the longer side of the gradient, all tiles of the shorter one inside
+    if (p.group_r) {
+      const int width = GL * p.nLt, first = pe / width * GL, in_grp = pe % width;
+      const int gsz = p.nRt - first < GL ? p.nRt - first : GL;
+      rt = first + in_grp % gsz;
+      lt = in_grp / gsz;
+    } else {
+      const int width = GL * p.nRt, first = pe / width * GL, in_grp = pe % width;
+      const int gsz = p.nLt - first < GL ? p.nLt - first : GL;
       lt = first + in_grp % gsz;
       rt = in_grp / gsz;
     }
+  } else {
+    const int64_t ntot = (int64_t)total_lt * p.nRt;
+    if (bid >= ntot) return;
+    const int64_t per = ntot / 8, rem = ntot % 8;
+    pid = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+    by_group = p.goff != nullptr && p.group_r;  // tile order per group, below
+    // inside the range: groups of GL L tiles, R tile index outer, L tile inner
+    const int64_t width = (int64_t)GL * p.nRt;
+    const int first = (int)(pid / width) * GL;
+    const int gsz = total_lt - first < GL ? total_lt - first : GL;
+    const int in_grp = (int)(pid % width);
+    lt = first + in_grp % gsz;
+    rt = in_grp / gsz;
   }
 
   int64_t l0;     // first L row of the tile
@@ -262,29 +305,22 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     kb0 = 0;
     nkb = p.nkb;
   } else {
-    g = lt / p.nLt;
-    lt -= g * p.nLt;
-    l0 = (int64_t)lt * BM;
+    l0 = (int64_t)__builtin_amdgcn_readfirstlane(lt) * BM;
     const int64_t left = p.Lrows - l0;
     lvalid = left < BM ? (int)left : BM;
-    kb0 = nkb = 0;
-    for (int base = 0, carry = 0; base < p.E; base += 64) {  // the padded contraction blocks of group g
-      gr = group_ranges<kBK>(p.goff, p.E, base, carry);
-      if (g - base < 64) {
-        kb0 = __builtin_amdgcn_readlane(gr.t_lo, g - base);
-        nkb = __builtin_amdgcn_readlane(gr.t_hi, g - base) - kb0;
-        break;
-      }
-      carry = gr.total;
-    }
+    kb0 = kb_lo;
+    nkb = kb_hi - kb_lo;
+    kb0 = __builtin_amdgcn_readfirstlane(kb0);
     // Operand buffers too short for the padded token count (ld_t below the device-side total): never
     // read past them, and make the failure visible: the group's gradient tile is written as NaN.
     if (kb0 + nkb > p.max_kb) {
       nkb = 0;
       short_operands = true;
     }
+    nkb = __builtin_amdgcn_readfirstlane(nkb);
   }
   g = __builtin_amdgcn_readfirstlane(g);
+  rt = __builtin_amdgcn_readfirstlane(rt);
   const int64_t r0 = (int64_t)rt * BN;
   const int64_t rleft = p.Rrows - r0;
   const int rvalid = rleft < BN ? (int)rleft : BN;  // a multiple of 128
@@ -828,7 +864,8 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   static_assert(WROWS <= 64 && WROWS % 8 == 0, "the staging region holds 64 rows");
   // (the bias is a compile-time case: without one the staging is two conversions and a write per
   // four values instead of a uniform branch, four adds and the moves that feed them)
-  auto flush = [&](auto tag, auto with_bias) {
+  // (inlined by order: called, it would hold everything it captures in memory)
+  auto flush = [&](auto tag, auto with_bias) __attribute__((always_inline)) {
     using ST = decltype(tag);  // staging type: OUT, or float when the old output is added in fp32
     constexpr bool kBias = decltype(with_bias)::value;
     constexpr int CW = 128 / (int)sizeof(ST);  // columns per chunk
@@ -932,7 +969,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     }
   };
   const bool with_bias = MODE == kRaggedRows && p.bias != nullptr;
-  auto flush_as = [&](auto tag) {
+  auto flush_as = [&](auto tag) __attribute__((always_inline)) {
     if constexpr (MODE == kRaggedRows) {
       if (with_bias) flush(tag, std::true_type{});
       else flush(tag, std::false_type{});
@@ -1110,7 +1147,7 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   p.Lrows = N; p.Rrows = K; p.nkb = 0; p.E = E; p.nRt = (int)((K + BN - 1) / BN); p.nLt = (int)((N + BM - 1) / BM);
   p.max_kb = (int)(ld_t / kBK);
   p.accumulate = accumulate;
-  const int64_t blocks = (int64_t)E * p.nLt * p.nRt;
+  const int64_t blocks = (int64_t)E * (((int64_t)p.nLt * p.nRt + 7) / 8) * 8;  // every XCD takes an eighth of a group
 #ifdef AAMD_TUNING
   if (cfg == 1) return launch_gemm<kRaggedK, true, CfgWgrad>(p, dw_dtype, blocks, st, g_opt);
 #endif
