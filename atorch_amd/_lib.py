@@ -68,6 +68,8 @@ SIGNATURES = {
     "aamd_unpermute_combine": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _int, _i64, _int, _vp, _vp]),
     "aamd_permute_rows_scaled": (_int, [_vp, _int, _i64, _i64, _vp, _int, _vp, _int, _i64, _vp, _int, _vp]),
     "aamd_unpermute_probs_grad": (_int, [_vp, _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, _vp]),
+    "aamd_unpermute_backward": (_int, [_vp, _int, _vp, _int, _i64, _i64, _vp, _vp, _int, _i64, _int, _vp, _vp, _vp]),
+    "aamd_group_offsets": (_int, [_vp, _int, _int, _vp, _vp]),
     "aamd_moe_preprocess_ws_ints": (_i64, [_i64, _int]),
     "aamd_moe_preprocess": (_int, [_vp, _int, _i64, _int, _vp, _vp, _vp, _vp, _vp]),
     "aamd_invert_permutation": (_int, [_vp, _i64, _i64, _vp, _vp]),
@@ -98,6 +100,22 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native host side (csrc/host.cpp): allocation and launch sequences, one call each."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise HipLibraryMissing(f"atorch_amd/_host.so cannot be loaded ({e}): build it with `python -m atorch_amd.csrc.build`")
+        _host = mod
+    return _host
+
+
 def check(rc: int):
     if rc != OK:
         msg = lib().aamd_last_error().decode("utf-8", "replace")
@@ -125,4 +143,5 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, as torch.cuda.current_stream() names it (which takes ten times as long)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())

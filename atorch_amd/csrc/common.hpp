@@ -236,12 +236,14 @@ __device__ __forceinline__ GroupRanges group_ranges(const int64_t* __restrict__ 
   return r;
 }
 // The group that holds tile t, its first tile and its rows, the same in every lane; g == E if t is past the last tile.
+// Without offsets there is one group of all M rows.
 struct GroupOfTile {
   int g, t_lo;
   int64_t r_lo, r_hi;
 };
 template <int TILE>
-__device__ __forceinline__ GroupOfTile find_group(const int64_t* __restrict__ goff, int E, int t) {
+__device__ __forceinline__ GroupOfTile find_group(const int64_t* __restrict__ goff, int E, int t, int64_t M) {
+  if (goff == nullptr) return {(int64_t)t * TILE < M ? 0 : E, 0, 0, M};
   int carry = 0;
   for (int base = 0; base < E; base += 64) {
     const GroupRanges r = group_ranges<TILE>(goff, E, base, carry);

@@ -924,7 +924,8 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
       const int64_t row_step = 8 * p.ldc;
       // accumulation into an fp32 output: the old values of all rows are requested before the
       // first is used (one trip to memory per chunk instead of one per row)
-      constexpr bool kAddF32 = sizeof(ST) == sizeof(OUT) && sizeof(OUT) == 4;
+      // (only the weight gradient accumulates; in the row-ragged kernels the old values cost registers and spills)
+      constexpr bool kAddF32 = MODE == kRaggedK && sizeof(ST) == sizeof(OUT) && sizeof(OUT) == 4;
       v4f olds[kAddF32 ? WROWS / 8 : 1];
       if constexpr (kAddF32) {
         if (p.accumulate) {
@@ -948,7 +949,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
         out_row += row_step;
         if (lrow < lvalid) {
           if constexpr (sizeof(ST) == sizeof(OUT)) {
-            if constexpr (sizeof(OUT) == 4) {
+            if constexpr (kAddF32) {
               // the output is not read again by this launch: streaming stores keep it from
               // evicting operand panels from L2 (measured +1-2 % where the output is large)
               if (p.accumulate) {
@@ -980,7 +981,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   if constexpr (sizeof(OUT) == 4) {
     flush_as(float{});
   } else {
-    if (p.accumulate) flush_as(float{});
+    if (MODE == kRaggedK && p.accumulate) flush_as(float{});
     else flush_as(u16{});
   }
 }

@@ -1,0 +1,415 @@
+// Host side of the ops in native code: output allocation, argument checks that need tensors, and the sequences of
+// launches an expert MLP is made of, one call from Python each.  The kernels are reached through the C ABI of
+// libatorch_amd_fp8.so; nothing here computes, synchronises or keeps state between calls.
+//
+// Why: a launch costs the host about 2.5 us, but a wrapper written in Python (two torch.empty, the current stream,
+// a ctypes call with a dozen arguments) costs 11 us, so that small and medium calls were bound by the host: a
+// decoding step of an MoE layer took 130 us of host time for 60 us of kernels.
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_strided.h>
+#include <ATen/ops/zeros.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <tuple>
+
+#include "../../include/atorch_amd_fp8.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+constexpr int64_t kTile = 128;
+
+void check(int rc) {
+  if (__builtin_expect(rc == AAMD_OK, 1)) return;
+  if (rc == AAMD_ERR_ARG) throw py::value_error(aamd_last_error());
+  throw std::runtime_error(aamd_last_error());
+}
+void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+void on_gpu(const Tensor& t) {
+  if (__builtin_expect(!t.is_cuda(), 0))
+    throw py::value_error("atorch_amd ops need tensors on the GPU (there is no CPU path)");
+}
+template <typename T = void>
+T* ptr(const Tensor& t) {
+  on_gpu(t);
+  return reinterpret_cast<T*>(t.data_ptr());
+}
+template <typename T = void>
+T* ptr(const OptTensor& t) {
+  return t.has_value() ? ptr<T>(*t) : nullptr;
+}
+int dtype_code(at::ScalarType dt, bool quantiser_input = false) {
+  if (dt == at::kBFloat16) return AAMD_BF16;
+  if (dt == at::kFloat) return AAMD_F32;
+  if (dt == at::kHalf && quantiser_input) return AAMD_F16;
+  throw py::value_error(std::string("atorch_amd: unsupported dtype ") + c10::toString(dt) +
+                        " (bf16 and fp32 are supported; fp16 as quantiser input)");
+}
+Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
+  on_gpu(like);
+  return at::empty(shape, at::TensorOptions().dtype(dt).device(like.device()));
+}
+constexpr auto kFp8 = at::kFloat8_e4m3fn;
+
+// the transposed codes of `rows` columns and ld_t padded tokens
+Tensor alloc_qt(int64_t rows, int64_t ld_t, bool blocked, const Tensor& like) {
+  return blocked ? empty({ld_t / kTile, rows, kTile}, kFp8, like) : empty({rows, ld_t}, kFp8, like);
+}
+int64_t qt_ld(const Tensor& q_t) { return q_t.dim() == 3 ? q_t.size(0) * kTile : q_t.size(1); }
+int64_t padded_bound(int64_t rows, int64_t groups) { return (rows / kTile + groups) * kTile; }
+
+// row-wise codes and scales, transposed codes and scales (undefined where not asked for)
+struct Quantised {
+  Tensor q, s, q_t, s_t;
+};
+using QuantTuple = std::tuple<OptTensor, OptTensor, Tensor, Tensor>;
+OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); }
+
+Quantised alloc_dual(int64_t M, int64_t cols, int64_t ld_t, bool rowwise, bool blocked, const Tensor& like) {
+  Quantised r;
+  if (rowwise) {
+    r.q = empty({M, cols}, kFp8, like);
+    r.s = empty({M, cols / kTile}, at::kFloat, like);
+  }
+  r.q_t = alloc_qt(cols, ld_t, blocked, like);
+  r.s_t = empty({ld_t / kTile, cols}, at::kFloat, like);
+  return r;
+}
+template <typename T = void>
+T* raw(const Tensor& t) {
+  return t.defined() ? ptr<T>(t) : nullptr;
+}
+
+// ---- quantisers ------------------------------------------------------------------------------
+std::tuple<Tensor, Tensor> tile_quant(const Tensor& x, double eps) {
+  const int64_t cols = x.size(-1), rows = cols ? x.numel() / cols : 0;
+  Tensor q = empty(x.sizes(), kFp8, x);
+  std::vector<int64_t> ss(x.sizes().begin(), x.sizes().end());
+  ss.back() = cols / kTile;
+  Tensor s = empty(ss, at::kFloat, x);
+  check(aamd_quant_1x128(ptr(x), dtype_code(x.scalar_type(), true), rows, cols, cols, ptr<uint8_t>(q), ptr<float>(s),
+                         (float)eps, stream()));
+  return {q, s};
+}
+
+std::tuple<Tensor, Tensor> permute_tile_quant(const Tensor& x, const Tensor& row_map, int64_t topk, int64_t n_out, double eps) {
+  const int64_t T = x.size(0), cols = x.size(1);
+  Tensor q = empty({n_out, cols}, kFp8, x), s = empty({n_out, cols / kTile}, at::kFloat, x);
+  check(aamd_permute_quant_1x128(ptr(x), dtype_code(x.scalar_type(), true), T, cols, cols, ptr<int32_t>(row_map), (int)topk,
+                                 n_out, ptr<uint8_t>(q), ptr<float>(s), (float)eps, stream()));
+  return {q, s};
+}
+
+// (without offsets: one group of all rows)
+Quantised dual(const Tensor& x, const OptTensor& goff, int64_t E, double eps, int64_t ld_t, bool rowwise, bool blocked) {
+  const int64_t M = x.size(0), cols = x.size(1);
+  Quantised r = alloc_dual(M, cols, ld_t, rowwise, blocked, x);
+  check(aamd_quant_1x128_dual_grouped(ptr(x), dtype_code(x.scalar_type(), true), M, cols, cols, ptr<int64_t>(goff), (int)E,
+                                      nullptr, raw<uint8_t>(r.q), raw<float>(r.s), ptr<uint8_t>(r.q_t), ptr<float>(r.s_t),
+                                      ld_t, blocked, (float)eps, stream()));
+  return r;
+}
+
+Quantised permute_dual(const Tensor& x, const Tensor& sorted_idx, int64_t topk, const Tensor& goff, int64_t E, double eps,
+                       int64_t ld_t, bool rowwise, bool blocked) {
+  const int64_t T = x.size(0), cols = x.size(1), M = sorted_idx.numel();
+  Quantised r = alloc_dual(M, cols, ld_t, rowwise, blocked, x);
+  check(aamd_permute_quant_1x128_dual_grouped(ptr(x), dtype_code(x.scalar_type(), true), T, cols, cols,
+                                              ptr<int64_t>(sorted_idx), (int)topk, M, ptr<int64_t>(goff), (int)E, nullptr,
+                                              raw<uint8_t>(r.q), raw<float>(r.s), ptr<uint8_t>(r.q_t), ptr<float>(r.s_t),
+                                              ld_t, blocked, (float)eps, stream()));
+  return r;
+}
+
+// the activation between the two linears, quantised: codes, scales and (keep) the activation itself
+std::tuple<Tensor, Tensor, OptTensor> act_quant(const Tensor& fc1, bool glu, bool keep) {
+  const int64_t width = fc1.size(-1), F = glu ? width / 2 : width, rows = width ? fc1.numel() / width : 0;
+  std::vector<int64_t> sh(fc1.sizes().begin(), fc1.sizes().end());
+  sh.back() = F;
+  Tensor q = empty(sh, kFp8, fc1);
+  Tensor h = keep ? empty(sh, at::kBFloat16, fc1) : Tensor();
+  sh.back() = F / kTile;
+  Tensor s = empty(sh, at::kFloat, fc1);
+  check((glu ? aamd_swiglu_quant_1x128 : aamd_gelu_quant_1x128)(ptr(fc1), rows, F, width, raw(h), ptr<uint8_t>(q), ptr<float>(s),
+                                                                stream()));
+  return {q, s, opt(h)};
+}
+
+// row-wise and transposed codes of the activation (grad undefined) or of the gradient through it
+std::tuple<Quantised, Tensor> act_dual(const Tensor& fc1, const Tensor& dh, bool glu, const Tensor& goff, int64_t E, int64_t ld_t,
+                                       bool rowwise, bool blocked, bool keep) {
+  const int64_t M = fc1.size(0), width = fc1.size(1), F = glu ? width / 2 : width;
+  const int64_t cols = glu && dh.defined() ? width : F;
+  Quantised r = alloc_dual(M, cols, ld_t, rowwise, blocked, fc1);
+  Tensor kept = keep ? empty({M, cols}, at::kBFloat16, fc1) : Tensor();
+  int rc;
+  if (!glu)
+    rc = aamd_gelu_quant_1x128_dual_grouped(ptr(fc1), raw(dh), M, F, F, ptr<int64_t>(goff), (int)E, nullptr, raw(kept),
+                                            raw<uint8_t>(r.q), raw<float>(r.s), ptr<uint8_t>(r.q_t), ptr<float>(r.s_t), ld_t,
+                                            blocked, stream());
+  else if (!dh.defined())
+    rc = aamd_swiglu_quant_1x128_dual_grouped(ptr(fc1), M, F, width, ptr<int64_t>(goff), (int)E, nullptr, raw(kept),
+                                              raw<uint8_t>(r.q), raw<float>(r.s), ptr<uint8_t>(r.q_t), ptr<float>(r.s_t), ld_t,
+                                              blocked, stream());
+  else
+    rc = aamd_swiglu_bwd_quant_1x128_dual_grouped(ptr(dh), F, ptr(fc1), width, M, F, ptr<int64_t>(goff), (int)E, nullptr,
+                                                  raw(kept), raw<uint8_t>(r.q), raw<float>(r.s), ptr<uint8_t>(r.q_t),
+                                                  ptr<float>(r.s_t), ld_t, blocked, stream());
+  check(rc);
+  return {r, kept};
+}
+
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose) {
+  const int64_t E = w.size(0), N = w.size(1), K = w.size(2);
+  Tensor q = empty({E, N, K}, kFp8, w), s = empty({E, N / kTile, K / kTile}, at::kFloat, w);
+  Tensor q_t = transpose ? empty({E, K, N}, kFp8, w) : Tensor();
+  Tensor s_t = transpose ? empty({E, K / kTile, N / kTile}, at::kFloat, w) : Tensor();
+  check(aamd_quant_128x128(ptr(w), dtype_code(w.scalar_type(), true), E, N, K, E > 1 ? w.stride(0) : N * K, ptr<uint8_t>(q),
+                           ptr<float>(s), raw<uint8_t>(q_t), raw<float>(s_t), (float)eps, stream()));
+  return {q, s, opt(q_t), opt(s_t)};
+}
+
+// ---- grouped GEMMs ---------------------------------------------------------------------------
+Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, const OptTensor& goff, const OptTensor& out,
+               at::ScalarType out_dtype, const OptTensor& bias) {
+  const int64_t M = a.size(0), K = a.size(1), E = b.size(0), N = b.size(1);
+  Tensor c = out.has_value() ? *out : empty({M, N}, out_dtype, a);
+  const bool b_tile_scaled = b_s.size(1) == N;
+  check(aamd_grouped_gemm_fp8_nt(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(b_s), b_tile_scaled,
+                                 ptr<int64_t>(goff), (int)E, nullptr, M, N, K, ptr(c), dtype_code(c.scalar_type()), c.stride(0),
+                                 ptr(bias), bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
+  return c;
+}
+
+Tensor gemm_wgrad(const Tensor& dy_t, const Tensor& sdy_t, const Tensor& x_t, const Tensor& sx_t, const Tensor& goff,
+                  const OptTensor& out, at::ScalarType out_dtype, bool accumulate) {
+  const bool blocked = dy_t.dim() == 3;
+  const int64_t N = blocked ? dy_t.size(1) : dy_t.size(0), K = blocked ? x_t.size(1) : x_t.size(0), E = goff.numel() - 1;
+  Tensor c = out.has_value() ? *out : empty({E, N, K}, out_dtype, dy_t);
+  check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(dy_t), ptr<float>(sdy_t), ptr<uint8_t>(x_t), ptr<float>(sx_t), qt_ld(dy_t),
+                                    blocked, ptr<int64_t>(goff), (int)E, nullptr, N, K, ptr(c), dtype_code(c.scalar_type()),
+                                    E > 1 ? c.stride(0) : N * K, accumulate, stream()));
+  return c;
+}
+
+// ---- routing ---------------------------------------------------------------------------------
+struct Routing {
+  Tensor sorted_idx, row_map, goff;
+};
+Routing route(const Tensor& ids, int64_t E, bool want_sorted) {
+  const int64_t n = ids.numel();
+  Routing r;
+  if (want_sorted) r.sorted_idx = empty({n}, at::kLong, ids);
+  r.row_map = empty({n}, at::kInt, ids);
+  r.goff = empty({E + 1}, at::kLong, ids);
+  Tensor ws = empty({std::max<int64_t>(1, aamd_moe_preprocess_ws_ints(n, (int)E))}, at::kInt, ids);
+  check(aamd_moe_preprocess(ptr(ids), ids.scalar_type() == at::kLong, n, (int)E, raw<int64_t>(r.sorted_idx), ptr<int32_t>(r.row_map),
+                            ptr<int64_t>(r.goff), ptr<int32_t>(ws), stream()));
+  return r;
+}
+std::tuple<OptTensor, Tensor, Tensor> moe_preprocess(const Tensor& ids, int64_t E, bool want_sorted) {
+  Routing r = route(ids, E, want_sorted);
+  return {opt(r.sorted_idx), r.row_map, r.goff};
+}
+
+Tensor invert_permutation(const Tensor& sorted_idx, int64_t n_flat) {
+  Tensor m = empty({n_flat}, at::kInt, sorted_idx);
+  check(aamd_invert_permutation(ptr<int64_t>(sorted_idx), sorted_idx.numel(), n_flat, ptr<int32_t>(m), stream()));
+  return m;
+}
+
+Tensor permute_rows(const Tensor& x, const Tensor& row_map, int64_t topk, int64_t n_out) {
+  Tensor out = empty({n_out, x.size(1)}, x.scalar_type(), x);
+  check(aamd_permute_rows(ptr(x), dtype_code(x.scalar_type()), x.size(0), x.size(1), ptr<int32_t>(row_map), (int)topk, n_out,
+                          ptr(out), stream()));
+  return out;
+}
+
+// rows and weights multiply in their common type: fp32 if either is
+at::ScalarType promote(const Tensor& y, const OptTensor& probs) {
+  return y.scalar_type() == at::kFloat || (probs.has_value() && probs->scalar_type() == at::kFloat) ? at::kFloat : y.scalar_type();
+}
+Tensor unpermute_combine(const Tensor& y, const Tensor& row_map, const OptTensor& probs, int64_t T, int64_t topk) {
+  const int64_t M = y.size(0), H = y.size(1);
+  const int pd = probs.has_value() ? dtype_code(probs->scalar_type()) : AAMD_NONE;
+  Tensor out = empty({T, H}, promote(y, probs), y);
+  check(aamd_unpermute_combine(ptr(y), dtype_code(y.scalar_type()), M, H, ptr<int32_t>(row_map), ptr(probs), pd, T, (int)topk,
+                               ptr(out), stream()));
+  return out;
+}
+
+Tensor permute_rows_scaled(const Tensor& x, const Tensor& row_map, int64_t topk, int64_t n_out, const OptTensor& probs,
+                           at::ScalarType out_dtype) {
+  const int64_t T = x.size(0), cols = x.size(1);
+  // dropped copies leave rows unwritten
+  Tensor out = n_out == T * topk ? empty({n_out, cols}, out_dtype, x)
+                                 : at::zeros({n_out, cols}, at::TensorOptions().dtype(out_dtype).device(x.device()));
+  const int pd = probs.has_value() ? dtype_code(probs->scalar_type()) : AAMD_NONE;
+  check(aamd_permute_rows_scaled(ptr(x), dtype_code(x.scalar_type()), T, cols, ptr<int32_t>(row_map), (int)topk, ptr(probs), pd,
+                                 n_out, ptr(out), dtype_code(out_dtype), stream()));
+  return out;
+}
+
+Tensor unpermute_probs_grad(const Tensor& dout, const Tensor& y, const Tensor& row_map, int64_t topk) {
+  const int64_t T = dout.size(0), H = dout.size(1);
+  Tensor dp = empty({T, topk}, at::kFloat, dout);
+  check(aamd_unpermute_probs_grad(ptr(dout), dtype_code(dout.scalar_type()), ptr(y), dtype_code(y.scalar_type()), y.size(0), H,
+                                  ptr<int32_t>(row_map), T, (int)topk, ptr<float>(dp), stream()));
+  return dp;
+}
+
+// Gradients of the combine: of the permuted rows and (in the weights' type) of the weights, in one pass.
+std::tuple<Tensor, Tensor> unpermute_backward(const Tensor& dout, const Tensor& y, const Tensor& row_map, const Tensor& probs,
+                                              int64_t topk) {
+  const int64_t T = dout.size(0), H = dout.size(1), M = y.size(0);
+  // dropped copies leave rows unwritten
+  Tensor drows = M == T * topk ? empty({M, H}, y.scalar_type(), y) : at::zeros({M, H}, y.options());
+  Tensor dprobs = empty(probs.sizes(), probs.scalar_type(), probs);
+  check(aamd_unpermute_backward(ptr(dout), dtype_code(dout.scalar_type()), ptr(y), dtype_code(y.scalar_type()), M, H,
+                                ptr<int32_t>(row_map), ptr(probs), dtype_code(probs.scalar_type()), T, (int)topk, ptr(drows),
+                                ptr(dprobs), stream()));
+  return {drows, dprobs};
+}
+
+// Exclusive prefix of rows per group, int64 [E + 1] on `device`, from a host list or an int64 tensor on either side.
+Tensor offsets_from_list(const std::vector<int64_t>& counts, at::Device device) {
+  Tensor goff = at::empty({(int64_t)counts.size() + 1}, at::TensorOptions().dtype(at::kLong).device(device));
+  check(aamd_group_offsets(counts.data(), 1, (int)counts.size(), ptr<int64_t>(goff), stream()));
+  return goff;
+}
+Tensor offsets_from_tensor(const Tensor& counts, at::Device device) {
+  Tensor goff = at::empty({counts.numel() + 1}, at::TensorOptions().dtype(at::kLong).device(device));
+  check(aamd_group_offsets(reinterpret_cast<const int64_t*>(counts.data_ptr()), !counts.is_cuda(), (int)counts.numel(),
+                           ptr<int64_t>(goff), stream()));
+  return goff;
+}
+
+// Equally shaped tensors as one [n, ...] tensor without a copy, when they are dense, lie one behind the other in one
+// storage; else nothing.  (Adjacent addresses are not enough: after module.to() or load_state_dict tensors may sit side
+// by side in memory and still own separate storages.)
+OptTensor stack_of(const std::vector<Tensor>& ts) {
+  if (ts.empty()) return {};
+  const Tensor& t0 = ts[0];
+  const int64_t n = t0.numel();
+  if (n == 0) return {};
+  const auto* base = static_cast<const char*>(t0.data_ptr());
+  const int64_t bytes = n * t0.element_size();
+  const auto& storage = t0.storage();
+  for (size_t i = 0; i < ts.size(); i++) {
+    const Tensor& t = ts[i];
+    if (!t.is_contiguous() || t.dtype() != t0.dtype() || t.sizes() != t0.sizes() ||
+        static_cast<const char*>(t.data_ptr()) != base + (int64_t)i * bytes || t.storage().data() != storage.data())
+      return {};
+  }
+  if ((t0.storage_offset() + (int64_t)ts.size() * n) * t0.element_size() > (int64_t)storage.nbytes()) return {};
+  std::vector<int64_t> sizes{(int64_t)ts.size()}, strides{n};
+  sizes.insert(sizes.end(), t0.sizes().begin(), t0.sizes().end());
+  strides.insert(strides.end(), t0.strides().begin(), t0.strides().end());
+  return t0.detach().as_strided(sizes, strides);
+}
+
+// ---- the expert MLP --------------------------------------------------------------------------
+// linear -> activation -> linear on rows grouped by expert.  With `row_map` the rows are the tokens of x in the order
+// of the routing (row_map, and sorted_idx where a backward follows), and the permute happens inside the quantiser.
+// Returns the output and what the backward reads: (out, fc1, qx_t, sx_t, qh_t, sh_t), the last five only with `train`.
+using MlpResult = std::tuple<Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
+MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
+                      const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
+                      const OptTensor& b2, bool glu, bool train) {
+  const int64_t E = q1.size(0);
+  const int64_t M = row_map.has_value() ? row_map->numel() : x.size(0);
+  Quantised qx;
+  const int64_t ld_t = padded_bound(M, E);
+  if (train)
+    qx = row_map.has_value() ? permute_dual(x, *sorted_idx, topk, goff, E, 0.0, ld_t, true, true)
+                             : dual(x, goff, E, 0.0, ld_t, true, true);
+  else
+    std::tie(qx.q, qx.s) = row_map.has_value() ? permute_tile_quant(x, *row_map, topk, M, 0.0) : tile_quant(x, 0.0);
+  Tensor fc1 = gemm_nt(qx.q, qx.s, q1, s1, goff, {}, at::kBFloat16, b1);
+  Quantised qh;
+  if (train) {
+    qh = std::get<0>(act_dual(fc1, Tensor(), glu, goff, E, ld_t, true, true, false));
+  } else {
+    OptTensor none;
+    std::tie(qh.q, qh.s, none) = act_quant(fc1, glu, false);
+  }
+  Tensor out = gemm_nt(qh.q, qh.s, q2, s2, goff, {}, x.scalar_type(), b2);
+  if (!train) return {out, {}, {}, {}, {}, {}};
+  return {out, fc1, qx.q_t, qx.s_t, qh.q_t, qh.s_t};
+}
+
+// The same from the router's choices: (out, sorted_idx, row_map, goff, y, ...): routing, MLP, weighted combine.
+using LayerResult = std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
+LayerResult layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids, int64_t topk, const Tensor& q1, const Tensor& s1,
+                          const Tensor& q2, const Tensor& s2, const OptTensor& b1, const OptTensor& b2, bool glu, bool train) {
+  Routing r = route(ids, q1.size(0), true);
+  MlpResult m = mlp_forward(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train);
+  Tensor& y = std::get<0>(m);
+  Tensor out = unpermute_combine(y, r.row_map, probs, x.size(0), topk);
+  return {out, r.sorted_idx, r.row_map, r.goff, train ? OptTensor(y) : OptTensor(),
+          std::get<1>(m), std::get<2>(m), std::get<3>(m), std::get<4>(m), std::get<5>(m)};
+}
+
+// Gradients of the MLP: (dx, dw1, dw2).  With topk > 0 the rows were tokens permuted through row_map, and dx goes back
+// to token order as the sum over a token's copies.
+std::tuple<Tensor, Tensor, Tensor> mlp_backward(const Tensor& dy, const Tensor& goff, const OptTensor& row_map, int64_t topk,
+                                                const Tensor& fc1, const Tensor& qx_t, const Tensor& sx_t, const Tensor& qh_t,
+                                                const Tensor& sh_t, const Tensor& q1_t, const Tensor& s1_t, const Tensor& q2,
+                                                const Tensor& s2, bool glu, bool transpose_w1, at::ScalarType x_dtype,
+                                                at::ScalarType w1_dtype, at::ScalarType w2_dtype) {
+  const int64_t E = goff.numel() - 1, ld_t = qt_ld(qx_t);
+  Quantised qdy = dual(dy, goff, E, 0.0, ld_t, true, true);
+  // through the second linear: dh = dy @ w2^T ([M, F]); dw2[f, h] = sum_m h[m, f] dy[m, h]
+  Tensor dh = gemm_nt(qdy.q, qdy.s, q2, s2, goff, {}, at::kBFloat16, {});
+  Tensor dw2 = gemm_wgrad(qh_t, sh_t, qdy.q_t, qdy.s_t, goff, {}, w2_dtype, false);
+  // through the activation, quantised by the kernel that computes it
+  Quantised qg = std::get<0>(act_dual(fc1, dh, glu, goff, E, ld_t, true, true, false));
+  // through the first linear: dx = dfc1 @ w1 ([M, H]); dw1[n, h] = sum_m dfc1[m, n] x[m, h]
+  Tensor dx = gemm_nt(qg.q, qg.s, q1_t, s1_t, goff, {}, x_dtype, {});
+  if (topk > 0) dx = unpermute_combine(dx, *row_map, {}, row_map->numel() / topk, topk);
+  Tensor dw1 = transpose_w1 ? gemm_wgrad(qg.q_t, qg.s_t, qx_t, sx_t, goff, {}, w1_dtype, false)
+                            : gemm_wgrad(qx_t, sx_t, qg.q_t, qg.s_t, goff, {}, w1_dtype, false);
+  return {dx, dw1, dw2};
+}
+
+QuantTuple pack(const Quantised& r) { return {opt(r.q), opt(r.s), r.q_t, r.s_t}; }
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.def("tile_quant", &tile_quant);
+  m.def("permute_tile_quant", &permute_tile_quant);
+  m.def("dual", [](const Tensor& x, const OptTensor& goff, int64_t E, double eps, int64_t ld_t, bool rowwise, bool blocked) {
+    return pack(dual(x, goff, E, eps, ld_t, rowwise, blocked));
+  });
+  m.def("permute_dual", [](const Tensor& x, const Tensor& sorted_idx, int64_t topk, const Tensor& goff, int64_t E, double eps,
+                           int64_t ld_t, bool rowwise, bool blocked) {
+    return pack(permute_dual(x, sorted_idx, topk, goff, E, eps, ld_t, rowwise, blocked));
+  });
+  m.def("act_quant", &act_quant);
+  m.def("act_dual", [](const Tensor& fc1, const OptTensor& dh, bool glu, const Tensor& goff, int64_t E, int64_t ld_t, bool rowwise,
+                       bool blocked, bool keep) {
+    auto [r, kept] = act_dual(fc1, dh.has_value() ? *dh : Tensor(), glu, goff, E, ld_t, rowwise, blocked, keep);
+    return std::make_tuple(opt(r.q), opt(r.s), r.q_t, r.s_t, opt(kept));
+  });
+  m.def("block_quant", &block_quant);
+  m.def("gemm_nt", &gemm_nt);
+  m.def("gemm_wgrad", &gemm_wgrad);
+  m.def("moe_preprocess", &moe_preprocess);
+  m.def("invert_permutation", &invert_permutation);
+  m.def("permute_rows", &permute_rows);
+  m.def("unpermute_combine", &unpermute_combine);
+  m.def("permute_rows_scaled", &permute_rows_scaled);
+  m.def("unpermute_probs_grad", &unpermute_probs_grad);
+  m.def("unpermute_backward", &unpermute_backward);
+  m.def("offsets_from_list", &offsets_from_list);
+  m.def("offsets_from_tensor", &offsets_from_tensor);
+  m.def("stack_of", &stack_of);
+  m.def("mlp_forward", &mlp_forward);
+  m.def("mlp_backward", &mlp_backward);
+  m.def("layer_forward", &layer_forward);
+}

@@ -258,6 +258,114 @@ __global__ __launch_bounds__(1024) void unpermute_probs_grad_kernel(const typena
 }
 
 // ---------------------------------------------------------------------------------------
+// Both gradients of the combine in one pass over the token's gradient row: drows[row_map[t*k+j]] = YT(dout[t] *
+// probs[t, j]) and dprobs[t, j] = <dout[t], y[row_map[t*k+j]]> in the weights' type.  Bound by memory: apart, the two
+// kernels read dout twice (a quarter of their bytes at top-2) and the weights' gradient needed a cast kernel.
+// A workgroup per token; a lane keeps its columns of dout in registers, the gathers of up to four slots go out
+// together, their products are stored and their dot products summed as they arrive.
+// ---------------------------------------------------------------------------------------
+template <typename DT, typename YT, int PD>
+__global__ __launch_bounds__(1024) void unpermute_backward_kernel(const typename DT::elem* __restrict__ dout,
+                                                                  const typename YT::elem* __restrict__ y, int64_t M, int H8,
+                                                                  const int32_t* __restrict__ row_map,
+                                                                  const void* __restrict__ probs, int topk,
+                                                                  typename YT::elem* __restrict__ drows,
+                                                                  void* __restrict__ dprobs) {
+  constexpr bool kYF32 = std::is_same<YT, F32>::value;
+  constexpr int kW = kYF32 ? 2 : 1;  // 16-byte words per 8 columns of a row
+  constexpr int B = 4;               // slots in flight
+  __shared__ int srow[kMaxTopk];
+  __shared__ float sprob[kMaxTopk];
+  __shared__ float red[16][kMaxTopk];
+  const int64_t t = blockIdx.x;
+  const int wave = (int)threadIdx.x >> 6, nwaves = (int)blockDim.x >> 6;
+  if ((int)threadIdx.x < topk) {
+    const int r = row_map[t * topk + threadIdx.x];
+    srow[threadIdx.x] = r >= 0 && r < M ? r : -1;  // a dropped copy: gradient 0
+    if constexpr (PD == AAMD_BF16) sprob[threadIdx.x] = bf16_bits_to_f32(reinterpret_cast<const u16*>(probs)[t * topk + threadIdx.x]);
+    else sprob[threadIdx.x] = reinterpret_cast<const float*>(probs)[t * topk + threadIdx.x];
+  }
+  __syncthreads();
+  const int64_t H = (int64_t)H8 * 8;
+  for (int j0 = 0; j0 < topk; j0 += B) {
+    float part[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) part[u] = 0.f;
+    for (int c = threadIdx.x; c < H8; c += blockDim.x) {
+      float a[8];
+      if constexpr (std::is_same<DT, F32>::value) {
+        const v4f lo = *reinterpret_cast<const v4f*>(dout + t * H + (int64_t)c * 8);
+        const v4f hi = *(reinterpret_cast<const v4f*>(dout + t * H + (int64_t)c * 8) + 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          a[i] = lo[i];
+          a[4 + i] = hi[i];
+        }
+      } else {
+        unpack8(*reinterpret_cast<const v4i*>(dout + t * H + (int64_t)c * 8), a);
+      }
+      v4i raw[B][kW];
+      int row[B];
+#pragma unroll
+      for (int u = 0; u < B; u++) {
+        // the row is the same in every lane; slots past topk and dropped copies are skipped by a branch of the whole wave
+        row[u] = j0 + u < topk ? __builtin_amdgcn_readfirstlane(srow[j0 + u < topk ? j0 + u : 0]) : -1;
+        const v4i* src = reinterpret_cast<const v4i*>(y + (int64_t)(row[u] < 0 ? 0 : row[u]) * H + (int64_t)c * 8);
+#pragma unroll
+        for (int w = 0; w < kW; w++) {
+          if (row[u] >= 0) raw[u][w] = __builtin_nontemporal_load(src + w);
+          else raw[u][w] = v4i{0, 0, 0, 0};
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < B; u++) {
+        if (row[u] < 0) continue;
+        const float pv = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sprob[j0 + u])));
+        float o[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) o[i] = a[i] * pv;
+        typename YT::elem* const dst = drows + (int64_t)row[u] * H + (int64_t)c * 8;
+        if constexpr (kYF32) {
+          __builtin_nontemporal_store(v4f{o[0], o[1], o[2], o[3]}, reinterpret_cast<v4f*>(dst));
+          __builtin_nontemporal_store(v4f{o[4], o[5], o[6], o[7]}, reinterpret_cast<v4f*>(dst) + 1);
+        } else {
+          v4i w;
+#pragma unroll
+          for (int i = 0; i < 4; i++) w[i] = (int)pack_bf16x2(o[2 * i], o[2 * i + 1]);
+          __builtin_nontemporal_store(w, reinterpret_cast<v4i*>(dst));
+        }
+        float b[8];
+        if constexpr (kYF32) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            b[i] = __int_as_float(raw[u][0][i]);
+            b[4 + i] = __int_as_float(raw[u][kW - 1][i]);
+          }
+        } else {
+          unpack8(raw[u][0], b);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) part[u] = part[u] + a[i] * b[i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      if (j0 + u >= topk) break;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) part[u] += __shfl_xor(part[u], off);
+      if ((threadIdx.x & 63) == 0) red[wave][j0 + u] = part[u];
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < topk) {
+    float sum = 0.f;
+    for (int w = 0; w < nwaves; w++) sum += red[w][threadIdx.x];
+    if constexpr (PD == AAMD_BF16) reinterpret_cast<u16*>(dprobs)[t * topk + threadIdx.x] = (u16)f32_to_bf16_bits(sum);
+    else reinterpret_cast<float*>(dprobs)[t * topk + threadIdx.x] = sum;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // inverse permutation
 // ---------------------------------------------------------------------------------------
 __global__ void fill_i32_kernel(int32_t* __restrict__ p, int64_t n, int32_t v) {
@@ -288,6 +396,16 @@ __device__ __forceinline__ int load_id(const ID* ids, int64_t i, int64_t n, int 
   if (i >= n) return -1;
   const int64_t e = (int64_t)ids[i];
   return (e >= 0 && e < E) ? (int)e : -1;  // out-of-range ids are dropped (row_map -1)
+}
+
+// lanes of this wave holding the same expert id (lanes without one: a mask of no use)
+__device__ __forceinline__ unsigned long long same_expert(int e, int E) {
+  unsigned long long peers = __ballot(e >= 0);
+  for (int b = 0; (1 << b) < E; b++) {
+    const unsigned long long vote = __ballot((e >> b) & 1);
+    peers &= ((e >> b) & 1) ? vote : ~vote;
+  }
+  return peers;
 }
 
 template <typename ID>
@@ -375,13 +493,7 @@ __global__ __launch_bounds__(256) void route_place_kernel(const ID* __restrict__
 #pragma unroll
   for (int it = 0; it < kChunk / 256; it++) {
     const int e = load_id(ids, base + it * 256 + threadIdx.x, n, E);
-    // lanes of this wave holding the same expert id
-    unsigned long long peers = __ballot(e >= 0);
-    if (e < 0) peers = ~peers;
-    for (int b = 0; (1 << b) < E; b++) {
-      const unsigned long long vote = __ballot((e >> b) & 1);
-      peers &= ((e >> b) & 1) ? vote : ~vote;
-    }
+    const unsigned long long peers = same_expert(e, E);
     const unsigned long long below = peers & ((1ull << lane) - 1ull);
     eid[it] = e;
     rank[it] = __popcll(below);
@@ -408,6 +520,194 @@ __global__ __launch_bounds__(256) void route_place_kernel(const ID* __restrict__
     const int pos = h[(it * 4 + wave) * E + eid[it]] + rank[it];
     row_map[flat] = pos;
     if (sorted_idx) sorted_idx[pos] = flat;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The same sort for fewer ids, with fewer launches (each of the four above is latency: 2 to 5 us whatever n is).
+// Up to 8192 ids: one workgroup does it all, ids and ranks in registers, counts of every (64 ids, expert) in LDS.
+// ---------------------------------------------------------------------------------------
+constexpr int kSmallRounds = 8;                         // rounds of 1024 ids
+constexpr int64_t kSmallMax = (int64_t)kSmallRounds * 1024;
+constexpr int64_t kSmallLds = 60 << 10;                 // bytes of counts
+
+// exclusive prefix of tot[0 .. E) into base[0 .. E), by one wave; returns the sum of all
+__device__ __forceinline__ int wave_exclusive_prefix(const int* tot, int* base, int E) {
+  int carry = 0;
+  for (int b = 0; b < E; b += 64) {
+    const int e = b + ((int)threadIdx.x & 63);
+    const int v = e < E ? tot[e] : 0;
+    const int incl = carry + wave_inclusive_sum(v);
+    if (e < E) base[e] = incl - v;
+    carry = __builtin_amdgcn_readlane(incl, 63);
+  }
+  return carry;
+}
+
+template <typename ID>
+__global__ __launch_bounds__(1024) void route_small_kernel(const ID* __restrict__ ids, int n, int E,
+                                                           int64_t* __restrict__ sorted_idx, int32_t* __restrict__ row_map,
+                                                           int64_t* __restrict__ goff) {
+  extern __shared__ int h[];  // [slots][E] counts, then each expert's prefix over the slots; [E] totals, then bases
+  const int slots = (n + 63) >> 6, wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+  int* const tot = h + slots * E;
+  for (int i = threadIdx.x; i < slots * E; i += 1024) h[i] = 0;
+  int eid[kSmallRounds], rank[kSmallRounds];
+#pragma unroll
+  for (int it = 0; it < kSmallRounds; it++) eid[it] = it * 1024 < n ? load_id(ids, it * 1024 + threadIdx.x, n, E) : -1;
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kSmallRounds; it++) {
+    if (it * 1024 + wave * 64 >= n) break;
+    const unsigned long long peers = same_expert(eid[it], E), below = peers & ((1ull << lane) - 1ull);
+    rank[it] = __popcll(below);
+    if (eid[it] >= 0 && below == 0) h[(it * 16 + wave) * E + eid[it]] = __popcll(peers);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 1024) {
+    int run = 0;
+    for (int s0 = 0; s0 < slots; s0 += 8) {  // eight counts at a time: their reads overlap
+      int c[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) c[u] = s0 + u < slots ? h[(s0 + u) * E + e] : 0;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        if (s0 + u < slots) h[(s0 + u) * E + e] = run;
+        run += c[u];
+      }
+    }
+    tot[e] = run;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int all = wave_exclusive_prefix(tot, tot, E);
+    for (int e = lane; e < E; e += 64) goff[e] = tot[e];
+    if (lane == 0) goff[E] = all;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kSmallRounds; it++) {
+    const int flat = it * 1024 + (int)threadIdx.x;
+    if (flat >= n) break;
+    if (eid[it] < 0) {
+      row_map[flat] = -1;
+      continue;
+    }
+    const int pos = tot[eid[it]] + h[(it * 16 + wave) * E + eid[it]] + rank[it];
+    row_map[flat] = pos;
+    if (sorted_idx) sorted_idx[pos] = flat;
+  }
+}
+
+// Up to kMidChunks chunks: the histogram, and a placement whose workgroups add up the chunks' counts themselves (at
+// most 512 x E ints from L2; more chunks than that and the scans as launches of their own are cheaper).
+constexpr int kMidChunks = 512;
+
+template <typename ID>
+__global__ __launch_bounds__(256) void route_count_kernel(const ID* __restrict__ ids, int64_t n, int E,
+                                                          int32_t* __restrict__ hist /* [chunk][E] */) {
+  extern __shared__ int cnt[];
+  for (int e = threadIdx.x; e < E; e += 256) cnt[e] = 0;
+  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * kChunk;
+#pragma unroll
+  for (int it = 0; it < kChunk / 256; it++) {
+    const int e = load_id(ids, base + it * 256 + threadIdx.x, n, E);
+    if (e >= 0) atomicAdd(&cnt[e], 1);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 256) hist[(int64_t)blockIdx.x * E + e] = cnt[e];
+}
+
+template <typename ID>
+__global__ __launch_bounds__(256) void route_place_scan_kernel(const ID* __restrict__ ids, int64_t n, int E, int nchunk,
+                                                               const int32_t* __restrict__ hist, int64_t* __restrict__ goff,
+                                                               int64_t* __restrict__ sorted_idx, int32_t* __restrict__ row_map) {
+  constexpr int kSlots = kChunk / 64;
+  extern __shared__ int h[];  // [kSlots][E] counts, [E] totals then bases, [E] ids of earlier chunks
+  int* const tot = h + kSlots * E;
+  int* const before = tot + E;
+  for (int i = threadIdx.x; i < (kSlots + 2) * E; i += 256) h[i] = 0;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, b = blockIdx.x;
+  const int64_t base = (int64_t)b * kChunk;
+  int eid[kChunk / 256], rank[kChunk / 256];
+#pragma unroll
+  for (int it = 0; it < kChunk / 256; it++) eid[it] = load_id(ids, base + it * 256 + threadIdx.x, n, E);
+  __syncthreads();
+  // experts across the lanes, chunks across the waves
+  for (int e = lane; e < E; e += 64) {
+    int all = 0, pre = 0;
+#pragma unroll 8
+    for (int c = wave; c < nchunk; c += 4) {
+      const int v = hist[(int64_t)c * E + e];
+      all += v;
+      pre += c < b ? v : 0;
+    }
+    atomicAdd(&tot[e], all);
+    atomicAdd(&before[e], pre);
+  }
+#pragma unroll
+  for (int it = 0; it < kChunk / 256; it++) {
+    const unsigned long long peers = same_expert(eid[it], E), below = peers & ((1ull << lane) - 1ull);
+    rank[it] = __popcll(below);
+    if (eid[it] >= 0 && below == 0) h[(it * 4 + wave) * E + eid[it]] = __popcll(peers);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int all = wave_exclusive_prefix(tot, tot, E);
+    if (b == 0) {
+      for (int e = lane; e < E; e += 64) goff[e] = tot[e];
+      if (lane == 0) goff[E] = all;
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 256) {
+    int run = tot[e] + before[e];
+    for (int sl = 0; sl < kSlots; sl++) {
+      const int c = h[sl * E + e];
+      h[sl * E + e] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kChunk / 256; it++) {
+    const int64_t flat = base + it * 256 + threadIdx.x;
+    if (flat >= n) continue;
+    if (eid[it] < 0) {
+      row_map[flat] = -1;
+      continue;
+    }
+    const int pos = h[(it * 4 + wave) * E + eid[it]] + rank[it];
+    row_map[flat] = pos;
+    if (sorted_idx) sorted_idx[pos] = flat;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Group offsets (exclusive prefix of the groups' rows, [E + 1]) from the rows per group.
+// ---------------------------------------------------------------------------------------
+// counts in host memory: the prefix is made on the host and travels in the kernel's arguments.  (A copy from pageable
+// host memory makes the host wait until the stream has drained: nothing could be enqueued ahead of the GPU.)
+constexpr int kOffsetsPerLaunch = 240;
+struct OffsetsArg {
+  int64_t v[kOffsetsPerLaunch];
+};
+__global__ __launch_bounds__(256) void store_offsets_kernel(const OffsetsArg a, int n, int64_t* __restrict__ goff) {
+  if ((int)threadIdx.x < n) goff[threadIdx.x] = a.v[threadIdx.x];
+}
+__global__ __launch_bounds__(64) void prefix_counts_kernel(const int64_t* __restrict__ counts, int E, int64_t* __restrict__ goff) {
+  const int lane = threadIdx.x;
+  int64_t carry = 0;
+  if (lane == 0) goff[0] = 0;
+  for (int base = 0; base < E; base += 64) {
+    int64_t v = base + lane < E ? counts[base + lane] : 0;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t o = __shfl_up(v, d);
+      if (lane >= d) v += o;
+    }
+    if (base + lane < E) goff[base + lane + 1] = carry + v;
+    carry += __shfl(v, 63);
   }
 }
 
@@ -737,7 +1037,28 @@ extern "C" int aamd_moe_preprocess(const void* expert_ids, int ids_are_i64, int6
   AAMD_REQUIRE(group_offsets && ws, "moe_preprocess: group_offsets / ws required");
   AAMD_REQUIRE(n == 0 || (expert_ids && row_map), "moe_preprocess: null pointer");
   hipStream_t st = (hipStream_t)stream;
+  const int64_t small_lds = ((n + 63) / 64 + 1) * E * (int64_t)sizeof(int);
+  if (n <= kSmallMax && small_lds <= kSmallLds) {
+    if (ids_are_i64)
+      route_small_kernel<int64_t><<<1, 1024, (size_t)small_lds, st>>>((const int64_t*)expert_ids, (int)n, E, sorted_idx, row_map, group_offsets);
+    else
+      route_small_kernel<int32_t><<<1, 1024, (size_t)small_lds, st>>>((const int32_t*)expert_ids, (int)n, E, sorted_idx, row_map, group_offsets);
+    AAMD_LAUNCH_CHECK("route_small");
+    return AAMD_OK;
+  }
   const int nchunk = (int)((n + kChunk - 1) / kChunk);
+  const size_t mid_lds = (size_t)(kChunk / 64 + 2) * E * sizeof(int);
+  if (nchunk <= kMidChunks && mid_lds <= (64 << 10)) {
+    if (ids_are_i64) {
+      route_count_kernel<int64_t><<<nchunk, 256, E * sizeof(int), st>>>((const int64_t*)expert_ids, n, E, ws);
+      route_place_scan_kernel<int64_t><<<nchunk, 256, mid_lds, st>>>((const int64_t*)expert_ids, n, E, nchunk, ws, group_offsets, sorted_idx, row_map);
+    } else {
+      route_count_kernel<int32_t><<<nchunk, 256, E * sizeof(int), st>>>((const int32_t*)expert_ids, n, E, ws);
+      route_place_scan_kernel<int32_t><<<nchunk, 256, mid_lds, st>>>((const int32_t*)expert_ids, n, E, nchunk, ws, group_offsets, sorted_idx, row_map);
+    }
+    AAMD_LAUNCH_CHECK("route_place_scan");
+    return AAMD_OK;
+  }
   const int nc = nchunk > 0 ? nchunk : 1;
   int32_t* hist = ws;
   int32_t* totals = ws + (int64_t)E * nc;
@@ -762,5 +1083,55 @@ extern "C" int aamd_moe_preprocess(const void* expert_ids, int ids_are_i64, int6
       route_place_kernel<int32_t><<<nchunk, 256, sh, st>>>((const int32_t*)expert_ids, n, E, nc, hist, group_offsets, sorted_idx, row_map);
     AAMD_LAUNCH_CHECK("route_place");
   }
+  return AAMD_OK;
+}
+
+extern "C" int aamd_group_offsets(const int64_t* counts, int counts_on_host, int E, int64_t* group_offsets, void* stream) {
+  AAMD_REQUIRE(E >= 1 && counts && group_offsets, "group_offsets: null pointer or no groups");
+  hipStream_t st = (hipStream_t)stream;
+  if (!counts_on_host) {
+    prefix_counts_kernel<<<1, 64, 0, st>>>(counts, E, group_offsets);
+    AAMD_LAUNCH_CHECK("group_offsets");
+    return AAMD_OK;
+  }
+  int64_t run = 0;
+  for (int base = 0; base <= E; base += kOffsetsPerLaunch) {
+    OffsetsArg a;
+    const int n = E + 1 - base < kOffsetsPerLaunch ? E + 1 - base : kOffsetsPerLaunch;
+    for (int i = 0; i < n; i++) {
+      a.v[i] = run;
+      if (base + i < E) run += counts[base + i];
+    }
+    store_offsets_kernel<<<1, 256, 0, st>>>(a, n, group_offsets + base);
+    AAMD_LAUNCH_CHECK("group_offsets");
+  }
+  return AAMD_OK;
+}
+
+extern "C" int aamd_unpermute_backward(const void* dout, int dout_dtype, const void* y, int y_dtype, int64_t M, int64_t H,
+                                       const int32_t* row_map, const void* probs, int probs_dtype, int64_t T, int topk,
+                                       void* drows, void* dprobs, void* stream) {
+  AAMD_REQUIRE(probs_dtype == AAMD_BF16 || probs_dtype == AAMD_F32, "unpermute_backward: unsupported probs dtype %d", probs_dtype);
+  AAMD_REQUIRE((y_dtype == AAMD_BF16 || y_dtype == AAMD_F32) &&
+                   dout_dtype == (y_dtype == AAMD_BF16 && probs_dtype == AAMD_BF16 ? AAMD_BF16 : AAMD_F32),
+               "unpermute_backward: dout must have the type of the combine's result");
+  AAMD_REQUIRE(M >= 0 && H >= 0 && T >= 0 && H % 8 == 0, "unpermute_backward: H=%lld must be a multiple of 8", (long long)H);
+  AAMD_REQUIRE(topk >= 1 && topk <= kMaxTopk && T < 0x7fffffffLL && M < 0x7fffffffLL, "unpermute_backward: bad topk / sizes");
+  if (T == 0 || H == 0) return AAMD_OK;
+  AAMD_REQUIRE(dout && row_map && probs && dprobs && ((y && drows) || M == 0), "unpermute_backward: null pointer");
+  AAMD_REQUIRE(((uintptr_t)y & 15) == 0 && ((uintptr_t)dout & 15) == 0 && ((uintptr_t)drows & 15) == 0,
+               "unpermute_backward: pointers must be 16-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  const int H8 = (int)(H / 8);
+  dim3 grid((unsigned)T), block((unsigned)threads_for_one_row(H8));
+  if (y_dtype == AAMD_BF16 && probs_dtype == AAMD_BF16)
+    unpermute_backward_kernel<BF16, BF16, AAMD_BF16><<<grid, block, 0, st>>>((const u16*)dout, (const u16*)y, M, H8, row_map, probs, topk, (u16*)drows, dprobs);
+  else if (y_dtype == AAMD_BF16)
+    unpermute_backward_kernel<F32, BF16, AAMD_F32><<<grid, block, 0, st>>>((const float*)dout, (const u16*)y, M, H8, row_map, probs, topk, (u16*)drows, dprobs);
+  else if (probs_dtype == AAMD_BF16)
+    unpermute_backward_kernel<F32, F32, AAMD_BF16><<<grid, block, 0, st>>>((const float*)dout, (const float*)y, M, H8, row_map, probs, topk, (float*)drows, dprobs);
+  else
+    unpermute_backward_kernel<F32, F32, AAMD_F32><<<grid, block, 0, st>>>((const float*)dout, (const float*)y, M, H8, row_map, probs, topk, (float*)drows, dprobs);
+  AAMD_LAUNCH_CHECK("unpermute_backward");
   return AAMD_OK;
 }

@@ -578,7 +578,7 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
 template <typename IN>
 __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ goff,
-    int E, uint8_t* __restrict__ q, float* __restrict__ s,
+    int E, int64_t M, uint8_t* __restrict__ q, float* __restrict__ s,
     uint8_t* __restrict__ q_t, float* __restrict__ s_t, int64_t ld_t, int blocked, float eps, int64_t gate_off,
     u16* __restrict__ h_out) {
   // the per-row-group column maxima are dead before the transposed codes are staged: one region
@@ -607,7 +607,7 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
     }
   }
   const int pt = (int)by, kc = (int)bx;
-  const GroupOfTile at = find_group<kTile>(goff, E, pt);
+  const GroupOfTile at = find_group<kTile>(goff, E, pt, M);
   if (at.g >= E) return;
   const int64_t m0 = at.r_lo + (int64_t)(pt - at.t_lo) * kTile;
   const int64_t left = at.r_hi - m0;
@@ -628,7 +628,7 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
 template <typename IN>
 __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ sorted_idx,
-    uint32_t magic, int sh, uint32_t T, const int64_t* __restrict__ goff, int E,
+    uint32_t magic, int sh, uint32_t T, const int64_t* __restrict__ goff, int E, int64_t M,
     uint8_t* __restrict__ q, float* __restrict__ s, uint8_t* __restrict__ q_t, float* __restrict__ s_t, int64_t ld_t,
     int blocked, float eps) {
   __shared__ __attribute__((aligned(16))) uint8_t tile_t[kTile * kTLd];
@@ -645,7 +645,7 @@ __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     }
   }
   const int pt = (int)by, kc = (int)bx;
-  const GroupOfTile at = find_group<kTile>(goff, E, pt);
+  const GroupOfTile at = find_group<kTile>(goff, E, pt, M);
   if (at.g >= E) return;
   const int64_t m0 = at.r_lo + (int64_t)(pt - at.t_lo) * kTile;
   const int64_t left = at.r_hi - m0;
@@ -851,7 +851,7 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
 __global__ __launch_bounds__(512, 4) void swiglu_bwd_dual_kernel(const u16* __restrict__ fc1, int64_t ld, int64_t gate_off,
                                                               const u16* __restrict__ dh, int64_t ld_dh, int nt,
                                                               const int64_t* __restrict__ goff,
-                                                              int E,
+                                                              int E, int64_t M,
                                                               uint8_t* __restrict__ q, float* __restrict__ s,
                                                               uint8_t* __restrict__ q_t, float* __restrict__ s_t,
                                                               int64_t ld_t, int blocked, u16* __restrict__ g_out) {
@@ -873,7 +873,7 @@ __global__ __launch_bounds__(512, 4) void swiglu_bwd_dual_kernel(const u16* __re
     }
   }
   const int pt = (int)by, f = (int)bx;
-  const GroupOfTile at = find_group<kTile>(goff, E, pt);
+  const GroupOfTile at = find_group<kTile>(goff, E, pt, M);
   if (at.g >= E) return;
   const int64_t m0 = at.r_lo + (int64_t)(pt - at.t_lo) * kTile;
   const int64_t left = at.r_hi - m0;
@@ -1056,7 +1056,7 @@ extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t
                (long long)cols);
   AAMD_REQUIRE(ldx >= cols && ldx % 8 == 0 && ldx < kMaxTileLd, "quant_dual: bad ldx=%lld", (long long)ldx);
   AAMD_REQUIRE(ld_t < kMaxTileLd, "quant_dual: ld_t=%lld too large", (long long)ld_t);
-  AAMD_REQUIRE(E >= 1 && group_offsets, "quant_dual: group_offsets required");
+  AAMD_REQUIRE(E >= 1 && (group_offsets || E == 1), "quant_dual: group_offsets required when E > 1");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "quant_dual: q_t / s_t required");
@@ -1073,11 +1073,11 @@ extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t
   dim3 grid((unsigned)(cols / kTile), (unsigned)grid_tiles), block(256);
   const int nt = (int)(cols / kTile);
   if (x_dtype == AAMD_BF16)
-    quant_dual_grouped_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
+    quant_dual_grouped_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   else if (x_dtype == AAMD_F16)
-    quant_dual_grouped_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
+    quant_dual_grouped_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   else
-    quant_dual_grouped_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
+    quant_dual_grouped_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   AAMD_LAUNCH_CHECK("quant_dual_grouped");
   return AAMD_OK;
 }
@@ -1095,7 +1095,7 @@ extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype,
   AAMD_REQUIRE(topk >= 1 && topk <= 32768, "permute_quant_dual: topk=%d out of range", topk);
   AAMD_REQUIRE(T * topk < ((int64_t)1 << 31) && M <= T * topk, "permute_quant_dual: T * topk must stay below 2^31 and M within it");
   AAMD_REQUIRE(ld_t < kMaxTileLd && cols < kMaxTileLd, "permute_quant_dual: ld_t=%lld too large", (long long)ld_t);
-  AAMD_REQUIRE(E >= 1 && group_offsets, "permute_quant_dual: group_offsets required");
+  AAMD_REQUIRE(E >= 1 && (group_offsets || E == 1), "permute_quant_dual: group_offsets required when E > 1");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "permute_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "permute_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "permute_quant_dual: q_t / s_t required");
@@ -1115,11 +1115,11 @@ extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype,
   dim3 grid((unsigned)(cols / kTile), (unsigned)grid_tiles), block(256);
   const int nt = (int)(cols / kTile);
   if (x_dtype == AAMD_BF16)
-    quant_dual_gather_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+    quant_dual_gather_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps);
   else if (x_dtype == AAMD_F16)
-    quant_dual_gather_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+    quant_dual_gather_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps);
   else
-    quant_dual_gather_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+    quant_dual_gather_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps);
   AAMD_LAUNCH_CHECK("permute_quant_dual_grouped");
   return AAMD_OK;
 }
@@ -1153,7 +1153,7 @@ extern "C" int aamd_swiglu_quant_1x128_dual_grouped(const void* fc1, int64_t M, 
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "swiglu_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && F >= 0 && F % kTile == 0, "swiglu_quant_dual: F=%lld must be a multiple of 128", (long long)F);
   AAMD_REQUIRE(ld >= 2 * F && ld % 8 == 0 && ld < kMaxTileLd && ld_t < kMaxTileLd, "swiglu_quant_dual: bad ld=%lld", (long long)ld);
-  AAMD_REQUIRE(E >= 1 && group_offsets, "swiglu_quant_dual: group_offsets required");
+  AAMD_REQUIRE(E >= 1 && (group_offsets || E == 1), "swiglu_quant_dual: group_offsets required when E > 1");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "swiglu_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "swiglu_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "swiglu_quant_dual: q_t / s_t required");
@@ -1166,7 +1166,7 @@ extern "C" int aamd_swiglu_quant_1x128_dual_grouped(const void* fc1, int64_t M, 
   AAMD_REQUIRE(grid_tiles <= 65535, "swiglu_quant_dual: more than 65535 token tiles");
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(F / kTile), (unsigned)grid_tiles), block(256);
-  quant_dual_grouped_kernel<GLU><<<grid, block, 0, st>>>((const u16*)fc1, ld, (int)(F / kTile), group_offsets, E,
+  quant_dual_grouped_kernel<GLU><<<grid, block, 0, st>>>((const u16*)fc1, ld, (int)(F / kTile), group_offsets, E, M,
                                                          q, s, q_t, s_t, ld_t, q_t_layout, 0.f, F, (u16*)h_out);
   AAMD_LAUNCH_CHECK("swiglu_quant_dual_grouped");
   return AAMD_OK;
@@ -1200,7 +1200,7 @@ extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh,
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "gelu_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && F >= 0 && F % kTile == 0, "gelu_quant_dual: F=%lld must be a multiple of 128", (long long)F);
   AAMD_REQUIRE(ld >= F && ld % 8 == 0 && ld < kMaxTileLd && ld_t < kMaxTileLd, "gelu_quant_dual: bad ld=%lld", (long long)ld);
-  AAMD_REQUIRE(E >= 1 && group_offsets, "gelu_quant_dual: group_offsets required");
+  AAMD_REQUIRE(E >= 1 && (group_offsets || E == 1), "gelu_quant_dual: group_offsets required when E > 1");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "gelu_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "gelu_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "gelu_quant_dual: q_t / s_t required");
@@ -1216,11 +1216,11 @@ extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh,
   dim3 grid((unsigned)(F / kTile), (unsigned)grid_tiles), block(256);
   gelu_lut_kernel<<<dim3((2 * kLutN + 255) / 256), dim3(256), 0, st>>>();
   if (dh == nullptr) {
-    quant_dual_grouped_kernel<GELU><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, q, s,
+    quant_dual_grouped_kernel<GELU><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, M, q, s,
                                                             q_t, s_t, ld_t, q_t_layout, 0.f, 0, (u16*)h_out);
   } else {
     const int64_t dh_off = (const u16*)dh - (const u16*)x;  // elements; the loader reads dh at x + dh_off
-    quant_dual_grouped_kernel<GELUB><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, q, s,
+    quant_dual_grouped_kernel<GELUB><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, M, q, s,
                                                              q_t, s_t, ld_t, q_t_layout, 0.f, dh_off, (u16*)h_out);
   }
   AAMD_LAUNCH_CHECK("gelu_quant_dual_grouped");
@@ -1237,7 +1237,7 @@ extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t 
   AAMD_REQUIRE(ld >= 2 * F && ld % 8 == 0 && ld_dh >= F && ld_dh % 8 == 0 && ld < kMaxTileLd && ld_dh < kMaxTileLd && ld_t < kMaxTileLd,
                "swiglu_bwd_quant_dual: bad ld=%lld / ld_dh=%lld",
                (long long)ld, (long long)ld_dh);
-  AAMD_REQUIRE(E >= 1 && group_offsets, "swiglu_bwd_quant_dual: group_offsets required");
+  AAMD_REQUIRE(E >= 1 && (group_offsets || E == 1), "swiglu_bwd_quant_dual: group_offsets required when E > 1");
   AAMD_REQUIRE(ld_t % kTile == 0 && ld_t >= 0, "swiglu_bwd_quant_dual: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE((q == nullptr) == (s == nullptr), "swiglu_bwd_quant_dual: q and s go together");
   AAMD_REQUIRE(q_t && s_t, "swiglu_bwd_quant_dual: q_t / s_t required");
@@ -1253,7 +1253,7 @@ extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t 
   const int nt = (int)(2 * F / kTile);
   dim3 grid((unsigned)(nt / 2), (unsigned)grid_tiles), block(512);  // two teams: the da and the db tile of a feature tile
   sigmoid_lut_kernel<<<dim3((2 * kSigN + 255) / 256), dim3(256), 0, st>>>();
-  swiglu_bwd_dual_kernel<<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, E,
+  swiglu_bwd_dual_kernel<<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, E, M,
                                                  q, s, q_t, s_t, ld_t, q_t_layout, (u16*)g_out);
   AAMD_LAUNCH_CHECK("swiglu_bwd_quant_dual_grouped");
   return AAMD_OK;

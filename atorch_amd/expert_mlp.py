@@ -31,6 +31,7 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import kernels
+from ._lib import host
 from .bias_gather_add import bias_gather_add_bw
 from .gmm import _offsets
 from .quantization import WeightCodeCache
@@ -62,67 +63,35 @@ def _quant_first_weight(w1, v1, transpose_w1, need_transpose=True):
     return q, s, q_t, s_t
 
 
-class _Fp8ExpertMlp(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, w1, w2, v1, b1, b2, batch_sizes, transpose_w1, activation, dispatch, is_first_microbatch,
-                weight_cache):
-        assert x.dim() == 2 and w1.dim() == 3 and w2.dim() == 3
-        E = w1.shape[0]
-        goff = dispatch.group_offsets if dispatch is not None else _offsets(batch_sizes, x.device)
-        train = any(ctx.needs_input_grad)  # all False under no_grad
-        glu = activation == "swiglu"
-        # first weight(s) as [E, N1, H] (rows = outputs), second as [E, H, F]: block quantisation
-        # commutes with the transpose, so both orientations come out of one launch each
-        quant1 = lambda t: _quant_first_weight(w1, v1, transpose_w1)  # noqa: E731
-        quant2 = lambda t: kernels.block_quant_batched(w2.detach().contiguous(), return_transpose=True)  # noqa: E731
-        if weight_cache is None:
-            (q1, s1, q1_t, s1_t), (q2, s2, q2_t, s2_t) = quant1(True), quant2(True)
-        else:
-            q1, s1, q1_t, s1_t = weight_cache.codes("w1", (w1, v1), is_first_microbatch, True, quant1)
-            q2, s2, q2_t, s2_t = weight_cache.codes("w2", (w2,), is_first_microbatch, True, quant2)
-        xc = x.detach().contiguous()
-        if dispatch is not None:
-            M = dispatch.sorted_indices.numel()
-            if train:
-                qx, sx, qx_t, sx_t = kernels.permute_tile_quant_dual_grouped(
-                    xc, dispatch.sorted_indices, dispatch.topk, goff, E, blocked=True
-                )
-            else:  # every token quantised once, its codes written to its top-k rows
-                qx, sx = kernels.permute_tile_quant(xc, dispatch.row_map, dispatch.topk, M)
-        elif train:
-            qx, sx, qx_t, sx_t = kernels.tile_quant_dual_grouped(xc, goff, E, blocked=True)
-        else:
-            qx, sx = kernels.tile_quant(xc)
-        fc1 = kernels.grouped_gemm_nt(qx, sx, q1, s1, goff, out_dtype=torch.bfloat16,
-                                      bias=b1.detach().contiguous() if b1 is not None else None)  # fmt: skip
-        if train:
-            quant = kernels.swiglu_tile_quant_dual_grouped if glu else kernels.gelu_tile_quant_dual_grouped
-            qh, sh, qh_t, sh_t = quant(fc1, goff, E, ld_t=kernels.qt_ld(qx_t), blocked=True)
-        else:
-            qh, sh = kernels.swiglu_tile_quant(fc1) if glu else kernels.gelu_tile_quant(fc1)
-        out = kernels.grouped_gemm_nt(qh, sh, q2_t, s2_t, goff, out_dtype=x.dtype,
-                                      bias=b2.detach().contiguous() if b2 is not None else None)  # fmt: skip
-        if train:
-            ctx.transpose_w1, ctx.glu, ctx.has_v1 = transpose_w1, glu, v1 is not None
-            ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
-            ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)
-            ctx.dispatch_topk = dispatch.topk if dispatch is not None else 0
-            ctx.num_tokens = x.shape[0]
-            row_map = dispatch.row_map if dispatch is not None else goff
-            ctx.save_for_backward(goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map)
-        return out
+def _weight_codes(w1, w2, v1, transpose_w1, is_first_microbatch, weight_cache):
+    """``(q1, s1, q1_t, s1_t), (q2, s2, q2_t, s2_t)``: the first weight(s) as [E, N1, H] (rows = outputs) and the second
+    as [E, F, H], each with its transpose; block quantisation commutes with the transpose, so both orientations
+    come out of one launch each."""
+    quant1 = lambda t: _quant_first_weight(w1, v1, transpose_w1)  # noqa: E731
+    quant2 = lambda t: kernels.block_quant_batched(w2.detach().contiguous(), return_transpose=True)  # noqa: E731
+    if weight_cache is None:
+        return quant1(True), quant2(True)
+    return (weight_cache.codes("w1", (w1, v1), is_first_microbatch, True, quant1),
+            weight_cache.codes("w2", (w2,), is_first_microbatch, True, quant2))  # fmt: skip
 
-    @staticmethod
-    def backward(ctx, dy):
-        goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map = ctx.saved_tensors
+
+def _bias(b):
+    return b.detach().contiguous() if b is not None else None
+
+
+def _mlp_backward(ctx, dy, goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map):
+    """``(dx, dw1, dw2, dv1, db1, db2)`` from the gradient of the MLP's output rows."""
+    x_dtype, w1_dtype, w2_dtype = ctx.dtypes
+    dy = dy.contiguous().to(torch.bfloat16)
+    db1 = db2 = None
+    if not (ctx.has_b1 or ctx.has_b2):
+        dx, dw1, dw2 = host().mlp_backward(dy, goff, row_map, ctx.dispatch_topk, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t,
+                                           q2, s2, ctx.glu, ctx.transpose_w1, x_dtype, w1_dtype, w2_dtype)  # fmt: skip
+    else:
         E = goff.numel() - 1
-        x_dtype, w1_dtype, w2_dtype = ctx.dtypes
-        dy = dy.contiguous().to(torch.bfloat16)
-        M = dy.shape[0]
         ld_t = kernels.qt_ld(qx_t)
-        bin_ids = None
-        if ctx.has_b1 or ctx.has_b2:  # expert of every row, from the device-side offsets (no host round trip)
-            bin_ids = torch.repeat_interleave(torch.arange(E, device=dy.device), goff[1:] - goff[:-1], output_size=M)
+        # expert of every row, from the device-side offsets (no host round trip)
+        bin_ids = torch.repeat_interleave(torch.arange(E, device=dy.device), goff[1:] - goff[:-1], output_size=dy.shape[0])
         db2 = bias_gather_add_bw(dy, bin_ids, E) if ctx.has_b2 else None
         qdy, sdy, qdy_t, sdy_t = kernels.tile_quant_dual_grouped(dy, goff, E, ld_t=ld_t, blocked=True)
         # through the second linear: dh = dy @ w2^T ([M, F]); dw2[f, h] = sum_m h[m, f] dy[m, h]
@@ -144,11 +113,80 @@ class _Fp8ExpertMlp(torch.autograd.Function):
             dw1 = kernels.grouped_gemm_wgrad(qg_t, sg_t, qx_t, sx_t, goff, out_dtype=w1_dtype)
         else:
             dw1 = kernels.grouped_gemm_wgrad(qx_t, sx_t, qg_t, sg_t, goff, out_dtype=w1_dtype)
-        dv1 = None
-        if ctx.has_v1:  # the gate and the up half of the gradient go back to their own parameters
-            dim = 1 if ctx.transpose_w1 else 2
-            dw1, dv1 = (t.contiguous() for t in torch.chunk(dw1, 2, dim=dim))
-        return dx, dw1, dw2, dv1, db1, db2, None, None, None, None, None, None
+    dv1 = None
+    if ctx.has_v1:  # the gate and the up half of the gradient go back to their own parameters
+        dim = 1 if ctx.transpose_w1 else 2
+        dw1, dv1 = (t.contiguous() for t in torch.chunk(dw1, 2, dim=dim))
+    return dx, dw1, dw2, dv1, db1, db2
+
+
+class _Fp8ExpertMlp(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w1, w2, v1, b1, b2, batch_sizes, transpose_w1, activation, dispatch, is_first_microbatch,
+                weight_cache):
+        assert x.dim() == 2 and w1.dim() == 3 and w2.dim() == 3
+        goff = dispatch.group_offsets if dispatch is not None else _offsets(batch_sizes, x.device)
+        train = any(ctx.needs_input_grad)  # all False under no_grad
+        glu = activation == "swiglu"
+        codes1, codes2 = _weight_codes(w1, w2, v1, transpose_w1, is_first_microbatch, weight_cache)
+        q1, s1, q1_t, s1_t = codes1
+        q2, s2, q2_t, s2_t = codes2
+        sorted_idx, row_map, topk = (None, None, 0) if dispatch is None else dispatch[:3]
+        out, fc1, qx_t, sx_t, qh_t, sh_t = host().mlp_forward(
+            x.detach().contiguous(), goff, sorted_idx, row_map, topk, q1, s1, q2_t, s2_t, _bias(b1), _bias(b2), glu, train
+        )
+        if train:
+            ctx.transpose_w1, ctx.glu, ctx.has_v1 = transpose_w1, glu, v1 is not None
+            ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
+            ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)
+            ctx.dispatch_topk = topk
+            ctx.num_tokens = x.shape[0]
+            ctx.save_for_backward(goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map)
+        return out
+
+    @staticmethod
+    def backward(ctx, dy):
+        return (*_mlp_backward(ctx, dy, *ctx.saved_tensors), None, None, None, None, None, None)
+
+
+class _Fp8MoeLayer(torch.autograd.Function):
+    """Routing, expert MLP and weighted combine as one function: the work of the three ops, one call into native code
+    per direction.  Returns the combined tokens; the routing is left in ``dispatcher``."""
+
+    @staticmethod
+    def forward(ctx, x, probs, w1, w2, v1, b1, b2, top_experts, dispatcher, transpose_w1, glu, is_first_microbatch,
+                weight_cache):
+        train = ctx is not None and any(ctx.needs_input_grad)
+        codes1, codes2 = _weight_codes(w1, w2, v1, transpose_w1, is_first_microbatch, weight_cache)
+        q1, s1, q1_t, s1_t = codes1
+        q2, s2, q2_t, s2_t = codes2
+        topk = dispatcher.topk
+        probs_c = probs.contiguous()
+        out, sorted_idx, row_map, goff, y, fc1, qx_t, sx_t, qh_t, sh_t = host().layer_forward(
+            x.contiguous(), probs_c, top_experts.contiguous(), topk, q1, s1, q2_t, s2_t, _bias(b1), _bias(b2), glu, train
+        )
+        dispatcher.set_routing(sorted_idx, row_map, goff)
+        if train:
+            ctx.transpose_w1, ctx.glu, ctx.has_v1 = transpose_w1, glu, v1 is not None
+            ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
+            ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)
+            ctx.dispatch_topk = topk
+            ctx.num_tokens = x.shape[0]
+            ctx.save_for_backward(y, probs_c, goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        y, probs, *saved = ctx.saved_tensors
+        row_map = saved[-1]
+        dout = dout.contiguous()
+        d_probs = None
+        if ctx.needs_input_grad[1]:
+            dy, d_probs = kernels.unpermute_backward(dout, y, row_map, probs, ctx.dispatch_topk)
+        else:
+            dy = kernels.permute_rows_scaled(dout, row_map, ctx.dispatch_topk, y.shape[0], probs, y.dtype)
+        dx, dw1, dw2, dv1, db1, db2 = _mlp_backward(ctx, dy, *saved)
+        return dx, d_probs, dw1, dw2, dv1, db1, db2, None, None, None, None, None, None
 
 
 def grouped_mlp(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,

@@ -12,18 +12,19 @@ from typing import Optional
 import torch
 
 from . import kernels
+from ._lib import host
 from .quantization import WeightCodeCache
 
 TILE = kernels.TILE
 
 
 def _offsets(batch_sizes: torch.Tensor, device) -> torch.Tensor:
-    """Exclusive prefix [E+1] on the device; computed where ``batch_sizes`` lives (the reference
-    passes a CPU tensor, grouped_gemm_moe.py:837), so a device tensor costs no host round trip."""
-    bs = batch_sizes.to(torch.int64)
-    off = torch.zeros(bs.numel() + 1, dtype=torch.int64, device=bs.device)
-    off[1:] = torch.cumsum(bs, 0)
-    return off.to(device)
+    """Exclusive prefix [E+1] on the device, in one launch.  The counts of a CPU tensor (the reference passes one,
+    grouped_gemm_moe.py:837) travel in the kernel's arguments: a copy from pageable memory would wait for the stream."""
+    bs = batch_sizes.reshape(-1).to(torch.int64).contiguous()
+    if not bs.is_cuda or bs.device == device:
+        return host().offsets_from_tensor(bs, device)
+    return host().offsets_from_tensor(bs.to(device), device)
 
 
 class _Fp8Gmm(torch.autograd.Function):

@@ -12,7 +12,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from ._lib import check, dtype_code, lib, ptr, stream
+from ._lib import check, dtype_code, host, lib, ptr, stream
 
 TILE = 128
 FP8 = torch.float8_e4m3fn
@@ -33,10 +33,13 @@ def padded_bound(rows: int, num_groups: int) -> int:
 
 
 def group_offsets_from_splits(splits: Sequence[int], device) -> torch.Tensor:
-    off = [0]
-    for m in splits:
-        off.append(off[-1] + int(m))
-    return torch.tensor(off, dtype=torch.int64, device=device)
+    device = torch.device(device)
+    if device.type != "cuda":
+        off = [0]
+        for m in splits:
+            off.append(off[-1] + int(m))
+        return torch.tensor(off, dtype=torch.int64, device=device)
+    return host().offsets_from_list([int(m) for m in splits], device)
 
 
 # ------------------------------------------------------------------------------------------
@@ -59,9 +62,9 @@ def tile_quant(
     assert block_size == TILE, "only block_size 128 is supported"
     assert x.is_contiguous()
     assert x.size(-1) % block_size == 0
-    cols = x.size(-1)
-    rows = x.numel() // cols if cols else 0
     if return_transpose:
+        cols = x.size(-1)
+        rows = x.numel() // cols if cols else 0
         assert x.dim() == 2, "return_transpose needs a 2-D input"
         if rows == 0:  # an empty group: nothing to launch
             return (
@@ -70,13 +73,9 @@ def tile_quant(
                 torch.empty((cols, 0), dtype=FP8, device=x.device),
                 torch.empty((cols, 0), dtype=torch.float32, device=x.device),
             )
-        goff = torch.tensor([0, rows], dtype=torch.int64, device=x.device)
-        y, s, y_t, s_t = tile_quant_dual_grouped(x, goff, 1, eps=eps, ld_t=padded_total([rows]))
+        y, s, y_t, s_t = host().dual(x, None, 1, eps, padded_total([rows]), True, False)
         return y, s, y_t[:, :rows], s_t.t()
-    y = torch.empty(x.shape, dtype=FP8, device=x.device)
-    s = torch.empty(*x.shape[:-1], cols // TILE, dtype=torch.float32, device=x.device)
-    check(lib().aamd_quant_1x128(ptr(x), dtype_code(x.dtype, True), rows, cols, cols, ptr(y), ptr(s), eps, stream()))
-    return y, s
+    return host().tile_quant(x, eps)
 
 
 def block_quant(
@@ -144,14 +143,7 @@ def permute_tile_quant(
     T, cols = x.shape
     assert cols % TILE == 0
     assert row_map.dtype == torch.int32 and row_map.numel() == T * topk and row_map.is_contiguous()
-    q = torch.empty((num_out_rows, cols), dtype=FP8, device=x.device)
-    s = torch.empty((num_out_rows, cols // TILE), dtype=torch.float32, device=x.device)
-    check(
-        lib().aamd_permute_quant_1x128(
-            ptr(x), dtype_code(x.dtype, True), T, cols, cols, ptr(row_map), topk, num_out_rows, ptr(q), ptr(s), eps, stream()
-        )
-    )
-    return q, s
+    return host().permute_tile_quant(x, row_map, topk, num_out_rows, eps)
 
 
 def permute_rows(x: torch.Tensor, row_map: torch.Tensor, topk: int, num_out_rows: int) -> torch.Tensor:
@@ -159,11 +151,7 @@ def permute_rows(x: torch.Tensor, row_map: torch.Tensor, topk: int, num_out_rows
     assert x.dim() == 2 and x.is_contiguous()
     T, cols = x.shape
     assert row_map.dtype == torch.int32 and row_map.numel() == T * topk and row_map.is_contiguous()
-    out = torch.empty((num_out_rows, cols), dtype=x.dtype, device=x.device)
-    check(
-        lib().aamd_permute_rows(ptr(x), dtype_code(x.dtype), T, cols, ptr(row_map), topk, num_out_rows, ptr(out), stream())
-    )
-    return out
+    return host().permute_rows(x, row_map, topk, num_out_rows)
 
 
 def _alloc_qt(rows: int, ld_t: int, blocked: bool, dev) -> torch.Tensor:
@@ -207,18 +195,7 @@ def tile_quant_dual_grouped(
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == num_groups + 1
     if ld_t is None:
         ld_t = padded_bound(M, num_groups)
-    dev = x.device
-    q = torch.empty((M, cols), dtype=FP8, device=dev) if rowwise else None
-    s = torch.empty((M, cols // TILE), dtype=torch.float32, device=dev) if rowwise else None
-    q_t = _alloc_qt(cols, ld_t, blocked, dev)
-    s_t = torch.empty((ld_t // TILE, cols), dtype=torch.float32, device=dev)
-    check(
-        lib().aamd_quant_1x128_dual_grouped(
-            ptr(x), dtype_code(x.dtype, True), M, cols, cols, ptr(group_offsets), num_groups, None,
-            ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), eps, stream(),
-        )
-    )  # fmt: skip
-    return q, s, q_t, s_t
+    return host().dual(x, group_offsets, num_groups, eps, ld_t, rowwise, blocked)
 
 
 def permute_tile_quant_dual_grouped(
@@ -244,18 +221,7 @@ def permute_tile_quant_dual_grouped(
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == num_groups + 1
     if ld_t is None:
         ld_t = padded_bound(M, num_groups)
-    dev = x.device
-    q = torch.empty((M, cols), dtype=FP8, device=dev) if rowwise else None
-    s = torch.empty((M, cols // TILE), dtype=torch.float32, device=dev) if rowwise else None
-    q_t = _alloc_qt(cols, ld_t, blocked, dev)
-    s_t = torch.empty((ld_t // TILE, cols), dtype=torch.float32, device=dev)
-    check(
-        lib().aamd_permute_quant_1x128_dual_grouped(
-            ptr(x), dtype_code(x.dtype, True), T, cols, cols, ptr(sorted_idx), topk, M, ptr(group_offsets), num_groups,
-            None, ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), eps, stream(),
-        )
-    )  # fmt: skip
-    return q, s, q_t, s_t
+    return host().permute_dual(x, sorted_idx, topk, group_offsets, num_groups, eps, ld_t, rowwise, blocked)
 
 
 def swiglu_tile_quant(fc1: torch.Tensor, return_activation: bool = False):
@@ -265,13 +231,7 @@ def swiglu_tile_quant(fc1: torch.Tensor, return_activation: bool = False):
     assert fc1.dtype == torch.bfloat16 and fc1.stride(-1) == 1 and fc1.is_contiguous()
     two_f = fc1.size(-1)
     assert two_f % (2 * TILE) == 0, "the gated width must be a multiple of 128"
-    F = two_f // 2
-    rows = fc1.numel() // two_f if two_f else 0
-    dev = fc1.device
-    q = torch.empty(*fc1.shape[:-1], F, dtype=FP8, device=dev)
-    s = torch.empty(*fc1.shape[:-1], F // TILE, dtype=torch.float32, device=dev)
-    h = torch.empty(*fc1.shape[:-1], F, dtype=torch.bfloat16, device=dev) if return_activation else None
-    check(lib().aamd_swiglu_quant_1x128(ptr(fc1), rows, F, two_f, ptr(h), ptr(q), ptr(s), stream()))
+    q, s, h = host().act_quant(fc1, True, return_activation)
     return (q, s, h) if return_activation else (q, s)
 
 
@@ -290,23 +250,11 @@ def swiglu_tile_quant_dual_grouped(
     assert fc1.dim() == 2 and fc1.is_contiguous() and fc1.dtype == torch.bfloat16
     M, two_f = fc1.shape
     assert two_f % (2 * TILE) == 0
-    F = two_f // 2
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == num_groups + 1
     if ld_t is None:
         ld_t = padded_bound(M, num_groups)
-    dev = fc1.device
-    q = torch.empty((M, F), dtype=FP8, device=dev) if rowwise else None
-    s = torch.empty((M, F // TILE), dtype=torch.float32, device=dev) if rowwise else None
-    q_t = _alloc_qt(F, ld_t, blocked, dev)
-    s_t = torch.empty((ld_t // TILE, F), dtype=torch.float32, device=dev)
-    h = torch.empty((M, F), dtype=torch.bfloat16, device=dev) if return_activation else None
-    check(
-        lib().aamd_swiglu_quant_1x128_dual_grouped(
-            ptr(fc1), M, F, two_f, ptr(group_offsets), num_groups, None, ptr(h),
-            ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), stream(),
-        )
-    )  # fmt: skip
-    return (q, s, q_t, s_t, h) if return_activation else (q, s, q_t, s_t)
+    res = host().act_dual(fc1, None, True, group_offsets, num_groups, ld_t, rowwise, blocked, return_activation)
+    return res if return_activation else res[:4]
 
 
 def swiglu_bwd_tile_quant_dual_grouped(
@@ -333,19 +281,8 @@ def swiglu_bwd_tile_quant_dual_grouped(
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == num_groups + 1
     if ld_t is None:
         ld_t = padded_bound(M, num_groups)
-    dev = fc1.device
-    q = torch.empty((M, two_f), dtype=FP8, device=dev) if rowwise else None
-    s = torch.empty((M, two_f // TILE), dtype=torch.float32, device=dev) if rowwise else None
-    q_t = _alloc_qt(two_f, ld_t, blocked, dev)
-    s_t = torch.empty((ld_t // TILE, two_f), dtype=torch.float32, device=dev)
-    g = torch.empty((M, two_f), dtype=torch.bfloat16, device=dev) if return_grad else None
-    check(
-        lib().aamd_swiglu_bwd_quant_1x128_dual_grouped(
-            ptr(dh), F, ptr(fc1), two_f, M, F, ptr(group_offsets), num_groups, None, ptr(g),
-            ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), stream(),
-        )
-    )  # fmt: skip
-    return (q, s, q_t, s_t, g) if return_grad else (q, s, q_t, s_t)
+    res = host().act_dual(fc1, dh, True, group_offsets, num_groups, ld_t, rowwise, blocked, return_grad)
+    return res if return_grad else res[:4]
 
 
 def gelu_tile_quant(x: torch.Tensor, return_activation: bool = False):
@@ -353,14 +290,8 @@ def gelu_tile_quant(x: torch.Tensor, return_activation: bool = False):
     grouped_gemm_moe.py:449) quantised 1x128 along the last dim without writing ``h``.
     Returns ``(q, s)`` or ``(q, s, h)``."""
     assert x.dtype == torch.bfloat16 and x.is_contiguous()
-    F = x.size(-1)
-    assert F % TILE == 0
-    rows = x.numel() // F if F else 0
-    dev = x.device
-    q = torch.empty(x.shape, dtype=FP8, device=dev)
-    s = torch.empty(*x.shape[:-1], F // TILE, dtype=torch.float32, device=dev)
-    h = torch.empty(x.shape, dtype=torch.bfloat16, device=dev) if return_activation else None
-    check(lib().aamd_gelu_quant_1x128(ptr(x), rows, F, F, ptr(h), ptr(q), ptr(s), stream()))
+    assert x.size(-1) % TILE == 0
+    q, s, h = host().act_quant(x, False, return_activation)
     return (q, s, h) if return_activation else (q, s)
 
 
@@ -385,38 +316,15 @@ def gelu_tile_quant_dual_grouped(
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == num_groups + 1
     if ld_t is None:
         ld_t = padded_bound(M, num_groups)
-    dev = x.device
-    q = torch.empty((M, F), dtype=FP8, device=dev) if rowwise else None
-    s = torch.empty((M, F // TILE), dtype=torch.float32, device=dev) if rowwise else None
-    q_t = _alloc_qt(F, ld_t, blocked, dev)
-    s_t = torch.empty((ld_t // TILE, F), dtype=torch.float32, device=dev)
-    h = torch.empty((M, F), dtype=torch.bfloat16, device=dev) if return_activation else None
-    check(
-        lib().aamd_gelu_quant_1x128_dual_grouped(
-            ptr(x), ptr(dh), M, F, F, ptr(group_offsets), num_groups, None, ptr(h),
-            ptr(q), ptr(s), ptr(q_t), ptr(s_t), ld_t, int(blocked), stream(),
-        )
-    )  # fmt: skip
-    return (q, s, q_t, s_t, h) if return_activation else (q, s, q_t, s_t)
+    res = host().act_dual(x, dh, False, group_offsets, num_groups, ld_t, rowwise, blocked, return_activation)
+    return res if return_activation else res[:4]
 
 
 def block_quant_batched(w: torch.Tensor, eps: float = 0.0, return_transpose: bool = False):
     """128x128 block quantisation of ``w [E, N, K]`` in one launch.
     Returns ``(q [E,N,K], s [E,N/128,K/128], q_t [E,K,N] | None, s_t [E,K/128,N/128] | None)``."""
     assert w.dim() == 3 and w.stride(2) == 1 and w.stride(1) == w.size(2), "rows of w must be dense"
-    E, N, K = w.shape
-    dev = w.device
-    q = torch.empty((E, N, K), dtype=FP8, device=dev)
-    s = torch.empty((E, N // TILE, K // TILE), dtype=torch.float32, device=dev)
-    q_t = torch.empty((E, K, N), dtype=FP8, device=dev) if return_transpose else None
-    s_t = torch.empty((E, K // TILE, N // TILE), dtype=torch.float32, device=dev) if return_transpose else None
-    estride = w.stride(0) if E > 1 else N * K
-    check(
-        lib().aamd_quant_128x128(
-            ptr(w), dtype_code(w.dtype, True), E, N, K, estride, ptr(q), ptr(s), ptr(q_t), ptr(s_t), eps, stream()
-        )
-    )
-    return q, s, q_t, s_t
+    return host().block_quant(w, eps, return_transpose)
 
 
 def grouped_gemm_nt(
@@ -435,22 +343,20 @@ def grouped_gemm_nt(
     E, N, Kb = b.shape
     assert Kb == K and a.stride(1) == 1 and b.is_contiguous() and a_s.is_contiguous() and b_s.is_contiguous()
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == E + 1
+    assert out is None or (out.shape == (M, N) and out.stride(1) == 1)
+    assert bias is None or (bias.shape == (E, N) and bias.is_contiguous())
+    pinned = _pinned_options()
+    if not pinned:
+        return host().gemm_nt(a, a_s, b, b_s, group_offsets, out, out_dtype, bias)
+    from . import _probes
+
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    assert out.shape == (M, N) and out.stride(1) == 1
-    b_tile_scaled = b_s.size(1) == N
-    if bias is not None:
-        assert bias.shape == (E, N) and bias.is_contiguous()
-    args = (ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), int(b_tile_scaled), ptr(group_offsets), E, None,
-            M, N, K, ptr(out), dtype_code(out.dtype), out.stride(0),
-            ptr(bias), dtype_code(bias.dtype) if bias is not None else _lib.NONE)  # fmt: skip
-    pinned = _pinned_options()
-    if pinned:
-        from . import _probes
-
-        _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nt(*args, _probes.options_array(pinned), stream()))
-    else:
-        check(lib().aamd_grouped_gemm_fp8_nt(*args, stream()))
+    _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nt(
+        ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), int(b_s.size(1) == N), ptr(group_offsets), E, None, M, N, K, ptr(out),
+        dtype_code(out.dtype), out.stride(0), ptr(bias), dtype_code(bias.dtype) if bias is not None else _lib.NONE,
+        _probes.options_array(pinned), stream(),
+    ))  # fmt: skip
     return out
 
 
@@ -475,20 +381,19 @@ def grouped_gemm_wgrad(
     assert qt_ld(x_t) == ld_t and dy_t.is_contiguous() and x_t.is_contiguous()
     assert sdy_t.shape == (ld_t // TILE, N) and sx_t.shape == (ld_t // TILE, K)
     assert sdy_t.is_contiguous() and sx_t.is_contiguous()
-    if out is None:
-        assert not accumulate
-        out = torch.empty((E, N, K), dtype=out_dtype, device=dy_t.device)
-    assert out.shape == (E, N, K) and out.stride(2) == 1 and out.stride(1) == K
-    estride = out.stride(0) if E > 1 else N * K
-    args = (ptr(dy_t), ptr(sdy_t), ptr(x_t), ptr(sx_t), ld_t, int(blocked), ptr(group_offsets), E, None, N, K,
-            ptr(out), dtype_code(out.dtype), estride, int(accumulate))  # fmt: skip
+    assert out is not None or not accumulate
+    assert out is None or (out.shape == (E, N, K) and out.stride(2) == 1 and out.stride(1) == K)
     pinned = _pinned_options()
-    if pinned:
-        from . import _probes
+    if not pinned:
+        return host().gemm_wgrad(dy_t, sdy_t, x_t, sx_t, group_offsets, out, out_dtype, accumulate)
+    from . import _probes
 
-        _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_wgrad(*args, _probes.options_array(pinned), stream()))
-    else:
-        check(lib().aamd_grouped_gemm_fp8_wgrad(*args, stream()))
+    if out is None:
+        out = torch.empty((E, N, K), dtype=out_dtype, device=dy_t.device)
+    _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_wgrad(
+        ptr(dy_t), ptr(sdy_t), ptr(x_t), ptr(sx_t), ld_t, int(blocked), ptr(group_offsets), E, None, N, K, ptr(out),
+        dtype_code(out.dtype), out.stride(0) if E > 1 else N * K, int(accumulate), _probes.options_array(pinned), stream(),
+    ))  # fmt: skip
     return out
 
 
@@ -497,26 +402,12 @@ def moe_preprocess(expert_ids: torch.Tensor, num_experts: int, want_sorted: bool
     Returns ``(sorted_indices int64 [n] | None, row_map int32 [n], group_offsets int64 [E+1])``."""
     flat = expert_ids.reshape(-1)
     assert flat.is_contiguous() and flat.dtype in (torch.int64, torch.int32)
-    n = flat.numel()
-    dev = flat.device
-    sorted_idx = torch.empty(n, dtype=torch.int64, device=dev) if want_sorted else None
-    row_map = torch.empty(n, dtype=torch.int32, device=dev)
-    goff = torch.empty(num_experts + 1, dtype=torch.int64, device=dev)
-    ws = torch.empty(max(1, lib().aamd_moe_preprocess_ws_ints(n, num_experts)), dtype=torch.int32, device=dev)
-    check(
-        lib().aamd_moe_preprocess(
-            ptr(flat), int(flat.dtype == torch.int64), n, num_experts, ptr(sorted_idx), ptr(row_map), ptr(goff),
-            ptr(ws), stream(),
-        )
-    )
-    return sorted_idx, row_map, goff
+    return host().moe_preprocess(flat, num_experts, want_sorted)
 
 
 def invert_permutation(sorted_indices: torch.Tensor, n_flat: int) -> torch.Tensor:
     si = sorted_indices.to(torch.int64).contiguous()
-    row_map = torch.empty(n_flat, dtype=torch.int32, device=si.device)
-    check(lib().aamd_invert_permutation(ptr(si), si.numel(), n_flat, ptr(row_map), stream()))
-    return row_map
+    return host().invert_permutation(si, n_flat)
 
 
 def unpermute_combine(
@@ -525,22 +416,11 @@ def unpermute_combine(
     """out[t] = sum_j probs[t,j] * y[row_map[t*topk+j]] in one gather-reduce pass (bf16 or fp32 rows;
     the result has the promoted dtype of rows and probs, as the reference's multiply gives it)."""
     assert y.dim() == 2 and y.is_contiguous() and y.dtype in (torch.bfloat16, torch.float32)
-    M, H = y.shape
     assert row_map.dtype == torch.int32 and row_map.numel() == num_tokens * topk
-    if probs is None:
-        pd, out_dtype = _lib.NONE, y.dtype
-    else:
+    if probs is not None:
         assert probs.shape == (num_tokens, topk)
         probs = probs.contiguous()
-        pd = dtype_code(probs.dtype)
-        out_dtype = torch.promote_types(y.dtype, probs.dtype)
-    out = torch.empty((num_tokens, H), dtype=out_dtype, device=y.device)
-    check(
-        lib().aamd_unpermute_combine(
-            ptr(y), dtype_code(y.dtype), M, H, ptr(row_map), ptr(probs), pd, num_tokens, topk, ptr(out), stream()
-        )
-    )
-    return out
+    return host().unpermute_combine(y, row_map, probs, num_tokens, topk)
 
 
 def permute_rows_scaled(
@@ -551,18 +431,19 @@ def permute_rows_scaled(
     assert x.dim() == 2 and x.is_contiguous()
     T, cols = x.shape
     assert row_map.dtype == torch.int32 and row_map.numel() == T * topk and row_map.is_contiguous()
-    alloc = torch.empty if num_out_rows == T * topk else torch.zeros  # dropped copies leave rows unwritten
-    out = alloc((num_out_rows, cols), dtype=out_dtype, device=x.device)
-    pd = _lib.NONE if probs is None else dtype_code(probs.dtype)
     if probs is not None:
         probs = probs.contiguous()
-    check(
-        lib().aamd_permute_rows_scaled(
-            ptr(x), dtype_code(x.dtype), T, cols, ptr(row_map), topk, ptr(probs), pd, num_out_rows, ptr(out),
-            dtype_code(out_dtype), stream(),
-        )
-    )  # fmt: skip
-    return out
+    return host().permute_rows_scaled(x, row_map, topk, num_out_rows, probs, out_dtype)
+
+
+def unpermute_backward(dout: torch.Tensor, y: torch.Tensor, row_map: torch.Tensor, probs: torch.Tensor, topk: int):
+    """Both gradients of ``unpermute_combine`` in one pass over ``dout``: ``(d_rows, d_probs)``, what
+    ``permute_rows_scaled`` and ``unpermute_probs_grad`` give, the latter in the weights' dtype."""
+    assert dout.dim() == 2 and dout.is_contiguous() and y.dim() == 2 and y.is_contiguous()
+    T, H = dout.shape
+    assert y.shape[1] == H and row_map.dtype == torch.int32 and row_map.numel() == T * topk
+    assert probs.shape == (T, topk)
+    return host().unpermute_backward(dout, y, row_map, probs.contiguous(), topk)
 
 
 def unpermute_probs_grad(dout: torch.Tensor, y: torch.Tensor, row_map: torch.Tensor, topk: int) -> torch.Tensor:
@@ -570,14 +451,7 @@ def unpermute_probs_grad(dout: torch.Tensor, y: torch.Tensor, row_map: torch.Ten
     assert dout.dim() == 2 and dout.is_contiguous() and y.dim() == 2 and y.is_contiguous()
     T, H = dout.shape
     assert y.shape[1] == H and row_map.dtype == torch.int32 and row_map.numel() == T * topk
-    dp = torch.empty((T, topk), dtype=torch.float32, device=dout.device)
-    check(
-        lib().aamd_unpermute_probs_grad(
-            ptr(dout), dtype_code(dout.dtype), ptr(y), dtype_code(y.dtype), y.shape[0], H, ptr(row_map), T, topk,
-            ptr(dp), stream(),
-        )
-    )  # fmt: skip
-    return dp
+    return host().unpermute_probs_grad(dout, y, row_map, topk)
 
 
 def split_views(t: torch.Tensor, splits: Sequence[int]) -> List[torch.Tensor]:

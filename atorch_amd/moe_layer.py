@@ -20,7 +20,7 @@ from typing import Callable, List, Optional, Tuple, Union
 
 import torch
 
-from .expert_mlp import grouped_mlp
+from .expert_mlp import _Fp8MoeLayer, grouped_mlp
 from .quantization import WeightCodeCache
 from .token_dispatcher import MoEAllToAllTokenDispatcher
 
@@ -147,6 +147,16 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         return self._forward_megatron(hidden_states, expert_weights, top_experts, se_fn1, se_fn2,
                                       se_fn2_additional_input, is_first_microbatch)  # fmt: skip
 
+    def _forward_fused(self, x, probs, top_experts, is_first_microbatch):
+        """Nothing happens between the experts and the combine: the layer is one function, one native call per
+        direction."""
+        p = self._parameters
+        assert x.dtype == torch.bfloat16, "the fused activation kernels read bf16"
+        assert probs.shape == top_experts.shape == (x.shape[0], self.topk), "router weights and choices are [tokens, topk]"
+        args = (x, probs, p["w1"], p["w2"], p.get("v1"), p.get("b1"), p.get("b2"), top_experts, self.token_dispatcher,
+                self.transpose_w1, self.use_swiglu, is_first_microbatch, self.weight_code_cache)  # fmt: skip
+        return _Fp8MoeLayer.apply(*args) if torch.is_grad_enabled() else _Fp8MoeLayer.forward(None, *args)
+
     def _forward_megatron(self, hidden_states, expert_weights, top_experts, se_fn1=None, se_fn2=None,
                           se_fn2_additional_input=None, is_first_microbatch=None):
         expert_weights = expert_weights.view(-1, expert_weights.shape[-1])
@@ -156,8 +166,10 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         x = hidden_states.reshape(-1, self.hidden_shape[-1])
         if x.shape[0] == 0:
             return hidden_states.clone()
-        # dispatch: only the routing is computed here; the permute itself happens inside the first quantiser
         d.hidden_shape, d.probs = self.hidden_shape, expert_weights
+        if se_fn1 is None and se_fn2 is None and not (self.training and self.output_dropout_prob > 0):
+            return self._forward_fused(x, expert_weights, top_experts, is_first_microbatch).view(self.hidden_shape)
+        # dispatch: only the routing is computed here; the permute itself happens inside the first quantiser
         d.preprocess(top_experts)
 
         se_intermediate = se_fn1(x) if se_fn1 is not None else None

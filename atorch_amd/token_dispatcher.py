@@ -54,6 +54,9 @@ class _UnpermuteCombine(torch.autograd.Function):
             probs = None
         dout = dout.contiguous()
         d_perm = d_probs = None
+        if probs is not None and ctx.needs_input_grad[0] and ctx.needs_input_grad[2]:
+            d_perm, d_probs = kernels.unpermute_backward(dout, permuted, row_map, probs, ctx.topk)
+            return d_perm, None, d_probs, None, None
         if ctx.needs_input_grad[0]:
             d_perm = kernels.permute_rows_scaled(dout, row_map, ctx.topk, permuted.shape[0], probs, permuted.dtype)
         if probs is not None and ctx.needs_input_grad[2]:
@@ -133,6 +136,10 @@ class MoETokenDispatcher:
             indices.contiguous(), self.num_experts
         )
         return self.group_offsets
+
+    def set_routing(self, sorted_indices: torch.Tensor, row_map: torch.Tensor, group_offsets: torch.Tensor):
+        """The results of ``preprocess`` when the routing was computed by the caller."""
+        self.sorted_indices, self.row_map, self.group_offsets = sorted_indices, row_map, group_offsets
 
     def token_permutation(self, hidden_states: torch.Tensor, max_prob: torch.Tensor, max_ind: torch.Tensor):
         self.hidden_shape = hidden_states.shape
@@ -216,10 +223,14 @@ class MoEAllToAllTokenDispatcher(MoETokenDispatcher):
     def preprocess(self, indices: torch.Tensor) -> torch.Tensor:
         """Tokens per local expert, int64 ``[E]`` on the device (token_dispatcher.py:297-353 without its
         ``.cpu()`` copies)."""
-        goff = super().preprocess(indices)
-        self.num_out_tokens = indices.numel()
-        self.reversed_local_input_permutation_mapping = self.sorted_indices
+        self.set_routing(*kernels.moe_preprocess(indices.contiguous(), self.num_experts))
+        goff = self.group_offsets
         return goff[1:] - goff[:-1]
+
+    def set_routing(self, sorted_indices: torch.Tensor, row_map: torch.Tensor, group_offsets: torch.Tensor):
+        super().set_routing(sorted_indices, row_map, group_offsets)
+        self.num_out_tokens = sorted_indices.numel()
+        self.reversed_local_input_permutation_mapping = sorted_indices
 
     def token_permutation(self, hidden_states: torch.Tensor, max_prob: torch.Tensor, max_ind: torch.Tensor,
                           se_fn1: Optional[Callable] = None):

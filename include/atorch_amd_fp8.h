@@ -92,7 +92,8 @@ int aamd_permute_rows(const void *x, int x_dtype, int64_t T, int64_t cols, const
  * quantized_grouped_linear.py:90-101 and :200-206; the transposed result is defined
  * in-tree as tile_quant(x_i.t().contiguous()), atorch/modules/fp8/scaled_linear.py:402-414,
  * with a partial last token tile zero padded.
- *   x [M, cols]; group_offsets [E+1] int64 (device) exclusive prefix of rows per group;
+ *   x [M, cols]; group_offsets [E+1] int64 (device) exclusive prefix of rows per group, or NULL for one group of
+ *   all rows (then E must be 1);
  *   q [M, cols], s [M, cols/128]              (both may be NULL: transposed only)
  *   q_t, in the layout q_t_layout names: token poff_g + m of column c holds the code of x[off_g + m, c], where
  *       poff_g = sum_{j<g} ceil(M_j/128)*128; pad tokens of a group are written 0
@@ -276,6 +277,25 @@ int aamd_permute_rows_scaled(const void *x, int x_dtype, int64_t T, int64_t cols
                              void *stream);
 int aamd_unpermute_probs_grad(const void *dout, int dout_dtype, const void *y, int y_dtype, int64_t M, int64_t H,
                               const int32_t *row_map, int64_t T, int topk, float *dprobs, void *stream);
+
+/*
+ * Both gradients of the combine in one pass: drows[row_map[t*topk+j]] = dout[t] * probs[t, j] rounded to the rows'
+ * type, dprobs[t, j] = sum_h dout[t, h] * y[row_map[t*topk+j], h] (fp32 sums) in the weights' type, 0 for a dropped
+ * copy.  What autograd makes of token_dispatcher.py:155-159.
+ *   dout [T, H] of the combine's result type (fp32 if rows or weights are), y and drows [M, H] of y_dtype, probs and
+ *   dprobs [T, topk] of probs_dtype; rows of drows no map entry points to are not written.
+ */
+int aamd_unpermute_backward(const void *dout, int dout_dtype, const void *y, int y_dtype, int64_t M, int64_t H,
+                            const int32_t *row_map, const void *probs, int probs_dtype, int64_t T, int topk,
+                            void *drows, void *dprobs, void *stream);
+
+/*
+ * group_offsets [E+1] int64 (device) = exclusive prefix of counts [E] int64, rows per group.  counts_on_host != 0:
+ * counts is host memory, read before the call returns, and nothing waits for the device.
+ * Replaces the cumulative sums and host copies around the grouped calls (grouped_gemm_moe.py:837,
+ * quantized_grouped_linear.py:90-101).
+ */
+int aamd_group_offsets(const int64_t *counts, int counts_on_host, int E, int64_t *group_offsets, void *stream);
 
 /*
  * Router preprocess on the device, no host round trip: histogram of expert ids,
