@@ -34,7 +34,7 @@ FP8 = kernels.FP8
 
 def parse_bool_env(name: str, default: str = "False") -> bool:
     """Same accepted spellings as atorch/common/env.py:6-13."""
-    v = os.getenv(name, default)
+    v = os.environ.get(name, default)
     if v in ("1", "True", "true"):
         return True
     if v in ("0", "False", "false"):
@@ -74,15 +74,43 @@ class QuantizeResult:
     scale_t: Optional[torch.Tensor] = None
 
 
-@dataclass
 class QuantizeResultCache:
     """Per-weight cache of the fp8 copies between microbatches
-    (quantized_grouped_linear.py:121-129, 467-470)."""
+    (quantized_grouped_linear.py:121-129, 467-470).
 
-    data: Optional[torch.Tensor] = None
-    scale: Optional[torch.Tensor] = None
-    data_t: Optional[torch.Tensor] = None
-    scale_t: Optional[torch.Tensor] = None
+    Holds either four tensors of its own or, after ``point_to``, a place in the stacked codes of all weights, whose
+    slices are made when somebody asks for them (the fused path reads the stack itself, and four views per expert and
+    call are most of its host time)."""
+
+    __slots__ = ("_own", "stack", "index")
+
+    def __init__(self, data: Optional[torch.Tensor] = None, scale: Optional[torch.Tensor] = None,
+                 data_t: Optional[torch.Tensor] = None, scale_t: Optional[torch.Tensor] = None):
+        self._own = [data, scale, data_t, scale_t]
+        self.stack = None
+        self.index = 0
+
+    def point_to(self, stack, index: int):
+        """Use entry ``index`` of ``stack`` = stacked (data, scale, data_t | None, scale_t | None)."""
+        self._own = [None, None, None, None]
+        self.stack = stack
+        self.index = index
+
+    def _get(self, k: int) -> Optional[torch.Tensor]:
+        if self._own[k] is None and self.stack is not None and self.stack[k] is not None:
+            self._own[k] = self.stack[k][self.index]
+        return self._own[k]
+
+    def _set(self, k: int, value: Optional[torch.Tensor]):
+        if self.stack is not None:
+            self._own = [self._get(i) for i in range(4)]
+            self.stack = None
+        self._own[k] = value
+
+    data = property(lambda self: self._get(0), lambda self, v: self._set(0, v))
+    scale = property(lambda self: self._get(1), lambda self, v: self._set(1, v))
+    data_t = property(lambda self: self._get(2), lambda self, v: self._set(2, v))
+    scale_t = property(lambda self: self._get(3), lambda self, v: self._set(3, v))
 
     def to_qresult(self) -> QuantizeResult:
         return QuantizeResult(self.data, self.scale, self.data_t, self.scale_t)
@@ -104,7 +132,7 @@ class WeightCodeCache:
 
     @staticmethod
     def _stamp(tensors):
-        return tuple((t.data_ptr(), t._version, tuple(t.shape), t.dtype) for t in tensors if t is not None)
+        return tuple((t.data_ptr(), t._version, t.shape, t.dtype) for t in tensors if t is not None)
 
     def codes(self, name: str, tensors, is_first_microbatch: Optional[bool], need_transpose: bool, quantise):
         """``quantise(need_transpose) -> (q, s, q_t | None, s_t | None)`` for the weight tensors ``tensors``."""
@@ -145,6 +173,12 @@ def _check_params(qparams: QParams):
     if shape not in ((1, TILE), (TILE, TILE)):
         raise ValueError(f"quant_tile_shape must be (1, 128) or (128, 128), got {shape}")
     return shape
+
+
+def check_recipe(qp: QLinearParams):
+    """The quantisers of a grouped linear: 1x128 activations and gradients, 128x128 weights."""
+    for params, shape in ((qp.x_params, (1, TILE)), (qp.w_params, (TILE, TILE)), (qp.g_params, (1, TILE))):
+        assert _check_params(params) == shape
 
 
 # ------------------------------------------------------------------------------------------
@@ -204,19 +238,9 @@ class HipQuantizeOp:
 
     supports_fused_grouped = True
 
-    def __init__(self):
-        self._offsets_cache = {}
-
     # -- group offsets on the device ---------------------------------------------------------
     def group_offsets(self, m_splits: Sequence[int], device) -> torch.Tensor:
-        key = (tuple(int(m) for m in m_splits), str(device))
-        t = self._offsets_cache.get(key)
-        if t is None:
-            if len(self._offsets_cache) > 64:
-                self._offsets_cache.clear()
-            t = kernels.group_offsets_from_splits(key[0], device)
-            self._offsets_cache[key] = t
-        return t
+        return kernels.group_offsets_from_splits(m_splits, device)
 
     # -- plugin interface: quantize ---------------------------------------------------------------
     def quantize(self, t: torch.Tensor, qparams: QParams, return_transpose: bool = False) -> QuantizeResult:
