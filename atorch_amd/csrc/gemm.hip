@@ -25,55 +25,17 @@
 // requested two steps ahead).  Rows are 128 bytes; the 16-byte chunks of a row
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
-#include "common.hpp"
+#include "gemm.hpp"
 #ifdef AAMD_TUNING
 #include "../../include/atorch_amd_probes.h"
 #endif
 
 namespace aamd {
 
-constexpr int kBK = 128;  // contraction bytes per step == scale block
-
-enum GemmMode { kRaggedRows = 0, kRaggedK = 1 };
-
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 // XOR swizzle of the 16-byte chunk index inside a 128-byte LDS row (depends on row % 16 only).
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-
-struct GemmParams {
-  const uint8_t* L;
-  const uint8_t* R;
-  const float* Ls;
-  const float* Rs;
-  void* C;
-  const void* bias;
-  const int64_t* goff;      // [E+1] rows per group prefix (device); nullptr: one group [0, Lrows)
-  int64_t ldl, ldr;                          // row strides of L and R (bytes)
-  int64_t l_kb_stride, r_kb_stride;          // bytes between consecutive 128-wide contraction blocks of a row
-  int64_t r_group_stride;                    // bytes between the R matrices of consecutive groups
-  int64_t ls_row_stride, ls_blk_stride;      // L scale (row, block) strides, floats
-  int64_t rs_row_stride, rs_blk_stride, rs_group_stride;
-  int64_t ldc, c_group_stride;               // elements
-  int64_t bias_group_stride;
-  int64_t Lrows;   // kRaggedRows: total token rows; kRaggedK: rows of L (= N of dW)
-  int64_t Rrows;   // rows of R per group
-  int nkb;         // kRaggedRows: K / 128
-  int E;
-  int nRt;         // R tiles
-  int nLt;         // kRaggedK: L tiles
-  int max_kb;      // kRaggedK: contraction blocks the operand buffers hold (ld_t / 128)
-  int accumulate;
-  int group_r;     // the tile order groups R tiles (inside each group of rows / expert) instead of L tiles
-  int bias_dtype;
-  int gl;          // L tiles that share an R panel in the tile order
-  int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
-};
-
-__device__ __forceinline__ v16f mfma_fp8_32x32x64(const v8i& a, const v8i& b, const v16f& c) {
-  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
-}
 
 template <typename OUT>
 __device__ __forceinline__ void store4(OUT* dst, v4f o, bool accumulate) {
@@ -125,13 +87,6 @@ __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-// A 64-bit offset the compiler can keep in scalar registers (it is the same in every lane).
-__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uint64_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
 template <int MODE, bool R_PER_ROW, typename OUT, typename C>
@@ -989,7 +944,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 // Launch choices a caller of the measurement build may pin per call (-1 = the library chooses, which is
 // all the product entry points ever pass).
 struct GemmOptions {
-  int tile = -1;      // 0: 128x128 tiles, 1: the large configuration
+  int tile = -1;      // 0: 128x128 tiles, 1: the large configuration, 2 / 3: the kernel for few rows, 3 in its split form
   int group_r = -1;   // tile order groups R tiles (1) or L tiles (0)
   int gl = -1;        // tiles that share a panel in the tile order
   int ls_batch = -1;  // 0: L scales fetched one contraction block at a time
@@ -1021,14 +976,46 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
   return AAMD_OK;
 }
 
-// Tile choice: large tiles whenever the problem has enough of them to fill the chip
-// (option "tile": 0 forces the small configuration, 1 the large one).
-static bool use_large_tiles(int64_t tiles_256, bool by_default, const GemmOptions& g_opt) {
-  if (g_opt.tile == 0) return false;
-  if (g_opt.tile == 1) return true;
-  // 256x256 tiles halve the bytes every CU pulls from L2 and measured faster wherever the launch
-  // still fills the GPU with them; small launches keep the 128x128 tiles (two workgroups per CU).
-  return by_default && tiles_256 >= 512;
+// Which kernel a row-ragged launch with block-scaled R takes: the one whose estimated time is least.  The estimates (us)
+// are fits to launches on MI355X of 1 to 4096 rows per group, 1 to 64 groups and 512 to 14336 outputs and contraction:
+//   - a tile of the 128x128 configuration costs 10 us outside its loop and 1 us per 128-deep step with two workgroups
+//     per CU (8 and 0.8 with one), and 512 run at a time, so a launch takes whole rounds of that;
+//   - a tile of the 256x256 configuration 8 us and 1.65 us per step (1.2 when the tiles are half empty: waves without
+//     rows only load), 256 at a time;
+//   - the kernel for few rows 1.4 ns per 64 x 64 x 128 block, spread over the chip, and 6 us in all;
+//   - and none can beat the weights' stream from memory, 5.2 TB/s in the first two and 6.2 in the third.
+// Token tiles are counted as the groups' expected number (their sizes are known on the device only): one per group with
+// few rows, half a tile more than the rows fill with many.  Examples, estimate (measured): 32768 rows in 8 groups,
+// 28672 x 4096: large 3.5 ms (3.6), small 4.4; one group of 4096 rows, 4096 x 14336: large 193, small 244 (270 us: the
+// rule that asked for 512 large tiles took them, and 256 are a full round); 8 groups of 16 rows, 4096 x 4096: few 35 (30),
+// small 42 (39).
+enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3 };
+static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, const GemmOptions& g_opt) {
+  if (g_opt.tile >= 0) return g_opt.tile == 1 && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
+  const int64_t groups = M < E ? M : E;
+  auto token_tiles = [&](int rows) -> double {
+    if (!grouped) return (double)((M + rows - 1) / rows);
+    const double many = (double)M / rows + 0.5 * (double)groups;
+    return many > (double)groups ? many : (double)groups;
+  };
+  auto rounds = [](double tiles, int at_a_time) { return (double)(int64_t)((tiles + at_a_time - 1) / at_a_time); };
+  const double weights = (double)groups * (double)N * (double)nkb * (double)kBK;  // bytes
+  const double few_blocks = token_tiles(64) * (double)(N / 64);
+  const double few = 6.0 + 1.4e-3 * few_blocks * (double)nkb;
+  const double tiles_s = token_tiles(128) * (double)(N / 128);
+  const double loop_s = tiles_s <= 256 ? 8.0 + 0.8 * (double)nkb : rounds(tiles_s, 512) * (10.0 + 1.0 * (double)nkb);
+  const double small = loop_s > weights / 5.2e6 ? loop_s : weights / 5.2e6;
+  // (the large configuration takes its scales in batches of eight contraction blocks)
+  const double rows_l = token_tiles(256) * 256.0;
+  const double loop_l = rounds(rows_l / 256.0 * (double)((N + 255) / 256), 256) * (8.0 + ((double)M > 0.5 * rows_l ? 1.65 : 1.2) * (double)nkb);
+  const double large = nkb < 8 ? 1e30 : loop_l > weights / 5.2e6 ? loop_l : weights / 5.2e6;
+  // the split form: with fewer workgroups than half the CUs the length of a wave's contraction is what counts
+  if (few <= small && few <= large) return few_blocks < 128 ? kFewRowsSplit : kFewRows;
+  return large < small ? kLargeTiles : kSmallTiles;
+}
+// Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
+static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
+  return g_opt.tile >= 0 ? g_opt.tile == 1 : tiles_256 >= 512;
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1059,10 +1046,9 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   // scale batches of eight contraction blocks; their 16-byte loads need aligned rows and whole groups of four blocks
   const bool batches = (K / kBK) >= 8 && g_opt.ls_batch != 0;
   const bool batches16 = batches && (K / kBK) % 4 == 0 && aligned16(a_s);
-  // tile-scaled B carries per-row R scales: use the configuration that has room for them; the 256x256
-  // configuration takes all its scales in batches (with 4-byte loads where the rows are not aligned)
-  const bool large = use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), true, g_opt) &&
-                     (b_tile_scaled || batches);
+  const NtKernel kernel = b_tile_scaled ? (use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), g_opt) ? kLargeTiles : kSmallTiles)
+                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, g_opt);
+  const bool large = kernel == kLargeTiles;
   const int BM = large ? CfgLarge::BM : CfgSmall::BM;
   const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : CfgLarge::BN) : CfgSmall::BN;
   GemmParams p = {};
@@ -1079,6 +1065,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   p.goff = group_offsets;
   p.Lrows = M; p.Rrows = N; p.nkb = (int)(K / kBK); p.E = E; p.nRt = (int)((N + BN - 1) / BN); p.nLt = 0;
   p.accumulate = 0;
+  if (kernel == kFewRows || kernel == kFewRowsSplit) return launch_few_rows(p, c_dtype, M, kernel == kFewRowsSplit, st);
   const int64_t max_lt = group_offsets ? M / BM + E : (M + BM - 1) / BM;
   const int64_t blocks = max_lt * p.nRt;
   if (large)

@@ -1,0 +1,57 @@
+// What the grouped GEMM kernels share: their parameters and the fp8 matrix instruction.
+#pragma once
+#include "common.hpp"
+
+namespace aamd {
+
+constexpr int kBK = 128;  // contraction bytes per step == scale block
+
+enum GemmMode { kRaggedRows = 0, kRaggedK = 1 };
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+struct GemmParams {
+  const uint8_t* L;
+  const uint8_t* R;
+  const float* Ls;
+  const float* Rs;
+  void* C;
+  const void* bias;
+  const int64_t* goff;      // [E+1] rows per group prefix (device); nullptr: one group [0, Lrows)
+  int64_t ldl, ldr;                          // row strides of L and R (bytes)
+  int64_t l_kb_stride, r_kb_stride;          // bytes between consecutive 128-wide contraction blocks of a row
+  int64_t r_group_stride;                    // bytes between the R matrices of consecutive groups
+  int64_t ls_row_stride, ls_blk_stride;      // L scale (row, block) strides, floats
+  int64_t rs_row_stride, rs_blk_stride, rs_group_stride;
+  int64_t ldc, c_group_stride;               // elements
+  int64_t bias_group_stride;
+  int64_t Lrows;   // kRaggedRows: total token rows; kRaggedK: rows of L (= N of dW)
+  int64_t Rrows;   // rows of R per group
+  int nkb;         // kRaggedRows: K / 128
+  int E;
+  int nRt;         // R tiles
+  int nLt;         // kRaggedK: L tiles
+  int max_kb;      // kRaggedK: contraction blocks the operand buffers hold (ld_t / 128)
+  int accumulate;
+  int group_r;     // the tile order groups R tiles (inside each group of rows / expert) instead of L tiles
+  int bias_dtype;
+  int gl;          // L tiles that share an R panel in the tile order
+  int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
+};
+
+__device__ __forceinline__ v16f mfma_fp8_32x32x64(const v8i& a, const v8i& b, const v16f& c) {
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+}
+
+// A 64-bit offset the compiler can keep in scalar registers (it is the same in every lane).
+__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uint64_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Row-ragged GEMM with block-scaled R for groups of few rows (gemm_few.hip); reads L, R, their scales and strides, C,
+// bias, goff, E, Lrows, Rrows and nkb of the parameters.
+int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, hipStream_t st);
+
+}  // namespace aamd

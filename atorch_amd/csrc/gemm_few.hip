@@ -1,0 +1,234 @@
+// Row-ragged block-scaled FP8 GEMM for groups of few rows (decoding, small batches, many experts).
+//
+// With at most a few dozen rows per group every weight byte is used once or twice, so the launch is bound by how fast
+// the weights stream from HBM, and the tiles of gemm.hip are the wrong shape for that: they stage 128 or 256 token
+// rows that are mostly not there, have one or two workgroups per CU with two steps of loads in flight, and a workgroup
+// walks the whole contraction alone, which leaves most of the chip idle when few groups have rows or the output is
+// small.  Here a wave takes 32 WTR weight rows x 32 WTL token rows, the waves of a workgroup split the contraction
+// (wave w takes the 128-deep blocks w, w + W, ...) and add up through the LDS at the end.
+// The arithmetic is that of gemm.hip: two chained v_mfma_f32_32x32x64_f8f6f4 per 128-deep block, the raw product folded
+// into fp32 accumulators with the block's scales; only the order of the sum over blocks differs.
+//
+// Measured (us, the 128 x 128 tiles of gemm.hip -> here; weights beyond the last-level cache):
+//   64 groups of 6 rows, 4096 x 7168 weights (1.88 GB)      358 -> 305  (6.2 TB/s; a stream that only reads: 7.1)
+//   64 groups of 6 rows, 7168 x 2048 weights (0.94 GB)      183 -> 157
+//   60 groups of 16 / 48 rows, 1408 x 2048 (0.17 GB)         49 -> 37 / 43
+//   8 groups of 16 / 48 rows, 4096 x 14336 (0.47 GB)        119 -> 81 / 113
+//   one group of 1 / 144 rows, 896 x 6016                    41 -> 9  (split form)
+// From about 64 rows per group the operand reuse of the larger tiles wins.
+#include "gemm.hpp"
+
+namespace aamd {
+
+// W waves, tiles of 32 WTR weight rows x 32 WTL token rows
+template <typename OUT, int W, int WTR, int WTL>
+__global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
+  constexpr int BL = 32 * WTL, BR = 32 * WTR;
+  constexpr int kPitch = BR + 4;  // floats per row of a wave's partial result in the LDS
+  constexpr int kStage = (BR + BL) * kBK + (WTL == 1 ? 256 : BL * 4 + 256);  // weight rows, token rows, scales
+  constexpr int kLds = W * (kStage > BL * kPitch * 4 ? kStage : BL * kPitch * 4);
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
+  float (*const part)[BL][kPitch] = reinterpret_cast<float (*)[BL][kPitch]>(lds);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hg = lane >> 5;
+
+  // ---- which tile: groups in order, inside a group the token tiles of one weight tile follow each other (they share
+  // the weights), every XCD a contiguous range
+  GroupRanges gr = {};
+  int total = (int)((p.Lrows + BL - 1) / BL);
+  if (p.goff != nullptr) {
+    gr = group_ranges<BL>(p.goff, p.E, 0, 0);
+    total = gr.total;
+    for (int base = 64; base < p.E; base += 64) total = group_ranges<BL>(p.goff, p.E, base, total).total;
+  }
+  const int64_t ntot = (int64_t)total * p.nRt, bid = blockIdx.x;
+  if (bid >= ntot) return;
+  const int64_t per = ntot / 8, rem = ntot % 8, xcd = bid % 8, idx = bid / 8;
+  const int64_t pid = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+  int g = 0, rt, lvalid;
+  int64_t l0;
+  if (p.goff != nullptr) {
+    g = p.E;
+    l0 = 0;
+    rt = lvalid = 0;
+    for (int base = 0; base < p.E; base += 64) {
+      if (base > 0) gr = group_ranges<BL>(p.goff, p.E, base, gr.total);
+      const unsigned long long hit = __ballot(pid >= (int64_t)gr.t_lo * p.nRt && pid < (int64_t)gr.t_hi * p.nRt);
+      if (hit != 0) {
+        const int src = __builtin_ctzll(hit);
+        const int t_lo = __builtin_amdgcn_readlane(gr.t_lo, src), nl = __builtin_amdgcn_readlane(gr.t_hi, src) - t_lo;
+        const int64_t r_lo = readlane_i64(gr.r_lo, src), r_hi = readlane_i64(gr.r_hi, src);
+        const uint32_t pe = (uint32_t)(pid - (int64_t)t_lo * p.nRt);
+        rt = (int)(pe / (uint32_t)nl);
+        l0 = r_lo + (int64_t)(pe - (uint32_t)rt * (uint32_t)nl) * BL;
+        lvalid = r_hi - l0 < BL ? (int)(r_hi - l0) : BL;
+        g = base + src;
+        break;
+      }
+    }
+    if (g >= p.E) return;
+  } else {
+    rt = (int)(pid / total);
+    l0 = (pid - (int64_t)rt * total) * BL;
+    lvalid = p.Lrows - l0 < BL ? (int)(p.Lrows - l0) : BL;
+  }
+  g = __builtin_amdgcn_readfirstlane(g);
+  rt = __builtin_amdgcn_readfirstlane(rt);
+  lvalid = __builtin_amdgcn_readfirstlane(lvalid);
+  l0 = uniform_i64(l0);
+  const int r0 = rt * BR;
+
+  // ---- operands: every wave stages its own blocks in its own part of the LDS, without barriers.
+  // One direct-to-LDS instruction moves 8 rows x 128 bytes, whole cache lines; the 16-byte chunks of a row are
+  // XOR-swizzled as in gemm.hip, so that fragment reads meet no bank twice.  (Loads straight into the matrix
+  // instruction's registers touch 32 lines each, four times over: with enough of them in flight to cover the latency
+  // the lines leave the 32 KB L1 in between and are fetched again.)  Token rows past the group's end are not
+  // loaded beyond the last slab of eight that holds one, re-read the last row inside it, and are not stored.
+  // One block in flight per wave and a dozen waves per CU: two or three blocks per wave measured no faster.
+  const int nkb = p.nkb;
+  uint8_t* const mine = lds + wave * kStage;
+  const uint8_t* const Lb = p.L + uniform_i64(l0 * p.ldl);
+  const uint8_t* const Rb = p.R + uniform_i64((int64_t)g * p.r_group_stride + (int64_t)r0 * p.ldr);
+  const int r8 = lane >> 3;
+  const uint32_t chunk[2] = {(uint32_t)(((lane & 7) ^ r8) << 4), (uint32_t)(((lane & 7) ^ r8 ^ 1) << 4)};
+  const uint32_t roff[2] = {(uint32_t)r8 * (uint32_t)p.ldr + chunk[0], (uint32_t)r8 * (uint32_t)p.ldr + chunk[1]};
+  uint32_t loff[4 * WTL];
+#pragma unroll
+  for (int n = 0; n < 4 * WTL; n++) {
+    const int row = n * 8 + r8 < lvalid ? n * 8 + r8 : lvalid - 1;
+    loff[n] = (uint32_t)row * (uint32_t)p.ldl + chunk[n & 1];
+  }
+  const int nl = (lvalid + 7) >> 3;  // slabs of token rows, >= 1
+  // scales of a block, [BL token rows][the weights' block]: with 32 token rows the upper lanes of the one load fetch
+  // the latter, else a load of its own does
+  const float* const rs = p.Rs + (int64_t)g * p.rs_group_stride + (int64_t)(r0 / kTile) * p.rs_row_stride;
+  const float* sbase[(WTL + 1) / 2];
+#pragma unroll
+  for (int n = 0; n < (WTL + 1) / 2; n++) {
+    const int row = n * 64 + lane < lvalid ? n * 64 + lane : lvalid - 1;
+    sbase[n] = WTL == 1 && lane >= 32 ? rs : p.Ls + (l0 + row) * p.ls_row_stride;
+  }
+  constexpr int kScales = (BR + BL) * kBK;  // offset in the stage
+  const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)mine;
+  auto load = [&](int k) __attribute__((always_inline)) {
+    const uint8_t* const R = Rb + (int64_t)k * kBK;
+    const uint8_t* const L = Lb + (int64_t)k * kBK;
+#pragma unroll
+    for (int n = 0; n < BR / 8; n++)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(roff[n & 1]), "s"(R + (int64_t)(n * 8) * p.ldr), "s"(base + n * 1024) : "memory");
+#pragma unroll
+    for (int n = 0; n < 4 * WTL; n++)
+      if (n < nl)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(loff[n]), "s"(L), "s"(base + BR * kBK + n * 1024) : "memory");
+#pragma unroll
+    for (int n = 0; n < (WTL + 1) / 2; n++)
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(sbase[n] + k), "s"(base + kScales + n * 256) : "memory");
+    if constexpr (WTL > 1)
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(rs + k), "s"(base + kScales + BL * 4) : "memory");
+  };
+  v16f acc[WTR][WTL], zero;
+#pragma unroll
+  for (int r = 0; r < 16; r++) zero[r] = 0.f;
+#pragma unroll
+  for (int i = 0; i < WTR; i++)
+#pragma unroll
+    for (int j = 0; j < WTL; j++) acc[i][j] = zero;
+  const int sw = (l32 & 7) ^ ((l32 >> 3) & 1);
+  if (wave < nkb) load(wave);
+  for (int kb = wave; kb < nkb; kb += W) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the block has landed
+    v8i rf[WTR][2], lf[WTL][2];
+    float sc[WTL];
+    auto frag = [&](const uint8_t* row, int h) {
+      const v4i lo = *reinterpret_cast<const v4i*>(row + (((4 * h + 2 * hg) ^ sw) << 4));
+      const v4i hi = *reinterpret_cast<const v4i*>(row + (((4 * h + 2 * hg + 1) ^ sw) << 4));
+      return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    const float* const S = reinterpret_cast<const float*>(mine + kScales);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+      for (int j = 0; j < WTL; j++) lf[j][h] = frag(mine + (BR + j * 32 + l32) * kBK, h);
+#pragma unroll
+      for (int i = 0; i < WTR; i++) rf[i][h] = frag(mine + (i * 32 + l32) * kBK, h);
+    }
+#pragma unroll
+    for (int j = 0; j < WTL; j++) sc[j] = S[j * 32 + l32] * S[BL];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and has been read: its place may be filled again
+    if (kb + W < nkb) load(kb + W);
+#pragma unroll
+    for (int i = 0; i < WTR; i++)
+#pragma unroll
+      for (int j = 0; j < WTL; j++) {
+        v16f pr = mfma_fp8_32x32x64(rf[i][0], lf[j][0], zero);
+        pr = mfma_fp8_32x32x64(rf[i][1], lf[j][1], pr);
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][j][r] = __builtin_fmaf(pr[r], sc[j], acc[i][j][r]);
+      }
+  }
+  __syncthreads();  // every wave is done with its stages: the memory holds the partial results now
+
+  // ---- sum over the waves, through the LDS; a lane holds column l32 and rows 8q + 4hg .. + 3 of every 32 x 32 sub-tile
+#pragma unroll
+  for (int i = 0; i < WTR; i++)
+#pragma unroll
+    for (int j = 0; j < WTL; j++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        *reinterpret_cast<v4f*>(&part[wave][j * 32 + l32][i * 32 + 8 * q + 4 * hg]) =
+            v4f{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  __syncthreads();
+  for (int c = tid; c < BL * (BR / 4); c += 64 * W) {
+    const int row = c / (BR / 4), col = (c % (BR / 4)) * 4;
+    if (row >= lvalid) break;  // (rows only grow with c)
+    v4f o = *reinterpret_cast<const v4f*>(&part[0][row][col]);
+#pragma unroll
+    for (int w = 1; w < W; w++) o += *reinterpret_cast<const v4f*>(&part[w][row][col]);
+    if (p.bias != nullptr) {
+      const int64_t at = (int64_t)g * p.bias_group_stride + r0 + col;
+      if (p.bias_dtype == AAMD_F32) {
+        o += *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(p.bias) + at);
+      } else {
+        const v2i raw = *reinterpret_cast<const v2i*>(reinterpret_cast<const u16*>(p.bias) + at);
+        o += v4f{bf16_bits_to_f32((uint32_t)raw[0] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[0] >> 16),
+                 bf16_bits_to_f32((uint32_t)raw[1] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[1] >> 16)};
+      }
+    }
+    OUT* const dst = reinterpret_cast<OUT*>(p.C) + (l0 + row) * p.ldc + r0 + col;
+    if constexpr (sizeof(OUT) == 4) {
+      *reinterpret_cast<v4f*>(dst) = o;
+    } else {
+      *reinterpret_cast<v2i*>(dst) = v2i{(int)pack_bf16x2(o[0], o[1]), (int)pack_bf16x2(o[2], o[3])};
+    }
+  }
+}
+
+// Upper bound of the token tiles of M rows in E groups (the groups' sizes are known on the device only).
+static int64_t few_rows_tiles(int64_t M, int E, int rows) {
+  const int64_t groups = M < E ? M : E;
+  return M / rows + groups < M ? M / rows + groups : M;
+}
+
+template <typename OUT, int W, int WTR, int WTL>
+static int launch_few(GemmParams p, int64_t M, hipStream_t st) {
+  p.nRt = (int)(p.Rrows / (32 * WTR));
+  const int64_t lt = p.goff ? few_rows_tiles(M, p.E, 32 * WTL) : (M + 32 * WTL - 1) / (32 * WTL);
+  const int64_t blocks = lt * p.nRt;
+  AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
+  few_rows_kernel<OUT, W, WTR, WTL><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p);
+  AAMD_LAUNCH_CHECK("grouped_gemm (few rows)");
+  return AAMD_OK;
+}
+
+// `split`: the form for launches of few workgroups, which divides the contraction among eight waves and takes half the
+// weight rows and token rows per workgroup.
+template <typename OUT>
+static int launch_few_as(const GemmParams& p, int64_t M, bool split, hipStream_t st) {
+  return split ? launch_few<OUT, 8, 1, 1>(p, M, st) : launch_few<OUT, 4, 2, 2>(p, M, st);
+}
+int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, hipStream_t st) {
+  return c_dtype == AAMD_BF16 ? launch_few_as<u16>(p, M, split, st) : launch_few_as<float>(p, M, split, st);
+}
+
+}  // namespace aamd
