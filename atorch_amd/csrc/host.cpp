@@ -15,6 +15,7 @@
 #include <tuple>
 
 #include "../../include/atorch_amd_fp8.h"
+#include "routing.hpp"
 
 namespace {
 
@@ -206,9 +207,10 @@ Routing route(const Tensor& ids, int64_t E, bool want_sorted) {
   if (want_sorted) r.sorted_idx = empty({n}, at::kLong, ids);
   r.row_map = empty({n}, at::kInt, ids);
   r.goff = empty({E + 1}, at::kLong, ids);
-  Tensor ws = empty({std::max<int64_t>(1, aamd_moe_preprocess_ws_ints(n, (int)E))}, at::kInt, ids);
+  // (the one-workgroup form needs no scratch)
+  Tensor ws = aamd_route_one_workgroup(n, E) ? Tensor() : empty({std::max<int64_t>(1, aamd_moe_preprocess_ws_ints(n, (int)E))}, at::kInt, ids);
   check(aamd_moe_preprocess(ptr(ids), ids.scalar_type() == at::kLong, n, (int)E, raw<int64_t>(r.sorted_idx), ptr<int32_t>(r.row_map),
-                            ptr<int64_t>(r.goff), ptr<int32_t>(ws), stream()));
+                            ptr<int64_t>(r.goff), raw<int32_t>(ws), stream()));
   return r;
 }
 std::tuple<OptTensor, Tensor, Tensor> moe_preprocess(const Tensor& ids, int64_t E, bool want_sorted) {
@@ -342,16 +344,17 @@ MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sort
   return {out, fc1, qx.q_t, qx.s_t, qh.q_t, qh.s_t};
 }
 
-// The same from the router's choices: (out, sorted_idx, row_map, goff, y, ...): routing, MLP, weighted combine.
-using LayerResult = std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
-LayerResult layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids, int64_t topk, const Tensor& q1, const Tensor& s1,
+// The same from the router's choices, routing and weighted combine included: (out, sorted_idx, row_map, goff) and, with
+// `train`, the experts' output and what mlp_forward returns for the backward.
+py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids, int64_t topk, const Tensor& q1, const Tensor& s1,
                           const Tensor& q2, const Tensor& s2, const OptTensor& b1, const OptTensor& b2, bool glu, bool train) {
   Routing r = route(ids, q1.size(0), true);
   MlpResult m = mlp_forward(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train);
   Tensor& y = std::get<0>(m);
   Tensor out = unpermute_combine(y, r.row_map, probs, x.size(0), topk);
-  return {out, r.sorted_idx, r.row_map, r.goff, train ? OptTensor(y) : OptTensor(),
-          std::get<1>(m), std::get<2>(m), std::get<3>(m), std::get<4>(m), std::get<5>(m)};
+  if (!train) return py::make_tuple(out, r.sorted_idx, r.row_map, r.goff);
+  return py::make_tuple(out, r.sorted_idx, r.row_map, r.goff, y, *std::get<1>(m), *std::get<2>(m), *std::get<3>(m),
+                        *std::get<4>(m), *std::get<5>(m));
 }
 
 // Gradients of the MLP: (dx, dw1, dw2).  With topk > 0 the rows were tokens permuted through row_map, and dx goes back
@@ -374,6 +377,29 @@ std::tuple<Tensor, Tensor, Tensor> mlp_backward(const Tensor& dy, const Tensor& 
   Tensor dw1 = transpose_w1 ? gemm_wgrad(qg.q_t, qg.s_t, qx_t, sx_t, goff, {}, w1_dtype, false)
                             : gemm_wgrad(qx_t, sx_t, qg.q_t, qg.s_t, goff, {}, w1_dtype, false);
   return {dx, dw1, dw2};
+}
+
+// ---- the grouped linear ----------------------------------------------------------------------
+// Forward on rows grouped by expert, from the groups' offsets or (goff empty) their sizes in a host list:
+// (out, goff, qx_t, sx_t), the last two only with `train`.
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> linear_forward(const Tensor& x, const OptTensor& goff_in,
+                                                                const std::vector<int64_t>& splits, const Tensor& qw, const Tensor& sw,
+                                                                const OptTensor& bias, at::ScalarType out_dtype, double eps,
+                                                                bool train) {
+  const int64_t E = qw.size(0);
+  Tensor goff = goff_in.has_value() ? *goff_in : offsets_from_list(splits, x.device());
+  Quantised q;
+  if (train) q = dual(x, goff, E, eps, padded_bound(x.size(0), E), true, true);
+  else std::tie(q.q, q.s) = tile_quant(x, eps);
+  return {gemm_nt(q.q, q.s, qw, sw, goff, {}, out_dtype, bias), goff, opt(q.q_t), opt(q.s_t)};
+}
+// Both gradients: (dx, dw); dw goes to `main_grad` (added or written over) where there is one.
+std::tuple<Tensor, Tensor> linear_backward(const Tensor& dy, const Tensor& goff, const Tensor& qx_t, const Tensor& sx_t,
+                                           const Tensor& qw_t, const Tensor& sw_t, at::ScalarType dx_dtype, const OptTensor& main_grad,
+                                           at::ScalarType dw_dtype, bool accumulate, double eps) {
+  Quantised q = dual(dy, goff, qw_t.size(0), eps, qt_ld(qx_t), true, true);
+  Tensor dx = gemm_nt(q.q, q.s, qw_t, sw_t, goff, {}, dx_dtype, {});
+  return {dx, gemm_wgrad(q.q_t, q.s_t, qx_t, sx_t, goff, main_grad, dw_dtype, accumulate)};
 }
 
 QuantTuple pack(const Quantised& r) { return {opt(r.q), opt(r.s), r.q_t, r.s_t}; }
@@ -409,6 +435,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("offsets_from_list", &offsets_from_list);
   m.def("offsets_from_tensor", &offsets_from_tensor);
   m.def("stack_of", &stack_of);
+  m.def("linear_forward", &linear_forward);
+  m.def("linear_backward", &linear_backward);
   m.def("mlp_forward", &mlp_forward);
   m.def("mlp_backward", &mlp_backward);
   m.def("layer_forward", &layer_forward);

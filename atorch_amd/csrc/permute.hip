@@ -1,6 +1,7 @@
 // Token routing kernels for gfx950: device-side router preprocess (histogram, scan, stable
 // counting sort), inverse permutation, and the fused unpermute + weighted combine.
 #include "common.hpp"
+#include "routing.hpp"
 
 // The combine reproduces "multiply, round, then sum": no fused multiply-add in this file.
 #pragma clang fp contract(off)
@@ -527,10 +528,6 @@ __global__ __launch_bounds__(256) void route_place_kernel(const ID* __restrict__
 // The same sort for fewer ids, with fewer launches (each of the four above is latency: 2 to 5 us whatever n is).
 // Up to 8192 ids: one workgroup does it all, ids and ranks in registers, counts of every (64 ids, expert) in LDS.
 // ---------------------------------------------------------------------------------------
-constexpr int kSmallRounds = 8;                         // rounds of 1024 ids
-constexpr int64_t kSmallMax = (int64_t)kSmallRounds * 1024;
-constexpr int64_t kSmallLds = 60 << 10;                 // bytes of counts
-
 // exclusive prefix of tot[0 .. E) into base[0 .. E), by one wave; returns the sum of all
 __device__ __forceinline__ int wave_exclusive_prefix(const int* tot, int* base, int E) {
   int carry = 0;
@@ -552,12 +549,12 @@ __global__ __launch_bounds__(1024) void route_small_kernel(const ID* __restrict_
   const int slots = (n + 63) >> 6, wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
   int* const tot = h + slots * E;
   for (int i = threadIdx.x; i < slots * E; i += 1024) h[i] = 0;
-  int eid[kSmallRounds], rank[kSmallRounds];
+  int eid[kRouteSmallRounds], rank[kRouteSmallRounds];
 #pragma unroll
-  for (int it = 0; it < kSmallRounds; it++) eid[it] = it * 1024 < n ? load_id(ids, it * 1024 + threadIdx.x, n, E) : -1;
+  for (int it = 0; it < kRouteSmallRounds; it++) eid[it] = it * 1024 < n ? load_id(ids, it * 1024 + threadIdx.x, n, E) : -1;
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < kSmallRounds; it++) {
+  for (int it = 0; it < kRouteSmallRounds; it++) {
     if (it * 1024 + wave * 64 >= n) break;
     const unsigned long long peers = same_expert(eid[it], E), below = peers & ((1ull << lane) - 1ull);
     rank[it] = __popcll(below);
@@ -586,7 +583,7 @@ __global__ __launch_bounds__(1024) void route_small_kernel(const ID* __restrict_
   }
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < kSmallRounds; it++) {
+  for (int it = 0; it < kRouteSmallRounds; it++) {
     const int flat = it * 1024 + (int)threadIdx.x;
     if (flat >= n) break;
     if (eid[it] < 0) {
@@ -1034,11 +1031,11 @@ extern "C" int aamd_moe_preprocess(const void* expert_ids, int ids_are_i64, int6
                                    int32_t* row_map, int64_t* group_offsets, int32_t* ws, void* stream) {
   AAMD_REQUIRE(n >= 0 && n < 0x7fffffffLL, "moe_preprocess: n out of range");
   AAMD_REQUIRE(E >= 1 && E <= 1024, "moe_preprocess: E=%d out of range [1, 1024]", E);
-  AAMD_REQUIRE(group_offsets && ws, "moe_preprocess: group_offsets / ws required");
+  AAMD_REQUIRE(group_offsets && (ws || aamd_route_one_workgroup(n, E)), "moe_preprocess: group_offsets / ws required");
   AAMD_REQUIRE(n == 0 || (expert_ids && row_map), "moe_preprocess: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  const int64_t small_lds = ((n + 63) / 64 + 1) * E * (int64_t)sizeof(int);
-  if (n <= kSmallMax && small_lds <= kSmallLds) {
+  if (aamd_route_one_workgroup(n, E)) {
+    const int64_t small_lds = aamd_route_small_lds(n, E);
     if (ids_are_i64)
       route_small_kernel<int64_t><<<1, 1024, (size_t)small_lds, st>>>((const int64_t*)expert_ids, (int)n, E, sorted_idx, row_map, group_offsets);
     else

@@ -71,6 +71,9 @@ def _weight_codes(w1, w2, v1, transpose_w1, is_first_microbatch, weight_cache):
     quant2 = lambda t: kernels.block_quant_batched(w2.detach().contiguous(), return_transpose=True)  # noqa: E731
     if weight_cache is None:
         return quant1(True), quant2(True)
+    held = weight_cache.held((("w1", (w1, v1)), ("w2", (w2,))), is_first_microbatch, True)
+    if held is not None:
+        return held
     return (weight_cache.codes("w1", (w1, v1), is_first_microbatch, True, quant1),
             weight_cache.codes("w2", (w2,), is_first_microbatch, True, quant2))  # fmt: skip
 
@@ -162,11 +165,12 @@ class _Fp8MoeLayer(torch.autograd.Function):
         q2, s2, q2_t, s2_t = codes2
         topk = dispatcher.topk
         probs_c = probs.contiguous()
-        out, sorted_idx, row_map, goff, y, fc1, qx_t, sx_t, qh_t, sh_t = host().layer_forward(
+        out, sorted_idx, row_map, goff, *saved = host().layer_forward(
             x.contiguous(), probs_c, top_experts.contiguous(), topk, q1, s1, q2_t, s2_t, _bias(b1), _bias(b2), glu, train
         )
         dispatcher.set_routing(sorted_idx, row_map, goff)
         if train:
+            y, fc1, qx_t, sx_t, qh_t, sh_t = saved
             ctx.transpose_w1, ctx.glu, ctx.has_v1 = transpose_w1, glu, v1 is not None
             ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
             ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)

@@ -159,16 +159,22 @@ class Grouped_GEMM_MoE(torch.nn.Module):
 
     def _forward_megatron(self, hidden_states, expert_weights, top_experts, se_fn1=None, se_fn2=None,
                           se_fn2_additional_input=None, is_first_microbatch=None):
-        expert_weights = expert_weights.view(-1, expert_weights.shape[-1])
-        top_experts = top_experts.view(-1, top_experts.shape[-1])
-        self.hidden_shape = hidden_states.shape
+        # (a call is a few dozen microseconds when decoding: nothing is reshaped that has its shape, and the attribute is
+        # set past Module.__setattr__)
+        if expert_weights.dim() != 2:
+            expert_weights = expert_weights.view(-1, expert_weights.shape[-1])
+        if top_experts.dim() != 2:
+            top_experts = top_experts.view(-1, top_experts.shape[-1])
+        shape = hidden_states.shape
+        self.__dict__["hidden_shape"] = shape
         d = self.token_dispatcher
-        x = hidden_states.reshape(-1, self.hidden_shape[-1])
+        x = hidden_states if len(shape) == 2 else hidden_states.reshape(-1, shape[-1])
         if x.shape[0] == 0:
             return hidden_states.clone()
-        d.hidden_shape, d.probs = self.hidden_shape, expert_weights
+        d.hidden_shape, d.probs = shape, expert_weights
         if se_fn1 is None and se_fn2 is None and not (self.training and self.output_dropout_prob > 0):
-            return self._forward_fused(x, expert_weights, top_experts, is_first_microbatch).view(self.hidden_shape)
+            out = self._forward_fused(x, expert_weights, top_experts, is_first_microbatch)
+            return out if len(shape) == 2 else out.view(shape)
         # dispatch: only the routing is computed here; the permute itself happens inside the first quantiser
         d.preprocess(top_experts)
 

@@ -19,6 +19,7 @@ Layout conventions of ``HipQuantizeOp`` results
       data ``[N, K]``, scale ``[N/128, K/128]``, data_t ``[K, N]``, scale_t ``[K/128, N/128]``.
 """
 import enum
+import operator
 import os
 from dataclasses import dataclass, field
 from typing import Any, List, Optional, Sequence, Tuple
@@ -74,6 +75,21 @@ class QuantizeResult:
     scale_t: Optional[torch.Tensor] = None
 
 
+class WeightCodeStack:
+    """Codes of all weights of a module, stacked (data, scale, data_t | None, scale_t | None), and the per-weight caches
+    that point into them.  ``whole`` while all of those still do."""
+
+    __slots__ = ("codes", "members", "whole")
+
+    def __init__(self, codes, caches):
+        self.codes, self.members, self.whole = codes, list(caches), True
+        for i, c in enumerate(self.members):
+            c.point_to(self, i)
+
+    def serves(self, caches) -> bool:
+        return self.whole and len(caches) == len(self.members) and all(map(operator.is_, caches, self.members))
+
+
 class QuantizeResultCache:
     """Per-weight cache of the fp8 copies between microbatches
     (quantized_grouped_linear.py:121-129, 467-470).
@@ -87,23 +103,26 @@ class QuantizeResultCache:
     def __init__(self, data: Optional[torch.Tensor] = None, scale: Optional[torch.Tensor] = None,
                  data_t: Optional[torch.Tensor] = None, scale_t: Optional[torch.Tensor] = None):
         self._own = [data, scale, data_t, scale_t]
-        self.stack = None
+        self.stack: Optional[WeightCodeStack] = None
         self.index = 0
 
-    def point_to(self, stack, index: int):
-        """Use entry ``index`` of ``stack`` = stacked (data, scale, data_t | None, scale_t | None)."""
+    def point_to(self, stack: "WeightCodeStack", index: int):
+        """Use entry ``index`` of ``stack``."""
+        if self.stack is not None:
+            self.stack.whole = False
         self._own = [None, None, None, None]
         self.stack = stack
         self.index = index
 
     def _get(self, k: int) -> Optional[torch.Tensor]:
-        if self._own[k] is None and self.stack is not None and self.stack[k] is not None:
-            self._own[k] = self.stack[k][self.index]
+        if self._own[k] is None and self.stack is not None and self.stack.codes[k] is not None:
+            self._own[k] = self.stack.codes[k][self.index]
         return self._own[k]
 
     def _set(self, k: int, value: Optional[torch.Tensor]):
         if self.stack is not None:
             self._own = [self._get(i) for i in range(4)]
+            self.stack.whole = False
             self.stack = None
         self._own[k] = value
 
@@ -146,6 +165,18 @@ class WeightCodeCache:
                 self._slots[name] = (stamp, codes)
             return codes
         return slot[1]
+
+    def held(self, wanted, is_first_microbatch: Optional[bool], need_transpose: bool):
+        """The codes of every ``(name, tensors)`` of ``wanted`` when all of them may be reused, else None."""
+        if is_first_microbatch or is_first_microbatch is None or force_quantize_per_microbatch():
+            return None
+        found = []
+        for name, tensors in wanted:
+            slot = self._slots.get(name)
+            if slot is None or slot[0] != self._stamp(tensors) or (need_transpose and slot[1][2] is None):
+                return None
+            found.append(slot[1])
+        return found
 
     def clear(self):
         self._slots.clear()
