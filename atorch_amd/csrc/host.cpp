@@ -357,26 +357,45 @@ py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids,
                         *std::get<4>(m), *std::get<5>(m));
 }
 
-// Gradients of the MLP: (dx, dw1, dw2).  With topk > 0 the rows were tokens permuted through row_map, and dx goes back
-// to token order as the sum over a token's copies.
-std::tuple<Tensor, Tensor, Tensor> mlp_backward(const Tensor& dy, const Tensor& goff, const OptTensor& row_map, int64_t topk,
-                                                const Tensor& fc1, const Tensor& qx_t, const Tensor& sx_t, const Tensor& qh_t,
-                                                const Tensor& sh_t, const Tensor& q1_t, const Tensor& s1_t, const Tensor& q2,
-                                                const Tensor& s2, bool glu, bool transpose_w1, at::ScalarType x_dtype,
-                                                at::ScalarType w1_dtype, at::ScalarType w2_dtype) {
+// Dual quantiser of a gradient with the sums of its columns per group, in `dtype`: a bias gradient on the side.
+std::tuple<Quantised, Tensor> dual_with_sums(int what, const Tensor& x, const Tensor& dh, const Tensor& goff, int64_t E,
+                                             int64_t ld_t, double eps, at::ScalarType dtype) {
+  const int64_t M = x.size(0), width = x.size(1);
+  Quantised r = alloc_dual(M, width, ld_t, true, true, x);
+  Tensor tiles = empty({ld_t / kTile, width}, at::kFloat, x), sums = empty({E, width}, dtype, x);
+  check(aamd_dual_grouped_with_sums(what, ptr(x), raw(dh), M, width, ptr<int64_t>(goff), (int)E, ptr<uint8_t>(r.q), ptr<float>(r.s),
+                                    ptr<uint8_t>(r.q_t), ptr<float>(r.s_t), ld_t, AAMD_QT_BLOCKED, (float)eps, ptr<float>(tiles), stream()));
+  check(aamd_group_sums(ptr<float>(tiles), width, ptr<int64_t>(goff), (int)E, ptr(sums), dtype_code(dtype), stream()));
+  return {r, sums};
+}
+
+// Gradients of the MLP: (dx, dw1, dw2, db1, db2), the last two where asked for.  With topk > 0 the rows were tokens
+// permuted through row_map, and dx goes back to token order as the sum over a token's copies.
+std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> mlp_backward(
+    const Tensor& dy, const Tensor& goff, const OptTensor& row_map, int64_t topk, const Tensor& fc1, const Tensor& qx_t,
+    const Tensor& sx_t, const Tensor& qh_t, const Tensor& sh_t, const Tensor& q1_t, const Tensor& s1_t, const Tensor& q2,
+    const Tensor& s2, bool glu, bool transpose_w1, bool want_b1, bool want_b2, at::ScalarType x_dtype, at::ScalarType w1_dtype,
+    at::ScalarType w2_dtype) {
   const int64_t E = goff.numel() - 1, ld_t = qt_ld(qx_t);
-  Quantised qdy = dual(dy, goff, E, 0.0, ld_t, true, true);
+  Quantised qdy, qg;
+  Tensor db1, db2;
+  if (want_b2) std::tie(qdy, db2) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, ld_t, 0.0, at::kBFloat16);
+  else qdy = dual(dy, goff, E, 0.0, ld_t, true, true);
   // through the second linear: dh = dy @ w2^T ([M, F]); dw2[f, h] = sum_m h[m, f] dy[m, h]
   Tensor dh = gemm_nt(qdy.q, qdy.s, q2, s2, goff, {}, at::kBFloat16, {});
   Tensor dw2 = gemm_wgrad(qh_t, sh_t, qdy.q_t, qdy.s_t, goff, {}, w2_dtype, false);
-  // through the activation, quantised by the kernel that computes it
-  Quantised qg = std::get<0>(act_dual(fc1, dh, glu, goff, E, ld_t, true, true, false));
+  // through the activation: the gradient of fc1 is quantised, and summed where there is a bias, by the kernel that
+  // computes it, and never written
+  if (want_b1)
+    std::tie(qg, db1) = dual_with_sums(glu ? AAMD_SUMS_SWIGLU_BWD : AAMD_SUMS_GELU_BWD, fc1, dh, goff, E, ld_t, 0.0, at::kBFloat16);
+  else
+    qg = std::get<0>(act_dual(fc1, dh, glu, goff, E, ld_t, true, true, false));
   // through the first linear: dx = dfc1 @ w1 ([M, H]); dw1[n, h] = sum_m dfc1[m, n] x[m, h]
   Tensor dx = gemm_nt(qg.q, qg.s, q1_t, s1_t, goff, {}, x_dtype, {});
   if (topk > 0) dx = unpermute_combine(dx, *row_map, {}, row_map->numel() / topk, topk);
   Tensor dw1 = transpose_w1 ? gemm_wgrad(qg.q_t, qg.s_t, qx_t, sx_t, goff, {}, w1_dtype, false)
                             : gemm_wgrad(qx_t, sx_t, qg.q_t, qg.s_t, goff, {}, w1_dtype, false);
-  return {dx, dw1, dw2};
+  return {dx, dw1, dw2, opt(db1), opt(db2)};
 }
 
 // ---- the grouped linear ----------------------------------------------------------------------
@@ -393,13 +412,19 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> linear_forward(const Tensor& x,
   else std::tie(q.q, q.s) = tile_quant(x, eps);
   return {gemm_nt(q.q, q.s, qw, sw, goff, {}, out_dtype, bias), goff, opt(q.q_t), opt(q.s_t)};
 }
-// Both gradients: (dx, dw); dw goes to `main_grad` (added or written over) where there is one.
-std::tuple<Tensor, Tensor> linear_backward(const Tensor& dy, const Tensor& goff, const Tensor& qx_t, const Tensor& sx_t,
-                                           const Tensor& qw_t, const Tensor& sw_t, at::ScalarType dx_dtype, const OptTensor& main_grad,
-                                           at::ScalarType dw_dtype, bool accumulate, double eps) {
-  Quantised q = dual(dy, goff, qw_t.size(0), eps, qt_ld(qx_t), true, true);
+// The gradients: (dx, dw, db); dw goes to `main_grad` (added or written over) where there is one; db [E, N] in fp32
+// where asked for (bf16 gradients only).
+std::tuple<Tensor, Tensor, OptTensor> linear_backward(const Tensor& dy, const Tensor& goff, const Tensor& qx_t, const Tensor& sx_t,
+                                                      const Tensor& qw_t, const Tensor& sw_t, at::ScalarType dx_dtype,
+                                                      const OptTensor& main_grad, at::ScalarType dw_dtype, bool accumulate,
+                                                      double eps, bool want_bias) {
+  const int64_t E = qw_t.size(0);
+  Quantised q;
+  Tensor db;
+  if (want_bias) std::tie(q, db) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, qt_ld(qx_t), eps, at::kFloat);
+  else q = dual(dy, goff, E, eps, qt_ld(qx_t), true, true);
   Tensor dx = gemm_nt(q.q, q.s, qw_t, sw_t, goff, {}, dx_dtype, {});
-  return {dx, gemm_wgrad(q.q_t, q.s_t, qx_t, sx_t, goff, main_grad, dw_dtype, accumulate)};
+  return {dx, gemm_wgrad(q.q_t, q.s_t, qx_t, sx_t, goff, main_grad, dw_dtype, accumulate), opt(db)};
 }
 
 QuantTuple pack(const Quantised& r) { return {opt(r.q), opt(r.s), r.q_t, r.s_t}; }
@@ -421,6 +446,11 @@ PYBIND11_MODULE(_host, m) {
                        bool blocked, bool keep) {
     auto [r, kept] = act_dual(fc1, dh.has_value() ? *dh : Tensor(), glu, goff, E, ld_t, rowwise, blocked, keep);
     return std::make_tuple(opt(r.q), opt(r.s), r.q_t, r.s_t, opt(kept));
+  });
+  m.def("dual_with_sums", [](int what, const Tensor& x, const OptTensor& dh, const Tensor& goff, int64_t E, int64_t ld_t, double eps,
+                             at::ScalarType dtype) {
+    auto [r, sums] = dual_with_sums(what, x, dh.has_value() ? *dh : Tensor(), goff, E, ld_t, eps, dtype);
+    return std::make_tuple(r.q, r.s, r.q_t, r.s_t, sums);
   });
   m.def("block_quant", &block_quant);
   m.def("gemm_nt", &gemm_nt);

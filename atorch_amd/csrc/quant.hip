@@ -5,6 +5,9 @@
 // All of them stream HBM with 128-bit accesses; amax reductions over a 128-element tile run
 // inside one 16-lane DPP row.  Scales and codes are part of a bit-exact contract, so every
 // quotient gives the code of the correctly rounded one (the IEEE division or its checked two-instruction form).
+#include <atomic>
+#include <mutex>
+
 #include "common.hpp"
 
 namespace aamd {
@@ -145,8 +148,8 @@ __device__ __forceinline__ float gelu_phi(float x, float* exp_neg_half_sq = null
 // two dozen vector instructions per value, which is what bounds the fused kernels.  The dual kernels therefore read
 // them from tables in LDS indexed by the bits of x, for |x| in [2^-14, 2^3) (17 binades x 128 x 2 signs); values
 // outside (exact zeros, outliers) take the arithmetic.  The tables are filled by the same functions, by a small
-// kernel ahead of every launch, into arrays of the library on the device: every call writes the same values, so
-// calls that overlap do not disturb each other.
+// kernel ahead of the launch, into arrays of the library on the device, until the host has seen that a fill has
+// completed (fill_table): every call writes the same values, so calls that overlap do not disturb each other.
 constexpr uint32_t kLutLo = (uint32_t)(127 - 14) << 7;        // first magnitude (bits without the sign) of the tables
 constexpr uint32_t kLutN = (uint32_t)(14 + 3) << 7;           // magnitudes per sign
 static __device__ __attribute__((aligned(16))) u16 g_gelu_lut[2 * kLutN];
@@ -467,12 +470,14 @@ __device__ __forceinline__ uint8_t* qt_tile(uint8_t* q_t, int blocked, int64_t c
 // (the launchers bound the row strides so that 128 rows stay below 2^32 bytes).
 // GATHER: row r of the tile is source row src_row[r] of x (the token permute fused in: x is in token order,
 // the outputs in expert-contiguous order); src_row lives in LDS and holds every valid row of the tile.
-template <typename IN, bool FULL, bool GATHER = false>
+// SUMS: the tile's column sums (a bias gradient's share of these 128 tokens) go to tile_sums[pt, column].
+template <typename IN, bool FULL, bool GATHER = false, bool SUMS = false>
 __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ x, uint32_t ldx, int nt, int64_t m0,
                                           int mvalid, int pt, int kc, uint8_t* __restrict__ q, float* __restrict__ s,
                                           uint8_t* __restrict__ q_t, float* __restrict__ s_t, uint32_t ld_t, int blocked,
                                           float eps, int64_t gate_off, u16* __restrict__ h_out, uint8_t* tile_t,
-                                          Divider* cdiv, const uint32_t* src_row = nullptr, const void* lut = nullptr) {
+                                          Divider* cdiv, const uint32_t* src_row = nullptr, const void* lut = nullptr,
+                                          float* __restrict__ tile_sums = nullptr) {
   const bool plain_div = !kBf16Values<IN> || eps != 0.f;  // see make_scale
   float (*part)[kTile] = reinterpret_cast<float (*)[kTile]>(tile_t);
   const int64_t cols = (int64_t)nt * kTile;
@@ -559,6 +564,26 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
     (s_t + (int64_t)pt * cols + (int64_t)kc * kTile)[(int)threadIdx.x] = dv.s;
   }
   __syncthreads();
+  if constexpr (SUMS) {  // in the region of the maxima, which have been read
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        if constexpr (kPacked) sum += __uint_as_float(j & 1 ? vp[i][j / 2] & 0xffff0000u : vp[i][j / 2] << 16);
+        else sum += v[i][j];
+      }
+      part[gr][c * 8 + j] = sum;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < kTile) {
+      float sum = part[0][(int)threadIdx.x];
+#pragma unroll
+      for (int i = 1; i < 16; i++) sum += part[i][(int)threadIdx.x];
+      tile_sums[(int64_t)pt * cols + (int64_t)kc * kTile + (int)threadIdx.x] = sum;
+    }
+    __syncthreads();
+  }
   // codes of the 8x8 register block, transposed through LDS, written as rows of 128 bytes
 #pragma unroll
   for (int j = 0; j < 8; j++) {
@@ -575,12 +600,12 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
   store_staged_tile(tile_t, out_t, ld_out);
 }
 
-template <typename IN>
+template <typename IN, bool SUMS = false>
 __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ goff,
     int E, int64_t M, uint8_t* __restrict__ q, float* __restrict__ s,
     uint8_t* __restrict__ q_t, float* __restrict__ s_t, int64_t ld_t, int blocked, float eps, int64_t gate_off,
-    u16* __restrict__ h_out) {
+    u16* __restrict__ h_out, float* __restrict__ tile_sums = nullptr) {
   // the per-row-group column maxima are dead before the transposed codes are staged: one region
   __shared__ __attribute__((aligned(16))) uint8_t tile_t[kTile * kTLd];
   static_assert(sizeof(float) * 16 * kTile <= sizeof(tile_t), "the column maxima fit in the staging region");
@@ -614,9 +639,9 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
   const int mvalid = left < kTile ? (int)left : kTile;
   if constexpr (kLutBytes<IN> != 0) __syncthreads();  // the copy of the table
   if (mvalid == kTile)
-    dual_tile<IN, true>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, gate_off, h_out, tile_t, cdiv, nullptr, lut_s);
+    dual_tile<IN, true, false, SUMS>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, gate_off, h_out, tile_t, cdiv, nullptr, lut_s, tile_sums);
   else
-    dual_tile<IN, false>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, gate_off, h_out, tile_t, cdiv, nullptr, lut_s);
+    dual_tile<IN, false, false, SUMS>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, gate_off, h_out, tile_t, cdiv, nullptr, lut_s, tile_sums);
 }
 
 // The dual quantiser with the token permute fused in: x holds the tokens in their original order, and permuted
@@ -670,8 +695,8 @@ __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
 // and dh and one sigmoid per position.
 // Thread (gr = tid / 16, c = tid % 16) holds rows gr*4 .. gr*4+3, columns c*8 .. c*8+7 of both tiles.
 // ---------------------------------------------------------------------------------------
-// sigmoid(a) in fp32 per bf16 value a, for |a| in [2^-14, 2^4), read from LDS like the GELU tables (filled ahead of
-// every launch by the kernel's own sigmoid; inside the table range a sigmoid(a) equals the scaled form's silu bit
+// sigmoid(a) in fp32 per bf16 value a, for |a| in [2^-14, 2^4), read from LDS like the GELU tables (filled
+// by the kernel's own sigmoid; inside the table range a sigmoid(a) equals the scaled form's silu bit
 // for bit: neither product leaves the normal range there)
 constexpr uint32_t kSigLo = (uint32_t)(127 - 14) << 7;
 constexpr uint32_t kSigN = (uint32_t)(14 + 4) << 7;
@@ -697,14 +722,14 @@ __device__ __forceinline__ int quant4(const float* v, const Divider& d) {
   return pack2_fp8<true>(t[2], t[3], pack2_fp8<false>(t[0], t[1], 0));
 }
 
-template <bool FULL>
+template <bool FULL, bool SUMS>
 __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa /* a at the tile's origin */, uint32_t ld,
                                                      int64_t gate_off, const u16* __restrict__ xd, uint32_t ld_dh, int nt,
                                                      int64_t m0, int mvalid, int pt, int f, uint8_t* __restrict__ q,
                                                      float* __restrict__ s, uint8_t* __restrict__ q_t,
                                                      float* __restrict__ s_t, uint32_t ld_t, int blocked,
                                                      u16* __restrict__ g_out, uint8_t (*tile_t)[kTile * kTLd],
-                                                     Divider (*cdiv)[kTile], const float* sig_lut) {
+                                                     Divider (*cdiv)[kTile], const float* sig_lut, float* __restrict__ tile_sums) {
   const int tid = threadIdx.x, gr = tid >> 4, c = tid & 15;
   const int half = nt / 2;
   const int64_t cols = (int64_t)nt * kTile;
@@ -823,6 +848,26 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
     (s_t + (int64_t)pt * cols + (int64_t)(w == 0 ? f : half + f) * kTile)[col] = dv.s;
   }
   __syncthreads();
+  if constexpr (SUMS) {  // column sums of both tiles, in the region of the maxima, which have been read
+#pragma unroll
+    for (int w = 0; w < 2; w++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum += __uint_as_float(j & 1 ? vp[w][i][j / 2] & 0xffff0000u : vp[w][i][j / 2] << 16);
+        part[w][gr][c * 8 + j] = sum;
+      }
+    __syncthreads();
+    if (tid < 2 * kTile) {
+      const int w = tid >> 7, col = tid & (kTile - 1);
+      float sum = part[w][0][col];
+#pragma unroll
+      for (int i = 1; i < 32; i++) sum += part[w][i][col];
+      tile_sums[(int64_t)pt * cols + (int64_t)(w == 0 ? f : half + f) * kTile + col] = sum;
+    }
+    __syncthreads();
+  }
   // ---- transposed codes through the LDS
 #pragma unroll
   for (int w = 0; w < 2; w++)
@@ -848,13 +893,15 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
   }
 }
 
+template <bool SUMS>
 __global__ __launch_bounds__(512, 4) void swiglu_bwd_dual_kernel(const u16* __restrict__ fc1, int64_t ld, int64_t gate_off,
                                                               const u16* __restrict__ dh, int64_t ld_dh, int nt,
                                                               const int64_t* __restrict__ goff,
                                                               int E, int64_t M,
                                                               uint8_t* __restrict__ q, float* __restrict__ s,
                                                               uint8_t* __restrict__ q_t, float* __restrict__ s_t,
-                                                              int64_t ld_t, int blocked, u16* __restrict__ g_out) {
+                                                              int64_t ld_t, int blocked, u16* __restrict__ g_out,
+                                                              float* __restrict__ tile_sums) {
   __shared__ __attribute__((aligned(16))) uint8_t tile_ts[2][kTile * kTLd];
   __shared__ Divider cdivs[2][kTile];
   __shared__ __attribute__((aligned(16))) float sig_s[2 * kSigN];
@@ -882,11 +929,11 @@ __global__ __launch_bounds__(512, 4) void swiglu_bwd_dual_kernel(const u16* __re
   const u16* const xd = dh + m0 * ld_dh + (int64_t)f * kTile;
   __syncthreads();  // the copy of the table
   if (mvalid == kTile)
-    swiglu_bwd_dual_tile<true>(xa, (uint32_t)ld, gate_off, xd, (uint32_t)ld_dh, nt, m0, mvalid, pt, f, q, s, q_t, s_t,
-                               (uint32_t)ld_t, blocked, g_out, tile_ts, cdivs, sig_s);
+    swiglu_bwd_dual_tile<true, SUMS>(xa, (uint32_t)ld, gate_off, xd, (uint32_t)ld_dh, nt, m0, mvalid, pt, f, q, s, q_t, s_t,
+                               (uint32_t)ld_t, blocked, g_out, tile_ts, cdivs, sig_s, tile_sums);
   else
-    swiglu_bwd_dual_tile<false>(xa, (uint32_t)ld, gate_off, xd, (uint32_t)ld_dh, nt, m0, mvalid, pt, f, q, s, q_t, s_t,
-                                (uint32_t)ld_t, blocked, g_out, tile_ts, cdivs, sig_s);
+    swiglu_bwd_dual_tile<false, SUMS>(xa, (uint32_t)ld, gate_off, xd, (uint32_t)ld_dh, nt, m0, mvalid, pt, f, q, s, q_t, s_t,
+                                (uint32_t)ld_t, blocked, g_out, tile_ts, cdivs, sig_s, tile_sums);
 }
 
 // The 8x8 byte matrix held as eight rows of two dwords, transposed with byte permutes: cols[j]
@@ -956,6 +1003,30 @@ __global__ __launch_bounds__(256) void quant_128x128_kernel(const typename IN::e
   }
 }
 
+// out[g, c] = the sum of tile_sums[t, c] over the token tiles t of group g: what is left of a bias gradient after the
+// quantisers have summed their tiles.  A thread per column, its loads independent of each other.
+template <typename OUT>
+__global__ __launch_bounds__(256) void group_sums_kernel(const float* __restrict__ tile_sums, int64_t cols,
+                                                         const int64_t* __restrict__ goff, int E, OUT* __restrict__ out) {
+  const int g = (int)blockIdx.y;
+  int t_lo = 0, t_hi = 0, carry = 0;
+  for (int base = 0; base <= g; base += 64) {
+    const GroupRanges r = group_ranges<kTile>(goff, E, base, carry);
+    if (g - base < 64) {
+      t_lo = __builtin_amdgcn_readlane(r.t_lo, g - base);
+      t_hi = __builtin_amdgcn_readlane(r.t_hi, g - base);
+    }
+    carry = r.total;
+  }
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= cols) return;
+  float sum = 0.f;
+#pragma unroll 8
+  for (int t = t_lo; t < t_hi; t++) sum += tile_sums[(int64_t)t * cols + c];
+  if constexpr (sizeof(OUT) == 4) out[(int64_t)g * cols + c] = sum;
+  else out[(int64_t)g * cols + c] = (OUT)f32_to_bf16_bits(sum);
+}
+
 template <typename OUT>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ q, const float* __restrict__ s,
                                                       int64_t M, int64_t N, int tile_scale,
@@ -996,6 +1067,45 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Makes sure that a table of constants on the current device is filled before what follows on the stream.  Until the
+// host sees the flag that a kernel behind a completed fill has set, every call fills the table again on its own stream,
+// so no call waits for another; after that a call launches nothing (a fill took 4.5 us of the stream's time ahead of
+// every launch).  A call under graph capture that finds no flag records the fill and leaves the flag alone: what is
+// captured has not run.
+__global__ void set_flag_kernel(int32_t* flag) { __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
+struct TableState {
+  std::atomic<int32_t*> flag[64];  // per device, in pinned host memory, kept until the process ends
+  std::mutex lock;
+};
+static int fill_table(TableState& state, void (*kernel)(), unsigned entries, hipStream_t st) {
+  int dev = -1;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+  const bool tracked = dev >= 0 && dev < 64;
+  int32_t* flag = tracked ? state.flag[dev].load(std::memory_order_acquire) : nullptr;
+  if (flag != nullptr && __atomic_load_n(flag, __ATOMIC_ACQUIRE) != 0) return AAMD_OK;
+  kernel<<<dim3((entries + 255) / 256), dim3(256), 0, st>>>();
+  AAMD_LAUNCH_CHECK("table of constants");
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (!tracked || hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return AAMD_OK;
+  if (flag == nullptr) {
+    std::lock_guard<std::mutex> guard(state.lock);
+    flag = state.flag[dev].load(std::memory_order_acquire);
+    if (flag == nullptr) {
+      if (hipHostMalloc(reinterpret_cast<void**>(&flag), sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();  // (another thread captures, or no pinned memory: the next call fills again)
+        return AAMD_OK;
+      }
+      *flag = 0;
+      state.flag[dev].store(flag, std::memory_order_release);
+    }
+  }
+  set_flag_kernel<<<1, 1, 0, st>>>(flag);
+  AAMD_LAUNCH_CHECK("table of constants (flag)");
+  return AAMD_OK;
+}
+static TableState g_gelu_tables, g_sigmoid_table;
 
 }  // namespace aamd
 
@@ -1046,10 +1156,9 @@ extern "C" int aamd_permute_quant_1x128(const void* x, int x_dtype, int64_t T, i
   return AAMD_OK;
 }
 
-extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t M, int64_t cols, int64_t ldx,
-                                             const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, uint8_t* q,
-                                             float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
-                                             float eps, void* stream) {
+static int quant_dual(const void* x, int x_dtype, int64_t M, int64_t cols, int64_t ldx, const int64_t* group_offsets, int E,
+                      uint8_t* q, float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout, float eps,
+                      float* tile_sums, void* stream) {
   AAMD_REQUIRE(x_dtype == AAMD_BF16 || x_dtype == AAMD_F32 || x_dtype == AAMD_F16, "quant_dual: unsupported dtype %d", x_dtype);
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && cols >= 0 && cols % kTile == 0, "quant_dual: cols=%lld must be a multiple of 128",
@@ -1072,7 +1181,9 @@ extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(cols / kTile), (unsigned)grid_tiles), block(256);
   const int nt = (int)(cols / kTile);
-  if (x_dtype == AAMD_BF16)
+  if (tile_sums)
+    quant_dual_grouped_kernel<BF16, true><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr, tile_sums);
+  else if (x_dtype == AAMD_BF16)
     quant_dual_grouped_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
   else if (x_dtype == AAMD_F16)
     quant_dual_grouped_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps, 0, nullptr);
@@ -1193,10 +1304,9 @@ extern "C" int aamd_gelu_quant_1x128(const void* x, int64_t rows, int64_t F, int
 }
 
 // dh == nullptr: forward (h = gelu(x)); else backward (g = dh * gelu'(x)), dh dense with the row stride of x
-extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh, int64_t M, int64_t F, int64_t ld,
-                                                  const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, void* h_out,
-                                                  uint8_t* q, float* s, uint8_t* q_t, float* s_t, int64_t ld_t,
-                                                  int q_t_layout, void* stream) {
+static int gelu_dual(const void* x, const void* dh, int64_t M, int64_t F, int64_t ld, const int64_t* group_offsets, int E,
+                     void* h_out, uint8_t* q, float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
+                     float* tile_sums, void* stream) {
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "gelu_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && F >= 0 && F % kTile == 0, "gelu_quant_dual: F=%lld must be a multiple of 128", (long long)F);
   AAMD_REQUIRE(ld >= F && ld % 8 == 0 && ld < kMaxTileLd && ld_t < kMaxTileLd, "gelu_quant_dual: bad ld=%lld", (long long)ld);
@@ -1214,24 +1324,27 @@ extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh,
   AAMD_REQUIRE(grid_tiles <= 65535, "gelu_quant_dual: more than 65535 token tiles");
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(F / kTile), (unsigned)grid_tiles), block(256);
-  gelu_lut_kernel<<<dim3((2 * kLutN + 255) / 256), dim3(256), 0, st>>>();
+  const int rc = fill_table(g_gelu_tables, gelu_lut_kernel, 2 * kLutN, st);
+  if (rc) return rc;
   if (dh == nullptr) {
     quant_dual_grouped_kernel<GELU><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, M, q, s,
                                                             q_t, s_t, ld_t, q_t_layout, 0.f, 0, (u16*)h_out);
   } else {
     const int64_t dh_off = (const u16*)dh - (const u16*)x;  // elements; the loader reads dh at x + dh_off
-    quant_dual_grouped_kernel<GELUB><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, M, q, s,
-                                                             q_t, s_t, ld_t, q_t_layout, 0.f, dh_off, (u16*)h_out);
+    if (tile_sums)
+      quant_dual_grouped_kernel<GELUB, true><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, M, q, s,
+                                                                     q_t, s_t, ld_t, q_t_layout, 0.f, dh_off, (u16*)h_out, tile_sums);
+    else
+      quant_dual_grouped_kernel<GELUB><<<grid, block, 0, st>>>((const u16*)x, ld, (int)(F / kTile), group_offsets, E, M, q, s,
+                                                               q_t, s_t, ld_t, q_t_layout, 0.f, dh_off, (u16*)h_out);
   }
   AAMD_LAUNCH_CHECK("gelu_quant_dual_grouped");
   return AAMD_OK;
 }
 
-extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t ld_dh, const void* fc1, int64_t ld,
-                                                        int64_t M, int64_t F, const int64_t* group_offsets, int E,
-                                                        int32_t* /*tile_ws*/, void* g_out, uint8_t* q, float* s,
-                                                        uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
-                                                        void* stream) {
+static int swiglu_bwd_dual(const void* dh, int64_t ld_dh, const void* fc1, int64_t ld, int64_t M, int64_t F,
+                           const int64_t* group_offsets, int E, void* g_out, uint8_t* q, float* s, uint8_t* q_t, float* s_t,
+                           int64_t ld_t, int q_t_layout, float* tile_sums, void* stream) {
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "swiglu_bwd_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && F >= 0 && F % kTile == 0, "swiglu_bwd_quant_dual: F=%lld must be a multiple of 128", (long long)F);
   AAMD_REQUIRE(ld >= 2 * F && ld % 8 == 0 && ld_dh >= F && ld_dh % 8 == 0 && ld < kMaxTileLd && ld_dh < kMaxTileLd && ld_t < kMaxTileLd,
@@ -1252,10 +1365,65 @@ extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t 
   hipStream_t st = (hipStream_t)stream;
   const int nt = (int)(2 * F / kTile);
   dim3 grid((unsigned)(nt / 2), (unsigned)grid_tiles), block(512);  // two teams: the da and the db tile of a feature tile
-  sigmoid_lut_kernel<<<dim3((2 * kSigN + 255) / 256), dim3(256), 0, st>>>();
-  swiglu_bwd_dual_kernel<<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, E, M,
-                                                 q, s, q_t, s_t, ld_t, q_t_layout, (u16*)g_out);
+  const int rc = fill_table(g_sigmoid_table, sigmoid_lut_kernel, 2 * kSigN, st);
+  if (rc) return rc;
+  if (tile_sums)
+    swiglu_bwd_dual_kernel<true><<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, E, M,
+                                                         q, s, q_t, s_t, ld_t, q_t_layout, (u16*)g_out, tile_sums);
+  else
+    swiglu_bwd_dual_kernel<false><<<grid, block, 0, st>>>((const u16*)fc1, ld, F, (const u16*)dh, ld_dh, nt, group_offsets, E, M,
+                                                          q, s, q_t, s_t, ld_t, q_t_layout, (u16*)g_out, nullptr);
   AAMD_LAUNCH_CHECK("swiglu_bwd_quant_dual_grouped");
+  return AAMD_OK;
+}
+
+// ---- the entry points of the three: without and with the column sums of the tiles
+extern "C" int aamd_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t M, int64_t cols, int64_t ldx,
+                                             const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, uint8_t* q,
+                                             float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
+                                             float eps, void* stream) {
+  return quant_dual(x, x_dtype, M, cols, ldx, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, nullptr, stream);
+}
+extern "C" int aamd_gelu_quant_1x128_dual_grouped(const void* x, const void* dh, int64_t M, int64_t F, int64_t ld,
+                                                  const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, void* h_out,
+                                                  uint8_t* q, float* s, uint8_t* q_t, float* s_t, int64_t ld_t,
+                                                  int q_t_layout, void* stream) {
+  return gelu_dual(x, dh, M, F, ld, group_offsets, E, h_out, q, s, q_t, s_t, ld_t, q_t_layout, nullptr, stream);
+}
+extern "C" int aamd_swiglu_bwd_quant_1x128_dual_grouped(const void* dh, int64_t ld_dh, const void* fc1, int64_t ld,
+                                                        int64_t M, int64_t F, const int64_t* group_offsets, int E,
+                                                        int32_t* /*tile_ws*/, void* g_out, uint8_t* q, float* s,
+                                                        uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
+                                                        void* stream) {
+  return swiglu_bwd_dual(dh, ld_dh, fc1, ld, M, F, group_offsets, E, g_out, q, s, q_t, s_t, ld_t, q_t_layout, nullptr, stream);
+}
+extern "C" int aamd_dual_grouped_with_sums(int what, const void* x, const void* dh, int64_t M, int64_t width,
+                                           const int64_t* group_offsets, int E, uint8_t* q, float* s, uint8_t* q_t,
+                                           float* s_t, int64_t ld_t, int q_t_layout, float eps, float* tile_sums,
+                                           void* stream) {
+  AAMD_REQUIRE(tile_sums != nullptr, "dual_grouped_with_sums: null sums");
+  AAMD_REQUIRE(what == AAMD_SUMS_PLAIN || dh != nullptr, "dual_grouped_with_sums: null gradient");
+  if (what == AAMD_SUMS_PLAIN)
+    return quant_dual(x, AAMD_BF16, M, width, width, group_offsets, E, q, s, q_t, s_t, ld_t, q_t_layout, eps, tile_sums, stream);
+  AAMD_REQUIRE(eps == 0.f, "dual_grouped_with_sums: eps must be 0 here");
+  if (what == AAMD_SUMS_GELU_BWD)
+    return gelu_dual(x, dh, M, width, width, group_offsets, E, nullptr, q, s, q_t, s_t, ld_t, q_t_layout, tile_sums, stream);
+  AAMD_REQUIRE(what == AAMD_SUMS_SWIGLU_BWD && width % 2 == 0, "dual_grouped_with_sums: unknown form %d", what);
+  return swiglu_bwd_dual(dh, width / 2, x, width, M, width / 2, group_offsets, E, nullptr, q, s, q_t, s_t, ld_t, q_t_layout,
+                         tile_sums, stream);
+}
+extern "C" int aamd_group_sums(const float* tile_sums, int64_t cols, const int64_t* group_offsets, int E, void* out,
+                               int out_dtype, void* stream) {
+  AAMD_REQUIRE(out_dtype == AAMD_BF16 || out_dtype == AAMD_F32, "group_sums: unsupported dtype %d", out_dtype);
+  AAMD_REQUIRE(cols >= 0 && E >= 1 && E <= 65535 && group_offsets, "group_sums: bad sizes");
+  if (cols == 0) return AAMD_OK;
+  AAMD_REQUIRE(tile_sums && out, "group_sums: null pointer");
+  dim3 grid((unsigned)((cols + 255) / 256), (unsigned)E);
+  if (out_dtype == AAMD_F32)
+    group_sums_kernel<float><<<grid, 256, 0, (hipStream_t)stream>>>(tile_sums, cols, group_offsets, E, (float*)out);
+  else
+    group_sums_kernel<u16><<<grid, 256, 0, (hipStream_t)stream>>>(tile_sums, cols, group_offsets, E, (u16*)out);
+  AAMD_LAUNCH_CHECK("group_sums");
   return AAMD_OK;
 }
 

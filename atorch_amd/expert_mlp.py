@@ -32,7 +32,6 @@ import torch
 
 from . import kernels
 from ._lib import host
-from .bias_gather_add import bias_gather_add_bw
 from .gmm import _offsets
 from .quantization import WeightCodeCache
 
@@ -86,36 +85,10 @@ def _mlp_backward(ctx, dy, goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2
     """``(dx, dw1, dw2, dv1, db1, db2)`` from the gradient of the MLP's output rows."""
     x_dtype, w1_dtype, w2_dtype = ctx.dtypes
     dy = dy.contiguous().to(torch.bfloat16)
-    db1 = db2 = None
-    if not (ctx.has_b1 or ctx.has_b2):
-        dx, dw1, dw2 = host().mlp_backward(dy, goff, row_map, ctx.dispatch_topk, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t,
-                                           q2, s2, ctx.glu, ctx.transpose_w1, x_dtype, w1_dtype, w2_dtype)  # fmt: skip
-    else:
-        E = goff.numel() - 1
-        ld_t = kernels.qt_ld(qx_t)
-        # expert of every row, from the device-side offsets (no host round trip)
-        bin_ids = torch.repeat_interleave(torch.arange(E, device=dy.device), goff[1:] - goff[:-1], output_size=dy.shape[0])
-        db2 = bias_gather_add_bw(dy, bin_ids, E) if ctx.has_b2 else None
-        qdy, sdy, qdy_t, sdy_t = kernels.tile_quant_dual_grouped(dy, goff, E, ld_t=ld_t, blocked=True)
-        # through the second linear: dh = dy @ w2^T ([M, F]); dw2[f, h] = sum_m h[m, f] dy[m, h]
-        dh = kernels.grouped_gemm_nt(qdy, sdy, q2, s2, goff, out_dtype=torch.bfloat16)
-        dw2 = kernels.grouped_gemm_wgrad(qh_t, sh_t, qdy_t, sdy_t, goff, out_dtype=w2_dtype)
-        # through the activation: the gradient of fc1 is quantised by the kernel that computes it and is
-        # written in bf16 only when a bias gradient needs its row sums
-        if ctx.glu:
-            res = kernels.swiglu_bwd_tile_quant_dual_grouped(dh, fc1, goff, E, ld_t=ld_t, blocked=True, return_grad=ctx.has_b1)
-        else:
-            res = kernels.gelu_tile_quant_dual_grouped(fc1, goff, E, dh=dh, ld_t=ld_t, blocked=True, return_activation=ctx.has_b1)
-        qg, sg, qg_t, sg_t = res[:4]
-        db1 = bias_gather_add_bw(res[4], bin_ids, E) if ctx.has_b1 else None
-        # through the first linear: dx = dfc1 @ w1 ([M, H]); dw1[n, h] = sum_m dfc1[m, n] x[m, h]
-        dx = kernels.grouped_gemm_nt(qg, sg, q1_t, s1_t, goff, out_dtype=x_dtype)
-        if ctx.dispatch_topk:  # back to token order: the sum over a token's copies (index_select's backward)
-            dx = kernels.unpermute_combine(dx, row_map, None, ctx.num_tokens, ctx.dispatch_topk)
-        if ctx.transpose_w1:
-            dw1 = kernels.grouped_gemm_wgrad(qg_t, sg_t, qx_t, sx_t, goff, out_dtype=w1_dtype)
-        else:
-            dw1 = kernels.grouped_gemm_wgrad(qx_t, sx_t, qg_t, sg_t, goff, out_dtype=w1_dtype)
+    dx, dw1, dw2, db1, db2 = host().mlp_backward(
+        dy, goff, row_map, ctx.dispatch_topk, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, ctx.glu, ctx.transpose_w1,
+        ctx.has_b1, ctx.has_b2, x_dtype, w1_dtype, w2_dtype,
+    )  # fmt: skip
     dv1 = None
     if ctx.has_v1:  # the gate and the up half of the gradient go back to their own parameters
         dim = 1 if ctx.transpose_w1 else 2
@@ -143,7 +116,6 @@ class _Fp8ExpertMlp(torch.autograd.Function):
             ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
             ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)
             ctx.dispatch_topk = topk
-            ctx.num_tokens = x.shape[0]
             ctx.save_for_backward(goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map)
         return out
 
@@ -175,7 +147,6 @@ class _Fp8MoeLayer(torch.autograd.Function):
             ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
             ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)
             ctx.dispatch_topk = topk
-            ctx.num_tokens = x.shape[0]
             ctx.save_for_backward(y, probs_c, goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map)
         return out
 

@@ -320,6 +320,24 @@ def gelu_tile_quant_dual_grouped(
     return res if return_activation else res[:4]
 
 
+def gradient_quant_with_sums(x: torch.Tensor, group_offsets: torch.Tensor, num_groups: int, dh: Optional[torch.Tensor] = None,
+                             activation: Optional[str] = None, ld_t: Optional[int] = None, eps: float = 0.0,
+                             sums_dtype=torch.float32):  # fmt: skip
+    """The dual quantiser of a gradient (blocked transposed codes) that also sums its columns per group, a bias
+    gradient: of ``x [M, N]`` bf16 itself, or, with ``dh``, of the gradient through ``activation`` ("gelu": x
+    [M, F]; "swiglu": x [M, 2F]).  Returns ``(q, s, q_t, s_t, sums [E, N])``."""
+    assert x.dim() == 2 and x.is_contiguous() and x.dtype == torch.bfloat16 and x.shape[1] % TILE == 0
+    assert (dh is None) == (activation is None) and activation in (None, "swiglu", "gelu")
+    if dh is not None:
+        F = x.shape[1] // (2 if activation == "swiglu" else 1)
+        assert dh.shape == (x.shape[0], F) and dh.is_contiguous() and dh.dtype == torch.bfloat16
+    assert group_offsets.dtype == torch.int64 and group_offsets.numel() == num_groups + 1
+    if ld_t is None:
+        ld_t = padded_bound(x.shape[0], num_groups)
+    what = {None: 0, "swiglu": 1, "gelu": 2}[activation]
+    return host().dual_with_sums(what, x, dh, group_offsets, num_groups, ld_t, eps, sums_dtype)
+
+
 def block_quant_batched(w: torch.Tensor, eps: float = 0.0, return_transpose: bool = False):
     """128x128 block quantisation of ``w [E, N, K]`` in one launch.
     Returns ``(q [E,N,K], s [E,N/128,K/128], q_t [E,K,N] | None, s_t [E,K/128,N/128] | None)``."""

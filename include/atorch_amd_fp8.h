@@ -279,6 +279,28 @@ int aamd_unpermute_probs_grad(const void *dout, int dout_dtype, const void *y, i
                               const int32_t *row_map, int64_t T, int topk, float *dprobs, void *stream);
 
 /*
+ * The dual quantiser of a gradient that also leaves the column sums of its 128-token tiles, and the sums of those over
+ * the groups: a bias gradient without another pass over the gradient (and, where the quantiser computes it, without
+ * writing it).  Replaces the row sums per expert beside the quantisation: bias_gather_add_bw
+ * (atorch/kernels/triton_jit/bias_gather_add.py:101-127), quantized_grouped_linear.py:84-86, 201.
+ *   what: AAMD_SUMS_PLAIN      the bf16 gradient itself, x [M, width]
+ *         AAMD_SUMS_GELU_BWD   dh gelu'(x) of x, dh [M, width] bf16
+ *         AAMD_SUMS_SWIGLU_BWD [da | db] of x = [a | b] [M, width], dh [M, width/2] bf16
+ *   q, s, q_t, s_t, ld_t, q_t_layout as for aamd_quant_1x128_dual_grouped with cols = width; eps 0 but for PLAIN
+ *   tile_sums [ld_t/128, width] fp32: row p/128 holds the sums of the tile at padded token p; rows of no tile are not
+ *   written
+ *   aamd_group_sums: out [E, cols] of out_dtype = sums of tile_sums over each group's tiles (0 for an empty group)
+ */
+#define AAMD_SUMS_PLAIN 0
+#define AAMD_SUMS_SWIGLU_BWD 1
+#define AAMD_SUMS_GELU_BWD 2
+int aamd_dual_grouped_with_sums(int what, const void *x, const void *dh, int64_t M, int64_t width,
+                                const int64_t *group_offsets, int E, uint8_t *q, float *s, uint8_t *q_t, float *s_t,
+                                int64_t ld_t, int q_t_layout, float eps, float *tile_sums, void *stream);
+int aamd_group_sums(const float *tile_sums, int64_t cols, const int64_t *group_offsets, int E, void *out, int out_dtype,
+                    void *stream);
+
+/*
  * Both gradients of the combine in one pass: drows[row_map[t*topk+j]] = dout[t] * probs[t, j] rounded to the rows'
  * type, dprobs[t, j] = sum_h dout[t, h] * y[row_map[t*topk+j], h] (fp32 sums) in the weights' type, 0 for a dropped
  * copy.  What autograd makes of token_dispatcher.py:155-159.
