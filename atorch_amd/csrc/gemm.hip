@@ -152,7 +152,9 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     const int pos = (int)idx - turn * per_x;
     g = turn;
     if (turn >= p.E) return;
-    if (p.E <= 64) {
+    if (p.goff == nullptr) {  // one group over the whole contraction
+      kb_hi = p.max_kb;
+    } else if (p.E <= 64) {
       gr = group_ranges<kBK>(p.goff, p.E, 0, 0);
       const int n = gr.t_hi - gr.t_lo;
       const bool live = lane < p.E;
@@ -1104,7 +1106,7 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   AAMD_REQUIRE(dw_dtype == AAMD_BF16 || dw_dtype == AAMD_F32, "grouped_gemm_wgrad: unsupported output dtype %d", dw_dtype);
   AAMD_REQUIRE(N >= 0 && K >= 0 && N % kTile == 0 && K % kTile == 0,
                "grouped_gemm_wgrad: N=%lld and K=%lld must be multiples of 128", (long long)N, (long long)K);
-  AAMD_REQUIRE(E >= 1 && group_offsets, "grouped_gemm_wgrad: group_offsets required");
+  AAMD_REQUIRE(E >= 1 && (group_offsets || E == 1), "grouped_gemm_wgrad: group_offsets required when E > 1");
   AAMD_REQUIRE(ld_t >= 0 && ld_t % kBK == 0, "grouped_gemm_wgrad: ld_t=%lld must be a multiple of 128", (long long)ld_t);
   AAMD_REQUIRE(ld_t < (1LL << 23), "grouped_gemm_wgrad: ld_t too large");
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "grouped_gemm_wgrad: unknown operand layout %d", q_t_layout);

@@ -197,6 +197,33 @@ Tensor gemm_wgrad(const Tensor& dy_t, const Tensor& sdy_t, const Tensor& x_t, co
   return c;
 }
 
+Tensor transpose_scales(const Tensor& s) {
+  Tensor t = empty({s.size(1), s.size(0)}, at::kFloat, s);
+  check(aamd_transpose_scales(ptr<float>(s), s.size(0), s.size(1), ptr<float>(t), stream()));
+  return t;
+}
+// C = A @ B^T of one group, 1x128 scales on A, 128x128 or 1x128 scales on B.
+Tensor fp8_gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, at::ScalarType dtype) {
+  const int64_t K = a.size(-1), M = K ? a.numel() / K : 0, N = b.size(0), blocks = K / kTile;
+  std::vector<int64_t> shape(a.sizes().begin(), a.sizes().end());
+  shape.back() = N;
+  Tensor c = empty(shape, dtype, a);
+  const bool b_tile_scaled = b_s.size(0) == N;
+  // Both sides scaled per row, as in the dense weight gradient: the weight-gradient kernel is built for it, but reads
+  // the scales block by block.  Two small launches turn them round, which pays for large outputs (us, without and with:
+  // 14336 x 4096 x 4096 327 -> 280, x 1024 117 -> 104, x 256 64 -> 58; 4096 x 4096 x 4096 95 -> 100; the results are equal).
+  constexpr int64_t kDenseWgradTiles = 2048;  // 128 x 128 outputs
+  if (b_tile_scaled && M % kTile == 0 && N % kTile == 0 && (M / kTile) * (N / kTile) >= kDenseWgradTiles) {
+    Tensor at = transpose_scales(a_s.view({M, blocks})), bt = transpose_scales(b_s);
+    check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(a), ptr<float>(at), ptr<uint8_t>(b), ptr<float>(bt), K, AAMD_QT_ROWS, nullptr,
+                                      1, nullptr, M, N, ptr(c), dtype_code(dtype), M * N, 0, stream()));
+    return c;
+  }
+  check(aamd_grouped_gemm_fp8_nt(ptr<uint8_t>(a), K, ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(b_s), b_tile_scaled, nullptr, 1,
+                                 nullptr, M, N, K, ptr(c), dtype_code(dtype), N, nullptr, AAMD_NONE, stream()));
+  return c;
+}
+
 // ---- routing ---------------------------------------------------------------------------------
 struct Routing {
   Tensor sorted_idx, row_map, goff;
@@ -455,6 +482,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("block_quant", &block_quant);
   m.def("gemm_nt", &gemm_nt);
   m.def("gemm_wgrad", &gemm_wgrad);
+  m.def("transpose_scales", &transpose_scales);
+  m.def("fp8_gemm", &fp8_gemm);
   m.def("moe_preprocess", &moe_preprocess);
   m.def("invert_permutation", &invert_permutation);
   m.def("permute_rows", &permute_rows);

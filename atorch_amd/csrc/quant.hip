@@ -1027,6 +1027,21 @@ __global__ __launch_bounds__(256) void group_sums_kernel(const float* __restrict
   else out[(int64_t)g * cols + c] = (OUT)f32_to_bf16_bits(sum);
 }
 
+// [rows, blocks] scales to [blocks, rows], through 32 x 32 tiles in the LDS
+__global__ __launch_bounds__(256) void transpose_scales_kernel(const float* __restrict__ s, int rows, int blocks,
+                                                               float* __restrict__ s_t) {
+  __shared__ float tile[32][33];
+  const int c = (int)threadIdx.x & 31, r = (int)threadIdx.x >> 5;
+  const int row0 = (int)blockIdx.x * 32, blk0 = (int)blockIdx.y * 32;
+#pragma unroll
+  for (int i = 0; i < 32; i += 8)
+    if (row0 + r + i < rows && blk0 + c < blocks) tile[r + i][c] = s[(int64_t)(row0 + r + i) * blocks + blk0 + c];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 32; i += 8)
+    if (row0 + c < rows && blk0 + r + i < blocks) s_t[(int64_t)(blk0 + r + i) * rows + row0 + c] = tile[c][r + i];
+}
+
 template <typename OUT>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ q, const float* __restrict__ s,
                                                       int64_t M, int64_t N, int tile_scale,
@@ -1449,6 +1464,16 @@ extern "C" int aamd_quant_128x128(const void* w, int w_dtype, int64_t E, int64_t
   else
     quant_128x128_kernel<F32><<<grid, block, 0, st>>>((const float*)w, expert_stride, N, K, q, s, q_t, s_t, eps);
   AAMD_LAUNCH_CHECK("quant_128x128");
+  return AAMD_OK;
+}
+
+extern "C" int aamd_transpose_scales(const float* s, int64_t rows, int64_t blocks, float* s_t, void* stream) {
+  AAMD_REQUIRE(rows >= 0 && blocks >= 0 && rows < 0x7fffffffLL && (blocks + 31) / 32 <= 65535, "transpose_scales: bad sizes");
+  if (rows == 0 || blocks == 0) return AAMD_OK;
+  AAMD_REQUIRE(s && s_t, "transpose_scales: null pointer");
+  transpose_scales_kernel<<<dim3((unsigned)((rows + 31) / 32), (unsigned)((blocks + 31) / 32)), 256, 0, (hipStream_t)stream>>>(
+      s, (int)rows, (int)blocks, s_t);
+  AAMD_LAUNCH_CHECK("transpose_scales");
   return AAMD_OK;
 }
 

@@ -114,20 +114,18 @@ def fp8_gemm(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.Ten
     (triton_kernel.py:198-210)."""
     assert a.is_contiguous() and b.is_contiguous()
     assert a_s.is_contiguous() and b_s.is_contiguous()
-    K = a.size(-1)
-    M = a.numel() // K
-    N = b.size(0)
-    c = torch.empty(*a.size()[:-1], N, dtype=dtype, device=a.device)
-    b_tile_scale = b_s.size(0) == b.size(0)
-    args = (ptr(a), K, ptr(a_s), ptr(b), ptr(b_s), int(b_tile_scale), None, 1, None, M, N, K,
-            ptr(c), dtype_code(dtype), N, None, _lib.NONE)  # fmt: skip
     pinned = _pinned_options()
-    if pinned:
-        from . import _probes
+    if not pinned:
+        return host().fp8_gemm(a, a_s, b, b_s, dtype)
+    from . import _probes
 
-        _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nt(*args, _probes.options_array(pinned), stream()))
-    else:
-        check(lib().aamd_grouped_gemm_fp8_nt(*args, stream()))
+    K = a.size(-1)
+    M, N = a.numel() // K, b.size(0)
+    c = torch.empty(*a.size()[:-1], N, dtype=dtype, device=a.device)
+    _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nt(
+        ptr(a), K, ptr(a_s), ptr(b), ptr(b_s), int(b_s.size(0) == N), None, 1, None, M, N, K, ptr(c), dtype_code(dtype), N, None,
+        _lib.NONE, _probes.options_array(pinned), stream(),
+    ))  # fmt: skip
     return c
 
 

@@ -240,6 +240,7 @@ int aamd_grouped_gemm_fp8_nt_static(const uint8_t *a, int64_t lda, const float *
  *   [ld_t/128, K, 128])
  *   dw [E, N, K] of dw_dtype (expert stride in elements); an empty group gives zeros,
  *   or leaves dw_g untouched when accumulate != 0.
+ *   group_offsets NULL: one group over all ld_t tokens (then E must be 1).
  *   ld_t must cover the padded token total sum_g ceil(M_g/128)*128, which only the device knows:
  *   a group whose tokens lie beyond ld_t gets NaN in its dw_g instead of a wrong finite gradient.
  */
@@ -299,6 +300,12 @@ int aamd_dual_grouped_with_sums(int what, const void *x, const void *dh, int64_t
                                 int64_t ld_t, int q_t_layout, float eps, float *tile_sums, void *stream);
 int aamd_group_sums(const float *tile_sums, int64_t cols, const int64_t *group_offsets, int E, void *out, int out_dtype,
                     void *stream);
+
+/*
+ * Scales [rows, blocks] (row-major, as the dense GEMM's callers hold them, triton_kernel.py:198-210) to the block-major
+ * [blocks, rows] that the weight-gradient GEMM reads.
+ */
+int aamd_transpose_scales(const float *s, int64_t rows, int64_t blocks, float *s_t, void *stream);
 
 /*
  * Both gradients of the combine in one pass: drows[row_map[t*topk+j]] = dout[t] * probs[t, j] rounded to the rows'
