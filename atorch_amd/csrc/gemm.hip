@@ -25,6 +25,8 @@
 // requested two steps ahead).  Rows are 128 bytes; the 16-byte chunks of a row
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
+#include <algorithm>
+
 #include "gemm.hpp"
 #ifdef AAMD_TUNING
 #include "../../include/atorch_amd_probes.h"
@@ -89,6 +91,232 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// ---- weight gradient of short groups -----------------------------------------------------------
+// A tile of a group of few rows is over after one or two 128-deep steps, and what it costs in grouped_gemm_kernel is the
+// workgroup's turnover: launch, group lookup, first loads and the stores follow each other, with two workgroups per CU to
+// hide one behind the other.  Here a workgroup takes `run` consecutive 128 x 128 tiles of the groups in `mask` (a row of
+// tiles of the output after the other) and the loads of the next step, which may be the next tile's, are in flight under
+// the step and the stores before it.  The arithmetic and its order are those of grouped_gemm_kernel: the same bits.
+// What bounds it is the stream of gradients written (and read, where they accumulate).
+//
+// LDS: two stages of 32 KB, [L rows | R rows], and their scales; the output of a tile is staged in the stage it was
+// computed from, 8 KB per wave, rows of 128 bytes with their 16-byte chunks XORed with three bits of the row.
+struct ShortTiles {
+  unsigned long long mask;  // groups
+  int total;                // their tiles
+  GroupRanges gr;           // lane e: the contraction blocks of group e
+};
+
+template <typename OUT, bool ACC>
+__device__ __forceinline__ void wgrad_short_tiles(const GemmParams& p, uint8_t* lds, float* Sc, const ShortTiles& st, int unit) {
+  constexpr int kStage = 2 * kTile * kBK;
+  constexpr int WT = 2;  // 2 x 2 waves of 2 x 2 sub-tiles
+  typedef typename std::conditional<ACC, float, OUT>::type ST;  // staging: float where the old output is added
+  constexpr int CW = 128 / (int)sizeof(ST), SUBS = CW / 32, VL = 16 / (int)sizeof(ST);
+  // vector memory instructions of a thread's stores of a tile, at least: what may stay in flight when the loads issued
+  // before them have to have landed
+  constexpr int kStores = 8 * (WT / SUBS);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hg = lane >> 5;
+  const int wr = wave >> 1, wl = wave & 1;
+  const int per_g = p.nLt * p.nRt;
+  int left = st.total - unit * p.run;  // tiles from the first of this unit to the end of the list
+  if (left <= 0) return;
+  if (left > p.run) left = p.run;
+
+  // ---- the tile under way: group, tile row and column, contraction blocks
+  struct Tile {
+    int g, lt, rt, kb, n;
+    bool nan;
+    unsigned long long rest;  // groups of the list behind g
+  };
+  auto enter = [&](Tile& t) {
+    t.kb = __builtin_amdgcn_readlane(st.gr.t_lo, t.g);
+    const int hi = __builtin_amdgcn_readlane(st.gr.t_hi, t.g);
+    t.nan = hi > p.max_kb;  // operand buffers too short: never read past them, and make the failure visible
+    t.n = t.nan ? 0 : hi - t.kb;
+  };
+  auto next_group = [&](Tile& t) {
+    t.g = __builtin_ctzll(t.rest);
+    t.rest &= t.rest - 1;
+    enter(t);
+  };
+  Tile cur;
+  {
+    int turn = unit * p.run / per_g;
+    const int pos = unit * p.run - turn * per_g;
+    cur.rest = st.mask;
+    for (; turn > 0; turn--) cur.rest &= cur.rest - 1;
+    next_group(cur);
+    cur.lt = pos / p.nRt;
+    cur.rt = pos - cur.lt * p.nRt;
+  }
+  auto advance = [&](Tile& t) {
+    if (++t.rt < p.nRt) return;
+    t.rt = 0;
+    if (++t.lt < p.nLt) return;
+    t.lt = 0;
+    next_group(t);
+  };
+
+  // ---- loads: the slabs and swizzle of grouped_gemm_kernel (rows and columns of the output are whole tiles here)
+  auto lds_addr = [](const void* q) { return (uint32_t)(uintptr_t)(lds_ptr_t)q; };
+  const int r8 = lane >> 3;
+  const uint32_t chunk = (uint32_t)(((lane & 7) ^ r8 ^ (wave & 1)) << 4);
+  const uint32_t voffL = (uint32_t)r8 * (uint32_t)p.ldl + chunk, voffR = (uint32_t)r8 * (uint32_t)p.ldr + chunk;
+  const uint32_t soff = (uint32_t)(tid & (kTile - 1)) * 4u;
+  auto load = [&](const Tile& t, int k, int s) {
+    const int64_t kb = t.kb + k;
+    const uint8_t* L = p.L + uniform_i64((int64_t)t.lt * kTile * p.ldl + kb * p.l_kb_stride);
+    const uint8_t* R = p.R + uniform_i64((int64_t)t.rt * kTile * p.ldr + kb * p.r_kb_stride);
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+      const int row = wave * 8 + 32 * n;
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voffL),
+                   "s"(L + (uint32_t)row * (uint32_t)p.ldl), "s"(lds_addr(lds) + (uint32_t)(s * kStage + row * kBK))
+                   : "memory");
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+      const int row = wave * 8 + 32 * n;
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voffR),
+                   "s"(R + (uint32_t)row * (uint32_t)p.ldr), "s"(lds_addr(lds) + (uint32_t)(s * kStage + (kTile + row) * kBK))
+                   : "memory");
+    }
+    // waves 0 and 1: the scales of the L rows, 2 and 3: of the R rows
+    const float* sb = wave < 2 ? p.Ls + (kb * p.ls_blk_stride + t.lt * kTile) : p.Rs + (kb * p.rs_blk_stride + t.rt * kTile);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(soff), "s"(sb),
+                 "s"(lds_addr(Sc) + (uint32_t)(s * 1024 + wave * 256))
+                 : "memory");
+  };
+
+  v16f acc[WT][WT], zero;
+#pragma unroll
+  for (int r = 0; r < 16; r++) zero[r] = 0.f;
+  auto clear = [&](const Tile& t) {
+    const float v = t.nan ? __builtin_nanf("") : 0.f;
+#pragma unroll
+    for (int i = 0; i < WT; i++)
+#pragma unroll
+      for (int j = 0; j < WT; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][j][r] = v;
+  };
+  const int sw = swz(l32);
+  auto compute = [&](int s) {
+    const uint8_t* const Lt = lds + s * kStage + (wl * 64 + l32) * kBK;
+    const uint8_t* const Rt = lds + s * kStage + (kTile + wr * 64 + l32) * kBK;
+    const float* const S = Sc + s * 256;
+    auto frag = [&](const uint8_t* row, int h) {
+      const v4i lo = *reinterpret_cast<const v4i*>(row + (((4 * h + 2 * hg) ^ sw) << 4));
+      const v4i hi = *reinterpret_cast<const v4i*>(row + (((4 * h + 2 * hg + 1) ^ sw) << 4));
+      return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    v8i lf[WT][2], rf[WT][2];
+    float cs[WT];
+#pragma unroll
+    for (int j = 0; j < WT; j++) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        lf[j][h] = frag(Lt + j * 32 * kBK, h);
+        rf[j][h] = frag(Rt + j * 32 * kBK, h);
+      }
+      cs[j] = S[wl * 64 + j * 32 + l32];
+    }
+#pragma unroll
+    for (int i = 0; i < WT; i++) {
+      v4f rs[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) rs[q] = *reinterpret_cast<const v4f*>(&S[kTile + wr * 64 + i * 32 + 8 * q + 4 * hg]);
+#pragma unroll
+      for (int j = 0; j < WT; j++) {
+        v16f pr = mfma_fp8_32x32x64(rf[i][0], lf[j][0], zero);
+        pr = mfma_fp8_32x32x64(rf[i][1], lf[j][1], pr);
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][j][r] = __builtin_fmaf(pr[r], cs[j] * rs[r / 4][r % 4], acc[i][j][r]);
+      }
+    }
+  };
+  auto store = [&](const Tile& t, int s) {
+    uint8_t* const stg = lds + s * kStage + wave * (64 * 128);
+    OUT* const Cg = reinterpret_cast<OUT*>(p.C) + (int64_t)t.g * p.c_group_stride;
+#pragma unroll
+    for (int ci = 0; ci < WT / SUBS; ci++) {
+#pragma unroll
+      for (int si = 0; si < SUBS; si++)
+#pragma unroll
+        for (int j = 0; j < WT; j++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const v16f& a = acc[ci * SUBS + si][j];
+            const v4f o = v4f{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+            const int row = j * 32 + l32, byte = (si * 32 + 8 * q + 4 * hg) * (int)sizeof(ST);
+            uint8_t* const dst = stg + row * 128 + (((byte >> 4) ^ ((row >> 1) & 7)) << 4) + (byte & 15);
+            if constexpr (sizeof(ST) == 4) *reinterpret_cast<v4f*>(dst) = o;
+            else *reinterpret_cast<v2i*>(dst) = v2i{(int)pack_bf16x2(o[0], o[1]), (int)pack_bf16x2(o[2], o[3])};
+          }
+      __builtin_amdgcn_wave_barrier();  // same wave, in-order LDS: the reads below see the writes above
+      OUT* const out0 = Cg + ((int64_t)t.lt * kTile + wl * 64 + r8) * p.ldc + (t.rt * kTile + wr * 64 + ci * CW + (lane & 7) * VL);
+      v4i raws[8];
+#pragma unroll
+      for (int ps = 0; ps < 8; ps++) {
+        const int row = ps * 8 + r8;
+        raws[ps] = *reinterpret_cast<const v4i*>(stg + row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+      }
+      if constexpr (ACC && sizeof(OUT) == 4) {
+#pragma unroll
+        for (int half = 0; half < 8; half += 4) {
+          v4f olds[4];
+#pragma unroll
+          for (int ps = 0; ps < 4; ps++) olds[ps] = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(out0 + (half + ps) * 8 * p.ldc));
+#pragma unroll
+          for (int ps = 0; ps < 4; ps++) {
+            const v4f o = __builtin_bit_cast(v4f, raws[half + ps]) + olds[ps];
+            __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(out0 + (half + ps) * 8 * p.ldc));
+          }
+        }
+      } else {
+#pragma unroll
+        for (int ps = 0; ps < 8; ps++) {
+          if constexpr (sizeof(ST) == sizeof(OUT)) __builtin_nontemporal_store(raws[ps], reinterpret_cast<v4i*>(out0 + ps * 8 * p.ldc));
+          else store4<OUT>(out0 + ps * 8 * p.ldc, __builtin_bit_cast(v4f, raws[ps]), true);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();  // the next chunk overwrites the region
+    }
+  };
+
+  if (cur.n > 0) load(cur, 0, 0);
+  clear(cur);
+  bool stored = false;
+  for (int k = 0, s = 0;; s ^= 1) {
+    const bool last = k + 1 >= cur.n;  // (a tile without a contraction is one empty step)
+    const bool more = !last || left > 1;
+    Tile nxt = cur;
+    int kn = k + 1;
+    if (last) {
+      kn = 0;
+      if (left > 1) advance(nxt);
+    }
+    // this step's loads have landed and every wave is done with the other stage (loads and stores are counted in order,
+    // and the stores of the tile before were issued behind these loads)
+    if (stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kStores) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (more && nxt.n > 0) load(nxt, kn, s ^ 1);
+    if (cur.n > 0) compute(s);
+    stored = last;
+    if (last) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave has read the stage
+      store(cur, s);
+      if (--left == 0) return;
+      clear(nxt);
+    }
+    cur = nxt;
+    k = kn;
+  }
+}
+
 template <int MODE, bool R_PER_ROW, typename OUT, typename C>
 __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kernel(const GemmParams p) {
   constexpr int BM = C::BM, BN = C::BN, NT = C::NT;
@@ -151,16 +379,34 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     const int turn = __builtin_amdgcn_readfirstlane((int)((uint32_t)idx / (uint32_t)per_x));
     const int pos = (int)idx - turn * per_x;
     g = turn;
-    if (turn >= p.E) return;
+    if (turn >= p.E && p.run == 0) return;
     if (p.goff == nullptr) {  // one group over the whole contraction
       kb_hi = p.max_kb;
     } else if (p.E <= 64) {
       gr = group_ranges<kBK>(p.goff, p.E, 0, 0);
       const int n = gr.t_hi - gr.t_lo;
-      const bool live = lane < p.E;
+      bool live = lane < p.E;
+      if constexpr (NT == 256) if (p.run > 0) {
+        // the groups of few blocks leave the list of this loop: behind the long groups' tiles a workgroup takes a run of
+        // theirs (and of the groups that the operand buffers do not hold, which are written as NaN)
+        const bool few = live && (gr.t_hi > p.max_kb || (n <= p.short_kb && (n > 0 || !p.accumulate)));
+        const bool none = n == 0 && p.accumulate;  // nothing to add
+        live = live && !few && !none;
+        const int nlong = __popcll(__ballot(live));
+        if (turn >= nlong) {
+          ShortTiles st;
+          st.mask = __ballot(few);
+          st.total = __popcll(st.mask) * per_g;
+          st.gr = gr;
+          const int unit = ((int)idx - nlong * per_x) * 8 + (int)xcd;
+          if (p.accumulate) wgrad_short_tiles<OUT, true>(p, lds, Sc0, st, unit);
+          else wgrad_short_tiles<OUT, false>(p, lds, Sc0, st, unit);
+          return;
+        }
+      }
       const unsigned long long big = __ballot(live && (int64_t)n * p.E > 2 * (int64_t)gr.total);
       const unsigned long long mid = __ballot(live && (int64_t)n * p.E > (int64_t)gr.total) & ~big;
-      const unsigned long long low = ((p.E == 64 ? 0ull : 1ull << p.E) - 1ull) & ~(big | mid);
+      const unsigned long long low = __ballot(live) & ~(big | mid);
       // this lane's group is the r-th of the order: all of `big`, then all of `mid`, then the rest
       const unsigned long long below = (1ull << lane) - 1ull;
       const int nbig = __popcll(big), nmid = __popcll(mid);
@@ -1020,6 +1266,25 @@ static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
   return g_opt.tile >= 0 ? g_opt.tile == 1 : tiles_256 >= 512;
 }
 
+// Weight gradient: the tiles of groups of at most kShortBlocks contraction blocks (1024 rows) are taken in runs
+// (wgrad_short_tiles) where the groups have kShortAverage blocks or fewer on average; longer ones cover a tile's turnover by
+// themselves.  Runs of four tiles (two for an fp32 output that is written only, whose stores alone keep the memory busy),
+// and fewer where the launch would have less than kShortUnits workgroups.  Measured on MI355X, us, one tile per workgroup
+// -> runs of 1 / 2 / 4 / 8 tiles with the line at 8 blocks, the line at 4 and runs of 4, and the stream of the outputs:
+//   64 groups, 8192 rows (Zipf), 2048 x 7168 bf16          531 -> 480 / 447 / 454 / 461, 478    342
+//   60 groups, 16001 rows (Zipf), 2816 x 2048 fp32, added  224 -> 178 / 169 / 151 / 164, 163
+//   60 groups, 32764 rows (uneven), 2816 x 2048 bf16       365 -> 362 / 333 / 321 / 340, 330    126
+//   60 groups, 4096 rows, 2816 x 2048 bf16                 201 -> 181 / 147 / 128 / 132, 139    126
+//   8 groups, 1000 rows, 4096 x 1024 bf16                   23 -> 23 / 19 / 19 / 19, 19          12
+//   60 groups, 400 rows, 1408 x 2048 fp32                  119 -> 115 / 118 / 139 / 162, 140    126
+//   8 groups, 8192 rows, 4096 x 4096 bf16                  221 -> 238 / 227 / 226 / 250, 210     49
+// (the last is where the average rule ends it: from there on both forms are within the noise of each other)
+constexpr int kShortBlocks = 8, kShortAverage = 8, kShortUnits = 1024;
+static bool use_short_runs(const GemmParams& p) {
+  return p.goff != nullptr && p.E <= 64 && p.max_kb <= (int64_t)kShortAverage * p.E &&
+         (int64_t)p.E * p.nLt * p.nRt < (1 << 27);
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace aamd
@@ -1137,7 +1402,15 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   p.Lrows = N; p.Rrows = K; p.nkb = 0; p.E = E; p.nRt = (int)((K + BN - 1) / BN); p.nLt = (int)((N + BM - 1) / BM);
   p.max_kb = (int)(ld_t / kBK);
   p.accumulate = accumulate;
-  const int64_t blocks = (int64_t)E * (((int64_t)p.nLt * p.nRt + 7) / 8) * 8;  // every XCD takes an eighth of a group
+  const int64_t per_g = (int64_t)p.nLt * p.nRt, per_x = (per_g + 7) / 8;  // every XCD takes an eighth of a group
+  int64_t blocks = (int64_t)E * per_x * 8;
+  if (g_opt.tile < 0 && use_short_runs(p)) {
+    p.short_kb = kShortBlocks;
+    p.run = (int)std::min<int64_t>(dw_dtype == AAMD_F32 && !accumulate ? 2 : 4, std::max<int64_t>(1, E * per_g / kShortUnits));
+    // long groups have more than short_kb blocks each, so that the operand buffers bound their number
+    const int64_t longs = std::min<int64_t>(E, p.max_kb / (p.short_kb + 1));
+    blocks = (longs * per_x + (E * per_g + 8 * p.run - 1) / (8 * p.run)) * 8;
+  }
 #ifdef AAMD_TUNING
   if (cfg == 1) return launch_gemm<kRaggedK, true, CfgWgrad>(p, dw_dtype, blocks, st, g_opt);
 #endif

@@ -36,6 +36,8 @@ struct GemmParams {
   int group_r;     // the tile order groups R tiles (inside each group of rows / expert) instead of L tiles
   int bias_dtype;
   int gl;          // L tiles that share an R panel in the tile order
+  int run;         // kRaggedK: tiles of short groups that a workgroup takes one after the other (0: none)
+  int short_kb;    // kRaggedK: the most contraction blocks of a short group
   int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
 };
 
