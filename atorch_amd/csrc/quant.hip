@@ -412,6 +412,16 @@ constexpr int kTLd = kTile + 16;  // LDS row stride (bytes) of the transposed co
 // 128 rows of a tile are addressed with 32-bit byte offsets: row strides (elements, at most 4 bytes each) stay below this
 constexpr int64_t kMaxTileLd = (int64_t)1 << 22;
 
+// A row past the group's end: zeros, or, where the activation comes from a table, values that are in it: zeros are not,
+// and took a tile of few rows through the out-of-line arithmetic, a call per pair (60 groups of 68 rows, 1408 columns,
+// GELU and its backward 27 -> 14 and 30 -> 15 us, SwiGLU backward 31 -> 23; 8 groups of 125 rows, 4096 columns, GELU 21 ->
+// 11; 32764 rows in 60 uneven groups 61 -> 49 and 70 -> 58).  The GELU's own result is cleared by its reader.
+constexpr v4i kOnes = {0x3f803f80, 0x3f803f80, 0x3f803f80, 0x3f803f80};  // bf16
+template <typename IN>
+__device__ __forceinline__ void absent_row(Raw8<IN>& raw) {
+  raw.zero();
+  if constexpr (std::is_same<IN, GELU>::value || std::is_same<IN, GELUB>::value) raw.a = kOnes;
+}
 // `x` is the tile's origin, the same in every lane; FULL: all 128 rows are valid
 template <typename IN, bool FULL>
 __device__ __forceinline__ void issue_tile_loads(const typename IN::elem* __restrict__ x, uint32_t ldx, int rows_valid,
@@ -424,7 +434,7 @@ __device__ __forceinline__ void issue_tile_loads(const typename IN::elem* __rest
     if (FULL || gr * 8 + i < rows_valid)
       raw[i].load(x, off0 + (uint32_t)i * ldx * kEl, gate_off);
     else
-      raw[i].zero();
+      absent_row(raw[i]);
   }
 }
 template <typename IN, bool FULL>
@@ -496,7 +506,7 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
       if (FULL || gr * 8 + i < mvalid)
         raw[i].load(x + (int64_t)src_row[gr * 8 + i] * ldx + (int64_t)kc * kTile, (uint32_t)c * 8 * kEl, gate_off);
       else
-        raw[i].zero();
+        absent_row(raw[i]);
     }
   } else {
     issue_tile_loads<IN, FULL>(x + m0 * ldx + (int64_t)kc * kTile, ldx, mvalid, raw, gate_off);
@@ -521,6 +531,10 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
     if constexpr (kPacked) {
       raw[i].pin();
       raw[i].get(vi, lut);  // the activation from its table in LDS
+      if constexpr (!FULL && std::is_same<IN, GELU>::value) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) vi[j] = live ? vi[j] : 0.f;
+      }
     } else {
       raw[i].get(vi);
     }
@@ -533,7 +547,9 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
     }
     if (hb != nullptr && live) st_nt(hb, (r * ucols + (uint32_t)c * 8) * 2, pack8_bf16(vi));
     if (qb != nullptr) {
-      const Divider dv = make_scale(row16_max(amax8(vi)), eps, plain_div);
+      // (a row past the group's end has no codes; a maximum of zero would send it through the plain division)
+      const float amax = row16_max(amax8(vi));
+      const Divider dv = make_scale(live ? amax : 1.f, eps, plain_div);
       const v2i codes = quant8(vi, dv);
       if (live) {
         st_nt(qb, r * ucols + (uint32_t)c * 8, codes);
@@ -745,7 +761,8 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
         rb[i] = ld16_nt(xa + gate_off, off0 + (uint32_t)i * ld * 2);
         rd[i] = ld16_nt(xd, off0d + (uint32_t)i * ld_dh * 2);
       } else {
-        ra[i] = rb[i] = rd[i] = v4i{0, 0, 0, 0};
+        ra[i] = kOnes;  // (absent: inside the table, and the gradient is zero with rd)
+        rb[i] = rd[i] = v4i{0, 0, 0, 0};
       }
     }
   }
@@ -760,6 +777,8 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
   // one row at a time, from the packed inputs to the stored codes of both tiles
 #pragma unroll
   for (int i = 0; i < 4; i++) {
+    const uint32_t r = (uint32_t)(gr * 4 + i);
+    const bool live = FULL || (int)r < mvalid;
     float fa[8], fb[8], fd[8], v[2][8];
     unpack8(ra[i], fa);
     unpack8(rb[i], fb);
@@ -809,8 +828,6 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
       v[0][k] = __uint_as_float(oa << 16);
       v[0][k + 1] = __uint_as_float(oa & 0xffff0000u);
     }
-    const uint32_t r = (uint32_t)(gr * 4 + i);
-    const bool live = FULL || (int)r < mvalid;
 #pragma unroll
     for (int w = 0; w < 2; w++) {
       const int kc = w == 0 ? f : half + f;
@@ -820,7 +837,8 @@ __device__ __forceinline__ void swiglu_bwd_dual_tile(const u16* __restrict__ xa 
         st_nt(g_out + m0 * cols + (int64_t)kc * kTile, (r * ucols + (uint32_t)c * 8) * 2,
               v4i{(int)vp[w][i][0], (int)vp[w][i][1], (int)vp[w][i][2], (int)vp[w][i][3]});
       if (q != nullptr) {
-        const Divider dv = make_scale(row16_max(amax8(v[w])), 0.f, false);
+        const float amax = row16_max(amax8(v[w]));
+        const Divider dv = make_scale(live ? amax : 1.f, 0.f, false);
         const v2i codes = quant8<false>(v[w], dv);
         if (live) {
           st_nt(q + m0 * cols + (int64_t)kc * kTile, r * ucols + (uint32_t)c * 8, codes);
