@@ -26,6 +26,7 @@
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
 #include <algorithm>
+#include <cmath>
 
 #include "gemm.hpp"
 #ifdef AAMD_TUNING
@@ -1225,40 +1226,44 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
 }
 
 // Which kernel a row-ragged launch with block-scaled R takes: the one whose estimated time is least.  The estimates (us)
-// are fits to launches on MI355X of 1 to 4096 rows per group, 1 to 64 groups and 512 to 14336 outputs and contraction:
-//   - a tile of the 128x128 configuration costs 10 us outside its loop and 1 us per 128-deep step with two workgroups
-//     per CU (8 and 0.8 with one), and 512 run at a time, so a launch takes whole rounds of that;
-//   - a tile of the 256x256 configuration 8 us and 1.65 us per step (1.2 when the tiles are half empty: waves without
-//     rows only load), 256 at a time;
-//   - the kernel for few rows 1.4 ns per 64 x 64 x 128 block, spread over the chip, and 6 us in all;
-//   - and none can beat the weights' stream from memory, 5.2 TB/s in the first two and 6.2 in the third.
+// are fits to 570 launches on MI355X of 64 to 40000 rows in 1 to 64 even or uneven groups, 512 to 18000 outputs and a
+// contraction of 512 to 14336, each with all of the kernels (n: its 128-deep steps):
+//   - a round of 512 tiles of the 128x128 configuration, two per CU, costs 2.4 us and 0.98 us per step, a launch of at most
+//     256 tiles 5.4 and 0.7;
+//   - a round of 256 tiles of the 256x256 configuration 5.9 us and 0.82 to 1.42 us per step, by how full its tiles are;
+//   - a 64 x 64 block of the kernel for few rows 2.1 ns and 1.06 ns per step, spread over the chip; a 32 x 32 block of its
+//     split form 2.1 and 0.45; and no less than a wave's own chain of every fourth (eighth) step;
+//   - and none can beat the weights' stream from memory, 5.2 to 6.2 TB/s.
 // Token tiles are counted as the groups' expected number (their sizes are known on the device only): one per group with
-// few rows, half a tile more than the rows fill with many.  Examples, estimate (measured): 32768 rows in 8 groups,
-// 28672 x 4096: large 3.5 ms (3.6), small 4.4; one group of 4096 rows, 4096 x 14336: large 193, small 244 (270 us: the
-// rule that asked for 512 large tiles took them, and 256 are a full round); 8 groups of 16 rows, 4096 x 4096: few 35 (30),
-// small 42 (39).
+// few rows, half a tile more than the rows fill with many.  Over those launches the kernel taken is 2.4 % slower than the
+// best of the four (geometric mean; 8.4 % with a first fit that priced the few-rows kernel without its fixed cost per
+// block and the small tiles too high).  Us, that fit -> this one: one group of 14441 rows, 5504 x 640 200 -> 91; 64 groups,
+// 8591 rows, 16256 x 768 372 -> 195; 4 groups, 2498 rows, 8832 x 512 51 -> 30; 64 groups, 10168 rows, 1536 x 9088: the
+// 256x256 tiles instead of the small ones.
 enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3 };
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return g_opt.tile == 1 && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const int64_t groups = M < E ? M : E;
+  const double n = (double)nkb;
   auto token_tiles = [&](int rows) -> double {
-    if (!grouped) return (double)((M + rows - 1) / rows);
-    const double many = (double)M / rows + 0.5 * (double)groups;
-    return many > (double)groups ? many : (double)groups;
+    if (!grouped || E == 1) return (double)((M + rows - 1) / rows);
+    return std::max((double)M / rows + 0.5 * (double)groups, (double)groups);
   };
-  auto rounds = [](double tiles, int at_a_time) { return (double)(int64_t)((tiles + at_a_time - 1) / at_a_time); };
-  const double weights = (double)groups * (double)N * (double)nkb * (double)kBK;  // bytes
-  const double few_blocks = token_tiles(64) * (double)(N / 64);
-  const double few = 6.0 + 1.4e-3 * few_blocks * (double)nkb;
+  // whole rounds where there are few; with many the tiles' times spread and half a round is lost at the end
+  auto rounds = [](double x) { return x <= 1.0 ? 1.0 : x < 3.0 ? std::ceil(x) : x + 0.5; };
+  const double weights = (double)groups * (double)N * n * (double)kBK * 1e-6;  // MB
   const double tiles_s = token_tiles(128) * (double)(N / 128);
-  const double loop_s = tiles_s <= 256 ? 8.0 + 0.8 * (double)nkb : rounds(tiles_s, 512) * (10.0 + 1.0 * (double)nkb);
-  const double small = loop_s > weights / 5.2e6 ? loop_s : weights / 5.2e6;
+  const double small = std::max(tiles_s <= 256.0 ? 5.4 + 0.7 * n : 2.5 + rounds(tiles_s / 512.0) * (2.4 + 0.98 * n), weights / 5.6);
   // (the large configuration takes its scales in batches of eight contraction blocks)
-  const double rows_l = token_tiles(256) * 256.0;
-  const double loop_l = rounds(rows_l / 256.0 * (double)((N + 255) / 256), 256) * (8.0 + ((double)M > 0.5 * rows_l ? 1.65 : 1.2) * (double)nkb);
-  const double large = nkb < 8 ? 1e30 : loop_l > weights / 5.2e6 ? loop_l : weights / 5.2e6;
-  // the split form: with fewer workgroups than half the CUs the length of a wave's contraction is what counts
-  if (few <= small && few <= large) return few_blocks < 128 ? kFewRowsSplit : kFewRows;
+  const double rows_l = token_tiles(256), fill = std::min(1.0, (double)M / (256.0 * rows_l));
+  const double loop_l = 2.3 + rounds(rows_l * (double)((N + 255) / 256) / 256.0) * (5.9 + (0.82 + 0.6 * fill) * n);
+  const double large = nkb < 8 ? 1e30 : std::max(loop_l, weights / 5.2);
+  const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_p = token_tiles(32) * (double)(N / 32);
+  const double few = std::max({4.5 + 1e-3 * blocks_f * (1.06 * n + 2.1), 1.5 + 1.1 * std::ceil(n / 4.0), weights / 6.2});
+  // (the split form where the length of a wave's contraction is what counts: few workgroups, or a long contraction)
+  const bool may_split = blocks_f < 128.0 || nkb >= 28;
+  const double split = may_split ? std::max({2.2 + 1e-3 * blocks_p * (0.45 * n + 2.1), 4.0 + 0.63 * std::ceil(n / 8.0), weights / 6.2}) : 1e30;
+  if (std::min(few, split) <= std::min(small, large)) return split < few ? kFewRowsSplit : kFewRows;
   return large < small ? kLargeTiles : kSmallTiles;
 }
 // Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
