@@ -1126,8 +1126,13 @@ static int fill_table(TableState& state, void (*kernel)(), unsigned entries, hip
     std::lock_guard<std::mutex> guard(state.lock);
     flag = state.flag[dev].load(std::memory_order_acquire);
     if (flag == nullptr) {
-      if (hipHostMalloc(reinterpret_cast<void**>(&flag), sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();  // (another thread captures, or no pinned memory: the next call fills again)
+      // (an allocation may not break a capture that another thread has under way)
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+      const hipError_t got = hipHostMalloc(reinterpret_cast<void**>(&flag), sizeof(int32_t), hipHostMallocDefault);
+      if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (got != hipSuccess) {
+        (void)hipGetLastError();  // (no pinned memory: the next call fills again)
         return AAMD_OK;
       }
       *flag = 0;
