@@ -147,14 +147,24 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         return self._forward_megatron(hidden_states, expert_weights, top_experts, se_fn1, se_fn2,
                                       se_fn2_additional_input, is_first_microbatch)  # fmt: skip
 
+    def _weight(self, name):
+        """``getattr(self, name)`` in a third of its time where the name is a parameter.  (A pruned or parametrised one is
+        not, nor is one that a wrapper keeps as a plain attribute.)"""
+        p = self._parameters
+        return p[name] if name in p else getattr(self, name)
+
     def _forward_fused(self, x, probs, top_experts, is_first_microbatch):
         """Nothing happens between the experts and the combine: the layer is one function, one native call per
         direction."""
-        p = self._parameters
         assert x.dtype == torch.bfloat16, "the fused activation kernels read bf16"
         assert probs.shape == top_experts.shape == (x.shape[0], self.topk), "router weights and choices are [tokens, topk]"
-        args = (x, probs, p["w1"], p["w2"], p.get("v1"), p.get("b1"), p.get("b2"), top_experts, self.token_dispatcher,
-                self.transpose_w1, self.use_swiglu, is_first_microbatch, self.weight_code_cache)  # fmt: skip
+        w1, w2 = self.scale_grad(self._weight("w1")), self.scale_grad(self._weight("w2"))
+        v1 = self.scale_grad(self._weight("v1")) if self.has_v1() else None
+        b1, b2 = (self._weight("b1"), self._weight("b2")) if self.use_bias else (None, None)
+        assert v1 is None or self.use_swiglu, "v1 is the up projection of a gated unit"
+        assert v1 is None or b1 is None, "bias not supported yet for not merge_w1_v1"
+        args = (x, probs, w1, w2, v1, b1, b2, top_experts, self.token_dispatcher, self.transpose_w1, self.use_swiglu,
+                is_first_microbatch, self.weight_code_cache)  # fmt: skip
         return _Fp8MoeLayer.apply(*args) if torch.is_grad_enabled() else _Fp8MoeLayer.forward(None, *args)
 
     def _forward_megatron(self, hidden_states, expert_weights, top_experts, se_fn1=None, se_fn2=None,

@@ -1,0 +1,113 @@
+"""The MoE layer takes its parameters as attributes of the module, wherever pruning, a parametrisation or a wrapper keeps
+them, and through ``scale_grad`` (grouped_gemm_moe.py:632-636).  On the CPU with the fused function replaced by a recorder."""
+import pytest
+import torch
+from torch.nn.utils import parametrize, prune
+
+from helpers import randn_bf16, topk_routing
+
+NAMES = ("w1", "w2", "v1", "b1", "b2")
+
+
+class _Double(torch.nn.Module):
+    def forward(self, w):
+        return w * 2
+
+
+def _layer(monkeypatch, cls=None, **kw):
+    from atorch_amd import moe_layer
+
+    seen = {}
+
+    class Recorder:
+        @staticmethod
+        def apply(x, probs, *args):
+            seen.update(zip(NAMES, args[:5]))
+            return x * sum(a.float().sum() for a in args[:5] if a is not None)
+
+        @staticmethod
+        def forward(ctx, *args):
+            return Recorder.apply(*args)
+
+    monkeypatch.setattr(moe_layer, "_Fp8MoeLayer", Recorder)
+    layer = (cls or moe_layer.Grouped_GEMM_MoE)(256, 128, 0.0, 4, 2, implementation_type="Megatron", dtype=torch.bfloat16, **kw)
+    idx, probs = topk_routing(8, 4, 2, seed=1)
+
+    def run():
+        seen.clear()
+        return layer(randn_bf16((8, 256), 2), probs.bfloat16(), idx)
+
+    return layer, seen, run
+
+
+def _check(layer, seen):
+    for name in NAMES:
+        want = getattr(layer, name, None)
+        assert (seen[name] is None) == (want is None) and (want is None or torch.equal(seen[name], want)), name
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("kw", [dict(use_swiglu=True), dict(use_bias=True), dict(use_swiglu=True, merge_w1_v1=False)],
+                         ids=["merged", "bias", "separate"])  # fmt: skip
+def test_plain_parameters(monkeypatch, kw, grad):
+    layer, seen, run = _layer(monkeypatch, **kw)
+    with torch.set_grad_enabled(grad):
+        run()
+    _check(layer, seen)
+    assert all(seen[n] is p for n, p in layer.named_parameters())
+
+
+def test_pruned_bias_stays_and_gets_its_gradient(monkeypatch):
+    layer, seen, run = _layer(monkeypatch, use_bias=True)
+    with torch.no_grad():
+        layer.b1.normal_()
+    prune.l1_unstructured(layer, "b1", 0.5)
+    run().sum().backward()
+    _check(layer, seen)
+    assert seen["b1"] is not None and int((seen["b1"] == 0).sum()) == seen["b1"].numel() // 2
+    assert layer.b1_orig.grad is not None
+
+
+@pytest.mark.parametrize("name", ["w1", "w2", "v1"])
+def test_parametrised_weights(monkeypatch, name):
+    layer, seen, run = _layer(monkeypatch, use_swiglu=True, merge_w1_v1=False)
+    plain = getattr(layer, name).detach().clone()
+    parametrize.register_parametrization(layer, name, _Double())
+    run()
+    _check(layer, seen)
+    assert torch.equal(seen[name], plain * 2)
+
+
+def test_parameters_kept_as_plain_attributes(monkeypatch):
+    layer, seen, run = _layer(monkeypatch, use_bias=True)
+    for name in ("w1", "w2", "b1", "b2"):  # what a sharding wrapper does between its gather and its release
+        t = getattr(layer, name).detach().clone() + 1
+        delattr(layer, name)
+        setattr(layer, name, t)
+    run()
+    _check(layer, seen)
+
+
+def test_weights_go_through_scale_grad(monkeypatch):
+    from atorch_amd.moe_layer import Grouped_GEMM_MoE
+
+    class Scaled(Grouped_GEMM_MoE):
+        def scale_grad(self, w):
+            return w * 0.5
+
+    layer, seen, run = _layer(monkeypatch, Scaled, use_swiglu=True, merge_w1_v1=False)
+    run()
+    assert all(torch.equal(seen[n], getattr(layer, n) * 0.5) for n in ("w1", "w2", "v1"))
+
+
+def test_switched_off_bias_and_forbidden_combinations(monkeypatch):
+    layer, seen, run = _layer(monkeypatch, use_bias=True)
+    layer.use_bias = False
+    run()
+    assert seen["b1"] is None and seen["b2"] is None
+    layer.v1 = torch.nn.Parameter(torch.zeros_like(layer.w1))  # an up projection without a gate
+    with pytest.raises(AssertionError):
+        run()
+    layer.use_swiglu = layer.use_bias = True
+    with pytest.raises(AssertionError):
+        run()
