@@ -28,6 +28,12 @@ void check(int rc) {
   if (rc == AAMD_ERR_ARG) throw py::value_error(aamd_last_error());
   throw std::runtime_error(aamd_last_error());
 }
+// Refuses what the kernels would answer with reads or writes out of range: they see pointers and sizes, not tensors.
+void require(bool ok, const char* what) {
+  if (__builtin_expect(ok, 1)) return;
+  PyErr_SetString(PyExc_AssertionError, what);
+  throw py::error_already_set();
+}
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 void on_gpu(const Tensor& t) {
@@ -229,6 +235,9 @@ struct Routing {
   Tensor sorted_idx, row_map, goff;
 };
 Routing route(const Tensor& ids, int64_t E, bool want_sorted) {
+  // (the kernels read whole words of the ids)
+  require((ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt) && ids.is_contiguous(),
+          "expert ids must be int64 or int32 and contiguous");
   const int64_t n = ids.numel();
   Routing r;
   if (want_sorted) r.sorted_idx = empty({n}, at::kLong, ids);
