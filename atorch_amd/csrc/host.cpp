@@ -34,6 +34,14 @@ void require(bool ok, const char* what) {
   PyErr_SetString(PyExc_AssertionError, what);
   throw py::error_already_set();
 }
+void check_offsets(const Tensor& goff, int64_t E) {
+  require(goff.scalar_type() == at::kLong && goff.numel() == E + 1 && goff.is_contiguous(),
+          "group offsets must be int64 [groups + 1] and contiguous");
+}
+void check_bias(const Tensor& bias, int64_t E, int64_t N) {
+  require(bias.dim() == 2 && bias.size(0) == E && bias.size(1) == N && bias.is_contiguous(),
+          "bias must be [groups, outputs] and contiguous");
+}
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 void on_gpu(const Tensor& t) {
@@ -114,6 +122,7 @@ std::tuple<Tensor, Tensor> permute_tile_quant(const Tensor& x, const Tensor& row
 // (without offsets: one group of all rows)
 Quantised dual(const Tensor& x, const OptTensor& goff, int64_t E, double eps, int64_t ld_t, bool rowwise, bool blocked) {
   const int64_t M = x.size(0), cols = x.size(1);
+  if (goff.has_value()) check_offsets(*goff, E);
   Quantised r = alloc_dual(M, cols, ld_t, rowwise, blocked, x);
   check(aamd_quant_1x128_dual_grouped(ptr(x), dtype_code(x.scalar_type(), true), M, cols, cols, ptr<int64_t>(goff), (int)E,
                                       nullptr, raw<uint8_t>(r.q), raw<float>(r.s), ptr<uint8_t>(r.q_t), ptr<float>(r.s_t),
@@ -124,6 +133,7 @@ Quantised dual(const Tensor& x, const OptTensor& goff, int64_t E, double eps, in
 Quantised permute_dual(const Tensor& x, const Tensor& sorted_idx, int64_t topk, const Tensor& goff, int64_t E, double eps,
                        int64_t ld_t, bool rowwise, bool blocked) {
   const int64_t T = x.size(0), cols = x.size(1), M = sorted_idx.numel();
+  check_offsets(goff, E);
   Quantised r = alloc_dual(M, cols, ld_t, rowwise, blocked, x);
   check(aamd_permute_quant_1x128_dual_grouped(ptr(x), dtype_code(x.scalar_type(), true), T, cols, cols,
                                               ptr<int64_t>(sorted_idx), (int)topk, M, ptr<int64_t>(goff), (int)E, nullptr,
@@ -151,6 +161,7 @@ std::tuple<Quantised, Tensor> act_dual(const Tensor& fc1, const Tensor& dh, bool
                                        bool rowwise, bool blocked, bool keep) {
   const int64_t M = fc1.size(0), width = fc1.size(1), F = glu ? width / 2 : width;
   const int64_t cols = glu && dh.defined() ? width : F;
+  check_offsets(goff, E);
   Quantised r = alloc_dual(M, cols, ld_t, rowwise, blocked, fc1);
   Tensor kept = keep ? empty({M, cols}, at::kBFloat16, fc1) : Tensor();
   int rc;
@@ -184,8 +195,14 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, do
 Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, const OptTensor& goff, const OptTensor& out,
                at::ScalarType out_dtype, const OptTensor& bias) {
   const int64_t M = a.size(0), K = a.size(1), E = b.size(0), N = b.size(1);
-  Tensor c = out.has_value() ? *out : empty({M, N}, out_dtype, a);
   const bool b_tile_scaled = b_s.size(1) == N;
+  require(b.size(2) == K && a.stride(1) == 1 && b.is_contiguous(), "rows and weights must share their contraction length");
+  require(a_s.numel() >= M * (K / kTile) && b_s.numel() >= E * (b_tile_scaled ? N : N / kTile) * (K / kTile) &&
+              a_s.is_contiguous() && b_s.is_contiguous(),
+          "scales do not cover the codes");
+  if (goff.has_value()) check_offsets(*goff, E);
+  if (bias.has_value()) check_bias(*bias, E, N);
+  Tensor c = out.has_value() ? *out : empty({M, N}, out_dtype, a);
   check(aamd_grouped_gemm_fp8_nt(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(b_s), b_tile_scaled,
                                  ptr<int64_t>(goff), (int)E, nullptr, M, N, K, ptr(c), dtype_code(c.scalar_type()), c.stride(0),
                                  ptr(bias), bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
@@ -196,6 +213,10 @@ Tensor gemm_wgrad(const Tensor& dy_t, const Tensor& sdy_t, const Tensor& x_t, co
                   const OptTensor& out, at::ScalarType out_dtype, bool accumulate) {
   const bool blocked = dy_t.dim() == 3;
   const int64_t N = blocked ? dy_t.size(1) : dy_t.size(0), K = blocked ? x_t.size(1) : x_t.size(0), E = goff.numel() - 1;
+  check_offsets(goff, E);
+  require(x_t.dim() == dy_t.dim() && qt_ld(x_t) == qt_ld(dy_t) && sdy_t.numel() >= qt_ld(dy_t) / kTile * N &&
+              sx_t.numel() >= qt_ld(dy_t) / kTile * K,
+          "transposed operands must share their layout and length, with a scale per row and block");
   Tensor c = out.has_value() ? *out : empty({E, N, K}, out_dtype, dy_t);
   check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(dy_t), ptr<float>(sdy_t), ptr<uint8_t>(x_t), ptr<float>(sx_t), qt_ld(dy_t),
                                     blocked, ptr<int64_t>(goff), (int)E, nullptr, N, K, ptr(c), dtype_code(c.scalar_type()),
@@ -320,6 +341,7 @@ Tensor offsets_from_list(const std::vector<int64_t>& counts, at::Device device) 
   return goff;
 }
 Tensor offsets_from_tensor(const Tensor& counts, at::Device device) {
+  require(counts.scalar_type() == at::kLong && counts.is_contiguous(), "rows per group must be int64 and contiguous");
   Tensor goff = at::empty({counts.numel() + 1}, at::TensorOptions().dtype(at::kLong).device(device));
   check(aamd_group_offsets(reinterpret_cast<const int64_t*>(counts.data_ptr()), !counts.is_cuda(), (int)counts.numel(),
                            ptr<int64_t>(goff), stream()));
@@ -354,11 +376,26 @@ OptTensor stack_of(const std::vector<Tensor>& ts) {
 // linear -> activation -> linear on rows grouped by expert.  With `row_map` the rows are the tokens of x in the order
 // of the routing (row_map, and sorted_idx where a backward follows), and the permute happens inside the quantiser.
 // Returns the output and what the backward reads: (out, fc1, qx_t, sx_t, qh_t, sh_t), the last five only with `train`.
+// (x, the codes of the weights [E, N1, H] and [E, H2, F] and the biases fit each other, before anything is launched)
+void check_mlp(const Tensor& x, const Tensor& q1, const Tensor& q2, const OptTensor& b1, const OptTensor& b2, bool glu) {
+  const int64_t E = q1.size(0), n1 = q1.size(1), F = q2.size(2);
+  require(x.dim() == 2 && x.is_contiguous() && q1.dim() == 3 && q2.dim() == 3 && x.size(1) == q1.size(2),
+          "hidden states and first weights must share the hidden size");
+  require(q2.size(0) == E && n1 == (glu ? 2 * F : F), "first and second weights must share the experts and the feed-forward size");
+  if (b1.has_value()) check_bias(*b1, E, n1);
+  if (b2.has_value()) check_bias(*b2, E, q2.size(1));
+}
 using MlpResult = std::tuple<Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
 MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
                       const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
                       const OptTensor& b2, bool glu, bool train) {
   const int64_t E = q1.size(0);
+  check_mlp(x, q1, q2, b1, b2, glu);
+  check_offsets(goff, E);
+  require(!row_map.has_value() || (row_map->scalar_type() == at::kInt && row_map->is_contiguous() && row_map->numel() == x.size(0) * topk),
+          "the row map must be int32 [tokens * topk] and contiguous");
+  require(!row_map.has_value() || !train || (sorted_idx->scalar_type() == at::kLong && sorted_idx->dim() == 1 && sorted_idx->is_contiguous()),
+          "the sorted indices must be int64, of one dimension and contiguous");
   const int64_t M = row_map.has_value() ? row_map->numel() : x.size(0);
   Quantised qx;
   const int64_t ld_t = padded_bound(M, E);
@@ -384,6 +421,10 @@ MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sort
 // `train`, the experts' output and what mlp_forward returns for the backward.
 py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids, int64_t topk, const Tensor& q1, const Tensor& s1,
                           const Tensor& q2, const Tensor& s2, const OptTensor& b1, const OptTensor& b2, bool glu, bool train) {
+  check_mlp(x, q1, q2, b1, b2, glu);
+  require(ids.numel() == x.size(0) * topk && probs.dim() == 2 && probs.size(0) == x.size(0) && probs.size(1) == topk &&
+              probs.is_contiguous() && q2.size(1) == x.size(1),
+          "router weights and choices are [tokens, topk], and the experts return the hidden size");
   Routing r = route(ids, q1.size(0), true);
   MlpResult m = mlp_forward(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train);
   Tensor& y = std::get<0>(m);
@@ -397,6 +438,7 @@ py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids,
 std::tuple<Quantised, Tensor> dual_with_sums(int what, const Tensor& x, const Tensor& dh, const Tensor& goff, int64_t E,
                                              int64_t ld_t, double eps, at::ScalarType dtype) {
   const int64_t M = x.size(0), width = x.size(1);
+  check_offsets(goff, E);
   Quantised r = alloc_dual(M, width, ld_t, true, true, x);
   Tensor tiles = empty({ld_t / kTile, width}, at::kFloat, x), sums = empty({E, width}, dtype, x);
   check(aamd_dual_grouped_with_sums(what, ptr(x), raw(dh), M, width, ptr<int64_t>(goff), (int)E, ptr<uint8_t>(r.q), ptr<float>(r.s),
@@ -413,6 +455,9 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> mlp_backward(
     const Tensor& s2, bool glu, bool transpose_w1, bool want_b1, bool want_b2, at::ScalarType x_dtype, at::ScalarType w1_dtype,
     at::ScalarType w2_dtype) {
   const int64_t E = goff.numel() - 1, ld_t = qt_ld(qx_t);
+  check_offsets(goff, E);
+  require(dy.size(0) == fc1.size(0) && dy.is_contiguous() && fc1.size(1) == q1_t.size(2) && q2.size(1) * (glu ? 2 : 1) == fc1.size(1),
+          "the gradient, the saved activations and the weights do not fit each other");
   Quantised qdy, qg;
   Tensor db1, db2;
   if (want_b2) std::tie(qdy, db2) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, ld_t, 0.0, at::kBFloat16);
@@ -442,6 +487,10 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> linear_forward(const Tensor& x,
                                                                 const OptTensor& bias, at::ScalarType out_dtype, double eps,
                                                                 bool train) {
   const int64_t E = qw.size(0);
+  require(x.dim() == 2 && x.is_contiguous() && qw.dim() == 3 && x.size(1) == qw.size(2), "GEMM not possible");
+  require(goff_in.has_value() || (int64_t)splits.size() == E, "Number of splits should match number of GEMMs.");
+  if (goff_in.has_value()) check_offsets(*goff_in, E);
+  if (bias.has_value()) check_bias(*bias, E, qw.size(1));
   Tensor goff = goff_in.has_value() ? *goff_in : offsets_from_list(splits, x.device());
   Quantised q;
   if (train) q = dual(x, goff, E, eps, padded_bound(x.size(0), E), true, true);
@@ -455,6 +504,7 @@ std::tuple<Tensor, Tensor, OptTensor> linear_backward(const Tensor& dy, const Te
                                                       const OptTensor& main_grad, at::ScalarType dw_dtype, bool accumulate,
                                                       double eps, bool want_bias) {
   const int64_t E = qw_t.size(0);
+  check_offsets(goff, E);
   Quantised q;
   Tensor db;
   if (want_bias) std::tie(q, db) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, qt_ld(qx_t), eps, at::kFloat);

@@ -48,3 +48,94 @@ def test_expert_ids(dtype):
     _sound(_layer, ids=torch.zeros((T, K), dtype=dtype))
     _sound(_host().moe_preprocess, torch.zeros(T * K, dtype=dtype), E, True)
     _refused(_host().moe_preprocess, torch.zeros(T * K, 2, dtype=dtype)[:, 0], E, True)
+
+
+@pytest.mark.parametrize("train", [True, False])
+@pytest.mark.parametrize("glu", [True, False])
+def test_layer_sizes_that_do_not_fit(glu, train):
+    n1 = 2 * F if glu else F
+    kw = dict(q1=(E, n1, H), glu=glu, train=train)
+    _sound(_layer, **kw, b1=(E, n1), b2=(E, H))
+    _refused(_layer, **kw, x=(T, 2 * H))  # wider rows than the weights'
+    _refused(_layer, **kw, q2=(E, H, 2 * F))  # another feed-forward size
+    _refused(_layer, **kw, q2=(E + 1, H, F))
+    _refused(_layer, **kw, q2=(E, 2 * H, F))
+    _refused(_layer, **kw, b1=(E, n1 // 2))
+    _refused(_layer, **kw, b1=(E - 1, n1))
+    _refused(_layer, **kw, b2=(E, 2 * H))
+    _refused(_layer, **kw, b2=torch.zeros((H, E), dtype=BF16).t())
+    _refused(_layer, **kw, probs=(T, K - 1))
+    _refused(_layer, **kw, probs=(T - 1, K))
+    _refused(_layer, **kw, topk=K + 1)
+    _refused(_layer, **kw, ids=torch.zeros((T + 1, K), dtype=torch.int64))
+
+
+def _offsets(groups=E, dtype=torch.int64):
+    return torch.zeros(groups + 1, dtype=dtype)
+
+
+@pytest.mark.parametrize("train", [True, False])
+def test_mlp_offsets_and_routing_that_do_not_fit(train):
+    def mlp(goff, row_map=None, sorted_idx=None, x=(T, H)):
+        return _host().mlp_forward(torch.zeros(x, dtype=BF16), goff, sorted_idx, row_map, K, *_codes(E, 2 * F, H), *_codes(E, H, F),
+                                   None, None, True, train)  # fmt: skip
+
+    routing = lambda n=T * K, m=torch.int32, s=torch.int64: (torch.zeros(n, dtype=m), torch.zeros(n, dtype=s))  # noqa: E731
+    _sound(mlp, _offsets())
+    _sound(mlp, _offsets(), *routing())
+    for goff in (_offsets(E - 1), _offsets(E + 1), _offsets(dtype=torch.int32)):
+        _refused(mlp, goff)
+        _refused(mlp, goff, *routing())
+    _refused(mlp, _offsets(), x=(T, 2 * H))
+    _refused(mlp, _offsets(), *routing(T * K + K))
+    _refused(mlp, _offsets(), *routing(m=torch.int64))
+    if train:  # (the forward alone reads the map)
+        _refused(mlp, _offsets(), *routing(s=torch.int32))
+
+
+def test_linear_and_gemm_sizes_that_do_not_fit():
+    h, N = _host(), 384
+    codes, scales = _codes(E, N, H)
+    row = lambda m, k: (torch.zeros((m, k), dtype=torch.uint8).view(FP8), torch.ones(m, k // TILE))  # noqa: E731
+    nt = lambda a, goff, bias=None, s=scales: h.gemm_nt(*a, codes, s, goff, None, BF16, bias)  # noqa: E731
+    _sound(nt, row(T, H), _offsets(), torch.zeros(E, N))
+    _refused(nt, row(T, 2 * H), _offsets())
+    _refused(nt, row(T, H), _offsets(E - 1))
+    _refused(nt, row(T, H), _offsets(), torch.zeros(E, 2 * N))
+    _refused(nt, row(T, H), _offsets(), s=scales[: E - 1])
+    _refused(nt, (row(T, H)[0], row(T - 1, H)[1]), _offsets())
+
+    def linear(x=(T, H), goff=None, splits=(), bias=None, train=True):
+        return h.linear_forward(torch.zeros(x, dtype=BF16), goff, list(splits), codes, scales, bias, BF16, 0.0, train)
+
+    for train in (True, False):
+        _sound(linear, goff=_offsets(), train=train)
+        _refused(linear, goff=_offsets(E + 1), train=train)
+        _refused(linear, splits=[T], train=train)
+        _refused(linear, x=(T, 2 * H), goff=_offsets(), train=train)
+        _refused(linear, goff=_offsets(), bias=torch.zeros(E, H), train=train)
+    _refused(h.offsets_from_tensor, torch.zeros(E, dtype=torch.int32), torch.device("cuda"))
+
+
+def test_dual_quantisers_with_offsets_of_another_length():
+    h, x = _host(), torch.zeros((T, H), dtype=BF16)
+    si = torch.zeros(T, dtype=torch.int64)
+    calls = [lambda g: h.dual(x, g, E, 0.0, 640, True, True), lambda g: h.permute_dual(x, si, 1, g, E, 0.0, 640, True, True),
+             lambda g: h.act_dual(x, None, True, g, E, 640, True, True, False),
+             lambda g: h.dual_with_sums(0, x, None, g, E, 640, 0.0, F32)]  # fmt: skip
+    for call in calls:
+        _sound(call, _offsets())
+        _refused(call, _offsets(E - 1))
+        _refused(call, _offsets(dtype=torch.int32))
+
+
+def test_weight_gradient_operands_that_do_not_fit():
+    h, ld = _host(), 512
+    op = lambda rows, n=ld: (torch.zeros((n // TILE, rows, TILE), dtype=torch.uint8).view(FP8), torch.ones(n // TILE, rows))  # noqa: E731
+    wgrad = lambda a, b, goff: h.gemm_wgrad(*a, *b, goff, None, F32, False)  # noqa: E731
+    _sound(wgrad, op(F), op(H), _offsets())
+    _refused(wgrad, op(F), op(H, ld // 2), _offsets())
+    _refused(wgrad, (op(F)[0], op(F, ld // 2)[1]), op(H), _offsets())
+    _refused(wgrad, op(F), op(H), _offsets(dtype=torch.int32))
+    rows = (torch.zeros((F, ld), dtype=torch.uint8).view(FP8), torch.ones(ld // TILE, F))
+    _refused(wgrad, rows, op(H), _offsets())
