@@ -394,9 +394,11 @@ MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sort
   check_offsets(goff, E);
   require(!row_map.has_value() || (row_map->scalar_type() == at::kInt && row_map->is_contiguous() && row_map->numel() == x.size(0) * topk),
           "the row map must be int32 [tokens * topk] and contiguous");
+  require(row_map.has_value() == sorted_idx.has_value() && (!row_map.has_value() || sorted_idx->numel() <= row_map->numel()),
+          "a routing has a row map and the sorted indices of the rows that are kept");
   require(!row_map.has_value() || !train || (sorted_idx->scalar_type() == at::kLong && sorted_idx->dim() == 1 && sorted_idx->is_contiguous()),
           "the sorted indices must be int64, of one dimension and contiguous");
-  const int64_t M = row_map.has_value() ? row_map->numel() : x.size(0);
+  const int64_t M = row_map.has_value() ? sorted_idx->numel() : x.size(0);  // (fewer than the map's entries where copies were dropped)
   Quantised qx;
   const int64_t ld_t = padded_bound(M, E);
   if (train)

@@ -89,6 +89,9 @@ def test_mlp_offsets_and_routing_that_do_not_fit(train):
     _refused(mlp, _offsets(), x=(T, 2 * H))
     _refused(mlp, _offsets(), *routing(T * K + K))
     _refused(mlp, _offsets(), *routing(m=torch.int64))
+    _sound(mlp, _offsets(), routing()[0], routing(T * K - 1)[1])  # a dropped copy
+    _refused(mlp, _offsets(), routing()[0], routing(T * K + 1)[1])
+    _refused(mlp, _offsets(), routing()[0])
     if train:  # (the forward alone reads the map)
         _refused(mlp, _offsets(), *routing(s=torch.int32))
 
