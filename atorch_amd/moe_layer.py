@@ -157,7 +157,8 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         """Nothing happens between the experts and the combine: the layer is one function, one native call per
         direction."""
         assert x.dtype == torch.bfloat16, "the fused activation kernels read bf16"
-        assert probs.shape == top_experts.shape == (x.shape[0], self.topk), "router weights and choices are [tokens, topk]"
+        T = x.shape[0]  # (choices may also come flattened, as other MoE layers pass them)
+        assert probs.shape == (T, self.topk) and top_experts.numel() == T * self.topk, "router weights and choices are [tokens, topk]"
         w1, w2 = self.scale_grad(self._weight("w1")), self.scale_grad(self._weight("w2"))
         v1 = self.scale_grad(self._weight("v1")) if self.has_v1() else None
         b1, b2 = (self._weight("b1"), self._weight("b2")) if self.use_bias else (None, None)

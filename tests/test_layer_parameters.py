@@ -111,3 +111,19 @@ def test_switched_off_bias_and_forbidden_combinations(monkeypatch):
     layer.use_swiglu = layer.use_bias = True
     with pytest.raises(AssertionError):
         run()
+
+
+@pytest.mark.parametrize("shape", [(8, 2), (16,), (16, 1), (4, 2, 2)])
+def test_router_choices_of_any_shape(monkeypatch, shape):
+    """What counts is one choice per token and slot, token by token (grouped_gemm_moe.py:650-652)."""
+    layer, seen, run = _layer(monkeypatch)
+    x, (idx, probs) = randn_bf16((8, 256), 2), topk_routing(8, 4, 2, seed=1)
+    layer(x, probs.bfloat16(), idx.view(shape))
+    assert seen
+    seen.clear()
+    for bad in (idx[:7], idx[:, :1], torch.cat([idx, idx[:1]])):
+        with pytest.raises(AssertionError):
+            layer(x, probs.bfloat16(), bad)
+    with pytest.raises(AssertionError):
+        layer(x, probs.bfloat16()[:, :1], idx)
+    assert not seen
