@@ -153,9 +153,16 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         p = self._parameters
         return p[name] if name in p else getattr(self, name)
 
+    def _nothing_between(self, dispatcher):
+        """True if nothing happens between the experts and the combine and both ends are this package's: the dropout is the
+        identity, nobody listens to it, and dispatcher and dropout are the modules the constructor made."""
+        drop = self._modules.get("dropout")
+        return (type(dispatcher) is MoEAllToAllTokenDispatcher and type(drop) is torch.nn.Dropout
+                and not (drop.training and drop.p > 0) and not drop._forward_hooks and not drop._forward_pre_hooks
+                and not drop._backward_hooks and not drop._backward_pre_hooks)  # fmt: skip
+
     def _forward_fused(self, x, probs, top_experts, is_first_microbatch):
-        """Nothing happens between the experts and the combine: the layer is one function, one native call per
-        direction."""
+        """The layer as one function, one native call per direction."""
         assert x.dtype == torch.bfloat16, "the fused activation kernels read bf16"
         T = x.shape[0]  # (choices may also come flattened, as other MoE layers pass them)
         assert probs.shape == (T, self.topk) and top_experts.numel() == T * self.topk, "router weights and choices are [tokens, topk]"
@@ -183,7 +190,7 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         if x.shape[0] == 0:
             return hidden_states.clone()
         d.hidden_shape, d.probs = shape, expert_weights
-        if se_fn1 is None and se_fn2 is None and not (self.training and self.output_dropout_prob > 0):
+        if se_fn1 is None and se_fn2 is None and self._nothing_between(d):
             out = self._forward_fused(x, expert_weights, top_experts, is_first_microbatch)
             return out if len(shape) == 2 else out.view(shape)
         # dispatch: only the routing is computed here; the permute itself happens inside the first quantiser

@@ -127,3 +127,52 @@ def test_router_choices_of_any_shape(monkeypatch, shape):
     with pytest.raises(AssertionError):
         layer(x, probs.bfloat16()[:, :1], idx)
     assert not seen
+
+
+def _stop(*args, **kw):
+    raise RuntimeError("composite")
+
+
+def _dropout_in_eval(layer):
+    layer.eval()
+    layer.dropout.p = 0.5
+    layer.dropout.train()  # sampling at inference
+
+
+def _other_probability(layer):
+    layer.dropout.p = 0.5  # the module's own, not the constructor's argument, is what counts
+
+
+def _other_module(layer):
+    layer.dropout = torch.nn.AlphaDropout(0.5)
+
+
+def _listener(layer):
+    layer.dropout.register_forward_hook(lambda m, args, out: None)
+
+
+def _own_dispatcher(layer):
+    from atorch_amd.token_dispatcher import MoEAllToAllTokenDispatcher
+
+    class Own(MoEAllToAllTokenDispatcher):
+        pass
+
+    layer.token_dispatcher = Own(4, [0, 1, 2, 3], 4, 2, False, False)
+
+
+@pytest.mark.parametrize("change", [_dropout_in_eval, _other_probability, _other_module, _listener, _own_dispatcher])
+def test_whatever_sits_between_experts_and_combine_runs(monkeypatch, change):
+    """The one-call form has no place for it: the composite of dispatch, experts, dropout and combine runs."""
+    layer, seen, run = _layer(monkeypatch)
+    run()
+    assert seen
+    layer.output_dropout_prob = 0.3  # (without meaning after construction)
+    run()
+    assert seen
+    change(layer)
+    monkeypatch.setattr(type(layer), "_mlp", _stop)
+    monkeypatch.setattr(layer.token_dispatcher, "preprocess", lambda ids: None)
+    monkeypatch.setattr(layer.token_dispatcher, "dispatch", lambda: None)
+    with pytest.raises(RuntimeError, match="composite"):
+        run()
+    assert not seen
