@@ -209,18 +209,30 @@ Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor
   return c;
 }
 
+void check_wgrad(const Tensor& dy_t, const Tensor& sdy_t, const Tensor& x_t, const Tensor& sx_t, const Tensor& goff, int64_t N, int64_t K) {
+  const int64_t ld_t = qt_ld(dy_t);
+  check_offsets(goff, goff.numel() - 1);
+  require(x_t.dim() == dy_t.dim() && qt_ld(x_t) == ld_t && dy_t.numel() == N * ld_t && x_t.numel() == K * ld_t &&
+              sdy_t.numel() >= ld_t / kTile * N && sx_t.numel() >= ld_t / kTile * K,
+          "transposed operands must share their layout and length, with a scale per row and block");
+}
+// dw[g] (+)= dY_g^T X_g into matrices [N, K] that lie `stride` elements apart
+void wgrad_into(const Tensor& dy_t, const Tensor& sdy_t, const Tensor& x_t, const Tensor& sx_t, const Tensor& goff, int64_t N, int64_t K,
+                void* dw, at::ScalarType dtype, int64_t stride, bool accumulate) {
+  check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(dy_t), ptr<float>(sdy_t), ptr<uint8_t>(x_t), ptr<float>(sx_t), qt_ld(dy_t),
+                                    dy_t.dim() == 3, ptr<int64_t>(goff), (int)(goff.numel() - 1), nullptr, N, K, dw,
+                                    dtype_code(dtype), stride, accumulate, stream()));
+}
 Tensor gemm_wgrad(const Tensor& dy_t, const Tensor& sdy_t, const Tensor& x_t, const Tensor& sx_t, const Tensor& goff,
                   const OptTensor& out, at::ScalarType out_dtype, bool accumulate) {
   const bool blocked = dy_t.dim() == 3;
-  const int64_t N = blocked ? dy_t.size(1) : dy_t.size(0), K = blocked ? x_t.size(1) : x_t.size(0), E = goff.numel() - 1;
-  check_offsets(goff, E);
-  require(x_t.dim() == dy_t.dim() && qt_ld(x_t) == qt_ld(dy_t) && sdy_t.numel() >= qt_ld(dy_t) / kTile * N &&
-              sx_t.numel() >= qt_ld(dy_t) / kTile * K,
-          "transposed operands must share their layout and length, with a scale per row and block");
+  const int64_t N = dy_t.size(blocked), K = x_t.size(blocked), E = goff.numel() - 1;
+  check_wgrad(dy_t, sdy_t, x_t, sx_t, goff, N, K);
+  require(!out.has_value() || (out->dim() == 3 && out->size(0) == E && out->size(1) == N && out->size(2) == K &&
+                               out->stride(2) == 1 && out->stride(1) == K),
+          "the output must be [groups, N, K] with dense matrices");
   Tensor c = out.has_value() ? *out : empty({E, N, K}, out_dtype, dy_t);
-  check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(dy_t), ptr<float>(sdy_t), ptr<uint8_t>(x_t), ptr<float>(sx_t), qt_ld(dy_t),
-                                    blocked, ptr<int64_t>(goff), (int)E, nullptr, N, K, ptr(c), dtype_code(c.scalar_type()),
-                                    E > 1 ? c.stride(0) : N * K, accumulate, stream()));
+  wgrad_into(dy_t, sdy_t, x_t, sx_t, goff, N, K, ptr(c), c.scalar_type(), E > 1 ? c.stride(0) : N * K, accumulate);
   return c;
 }
 
@@ -372,6 +384,29 @@ OptTensor stack_of(const std::vector<Tensor>& ts) {
   return t0.detach().as_strided(sizes, strides);
 }
 
+// Where tensors of n elements lie that are dense and equally far apart in memory, in one storage or in several (gradient
+// buffers that also hold the biases' gradients, tensors taken one by one from the allocator); nothing else fits a
+// kernel's base address and stride.  Aligned for the kernels' 16-byte accesses.
+struct Spaced {
+  void* base;
+  int64_t stride;  // elements
+};
+std::optional<Spaced> spaced(const std::vector<Tensor>& ts, int64_t n) {
+  if (ts.empty() || n == 0) return {};
+  const Tensor& t0 = ts[0];
+  auto* const base = static_cast<char*>(t0.data_ptr());
+  const int64_t size = t0.element_size();
+  const int64_t step = ts.size() > 1 ? static_cast<char*>(ts[1].data_ptr()) - base : n * size;
+  if (step < n * size || step % (8 * size) != 0 || reinterpret_cast<uintptr_t>(base) % 16 != 0) return {};
+  for (size_t i = 0; i < ts.size(); i++) {
+    const Tensor& t = ts[i];
+    if (!t.is_contiguous() || t.numel() != n || t.scalar_type() != t0.scalar_type() || t.device() != t0.device() ||
+        static_cast<char*>(t.data_ptr()) != base + (int64_t)i * step)
+      return {};
+  }
+  return Spaced{base, step / size};
+}
+
 // ---- the expert MLP --------------------------------------------------------------------------
 // linear -> activation -> linear on rows grouped by expert.  With `row_map` the rows are the tokens of x in the order
 // of the routing (row_map, and sorted_idx where a backward follows), and the permute happens inside the quantiser.
@@ -499,20 +534,33 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> linear_forward(const Tensor& x,
   else std::tie(q.q, q.s) = tile_quant(x, eps);
   return {gemm_nt(q.q, q.s, qw, sw, goff, {}, out_dtype, bias), goff, opt(q.q_t), opt(q.s_t)};
 }
-// The gradients: (dx, dw, db); dw goes to `main_grad` (added or written over) where there is one; db [E, N] in fp32
-// where asked for (bf16 gradients only).
-std::tuple<Tensor, Tensor, OptTensor> linear_backward(const Tensor& dy, const Tensor& goff, const Tensor& qx_t, const Tensor& sx_t,
-                                                      const Tensor& qw_t, const Tensor& sw_t, at::ScalarType dx_dtype,
-                                                      const OptTensor& main_grad, at::ScalarType dw_dtype, bool accumulate,
-                                                      double eps, bool want_bias) {
-  const int64_t E = qw_t.size(0);
+// The gradients: (dx, dw, db), db [E, N] in fp32 where asked for (bf16 gradients only).  `mains`: the weights' gradient
+// buffers; where they are equally far apart the gradient is added to them (`accumulate`) or written over them and dw is
+// empty, else it comes in a buffer of its own.
+std::tuple<Tensor, OptTensor, OptTensor> linear_backward(const Tensor& dy, const Tensor& goff, const Tensor& qx_t, const Tensor& sx_t,
+                                                         const Tensor& qw_t, const Tensor& sw_t, at::ScalarType dx_dtype,
+                                                         const std::optional<std::vector<Tensor>>& mains, at::ScalarType dw_dtype,
+                                                         bool accumulate, double eps, bool want_bias) {
+  const int64_t E = qw_t.size(0), K = qw_t.size(1), N = qw_t.size(2);
   check_offsets(goff, E);
+  std::optional<Spaced> main;
+  at::ScalarType main_dtype = at::kFloat;
+  if (mains.has_value()) {
+    require((int64_t)mains->size() == E, "one gradient buffer per weight");
+    for (const Tensor& m : *mains) require(m.numel() == N * K, "a gradient buffer has another size than its weight");
+    main_dtype = mains->front().scalar_type();
+    if (main_dtype == at::kFloat || main_dtype == at::kBFloat16) main = spaced(*mains, N * K);
+  }
   Quantised q;
   Tensor db;
   if (want_bias) std::tie(q, db) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, qt_ld(qx_t), eps, at::kFloat);
   else q = dual(dy, goff, E, eps, qt_ld(qx_t), true, true);
   Tensor dx = gemm_nt(q.q, q.s, qw_t, sw_t, goff, {}, dx_dtype, {});
-  return {dx, gemm_wgrad(q.q_t, q.s_t, qx_t, sx_t, goff, main_grad, dw_dtype, accumulate), opt(db)};
+  if (!main.has_value()) return {dx, gemm_wgrad(q.q_t, q.s_t, qx_t, sx_t, goff, {}, dw_dtype, false), opt(db)};
+  on_gpu(mains->front());
+  check_wgrad(q.q_t, q.s_t, qx_t, sx_t, goff, N, K);
+  wgrad_into(q.q_t, q.s_t, qx_t, sx_t, goff, N, K, main->base, main_dtype, main->stride, accumulate);
+  return {dx, {}, opt(db)};
 }
 
 QuantTuple pack(const Quantised& r) { return {opt(r.q), opt(r.s), r.q_t, r.s_t}; }
@@ -555,6 +603,10 @@ PYBIND11_MODULE(_host, m) {
   m.def("offsets_from_list", &offsets_from_list);
   m.def("offsets_from_tensor", &offsets_from_tensor);
   m.def("stack_of", &stack_of);
+  m.def("spaced", [](const std::vector<Tensor>& ts, int64_t n) {
+    const auto s = spaced(ts, n);
+    return s.has_value() ? std::optional(std::make_tuple(reinterpret_cast<uintptr_t>(s->base), s->stride)) : std::nullopt;
+  });
   m.def("linear_forward", &linear_forward);
   m.def("linear_backward", &linear_backward);
   m.def("mlp_forward", &mlp_forward);

@@ -142,3 +142,7 @@ def test_weight_gradient_operands_that_do_not_fit():
     _refused(wgrad, op(F), op(H), _offsets(dtype=torch.int32))
     rows = (torch.zeros((F, ld), dtype=torch.uint8).view(FP8), torch.ones(ld // TILE, F))
     _refused(wgrad, rows, op(H), _offsets())
+    into = lambda *shape: h.gemm_wgrad(*op(F), *op(H), _offsets(), torch.zeros(shape), F32, True)  # noqa: E731
+    _sound(into, E, F, H)
+    for shape in ((E - 1, F, H), (E, F - 1, H), (E, F, 2 * H), (E, F * H)):
+        _refused(into, *shape)
