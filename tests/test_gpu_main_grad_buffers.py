@@ -64,7 +64,7 @@ def test_what_counts_as_equally_far_apart():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("layout", LAYOUTS)
 def test_main_grad_buffers(dev, layout, dtype):
     from atorch_amd.grouped_linear import ATorchGroupedLinear
@@ -85,6 +85,7 @@ def test_main_grad_buffers(dev, layout, dtype):
             results.append([m.clone() for m in mains])
     for got, want in zip(results[3:], results[:3]):
         for i in range(E):
+            # (also from a buffer of its own: the sum is fp32 and rounded once)
             assert torch.equal(got[i].view(N, K), want[i])
     assert gaps is None or torch.all(gaps == 0.25)
     if layout in (_with_biases, _flat):  # in place: no more memory than dense buffers ask for
