@@ -8,6 +8,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_strided.h>
+#include <ATen/ops/stack.h>
 #include <ATen/ops/zeros.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/utils/pybind.h>
@@ -179,16 +180,6 @@ std::tuple<Quantised, Tensor> act_dual(const Tensor& fc1, const Tensor& dh, bool
                                                   ptr<float>(r.s_t), ld_t, blocked, stream());
   check(rc);
   return {r, kept};
-}
-
-std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose) {
-  const int64_t E = w.size(0), N = w.size(1), K = w.size(2);
-  Tensor q = empty({E, N, K}, kFp8, w), s = empty({E, N / kTile, K / kTile}, at::kFloat, w);
-  Tensor q_t = transpose ? empty({E, K, N}, kFp8, w) : Tensor();
-  Tensor s_t = transpose ? empty({E, K / kTile, N / kTile}, at::kFloat, w) : Tensor();
-  check(aamd_quant_128x128(ptr(w), dtype_code(w.scalar_type(), true), E, N, K, E > 1 ? w.stride(0) : N * K, ptr<uint8_t>(q),
-                           ptr<float>(s), raw<uint8_t>(q_t), raw<float>(s_t), (float)eps, stream()));
-  return {q, s, opt(q_t), opt(s_t)};
 }
 
 // ---- grouped GEMMs ---------------------------------------------------------------------------
@@ -407,6 +398,50 @@ std::optional<Spaced> spaced(const std::vector<Tensor>& ts, int64_t n) {
   return Spaced{base, step / size};
 }
 
+// 128x128 codes of weights [N, K] into stacked outputs
+struct BlockQuantised {
+  Tensor q, s, q_t, s_t;
+  BlockQuantised(int64_t E, int64_t N, int64_t K, bool transpose, const Tensor& like)
+      : q(empty({E, N, K}, kFp8, like)), s(empty({E, N / kTile, K / kTile}, at::kFloat, like)) {
+    if (!transpose) return;
+    q_t = empty({E, K, N}, kFp8, like);
+    s_t = empty({E, K / kTile, N / kTile}, at::kFloat, like);
+  }
+  void run(const void* w, at::ScalarType dtype, int64_t first, int64_t E, int64_t stride, double eps) {
+    const int64_t N = q.size(1), K = q.size(2), at = first * N * K, at_s = first * (N / kTile) * (K / kTile);
+    check(aamd_quant_128x128(w, dtype_code(dtype, true), E, N, K, stride, ptr<uint8_t>(q) + at, ptr<float>(s) + at_s,
+                             q_t.defined() ? ptr<uint8_t>(q_t) + at : nullptr, s_t.defined() ? ptr<float>(s_t) + at_s : nullptr,
+                             (float)eps, stream()));
+  }
+  std::tuple<Tensor, Tensor, OptTensor, OptTensor> get() const { return {q, s, opt(q_t), opt(s_t)}; }
+};
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose) {
+  const int64_t E = w.size(0), N = w.size(1), K = w.size(2);
+  BlockQuantised r(E, N, K, transpose, w);
+  r.run(ptr(w), w.scalar_type(), 0, E, E > 1 ? w.stride(0) : N * K, eps);
+  return r.get();
+}
+// The same from separate tensors of one shape: in one launch where they are equally far apart; else in one launch each or,
+// small ones, from a copy (us, the one launch / copied / one launch each: 60 x 512 x 512 13 / 28 / 232, 60 x 1024 x 1024
+// 44 / 94 / 246, 8 x 1024 x 4096 24 / 51 / 39, 64 x 1408 x 2048 126 / 363 / 290, 8 x 28672 x 4096 661 / 1949 / 702).
+constexpr int64_t kWeightOfItsOwn = (int64_t)1 << 21;  // elements
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant_list(const std::vector<Tensor>& ws, double eps, bool transpose) {
+  require(!ws.empty() && ws[0].dim() == 2, "weights must be matrices");
+  const int64_t E = (int64_t)ws.size(), N = ws[0].size(0), K = ws[0].size(1);
+  bool direct = N * K >= kWeightOfItsOwn;
+  for (const Tensor& w : ws) {
+    require(w.sizes() == ws[0].sizes() && w.scalar_type() == ws[0].scalar_type(), "weights must share shape and type");
+    direct = direct && w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+  }
+  const auto at = spaced(ws, N * K);
+  if (!at.has_value() && !direct) return block_quant(at::stack(ws), eps, transpose);
+  BlockQuantised r(E, N, K, transpose, ws[0]);
+  if (at.has_value()) r.run(at->base, ws[0].scalar_type(), 0, E, at->stride, eps);
+  else
+    for (int64_t e = 0; e < E; e++) r.run(ptr(ws[e]), ws[e].scalar_type(), e, 1, N * K, eps);
+  return r.get();
+}
+
 // ---- the expert MLP --------------------------------------------------------------------------
 // linear -> activation -> linear on rows grouped by expert.  With `row_map` the rows are the tokens of x in the order
 // of the routing (row_map, and sorted_idx where a backward follows), and the permute happens inside the quantiser.
@@ -589,6 +624,7 @@ PYBIND11_MODULE(_host, m) {
     return std::make_tuple(r.q, r.s, r.q_t, r.s_t, sums);
   });
   m.def("block_quant", &block_quant);
+  m.def("block_quant_list", &block_quant_list);
   m.def("gemm_nt", &gemm_nt);
   m.def("gemm_wgrad", &gemm_wgrad);
   m.def("transpose_scales", &transpose_scales);
