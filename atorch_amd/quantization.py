@@ -90,6 +90,20 @@ class WeightCodeStack:
         return self.whole and len(caches) == len(self.members) and all(map(operator.is_, caches, self.members))
 
 
+class _CodeField:
+    """A field of ``QuantizeResultCache``: tensor ``k`` of the cache's own four, or its place in the stack."""
+
+    def __init__(self, k: int):
+        self.k = k
+
+    def __get__(self, cache, owner=None) -> Optional[torch.Tensor]:
+        return None if cache is None else cache._get(self.k)  # (the class attribute is the field's default)
+
+    def __set__(self, cache, value: Optional[torch.Tensor]):
+        cache._set(self.k, value)
+
+
+@dataclass
 class QuantizeResultCache:
     """Per-weight cache of the fp8 copies between microbatches
     (quantized_grouped_linear.py:121-129, 467-470).
@@ -98,13 +112,16 @@ class QuantizeResultCache:
     slices are made when somebody asks for them (the fused path reads the stack itself, and four views per expert and
     call are most of its host time)."""
 
-    __slots__ = ("_own", "stack", "index")
+    data: Optional[torch.Tensor] = _CodeField(0)
+    scale: Optional[torch.Tensor] = _CodeField(1)
+    data_t: Optional[torch.Tensor] = _CodeField(2)
+    scale_t: Optional[torch.Tensor] = _CodeField(3)
 
-    def __init__(self, data: Optional[torch.Tensor] = None, scale: Optional[torch.Tensor] = None,
-                 data_t: Optional[torch.Tensor] = None, scale_t: Optional[torch.Tensor] = None):
-        self._own = [data, scale, data_t, scale_t]
-        self.stack: Optional[WeightCodeStack] = None
-        self.index = 0
+    def __new__(cls, *args, **kw):
+        self = super().__new__(cls)
+        self._own = [None, None, None, None]
+        self.stack, self.index = None, 0
+        return self
 
     def point_to(self, stack: "WeightCodeStack", index: int):
         """Use entry ``index`` of ``stack``."""
@@ -125,11 +142,6 @@ class QuantizeResultCache:
             self.stack.whole = False
             self.stack = None
         self._own[k] = value
-
-    data = property(lambda self: self._get(0), lambda self, v: self._set(0, v))
-    scale = property(lambda self: self._get(1), lambda self, v: self._set(1, v))
-    data_t = property(lambda self: self._get(2), lambda self, v: self._set(2, v))
-    scale_t = property(lambda self: self._get(3), lambda self, v: self._set(3, v))
 
     def to_qresult(self) -> QuantizeResult:
         return QuantizeResult(self.data, self.scale, self.data_t, self.scale_t)
