@@ -1235,11 +1235,13 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
 //     split form 2.1 and 0.45; and no less than a wave's own chain of every fourth (eighth) step;
 //   - and none can beat the weights' stream from memory, 5.2 to 6.2 TB/s.
 // Token tiles are counted as the groups' expected number (their sizes are known on the device only): one per group with
-// few rows, half a tile more than the rows fill with many.  Over those launches the kernel taken is 2.4 % slower than the
-// best of the four (geometric mean; 8.4 % with a first fit that priced the few-rows kernel without its fixed cost per
-// block and the small tiles too high).  Us, that fit -> this one: one group of 14441 rows, 5504 x 640 200 -> 91; 64 groups,
-// 8591 rows, 16256 x 768 372 -> 195; 4 groups, 2498 rows, 8832 x 512 51 -> 30; 64 groups, 10168 rows, 1536 x 9088: the
-// 256x256 tiles instead of the small ones.
+// few rows, half a tile more than the rows fill with many.  Over those launches, the ones the fit was made from, the kernel
+// taken is 2.4 % slower than the best of the four (geometric mean).  They repeat one launch on the same operands, which then
+// come from a cache, so the estimates rank the kernels better than they give their times: in a pass over new operands the
+// launches of a few microseconds take longer (estimated -> traced: 4 groups of 512 rows, 1024 x 512 7.9 -> 11.3; 8 groups of
+// 125 rows on the kernel for few rows 15.8 -> 25.5, on the small tiles 12.7 -> 19.0).  What they decide, us, the 256x256 tiles
+// or the kernel for few rows priced wrong -> this fit: one group of 14441 rows, 5504 x 640 200 -> 91; 64 groups, 8591 rows,
+// 16256 x 768 372 -> 195; 4 groups, 2498 rows, 8832 x 512 51 -> 30.
 enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3 };
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return g_opt.tile == 1 && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
@@ -1260,7 +1262,13 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   const double large = nkb < 8 ? 1e30 : std::max(loop_l, weights / 5.2);
   const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_p = token_tiles(32) * (double)(N / 32);
   const double few = std::max({4.5 + 1e-3 * blocks_f * (1.06 * n + 2.1), 1.5 + 1.1 * std::ceil(n / 4.0), weights / 6.2});
-  // (the split form where the length of a wave's contraction is what counts: few workgroups, or a long contraction)
+  // The split form where the length of a wave's contraction is what counts: few workgroups, or a long contraction.  Traced on
+  // weights out of the caches and rows just quantised, us, 64 x 64 blocks and their split form (its estimate): up to 256
+  // blocks the split form is the faster one at any length (128 blocks, 16 steps 7.8 and 5.8 (5.3), 28 steps 12.7 and 8.6
+  // (6.5); 176, 16: 7.8 and 6.9 (5.5); 256, 16: 10.4 and 9.6 (7.0)), from 512 on it is not (8 steps 10.2 and 10.5 (8.0), 16
+  // steps 15.2 and 15.9 (11.7), 28 steps 23.4 and 24.1 (18.9)) unless the weights' stream bounds both (1024, 56: 79 and 76).
+  // Its estimate is 1 to 5 us too low in between, so that without a line it would be taken at 512 blocks too; the line at 128
+  // gives up what it gains between 128 and 256 blocks on short contractions, up to 2 us a launch.
   const bool may_split = blocks_f < 128.0 || nkb >= 28;
   const double split = may_split ? std::max({2.2 + 1e-3 * blocks_p * (0.45 * n + 2.1), 4.0 + 0.63 * std::ceil(n / 8.0), weights / 6.2}) : 1e30;
   if (std::min(few, split) <= std::min(small, large)) return split < few ? kFewRowsSplit : kFewRows;
@@ -1362,7 +1370,7 @@ extern "C" int aamd_grouped_gemm_fp8_nt_static(const uint8_t* a, int64_t lda, co
                                                const float* b_s, int b_tile_scaled, const int64_t* group_offsets,
                                                int E, int64_t M, int64_t N, int64_t K, void* c, int c_dtype,
                                                int64_t ldc, const void* bias, int bias_dtype, void* stream) {
-  AAMD_REQUIRE(E >= 1 && E <= AAMD_STATIC_MAX_GROUPS, "grouped_gemm_nt_static: E=%d exceeds the %d groups the static scratch holds",
+  AAMD_REQUIRE(E >= 1 && E <= AAMD_STATIC_MAX_GROUPS, "grouped_gemm_nt_static: E=%d exceeds the limit of %d groups (no static scratch is behind it; it is the entry point's contract)",
                E, AAMD_STATIC_MAX_GROUPS);
   return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
                       stream);

@@ -85,7 +85,8 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
   // instruction's registers touch 32 lines each, four times over: with enough of them in flight to cover the latency
   // the lines leave the 32 KB L1 in between and are fetched again.)  Token rows past the group's end are not
   // loaded beyond the last slab of eight that holds one, re-read the last row inside it, and are not stored.
-  // One block in flight per wave and a dozen waves per CU: two or three blocks per wave measured no faster.
+  // One block in flight per wave, and two workgroups per CU, of 69.6 KB of LDS (8 waves) or, in the split form, 67.6 KB (16
+  // waves): two or three blocks per wave measured no faster where the weights' stream is the bound (1.9 GB).
   const int nkb = p.nkb;
   uint8_t* const mine = lds + wave * kStage;
   const uint8_t* const Lb = p.L + uniform_i64(l0 * p.ldl);

@@ -1494,8 +1494,9 @@ extern "C" int aamd_quant_128x128(const void* w, int w_dtype, int64_t E, int64_t
   AAMD_REQUIRE(N / kTile <= 65535 && E <= 65535, "quant_128x128: grid too large");
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(K / kTile), (unsigned)(N / kTile), (unsigned)E), block(256);
-  // Weights that the last-level cache holds are as fast in plain order or faster (1 x 14336 x 4096 41 us, 43 with rows per
-  // XCD; 60 x 2048 x 1408 110 both ways; 16 x 3072 x 5120 176 and 171).
+  // Below 2^27 elements (256 MB of bf16, what the last-level cache holds) plain order is as fast or faster: 1 x 14336 x 4096
+  // 42 us, 43 with rows per XCD; 8 x 4096 x 1024 23 both ways.  A little above it the two differ little (60 x 2048 x 1408,
+  // 1.3 times the line, 110 both ways; 16 x 3072 x 5120, 1.9 times, 176 and 172), far above it by 4 to 9 % (see the kernel).
   const int rows_per_xcd = E * N * K >= kBlockOrderElements;
   if (w_dtype == AAMD_BF16)
     quant_128x128_kernel<BF16><<<grid, block, 0, st>>>((const u16*)w, expert_stride, N, K, q, s, q_t, s_t, eps, rows_per_xcd);
