@@ -72,9 +72,10 @@ Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
 constexpr auto kFp8 = at::kFloat8_e4m3fn;
 
 // the transposed codes of `rows` columns and ld_t padded tokens
-Tensor alloc_qt(int64_t rows, int64_t ld_t, bool blocked, const Tensor& like) {
-  return blocked ? empty({ld_t / kTile, rows, kTile}, kFp8, like) : empty({rows, ld_t}, kFp8, like);
+c10::SmallVector<int64_t, 3> qt_shape(int64_t rows, int64_t ld_t, bool blocked) {
+  return blocked ? c10::SmallVector<int64_t, 3>{ld_t / kTile, rows, kTile} : c10::SmallVector<int64_t, 3>{rows, ld_t};
 }
+Tensor alloc_qt(int64_t rows, int64_t ld_t, bool blocked, const Tensor& like) { return empty(qt_shape(rows, ld_t, blocked), kFp8, like); }
 int64_t qt_ld(const Tensor& q_t) { return q_t.dim() == 3 ? q_t.size(0) * kTile : q_t.size(1); }
 int64_t padded_bound(int64_t rows, int64_t groups) { return (rows / kTile + groups) * kTile; }
 
@@ -622,6 +623,10 @@ PYBIND11_MODULE(_host, m) {
                              at::ScalarType dtype) {
     auto [r, sums] = dual_with_sums(what, x, dh.has_value() ? *dh : Tensor(), goff, E, ld_t, eps, dtype);
     return std::make_tuple(r.q, r.s, r.q_t, r.s_t, sums);
+  });
+  m.def("qt_shape", [](int64_t rows, int64_t ld_t, bool blocked) {
+    const auto shape = qt_shape(rows, ld_t, blocked);
+    return std::vector<int64_t>(shape.begin(), shape.end());
   });
   m.def("block_quant", &block_quant);
   m.def("block_quant_list", &block_quant_list);

@@ -153,10 +153,10 @@ def permute_rows(x: torch.Tensor, row_map: torch.Tensor, topk: int, num_out_rows
 
 
 def _alloc_qt(rows: int, ld_t: int, blocked: bool, dev) -> torch.Tensor:
-    """The transposed codes of ``rows`` columns and ``ld_t`` padded tokens: ``[rows, ld_t]``, or, blocked,
-    ``[ld_t/128, rows, 128]`` (token-block-major: every 128 x 128 tile is 16 KB of consecutive bytes)."""
-    shape = (ld_t // TILE, rows, TILE) if blocked else (rows, ld_t)
-    return torch.empty(shape, dtype=FP8, device=dev)
+    """A buffer for the transposed codes of ``rows`` columns and ``ld_t`` padded tokens in the shape the quantisers give
+    them (``qt_shape`` in csrc/host.cpp): ``[rows, ld_t]``, or, blocked, ``[ld_t/128, rows, 128]`` (token-block-major: every
+    128 x 128 tile is 16 KB of consecutive bytes).  For callers of the C ABI, which allocate themselves."""
+    return torch.empty(host().qt_shape(rows, ld_t, blocked), dtype=FP8, device=dev)
 
 
 def qt_ld(q_t: torch.Tensor) -> int:
