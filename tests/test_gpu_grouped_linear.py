@@ -336,49 +336,60 @@ def test_baseline_first_configuration_end_to_end(oracle, dev):
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("fuse", [False, True])
 def test_module_with_device_group_offsets_equals_host_splits(dev, bias, fuse):
-    """forward(inp, None, group_offsets=...) runs the same kernels as forward(inp, m_splits): identical
-    outputs and gradients, bit for bit, with bias, fused wgrad accumulation and under no_grad."""
+    """forward(inp, None, group_offsets=...) and forward(inp, m_splits), which are one function on whole buffers, against
+    the reference's own call sequence over lists of groups, which another operator object takes: identical outputs and
+    gradients, bit for bit, with bias, fused wgrad accumulation and under no_grad."""
     from atorch_amd import kernels
     from atorch_amd.grouped_linear import ATorchGroupedLinear
+    from atorch_amd.quantization import HipQuantizeOp, default_qlinear_params
+
+    class ListOp(HipQuantizeOp):
+        lists = 0
+
+        def grouped_qgemm(self, *args, **kw):
+            ListOp.lists += 1
+            return super().grouped_qgemm(*args, **kw)
 
     E, K, N = 5, 256, 384
     splits = [130, 0, 257, 64, 91]
     M = sum(splits)
     torch.manual_seed(4)
+    params = [default_qlinear_params() for _ in range(3)]
+    params[0].quantize_op = ListOp()
     mods = [ATorchGroupedLinear(E, K, N, bias=bias, params_dtype=torch.bfloat16, device=dev,
-                                fuse_wgrad_accumulation=fuse) for _ in range(2)]  # fmt: skip
+                                fuse_wgrad_accumulation=fuse, qlinear_params=p) for p in params]  # fmt: skip
     with torch.no_grad():
         for i in range(E):
-            mods[1].get_parameter(f"weight{i}").copy_(mods[0].get_parameter(f"weight{i}"))
-            if bias:
-                b = randn_bf16((N,), 80 + i).to(dev)
-                mods[0].get_parameter(f"bias{i}").copy_(b)
-                mods[1].get_parameter(f"bias{i}").copy_(b)
-            if fuse:
-                mg = torch.rand(N, K, generator=torch.Generator().manual_seed(i)).to(dev)
-                mods[0].get_parameter(f"weight{i}").main_grad = mg.clone()
-                mods[1].get_parameter(f"weight{i}").main_grad = mg.clone()
+            b = randn_bf16((N,), 80 + i).to(dev)
+            mg = torch.rand(N, K, generator=torch.Generator().manual_seed(i)).to(dev)
+            for m in mods:
+                m.get_parameter(f"weight{i}").copy_(mods[0].get_parameter(f"weight{i}"))
+                if bias:
+                    m.get_parameter(f"bias{i}").copy_(b)
+                if fuse:
+                    m.get_parameter(f"weight{i}").main_grad = mg.clone()
     x = heavy_tailed((M, K), 21).to(dev)
     dy = randn_bf16((M, N), 22, std=1e-2).to(dev)
     goff = kernels.group_offsets_from_splits(splits, dev)
-    xa, xb = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
-    oa = mods[0](xa, splits)
-    ob = mods[1](xb, None, group_offsets=goff)
-    assert torch.equal(oa, ob)
-    oa.backward(dy)
-    ob.backward(dy)
-    assert torch.equal(xa.grad, xb.grad)
-    for i in range(E):
-        wa, wb = mods[0].get_parameter(f"weight{i}"), mods[1].get_parameter(f"weight{i}")
-        if fuse:
-            assert wa.grad is None and wb.grad is None and torch.equal(wa.main_grad, wb.main_grad)
-        else:
-            assert torch.equal(wa.grad, wb.grad)
-        if bias:
-            ga, gb = mods[0].get_parameter(f"bias{i}").grad, mods[1].get_parameter(f"bias{i}").grad
-            torch.testing.assert_close(ga.float(), gb.float(), rtol=2e-2, atol=1e-4)  # order of an fp32 sum
+    xs = [x.clone().requires_grad_(True) for _ in mods]
+    outs = [mods[0](xs[0], splits), mods[1](xs[1], splits), mods[2](xs[2], None, group_offsets=goff)]
+    for o in outs:
+        o.backward(dy)
+    assert ListOp.lists == 3  # forward, both gradients
+    for m, xg, o in zip(mods[1:], xs[1:], outs[1:]):
+        assert torch.equal(o, outs[0]) and torch.equal(xg.grad, xs[0].grad)
+        for i in range(E):
+            wa, wb = mods[0].get_parameter(f"weight{i}"), m.get_parameter(f"weight{i}")
+            if fuse:
+                assert wa.grad is None and wb.grad is None and torch.equal(wa.main_grad, wb.main_grad)
+            else:
+                assert torch.equal(wa.grad, wb.grad)
+            if bias:
+                ga, gb = mods[0].get_parameter(f"bias{i}").grad, m.get_parameter(f"bias{i}").grad
+                torch.testing.assert_close(ga.float(), gb.float(), rtol=2e-2, atol=1e-4)  # order of an fp32 sum
     with torch.no_grad():
-        assert torch.equal(mods[1](x, None, group_offsets=goff, is_first_microbatch=False), oa.detach())
+        assert torch.equal(mods[2](x, None, group_offsets=goff, is_first_microbatch=False), outs[0].detach())
+        assert torch.equal(mods[1](x, splits, is_first_microbatch=False), outs[0].detach())
 
 
 def test_module_moved_to_the_device_runs_the_device_offset_path(dev):

@@ -1,9 +1,8 @@
-"""The entry point that allocates nothing, aamd_grouped_gemm_fp8_nt_static: the tile prefix lives in a
-static device array of the library instead of a caller workspace.  Called through the C ABI with raw
-ctypes and compared bit for bit with aamd_grouped_gemm_fp8_nt on the same operands and, within the GEMM
-tolerance, with the float64 dequantise-and-matmul definition, twice in a row: first a launch that takes the
-256 x 256 tiles (a prefix of 256-row tiles in the scratch), then a smaller one with fewer groups and rows on the
-128 x 128 tiles, so stale scratch contents would show."""
+"""aamd_grouped_gemm_fp8_nt_static, the entry point without a workspace argument.  It runs the kernels of
+aamd_grouped_gemm_fp8_nt, so that equality with it checks the arguments of the shorter signature; what both compute is
+held, within the GEMM tolerance, to the float64 dequantise-and-matmul definition.  Called through the C ABI with raw
+ctypes: a launch with more groups than a wave has lanes on the 256 x 256 tiles, then a smaller one with few groups, neither
+of which may allocate device memory."""
 import ctypes
 
 import pytest
