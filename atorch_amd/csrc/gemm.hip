@@ -1142,6 +1142,12 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
           }
 #pragma unroll
           for (int ps = 0; ps < WROWS / 8; ps++) asm volatile("" : "+v"(olds[ps]));
+          // (added here, not at the stores: held next to the new values until then they do not fit, and ten registers of
+          // every thread went through memory, an eighth of what the launch writes.  Us with and
+          // without: 8 groups of 4096 rows, 28672 x 4096 outputs written over 4800, 4660, added 5480, 4975; 60 groups of 1092
+          // rows, 2816 x 2048, 756, 670 and 990, 806)
+#pragma unroll
+          for (int ps = 0; ps < WROWS / 8; ps++) raws[ps] = __builtin_bit_cast(v4i, __builtin_bit_cast(v4f, raws[ps]) + olds[ps]);
         }
       }
       OUT* out_row = out_row0;
@@ -1153,18 +1159,9 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
         out_row += row_step;
         if (lrow < lvalid) {
           if constexpr (sizeof(ST) == sizeof(OUT)) {
-            if constexpr (kAddF32) {
-              // the output is not read again by this launch: streaming stores keep it from
-              // evicting operand panels from L2 (measured +1-2 % where the output is large)
-              if (p.accumulate) {
-                const v4f o = __builtin_bit_cast(v4f, raw) + olds[ps];
-                __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(out));
-              } else {
-                __builtin_nontemporal_store(raw, reinterpret_cast<v4i*>(out));
-              }
-            } else {
-              __builtin_nontemporal_store(raw, reinterpret_cast<v4i*>(out));
-            }
+            // the output is not read again by this launch: streaming stores keep it from
+            // evicting operand panels from L2 (measured +1-2 % where the output is large)
+            __builtin_nontemporal_store(raw, reinterpret_cast<v4i*>(out));
           } else {  // fp32 staging, bf16 output with accumulation
             store4<OUT>(out, __builtin_bit_cast(v4f, raw), true);
           }
