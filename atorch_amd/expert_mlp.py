@@ -66,13 +66,14 @@ def _weight_codes(w1, w2, v1, transpose_w1, is_first_microbatch, weight_cache):
     """``(q1, s1, q1_t, s1_t), (q2, s2, q2_t, s2_t)``: the first weight(s) as [E, N1, H] (rows = outputs) and the second
     as [E, F, H], each with its transpose; block quantisation commutes with the transpose, so both orientations
     come out of one launch each."""
+    if weight_cache is not None:
+        held = weight_cache.held((("w1", (w1, v1)), ("w2", (w2,))), is_first_microbatch, True)
+        if held is not None:
+            return held
     quant1 = lambda t: _quant_first_weight(w1, v1, transpose_w1)  # noqa: E731
     quant2 = lambda t: kernels.block_quant_batched(w2.detach().contiguous(), return_transpose=True)  # noqa: E731
     if weight_cache is None:
         return quant1(True), quant2(True)
-    held = weight_cache.held((("w1", (w1, v1)), ("w2", (w2,))), is_first_microbatch, True)
-    if held is not None:
-        return held
     return (weight_cache.codes("w1", (w1, v1), is_first_microbatch, True, quant1),
             weight_cache.codes("w2", (w2,), is_first_microbatch, True, quant2))  # fmt: skip
 

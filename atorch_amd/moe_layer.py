@@ -107,7 +107,9 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         self.hidden_shape = None
 
     def has_v1(self):
-        return hasattr(self, "v1") and self.v1 is not None
+        # (hasattr takes a microsecond to say no)
+        kept = "v1" in self._parameters or "v1" in self.__dict__ or "v1" in self._buffers or hasattr(type(self), "v1")
+        return kept and self.v1 is not None
 
     def scale_grad(self, w):
         return w  # gradient_scale is None without expert parallelism (grouped_gemm_moe.py:427-431, 632-636)
@@ -147,28 +149,25 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         return self._forward_megatron(hidden_states, expert_weights, top_experts, se_fn1, se_fn2,
                                       se_fn2_additional_input, is_first_microbatch)  # fmt: skip
 
-    def _weight(self, name):
-        """``getattr(self, name)`` in a third of its time where the name is a parameter.  (A pruned or parametrised one is
-        not, nor is one that a wrapper keeps as a plain attribute.)"""
-        p = self._parameters
-        return p[name] if name in p else getattr(self, name)
-
     def _nothing_between(self, dispatcher):
         """True if nothing happens between the experts and the combine and both ends are this package's: the dropout is the
         identity, nobody listens to it, and dispatcher and dropout are the modules the constructor made."""
         drop = self._modules.get("dropout")
         return (type(dispatcher) is MoEAllToAllTokenDispatcher and type(drop) is torch.nn.Dropout
-                and not (drop.training and drop.p > 0) and not drop._forward_hooks and not drop._forward_pre_hooks
-                and not drop._backward_hooks and not drop._backward_pre_hooks)  # fmt: skip
+                and not (drop.training and drop.p > 0 or drop._forward_hooks or drop._forward_pre_hooks
+                         or drop._backward_hooks or drop._backward_pre_hooks))  # fmt: skip
 
     def _forward_fused(self, x, probs, top_experts, is_first_microbatch):
-        """The layer as one function, one native call per direction."""
+        """The layer as one function, one native call per direction, which compares the sizes.  (Choices may also come
+        flattened, as other MoE layers pass them.)"""
         assert x.dtype == torch.bfloat16, "the fused activation kernels read bf16"
-        T = x.shape[0]  # (choices may also come flattened, as other MoE layers pass them)
-        assert probs.shape == (T, self.topk) and top_experts.numel() == T * self.topk, "router weights and choices are [tokens, topk]"
-        w1, w2 = self.scale_grad(self._weight("w1")), self.scale_grad(self._weight("w2"))
-        v1 = self.scale_grad(self._weight("v1")) if self.has_v1() else None
-        b1, b2 = (self._weight("b1"), self._weight("b2")) if self.use_bias else (None, None)
+        # (looked up where they mostly are, a third of an attribute's time; a pruned or parametrised one is no parameter, nor is
+        # one that a wrapper keeps as a plain attribute)
+        p = self._parameters
+        w1 = self.scale_grad(p["w1"] if "w1" in p else self.w1)
+        w2 = self.scale_grad(p["w2"] if "w2" in p else self.w2)
+        v1 = self.scale_grad(self.v1) if self.has_v1() else None
+        b1, b2 = (self.b1, self.b2) if self.use_bias else (None, None)
         assert v1 is None or self.use_swiglu, "v1 is the up projection of a gated unit"
         assert v1 is None or b1 is None, "bias not supported yet for not merge_w1_v1"
         args = (x, probs, w1, w2, v1, b1, b2, top_experts, self.token_dispatcher, self.transpose_w1, self.use_swiglu,
