@@ -19,6 +19,7 @@ import logging
 from typing import Callable, List, Optional, Tuple, Union
 
 import torch
+from torch.autograd import forward_ad
 
 from .expert_mlp import _Fp8MoeLayer, grouped_mlp
 from .quantization import WeightCodeCache
@@ -172,7 +173,9 @@ class Grouped_GEMM_MoE(torch.nn.Module):
         assert v1 is None or b1 is None, "bias not supported yet for not merge_w1_v1"
         args = (x, probs, w1, w2, v1, b1, b2, top_experts, self.token_dispatcher, self.transpose_w1, self.use_swiglu,
                 is_first_microbatch, self.weight_code_cache)  # fmt: skip
-        return _Fp8MoeLayer.apply(*args) if torch.is_grad_enabled() else _Fp8MoeLayer.forward(None, *args)
+        # (past autograd only where nobody else looks either: a dual number is refused and a trace records the function there)
+        plain = not torch.is_grad_enabled() and forward_ad._current_level < 0 and not torch.jit.is_tracing()
+        return _Fp8MoeLayer.forward(None, *args) if plain else _Fp8MoeLayer.apply(*args)
 
     def _forward_megatron(self, hidden_states, expert_weights, top_experts, se_fn1=None, se_fn2=None,
                           se_fn2_additional_input=None, is_first_microbatch=None):

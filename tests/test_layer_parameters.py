@@ -169,3 +169,30 @@ def test_whatever_sits_between_experts_and_combine_runs(monkeypatch, change):
     with pytest.raises(RuntimeError, match="composite"):
         run()
     assert not seen
+
+
+@pytest.mark.filterwarnings("ignore")  # (what a tracer says of sizes)
+def test_forward_mode_and_tracing_do_not_pass_the_function_by(monkeypatch):
+    """Without gradients the function's forward is called as it is, but not on dual numbers, whose tangent it would drop, and
+    not in a trace, which would keep its empty buffers and none of its launches."""
+    from torch.autograd import forward_ad
+
+    from atorch_amd import moe_layer
+
+    layer, seen, run = _layer(monkeypatch)
+    layer.requires_grad_(False)
+    calls = []
+    recorder = moe_layer._Fp8MoeLayer
+    apply = recorder.apply
+    monkeypatch.setattr(recorder, "apply", staticmethod(lambda *a: (calls.append("apply"), apply(*a))[1]))
+    monkeypatch.setattr(recorder, "forward", staticmethod(lambda ctx, *a: (calls.append("forward"), apply(*a))[1]))
+    x, (idx, probs) = randn_bf16((8, 256), 2), topk_routing(8, 4, 2, seed=1)
+    probs = probs.bfloat16()
+    with torch.no_grad():
+        layer(x, probs, idx)
+        with forward_ad.dual_level():
+            layer(forward_ad.make_dual(x, torch.ones_like(x)), probs, idx)
+        torch.jit.trace(lambda t: layer(t, probs, idx), (x,), check_trace=False)
+        layer(x, probs, idx)
+    layer(x, probs, idx)
+    assert calls == ["forward", "apply", "apply", "forward", "apply"]
