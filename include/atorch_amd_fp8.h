@@ -5,7 +5,9 @@
  * Conventions
  *   - every pointer is a DEVICE pointer owned by the caller (the caller
  *     allocates all outputs and workspaces); nothing here allocates device
- *     memory or synchronises the host with the device;
+ *     memory or synchronises the host with the device (the dual GELU and the
+ *     SwiGLU-backward quantisers take four bytes of pinned host memory each
+ *     in their first call on a device that is not captured);
  *   - `stream` is a hipStream_t passed as void* (NULL = the default stream);
  *     kernels are only enqueued;
  *   - functions return AAMD_OK (0) or an error code; aamd_last_error() gives
@@ -211,6 +213,8 @@ int aamd_gelu_quant_1x128_dual_grouped(const void *x, const void *dh, int64_t M,
  *   c [M, N] of c_dtype (row stride ldc elements, rows 16-byte aligned); rows of empty groups are not touched
  *   bias [E, N] of bias_dtype or NULL (AAMD_NONE); tile_ws: not used; may be NULL.
  *   K % 128 == 0, N % 128 == 0.
+ * The kernel is chosen by M, N, K and E, and the one for few rows adds the 128-deep blocks in another order: a row's fp32
+ * sum is the same in every launch of one size, and may differ in its last bits between launches of different sizes.
  */
 int aamd_grouped_gemm_fp8_nt(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b, const float *b_s,
                              int b_tile_scaled, const int64_t *group_offsets, int E, int32_t *tile_ws, int64_t M,
