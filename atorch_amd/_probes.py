@@ -17,6 +17,10 @@ SIGNATURES = {
         _int,
         [_vp, _i64, _vp, _vp, _vp, _int, _vp, _int, _vp, _i64, _i64, _i64, _vp, _int, _i64, _vp, _int, _opts, _vp],
     ),
+    "aamd_tuning_grouped_gemm_fp8_nn": (
+        _int,
+        [_vp, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int, _i64, _vp, _int, _opts, _vp],
+    ),
     "aamd_tuning_grouped_gemm_fp8_wgrad": (
         _int,
         [_vp, _vp, _vp, _vp, _i64, _int, _vp, _int, _vp, _i64, _i64, _vp, _int, _i64, _int, _opts, _vp],

@@ -81,17 +81,6 @@ typedef Cfg<2, 2, 2, 2, 3> CfgSmall;  // 256 threads, 128 (L) x 128 (R), two wor
 typedef Cfg<2, 4, 4, 2, 1, true> CfgLarge;  // 512 threads, 256 (L) x 256 (R); one product buffer: 256 registers per lane
 typedef Cfg<2, 4, 2, 2> CfgWgrad;  // 512 threads, 256 (L) x 128 (R): room for the per-row R scales
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant
-// expression inside the body.
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // ---- weight gradient of short groups -----------------------------------------------------------
 // A tile of a group of few rows is over after one or two 128-deep steps, and what it costs in grouped_gemm_kernel is the
 // workgroup's turnover: launch, group lookup, first loads and the stores follow each other, with two workgroups per CU to
@@ -318,7 +307,14 @@ __device__ __forceinline__ void wgrad_short_tiles(const GemmParams& p, uint8_t* 
   }
 }
 
-template <int MODE, bool R_PER_ROW, typename OUT, typename C>
+// R_ROWS: the R operand as it is stored where its contraction runs down the rows, [contraction, Rrows] (the codes of a
+// weight read for the product with its transpose: one scale per 128x128 block, so that the codes are the same bytes in
+// either orientation).  A step's R tile is then 128 rows of BN bytes, and the fragments are read with
+// ds_read_b64_tr_b8: of every 16 lanes, lanes 2r and 2r + 1 name the halves of 16 bytes of row r, and lane l receives
+// byte l of the eight rows.  The 16-byte chunks of a row are XORed with twice the low bits of its place among the rows
+// that share the 64 banks, so that the 32 lanes of a read phase (two chunks of eight rows) meet no bank twice (measured: 2.0
+// clocks per instruction and CU with eight waves, as ds_read_b64 of consecutive bytes; 12 without the XOR).
+template <int MODE, bool R_PER_ROW, typename OUT, typename C, bool R_ROWS>
 __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kernel(const GemmParams p) {
   constexpr int BM = C::BM, BN = C::BN, NT = C::NT;
   // LDS: two stages of an L tile and an R tile of 128-byte rows, then the two stages' scales
@@ -330,6 +326,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   // kRaggedRows keeps two batches of L scales besides: [BM rows][8 contraction blocks] floats each.
   constexpr int kLsBatch = MODE == kRaggedRows ? BM * 8 * 4 : 0;
   static_assert(NT == 2 * BM, "two threads fetch the 32 bytes of a row's scale batch");
+  static_assert(!R_ROWS || (MODE == kRaggedRows && !R_PER_ROW), "one scale per row along the contraction has one orientation");
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kStage + 2 * NT * 4 + 2 * kLsBatch];
   // both L stages first, then both R stages: every fragment of a side is within 64 KB of one base
   // address, so the stage and the sub-tile row go into the immediate offset of the LDS reads
@@ -531,7 +528,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 
   // uniform tile bases + per-thread 32-bit offsets
   const uint8_t* Lbase = p.L + uniform_i64(l0 * p.ldl + (int64_t)kb0 * p.l_kb_stride);
-  const uint8_t* Rbase = p.R + uniform_i64((int64_t)g * p.r_group_stride + r0 * p.ldr + (int64_t)kb0 * p.r_kb_stride);
+  const uint8_t* Rbase = p.R + uniform_i64((int64_t)g * p.r_group_stride + (R_ROWS ? r0 : r0 * p.ldr) + (int64_t)kb0 * p.r_kb_stride);
   const float* Lsg = p.Ls + (int64_t)kb0 * p.ls_blk_stride;
   const float* Rsg = p.Rs + (int64_t)g * p.rs_group_stride + (int64_t)kb0 * p.rs_blk_stride;
 
@@ -553,7 +550,16 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   const int bmaxL = ((availL - 1) >> 3) << 3, tailL = availL - bmaxL;
   const uint32_t voffL = (uint32_t)r8 * (uint32_t)p.ldl + chunk;
   const uint32_t voffLt = (uint32_t)(r8 < tailL ? r8 : tailL - 1) * (uint32_t)p.ldl + chunk;
-  const uint32_t voffR = (uint32_t)r8 * (uint32_t)p.ldr + chunk;  // rvalid is a multiple of 128: whole slabs
+  // rvalid is a multiple of 128: whole slabs
+  uint32_t voffR = (uint32_t)r8 * (uint32_t)p.ldr + chunk;
+  if constexpr (R_ROWS) {
+    // 1 KB = 1024 / BN rows of the tile; columns past the valid ones re-read valid ones of the same row
+    constexpr int kChunks = BN / 16;
+    const int row = ((wave * 1024) / BN + lane / kChunks) & 7;
+    const int ch = ((lane % kChunks) ^ (2 * (row / (256 / BN)))) & (rvalid / 16 - 1);
+    static_assert((BN == 256 || BN == 128) && (NT * 16 / BN) % 8 == 0, "the swizzle of a slab depends on the wave only");
+    voffR = (uint32_t)(lane / kChunks) * (uint32_t)p.ldr + (uint32_t)ch * 16u;
+  }
   uint32_t lslab[C::LCH], rslab[C::RCH];  // scalar byte offsets of the slabs
   bool ltail[C::LCH];
 #pragma unroll
@@ -565,7 +571,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 #pragma unroll
   for (int n = 0; n < C::RCH; n++) {
     const int b = wave * 8 + (NT / 8) * n;
-    rslab[n] = __builtin_amdgcn_readfirstlane((uint32_t)(b < rvalid ? b : rvalid - 8) * (uint32_t)p.ldr);
+    rslab[n] = __builtin_amdgcn_readfirstlane((uint32_t)(R_ROWS ? b * kBK / BN : b < rvalid ? b : rvalid - 8) * (uint32_t)p.ldr);
   }
   // scales: thread t < BM fetches the L scale of row t; thread BM + t the R scale of row t
   // (per-row scales) or of 128-row block t (block scales); the rest re-read a valid value.
@@ -695,10 +701,41 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       la[h][c] = (uint32_t)(uintptr_t)(lds_ptr_t)Lbuf0 + (uint32_t)((wlrow0 + l32) * kBK + chk[h][c]);
-      ra[h][c] = (uint32_t)(uintptr_t)(lds_ptr_t)Rbuf0 + (uint32_t)((wrow0 + l32) * kBK + chk[h][c]);
+      if constexpr (R_ROWS) {
+        // sub-tile row i = 2 h + c: the half chunk of contraction row 32 hg + tr that this lane names; the other rows of its
+        // fragment are 8 and 64 rows on
+        const int i = (2 * h + c) % C::WTR, tr = (lane & 15) >> 1;
+        const int ch = (wrow0 / 16 + 2 * i + ((lane >> 4) & 1)) ^ (2 * (tr / (256 / BN)));
+        ra[h][c] = (uint32_t)(uintptr_t)(lds_ptr_t)Rbuf0 + (uint32_t)((32 * hg + tr) * BN + ch * 16 + (lane & 1) * 8);
+      } else {
+        ra[h][c] = (uint32_t)(uintptr_t)(lds_ptr_t)Rbuf0 + (uint32_t)((wrow0 + l32) * kBK + chk[h][c]);
+      }
       asm volatile("" : "+v"(la[h][c]));
       asm volatile("" : "+v"(ra[h][c]));
     }
+  static_assert(!R_ROWS || C::WTR <= 4, "an address per sub-tile row");
+  // fragment of sub-tile row `sub` (32 rows each) of one side in stage s, K half h
+  typedef const __attribute__((address_space(3))) v4i* lds_v4i_t;
+  auto frag = [&](const uint32_t (&base)[2][2], int s, int rows_per_stage, int sub, int h) __attribute__((always_inline)) {
+    const uint32_t delta = (uint32_t)((s * rows_per_stage + sub * 32) * kBK);
+    const v4i lo = *(lds_v4i_t)(uintptr_t)(base[h][0] + delta);
+    const v4i hi = *(lds_v4i_t)(uintptr_t)(base[h][1] + delta);
+    return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+  auto fragR = [&](int s, int sub, int h) __attribute__((always_inline)) {
+    if constexpr (R_ROWS) {
+      v8i f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const v2i o = lds_read_transposed(ra[sub / 2][sub % 2] + (uint32_t)(s * BN * kBK + (64 * h + 8 * j) * BN));
+        f[2 * j] = o[0];
+        f[2 * j + 1] = o[1];
+      }
+      return f;
+    } else {
+      return frag(ra, s, BN, sub, h);
+    }
+  };
   const bool wave_active = wrow0 < rvalid;        // whole wave in or out: rvalid % 128 == 0
   // a wave none of whose L rows or R rows is valid takes part in loads and barriers only
   const bool has_work = __builtin_amdgcn_readfirstlane((int)(wave_active && wlrow0 < lvalid)) != 0;
@@ -725,40 +762,32 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     const float* Lsc = batch ? LsB0 + (bsel & 1) * (BM * 8) + (kb - batch_start(bsel)) : Sct;
     const int lsc_stride = batch ? 8 : 1;
     const float* Rsc = Sct + BM;
-    // fragment of sub-tile row `sub` (32 rows each) of one side, K half h
-    typedef const __attribute__((address_space(3))) v4i* lds_v4i_t;
-    auto load_frag = [&](const uint32_t (&base)[2][2], int rows_per_stage, int sub, int h) {
-      const uint32_t delta = (uint32_t)((stage * rows_per_stage + sub * 32) * kBK);
-      const v4i lo = *(lds_v4i_t)(uintptr_t)(base[h][0] + delta);
-      const v4i hi = *(lds_v4i_t)(uintptr_t)(base[h][1] + delta);
-      return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    };
     v8i lf[C::WTL][2];
     float cs[C::WTL];
     const float rblk = R_PER_ROW ? 1.f : Rsc[wrow0 / kTile];
     v8i rf[2][2];
     // LDS reads in the order of first use: the first MFMA waits for two fragments only, the rest
     // arrive in its shadow
-    lf[0][0] = load_frag(la, BM, 0, 0);
-    rf[0][0] = load_frag(ra, BN, 0, 0);
+    lf[0][0] = frag(la, stage, BM, 0, 0);
+    rf[0][0] = fragR(stage, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
-    lf[0][1] = load_frag(la, BM, 0, 1);
-    rf[0][1] = load_frag(ra, BN, 0, 1);
+    lf[0][1] = frag(la, stage, BM, 0, 1);
+    rf[0][1] = fragR(stage, 0, 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < C::WTL; j++) {
       const int row = wlrow0 + j * 32 + l32;
       if (j > 0) {
-        lf[j][0] = load_frag(la, BM, j, 0);
-        lf[j][1] = load_frag(la, BM, j, 1);
+        lf[j][0] = frag(la, stage, BM, j, 0);
+        lf[j][1] = frag(la, stage, BM, j, 1);
       }
       cs[j] = Lsc[row * lsc_stride] * rblk;
     }
     v4f rs[2][4];  // R_PER_ROW: scales of the 16 R rows this lane holds in a sub-tile
     auto load_r = [&](int i) {
       if (i > 0) {
-        rf[i & 1][0] = load_frag(ra, BN, i, 0);
-        rf[i & 1][1] = load_frag(ra, BN, i, 1);
+        rf[i & 1][0] = fragR(stage, i, 0);
+        rf[i & 1][1] = fragR(stage, i, 1);
       }
       if constexpr (R_PER_ROW) {
 #pragma unroll
@@ -871,13 +900,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     constexpr int PT = (C::WTR - 1) * C::WTL - 1;  // the sub-tile in front of barrier P
     constexpr int RPER = C::RCH / C::WTL;
     auto kclamp = [&](int k) { return k < nkb ? k : nkb - 1; };
-    typedef const __attribute__((address_space(3))) v4i* lds_v4i_t;
-    auto frag = [&](const uint32_t (&base)[2][2], int stage, int rows_per_stage, int sub, int h) {
-      const uint32_t delta = (uint32_t)((stage * rows_per_stage + sub * 32) * kBK);
-      const v4i lo = *(lds_v4i_t)(uintptr_t)(base[h][0] + delta);
-      const v4i hi = *(lds_v4i_t)(uintptr_t)(base[h][1] + delta);
-      return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    };
     // Scales of this pipeline come in batches of eight contraction blocks only (the launcher takes the other
     // configuration when K has fewer than eight blocks), so a
     // step issues no scale load and takes no branch: batch b (blocks 8 b .. 8 b + 7, the last one shifted
@@ -894,7 +916,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     const int rlane_blk = ((lane >> 1) & 1) < rblocks ? (lane >> 1) & 1 : rblocks - 1;
     const uint32_t roff = ((uint32_t)rlane_blk * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 1) * 4u) * 4u;
     const int rlane_blk1 = ((lane >> 3) & 1) < rblocks ? (lane >> 3) & 1 : rblocks - 1;
-    const uint32_t roff1 = ((uint32_t)rlane_blk1 * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 7)) * 4u;
+    const uint32_t roff1 = ((uint32_t)rlane_blk1 * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 7) * (uint32_t)p.rs_blk_stride) * 4u;
     uint32_t boff1[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -903,20 +925,22 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     }
     auto dma_batches = [&](int b) {
       const uint8_t* lsb = reinterpret_cast<const uint8_t*>(Lsg + uniform_i64(l0 * p.ls_row_stride + batch_start(b)));
-      const uint8_t* rsb = reinterpret_cast<const uint8_t*>(Rsg + uniform_i64((r0 / kTile) * p.rs_row_stride + batch_start(b)));
+      const uint8_t* rsb = reinterpret_cast<const uint8_t*>(Rsg + uniform_i64((r0 / kTile) * p.rs_row_stride + batch_start(b) * p.rs_blk_stride));
       const uint32_t ldst = lds_addr(LsB0 + (b & 1) * (BM * 8)) + (uint32_t)(wave * 1024);
       const uint32_t rdst = lds_addr(RsB0 + (b & 1) * NT);
       if (x4) {
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(boff), "s"(lsb), "s"(ldst) : "memory");
-        if (wave == 0)
+        if (!R_ROWS && wave == 0)
           asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(roff), "s"(rsb), "s"(rdst) : "memory");
       } else {
 #pragma unroll
         for (int q = 0; q < 4; q++)
           asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(boff1[q]), "s"(lsb), "s"(ldst + (uint32_t)(q * 256)) : "memory");
-        if (wave == 0)
+        if (!R_ROWS && wave == 0)
           asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(roff1), "s"(rsb), "s"(rdst) : "memory");
       }
+      if (R_ROWS && wave == 0)  // a row of scales per contraction block: never 16 bytes of one block
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(roff1), "s"(rsb), "s"(rdst) : "memory");
     };
     if (nkb > 0) {
       dmaL(0, Lbuf0, Sc0);  // (the per-step scale hooks of these helpers are off: see step_scale)
@@ -956,7 +980,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           lf[0][h] = frag(la, 0, BM, 0, h);
-          rf[0][h] = frag(ra, 0, BN, 0, h);
+          rf[0][h] = fragR(0, 0, h);
         }
 #pragma unroll
         for (int j = 1; j < C::WTL; j++)
@@ -988,7 +1012,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
             if constexpr (t < C::LCH) dmaL_tile(t, k2, Lc);
             if constexpr (j == 0 && i + 1 < C::WTR) {
 #pragma unroll
-              for (int h = 0; h < 2; h++) rf[(i + 1) & 1][h] = frag(ra, s, BN, i + 1, h);
+              for (int h = 0; h < 2; h++) rf[(i + 1) & 1][h] = fragR(s, i + 1, h);
             }
             if constexpr (t == PT) {
               __builtin_amdgcn_sched_barrier(0);
@@ -999,7 +1023,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
               }
               // row C::WTR - 2 has been consumed: its registers take the first R row of the next step
 #pragma unroll
-              for (int h = 0; h < 2; h++) rf[0][h] = frag(ra, s ^ 1, BN, 0, h);
+              for (int h = 0; h < 2; h++) rf[0][h] = fragR(s ^ 1, 0, h);
               read_scales(kclamp(kb + 1), csn, rblkn);
             }
             if constexpr (t > PT) {
@@ -1196,7 +1220,7 @@ struct GemmOptions {
   int ls_batch = -1;  // 0: L scales fetched one contraction block at a time
 };
 
-template <int MODE, bool R_PER_ROW, typename C>
+template <int MODE, bool R_PER_ROW, typename C, bool R_ROWS = false>
 static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st, const GemmOptions& g_opt) {
   if (blocks <= 0) return AAMD_OK;
   // L tiles per group of the tile order: 8 for the row-ragged launches; 4 for wgrad, whose operand
@@ -1215,9 +1239,9 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
   AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
   dim3 grid((unsigned)blocks), block(C::NT);
   if (c_dtype == AAMD_BF16)
-    grouped_gemm_kernel<MODE, R_PER_ROW, u16, C><<<grid, block, 0, st>>>(p);
+    grouped_gemm_kernel<MODE, R_PER_ROW, u16, C, R_ROWS><<<grid, block, 0, st>>>(p);
   else
-    grouped_gemm_kernel<MODE, R_PER_ROW, float, C><<<grid, block, 0, st>>>(p);
+    grouped_gemm_kernel<MODE, R_PER_ROW, float, C, R_ROWS><<<grid, block, 0, st>>>(p);
   AAMD_LAUNCH_CHECK("grouped_gemm");
   return AAMD_OK;
 }
@@ -1240,7 +1264,9 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
 // or the kernel for few rows priced wrong -> this fit: one group of 14441 rows, 5504 x 640 200 -> 91; 64 groups, 8591 rows,
 // 16256 x 768 372 -> 195; 4 groups, 2498 rows, 8832 x 512 51 -> 30.
 enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3 };
-static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, const GemmOptions& g_opt) {
+// (weights read along their rows, b_rows: the same line but for the split form, which they do not have; 128 x 32 blocks of the
+// kernel for few rows are as many as 64 x 64 ones)
+static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return g_opt.tile == 1 && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const int64_t groups = M < E ? M : E;
   const double n = (double)nkb;
@@ -1266,7 +1292,7 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   // steps 15.2 and 15.9 (11.7), 28 steps 23.4 and 24.1 (18.9)) unless the weights' stream bounds both (1024, 56: 79 and 76).
   // Its estimate is 1 to 5 us too low in between, so that without a line it would be taken at 512 blocks too; the line at 128
   // gives up what it gains between 128 and 256 blocks on short contractions, up to 2 us a launch.
-  const bool may_split = blocks_f < 128.0 || nkb >= 28;
+  const bool may_split = !b_rows && (blocks_f < 128.0 || nkb >= 28);
   const double split = may_split ? std::max({2.2 + 1e-3 * blocks_p * (0.45 * n + 2.1), 4.0 + 0.63 * std::ceil(n / 8.0), weights / 6.2}) : 1e30;
   if (std::min(few, split) <= std::min(small, large)) return split < few ? kFewRowsSplit : kFewRows;
   return large < small ? kLargeTiles : kSmallTiles;
@@ -1301,8 +1327,9 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 using namespace aamd;
 
+// b_rows: b is [E, K, N], b_s [E, K/128, N/128] (see R_ROWS); block scales only.
 static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
-                        int b_tile_scaled, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
+                        int b_tile_scaled, bool b_rows, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
                         int c_dtype, int64_t ldc, const void* bias, int bias_dtype, void* stream,
                         const GemmOptions& g_opt = GemmOptions()) {
   AAMD_REQUIRE(c_dtype == AAMD_BF16 || c_dtype == AAMD_F32, "grouped_gemm_nt: unsupported output dtype %d", c_dtype);
@@ -1318,13 +1345,13 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   AAMD_REQUIRE(ldc >= N && (ldc * (c_dtype == AAMD_BF16 ? 2 : 4)) % 16 == 0 && aligned16(c),
                "grouped_gemm_nt: output rows must be 16-byte aligned");
   AAMD_REQUIRE(K > 0, "grouped_gemm_nt: K must be positive");
-  AAMD_REQUIRE(lda < (1LL << 23) && K < (1LL << 23), "grouped_gemm_nt: row stride too large");
+  AAMD_REQUIRE(lda < (1LL << 23) && K < (1LL << 23) && (!b_rows || N < (1LL << 23)), "grouped_gemm_nt: row stride too large");
   hipStream_t st = (hipStream_t)stream;
   // scale batches of eight contraction blocks; their 16-byte loads need aligned rows and whole groups of four blocks
   const bool batches = (K / kBK) >= 8 && g_opt.ls_batch != 0;
   const bool batches16 = batches && (K / kBK) % 4 == 0 && aligned16(a_s);
   const NtKernel kernel = b_tile_scaled ? (use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), g_opt) ? kLargeTiles : kSmallTiles)
-                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, g_opt);
+                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, g_opt);
   const bool large = kernel == kLargeTiles;
   const int BM = large ? CfgLarge::BM : CfgSmall::BM;
   const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : CfgLarge::BN) : CfgSmall::BN;
@@ -1337,14 +1364,21 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   p.Rs = b_s;
   p.rs_row_stride = K / kBK; p.rs_blk_stride = 1;
   p.rs_group_stride = b_tile_scaled ? N * (K / kBK) : (N / kTile) * (K / kBK);
+  if (b_rows) {
+    p.ldr = N; p.r_kb_stride = N * kBK;
+    p.rs_row_stride = 1; p.rs_blk_stride = N / kTile;
+  }
   p.C = c; p.ldc = ldc; p.c_group_stride = 0;
   p.bias = bias; p.bias_dtype = bias_dtype; p.bias_group_stride = N;
   p.goff = group_offsets;
   p.Lrows = M; p.Rrows = N; p.nkb = (int)(K / kBK); p.E = E; p.nRt = (int)((N + BN - 1) / BN); p.nLt = 0;
   p.accumulate = 0;
-  if (kernel == kFewRows || kernel == kFewRowsSplit) return launch_few_rows(p, c_dtype, M, kernel == kFewRowsSplit, st);
+  if (kernel == kFewRows || kernel == kFewRowsSplit) return launch_few_rows(p, c_dtype, M, kernel == kFewRowsSplit, b_rows, st);
   const int64_t max_lt = group_offsets ? M / BM + E : (M + BM - 1) / BM;
   const int64_t blocks = max_lt * p.nRt;
+  if (b_rows)
+    return large ? launch_gemm<kRaggedRows, false, CfgLarge, true>(p, c_dtype, blocks, st, g_opt)
+                 : launch_gemm<kRaggedRows, false, CfgSmall, true>(p, c_dtype, blocks, st, g_opt);
   if (large)
     return b_tile_scaled ? launch_gemm<kRaggedRows, true, CfgWgrad>(p, c_dtype, blocks, st, g_opt)
                          : launch_gemm<kRaggedRows, false, CfgLarge>(p, c_dtype, blocks, st, g_opt);
@@ -1357,7 +1391,7 @@ extern "C" int aamd_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, const flo
                                         const float* b_s, int b_tile_scaled, const int64_t* group_offsets, int E,
                                         int32_t* /*tile_ws*/, int64_t M, int64_t N, int64_t K, void* c, int c_dtype,
                                         int64_t ldc, const void* bias, int bias_dtype, void* stream) {
-  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
+  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, false, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
                       stream);
 }
 
@@ -1369,8 +1403,14 @@ extern "C" int aamd_grouped_gemm_fp8_nt_static(const uint8_t* a, int64_t lda, co
                                                int64_t ldc, const void* bias, int bias_dtype, void* stream) {
   AAMD_REQUIRE(E >= 1 && E <= AAMD_STATIC_MAX_GROUPS, "grouped_gemm_nt_static: E=%d exceeds the limit of %d groups (no static scratch is behind it; it is the entry point's contract)",
                E, AAMD_STATIC_MAX_GROUPS);
-  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
+  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, false, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
                       stream);
+}
+
+extern "C" int aamd_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
+                                        const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
+                                        int c_dtype, int64_t ldc, const void* bias, int bias_dtype, void* stream) {
+  return gemm_nt_impl(a, lda, a_s, b, b_s, 0, true, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype, stream);
 }
 #endif  // !AAMD_TUNING
 
@@ -1447,8 +1487,17 @@ extern "C" int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, co
   AAMD_REQUIRE(opts != nullptr, "tuning_grouped_gemm_nt: null options");
   GemmOptions o;
   o.tile = opts[0]; o.group_r = opts[1]; o.gl = opts[2]; o.ls_batch = opts[3];
-  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
+  return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, false, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
                       stream, o);
+}
+extern "C" int aamd_tuning_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b,
+                                               const float* b_s, const int64_t* group_offsets, int E, int64_t M, int64_t N,
+                                               int64_t K, void* c, int c_dtype, int64_t ldc, const void* bias, int bias_dtype,
+                                               const int* opts, void* stream) {
+  AAMD_REQUIRE(opts != nullptr, "tuning_grouped_gemm_nn: null options");
+  GemmOptions o;
+  o.tile = opts[0]; o.group_r = opts[1]; o.gl = opts[2]; o.ls_batch = opts[3];
+  return gemm_nt_impl(a, lda, a_s, b, b_s, 0, true, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype, stream, o);
 }
 extern "C" int aamd_tuning_grouped_gemm_fp8_wgrad(const uint8_t* dyt, const float* sdyt, const uint8_t* xt,
                                                   const float* sxt, int64_t ld_t, int q_t_layout,

@@ -45,6 +45,11 @@ __device__ __forceinline__ v16f mfma_fp8_32x32x64(const v8i& a, const v8i& b, co
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
 }
 
+// Eight bytes of an 8 (rows) x 16 (bytes) block in the LDS, transposed: see grouped_gemm_kernel.
+__device__ __forceinline__ v2i lds_read_transposed(uint32_t addr) {
+  return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(uintptr_t)addr);
+}
+
 // A 64-bit offset the compiler can keep in scalar registers (it is the same in every lane).
 __device__ __forceinline__ int64_t uniform_i64(int64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uint64_t)v);
@@ -52,8 +57,19 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant
+// expression inside the body.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
 // Row-ragged GEMM with block-scaled R for groups of few rows (gemm_few.hip); reads L, R, their scales and strides, C,
-// bias, goff, E, Lrows, Rrows and nkb of the parameters.
-int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, hipStream_t st);
+// bias, goff, E, Lrows, Rrows and nkb of the parameters.  r_rows: R is stored [contraction, Rrows] (R_ROWS of gemm.hip).
+int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st);
 
 }  // namespace aamd

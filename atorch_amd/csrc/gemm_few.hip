@@ -20,15 +20,21 @@
 
 namespace aamd {
 
-// W waves, tiles of 32 WTR weight rows x 32 WTL token rows
-template <typename OUT, int W, int WTR, int WTL>
+// W waves, tiles of 32 WTR weight rows x 32 WTL token rows.  R_ROWS: the weights are stored [contraction, Rrows] and read
+// transposed from the LDS, as in gemm.hip; a block of them is 128 rows of BR bytes there.  That form takes whole cache lines
+// of a row, 128 weight rows x 32 token rows (us, 64 and 32 weight rows x 64 and 32 token rows, 128 x 32 with three waves, with
+// four, and the other orientation: 64 groups of 6 rows, 7168 x 2048 197, 260, 166, 167, 159; 4096 x 7168 350, 474, 324, 326,
+// 307; 64 uneven groups of 128, 2048 x 7168 324, 817, 254, 253, 284), its scales in registers so that two workgroups of
+// 80 KB fit a CU.
+template <typename OUT, int W, int WTR, int WTL, bool R_ROWS>
 __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
   constexpr int BL = 32 * WTL, BR = 32 * WTR;
   constexpr int kPitch = BR + 4;  // floats per row of a wave's partial result in the LDS
-  constexpr int kStage = (BR + BL) * kBK + (WTL == 1 ? 256 : BL * 4 + 256);  // weight rows, token rows, scales
-  constexpr int kLds = W * (kStage > BL * kPitch * 4 ? kStage : BL * kPitch * 4);
+  constexpr int kStage = (BR + BL) * kBK + (WTL == 1 ? 0 : BL * 4 + 256);  // weight rows, token rows, scales
+  constexpr int PL = WTR > 2 ? 32 : BL;  // token rows whose partial results are in the LDS at a time
+  constexpr int kLds = W * (kStage > PL * kPitch * 4 ? kStage : PL * kPitch * 4);
   __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
-  float (*const part)[BL][kPitch] = reinterpret_cast<float (*)[BL][kPitch]>(lds);
+  float (*const part)[PL][kPitch] = reinterpret_cast<float (*)[PL][kPitch]>(lds);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hg = lane >> 5;
@@ -90,10 +96,16 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
   const int nkb = p.nkb;
   uint8_t* const mine = lds + wave * kStage;
   const uint8_t* const Lb = p.L + uniform_i64(l0 * p.ldl);
-  const uint8_t* const Rb = p.R + uniform_i64((int64_t)g * p.r_group_stride + (int64_t)r0 * p.ldr);
+  const uint8_t* const Rb = p.R + uniform_i64((int64_t)g * p.r_group_stride + (R_ROWS ? (int64_t)r0 : (int64_t)r0 * p.ldr));
   const int r8 = lane >> 3;
   const uint32_t chunk[2] = {(uint32_t)(((lane & 7) ^ r8) << 4), (uint32_t)(((lane & 7) ^ r8 ^ 1) << 4)};
   const uint32_t roff[2] = {(uint32_t)r8 * (uint32_t)p.ldr + chunk[0], (uint32_t)r8 * (uint32_t)p.ldr + chunk[1]};
+  // (R_ROWS) the chunks of row k are XORed with twice its place among the eight rows that are read together, counted in
+  // rows of 256 bytes
+  constexpr int kChunks = BR / 16, kRowsPer1K = 1024 / BR, kRowsPer256 = 256 / BR;
+  const uint32_t roff_t = (uint32_t)(lane / kChunks) * (uint32_t)p.ldr +
+                          (uint32_t)((lane % kChunks) ^ (2 * (((lane / kChunks) & 7) / kRowsPer256))) * 16u;
+  const int tr = (lane & 15) >> 1;
   uint32_t loff[4 * WTL];
 #pragma unroll
   for (int n = 0; n < 4 * WTL; n++) {
@@ -101,32 +113,38 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
     loff[n] = (uint32_t)row * (uint32_t)p.ldl + chunk[n & 1];
   }
   const int nl = (lvalid + 7) >> 3;  // slabs of token rows, >= 1
-  // scales of a block, [BL token rows][the weights' block]: with 32 token rows the upper lanes of the one load fetch
-  // the latter, else a load of its own does
+  // scales of a block: with 32 token rows in registers, requested ahead of the block, else [BL token rows][the weights' block]
+  // in the stage
   const float* const rs = p.Rs + (int64_t)g * p.rs_group_stride + (int64_t)(r0 / kTile) * p.rs_row_stride;
   const float* sbase[(WTL + 1) / 2];
 #pragma unroll
   for (int n = 0; n < (WTL + 1) / 2; n++) {
-    const int row = n * 64 + lane < lvalid ? n * 64 + lane : lvalid - 1;
-    sbase[n] = WTL == 1 && lane >= 32 ? rs : p.Ls + (l0 + row) * p.ls_row_stride;
+    const int row = WTL == 1 ? l32 : n * 64 + lane;
+    sbase[n] = p.Ls + (l0 + (row < lvalid ? row : lvalid - 1)) * p.ls_row_stride;
   }
+  float ls_next = 0.f, rs_next = 0.f;  // (WTL == 1)
   constexpr int kScales = (BR + BL) * kBK;  // offset in the stage
   const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)mine;
   auto load = [&](int k) __attribute__((always_inline)) {
-    const uint8_t* const R = Rb + (int64_t)k * kBK;
+    const uint8_t* const R = Rb + k * p.r_kb_stride;
     const uint8_t* const L = Lb + (int64_t)k * kBK;
+    if constexpr (WTL == 1) {
+      ls_next = sbase[0][k];
+      rs_next = rs[k * p.rs_blk_stride];
+    }
 #pragma unroll
     for (int n = 0; n < BR / 8; n++)
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(roff[n & 1]), "s"(R + (int64_t)(n * 8) * p.ldr), "s"(base + n * 1024) : "memory");
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(R_ROWS ? roff_t : roff[n & 1]), "s"(R + (int64_t)(n * (R_ROWS ? kRowsPer1K : 8)) * p.ldr), "s"(base + n * 1024) : "memory");
 #pragma unroll
     for (int n = 0; n < 4 * WTL; n++)
       if (n < nl)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(loff[n]), "s"(L), "s"(base + BR * kBK + n * 1024) : "memory");
+    if constexpr (WTL > 1) {
 #pragma unroll
-    for (int n = 0; n < (WTL + 1) / 2; n++)
-      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(sbase[n] + k), "s"(base + kScales + n * 256) : "memory");
-    if constexpr (WTL > 1)
-      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(rs + k), "s"(base + kScales + BL * 4) : "memory");
+      for (int n = 0; n < (WTL + 1) / 2; n++)
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(sbase[n] + k), "s"(base + kScales + n * 256) : "memory");
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(rs + k * p.rs_blk_stride), "s"(base + kScales + BL * 4) : "memory");
+    }
   };
   v16f acc[WTR][WTL], zero;
 #pragma unroll
@@ -152,10 +170,22 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
 #pragma unroll
       for (int j = 0; j < WTL; j++) lf[j][h] = frag(mine + (BR + j * 32 + l32) * kBK, h);
 #pragma unroll
-      for (int i = 0; i < WTR; i++) rf[i][h] = frag(mine + (i * 32 + l32) * kBK, h);
+      for (int i = 0; i < WTR; i++) {
+        if constexpr (R_ROWS) {
+          const uint32_t at = base + (uint32_t)((64 * h + 32 * hg + tr) * BR + (((2 * i + ((lane >> 4) & 1)) ^ (2 * (tr / kRowsPer256))) << 4) + (lane & 1) * 8);
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const v2i o = lds_read_transposed(at + (uint32_t)(8 * j * BR));
+            rf[i][h][2 * j] = o[0];
+            rf[i][h][2 * j + 1] = o[1];
+          }
+        } else {
+          rf[i][h] = frag(mine + (i * 32 + l32) * kBK, h);
+        }
+      }
     }
 #pragma unroll
-    for (int j = 0; j < WTL; j++) sc[j] = S[j * 32 + l32] * S[BL];
+    for (int j = 0; j < WTL; j++) sc[j] = WTL == 1 ? ls_next * rs_next : S[j * 32 + l32] * S[BL];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and has been read: its place may be filled again
     if (kb + W < nkb) load(kb + W);
 #pragma unroll
@@ -171,38 +201,44 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
   __syncthreads();  // every wave is done with its stages: the memory holds the partial results now
 
   // ---- sum over the waves, through the LDS; a lane holds column l32 and rows 8q + 4hg .. + 3 of every 32 x 32 sub-tile
+  // (with 128 weight rows 32 token rows at a time, which fit the stages' memory)
+  static_for<BL / PL>([&](auto J0) {
+    constexpr int j0 = decltype(J0)::value * (PL / 32);
+    if (j0 > 0) __syncthreads();
 #pragma unroll
-  for (int i = 0; i < WTR; i++)
+    for (int i = 0; i < WTR; i++)
 #pragma unroll
-    for (int j = 0; j < WTL; j++)
+      for (int j = 0; j < PL / 32; j++)
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        *reinterpret_cast<v4f*>(&part[wave][j * 32 + l32][i * 32 + 8 * q + 4 * hg]) =
-            v4f{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-  __syncthreads();
-  for (int c = tid; c < BL * (BR / 4); c += 64 * W) {
-    const int row = c / (BR / 4), col = (c % (BR / 4)) * 4;
-    if (row >= lvalid) break;  // (rows only grow with c)
-    v4f o = *reinterpret_cast<const v4f*>(&part[0][row][col]);
+        for (int q = 0; q < 4; q++) {
+          const v16f& a = acc[i][j0 + j];
+          *reinterpret_cast<v4f*>(&part[wave][j * 32 + l32][i * 32 + 8 * q + 4 * hg]) = v4f{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+        }
+    __syncthreads();
+    for (int c = tid; c < PL * (BR / 4); c += 64 * W) {
+      const int prow = c / (BR / 4), row = j0 * 32 + prow, col = (c % (BR / 4)) * 4;
+      if (row >= lvalid) break;  // (rows only grow with c)
+      v4f o = *reinterpret_cast<const v4f*>(&part[0][prow][col]);
 #pragma unroll
-    for (int w = 1; w < W; w++) o += *reinterpret_cast<const v4f*>(&part[w][row][col]);
-    if (p.bias != nullptr) {
-      const int64_t at = (int64_t)g * p.bias_group_stride + r0 + col;
-      if (p.bias_dtype == AAMD_F32) {
-        o += *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(p.bias) + at);
+      for (int w = 1; w < W; w++) o += *reinterpret_cast<const v4f*>(&part[w][prow][col]);
+      if (p.bias != nullptr) {
+        const int64_t at = (int64_t)g * p.bias_group_stride + r0 + col;
+        if (p.bias_dtype == AAMD_F32) {
+          o += *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(p.bias) + at);
+        } else {
+          const v2i raw = *reinterpret_cast<const v2i*>(reinterpret_cast<const u16*>(p.bias) + at);
+          o += v4f{bf16_bits_to_f32((uint32_t)raw[0] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[0] >> 16),
+                   bf16_bits_to_f32((uint32_t)raw[1] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[1] >> 16)};
+        }
+      }
+      OUT* const dst = reinterpret_cast<OUT*>(p.C) + (l0 + row) * p.ldc + r0 + col;
+      if constexpr (sizeof(OUT) == 4) {
+        *reinterpret_cast<v4f*>(dst) = o;
       } else {
-        const v2i raw = *reinterpret_cast<const v2i*>(reinterpret_cast<const u16*>(p.bias) + at);
-        o += v4f{bf16_bits_to_f32((uint32_t)raw[0] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[0] >> 16),
-                 bf16_bits_to_f32((uint32_t)raw[1] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[1] >> 16)};
+        *reinterpret_cast<v2i*>(dst) = v2i{(int)pack_bf16x2(o[0], o[1]), (int)pack_bf16x2(o[2], o[3])};
       }
     }
-    OUT* const dst = reinterpret_cast<OUT*>(p.C) + (l0 + row) * p.ldc + r0 + col;
-    if constexpr (sizeof(OUT) == 4) {
-      *reinterpret_cast<v4f*>(dst) = o;
-    } else {
-      *reinterpret_cast<v2i*>(dst) = v2i{(int)pack_bf16x2(o[0], o[1]), (int)pack_bf16x2(o[2], o[3])};
-    }
-  }
+  });
 }
 
 // Upper bound of the token tiles of M rows in E groups (the groups' sizes are known on the device only).
@@ -211,13 +247,13 @@ static int64_t few_rows_tiles(int64_t M, int E, int rows) {
   return M / rows + groups < M ? M / rows + groups : M;
 }
 
-template <typename OUT, int W, int WTR, int WTL>
+template <typename OUT, int W, int WTR, int WTL, bool R_ROWS>
 static int launch_few(GemmParams p, int64_t M, hipStream_t st) {
   p.nRt = (int)(p.Rrows / (32 * WTR));
   const int64_t lt = p.goff ? few_rows_tiles(M, p.E, 32 * WTL) : (M + 32 * WTL - 1) / (32 * WTL);
   const int64_t blocks = lt * p.nRt;
   AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
-  few_rows_kernel<OUT, W, WTR, WTL><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p);
+  few_rows_kernel<OUT, W, WTR, WTL, R_ROWS><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p);
   AAMD_LAUNCH_CHECK("grouped_gemm (few rows)");
   return AAMD_OK;
 }
@@ -225,11 +261,12 @@ static int launch_few(GemmParams p, int64_t M, hipStream_t st) {
 // `split`: the form for launches of few workgroups, which divides the contraction among eight waves and takes half the
 // weight rows and token rows per workgroup.
 template <typename OUT>
-static int launch_few_as(const GemmParams& p, int64_t M, bool split, hipStream_t st) {
-  return split ? launch_few<OUT, 8, 1, 1>(p, M, st) : launch_few<OUT, 4, 2, 2>(p, M, st);
+static int launch_few_as(const GemmParams& p, int64_t M, bool split, bool r_rows, hipStream_t st) {
+  if (r_rows) return launch_few<OUT, 4, 4, 1, true>(p, M, st);
+  return split ? launch_few<OUT, 8, 1, 1, false>(p, M, st) : launch_few<OUT, 4, 2, 2, false>(p, M, st);
 }
-int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, hipStream_t st) {
-  return c_dtype == AAMD_BF16 ? launch_few_as<u16>(p, M, split, st) : launch_few_as<float>(p, M, split, st);
+int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st) {
+  return c_dtype == AAMD_BF16 ? launch_few_as<u16>(p, M, split, r_rows, st) : launch_few_as<float>(p, M, split, r_rows, st);
 }
 
 }  // namespace aamd

@@ -184,18 +184,29 @@ std::tuple<Quantised, Tensor> act_dual(const Tensor& fc1, const Tensor& dh, bool
 }
 
 // ---- grouped GEMMs ---------------------------------------------------------------------------
+// Is the stack b [E, N, K] the transposed view of a dense [E, K, N]?  (Sizes are multiples of 128.)
+bool is_transposed_view(const Tensor& b) {
+  return b.dim() == 3 && b.size(2) > 1 && b.stride(1) == 1 && b.stride(2) == b.size(1) && b.stride(0) == b.size(1) * b.size(2);
+}
 Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, const OptTensor& goff, const OptTensor& out,
                at::ScalarType out_dtype, const OptTensor& bias) {
   const int64_t M = a.size(0), K = a.size(1), E = b.size(0), N = b.size(1);
-  const bool b_tile_scaled = b_s.size(1) == N;
-  require(b.size(2) == K && a.stride(1) == 1 && b.is_contiguous(), "rows and weights must share their contraction length");
-  require(a_s.numel() >= M * (K / kTile) && b_s.numel() >= E * (b_tile_scaled ? N : N / kTile) * (K / kTile) &&
-              a_s.is_contiguous() && b_s.is_contiguous(),
+  const bool b_rows = is_transposed_view(b), b_tile_scaled = !b_rows && b_s.size(1) == N;
+  require(b.size(2) == K && a.stride(1) == 1 && (b_rows || b.is_contiguous()), "rows and weights must share their contraction length");
+  require(a_s.numel() >= M * (K / kTile) && b_s.numel() >= E * (b_tile_scaled ? N : N / kTile) * (K / kTile) && a_s.is_contiguous() &&
+              (!b_rows || (b_s.dim() == 3 && b_s.size(1) == N / kTile)),
           "scales do not cover the codes");
+  // (codes and scales come as views of one layout; who keeps tensors for a backward may have made one of them dense)
+  const Tensor bs = b_rows ? b_s.transpose(1, 2).contiguous() : b_s.contiguous();
   if (goff.has_value()) check_offsets(*goff, E);
   if (bias.has_value()) check_bias(*bias, E, N);
   Tensor c = out.has_value() ? *out : empty({M, N}, out_dtype, a);
-  check(aamd_grouped_gemm_fp8_nt(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(b_s), b_tile_scaled,
+  if (b_rows)
+    check(aamd_grouped_gemm_fp8_nn(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(bs), ptr<int64_t>(goff),
+                                   (int)E, M, N, K, ptr(c), dtype_code(c.scalar_type()), c.stride(0), ptr(bias),
+                                   bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
+  else
+    check(aamd_grouped_gemm_fp8_nt(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(bs), b_tile_scaled,
                                  ptr<int64_t>(goff), (int)E, nullptr, M, N, K, ptr(c), dtype_code(c.scalar_type()), c.stride(0),
                                  ptr(bias), bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
   return c;
@@ -399,34 +410,53 @@ std::optional<Spaced> spaced(const std::vector<Tensor>& ts, int64_t n) {
   return Spaced{base, step / size};
 }
 
-// 128x128 codes of weights [N, K] into stacked outputs
+// 128x128 codes of weights [N, K] into stacked outputs: as stored, and with `transpose` in the other orientation too.  The
+// scale is that of a whole block, so the codes are the same bytes either way, and with `one` only one orientation is
+// written and the other pair is its transposed view, which gemm_nt reads as well: kStored writes the codes as stored,
+// kTurned the transposed ones.  (A weight is read by two products, one along each side.)
+enum Written { kBoth = 0, kStored = 1, kTurned = 2 };
 struct BlockQuantised {
   Tensor q, s, q_t, s_t;
-  BlockQuantised(int64_t E, int64_t N, int64_t K, bool transpose, const Tensor& like)
-      : q(empty({E, N, K}, kFp8, like)), s(empty({E, N / kTile, K / kTile}, at::kFloat, like)) {
-    if (!transpose) return;
-    q_t = empty({E, K, N}, kFp8, like);
-    s_t = empty({E, K / kTile, N / kTile}, at::kFloat, like);
+  int64_t N, K;
+  BlockQuantised(int64_t E, int64_t N, int64_t K, bool transpose, int one, const Tensor& like) : N(N), K(K) {
+    require(one >= kBoth && one <= kTurned && (transpose || one == kBoth), "one written orientation stands for two");
+    if (one != kTurned) {
+      q = empty({E, N, K}, kFp8, like);
+      s = empty({E, N / kTile, K / kTile}, at::kFloat, like);
+    }
+    if (transpose && one != kStored) {
+      q_t = empty({E, K, N}, kFp8, like);
+      s_t = empty({E, K / kTile, N / kTile}, at::kFloat, like);
+    }
   }
   void run(const void* w, at::ScalarType dtype, int64_t first, int64_t E, int64_t stride, double eps) {
-    const int64_t N = q.size(1), K = q.size(2), at = first * N * K, at_s = first * (N / kTile) * (K / kTile);
-    check(aamd_quant_128x128(w, dtype_code(dtype, true), E, N, K, stride, ptr<uint8_t>(q) + at, ptr<float>(s) + at_s,
+    const int64_t at = first * N * K, at_s = first * (N / kTile) * (K / kTile);
+    if (!q.defined())
+      check(aamd_quant_128x128_t(w, dtype_code(dtype, true), E, N, K, stride, ptr<uint8_t>(q_t) + at, ptr<float>(s_t) + at_s,
+                                 (float)eps, stream()));
+    else
+      check(aamd_quant_128x128(w, dtype_code(dtype, true), E, N, K, stride, ptr<uint8_t>(q) + at, ptr<float>(s) + at_s,
                              q_t.defined() ? ptr<uint8_t>(q_t) + at : nullptr, s_t.defined() ? ptr<float>(s_t) + at_s : nullptr,
                              (float)eps, stream()));
   }
-  std::tuple<Tensor, Tensor, OptTensor, OptTensor> get() const { return {q, s, opt(q_t), opt(s_t)}; }
+  std::tuple<Tensor, Tensor, OptTensor, OptTensor> get(bool transpose) const {
+    if (!transpose) return {q, s, {}, {}};
+    if (!q.defined()) return {q_t.transpose(1, 2), s_t.transpose(1, 2), q_t, s_t};
+    if (!q_t.defined()) return {q, s, q.transpose(1, 2), s.transpose(1, 2)};
+    return {q, s, q_t, s_t};
+  }
 };
-std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose) {
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose, int one) {
   const int64_t E = w.size(0), N = w.size(1), K = w.size(2);
-  BlockQuantised r(E, N, K, transpose, w);
+  BlockQuantised r(E, N, K, transpose, one, w);
   r.run(ptr(w), w.scalar_type(), 0, E, E > 1 ? w.stride(0) : N * K, eps);
-  return r.get();
+  return r.get(transpose);
 }
 // The same from separate tensors of one shape: in one launch where they are equally far apart; else in one launch each or,
 // small ones, from a copy (us, the one launch / copied / one launch each: 60 x 512 x 512 13 / 28 / 232, 60 x 1024 x 1024
 // 44 / 94 / 246, 8 x 1024 x 4096 24 / 51 / 39, 64 x 1408 x 2048 126 / 363 / 290, 8 x 28672 x 4096 661 / 1949 / 702).
 constexpr int64_t kWeightOfItsOwn = (int64_t)1 << 21;  // elements
-std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant_list(const std::vector<Tensor>& ws, double eps, bool transpose) {
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant_list(const std::vector<Tensor>& ws, double eps, bool transpose, int one) {
   require(!ws.empty() && ws[0].dim() == 2, "weights must be matrices");
   const int64_t E = (int64_t)ws.size(), N = ws[0].size(0), K = ws[0].size(1);
   bool direct = N * K >= kWeightOfItsOwn;
@@ -435,12 +465,12 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant_list(const std::vec
     direct = direct && w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
   }
   const auto at = spaced(ws, N * K);
-  if (!at.has_value() && !direct) return block_quant(at::stack(ws), eps, transpose);
-  BlockQuantised r(E, N, K, transpose, ws[0]);
+  if (!at.has_value() && !direct) return block_quant(at::stack(ws), eps, transpose, one);
+  BlockQuantised r(E, N, K, transpose, one, ws[0]);
   if (at.has_value()) r.run(at->base, ws[0].scalar_type(), 0, E, at->stride, eps);
   else
     for (int64_t e = 0; e < E; e++) r.run(ptr(ws[e]), ws[e].scalar_type(), e, 1, N * K, eps);
-  return r.get();
+  return r.get(transpose);
 }
 
 // ---- the expert MLP --------------------------------------------------------------------------
@@ -628,8 +658,8 @@ PYBIND11_MODULE(_host, m) {
     const auto shape = qt_shape(rows, ld_t, blocked);
     return std::vector<int64_t>(shape.begin(), shape.end());
   });
-  m.def("block_quant", &block_quant);
-  m.def("block_quant_list", &block_quant_list);
+  m.def("block_quant", &block_quant, py::arg("w"), py::arg("eps"), py::arg("transpose"), py::arg("one") = (int)kBoth);
+  m.def("block_quant_list", &block_quant_list, py::arg("ws"), py::arg("eps"), py::arg("transpose"), py::arg("one") = (int)kBoth);
   m.def("gemm_nt", &gemm_nt);
   m.def("gemm_wgrad", &gemm_wgrad);
   m.def("transpose_scales", &transpose_scales);

@@ -1014,15 +1014,16 @@ __global__ __launch_bounds__(256) void quant_128x128_kernel(const typename IN::e
   const Divider dv = make_scale(m, eps, plain_div);
   const float sc = dv.s;
   if (threadIdx.x == 0) {
-    s[((int64_t)e * nnb + nb) * nkb + kb] = sc;
+    if (s != nullptr) s[((int64_t)e * nnb + nb) * nkb + kb] = sc;
     if (s_t != nullptr) s_t[((int64_t)e * nkb + kb) * nnb + nb] = sc;
   }
-  uint8_t* qe = q + (int64_t)e * N * K + (int64_t)nb * kTile * K + (int64_t)kb * kTile;
   v2i codes[8];
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    codes[i] = quant8(v[i], dv);
-    st_nt(qe, (uint32_t)(gr * 8 + i) * (uint32_t)K + (uint32_t)c * 8, codes[i]);
+  for (int i = 0; i < 8; i++) codes[i] = quant8(v[i], dv);
+  if (q != nullptr) {
+    uint8_t* qe = q + (int64_t)e * N * K + (int64_t)nb * kTile * K + (int64_t)kb * kTile;
+#pragma unroll
+    for (int i = 0; i < 8; i++) st_nt(qe, (uint32_t)(gr * 8 + i) * (uint32_t)K + (uint32_t)c * 8, codes[i]);
   }
   if (q_t != nullptr) {
     // one scale for the whole block: the transposed copy holds the same codes, so the 8x8 block of
@@ -1479,18 +1480,17 @@ extern "C" int aamd_group_sums(const float* tile_sums, int64_t cols, const int64
   return AAMD_OK;
 }
 
-extern "C" int aamd_quant_128x128(const void* w, int w_dtype, int64_t E, int64_t N, int64_t K,
-                                  int64_t expert_stride, uint8_t* q, float* s, uint8_t* q_t, float* s_t, float eps,
-                                  void* stream) {
+// q and s, or q_t and s_t, may be null
+static int block_quant_impl(const void* w, int w_dtype, int64_t E, int64_t N, int64_t K, int64_t expert_stride, uint8_t* q,
+                            float* s, uint8_t* q_t, float* s_t, float eps, void* stream) {
   AAMD_REQUIRE(w_dtype == AAMD_BF16 || w_dtype == AAMD_F32 || w_dtype == AAMD_F16, "quant_128x128: unsupported dtype %d", w_dtype);
   AAMD_REQUIRE(E >= 0 && N >= 0 && K >= 0 && N % kTile == 0 && K % kTile == 0,
                "quant_128x128: N=%lld and K=%lld must be multiples of 128", (long long)N, (long long)K);
-  AAMD_REQUIRE((q_t == nullptr) == (s_t == nullptr), "quant_128x128: q_t and s_t go together");
   AAMD_REQUIRE(N < kMaxTileLd && K < kMaxTileLd, "quant_128x128: N=%lld or K=%lld too large", (long long)N, (long long)K);
   if (E == 0 || N == 0 || K == 0) return AAMD_OK;
-  AAMD_REQUIRE(w && q && s, "quant_128x128: null pointer");
+  AAMD_REQUIRE(w && ((q && s) || (q_t && s_t)), "quant_128x128: null pointer");
   AAMD_REQUIRE(expert_stride >= N * K && expert_stride % 8 == 0, "quant_128x128: bad expert stride");
-  AAMD_REQUIRE(aligned16(w) && aligned16(q) && (!q_t || aligned16(q_t)), "quant_128x128: pointers must be 16-byte aligned");
+  AAMD_REQUIRE(aligned16(w) && (!q || aligned16(q)) && (!q_t || aligned16(q_t)), "quant_128x128: pointers must be 16-byte aligned");
   AAMD_REQUIRE(N / kTile <= 65535 && E <= 65535, "quant_128x128: grid too large");
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(K / kTile), (unsigned)(N / kTile), (unsigned)E), block(256);
@@ -1506,6 +1506,19 @@ extern "C" int aamd_quant_128x128(const void* w, int w_dtype, int64_t E, int64_t
     quant_128x128_kernel<F32><<<grid, block, 0, st>>>((const float*)w, expert_stride, N, K, q, s, q_t, s_t, eps, rows_per_xcd);
   AAMD_LAUNCH_CHECK("quant_128x128");
   return AAMD_OK;
+}
+
+extern "C" int aamd_quant_128x128(const void* w, int w_dtype, int64_t E, int64_t N, int64_t K,
+                                  int64_t expert_stride, uint8_t* q, float* s, uint8_t* q_t, float* s_t, float eps,
+                                  void* stream) {
+  AAMD_REQUIRE((q_t == nullptr) == (s_t == nullptr), "quant_128x128: q_t and s_t go together");
+  AAMD_REQUIRE((q && s) || E <= 0 || N <= 0 || K <= 0, "quant_128x128: null pointer");
+  return block_quant_impl(w, w_dtype, E, N, K, expert_stride, q, s, q_t, s_t, eps, stream);
+}
+
+extern "C" int aamd_quant_128x128_t(const void* w, int w_dtype, int64_t E, int64_t N, int64_t K, int64_t expert_stride,
+                                    uint8_t* q_t, float* s_t, float eps, void* stream) {
+  return block_quant_impl(w, w_dtype, E, N, K, expert_stride, nullptr, nullptr, q_t, s_t, eps, stream);
 }
 
 extern "C" int aamd_transpose_scales(const float* s, int64_t rows, int64_t blocks, float* s_t, void* stream) {

@@ -47,31 +47,30 @@ class TokenDispatch(NamedTuple):
 
 def _quant_first_weight(w1, v1, transpose_w1, need_transpose=True):
     """Codes and scales of the first layer as the logical ``[E, N1, H]`` operand (N1 = 2F with SwiGLU) and
-    its transpose ``[E, H, N1]``, from ``w1`` (and ``v1``) in either storage orientation."""
-    q, s, q_t, s_t = kernels.block_quant_batched(w1.detach().contiguous(), return_transpose=True)
-    if v1 is not None:
-        qv, sv, qv_t, sv_t = kernels.block_quant_batched(v1.detach().contiguous(), return_transpose=True)
-        if transpose_w1:  # stored [E, F, H]: gate rows on top of up rows
-            q, s = torch.cat([q, qv], dim=1), torch.cat([s, sv], dim=1)
-            q_t, s_t = torch.cat([q_t, qv_t], dim=2), torch.cat([s_t, sv_t], dim=2)
-        else:  # stored [E, H, F]
-            q, s = torch.cat([q, qv], dim=2), torch.cat([s, sv], dim=2)
-            q_t, s_t = torch.cat([q_t, qv_t], dim=1), torch.cat([s_t, sv_t], dim=1)
-    if not transpose_w1:
-        q, s, q_t, s_t = q_t, s_t, q, s
-    return q, s, q_t, s_t
+    its transpose ``[E, H, N1]``, from ``w1`` (and ``v1``) in either storage orientation.  The forward's operand is
+    written; the other is its view."""
+    first = 0 if transpose_w1 else 2  # stored [E, F, H] or [E, H, F]
+    parts = [_written_once(w, not transpose_w1)[first : first + 2] for w in (w1, v1) if w is not None]
+    # gate rows on top of up rows
+    q, s = parts[0] if v1 is None else (torch.cat(p, dim=1) for p in zip(*parts))
+    return q, s, q.transpose(1, 2), s.transpose(1, 2)
+
+
+def _written_once(w, turned):
+    return kernels.block_quant_batched(w.detach().contiguous(), return_transpose=True,
+                                       written=kernels.TURNED if turned else kernels.STORED)  # fmt: skip
 
 
 def _weight_codes(w1, w2, v1, transpose_w1, is_first_microbatch, weight_cache):
     """``(q1, s1, q1_t, s1_t), (q2, s2, q2_t, s2_t)``: the first weight(s) as [E, N1, H] (rows = outputs) and the second
-    as [E, F, H], each with its transpose; block quantisation commutes with the transpose, so both orientations
-    come out of one launch each."""
+    as [E, F, H], each with its transpose; block quantisation commutes with the transpose, so the codes of one
+    orientation are those of the other as well: the forward's operands are written, the backward reads their views."""
     if weight_cache is not None:
         held = weight_cache.held((("w1", (w1, v1)), ("w2", (w2,))), is_first_microbatch, True)
         if held is not None:
             return held
     quant1 = lambda t: _quant_first_weight(w1, v1, transpose_w1)  # noqa: E731
-    quant2 = lambda t: kernels.block_quant_batched(w2.detach().contiguous(), return_transpose=True)  # noqa: E731
+    quant2 = lambda t: _written_once(w2, True)  # noqa: E731
     if weight_cache is None:
         return quant1(True), quant2(True)
     return (weight_cache.codes("w1", (w1, v1), is_first_microbatch, True, quant1),

@@ -37,8 +37,10 @@ class _Fp8Gmm(torch.autograd.Function):
         # weight as [E, N, K]: block quantisation commutes with the transpose, so for
         # trans_b == False the transposed output of the quantiser is the [N, K] operand.
         # Under no_grad only the orientation the forward GEMM reads is needed when that is the stored one.
+        # Codes are written in one orientation: as stored where both products follow, else the forward's.
         both = need_grad or not trans_b
-        quantise = lambda t: kernels.block_quant_batched(b.detach().contiguous(), return_transpose=t)  # noqa: E731
+        written = kernels.STORED if need_grad or trans_b else kernels.TURNED
+        quantise = lambda t: kernels.block_quant_batched(b.detach().contiguous(), return_transpose=t, written=written)  # noqa: E731
         if weight_cache is None:
             qb, sb, qb_t, sb_t = quantise(both)
         else:

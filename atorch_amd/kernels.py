@@ -336,11 +336,17 @@ def gradient_quant_with_sums(x: torch.Tensor, group_offsets: torch.Tensor, num_g
     return host().dual_with_sums(what, x, dh, group_offsets, num_groups, ld_t, eps, sums_dtype)
 
 
-def block_quant_batched(w: torch.Tensor, eps: float = 0.0, return_transpose: bool = False):
+# which orientation of a weight's codes is written (csrc/host.cpp): both, the one of the weight's own layout, the other one
+BOTH, STORED, TURNED = 0, 1, 2
+
+
+def block_quant_batched(w: torch.Tensor, eps: float = 0.0, return_transpose: bool = False, written: int = BOTH):
     """128x128 block quantisation of ``w [E, N, K]`` in one launch.
-    Returns ``(q [E,N,K], s [E,N/128,K/128], q_t [E,K,N] | None, s_t [E,K/128,N/128] | None)``."""
+    Returns ``(q [E,N,K], s [E,N/128,K/128], q_t [E,K,N] | None, s_t [E,K/128,N/128] | None)``.  With
+    ``return_transpose``, ``written`` STORED (TURNED) writes only q and s (q_t and s_t), and the other two are their
+    transposed views, which ``grouped_gemm_nt`` takes as well."""
     assert w.dim() == 3 and w.stride(2) == 1 and w.stride(1) == w.size(2), "rows of w must be dense"
-    return host().block_quant(w, eps, return_transpose)
+    return host().block_quant(w, eps, return_transpose, written if return_transpose else BOTH)
 
 
 def grouped_gemm_nt(
@@ -354,10 +360,13 @@ def grouped_gemm_nt(
     bias: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """out[m] = a[m] @ b[g(m)]^T with block scales, for rows m of group g (device offsets).
-    a [M,K] fp8, a_s [M,K/128], b [E,N,K] fp8, b_s [E,N/128,K/128] or [E,N,K/128]."""
+    a [M,K] fp8, a_s [M,K/128], b [E,N,K] fp8, b_s [E,N/128,K/128] or [E,N,K/128]; b with block scales may also be the
+    transposed view of dense codes [E,K,N], and b_s that of their scales."""
     M, K = a.shape
     E, N, Kb = b.shape
-    assert Kb == K and a.stride(1) == 1 and b.is_contiguous() and a_s.is_contiguous() and b_s.is_contiguous()
+    turned = not b.is_contiguous()
+    dense, dense_s = (b.transpose(1, 2), b_s.transpose(1, 2)) if turned else (b, b_s)
+    assert Kb == K and a.stride(1) == 1 and dense.is_contiguous() and a_s.is_contiguous() and dense_s.is_contiguous()
     assert group_offsets.dtype == torch.int64 and group_offsets.numel() == E + 1
     assert out is None or (out.shape == (M, N) and out.stride(1) == 1)
     assert bias is None or (bias.shape == (E, N) and bias.is_contiguous())
@@ -368,11 +377,14 @@ def grouped_gemm_nt(
 
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nt(
-        ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), int(b_s.size(1) == N), ptr(group_offsets), E, None, M, N, K, ptr(out),
-        dtype_code(out.dtype), out.stride(0), ptr(bias), dtype_code(bias.dtype) if bias is not None else _lib.NONE,
-        _probes.options_array(pinned), stream(),
-    ))  # fmt: skip
+    rest = (M, N, K, ptr(out), dtype_code(out.dtype), out.stride(0), ptr(bias),
+            dtype_code(bias.dtype) if bias is not None else _lib.NONE, _probes.options_array(pinned), stream())  # fmt: skip
+    if turned:
+        _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nn(
+            ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), ptr(group_offsets), E, *rest))  # fmt: skip
+    else:
+        _probes.check(_probes.lib().aamd_tuning_grouped_gemm_fp8_nt(
+            ptr(a), a.stride(0), ptr(a_s), ptr(b), ptr(b_s), int(b_s.size(1) == N), ptr(group_offsets), E, None, *rest))  # fmt: skip
     return out
 
 

@@ -76,8 +76,8 @@ class QuantizeResult:
 
 
 class WeightCodeStack:
-    """Codes of all weights of a module, stacked (data, scale, data_t | None, scale_t | None), and the per-weight caches
-    that point into them.  ``whole`` while all of those still do."""
+    """Codes of all weights of a module, stacked (data, scale, data_t | None, scale_t | None; the latter two may be views of
+    the former), and the per-weight caches that point into them.  ``whole`` while all of those still do."""
 
     __slots__ = ("codes", "members", "whole")
 
@@ -133,7 +133,8 @@ class QuantizeResultCache:
 
     def _get(self, k: int) -> Optional[torch.Tensor]:
         if self._own[k] is None and self.stack is not None and self.stack.codes[k] is not None:
-            self._own[k] = self.stack.codes[k][self.index]
+            # (the stack may hold one orientation and a view of it)
+            self._own[k] = self.stack.codes[k][self.index].contiguous()
         return self._own[k]
 
     def _set(self, k: int, value: Optional[torch.Tensor]):

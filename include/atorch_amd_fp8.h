@@ -140,6 +140,14 @@ int aamd_quant_128x128(const void *w, int w_dtype, int64_t E, int64_t N, int64_t
                        uint8_t *q, float *s, uint8_t *q_t, float *s_t, float eps, void *stream);
 
 /*
+ * The codes of aamd_quant_128x128 in the transposed orientation only (q_t [E, K, N], s_t [E, K/128, N/128]): a weight whose
+ * product reads it that way, where the other product reads the same bytes through aamd_grouped_gemm_fp8_nn.
+ * Replaces the transposed half of quantize_square_blockwise, cuda_kernel.py:41-61.
+ */
+int aamd_quant_128x128_t(const void *w, int w_dtype, int64_t E, int64_t N, int64_t K, int64_t expert_stride,
+                         uint8_t *q_t, float *s_t, float eps, void *stream);
+
+/*
  * Dequantisation y = code * scale.
  * Replaces dequant, triton_kernel.py:49-91.  tile_scale != 0: s [M, N/128]; else s [M/128, N/128].
  */
@@ -220,6 +228,18 @@ int aamd_grouped_gemm_fp8_nt(const uint8_t *a, int64_t lda, const float *a_s, co
                              int b_tile_scaled, const int64_t *group_offsets, int E, int32_t *tile_ws, int64_t M,
                              int64_t N, int64_t K, void *c, int c_dtype, int64_t ldc, const void *bias,
                              int bias_dtype, void *stream);
+
+/*
+ * The same GEMM with the weights stored as their contraction runs down the rows, b [E, K, N] and b_s [E, K/128, N/128]
+ * (block scales): C[m, n] = sum_kb dot(A[m, kb], B_g[kb, n]) * a_s[m, kb] * b_s_g[kb, n/128] (+ bias_g[n]).  The gradient of
+ * the rows reads the codes of the forward product this way (and a weight stored [E, K, N] those of its own layout), so that
+ * one orientation of the codes is written and kept; results are those of aamd_grouped_gemm_fp8_nt on the transposed codes,
+ * bit for bit where both take the same kernel.  N < 2^23; everything else as there.
+ * Replaces quantize_op.grouped_qgemm for dgrad, quantized_grouped_linear.py:214-223.
+ */
+int aamd_grouped_gemm_fp8_nn(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b, const float *b_s,
+                             const int64_t *group_offsets, int E, int64_t M, int64_t N, int64_t K, void *c, int c_dtype,
+                             int64_t ldc, const void *bias, int bias_dtype, void *stream);
 
 /*
  * aamd_grouped_gemm_fp8_nt for callers that cannot allocate device memory (code under HIP graph

@@ -20,10 +20,10 @@ extern "C" {
 const char *aamd_probes_last_error(void);
 
 /*
- * The grouped GEMMs of the product library (same kernels, same arguments as aamd_grouped_gemm_fp8_nt and
+ * The grouped GEMMs of the product library (same kernels, same arguments as aamd_grouped_gemm_fp8_nt, _nn and
  * aamd_grouped_gemm_fp8_wgrad) with the launch choices the library otherwise makes by itself pinned for
  * this one call: opts = {tile, group_r, gl, ls_batch}, each -1 for the library's own choice.
- *   tile: 0 = 128x128 tiles, 1 = the large configuration (wgrad: 256x128 tiles);
+ *   tile: 0 = 128x128 tiles, 1 = the large configuration (wgrad: 256x128 tiles), 2 / 3 = the kernel for few rows and its split form;
  *   group_r: the tile order groups R tiles (1) or L tiles (0); gl: tiles sharing a panel in the tile order;
  *   ls_batch: 0 = scales fetched one contraction block at a time (which the 128x128 tiles do: the large
  *   configuration of the block-scaled GEMM takes its scales in batches only and is then not chosen).
@@ -33,6 +33,10 @@ int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t *a, int64_t lda, const float *
                                     const float *b_s, int b_tile_scaled, const int64_t *group_offsets, int E,
                                     int32_t *tile_ws, int64_t M, int64_t N, int64_t K, void *c, int c_dtype,
                                     int64_t ldc, const void *bias, int bias_dtype, const int *opts, void *stream);
+int aamd_tuning_grouped_gemm_fp8_nn(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b, const float *b_s,
+                                    const int64_t *group_offsets, int E, int64_t M, int64_t N, int64_t K, void *c,
+                                    int c_dtype, int64_t ldc, const void *bias, int bias_dtype, const int *opts,
+                                    void *stream);
 int aamd_tuning_grouped_gemm_fp8_wgrad(const uint8_t *dyt, const float *sdyt, const uint8_t *xt, const float *sxt,
                                        int64_t ld_t, int q_t_layout, const int64_t *group_offsets, int E,
                                        int32_t *tile_ws, int64_t N, int64_t K, void *dw, int dw_dtype,
