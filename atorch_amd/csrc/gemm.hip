@@ -21,8 +21,8 @@
 // matrix pipe busy.
 //
 // Data path: global -> LDS directly (global_load_lds, 16 bytes per lane, no register stop),
-// two stages, one workgroup barrier per step (two in the 256x256 configuration, whose L tile is
-// requested two steps ahead).  Rows are 128 bytes; the 16-byte chunks of a row
+// two stages, one workgroup barrier per step.  (Row-ragged launches on 256 x 256 tiles have a kernel of
+// their own, gemm_rows.hip.)  Rows are 128 bytes; the 16-byte chunks of a row
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
 #include <algorithm>
@@ -61,9 +61,8 @@ __device__ __forceinline__ void store4(OUT* dst, v4f o, bool accumulate) {
 }
 
 // Tile configuration: WR x WL waves, each computing (WTR*32) R rows x (WTL*32) L rows.
-template <int WR_, int WL_, int WTR_, int WTL_, int PRB_ = 2, bool LAHEAD_ = false>
+template <int WR_, int WL_, int WTR_, int WTL_, int PRB_ = 2>
 struct Cfg {
-  static constexpr bool LAHEAD = LAHEAD_;  // load the L tile two steps ahead (extra barrier per step)
   static constexpr int WR = WR_, WL = WL_, WTR = WTR_, WTL = WTL_;
   static constexpr int PRB = PRB_;  // raw-product buffers: 2 folds a sub-tile under the next one's MFMAs
   static constexpr int NT = 64 * WR * WL;   // threads
@@ -78,7 +77,6 @@ struct Cfg {
   static_assert((NT / 8) % 16 == 0, "the swizzle of a slab depends on the wave only");
 };
 typedef Cfg<2, 2, 2, 2, 3> CfgSmall;  // 256 threads, 128 (L) x 128 (R), two workgroups per CU
-typedef Cfg<2, 4, 4, 2, 1, true> CfgLarge;  // 512 threads, 256 (L) x 256 (R); one product buffer: 256 registers per lane
 typedef Cfg<2, 4, 2, 2> CfgWgrad;  // 512 threads, 256 (L) x 128 (R): room for the per-row R scales
 
 // ---- weight gradient of short groups -----------------------------------------------------------
@@ -602,8 +600,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   // are fetched every eighth step, 16 bytes per thread, into [row][8] floats.  The last batch is
   // shifted back so that it ends at the last block.
   const bool batch = MODE == kRaggedRows && p.ls_batch != 0;  // uniform; implies nkb >= 8
-  // this wave loads a scale every step (never in the configuration that takes all its scales in batches)
-  const bool step_scale = !C::LAHEAD && !(batch && l_side);
+  const bool step_scale = !(batch && l_side);  // this wave loads a scale every step
   const int brow = (tid >> 1) < lvalid ? (tid >> 1) : lvalid - 1;
   const uint32_t boff = ((uint32_t)brow * (uint32_t)p.ls_row_stride + (uint32_t)(tid & 1) * 4u) * 4u;
   auto batch_start = [&](int b) { return 8 * b + 8 <= nkb ? 8 * b : nkb - 8; };
@@ -641,10 +638,8 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
                  : "memory");
   };
   auto dmaR_scales = [&](int kb, float* Sd) {
-    if constexpr (!C::LAHEAD) {
-      if (!l_side) dma_scale(kb, Sd);
-      if (batch && (kb & 7) == 0) dma_scale_batch(kb >> 3);  // lands a step before its first use
-    }
+    if (!l_side) dma_scale(kb, Sd);
+    if (batch && (kb & 7) == 0) dma_scale_batch(kb >> 3);  // lands a step before its first use
   };
   auto dmaL_one = [&](int n, int kb, uint8_t* Ld, float* Sd) {
     dmaL_tile(n, kb, Ld);
@@ -755,7 +750,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   // the workgroup barrier.  Branch free: waves outside a partial R tile compute on clamped
   // rows and skip only the final store.
   constexpr int NTILES = C::WTR * C::WTL;
-  auto compute = [&](int kb, int stage, const float* Sct, auto&& after_l_reads, auto&& per_tile) {
+  auto compute = [&](int kb, int stage, const float* Sct) {
     __builtin_amdgcn_sched_barrier(0);
     // L scale of tile row r: Lsc[r * lsc_stride]
     const int bsel = kb >> 3;
@@ -835,10 +830,6 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
       // the next R row overwrites the fragment and scale slot of row i - 1, whose last fold is done
       if (j == 0 && i + 1 < C::WTR) load_r(i + 1);
       __builtin_amdgcn_sched_barrier(0);
-      // every L fragment has been an MFMA operand by now, so it has left the LDS: the hook (a
-      // barrier and the next L loads) costs no extra wait here
-      per_tile(T);
-      if (t == C::WTL - 1) after_l_reads();
     });
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -854,230 +845,28 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  auto nothing = [] {};
-  auto no_feed = [](auto) {};
   // Two workgroups per CU: the loads of a step go out in one burst after the barrier (issued a few
   // at a time behind the sub-tiles they measured 6 % slower here: they have less time to arrive,
   // and the other workgroup already fills the issue gap).
-  if constexpr (!C::LAHEAD) {
-    if (nkb > 0) dma(0, Lbuf0, Rbuf0, Sc0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    // a wave without valid rows runs its own copy of the loop, loads and barriers only
-    auto loop = [&](auto W) {
-      constexpr bool kWork = decltype(W)::value;
-      int kb = 0;
-      for (; kb + 1 < nkb; kb += 2) {  // two steps per trip: the stage addresses are compile-time constants
-        dma(kb + 1, Lbuf1, Rbuf1, Sc1);
-        if constexpr (kWork) compute(kb, 0, Sc0, nothing, no_feed);
-        dma_wait_and_sync();
-        dma(kb + 2 < nkb ? kb + 2 : kb + 1, Lbuf0, Rbuf0, Sc0);  // the last prefetch re-reads a valid block
-        if constexpr (kWork) compute(kb + 1, 1, Sc1, nothing, no_feed);
-        dma_wait_and_sync();
-      }
-      if constexpr (kWork)
-        if (kb < nkb) compute(kb, 0, Sc0, nothing, no_feed);  // odd number of steps
-    };
-    if (has_work) loop(std::true_type{});
-    else loop(std::false_type{});
-  } else {
-    // One workgroup per CU, eight waves, two per SIMD.  The matrix pipe of a SIMD idles whenever both
-    // of its waves are away from their MFMAs at the same time, which is what a workgroup barrier
-    // followed by LDS reads produces.  So the two barriers of a step stand where register-resident
-    // MFMA work follows them:
-    //   Q (start of step k): every wave holds the L fragments of step k, so the L half of stage k is
-    //     free and the L tile of step k+2 is requested behind the first sub-tiles;
-    //   P (before the last R row of sub-tiles): every wave has read the last fragments of stage k
-    //     and the tiles of step k+1 have landed; behind it the R tile of step k+2 is requested and
-    //     the first fragments of step k+1 are read from the LDS while the last R row, whose operands
-    //     are already in registers, runs on the matrix pipe.  The fragment registers of step k are
-    //     reused as they die, so the prefetch costs no registers.
-    // The fold of the sub-tile in front of a barrier is issued behind it: the wave that arrives last
-    // has just issued its MFMAs, and the one that waited folds while those still run.
-    // Loads complete in issue order, so "all but the newest L group" is one wait count.  Past the
-    // end the loads re-read the last block to keep the counts uniform.
-    static_assert(!R_PER_ROW && MODE == kRaggedRows, "the two-barrier pipeline is written for block-scaled R operands");
-    static_assert(C::PRB == 1 && C::WTR % 2 == 0 && C::RCH % C::WTL == 0 && C::LCH <= NTILES, "pipeline shape");
-    constexpr int PT = (C::WTR - 1) * C::WTL - 1;  // the sub-tile in front of barrier P
-    constexpr int RPER = C::RCH / C::WTL;
-    auto kclamp = [&](int k) { return k < nkb ? k : nkb - 1; };
-    // Scales of this pipeline come in batches of eight contraction blocks only (the launcher takes the other
-    // configuration when K has fewer than eight blocks), so a
-    // step issues no scale load and takes no branch: batch b (blocks 8 b .. 8 b + 7, the last one shifted
-    // back to end at the last block) is requested behind barrier P of step 8 (b - 1), eight steps before
-    // its first use.  L scales: every wave fetches 32 rows x 32 bytes into LsB[b & 1][row][8]; R block
-    // scales: wave 0 fetches the tile's two 128-row blocks x 32 bytes into RsB[b & 1][block][8] (lanes past
-    // the fourth repeat those addresses: the direct-to-LDS load always writes 1 KB).
-    // Scale rows that are not 16-byte aligned (a number of contraction blocks that is not a multiple of four, an
-    // unaligned base) take 4-byte loads instead: four per wave and batch for the L scales (lane l of load q fetches
-    // float 64 q + l of the wave's 32 rows x 8 floats), one for the R scales.
-    float* const RsB0 = Sc0;  // [2][NT] floats, the first 16 of each in use
-    const bool x4 = p.ls_batch == 1;
-    const int rblocks = rvalid / kTile;
-    const int rlane_blk = ((lane >> 1) & 1) < rblocks ? (lane >> 1) & 1 : rblocks - 1;
-    const uint32_t roff = ((uint32_t)rlane_blk * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 1) * 4u) * 4u;
-    const int rlane_blk1 = ((lane >> 3) & 1) < rblocks ? (lane >> 3) & 1 : rblocks - 1;
-    const uint32_t roff1 = ((uint32_t)rlane_blk1 * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 7) * (uint32_t)p.rs_blk_stride) * 4u;
-    uint32_t boff1[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int row = wave * 32 + q * 8 + (lane >> 3);
-      boff1[q] = ((uint32_t)(row < lvalid ? row : lvalid - 1) * (uint32_t)p.ls_row_stride + (uint32_t)(lane & 7)) * 4u;
+  if (nkb > 0) dma(0, Lbuf0, Rbuf0, Sc0);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // a wave without valid rows runs its own copy of the loop, loads and barriers only
+  auto loop = [&](auto W) {
+    constexpr bool kWork = decltype(W)::value;
+    int kb = 0;
+    for (; kb + 1 < nkb; kb += 2) {  // two steps per trip: the stage addresses are compile-time constants
+      dma(kb + 1, Lbuf1, Rbuf1, Sc1);
+      if constexpr (kWork) compute(kb, 0, Sc0);
+      dma_wait_and_sync();
+      dma(kb + 2 < nkb ? kb + 2 : kb + 1, Lbuf0, Rbuf0, Sc0);  // the last prefetch re-reads a valid block
+      if constexpr (kWork) compute(kb + 1, 1, Sc1);
+      dma_wait_and_sync();
     }
-    auto dma_batches = [&](int b) {
-      const uint8_t* lsb = reinterpret_cast<const uint8_t*>(Lsg + uniform_i64(l0 * p.ls_row_stride + batch_start(b)));
-      const uint8_t* rsb = reinterpret_cast<const uint8_t*>(Rsg + uniform_i64((r0 / kTile) * p.rs_row_stride + batch_start(b) * p.rs_blk_stride));
-      const uint32_t ldst = lds_addr(LsB0 + (b & 1) * (BM * 8)) + (uint32_t)(wave * 1024);
-      const uint32_t rdst = lds_addr(RsB0 + (b & 1) * NT);
-      if (x4) {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(boff), "s"(lsb), "s"(ldst) : "memory");
-        if (!R_ROWS && wave == 0)
-          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(roff), "s"(rsb), "s"(rdst) : "memory");
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(boff1[q]), "s"(lsb), "s"(ldst + (uint32_t)(q * 256)) : "memory");
-        if (!R_ROWS && wave == 0)
-          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(roff1), "s"(rsb), "s"(rdst) : "memory");
-      }
-      if (R_ROWS && wave == 0)  // a row of scales per contraction block: never 16 bytes of one block
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(roff1), "s"(rsb), "s"(rdst) : "memory");
-    };
-    if (nkb > 0) {
-      dmaL(0, Lbuf0, Sc0);  // (the per-step scale hooks of these helpers are off: see step_scale)
-      dmaR(0, Rbuf0, Sc0);
-      dma_batches(0);
-      dmaL(kclamp(1), Lbuf1, Sc1);
-      dmaR(kclamp(1), Rbuf1, Sc1);
-      // the tiles of step 0 and the first scale batch have landed; those of step 1 may still be on their way
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::LCH + C::RCH) : "memory");
-      auto barrier_q = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-      // all but this step's L tile loads have landed (loads complete in issue order)
-      auto barrier_p = [&]() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::LCH) : "memory"); };
-      if (has_work) {
-        v8i lf[C::WTL][2], rf[2][2];
-        float cs[C::WTL], csn[C::WTL], rblkn;
-        float cs_last = 0.f;  // scale of the sub-tile whose fold is still owed (the last one of the step before)
-        v16f pr, zero;
-#pragma unroll
-        for (int r = 0; r < 16; r++) zero[r] = pr[r] = 0.f;
-        // scales of step kb: the lane's L row scales and the R block scale of the wave; their product is
-        // formed where it is first needed, not where the reads are issued
-        auto read_scales = [&](int kb, float (&dst)[C::WTL], float& rblk) {
-          const int b = kb >> 3, in_batch = kb - batch_start(b);
-          const float* Lsc = LsB0 + (b & 1) * (BM * 8) + in_batch;
-          rblk = RsB0[(b & 1) * NT + (wrow0 / kTile) * 8 + in_batch];
-#pragma unroll
-          for (int j = 0; j < C::WTL; j++) dst[j] = Lsc[(wlrow0 + j * 32 + l32) * 8];
-        };
-        // (the empty volatile statements pin MFMAs and folds between the memory instructions around
-        // them: plain arithmetic is otherwise free to drift past inline assembly)
-        auto fold = [&](int i, int j, float sc) {
-#pragma unroll
-          for (int r = 0; r < 16; r++) acc[i][j][r] = __builtin_fmaf(pr[r], sc, acc[i][j][r]);
-          asm volatile("" : "+v"(acc[i][j]));
-        };
-        // fragments and scales of step 0
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          lf[0][h] = frag(la, 0, BM, 0, h);
-          rf[0][h] = fragR(0, 0, h);
-        }
-#pragma unroll
-        for (int j = 1; j < C::WTL; j++)
-#pragma unroll
-          for (int h = 0; h < 2; h++) lf[j][h] = frag(la, 0, BM, j, h);
-        read_scales(0, cs, rblkn);
-#pragma unroll
-        for (int j = 0; j < C::WTL; j++) cs[j] *= rblkn;
-        // FIRST: the first step of a run of eight, which requests the next scale batch behind barrier P
-        auto step = [&](int kb, auto S, auto FIRST) {
-          constexpr int s = decltype(S)::value;
-          constexpr bool kFirst = decltype(FIRST)::value;
-          uint8_t* const Lc = s ? Lbuf1 : Lbuf0;
-          uint8_t* const Rc = s ? Rbuf1 : Rbuf0;
-          const int k2 = kclamp(kb + 2);
-          __builtin_amdgcn_sched_barrier(0);
-          barrier_q();
-          __builtin_amdgcn_sched_barrier(0);
-          fold(C::WTR - 1, C::WTL - 1, cs_last);  // owed by the step before (adds zero in the first step)
-          static_for<NTILES>([&](auto T) {
-            constexpr int t = decltype(T)::value;
-            constexpr int i = t / C::WTL, j = t % C::WTL;
-            __builtin_amdgcn_sched_barrier(0);
-            pr = mfma_fp8_32x32x64(rf[i & 1][0], lf[j][0], zero);
-            pr = mfma_fp8_32x32x64(rf[i & 1][1], lf[j][1], pr);
-            asm volatile("" : "+v"(pr));
-            __builtin_amdgcn_sched_barrier(0);
-            // memory instructions go out while the MFMAs run, ahead of the fold that waits for them
-            if constexpr (t < C::LCH) dmaL_tile(t, k2, Lc);
-            if constexpr (j == 0 && i + 1 < C::WTR) {
-#pragma unroll
-              for (int h = 0; h < 2; h++) rf[(i + 1) & 1][h] = fragR(s, i + 1, h);
-            }
-            if constexpr (t == PT) {
-              __builtin_amdgcn_sched_barrier(0);
-              barrier_p();
-              __builtin_amdgcn_sched_barrier(0);
-              if constexpr (kFirst) {
-                if (kb + 8 < nkb) dma_batches((kb >> 3) + 1);
-              }
-              // row C::WTR - 2 has been consumed: its registers take the first R row of the next step
-#pragma unroll
-              for (int h = 0; h < 2; h++) rf[0][h] = fragR(s ^ 1, 0, h);
-              read_scales(kclamp(kb + 1), csn, rblkn);
-            }
-            if constexpr (t > PT) {
-              constexpr int jn = t - PT - 1;  // == j: this sub-tile was the last user of lf[j]
-              static_for<RPER>([&](auto N) { dmaR_tile(jn * RPER + decltype(N)::value, k2, Rc); });
-#pragma unroll
-              for (int h = 0; h < 2; h++) lf[jn][h] = frag(la, s ^ 1, BM, jn, h);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (t + 1 < NTILES) fold(i, j, cs[j]);
-          });
-          cs_last = cs[C::WTL - 1];
-#pragma unroll
-          for (int j = 0; j < C::WTL; j++) cs[j] = csn[j] * rblkn;
-        };
-        // runs of eight steps (the contraction has at least eight blocks; the last run may be shorter), two
-        // steps per trip so that the stage addresses are compile-time constants
-        constexpr std::integral_constant<int, 0> S0{};
-        constexpr std::integral_constant<int, 1> S1{};
-        for (int kb = 0; kb < nkb; kb += 8) {
-          const int n = nkb - kb < 8 ? nkb - kb : 8;
-          step(kb, S0, std::true_type{});
-          if (n > 1) step(kb + 1, S1, std::false_type{});
-          int kk = 2;
-          for (; kk + 1 < n; kk += 2) {
-            step(kb + kk, S0, std::false_type{});
-            step(kb + kk + 1, S1, std::false_type{});
-          }
-          if (kk < n) step(kb + kk, S0, std::false_type{});  // odd number of steps
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        fold(C::WTR - 1, C::WTL - 1, cs_last);
-      } else {
-        // a wave without valid rows: loads and barriers only, in the order of the working waves
-        auto step = [&](int kb, uint8_t* Lc, uint8_t* Rc, bool first) {
-          const int k2 = kclamp(kb + 2);
-          barrier_q();
-#pragma unroll
-          for (int n = 0; n < C::LCH; n++) dmaL_tile(n, k2, Lc);
-          barrier_p();
-          if (first && kb + 8 < nkb) dma_batches((kb >> 3) + 1);
-#pragma unroll
-          for (int n = 0; n < C::RCH; n++) dmaR_tile(n, k2, Rc);
-        };
-        int kb = 0;
-        for (; kb + 1 < nkb; kb += 2) {
-          step(kb, Lbuf0, Rbuf0, (kb & 7) == 0);
-          step(kb + 1, Lbuf1, Rbuf1, false);
-        }
-        if (kb < nkb) step(kb, Lbuf0, Rbuf0, (kb & 7) == 0);
-      }
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the trailing loads must not land in the epilogue's staging
-    }
-  }
+    if constexpr (kWork)
+      if (kb < nkb) compute(kb, 0, Sc0);  // odd number of steps
+  };
+  if (has_work) loop(std::true_type{});
+  else loop(std::false_type{});
 
   // ---- epilogue ------------------------------------------------------------------------------
   // A lane holds, for one output row, groups of four consecutive columns; stored directly that
@@ -1220,9 +1009,9 @@ struct GemmOptions {
   int ls_batch = -1;  // 0: L scales fetched one contraction block at a time
 };
 
-template <int MODE, bool R_PER_ROW, typename C, bool R_ROWS = false>
-static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st, const GemmOptions& g_opt) {
-  if (blocks <= 0) return AAMD_OK;
+// Tiles that share panels: the order of the tiles (rows: L rows of a tile).
+template <int MODE>
+static void tile_order(GemmParams& p, int rows, const GemmOptions& g_opt) {
   // L tiles per group of the tile order: 8 for the row-ragged launches; 4 for wgrad, whose operand
   // panels run over all tokens of an expert and are several times larger (measured: 5 % faster
   // at 4096 tokens per expert and 28672 x 4096 outputs, within 3 % either way elsewhere)
@@ -1230,12 +1019,17 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
   // group along the side with more tiles per expert (row-ragged launches: batches of 4 R tiles measured 1 % faster
   // than the L grouping with many small groups, the same with few large ones)
   if (MODE == kRaggedK) p.group_r = p.nRt > p.nLt;
-  else p.group_r = p.goff != nullptr && (int64_t)p.nRt * C::BM * p.E > p.Lrows;
+  else p.group_r = p.goff != nullptr && (int64_t)p.nRt * rows * p.E > p.Lrows;
   if (MODE == kRaggedRows && p.group_r) p.gl = 4;
   // per-call overrides (measurement build only)
   if (g_opt.group_r >= 0) p.group_r = g_opt.group_r != 0 && (MODE == kRaggedK || p.goff != nullptr);
   if (g_opt.gl > 0) p.gl = g_opt.gl;
+}
 
+template <int MODE, bool R_PER_ROW, typename C, bool R_ROWS = false>
+static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st, const GemmOptions& g_opt) {
+  if (blocks <= 0) return AAMD_OK;
+  tile_order<MODE>(p, C::BM, g_opt);
   AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
   dim3 grid((unsigned)blocks), block(C::NT);
   if (c_dtype == AAMD_BF16)
@@ -1352,13 +1146,15 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   const bool batches16 = batches && (K / kBK) % 4 == 0 && aligned16(a_s);
   const NtKernel kernel = b_tile_scaled ? (use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), g_opt) ? kLargeTiles : kSmallTiles)
                                         : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, g_opt);
-  const bool large = kernel == kLargeTiles;
-  const int BM = large ? CfgLarge::BM : CfgSmall::BM;
-  const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : CfgLarge::BN) : CfgSmall::BN;
+  // (output rows of 8 M elements are out of reach of the large tiles' 32-bit offsets)
+  const bool large = kernel == kLargeTiles && (b_tile_scaled || ldc < (1LL << 23));
+  const int BM = large ? kLargeTile : CfgSmall::BM;
+  const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : kLargeTile) : CfgSmall::BN;
+  static_assert(CfgWgrad::BM == kLargeTile, "L rows of a large tile");
   GemmParams p = {};
   p.L = a; p.ldl = lda; p.Ls = a_s; p.ls_row_stride = K / kBK; p.ls_blk_stride = 1;
   p.l_kb_stride = p.r_kb_stride = kBK;
-  // 1: batches by 16-byte loads; 2 (256x256 configuration only): by 4-byte loads
+  // 1: batches by 16-byte loads; 2 (256x256 tiles only): by 4-byte loads
   p.ls_batch = large && !b_tile_scaled ? (batches16 && aligned16(b_s) ? 1 : 2) : (batches16 ? 1 : 0);
   p.R = b; p.ldr = K; p.r_group_stride = N * K;
   p.Rs = b_s;
@@ -1376,12 +1172,12 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   if (kernel == kFewRows || kernel == kFewRowsSplit) return launch_few_rows(p, c_dtype, M, kernel == kFewRowsSplit, b_rows, st);
   const int64_t max_lt = group_offsets ? M / BM + E : (M + BM - 1) / BM;
   const int64_t blocks = max_lt * p.nRt;
-  if (b_rows)
-    return large ? launch_gemm<kRaggedRows, false, CfgLarge, true>(p, c_dtype, blocks, st, g_opt)
-                 : launch_gemm<kRaggedRows, false, CfgSmall, true>(p, c_dtype, blocks, st, g_opt);
-  if (large)
-    return b_tile_scaled ? launch_gemm<kRaggedRows, true, CfgWgrad>(p, c_dtype, blocks, st, g_opt)
-                         : launch_gemm<kRaggedRows, false, CfgLarge>(p, c_dtype, blocks, st, g_opt);
+  if (large && !b_tile_scaled) {
+    tile_order<kRaggedRows>(p, kLargeTile, g_opt);
+    return launch_row_tiles(p, c_dtype, blocks, b_rows, st);
+  }
+  if (b_rows) return launch_gemm<kRaggedRows, false, CfgSmall, true>(p, c_dtype, blocks, st, g_opt);
+  if (large) return launch_gemm<kRaggedRows, true, CfgWgrad>(p, c_dtype, blocks, st, g_opt);
   return b_tile_scaled ? launch_gemm<kRaggedRows, true, CfgSmall>(p, c_dtype, blocks, st, g_opt)
                        : launch_gemm<kRaggedRows, false, CfgSmall>(p, c_dtype, blocks, st, g_opt);
 }

@@ -5,6 +5,7 @@
 namespace aamd {
 
 constexpr int kBK = 128;  // contraction bytes per step == scale block
+constexpr int kLargeTile = 256;  // rows of an L and R tile of gemm_rows.hip
 
 enum GemmMode { kRaggedRows = 0, kRaggedK = 1 };
 
@@ -71,5 +72,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // Row-ragged GEMM with block-scaled R for groups of few rows (gemm_few.hip); reads L, R, their scales and strides, C,
 // bias, goff, E, Lrows, Rrows and nkb of the parameters.  r_rows: R is stored [contraction, Rrows] (R_ROWS of gemm.hip).
 int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st);
+
+// Row-ragged GEMM with block-scaled R on 256 x 256 tiles (gemm_rows.hip): at least eight contraction blocks, p.ls_batch 1 where
+// rows of scales are 16-byte aligned; `tiles`: no fewer than there are.
+int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st);
 
 }  // namespace aamd

@@ -1,0 +1,647 @@
+// Row-ragged block-scaled FP8 GEMM on 256 x 256 tiles, one persistent workgroup per CU (forward, dgrad, dense).
+//
+// What a step does and why is the same as in gemm.hip: 128-deep blocks, two chained v_mfma_f32_32x32x64_f8f6f4 per 32 x 32
+// sub-tile, the raw product folded into fp32 accumulators with the block's scales, operands moved global -> LDS without a
+// register stop, 16-byte chunks XOR-swizzled.  Eight waves of 128 (R) x 64 (L), two per SIMD.
+//
+// The matrix pipe of a SIMD idles whenever both of its waves are away from their MFMAs at the same time, which is what a
+// workgroup barrier followed by LDS reads produces.  So the two barriers of a step stand where register-resident MFMA work
+// follows them:
+//   Q (start of step k): every wave holds the L fragments of step k, so the L half of its stage is free and the L tile of
+//     step k + 2 is requested behind the first sub-tiles;
+//   P (before the last R row of sub-tiles): every wave has read the last fragments of the stage and the tiles of step k + 1
+//     have landed; behind it the R tile of step k + 2 is requested and the first fragments of step k + 1 are read while the
+//     last R row, whose operands are already in registers, runs on the matrix pipe.
+// The fold of the sub-tile in front of a barrier is issued behind it.
+//
+// One workgroup per tile costs 9 to 10 us beside the steps of 1.45 us (stamps taken inside the kernel, 32768 rows x 28672
+// outputs x 4096 in 8 groups): 2.0 from the end of one workgroup to the start of the next on a CU, 1.7 to find its group, 2.0
+// until its first operands are there, 4.1 to turn the tile round through the LDS and store it.  So a workgroup stays and takes
+// one tile after the other, and the steps of its tiles are one stream: the last two steps of a tile request the first two
+// blocks of the next one, its last step reads the next one's first fragments, and the finished tile goes from the registers
+// to memory (lanes swap halves, so that four of them hold 64 consecutive bytes of a row) while those loads are in flight, as
+// the stage buffers hold them.  What a tile needs besides are scalars: rows past its end and columns past the weights' end
+// are left to the range check of buffer instructions, which neither reads nor writes them.
+#include <algorithm>
+
+#include "gemm.hpp"
+
+namespace aamd {
+
+namespace rows {
+constexpr int BM = 256, BN = 256, NT = 512, WTR = 4, WTL = 2, NTILES = WTR * WTL;
+constexpr int kSide = 256 * kBK;        // bytes of an L (R) tile of a step
+constexpr int kScaleBatch = BM * 8 + 256;  // floats: the scales of eight contraction blocks, [L row][8] and [R block][8]
+constexpr int kLds = 4 * kSide + 2 * kScaleBatch * 4 + 64 * (int)sizeof(int64_t) * 3;
+constexpr int kWorkgroups = 256;        // one per CU
+}  // namespace rows
+
+// A raw buffer of `bytes` bytes at `base`: reads past it give 0, writes past it are dropped.
+__device__ __forceinline__ v4i buffer_at(const void* base, uint32_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};  // (addresses have 47 bits)
+}
+template <int OFFSET>
+__device__ __forceinline__ void load_lds_x4(uint32_t off, const v4i& buf, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buf), "s"(lds), "i"(OFFSET) : "memory", "scc");
+}
+__device__ __forceinline__ void advance_buffer(v4i& b, int64_t by) {
+  const uint64_t a = (((uint64_t)(uint32_t)b[1] << 32) | (uint32_t)b[0]) + (uint64_t)by;
+  b[0] = (int)(uint32_t)a;
+  b[1] = (int)(uint32_t)(a >> 32);
+}
+__device__ __forceinline__ void load_lds_x1(uint32_t off, const v4i& buf, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(buf), "s"(lds) : "memory");
+}
+
+// A uniform value the compiler knows nothing about: a branch on it inside the tile loop stays there (a loop per case would be a
+// copy of the whole kernel each).
+__device__ __forceinline__ int opaque(int v) {
+  v = __builtin_amdgcn_readfirstlane(v);
+  asm volatile("" : "+s"(v));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+// The lane, counted anew: what is computed from it lives where it is used, not in registers across the tile loop.
+__device__ __forceinline__ int lane_here() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+// (the compiler does not see what is inside: five wait states in front, for scalar registers that the vector unit has just
+// written, and two behind, before the data registers are written again)
+__device__ __forceinline__ uint64_t args_here() {
+  uint64_t a = (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return (uint64_t)uniform_i64((int64_t)a);
+}
+template <int OFFSET>
+__device__ __forceinline__ void store_x4(const v4i& v, uint32_t off, const v4i& buf) {
+  asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, 0 offen offset:%3\n\ts_nop 1" ::"v"(v), "v"(off), "s"(buf), "n"(OFFSET) : "memory");
+}
+
+// a.upper half of the lanes <-> b.lower half; odd rows of 16 lanes of a <-> even rows of b
+__device__ __forceinline__ void swap32(int& a, int& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = (int)r[0];
+  b = (int)r[1];
+}
+__device__ __forceinline__ void swap16(int& a, int& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = (int)r[0];
+  b = (int)r[1];
+}
+
+// R_ROWS: the R operand is stored [contraction, Rrows] and its fragments are read transposed, see grouped_gemm_kernel.
+// PAIRS: an even number of steps per tile, so that a step's number says which stage it works on and the stage goes into the
+// immediate offset of its LDS reads; else the addresses change with every step (eight instructions more, 2 % of it).
+template <typename OUT, bool R_ROWS, bool PAIRS>
+__global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams p) {
+  // (the arguments of what is done once per tile are fetched there: scalar registers are short in the loop; in front of it
+  // they come all at once)
+  auto args = [&]() __attribute__((always_inline)) { return (const __attribute__((address_space(4))) GemmParams*)(uintptr_t)args_here(); };
+  using namespace rows;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
+  // [L stage 0 | L stage 1 | R stage 0 | R stage 1 | two batches of scales | rows and tiles of the groups]
+  float* const scales = reinterpret_cast<float*>(lds + 4 * kSide);
+  int64_t* const table = reinterpret_cast<int64_t*>(scales + 2 * kScaleBatch);
+  auto lds_addr = [](const void* q) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)q; };
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hg = lane >> 5;
+  const int nkb = p.nkb;
+
+  // ---- the tiles of this workgroup ------------------------------------------------------------
+  // Workgroup ids go round-robin over the 8 XCDs; every XCD gets one contiguous range of tile ids, in which tiles that share
+  // operand panels are neighbours, and its workgroups take them side by side.  (Which one of them takes which tile of a round
+  // rotates, so that no workgroup gets the short last tile of every group.)
+  GroupRanges gr = {};
+  int total_lt = (int)((p.Lrows + BM - 1) / BM);
+  if (p.goff != nullptr) {
+    gr = group_ranges<BM>(p.goff, p.E, 0, 0);
+    total_lt = gr.total;
+    for (int base = 64; base < p.E; base += 64) total_lt = group_ranges<BM>(p.goff, p.E, base, total_lt).total;
+    if (p.E <= 64) {  // the group of every later tile is found from here
+      table[lane * 3] = gr.r_lo;
+      table[lane * 3 + 1] = gr.r_hi;
+      table[lane * 3 + 2] = (int64_t)(((uint64_t)(uint32_t)gr.t_hi << 32) | (uint32_t)gr.t_lo);
+    }  // (every wave writes the same values, and reads what it wrote)
+  }
+  const uint32_t nRt = (uint32_t)p.nRt, ntot = (uint32_t)total_lt * nRt;
+  const uint32_t xcd = blockIdx.x & 7u, nwg = gridDim.x >> 3;
+  const uint32_t per = ntot >> 3, rem = ntot & 7u;
+  const uint32_t first_tile = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
+  const uint32_t end_tile = first_tile + per + (xcd < rem ? 1u : 0u);
+
+  struct Tile {
+    int64_t l0;               // first L row
+    int g, lvalid, r0, rvalid;  // group, valid L rows, first R row and valid R rows (a multiple of 128)
+  };
+  auto tile_of = [&](uint32_t pid, auto a) __attribute__((always_inline)) {
+    const uint32_t GL = (uint32_t)a->gl;
+    Tile t;
+    uint32_t lt, rt;
+    // groups of GL L tiles, R tile index outer, L tile inner
+    {
+      const uint32_t width = GL * nRt, grp = pid / width, in = pid - grp * width, first = grp * GL;
+      const uint32_t gsz = (uint32_t)total_lt - first < GL ? (uint32_t)total_lt - first : GL;
+      rt = in / gsz;
+      lt = first + (in - rt * gsz);
+    }
+    t.g = 0;
+    int64_t r_lo = 0, r_hi = a->Lrows;
+    uint32_t t_lo = 0;
+    if (opaque(a->goff != nullptr)) {
+      // exactly one group holds the tile; with group_r the tile ids of a group are contiguous, in batches of GL R tiles, all L
+      // tiles of the group inside a batch, R index fastest: the weights, the large operand, are then fetched once
+      const int by_group = opaque(a->group_r), in_table = opaque(a->E <= 64);
+      GroupRanges r;
+      if (in_table) {
+        const int64_t* const e = table + lane_here() * 3;
+        r.r_lo = e[0];
+        r.r_hi = e[1];
+        const int64_t tt = e[2];
+        r.t_lo = (int)(uint32_t)(uint64_t)tt;
+        r.t_hi = (int)(uint32_t)((uint64_t)tt >> 32);
+      }
+      for (int base = 0, carry = 0; base < a->E; base += 64) {
+        if (!in_table) {
+          r = group_ranges<BM>(a->goff, a->E, base, carry);
+          carry = r.total;
+        }
+        const bool mine = by_group ? pid >= (uint32_t)r.t_lo * nRt && pid < (uint32_t)r.t_hi * nRt
+                                    : lt >= (uint32_t)r.t_lo && lt < (uint32_t)r.t_hi;  // (empty groups hold no tile)
+        const unsigned long long hit = __ballot(mine);
+        if (hit != 0) {
+          const int src = __builtin_ctzll(hit);
+          t.g = base + src;
+          t_lo = (uint32_t)__builtin_amdgcn_readlane(r.t_lo, src);
+          r_lo = readlane_i64(r.r_lo, src);
+          r_hi = readlane_i64(r.r_hi, src);
+          if (by_group) {
+            const uint32_t nl = (uint32_t)__builtin_amdgcn_readlane(r.t_hi, src) - t_lo;
+            const uint32_t pe = pid - t_lo * nRt, width = GL * nl, batch = pe / width, in = pe - batch * width, first = batch * GL;
+            const uint32_t gsz = nRt - first < GL ? nRt - first : GL;
+            const uint32_t l = in / gsz;
+            rt = first + (in - l * gsz);
+            lt = t_lo + l;
+          }
+          break;
+        }
+      }
+    }
+    t.l0 = uniform_i64(r_lo + (int64_t)(lt - t_lo) * BM);
+    const int64_t left = (r_hi < a->Lrows ? r_hi : a->Lrows) - t.l0;
+    t.lvalid = __builtin_amdgcn_readfirstlane(left < BM ? (int)left : BM);
+    t.g = __builtin_amdgcn_readfirstlane(t.g);
+    t.r0 = __builtin_amdgcn_readfirstlane((int)(rt * BN));
+    t.rvalid = (int)(a->Rrows - t.r0 < BN ? a->Rrows - t.r0 : BN);
+    return t;
+  };
+  uint32_t round_first = first_tile, turn = blockIdx.x >> 3;
+  auto take = [&](uint32_t& pid) __attribute__((always_inline)) {  // the next tile of this workgroup, false if there is none
+    pid = round_first + turn;
+    round_first += nwg;
+    turn += nwg > 5u ? 5u : 1u;
+    turn = turn >= nwg ? turn - nwg : turn;
+    return pid < end_tile;
+  };
+  uint32_t pid;
+  if (!take(pid)) return;  // (rounds before the last are whole, so a workgroup that has no tile in one has none later)
+  // (plain variables: as structures the two would live in memory)
+  int64_t c_l0, n_l0;
+  int c_g, c_lvalid, c_r0, c_rvalid, n_g, n_lvalid, n_r0, n_rvalid;
+  auto take_tile = [&](uint32_t id, auto a) __attribute__((always_inline)) {
+    const Tile t = tile_of(id, a);
+    n_l0 = t.l0, n_g = t.g, n_lvalid = t.lvalid, n_r0 = t.r0, n_rvalid = t.rvalid;
+  };
+  auto next_is_current = [&]() __attribute__((always_inline)) { c_l0 = n_l0, c_g = n_g, c_lvalid = n_lvalid, c_r0 = n_r0, c_rvalid = n_rvalid; };
+  auto current = [&]() __attribute__((always_inline)) { return Tile{c_l0, c_g, c_lvalid, c_r0, c_rvalid}; };
+  auto next = [&]() __attribute__((always_inline)) { return Tile{n_l0, n_g, n_lvalid, n_r0, n_rvalid}; };
+  take_tile(pid, &p);
+  next_is_current();
+
+  // ---- loads -------------------------------------------------------------------------------------
+  // A wave instruction of a tile load fills 1 KB of the LDS, lane l at base + 16 l; lane l fetches the chunk the swizzle puts
+  // there.  n-th instruction of wave w: rows 8 w + 64 n .. + 7 of the tile (R_ROWS: contraction rows 4 w + 32 n .. + 3).
+  const int r8 = lane >> 3;
+  const uint32_t chunk = (uint32_t)(((lane & 7) ^ r8 ^ (wave & 1)) << 4);
+  uint32_t voffL[4], voffR[4];
+  const int rrow = R_ROWS ? wave * 4 + (lane >> 4) : wave * 8 + r8;
+#pragma unroll
+  for (int n = 0; n < 4; n++) {
+    voffL[n] = (uint32_t)(wave * 8 + 64 * n + r8) * (uint32_t)p.ldl + chunk;
+    voffR[n] = (uint32_t)(rrow + (R_ROWS ? 32 : 64) * n) * (uint32_t)p.ldr + (R_ROWS ? (uint32_t)(((lane & 15) ^ (2 * (rrow & 7))) << 4) : chunk);
+  }
+  // Where the next block to be requested lies: it runs through the blocks of a tile and on into the next tile; behind the
+  // last one it stays on the last block, to keep the wait counts uniform.
+  v4i lbuf, rbuf;
+  int to_load = nkb;   // blocks left in the tile
+  int next_block = 0;  // of the tile next(): 0, or the last one where that is still the tile under way
+  auto enter_next = [&](auto a) __attribute__((always_inline)) {
+    const int64_t l_at = n_l0 * a->ldl + next_block * kBK;
+    const int64_t r_at = (int64_t)n_g * a->r_group_stride + (R_ROWS ? (int64_t)n_r0 : n_r0 * a->ldr) + next_block * a->r_kb_stride;
+    lbuf = buffer_at(a->L + uniform_i64(l_at), (uint32_t)__builtin_amdgcn_readfirstlane((n_lvalid - 1) * (int)a->ldl + kBK));
+    rbuf = buffer_at(a->R + uniform_i64(r_at), (uint32_t)__builtin_amdgcn_readfirstlane(
+                                                   R_ROWS ? 127 * (int)a->ldr + n_rvalid : (n_rvalid - 1) * (int)a->ldr + kBK));
+    to_load = nkb - next_block;
+  };
+  enter_next(&p);
+  auto advance = [&]() __attribute__((always_inline)) {
+    advance_buffer(lbuf, kBK);
+    advance_buffer(rbuf, p.r_kb_stride);
+    if (--to_load == 0) enter_next(args());
+  };
+  // where this wave's loads go, in the stage of the step under way (PAIRS: in stage 0)
+  uint32_t to_lds = lds_addr(lds) + (uint32_t)(wave * 1024);
+  auto load_l = [&](auto S, auto N) __attribute__((always_inline)) {
+    load_lds_x4<(PAIRS ? decltype(S)::value * kSide : 0) + decltype(N)::value * 8192>(voffL[decltype(N)::value], lbuf, to_lds);
+  };
+  auto load_r = [&](auto S, auto N) __attribute__((always_inline)) {
+    load_lds_x4<2 * kSide + (PAIRS ? decltype(S)::value * kSide : 0) + decltype(N)::value * 8192>(voffR[decltype(N)::value], rbuf, to_lds);
+  };
+  auto load_tile = [&](auto S) __attribute__((always_inline)) {
+    static_for<4>([&](auto N) __attribute__((always_inline)) { load_l(S, N); });
+    static_for<4>([&](auto N) __attribute__((always_inline)) { load_r(S, N); });
+  };
+  auto other_stage = [&]() __attribute__((always_inline)) {
+    if constexpr (!PAIRS) to_lds ^= kSide;
+  };
+
+  // Scales come in batches of eight contraction blocks (the last batch of a tile is shifted back to end at its last block): a
+  // row of 32 bytes per L row and per 128 R rows.  Batch b of a tile is
+  // requested in step 8 b - 3, batch 0 of the next tile in one of the last three steps (see `ask_next`), when the batch before
+  // the one in use has been read for the last time.  Rows of scales that are not 16-byte aligned take 4-byte loads.
+  const int x4 = p.ls_batch == 1;
+  const uint32_t lsr = (uint32_t)p.ls_row_stride, rsr = (uint32_t)p.rs_row_stride, rsb = (uint32_t)p.rs_blk_stride;
+  auto batch_start = [&](int b) __attribute__((always_inline)) { return 8 * b + 8 <= nkb ? 8 * b : nkb - 8; };
+  auto ask_scales = [&](const Tile t, int b, int parity, auto a) __attribute__((always_inline)) {
+    const int at = batch_start(b), ln = lane_here();
+    const v4i lb = buffer_at(a->Ls + uniform_i64(t.l0 * lsr + at), (uint32_t)__builtin_amdgcn_readfirstlane(((t.lvalid - 1) * (int)lsr + 8) * 4));
+    const uint32_t ld = lds_addr(scales + parity * kScaleBatch) + (uint32_t)(wave * 1024);
+    const int wide = opaque(x4);
+    if (wide) {
+      load_lds_x4<0>(((uint32_t)(wave * 32 + (ln >> 1)) * lsr + (uint32_t)(ln & 1) * 4u) * 4u, lb, ld);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        load_lds_x1(((uint32_t)(wave * 32 + q * 8 + (ln >> 3)) * lsr + (uint32_t)(ln & 7)) * 4u, lb, ld + (uint32_t)(q * 256));
+    }
+    if (wave == 0) {
+      const int blocks = t.rvalid / kTile;
+      const v4i rb = buffer_at(a->Rs + uniform_i64((int64_t)t.g * a->rs_group_stride + (int64_t)(t.r0 / kTile) * rsr + (int64_t)at * rsb),
+                               (uint32_t)__builtin_amdgcn_readfirstlane((R_ROWS ? 7 * (int)rsb + blocks : (blocks - 1) * (int)rsr + 8) * 4));
+      const uint32_t rd = lds_addr(scales + parity * kScaleBatch + BM * 8);
+      if (wide && !R_ROWS) load_lds_x4<0>(((uint32_t)((ln >> 1) & 1) * rsr + (uint32_t)(ln & 1) * 4u) * 4u, rb, rd);
+      else load_lds_x1(((uint32_t)((ln >> 3) & 1) * rsr + (uint32_t)(ln & 7) * rsb) * 4u, rb, rd);
+    }
+  };
+
+  // ---- matrix tiling: as in grouped_gemm_kernel.  The two waves of a SIMD (w and w + 4) share their R half and take L row
+  // blocks half a tile apart, so that a tile whose valid rows end in its first half keeps a working wave on every SIMD.
+  const int wr = wave & 1, wl = ((wave & 3) >> 1) + 2 * (wave >> 2);
+  const int wrow0 = wr * WTR * 32, wlrow0 = wl * WTL * 32;
+  const int sw = (l32 & 7) ^ ((l32 >> 3) & 1);
+  uint32_t la[2][2], ra[2][2];  // LDS addresses of this lane's chunks, stage 0
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const uint32_t chk = (uint32_t)(((4 * h + 2 * hg + c) ^ sw) << 4);
+      la[h][c] = lds_addr(lds) + (uint32_t)((wlrow0 + l32) * kBK) + chk;
+      if constexpr (R_ROWS) {
+        const int tr = (lane & 15) >> 1;
+        const int ch = (wrow0 / 16 + 2 * (2 * h + c) + ((lane >> 4) & 1)) ^ (2 * tr);
+        ra[h][c] = lds_addr(lds) + 2 * kSide + (uint32_t)((32 * hg + tr) * BN + ch * 16 + (lane & 1) * 8);
+      } else {
+        ra[h][c] = lds_addr(lds) + 2 * kSide + (uint32_t)((wrow0 + l32) * kBK) + chk;
+      }
+    }
+  // (without PAIRS: during a step `la` names the stage of the next one, and `ra` too from the middle of the step on)
+  auto other_l = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) la[h][c] ^= kSide;
+  };
+  auto other_r = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) ra[h][c] ^= kSide;
+  };
+  typedef const __attribute__((address_space(3))) v4i* lds_v4i_t;
+  auto frag = [&](const uint32_t (&base)[2][2], int s, int sub, int h) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)((PAIRS ? s * kSide : 0) + sub * 32 * kBK);
+    const v4i lo = *(lds_v4i_t)(uintptr_t)(base[h][0] + at);
+    const v4i hi = *(lds_v4i_t)(uintptr_t)(base[h][1] + at);
+    return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+  auto fragR = [&](int s, int sub, int h) __attribute__((always_inline)) {
+    if constexpr (R_ROWS) {
+      v8i f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const v2i o = lds_read_transposed(ra[sub / 2][sub % 2] + (uint32_t)((PAIRS ? s * kSide : 0) + (64 * h + 8 * j) * BN));
+        f[2 * j] = o[0];
+        f[2 * j + 1] = o[1];
+      }
+      return f;
+    } else {
+      return frag(ra, s, sub, h);
+    }
+  };
+  auto barrier_q = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+  v16f acc[WTR][WTL], pr;
+  v8i lf[WTL][2], rf[2][2];
+  float cs[WTL], csn[WTL], rblkn, cs_last = 0.f;
+
+  // Scales of a block: the lane's L row scales and the wave's R block scale; sc_at: where the next block's are, sc_left: blocks
+  // from there to the end of the batch, sc_more: batches of the tile behind it.
+  const int last_batch = (nkb - 1) >> 3, in_last = nkb - 8 * last_batch;
+  int sc_parity = 0;  // of the tile's batch 0
+  uint32_t sc_at = 0;
+  int sc_left = 0, sc_more = 0;
+  const uint32_t sc_l = lds_addr(scales) + (uint32_t)((wlrow0 + l32) * 32), sc_r = lds_addr(scales) + (uint32_t)(BM * 32 + (wrow0 / kTile) * 32);
+  auto read_scales = [&]() __attribute__((always_inline)) {
+    typedef const __attribute__((address_space(3))) float* lds_float_t;
+    const lds_float_t l = (lds_float_t)(uintptr_t)(sc_l + sc_at);
+    rblkn = *(lds_float_t)(uintptr_t)(sc_r + sc_at);
+#pragma unroll
+    for (int j = 0; j < WTL; j++) csn[j] = l[j * 32 * 8];
+    sc_at += 4;
+    if (--sc_left == 0) {
+      // (the first word of the other batch; past the tile's last block nobody uses what is read)
+      sc_at = sc_at > kScaleBatch * 4u ? 0u : kScaleBatch * 4u;
+      sc_left = 8;
+      if (--sc_more == 0) {  // the last batch ends at the last block
+        sc_left = in_last;
+        sc_at += (uint32_t)(8 - in_last) * 4u;
+      }
+    }
+  };
+  auto first_scales = [&]() __attribute__((always_inline)) {
+    sc_at = (uint32_t)(sc_parity * kScaleBatch * 4);
+    sc_left = 8;
+    sc_more = last_batch;
+    read_scales();
+  };
+  // The step that requests batch 0 of the next tile: from step 8 last_batch - 1 on the batch in front of the last is free, and
+  // the last step comes too late for what the next tile begins with.
+  const int ask_next = nkb - 4 > 8 * last_batch - 1 ? nkb - 4 : 8 * last_batch - 1;
+  int ask_at = 0, ask_batch = 0;
+  auto first_ask = [&]() __attribute__((always_inline)) {
+    ask_batch = 1;
+    ask_at = last_batch > 0 ? 5 : ask_next;
+  };
+
+  // (the empty volatile statements pin MFMAs and folds between the memory instructions around them)
+  auto fold = [&](int i, int j, float sc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[i][j][r] = __builtin_fmaf(pr[r], sc, acc[i][j][r]);
+    asm volatile("" : "+v"(acc[i][j]));
+  };
+  auto first_fragments = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      rf[0][h] = fragR(0, 0, h);
+#pragma unroll
+      for (int j = 0; j < WTL; j++) lf[j][h] = frag(la, 0, j, h);
+    }
+  };
+
+  auto ask_in_step = [&](int kb) __attribute__((always_inline)) {
+    if (kb != ask_at) return;
+    const bool of_next = ask_batch > last_batch;
+    ask_scales(Tile{of_next ? +n_l0 : +c_l0, of_next ? +n_g : +c_g, of_next ? +n_lvalid : +c_lvalid, of_next ? +n_r0 : +c_r0,
+                    of_next ? +n_rvalid : +c_rvalid}, of_next ? 0 : ask_batch, (sc_parity + ask_batch) & 1, args());
+    ask_batch++;
+    ask_at = ask_batch <= last_batch ? kb + 8 : ask_batch == last_batch + 1 ? ask_next : -1;
+  };
+
+  constexpr int PT = (WTR - 1) * WTL - 1;  // the sub-tile in front of barrier P
+  constexpr int kStores = NTILES * (sizeof(OUT) == 4 ? 4 : 2);  // of a wave and tile
+  bool stored = false;
+  // S: the stage (0 without PAIRS)
+  auto step = [&](int kb, auto S) __attribute__((always_inline)) {
+    constexpr int s = decltype(S)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_q();
+    __builtin_amdgcn_sched_barrier(0);
+    fold(WTR - 1, WTL - 1, cs_last);  // owed by the step before (adds zero in the first one)
+    if (!PAIRS) other_l();
+    static_for<NTILES>([&](auto T) __attribute__((always_inline)) {
+      constexpr int t = decltype(T)::value;
+      constexpr int i = t / WTL, j = t % WTL;
+      __builtin_amdgcn_sched_barrier(0);
+      pr = mfma_fp8_32x32x64(rf[i & 1][0], lf[j][0], v16f{});
+      pr = mfma_fp8_32x32x64(rf[i & 1][1], lf[j][1], pr);
+      asm volatile("" : "+v"(pr));
+      __builtin_amdgcn_sched_barrier(0);
+      // memory instructions go out while the MFMAs run, ahead of the fold that waits for them
+      if constexpr (t < 4) load_l(S, T);
+      if constexpr (j == 0 && i + 1 < WTR) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) rf[(i + 1) & 1][h] = fragR(s, i + 1, h);
+      }
+      if constexpr (t == PT) {
+        __builtin_amdgcn_sched_barrier(0);
+        // all but this step's L tile loads have landed (loads and stores are counted in issue order; the stores of the tile
+        // before were issued behind the loads this step waits for)
+        if (kb == 0 && stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + kStores) : "memory");
+        else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        ask_in_step(kb);
+        if (!PAIRS) other_r();
+        // row WTR - 2 has been consumed: its registers take the first R row of the next step
+#pragma unroll
+        for (int h = 0; h < 2; h++) rf[0][h] = fragR(s ^ 1, 0, h);
+        read_scales();
+      }
+      if constexpr (t > PT) {
+        constexpr int jn = t - PT - 1;  // == j: this sub-tile was the last user of lf[j]
+        load_r(S, std::integral_constant<int, 2 * jn>{});
+        load_r(S, std::integral_constant<int, 2 * jn + 1>{});
+#pragma unroll
+        for (int h = 0; h < 2; h++) lf[jn][h] = frag(la, s ^ 1, jn, h);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (t + 1 < NTILES) fold(i, j, cs[j]);
+    });
+    cs_last = cs[WTL - 1];
+#pragma unroll
+    for (int j = 0; j < WTL; j++) cs[j] = csn[j] * rblkn;
+    advance();
+    other_stage();
+  };
+  // a wave without valid rows: loads and barriers only, in the order of the working waves
+  auto idle_step = [&](int kb, auto S) __attribute__((always_inline)) {
+    barrier_q();
+    static_for<4>([&](auto N) __attribute__((always_inline)) { load_l(S, N); });
+    if (kb == 0 && stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + kStores) : "memory");
+    else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    ask_in_step(kb);
+    static_for<4>([&](auto N) __attribute__((always_inline)) { load_r(S, N); });
+    advance();
+    other_stage();
+  };
+
+  // ---- a finished tile: registers -> memory.  A lane holds, for output row l32 of a sub-tile, columns 8 q + 4 hg .. + 3 (q =
+  // 0 .. 3).  Lanes exchange what they hold until a lane has 16 bytes and four lanes 64 consecutive bytes of a row; 16 rows
+  // to an instruction.
+  auto store_tile = [&](const Tile t) __attribute__((always_inline)) {
+    const auto a = args();
+    constexpr uint32_t kEl = sizeof(OUT);
+    const int left = t.lvalid - wlrow0, rows = left < 64 ? left : 64;
+    const v4i out = buffer_at(reinterpret_cast<OUT*>(a->C) + ((t.l0 + wlrow0) * a->ldc + t.r0 + wrow0),
+                              ((uint32_t)(rows - 1) * (uint32_t)a->ldc + 128u) * kEl);
+    const int ln = lane_here(), b4 = (ln >> 4) & 1, h5 = ln >> 5;
+    const uint32_t at = ((uint32_t)(ln & 15) * (uint32_t)a->ldc + (uint32_t)(kEl == 4 ? 8 * b4 + 4 * h5 : 8 * (2 * b4 + h5))) * kEl;
+    if (opaque(a->bias != nullptr)) {
+#pragma unroll
+      for (int i = 0; i < WTR; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int64_t col = (int64_t)t.g * a->bias_group_stride + t.r0 + wrow0 + i * 32 + 8 * q + 4 * h5;
+          v4f b;
+          if (opaque(a->bias_dtype == AAMD_F32)) {
+            b = *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(a->bias) + col);
+          } else {
+            const v2i raw = *reinterpret_cast<const v2i*>(reinterpret_cast<const u16*>(a->bias) + col);
+            b = v4f{bf16_bits_to_f32((uint32_t)raw[0] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[0] >> 16),
+                    bf16_bits_to_f32((uint32_t)raw[1] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[1] >> 16)};
+          }
+#pragma unroll
+          for (int j = 0; j < WTL; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][4 * q + r] += b[r];
+        }
+    }
+    static_for<NTILES>([&](auto T) __attribute__((always_inline)) {
+      constexpr int i = decltype(T)::value % WTR, j = decltype(T)::value / WTR;
+      const v16f& o = acc[i][j];
+      const uint32_t row = at + (uint32_t)(j * 32) * (uint32_t)a->ldc * kEl, row16 = row + 16u * (uint32_t)a->ldc * kEl;
+      if constexpr (kEl == 4) {
+#pragma unroll
+        for (int qp = 0; qp < 2; qp++) {
+          v4i x, y;
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float f = o[8 * qp + r], h = o[8 * qp + 4 + r];
+            int u = __builtin_bit_cast(int, f), v = __builtin_bit_cast(int, h);
+            swap16(u, v);
+            x[r] = u;
+            y[r] = v;
+          }
+          store_x4<i * 32 * 4>(x, row + (uint32_t)(qp * 64), out);
+          store_x4<i * 32 * 4>(y, row16 + (uint32_t)(qp * 64), out);
+        }
+      } else {
+        int w[2][4];  // [pair of q][the 16 bytes of q = 2 pair + hg]
+#pragma unroll
+        for (int qp = 0; qp < 2; qp++)
+#pragma unroll
+          for (int r = 0; r < 2; r++) {
+            int u = (int)pack_bf16x2(o[8 * qp + 2 * r], o[8 * qp + 2 * r + 1]), v = (int)pack_bf16x2(o[8 * qp + 4 + 2 * r], o[8 * qp + 5 + 2 * r]);
+            swap32(u, v);
+            w[qp][r] = u;
+            w[qp][2 + r] = v;
+          }
+        v4i x, y;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          swap16(w[0][r], w[1][r]);
+          x[r] = w[0][r];
+          y[r] = w[1][r];
+        }
+        store_x4<i * 32 * 2>(x, row, out);
+        store_x4<i * 32 * 2>(y, row16, out);
+      }
+    });
+  };
+
+  // ---- the first tile's blocks 0 and 1
+  constexpr std::integral_constant<int, 0> S0{};
+  constexpr std::integral_constant<int, 1> S1{};
+  load_tile(S0);
+  ask_scales(current(), 0, 0, &p);
+  advance_buffer(lbuf, kBK);
+  advance_buffer(rbuf, p.r_kb_stride);
+  other_stage();
+  load_tile(S1);
+  advance_buffer(lbuf, kBK);
+  advance_buffer(rbuf, p.r_kb_stride);
+  other_stage();
+  to_load -= 2;
+
+  bool first = true;
+  for (;;) {
+    const bool more = take(pid);
+    if (more) take_tile(pid, args());
+    next_block = more ? 0 : nkb - 1;
+    first_ask();
+    if (first) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the first tile's block 0 and scales
+    first = false;
+    const bool work = wrow0 < c_rvalid && wlrow0 < c_lvalid;
+    if (work) {
+      first_fragments();
+      first_scales();
+#pragma unroll
+      for (int j = 0; j < WTL; j++) cs[j] = csn[j] * rblkn;
+#pragma unroll
+      for (int i = 0; i < WTR; i++)
+#pragma unroll
+        for (int j = 0; j < WTL; j++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r++) pr[r] = 0.f;
+      cs_last = 0.f;
+      for (int kb = 0; kb < nkb; kb++) {
+        step(kb, S0);
+        if constexpr (PAIRS) step(++kb, S1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      fold(WTR - 1, WTL - 1, cs_last);
+      store_tile(current());
+    } else {
+      for (int kb = 0; kb < nkb; kb++) {
+        idle_step(kb, S0);
+        if constexpr (PAIRS) idle_step(++kb, S1);
+      }
+      if (!PAIRS) {
+        other_l();
+        other_r();
+      }
+    }
+    stored = work;
+    if (!more) break;
+    sc_parity = (sc_parity + last_batch + 1) & 1;
+    next_is_current();
+  }
+  // No load may land in an LDS that is no longer this workgroup's; the stores behind the last loads need nobody to wait.
+  if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStores) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <typename OUT, bool R_ROWS>
+static void launch_row_tiles_as(const GemmParams& p, unsigned blocks, hipStream_t st) {
+  if (p.nkb % 2 == 0) row_tiles_kernel<OUT, R_ROWS, true><<<blocks, rows::NT, 0, st>>>(p);
+  else row_tiles_kernel<OUT, R_ROWS, false><<<blocks, rows::NT, 0, st>>>(p);
+}
+int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st) {
+  AAMD_REQUIRE(tiles < 0x7fffffffLL, "grouped_gemm: grid too large");
+  const unsigned blocks = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, rows::kWorkgroups);
+  if (c_dtype == AAMD_BF16) {
+    if (r_rows) launch_row_tiles_as<u16, true>(p, blocks, st);
+    else launch_row_tiles_as<u16, false>(p, blocks, st);
+  } else {
+    if (r_rows) launch_row_tiles_as<float, true>(p, blocks, st);
+    else launch_row_tiles_as<float, false>(p, blocks, st);
+  }
+  AAMD_LAUNCH_CHECK("grouped_gemm (256 x 256 tiles)");
+  return AAMD_OK;
+}
+
+}  // namespace aamd
