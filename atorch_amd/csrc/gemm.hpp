@@ -39,6 +39,7 @@ struct GemmParams {
   int gl;          // L tiles that share an R panel in the tile order
   int run;         // kRaggedK: tiles of short groups that a workgroup takes one after the other (0: none)
   int short_kb;    // kRaggedK: the most contraction blocks of a short group
+  int stream_out;  // row_tiles_kernel: the output is stored past the caches
   int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
 };
 

@@ -24,7 +24,7 @@
 // are left to the range check of buffer instructions, which neither reads nor writes them.
 #include <algorithm>
 
-#include "gemm.hpp"
+#include "gemm_tiles.hpp"
 
 namespace aamd {
 
@@ -35,61 +35,6 @@ constexpr int kScaleBatch = BM * 8 + 256;  // floats: the scales of eight contra
 constexpr int kLds = 4 * kSide + 2 * kScaleBatch * 4 + 64 * (int)sizeof(int64_t) * 3;
 constexpr int kWorkgroups = 256;        // one per CU
 }  // namespace rows
-
-// A raw buffer of `bytes` bytes at `base`: reads past it give 0, writes past it are dropped.
-__device__ __forceinline__ v4i buffer_at(const void* base, uint32_t bytes) {
-  const uint64_t a = (uint64_t)(uintptr_t)base;
-  return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};  // (addresses have 47 bits)
-}
-template <int OFFSET>
-__device__ __forceinline__ void load_lds_x4(uint32_t off, const v4i& buf, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buf), "s"(lds), "i"(OFFSET) : "memory", "scc");
-}
-__device__ __forceinline__ void advance_buffer(v4i& b, int64_t by) {
-  const uint64_t a = (((uint64_t)(uint32_t)b[1] << 32) | (uint32_t)b[0]) + (uint64_t)by;
-  b[0] = (int)(uint32_t)a;
-  b[1] = (int)(uint32_t)(a >> 32);
-}
-__device__ __forceinline__ void load_lds_x1(uint32_t off, const v4i& buf, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(buf), "s"(lds) : "memory");
-}
-
-// A uniform value the compiler knows nothing about: a branch on it inside the tile loop stays there (a loop per case would be a
-// copy of the whole kernel each).
-__device__ __forceinline__ int opaque(int v) {
-  v = __builtin_amdgcn_readfirstlane(v);
-  asm volatile("" : "+s"(v));
-  return __builtin_amdgcn_readfirstlane(v);
-}
-// The lane, counted anew: what is computed from it lives where it is used, not in registers across the tile loop.
-__device__ __forceinline__ int lane_here() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-  return l;
-}
-// (the compiler does not see what is inside: five wait states in front, for scalar registers that the vector unit has just
-// written, and two behind, before the data registers are written again)
-__device__ __forceinline__ uint64_t args_here() {
-  uint64_t a = (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(a));
-  return (uint64_t)uniform_i64((int64_t)a);
-}
-template <int OFFSET>
-__device__ __forceinline__ void store_x4(const v4i& v, uint32_t off, const v4i& buf) {
-  asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, 0 offen offset:%3\n\ts_nop 1" ::"v"(v), "v"(off), "s"(buf), "n"(OFFSET) : "memory");
-}
-
-// a.upper half of the lanes <-> b.lower half; odd rows of 16 lanes of a <-> even rows of b
-__device__ __forceinline__ void swap32(int& a, int& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  a = (int)r[0];
-  b = (int)r[1];
-}
-__device__ __forceinline__ void swap16(int& a, int& b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-  a = (int)r[0];
-  b = (int)r[1];
-}
 
 // R_ROWS: the R operand is stored [contraction, Rrows] and its fragments are read transposed, see grouped_gemm_kernel.
 // PAIRS: an even number of steps per tile, so that a step's number says which stage it works on and the stage goes into the
@@ -104,7 +49,6 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   // [L stage 0 | L stage 1 | R stage 0 | R stage 1 | two batches of scales | rows and tiles of the groups]
   float* const scales = reinterpret_cast<float*>(lds + 4 * kSide);
   int64_t* const table = reinterpret_cast<int64_t*>(scales + 2 * kScaleBatch);
-  auto lds_addr = [](const void* q) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)q; };
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -253,7 +197,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
     if (--to_load == 0) enter_next(args());
   };
   // where this wave's loads go, in the stage of the step under way (PAIRS: in stage 0)
-  uint32_t to_lds = lds_addr(lds) + (uint32_t)(wave * 1024);
+  uint32_t to_lds = lds_offset(lds) + (uint32_t)(wave * 1024);
   auto load_l = [&](auto S, auto N) __attribute__((always_inline)) {
     load_lds_x4<(PAIRS ? decltype(S)::value * kSide : 0) + decltype(N)::value * 8192>(voffL[decltype(N)::value], lbuf, to_lds);
   };
@@ -278,7 +222,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   auto ask_scales = [&](const Tile t, int b, int parity, auto a) __attribute__((always_inline)) {
     const int at = batch_start(b), ln = lane_here();
     const v4i lb = buffer_at(a->Ls + uniform_i64(t.l0 * lsr + at), (uint32_t)__builtin_amdgcn_readfirstlane(((t.lvalid - 1) * (int)lsr + 8) * 4));
-    const uint32_t ld = lds_addr(scales + parity * kScaleBatch) + (uint32_t)(wave * 1024);
+    const uint32_t ld = lds_offset(scales + parity * kScaleBatch) + (uint32_t)(wave * 1024);
     const int wide = opaque(x4);
     if (wide) {
       load_lds_x4<0>(((uint32_t)(wave * 32 + (ln >> 1)) * lsr + (uint32_t)(ln & 1) * 4u) * 4u, lb, ld);
@@ -291,7 +235,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
       const int blocks = t.rvalid / kTile;
       const v4i rb = buffer_at(a->Rs + uniform_i64((int64_t)t.g * a->rs_group_stride + (int64_t)(t.r0 / kTile) * rsr + (int64_t)at * rsb),
                                (uint32_t)__builtin_amdgcn_readfirstlane((R_ROWS ? 7 * (int)rsb + blocks : (blocks - 1) * (int)rsr + 8) * 4));
-      const uint32_t rd = lds_addr(scales + parity * kScaleBatch + BM * 8);
+      const uint32_t rd = lds_offset(scales + parity * kScaleBatch + BM * 8);
       if (wide && !R_ROWS) load_lds_x4<0>(((uint32_t)((ln >> 1) & 1) * rsr + (uint32_t)(ln & 1) * 4u) * 4u, rb, rd);
       else load_lds_x1(((uint32_t)((ln >> 3) & 1) * rsr + (uint32_t)(ln & 7) * rsb) * 4u, rb, rd);
     }
@@ -308,13 +252,13 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       const uint32_t chk = (uint32_t)(((4 * h + 2 * hg + c) ^ sw) << 4);
-      la[h][c] = lds_addr(lds) + (uint32_t)((wlrow0 + l32) * kBK) + chk;
+      la[h][c] = lds_offset(lds) + (uint32_t)((wlrow0 + l32) * kBK) + chk;
       if constexpr (R_ROWS) {
         const int tr = (lane & 15) >> 1;
         const int ch = (wrow0 / 16 + 2 * (2 * h + c) + ((lane >> 4) & 1)) ^ (2 * tr);
-        ra[h][c] = lds_addr(lds) + 2 * kSide + (uint32_t)((32 * hg + tr) * BN + ch * 16 + (lane & 1) * 8);
+        ra[h][c] = lds_offset(lds) + 2 * kSide + (uint32_t)((32 * hg + tr) * BN + ch * 16 + (lane & 1) * 8);
       } else {
-        ra[h][c] = lds_addr(lds) + 2 * kSide + (uint32_t)((wrow0 + l32) * kBK) + chk;
+        ra[h][c] = lds_offset(lds) + 2 * kSide + (uint32_t)((wrow0 + l32) * kBK) + chk;
       }
     }
   // (without PAIRS: during a step `la` names the stage of the next one, and `ra` too from the middle of the step on)
@@ -363,7 +307,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   int sc_parity = 0;  // of the tile's batch 0
   uint32_t sc_at = 0;
   int sc_left = 0, sc_more = 0;
-  const uint32_t sc_l = lds_addr(scales) + (uint32_t)((wlrow0 + l32) * 32), sc_r = lds_addr(scales) + (uint32_t)(BM * 32 + (wrow0 / kTile) * 32);
+  const uint32_t sc_l = lds_offset(scales) + (uint32_t)((wlrow0 + l32) * 32), sc_r = lds_offset(scales) + (uint32_t)(BM * 32 + (wrow0 / kTile) * 32);
   auto read_scales = [&]() __attribute__((always_inline)) {
     typedef const __attribute__((address_space(3))) float* lds_float_t;
     const lds_float_t l = (lds_float_t)(uintptr_t)(sc_l + sc_at);
@@ -487,17 +431,15 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
     other_stage();
   };
 
-  // ---- a finished tile: registers -> memory.  A lane holds, for output row l32 of a sub-tile, columns 8 q + 4 hg .. + 3 (q =
-  // 0 .. 3).  Lanes exchange what they hold until a lane has 16 bytes and four lanes 64 consecutive bytes of a row; 16 rows
-  // to an instruction.
+  // ---- a finished tile: registers -> memory
   auto store_tile = [&](const Tile t) __attribute__((always_inline)) {
     const auto a = args();
     constexpr uint32_t kEl = sizeof(OUT);
     const int left = t.lvalid - wlrow0, rows = left < 64 ? left : 64;
     const v4i out = buffer_at(reinterpret_cast<OUT*>(a->C) + ((t.l0 + wlrow0) * a->ldc + t.r0 + wrow0),
                               ((uint32_t)(rows - 1) * (uint32_t)a->ldc + 128u) * kEl);
-    const int ln = lane_here(), b4 = (ln >> 4) & 1, h5 = ln >> 5;
-    const uint32_t at = ((uint32_t)(ln & 15) * (uint32_t)a->ldc + (uint32_t)(kEl == 4 ? 8 * b4 + 4 * h5 : 8 * (2 * b4 + h5))) * kEl;
+    const int ln = lane_here(), h5 = ln >> 5;
+    const uint32_t at = store_offset<OUT>(ln, (uint32_t)a->ldc);
     if (opaque(a->bias != nullptr)) {
 #pragma unroll
       for (int i = 0; i < WTR; i++)
@@ -518,47 +460,15 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
             for (int r = 0; r < 4; r++) acc[i][j][4 * q + r] += b[r];
         }
     }
-    static_for<NTILES>([&](auto T) __attribute__((always_inline)) {
-      constexpr int i = decltype(T)::value % WTR, j = decltype(T)::value / WTR;
-      const v16f& o = acc[i][j];
-      const uint32_t row = at + (uint32_t)(j * 32) * (uint32_t)a->ldc * kEl, row16 = row + 16u * (uint32_t)a->ldc * kEl;
-      if constexpr (kEl == 4) {
-#pragma unroll
-        for (int qp = 0; qp < 2; qp++) {
-          v4i x, y;
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float f = o[8 * qp + r], h = o[8 * qp + 4 + r];
-            int u = __builtin_bit_cast(int, f), v = __builtin_bit_cast(int, h);
-            swap16(u, v);
-            x[r] = u;
-            y[r] = v;
-          }
-          store_x4<i * 32 * 4>(x, row + (uint32_t)(qp * 64), out);
-          store_x4<i * 32 * 4>(y, row16 + (uint32_t)(qp * 64), out);
-        }
-      } else {
-        int w[2][4];  // [pair of q][the 16 bytes of q = 2 pair + hg]
-#pragma unroll
-        for (int qp = 0; qp < 2; qp++)
-#pragma unroll
-          for (int r = 0; r < 2; r++) {
-            int u = (int)pack_bf16x2(o[8 * qp + 2 * r], o[8 * qp + 2 * r + 1]), v = (int)pack_bf16x2(o[8 * qp + 4 + 2 * r], o[8 * qp + 5 + 2 * r]);
-            swap32(u, v);
-            w[qp][r] = u;
-            w[qp][2 + r] = v;
-          }
-        v4i x, y;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          swap16(w[0][r], w[1][r]);
-          x[r] = w[0][r];
-          y[r] = w[1][r];
-        }
-        store_x4<i * 32 * 2>(x, row, out);
-        store_x4<i * 32 * 2>(y, row16, out);
-      }
-    });
+    auto store_as = [&](auto nt) __attribute__((always_inline)) {
+      static_for<NTILES / 2>([&](auto T) __attribute__((always_inline)) {
+        constexpr int i = 2 * (decltype(T)::value % (WTR / 2)), j = decltype(T)::value / (WTR / 2);
+        store_sub_tiles<OUT, i * 32, decltype(nt)::value>(acc[i][j], acc[i + 1][j], at + (uint32_t)(j * 32) * (uint32_t)a->ldc * kEl,
+                                                          (uint32_t)a->ldc, out);
+      });
+    };
+    if (opaque(a->stream_out)) store_as(std::true_type{});
+    else store_as(std::false_type{});
   };
 
   // ---- the first tile's blocks 0 and 1
@@ -633,6 +543,10 @@ static void launch_row_tiles_as(const GemmParams& p, unsigned blocks, hipStream_
 int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st) {
   AAMD_REQUIRE(tiles < 0x7fffffffLL, "grouped_gemm: grid too large");
   const unsigned blocks = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, rows::kWorkgroups);
+  // Streaming stores keep a large output from evicting the operands from the last-level cache, and cost a launch that is short
+  // of steps to hide them (us, plain and streaming: 4096 x 32768 outputs (268 MB), contraction 4096 492 -> 464, 2048 267 -> 272,
+  // 1024 160 -> 175; 32768 x 28672 (1.9 GB), 4096 3449 -> 3414; 4096 x 14336 (117 MB), 4096 222 both).
+  p.stream_out = p.nkb >= 32 && p.Lrows * p.Rrows * (c_dtype == AAMD_BF16 ? 2 : 4) >= (int64_t)1 << 28;
   if (c_dtype == AAMD_BF16) {
     if (r_rows) launch_row_tiles_as<u16, true>(p, blocks, st);
     else launch_row_tiles_as<u16, false>(p, blocks, st);
