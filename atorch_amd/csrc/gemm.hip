@@ -1040,6 +1040,15 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
   return AAMD_OK;
 }
 
+// The 256 x 256 tiles' last round may share out its contraction (row_tiles_kernel) from this many blocks on.  Measured on MI355X,
+// us, without and with, 4096 outputs, one round of 256 tiles and a last one of 1 / 4 / 8 / 12 / 16 tiles per XCD (in 8 / 8 / 4 / 2 /
+// 2 parts): 48 blocks 148 / 150 / 154 / 157 / 161 -> 123 / 128 / 138 / 149 / 159, 64 blocks 193 / 197 / 203 / 206 / 210 -> 155 /
+// 163 / 170 / 187 / 200, 112 blocks 327 / 337 / 345 / 349 / 354 -> 245 / 256 / 273 / 303 / 322; 32 blocks, 16 tiles 112 -> 122.
+// Where nothing is shared the second launch costs 2 to 4 us of at least 100.
+constexpr int kSplitBlocks = 48;
+// The most parts of a contraction: eight blocks at least in each, see row_part.
+static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8); }
+
 // Which kernel a row-ragged launch with block-scaled R takes: the one whose estimated time is least.  The estimates (us)
 // are fits to 570 launches on MI355X of 64 to 40000 rows in 1 to 64 even or uneven groups, 512 to 18000 outputs and a
 // contraction of 512 to 14336, each with all of the kernels (n: its 128-deep steps):
@@ -1060,7 +1069,8 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
 enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3 };
 // (weights read along their rows, b_rows: the same line but for the split form, which they do not have; 128 x 32 blocks of the
 // kernel for few rows are as many as 64 x 64 ones)
-static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, const GemmOptions& g_opt) {
+// share_last: with a workspace for parts of the last round of 256 x 256 tiles.
+static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return g_opt.tile == 1 && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const int64_t groups = M < E ? M : E;
   const double n = (double)nkb;
@@ -1075,7 +1085,12 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   const double small = std::max(tiles_s <= 256.0 ? 5.4 + 0.7 * n : 2.5 + rounds(tiles_s / 512.0) * (2.4 + 0.98 * n), weights / 5.6);
   // (the large configuration takes its scales in batches of eight contraction blocks)
   const double rows_l = token_tiles(256), fill = std::min(1.0, (double)M / (256.0 * rows_l));
-  const double loop_l = 2.3 + rounds(rows_l * (double)((N + 255) / 256) / 256.0) * (5.9 + (0.82 + 0.6 * fill) * n);
+  const double rounds_l = rows_l * (double)((N + 255) / 256) / 256.0, step_l = 0.82 + 0.6 * fill;
+  double loop_l = 2.3 + rounds(rounds_l) * (5.9 + step_l * n);
+  // (a last round in parts, after one or two whole ones: its steps, and 33 us for writing and adding the parts)
+  const double whole = std::floor(rounds_l), parts = std::min((double)row_max_split(nkb), std::floor(1.0 / (rounds_l - whole + 1e-9)));
+  if (share_last && whole >= 1.0 && whole < 3.0 && parts >= 2.0 && rounds_l > whole)
+    loop_l = std::min(loop_l, 2.3 + whole * (5.9 + step_l * n) + 33.0 + step_l * n / parts);
   const double large = nkb < 8 ? 1e30 : std::max(loop_l, weights / 5.2);
   const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_p = token_tiles(32) * (double)(N / 32);
   const double few = std::max({4.5 + 1e-3 * blocks_f * (1.06 * n + 2.1), 1.5 + 1.1 * std::ceil(n / 4.0), weights / 6.2});
@@ -1125,7 +1140,7 @@ using namespace aamd;
 static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
                         int b_tile_scaled, bool b_rows, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
                         int c_dtype, int64_t ldc, const void* bias, int bias_dtype, void* stream,
-                        const GemmOptions& g_opt = GemmOptions()) {
+                        const GemmOptions& g_opt = GemmOptions(), float* ws = nullptr) {
   AAMD_REQUIRE(c_dtype == AAMD_BF16 || c_dtype == AAMD_F32, "grouped_gemm_nt: unsupported output dtype %d", c_dtype);
   AAMD_REQUIRE(M >= 0 && N >= 0 && K >= 0, "grouped_gemm_nt: negative size");
   AAMD_REQUIRE(K % kBK == 0 && N % kTile == 0, "grouped_gemm_nt: K=%lld and N=%lld must be multiples of 128",
@@ -1145,7 +1160,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   const bool batches = (K / kBK) >= 8 && g_opt.ls_batch != 0;
   const bool batches16 = batches && (K / kBK) % 4 == 0 && aligned16(a_s);
   const NtKernel kernel = b_tile_scaled ? (use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), g_opt) ? kLargeTiles : kSmallTiles)
-                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, g_opt);
+                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, ws != nullptr, g_opt);
   // (output rows of 8 M elements are out of reach of the large tiles' 32-bit offsets)
   const bool large = kernel == kLargeTiles && (b_tile_scaled || ldc < (1LL << 23));
   const int BM = large ? kLargeTile : CfgSmall::BM;
@@ -1174,6 +1189,8 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   const int64_t blocks = max_lt * p.nRt;
   if (large && !b_tile_scaled) {
     tile_order<kRaggedRows>(p, kLargeTile, g_opt);
+    p.ws = ws;
+    p.max_split = ws != nullptr ? row_max_split(p.nkb) : 1;
     return launch_row_tiles(p, c_dtype, blocks, b_rows, st);
   }
   if (b_rows) return launch_gemm<kRaggedRows, false, CfgSmall, true>(p, c_dtype, blocks, st, g_opt);
@@ -1207,6 +1224,23 @@ extern "C" int aamd_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const flo
                                         const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
                                         int c_dtype, int64_t ldc, const void* bias, int bias_dtype, void* stream) {
   return gemm_nt_impl(a, lda, a_s, b, b_s, 0, true, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype, stream);
+}
+
+extern "C" int64_t aamd_grouped_gemm_fp8_ws_bytes(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows) {
+  const int64_t nkb = K / kBK;
+  if (M <= 0 || N <= 0 || E < 1 || nkb < kSplitBlocks) return 0;
+  // (the tiles of groups are counted on the device)
+  const int64_t tiles = (M + kLargeTile - 1) / kLargeTile * ((N + kLargeTile - 1) / kLargeTile), left = (tiles + 7) / 8 % 32;
+  if (!grouped && (left == 0 || left > 16)) return 0;
+  return choose_nt(M, N, nkb, E, grouped != 0, b_rows != 0, true, GemmOptions()) == kLargeTiles ? kRowPartsBytes : 0;
+}
+extern "C" int aamd_grouped_gemm_fp8_ws(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
+                                        int b_rows, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
+                                        int c_dtype, int64_t ldc, const void* bias, int bias_dtype, float* ws, int64_t ws_bytes,
+                                        void* stream) {
+  AAMD_REQUIRE(ws == nullptr || (ws_bytes >= kRowPartsBytes && aligned16(ws)), "grouped_gemm_ws: the workspace needs %lld bytes, 16-byte aligned", (long long)kRowPartsBytes);
+  return gemm_nt_impl(a, lda, a_s, b, b_s, 0, b_rows != 0, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype, stream,
+                      GemmOptions(), ws);
 }
 #endif  // !AAMD_TUNING
 

@@ -39,6 +39,8 @@ struct GemmParams {
   int gl;          // L tiles that share an R panel in the tile order
   int run;         // kRaggedK: tiles of short groups that a workgroup takes one after the other (0: none)
   int short_kb;    // kRaggedK: the most contraction blocks of a short group
+  int max_split;   // row_tiles_kernel: the most parts of a tile's contraction; more than one: ws holds kRowPartsBytes
+  float* ws;
   int stream_out;  // row_tiles_kernel: the output is stored past the caches
   int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
 };
@@ -74,6 +76,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // bias, goff, E, Lrows, Rrows and nkb of the parameters.  r_rows: R is stored [contraction, Rrows] (R_ROWS of gemm.hip).
 int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st);
 
+constexpr int64_t kRowPartsBytes = (int64_t)256 * kLargeTile * kLargeTile * 4;  // a tile of fp32 for each of 256 workgroups
 // Row-ragged GEMM with block-scaled R on 256 x 256 tiles (gemm_rows.hip): at least eight contraction blocks, p.ls_batch 1 where
 // rows of scales are 16-byte aligned; `tiles`: no fewer than there are.
 int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st);

@@ -22,6 +22,10 @@
 // to memory (lanes swap halves, so that four of them hold 64 consecutive bytes of a row) while those loads are in flight, as
 // the stage buffers hold them.  What a tile needs besides are scalars: rows past its end and columns past the weights' end
 // are left to the range check of buffer instructions, which neither reads nor writes them.
+//
+// The last round of tiles seldom fills the card.  Where at most half the workgroups of an XCD have a tile in it and the
+// contraction is long, two to eight of them share the contraction of a tile: each leaves its fp32 sums in a workspace, and a
+// second kernel adds them in the order of the contraction, so that the result does not depend on which comes first.
 #include <algorithm>
 
 #include "gemm_tiles.hpp"
@@ -35,6 +39,100 @@ constexpr int kScaleBatch = BM * 8 + 256;  // floats: the scales of eight contra
 constexpr int kLds = 4 * kSide + 2 * kScaleBatch * 4 + 64 * (int)sizeof(int64_t) * 3;
 constexpr int kWorkgroups = 256;        // one per CU
 }  // namespace rows
+
+// A tile of the output, or a part of its contraction.
+struct RowTile {
+  int64_t l0;                 // first L row
+  int g, lvalid, r0, rvalid;  // group, valid L rows, first R row and valid R rows (a multiple of 128)
+  int kb0, steps;             // contraction blocks
+};
+// Tile `pid` of the launch (its whole contraction).  table: rows and tiles of up to 64 groups in the LDS, or null.
+template <typename ARGS>
+__device__ __forceinline__ RowTile row_tile(ARGS a, const int64_t* table, uint32_t pid, uint32_t nRt, int total_lt) {
+  using namespace rows;
+  const uint32_t GL = (uint32_t)a->gl;
+  RowTile t;
+  uint32_t lt, rt;
+  // groups of GL L tiles, R tile index outer, L tile inner
+  {
+    const uint32_t width = GL * nRt, grp = pid / width, in = pid - grp * width, first = grp * GL;
+    const uint32_t gsz = (uint32_t)total_lt - first < GL ? (uint32_t)total_lt - first : GL;
+    rt = in / gsz;
+    lt = first + (in - rt * gsz);
+  }
+  t.g = 0;
+  int64_t r_lo = 0, r_hi = a->Lrows;
+  uint32_t t_lo = 0;
+  if (opaque(a->goff != nullptr)) {
+    // exactly one group holds the tile; with group_r the tile ids of a group are contiguous, in batches of GL R tiles, all L
+    // tiles of the group inside a batch, R index fastest: the weights, the large operand, are then fetched once
+    const int by_group = opaque(a->group_r), in_table = opaque(table != nullptr);
+    GroupRanges r;
+    if (in_table) {
+      const int64_t* const e = table + lane_here() * 3;
+      r.r_lo = e[0];
+      r.r_hi = e[1];
+      const int64_t tt = e[2];
+      r.t_lo = (int)(uint32_t)(uint64_t)tt;
+      r.t_hi = (int)(uint32_t)((uint64_t)tt >> 32);
+    }
+    for (int base = 0, carry = 0; base < a->E; base += 64) {
+      if (!in_table) {
+        r = group_ranges<BM>(a->goff, a->E, base, carry);
+        carry = r.total;
+      }
+      const bool mine = by_group ? pid >= (uint32_t)r.t_lo * nRt && pid < (uint32_t)r.t_hi * nRt
+                                  : lt >= (uint32_t)r.t_lo && lt < (uint32_t)r.t_hi;  // (empty groups hold no tile)
+      const unsigned long long hit = __ballot(mine);
+      if (hit != 0) {
+        const int src = __builtin_ctzll(hit);
+        t.g = base + src;
+        t_lo = (uint32_t)__builtin_amdgcn_readlane(r.t_lo, src);
+        r_lo = readlane_i64(r.r_lo, src);
+        r_hi = readlane_i64(r.r_hi, src);
+        if (by_group) {
+          const uint32_t nl = (uint32_t)__builtin_amdgcn_readlane(r.t_hi, src) - t_lo;
+          const uint32_t pe = pid - t_lo * nRt, width = GL * nl, batch = pe / width, in = pe - batch * width, first = batch * GL;
+          const uint32_t gsz = nRt - first < GL ? nRt - first : GL;
+          const uint32_t l = in / gsz;
+          rt = first + (in - l * gsz);
+          lt = t_lo + l;
+        }
+        break;
+      }
+    }
+  }
+  t.l0 = uniform_i64(r_lo + (int64_t)(lt - t_lo) * BM);
+  const int64_t left = (r_hi < a->Lrows ? r_hi : a->Lrows) - t.l0;
+  t.lvalid = __builtin_amdgcn_readfirstlane(left < BM ? (int)left : BM);
+  t.g = __builtin_amdgcn_readfirstlane(t.g);
+  t.r0 = __builtin_amdgcn_readfirstlane((int)(rt * BN));
+  t.rvalid = (int)(a->Rrows - t.r0 < BN ? a->Rrows - t.r0 : BN);
+  t.kb0 = 0;
+  t.steps = a->nkb;
+  return t;
+}
+
+// The tiles of an XCD, a contiguous range, and how its workgroups share what is left in the last round: with few tiles left
+// several of them take parts of the contraction of one.
+struct RowTiles {
+  uint32_t first, end;
+  __device__ RowTiles(uint32_t ntot, uint32_t xcd) {
+    const uint32_t per = ntot >> 3, rem = ntot & 7u;
+    first = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
+    end = first + per + (xcd < rem ? 1u : 0u);
+  }
+};
+// Workgroups per tile when `left` tiles are left for nwg of them: 1, or up to max_split.
+__device__ __forceinline__ uint32_t row_split(uint32_t left, uint32_t nwg, uint32_t max_split) {
+  const uint32_t s = left > 0 ? nwg / left : 1;
+  return s < 1 ? 1 : s < max_split ? s : max_split;
+}
+// First contraction block of a part: whole groups of four (16 bytes of scales) but for the end of the last part.  With
+// nkb >= 8 split every part has eight blocks or more.
+__device__ __forceinline__ uint32_t row_part(uint32_t nkb, uint32_t split, uint32_t part) {
+  return part == split ? nkb : 4u * ((nkb >> 2) * part / split);
+}
 
 // R_ROWS: the R operand is stored [contraction, Rrows] and its fragments are read transposed, see grouped_gemm_kernel.
 // PAIRS: an even number of steps per tile, so that a step's number says which stage it works on and the stage goes into the
@@ -53,7 +151,6 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hg = lane >> 5;
-  const int nkb = p.nkb;
 
   // ---- the tiles of this workgroup ------------------------------------------------------------
   // Workgroup ids go round-robin over the 8 XCDs; every XCD gets one contiguous range of tile ids, in which tiles that share
@@ -73,95 +170,46 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   }
   const uint32_t nRt = (uint32_t)p.nRt, ntot = (uint32_t)total_lt * nRt;
   const uint32_t xcd = blockIdx.x & 7u, nwg = gridDim.x >> 3;
-  const uint32_t per = ntot >> 3, rem = ntot & 7u;
-  const uint32_t first_tile = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
-  const uint32_t end_tile = first_tile + per + (xcd < rem ? 1u : 0u);
+  const RowTiles mine(ntot, xcd);
 
-  struct Tile {
-    int64_t l0;               // first L row
-    int g, lvalid, r0, rvalid;  // group, valid L rows, first R row and valid R rows (a multiple of 128)
-  };
-  auto tile_of = [&](uint32_t pid, auto a) __attribute__((always_inline)) {
-    const uint32_t GL = (uint32_t)a->gl;
-    Tile t;
-    uint32_t lt, rt;
-    // groups of GL L tiles, R tile index outer, L tile inner
-    {
-      const uint32_t width = GL * nRt, grp = pid / width, in = pid - grp * width, first = grp * GL;
-      const uint32_t gsz = (uint32_t)total_lt - first < GL ? (uint32_t)total_lt - first : GL;
-      rt = in / gsz;
-      lt = first + (in - rt * gsz);
-    }
-    t.g = 0;
-    int64_t r_lo = 0, r_hi = a->Lrows;
-    uint32_t t_lo = 0;
-    if (opaque(a->goff != nullptr)) {
-      // exactly one group holds the tile; with group_r the tile ids of a group are contiguous, in batches of GL R tiles, all L
-      // tiles of the group inside a batch, R index fastest: the weights, the large operand, are then fetched once
-      const int by_group = opaque(a->group_r), in_table = opaque(a->E <= 64);
-      GroupRanges r;
-      if (in_table) {
-        const int64_t* const e = table + lane_here() * 3;
-        r.r_lo = e[0];
-        r.r_hi = e[1];
-        const int64_t tt = e[2];
-        r.t_lo = (int)(uint32_t)(uint64_t)tt;
-        r.t_hi = (int)(uint32_t)((uint64_t)tt >> 32);
-      }
-      for (int base = 0, carry = 0; base < a->E; base += 64) {
-        if (!in_table) {
-          r = group_ranges<BM>(a->goff, a->E, base, carry);
-          carry = r.total;
-        }
-        const bool mine = by_group ? pid >= (uint32_t)r.t_lo * nRt && pid < (uint32_t)r.t_hi * nRt
-                                    : lt >= (uint32_t)r.t_lo && lt < (uint32_t)r.t_hi;  // (empty groups hold no tile)
-        const unsigned long long hit = __ballot(mine);
-        if (hit != 0) {
-          const int src = __builtin_ctzll(hit);
-          t.g = base + src;
-          t_lo = (uint32_t)__builtin_amdgcn_readlane(r.t_lo, src);
-          r_lo = readlane_i64(r.r_lo, src);
-          r_hi = readlane_i64(r.r_hi, src);
-          if (by_group) {
-            const uint32_t nl = (uint32_t)__builtin_amdgcn_readlane(r.t_hi, src) - t_lo;
-            const uint32_t pe = pid - t_lo * nRt, width = GL * nl, batch = pe / width, in = pe - batch * width, first = batch * GL;
-            const uint32_t gsz = nRt - first < GL ? nRt - first : GL;
-            const uint32_t l = in / gsz;
-            rt = first + (in - l * gsz);
-            lt = t_lo + l;
-          }
-          break;
-        }
+  uint32_t round_first = mine.first, turn = blockIdx.x >> 3;
+  // the next tile of this workgroup, false if there is none; part and parts: of the contraction it takes, slot: where a part goes
+  uint32_t part = 0, parts = 1;
+  int n_slot = -1;
+  auto take = [&](uint32_t& pid) __attribute__((always_inline)) {
+    const uint32_t left = mine.end > round_first ? mine.end - round_first : 0u;
+    uint32_t at = turn;
+    if (left < nwg && p.max_split > 1) {
+      parts = row_split(left, nwg, (uint32_t)p.max_split);
+      if (parts > 1) {
+        n_slot = turn < left * parts ? (int)(xcd * nwg + turn) : -1;
+        part = turn / left;
+        at = n_slot >= 0 ? turn - part * left : left;
       }
     }
-    t.l0 = uniform_i64(r_lo + (int64_t)(lt - t_lo) * BM);
-    const int64_t left = (r_hi < a->Lrows ? r_hi : a->Lrows) - t.l0;
-    t.lvalid = __builtin_amdgcn_readfirstlane(left < BM ? (int)left : BM);
-    t.g = __builtin_amdgcn_readfirstlane(t.g);
-    t.r0 = __builtin_amdgcn_readfirstlane((int)(rt * BN));
-    t.rvalid = (int)(a->Rrows - t.r0 < BN ? a->Rrows - t.r0 : BN);
-    return t;
-  };
-  uint32_t round_first = first_tile, turn = blockIdx.x >> 3;
-  auto take = [&](uint32_t& pid) __attribute__((always_inline)) {  // the next tile of this workgroup, false if there is none
-    pid = round_first + turn;
+    pid = round_first + at;
     round_first += nwg;
     turn += nwg > 5u ? 5u : 1u;
     turn = turn >= nwg ? turn - nwg : turn;
-    return pid < end_tile;
+    return at < left;
   };
   uint32_t pid;
   if (!take(pid)) return;  // (rounds before the last are whole, so a workgroup that has no tile in one has none later)
   // (plain variables: as structures the two would live in memory)
   int64_t c_l0, n_l0;
-  int c_g, c_lvalid, c_r0, c_rvalid, n_g, n_lvalid, n_r0, n_rvalid;
+  int c_g, c_lvalid, c_r0, c_rvalid, c_kb0, c_steps, c_slot, n_g, n_lvalid, n_r0, n_rvalid, n_kb0, n_steps;
   auto take_tile = [&](uint32_t id, auto a) __attribute__((always_inline)) {
-    const Tile t = tile_of(id, a);
-    n_l0 = t.l0, n_g = t.g, n_lvalid = t.lvalid, n_r0 = t.r0, n_rvalid = t.rvalid;
+    const RowTile t = row_tile(a, opaque(a->goff != nullptr && a->E <= 64) ? table : nullptr, id, nRt, total_lt);
+    n_l0 = t.l0, n_g = t.g, n_lvalid = t.lvalid, n_r0 = t.r0, n_rvalid = t.rvalid, n_kb0 = 0, n_steps = t.steps;
+    if (n_slot >= 0) {
+      n_kb0 = (int)row_part((uint32_t)t.steps, parts, part);
+      n_steps = (int)row_part((uint32_t)t.steps, parts, part + 1) - n_kb0;
+    }
   };
-  auto next_is_current = [&]() __attribute__((always_inline)) { c_l0 = n_l0, c_g = n_g, c_lvalid = n_lvalid, c_r0 = n_r0, c_rvalid = n_rvalid; };
-  auto current = [&]() __attribute__((always_inline)) { return Tile{c_l0, c_g, c_lvalid, c_r0, c_rvalid}; };
-  auto next = [&]() __attribute__((always_inline)) { return Tile{n_l0, n_g, n_lvalid, n_r0, n_rvalid}; };
+  auto next_is_current = [&]() __attribute__((always_inline)) {
+    c_l0 = n_l0, c_g = n_g, c_lvalid = n_lvalid, c_r0 = n_r0, c_rvalid = n_rvalid, c_kb0 = n_kb0, c_steps = n_steps, c_slot = n_slot;
+  };
+  auto current = [&]() __attribute__((always_inline)) { return RowTile{c_l0, c_g, c_lvalid, c_r0, c_rvalid, c_kb0, c_steps}; };
   take_tile(pid, &p);
   next_is_current();
 
@@ -180,15 +228,16 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   // Where the next block to be requested lies: it runs through the blocks of a tile and on into the next tile; behind the
   // last one it stays on the last block, to keep the wait counts uniform.
   v4i lbuf, rbuf;
-  int to_load = nkb;   // blocks left in the tile
-  int next_block = 0;  // of the tile next(): 0, or the last one where that is still the tile under way
+  int to_load;         // blocks left in the tile
+  int next_block = 0;  // of the next tile: 0, or the last one where that is still the tile under way
   auto enter_next = [&](auto a) __attribute__((always_inline)) {
-    const int64_t l_at = n_l0 * a->ldl + next_block * kBK;
-    const int64_t r_at = (int64_t)n_g * a->r_group_stride + (R_ROWS ? (int64_t)n_r0 : n_r0 * a->ldr) + next_block * a->r_kb_stride;
+    const int block = n_kb0 + next_block;
+    const int64_t l_at = n_l0 * a->ldl + block * kBK;
+    const int64_t r_at = (int64_t)n_g * a->r_group_stride + (R_ROWS ? (int64_t)n_r0 : n_r0 * a->ldr) + block * a->r_kb_stride;
     lbuf = buffer_at(a->L + uniform_i64(l_at), (uint32_t)__builtin_amdgcn_readfirstlane((n_lvalid - 1) * (int)a->ldl + kBK));
     rbuf = buffer_at(a->R + uniform_i64(r_at), (uint32_t)__builtin_amdgcn_readfirstlane(
                                                    R_ROWS ? 127 * (int)a->ldr + n_rvalid : (n_rvalid - 1) * (int)a->ldr + kBK));
-    to_load = nkb - next_block;
+    to_load = n_steps - next_block;
   };
   enter_next(&p);
   auto advance = [&]() __attribute__((always_inline)) {
@@ -218,9 +267,8 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   // the one in use has been read for the last time.  Rows of scales that are not 16-byte aligned take 4-byte loads.
   const int x4 = p.ls_batch == 1;
   const uint32_t lsr = (uint32_t)p.ls_row_stride, rsr = (uint32_t)p.rs_row_stride, rsb = (uint32_t)p.rs_blk_stride;
-  auto batch_start = [&](int b) __attribute__((always_inline)) { return 8 * b + 8 <= nkb ? 8 * b : nkb - 8; };
-  auto ask_scales = [&](const Tile t, int b, int parity, auto a) __attribute__((always_inline)) {
-    const int at = batch_start(b), ln = lane_here();
+  auto ask_scales = [&](const RowTile t, int b, int parity, auto a) __attribute__((always_inline)) {
+    const int at = t.kb0 + (8 * b + 8 <= t.steps ? 8 * b : t.steps - 8), ln = lane_here();
     const v4i lb = buffer_at(a->Ls + uniform_i64(t.l0 * lsr + at), (uint32_t)__builtin_amdgcn_readfirstlane(((t.lvalid - 1) * (int)lsr + 8) * 4));
     const uint32_t ld = lds_offset(scales + parity * kScaleBatch) + (uint32_t)(wave * 1024);
     const int wide = opaque(x4);
@@ -303,7 +351,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
 
   // Scales of a block: the lane's L row scales and the wave's R block scale; sc_at: where the next block's are, sc_left: blocks
   // from there to the end of the batch, sc_more: batches of the tile behind it.
-  const int last_batch = (nkb - 1) >> 3, in_last = nkb - 8 * last_batch;
+  int last_batch = 0, in_last = 0;  // of the tile under way: its last batch, and the blocks of it that are new
   int sc_parity = 0;  // of the tile's batch 0
   uint32_t sc_at = 0;
   int sc_left = 0, sc_more = 0;
@@ -333,9 +381,9 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   };
   // The step that requests batch 0 of the next tile: from step 8 last_batch - 1 on the batch in front of the last is free, and
   // the last step comes too late for what the next tile begins with.
-  const int ask_next = nkb - 4 > 8 * last_batch - 1 ? nkb - 4 : 8 * last_batch - 1;
-  int ask_at = 0, ask_batch = 0;
+  int ask_at = 0, ask_batch = 0, ask_next = 0;
   auto first_ask = [&]() __attribute__((always_inline)) {
+    ask_next = c_steps - 4 > 8 * last_batch - 1 ? c_steps - 4 : 8 * last_batch - 1;
     ask_batch = 1;
     ask_at = last_batch > 0 ? 5 : ask_next;
   };
@@ -358,8 +406,9 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   auto ask_in_step = [&](int kb) __attribute__((always_inline)) {
     if (kb != ask_at) return;
     const bool of_next = ask_batch > last_batch;
-    ask_scales(Tile{of_next ? +n_l0 : +c_l0, of_next ? +n_g : +c_g, of_next ? +n_lvalid : +c_lvalid, of_next ? +n_r0 : +c_r0,
-                    of_next ? +n_rvalid : +c_rvalid}, of_next ? 0 : ask_batch, (sc_parity + ask_batch) & 1, args());
+    ask_scales(RowTile{of_next ? +n_l0 : +c_l0, of_next ? +n_g : +c_g, of_next ? +n_lvalid : +c_lvalid, of_next ? +n_r0 : +c_r0,
+                       of_next ? +n_rvalid : +c_rvalid, of_next ? +n_kb0 : +c_kb0, of_next ? +n_steps : +c_steps},
+               of_next ? 0 : ask_batch, (sc_parity + ask_batch) & 1, args());
     ask_batch++;
     ask_at = ask_batch <= last_batch ? kb + 8 : ask_batch == last_batch + 1 ? ask_next : -1;
   };
@@ -432,10 +481,19 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   };
 
   // ---- a finished tile: registers -> memory
-  auto store_tile = [&](const Tile t) __attribute__((always_inline)) {
+  auto store_tile = [&](const RowTile t) __attribute__((always_inline)) {
     const auto a = args();
     constexpr uint32_t kEl = sizeof(OUT);
     const int left = t.lvalid - wlrow0, rows = left < 64 ? left : 64;
+    if (opaque(c_slot >= 0)) {  // a part: as it is, into the workspace
+      const v4i out = buffer_at(a->ws + ((int64_t)c_slot * (BM * BN) + wlrow0 * BN + wrow0), ((uint32_t)(rows - 1) * BN + 128u) * 4u);
+      const uint32_t at = store_offset<float>(lane_here(), BN);
+      static_for<NTILES / 2>([&](auto T) __attribute__((always_inline)) {
+        constexpr int i = 2 * (decltype(T)::value % (WTR / 2)), j = decltype(T)::value / (WTR / 2);
+        store_sub_tiles<float, i * 32, false>(acc[i][j], acc[i + 1][j], at + (uint32_t)(j * 32 * BN * 4), BN, out);
+      });
+      return;
+    }
     const v4i out = buffer_at(reinterpret_cast<OUT*>(a->C) + ((t.l0 + wlrow0) * a->ldc + t.r0 + wrow0),
                               ((uint32_t)(rows - 1) * (uint32_t)a->ldc + 128u) * kEl);
     const int ln = lane_here(), h5 = ln >> 5;
@@ -489,7 +547,9 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   for (;;) {
     const bool more = take(pid);
     if (more) take_tile(pid, args());
-    next_block = more ? 0 : nkb - 1;
+    next_block = more ? 0 : n_steps - 1;
+    last_batch = (c_steps - 1) >> 3;
+    in_last = c_steps - 8 * last_batch;
     first_ask();
     if (first) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the first tile's block 0 and scales
     first = false;
@@ -508,7 +568,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
 #pragma unroll
       for (int r = 0; r < 16; r++) pr[r] = 0.f;
       cs_last = 0.f;
-      for (int kb = 0; kb < nkb; kb++) {
+      for (int kb = 0; kb < c_steps; kb++) {
         step(kb, S0);
         if constexpr (PAIRS) step(++kb, S1);
       }
@@ -516,11 +576,11 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
       fold(WTR - 1, WTL - 1, cs_last);
       store_tile(current());
     } else {
-      for (int kb = 0; kb < nkb; kb++) {
+      for (int kb = 0; kb < c_steps; kb++) {
         idle_step(kb, S0);
         if constexpr (PAIRS) idle_step(++kb, S1);
       }
-      if (!PAIRS) {
+      if (!PAIRS && (c_steps & 1)) {
         other_l();
         other_r();
       }
@@ -535,6 +595,52 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// The sums of the parts of the tiles that row_tiles_kernel has split, in the order of the contraction, with the bias: eight XCDs x
+// tiles left in the last round x eight slices of 32 rows.  Bound by memory, of which some is still in the caches: 12 tiles per XCD
+// in two parts, 50 MB, 17 us; slices of 32 rows make 768 workgroups of them, and one load of 16 bytes per lane and part is
+// in flight for each of eight rows.
+template <typename OUT>
+__global__ __launch_bounds__(256) void row_parts_kernel(const GemmParams p) {
+  using namespace rows;
+  constexpr int kSlices = 8, kRows = BM / kSlices;
+  constexpr uint32_t nwg = kWorkgroups / 8;
+  const uint32_t xcd = blockIdx.x & 7u, j = (blockIdx.x >> 3) / kSlices, slice = (blockIdx.x >> 3) % kSlices;
+  int total_lt = (int)((p.Lrows + BM - 1) / BM);
+  if (p.goff != nullptr) {
+    total_lt = group_ranges<BM>(p.goff, p.E, 0, 0).total;
+    for (int base = 64; base < p.E; base += 64) total_lt = group_ranges<BM>(p.goff, p.E, base, total_lt).total;
+  }
+  const RowTiles mine((uint32_t)total_lt * (uint32_t)p.nRt, xcd);
+  const uint32_t left = (mine.end - mine.first) % nwg, parts = row_split(left, nwg, (uint32_t)p.max_split);
+  if (parts < 2 || j >= left) return;
+  const RowTile t = row_tile(&p, nullptr, mine.end - left + j, (uint32_t)p.nRt, total_lt);
+  const int col = (int)(threadIdx.x & 63) * 4, row0 = (int)(slice * kRows + (threadIdx.x >> 6));
+  if (col >= t.rvalid) return;
+  v4f b = {0.f, 0.f, 0.f, 0.f};
+  if (p.bias != nullptr) {
+    const int64_t at = (int64_t)t.g * p.bias_group_stride + t.r0 + col;
+    if (p.bias_dtype == AAMD_F32) {
+      b = *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(p.bias) + at);
+    } else {
+      const v2i raw = *reinterpret_cast<const v2i*>(reinterpret_cast<const u16*>(p.bias) + at);
+      b = v4f{bf16_bits_to_f32((uint32_t)raw[0] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[0] >> 16),
+              bf16_bits_to_f32((uint32_t)raw[1] & 0xffffu), bf16_bits_to_f32((uint32_t)raw[1] >> 16)};
+    }
+  }
+  const float* const from = p.ws + ((int64_t)(xcd * nwg + j) * (BM * BN) + col);
+#pragma unroll
+  for (int r = 0; r < kRows; r += 4) {
+    const int row = row0 + r;
+    if (row >= t.lvalid) return;
+    v4f sum = *reinterpret_cast<const v4f*>(from + row * BN);
+    for (uint32_t i = 1; i < parts; i++) sum += *reinterpret_cast<const v4f*>(from + (int64_t)(i * left) * (BM * BN) + row * BN);
+    sum += b;
+    OUT* const out = reinterpret_cast<OUT*>(p.C) + (t.l0 + row) * p.ldc + t.r0 + col;
+    if constexpr (sizeof(OUT) == 4) *reinterpret_cast<v4f*>(out) = sum;
+    else *reinterpret_cast<v2i*>(out) = v2i{(int)pack_bf16x2(sum[0], sum[1]), (int)pack_bf16x2(sum[2], sum[3])};
+  }
+}
+
 template <typename OUT, bool R_ROWS>
 static void launch_row_tiles_as(const GemmParams& p, unsigned blocks, hipStream_t st) {
   if (p.nkb % 2 == 0) row_tiles_kernel<OUT, R_ROWS, true><<<blocks, rows::NT, 0, st>>>(p);
@@ -542,11 +648,12 @@ static void launch_row_tiles_as(const GemmParams& p, unsigned blocks, hipStream_
 }
 int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st) {
   AAMD_REQUIRE(tiles < 0x7fffffffLL, "grouped_gemm: grid too large");
-  const unsigned blocks = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, rows::kWorkgroups);
+  unsigned blocks = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, rows::kWorkgroups);
   // Streaming stores keep a large output from evicting the operands from the last-level cache, and cost a launch that is short
   // of steps to hide them (us, plain and streaming: 4096 x 32768 outputs (268 MB), contraction 4096 492 -> 464, 2048 267 -> 272,
   // 1024 160 -> 175; 32768 x 28672 (1.9 GB), 4096 3449 -> 3414; 4096 x 14336 (117 MB), 4096 222 both).
   p.stream_out = p.nkb >= 32 && p.Lrows * p.Rrows * (c_dtype == AAMD_BF16 ? 2 : 4) >= (int64_t)1 << 28;
+  if (p.max_split > 1) blocks = rows::kWorkgroups;
   if (c_dtype == AAMD_BF16) {
     if (r_rows) launch_row_tiles_as<u16, true>(p, blocks, st);
     else launch_row_tiles_as<u16, false>(p, blocks, st);
@@ -555,6 +662,12 @@ int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipS
     else launch_row_tiles_as<float, false>(p, blocks, st);
   }
   AAMD_LAUNCH_CHECK("grouped_gemm (256 x 256 tiles)");
+  if (p.max_split > 1) {
+    const unsigned sums = 8 * (rows::kWorkgroups / 8 / 2) * 8;  // (a tile is split where at most half the workgroups have one)
+    if (c_dtype == AAMD_BF16) row_parts_kernel<u16><<<sums, 256, 0, st>>>(p);
+    else row_parts_kernel<float><<<sums, 256, 0, st>>>(p);
+    AAMD_LAUNCH_CHECK("grouped_gemm (parts)");
+  }
   return AAMD_OK;
 }
 

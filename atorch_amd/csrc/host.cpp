@@ -188,6 +188,16 @@ std::tuple<Quantised, Tensor> act_dual(const Tensor& fc1, const Tensor& dh, bool
 bool is_transposed_view(const Tensor& b) {
   return b.dim() == 3 && b.size(2) > 1 && b.stride(1) == 1 && b.stride(2) == b.size(1) && b.stride(0) == b.size(1) * b.size(2);
 }
+// Workspace of a GEMM with block-scaled weights; undefined where it has no use for one, or where there is no memory for it.
+Tensor gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t E, bool grouped, bool b_rows, const Tensor& like) {
+  const int64_t bytes = aamd_grouped_gemm_fp8_ws_bytes(M, N, K, (int)E, grouped, b_rows);
+  if (bytes == 0) return Tensor();
+  try {
+    return empty({bytes / 4}, at::kFloat, like);
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
+}
 Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, const OptTensor& goff, const OptTensor& out,
                at::ScalarType out_dtype, const OptTensor& bias) {
   const int64_t M = a.size(0), K = a.size(1), E = b.size(0), N = b.size(1);
@@ -201,7 +211,13 @@ Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor
   if (goff.has_value()) check_offsets(*goff, E);
   if (bias.has_value()) check_bias(*bias, E, N);
   Tensor c = out.has_value() ? *out : empty({M, N}, out_dtype, a);
-  if (b_rows)
+  const Tensor ws = b_tile_scaled ? Tensor() : gemm_workspace(M, N, K, E, goff.has_value(), b_rows, a);
+  if (ws.defined())
+    check(aamd_grouped_gemm_fp8_ws(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(bs), b_rows,
+                                   ptr<int64_t>(goff), (int)E, M, N, K, ptr(c), dtype_code(c.scalar_type()), c.stride(0), ptr(bias),
+                                   bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, ptr<float>(ws), ws.numel() * 4,
+                                   stream()));
+  else if (b_rows)
     check(aamd_grouped_gemm_fp8_nn(ptr<uint8_t>(a), a.stride(0), ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(bs), ptr<int64_t>(goff),
                                    (int)E, M, N, K, ptr(c), dtype_code(c.scalar_type()), c.stride(0), ptr(bias),
                                    bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
@@ -259,6 +275,12 @@ Tensor fp8_gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tenso
     Tensor at = transpose_scales(a_s.view({M, blocks})), bt = transpose_scales(b_s);
     check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(a), ptr<float>(at), ptr<uint8_t>(b), ptr<float>(bt), K, AAMD_QT_ROWS, nullptr,
                                       1, nullptr, M, N, ptr(c), dtype_code(dtype), M * N, 0, stream()));
+    return c;
+  }
+  const Tensor ws = b_tile_scaled ? Tensor() : gemm_workspace(M, N, K, 1, false, false, a);
+  if (ws.defined()) {
+    check(aamd_grouped_gemm_fp8_ws(ptr<uint8_t>(a), K, ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(b_s), 0, nullptr, 1, M, N, K, ptr(c),
+                                   dtype_code(dtype), N, nullptr, AAMD_NONE, ptr<float>(ws), ws.numel() * 4, stream()));
     return c;
   }
   check(aamd_grouped_gemm_fp8_nt(ptr<uint8_t>(a), K, ptr<float>(a_s), ptr<uint8_t>(b), ptr<float>(b_s), b_tile_scaled, nullptr, 1,

@@ -242,6 +242,21 @@ int aamd_grouped_gemm_fp8_nn(const uint8_t *a, int64_t lda, const float *a_s, co
                              int64_t ldc, const void *bias, int bias_dtype, void *stream);
 
 /*
+ * The two GEMMs above (b_rows == 0 as _nt with block scales, else as _nn) with a workspace that lets them share out the
+ * contraction of the last output tiles, where fewer of those are left than the card has units.  ws_bytes() says what a
+ * launch of this size can use (0: nothing); ws may be NULL, is 16-byte aligned and belongs to the call until it has run on
+ * the stream.  The sum of a row in such a tile is made of up to eight partial sums, added in the order of the contraction;
+ * which tiles those are depends on the sizes of the groups.
+ * Replaces fp8_gemm / fp8_gemm_kernel, triton_kernel.py:143-210, and quantize_op.grouped_qgemm for fprop and dgrad,
+ * quantized_grouped_linear.py:141-151, 214-223, as they do.
+ */
+int64_t aamd_grouped_gemm_fp8_ws_bytes(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows);
+int aamd_grouped_gemm_fp8_ws(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b, const float *b_s,
+                             int b_rows, const int64_t *group_offsets, int E, int64_t M, int64_t N, int64_t K, void *c,
+                             int c_dtype, int64_t ldc, const void *bias, int bias_dtype, float *ws, int64_t ws_bytes,
+                             void *stream);
+
+/*
  * aamd_grouped_gemm_fp8_nt for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): the same arguments without
  * tile_ws.  No counterpart in the reference.  The call allocates and
