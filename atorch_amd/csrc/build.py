@@ -16,8 +16,8 @@ import sys
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ["capi.hip", "quant.hip", "permute.hip", "gemm.hip", "gemm_rows.hip", "gemm_few.hip"]
-PROBE_SOURCES = ["capi.hip", "gemm.hip", "gemm_rows.hip", "gemm_few.hip", "probe.hip"]  # compiled with -DAAMD_TUNING
+SOURCES = ["capi.hip", "quant.hip", "permute.hip", "gemm.hip", "gemm_rows.hip", "gemm_wgrad.hip", "gemm_few.hip"]
+PROBE_SOURCES = ["capi.hip", "gemm.hip", "gemm_rows.hip", "gemm_wgrad.hip", "gemm_few.hip", "probe.hip"]  # compiled with -DAAMD_TUNING
 LIB = os.path.join(HERE, "libatorch_amd_fp8.so")
 HOST = os.path.join(os.path.dirname(HERE), "_host.so")
 PROBES_LIB = os.path.join(HERE, "libatorch_amd_probes.so")

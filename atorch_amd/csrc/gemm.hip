@@ -1130,6 +1130,30 @@ static bool use_short_runs(const GemmParams& p) {
          (int64_t)p.E * p.nLt * p.nRt < (1 << 27);
 }
 
+// Weight gradient on 256 x 256 tiles (wgrad_tiles_kernel)?  Its workgroups take their tiles in a fixed order, a round of 256 after the
+// other, so a group's tiles have to fill their rounds nearly (the length of a round is its group's, known on the device only),
+// and so have all of them.  Measured on MI355X, bf16, us, 128 x 128 tiles -> these:
+//   32768 rows in 8 groups (33 blocks each), 28672 x 4096 4495 -> 4119, Zipf 4540 -> 4183; 4096 x 14336 2244 -> 2095, Zipf 2236 -> 2169
+//   16384 rows in 16 groups (8), 4096 x 4096 436 -> 374, Zipf 426 -> 397; 12288 (6) 399 -> 319, Zipf 316 -> 331
+//   8192 rows in 8 groups (8), 28672 x 4096 1624 -> 1301; 3584 x 8192 397 -> 334; 4096 x 14336, Zipf 739 -> 673
+//   4096 rows in 8 groups (4), 28672 x 4096 970 -> 840, Zipf 871 -> 878; 4096 x 4096 148 -> 120, Zipf 133 -> 128; 2048 (2) 589 -> 631
+//   rounds that are not filled: 131072 rows in 60 groups (Zipf), 2816 x 2048 (88 tiles a group) 1037 -> 1425; one group of 16384,
+//   14336 x 4096 (3.5 rounds) 996 -> 1113
+// fp32, whose stores are twice as long and come at once: 32768 rows in 8 groups, 28672 x 4096 4569 -> 4397, 16384, 14336 x 4096
+// 1355 -> 1296, 32768, 4096 x 4096 658 -> 645, 16384 in 16 groups 447 -> 464.
+static bool use_large_wgrad(const GemmParams& p, int c_dtype, const GemmOptions& g_opt) {
+  const bool can = p.E <= 64 && !p.accumulate && p.Lrows < (1 << 23) && p.Rrows < (1 << 23);
+  if (g_opt.tile >= 0) return can && g_opt.tile == 1;
+  if (!can) return false;
+  const int64_t blocks = p.goff != nullptr ? p.max_kb - p.E : p.max_kb;  // (the operands are padded to whole blocks per group)
+  const int64_t tiles = ((p.Lrows + kLargeTile - 1) / kLargeTile) * ((p.Rrows + kLargeTile - 1) / kLargeTile), per_x = (tiles + 7) / 8;
+  const int64_t group_rounds = (per_x + 31) / 32, rounds = (p.E * per_x + 31) / 32;
+  const double full = (double)p.Lrows * (double)p.Rrows / (256.0 * kLargeTile * kLargeTile);  // rounds a group would fill
+  if ((double)group_rounds > 1.15 * full || (double)rounds > 1.05 * p.E * full) return false;
+  if (c_dtype == AAMD_F32) return blocks >= 16LL * p.E && rounds >= 24;
+  return blocks >= 8LL * p.E || (p.E <= 8 && blocks >= 4LL * p.E);
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace aamd
@@ -1274,14 +1298,15 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   p.C = dw; p.ldc = K; p.c_group_stride = expert_stride;
   p.bias = nullptr; p.bias_dtype = AAMD_NONE; p.bias_group_stride = 0;
   p.goff = group_offsets;
-  // per-row scales on both operands: the 128x128 configuration measured faster for wgrad
-  // (measurement build: tile 1 = 256 x 128)
-  const int cfg = g_opt.tile > 0 ? 1 : 0;
-  const int BM = cfg ? CfgWgrad::BM : CfgSmall::BM;
-  const int BN = cfg ? CfgWgrad::BN : CfgSmall::BN;
-  p.Lrows = N; p.Rrows = K; p.nkb = 0; p.E = E; p.nRt = (int)((K + BN - 1) / BN); p.nLt = (int)((N + BM - 1) / BM);
+  p.Lrows = N; p.Rrows = K; p.nkb = 0; p.E = E;
   p.max_kb = (int)(ld_t / kBK);
   p.accumulate = accumulate;
+  if (use_large_wgrad(p, dw_dtype, g_opt)) {
+    p.nLt = (int)((N + kLargeTile - 1) / kLargeTile); p.nRt = (int)((K + kLargeTile - 1) / kLargeTile);
+    tile_order<kRaggedK>(p, kLargeTile, g_opt);
+    return launch_wgrad_tiles(p, dw_dtype, st);
+  }
+  p.nLt = (int)(N / kTile); p.nRt = (int)(K / kTile);
   const int64_t per_g = (int64_t)p.nLt * p.nRt, per_x = (per_g + 7) / 8;  // every XCD takes an eighth of a group
   int64_t blocks = (int64_t)E * per_x * 8;
   if (g_opt.tile < 0 && use_short_runs(p)) {
@@ -1291,9 +1316,6 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
     const int64_t longs = std::min<int64_t>(E, p.max_kb / (p.short_kb + 1));
     blocks = (longs * per_x + (E * per_g + 8 * p.run - 1) / (8 * p.run)) * 8;
   }
-#ifdef AAMD_TUNING
-  if (cfg == 1) return launch_gemm<kRaggedK, true, CfgWgrad>(p, dw_dtype, blocks, st, g_opt);
-#endif
   return launch_gemm<kRaggedK, true, CfgSmall>(p, dw_dtype, blocks, st, g_opt);
 }
 

@@ -80,5 +80,7 @@ constexpr int64_t kRowPartsBytes = (int64_t)256 * kLargeTile * kLargeTile * 4;  
 // Row-ragged GEMM with block-scaled R on 256 x 256 tiles (gemm_rows.hip): at least eight contraction blocks, p.ls_batch 1 where
 // rows of scales are 16-byte aligned; `tiles`: no fewer than there are.
 int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st);
+// Weight gradient on 256 x 256 tiles (gemm_wgrad.hip): at most 64 groups, written and not added to.
+int launch_wgrad_tiles(const GemmParams& p, int c_dtype, hipStream_t st);
 
 }  // namespace aamd

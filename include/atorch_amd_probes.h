@@ -23,7 +23,7 @@ const char *aamd_probes_last_error(void);
  * The grouped GEMMs of the product library (same kernels, same arguments as aamd_grouped_gemm_fp8_nt, _nn and
  * aamd_grouped_gemm_fp8_wgrad) with the launch choices the library otherwise makes by itself pinned for
  * this one call: opts = {tile, group_r, gl, ls_batch}, each -1 for the library's own choice.
- *   tile: 0 = 128x128 tiles, 1 = the large configuration (wgrad: 256x128 tiles), 2 / 3 = the kernel for few rows and its split form;
+ *   tile: 0 = 128x128 tiles, 1 = the large configuration (wgrad: 256x256 tiles), 2 / 3 = the kernel for few rows and its split form;
  *   group_r: the tile order groups R tiles (1) or L tiles (0); gl: tiles sharing a panel in the tile order;
  *   ls_batch: 0 = scales fetched one contraction block at a time (which the 128x128 tiles do: the large
  *   configuration of the block-scaled GEMM takes its scales in batches only and is then not chosen).
