@@ -62,6 +62,11 @@ SIGNATURES = {
         _int,
         [_vp, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int, _i64, _vp, _int, _vp],
     ),
+    "aamd_quant_grouped_gemm_fits": (_int, [_i64, _i64, _i64, _int, _i64]),
+    "aamd_quant_grouped_gemm_fp8_nt": (
+        _int,
+        [_int, _vp, _i64, _vp, _int, _i64, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _int, _vp],
+    ),
     "aamd_grouped_gemm_fp8_ws_bytes": (_i64, [_i64, _i64, _i64, _int, _int, _int]),
     "aamd_grouped_gemm_fp8_ws": (
         _int,

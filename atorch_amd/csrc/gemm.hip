@@ -1250,6 +1250,49 @@ extern "C" int aamd_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const flo
   return gemm_nt_impl(a, lda, a_s, b, b_s, 0, true, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype, stream);
 }
 
+constexpr int64_t kQuantisingRows = 64;
+static NtKernel quantising_kernel(int64_t M, int64_t N, int64_t K, int E) {
+  if (M < 1 || M > kQuantisingRows || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || K >= (1LL << 23)) return kSmallTiles;
+  return choose_nt(M, N, K / kBK, E, true, false, false, GemmOptions());
+}
+// Worth it?  It saves a launch of 3 to 4 us and puts a tenth of a microsecond into every step of every round of workgroups, four
+// rows of a group at a time; from the ninth row on the rows of a step are fetched when their turn comes.  A block of experts,
+// SwiGLU, us, with both of its quantisers as launches -> in the GEMMs (E, H, F, k; T tokens): 60, 2048, 1408, 4: T 1 30.1 -> 22.3,
+// 2 31.0 -> 24.9, 4 39.5 -> 34.0, 8 50.7 -> 47.8; 64, 7168, 2048, 8: T 1 85.4 -> 79.7, 4 230 -> 226; 8, 4096, 14336, 2 (long
+// streams: 40 and more steps): T 1 75.8 -> 72.0, 4 219 -> 225, 8 242 -> 251, 16 247 -> 316; one group of 32 rows, 1024 x 4096
+// 28.7 -> 49.2.
+extern "C" int aamd_quant_grouped_gemm_fits(int64_t M, int64_t N, int64_t K, int E, int64_t most) {
+  const NtKernel kernel = quantising_kernel(M, N, K, E);
+  if (kernel != kFewRows && kernel != kFewRowsSplit) return 0;
+  const int64_t groups = M < E ? M : E, nkb = K / kBK;
+  const int waves = kernel == kFewRows ? 4 : 8, rows = kernel == kFewRows ? 64 : 32;
+  const double rounds = std::max(1.0, (double)(groups * (N / rows)) / 512.0);
+  return most <= 8 && rounds * (double)((nkb + waves - 1) / waves) <= 24.0;
+}
+extern "C" int aamd_quant_grouped_gemm_fp8_nt(int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
+                                              const uint8_t* b, const float* b_s, const int64_t* group_offsets, int E, int64_t M,
+                                              int64_t N, int64_t K, void* c, int64_t ldc, const void* bias, int bias_dtype,
+                                              void* stream) {
+  AAMD_REQUIRE(what >= AAMD_ROWS_PERMUTED && what <= AAMD_ROWS_GELU, "quant_grouped_gemm_nt: unknown source %d", what);
+  const NtKernel kernel = quantising_kernel(M, N, K, E);
+  AAMD_REQUIRE(kernel == kFewRows || kernel == kFewRowsSplit, "quant_grouped_gemm_nt: not for M=%lld, N=%lld, K=%lld in %d groups", (long long)M,
+               (long long)N, (long long)K, E);
+  AAMD_REQUIRE(bias == nullptr || bias_dtype == AAMD_BF16 || bias_dtype == AAMD_F32, "quant_grouped_gemm_nt: bad bias dtype");
+  AAMD_REQUIRE(rows && b && b_s && c && group_offsets && (what != AAMD_ROWS_PERMUTED || (sorted_idx && topk >= 1 && T >= 1 && T < (1LL << 31))),
+               "quant_grouped_gemm_nt: null pointer or bad routing");
+  AAMD_REQUIRE(ld >= (what == AAMD_ROWS_SWIGLU ? 2 * K : K) && ld % 8 == 0 && aligned16(rows) && aligned16(b), "quant_grouped_gemm_nt: operands must be 16-byte aligned");
+  AAMD_REQUIRE(ldc >= N && ldc % 8 == 0 && aligned16(c), "quant_grouped_gemm_nt: output rows must be 16-byte aligned");
+  GemmParams p = {};
+  p.r_kb_stride = kBK;
+  p.R = b; p.ldr = K; p.r_group_stride = N * K;
+  p.Rs = b_s; p.rs_row_stride = K / kBK; p.rs_blk_stride = 1; p.rs_group_stride = (N / kTile) * (K / kBK);
+  p.C = c; p.ldc = ldc;
+  p.bias = bias; p.bias_dtype = bias_dtype; p.bias_group_stride = N;
+  p.goff = group_offsets;
+  p.Lrows = M; p.Rrows = N; p.nkb = (int)(K / kBK); p.E = E;
+  return launch_few_rows_quantising(p, what, rows, ld, sorted_idx, topk, T, M, kernel == kFewRowsSplit, (hipStream_t)stream);
+}
+
 extern "C" int64_t aamd_grouped_gemm_fp8_ws_bytes(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows) {
   const int64_t nkb = K / kBK;
   if (M <= 0 || N <= 0 || E < 1 || nkb < kSplitBlocks) return 0;

@@ -75,6 +75,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // Row-ragged GEMM with block-scaled R for groups of few rows (gemm_few.hip); reads L, R, their scales and strides, C,
 // bias, goff, E, Lrows, Rrows and nkb of the parameters.  r_rows: R is stored [contraction, Rrows] (R_ROWS of gemm.hip).
 int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st);
+// The same from bf16 rows, see aamd_quant_grouped_gemm_fp8_nt.
+int launch_few_rows_quantising(const GemmParams& p, int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
+                               int64_t M, bool split, hipStream_t st);
 
 constexpr int64_t kRowPartsBytes = (int64_t)256 * kLargeTile * kLargeTile * 4;  // a tile of fp32 for each of 256 workgroups
 // Row-ragged GEMM with block-scaled R on 256 x 256 tiles (gemm_rows.hip): at least eight contraction blocks, p.ls_batch 1 where

@@ -17,8 +17,19 @@
 //   one group of 1 / 144 rows, 896 x 6016                    41 -> 9  (split form)
 // From about 64 rows per group the operand reuse of the larger tiles wins.
 #include "gemm.hpp"
+#include "quant.hpp"
 
 namespace aamd {
+
+// Token rows that come as bf16 and are quantised by the waves that multiply them: read through a routing (BF16: row j is row
+// sorted_idx[j] / topk of `rows`), or the activation of the rows as they are (GLU, GELU).
+struct FewSource {
+  const u16* rows;
+  int64_t ld, gate_off;        // elements
+  const int64_t* sorted_idx;
+  uint32_t topk, T;
+};
+struct Codes {};  // the token rows are codes
 
 // W waves, tiles of 32 WTR weight rows x 32 WTL token rows.  R_ROWS: the weights are stored [contraction, Rrows] and read
 // transposed from the LDS, as in gemm.hip; a block of them is 128 rows of BR bytes there.  That form takes whole cache lines
@@ -26,11 +37,17 @@ namespace aamd {
 // four, and the other orientation: 64 groups of 6 rows, 7168 x 2048 197, 260, 166, 167, 159; 4096 x 7168 350, 474, 324, 326,
 // 307; 64 uneven groups of 128, 2048 x 7168 324, 817, 254, 253, 284), its scales in registers so that two workgroups of
 // 80 KB fit a CU.
-template <typename OUT, int W, int WTR, int WTL, bool R_ROWS>
-__global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
+//
+// IN: what the token rows are.  A launch of a few rows is as long as its latencies, and quantising the rows ahead of it is another
+// one; here every wave quantises the 128-wide blocks of its own steps, four rows at a time, into its stage while its weights are on
+// their way (one token, four of 60 experts, 2048 wide: quantiser 3.4 + GEMM 7.0 us, activation 2.6 + GEMM 6.0).  The arithmetic is
+// that of quant_1x128_kernel: the same codes.
+template <typename OUT, int W, int WTR, int WTL, bool R_ROWS, typename IN = Codes>
+__global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, const FewSource src) {
+  constexpr bool kQuantise = !std::is_same<IN, Codes>::value;
   constexpr int BL = 32 * WTL, BR = 32 * WTR;
   constexpr int kPitch = BR + 4;  // floats per row of a wave's partial result in the LDS
-  constexpr int kStage = (BR + BL) * kBK + (WTL == 1 ? 0 : BL * 4 + 256);  // weight rows, token rows, scales
+  constexpr int kStage = (BR + BL) * kBK + (WTL == 1 && !kQuantise ? 0 : BL * 4 + 256);  // weight rows, token rows, scales
   constexpr int PL = WTR > 2 ? 32 : BL;  // token rows whose partial results are in the LDS at a time
   constexpr int kLds = W * (kStage > PL * kPitch * 4 ? kStage : PL * kPitch * 4);
   __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
@@ -123,12 +140,41 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
     sbase[n] = p.Ls + (l0 + (row < lvalid ? row : lvalid - 1)) * p.ls_row_stride;
   }
   float ls_next = 0.f, rs_next = 0.f;  // (WTL == 1)
+  // (kQuantise) the first eight rows are requested with the weights; 16 lanes per row
+  constexpr int kAhead = 2;
+  typedef typename std::conditional<kQuantise, IN, BF16>::type Elem;
+  Raw8<Elem> raw[kAhead];
+  const int q4 = lane >> 4, q16 = lane & 15;
+  auto raw_row = [&](int r) __attribute__((always_inline)) {  // clamped to the rows there are
+    const int64_t row = l0 + (r < lvalid ? r : lvalid - 1);
+    if constexpr (std::is_same<IN, BF16>::value) {
+      const uint32_t token = (uint32_t)src.sorted_idx[row] / src.topk;
+      return src.rows + (int64_t)(token < src.T ? token : src.T - 1) * src.ld;
+    } else {
+      return src.rows + row * src.ld;
+    }
+  };
+  auto request = [&](Raw8<Elem>& to, const u16* row, int k) __attribute__((always_inline)) {
+    const u16* const from = row + k * kTile + q16 * 8;
+    to.a = *reinterpret_cast<const v4i*>(from);
+    if constexpr (std::is_same<IN, GLU>::value) to.b = *reinterpret_cast<const v4i*>(from + src.gate_off);
+  };
+  const u16* raw_at[kAhead] = {};
+  if constexpr (kQuantise) {
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) raw_at[u] = raw_row(4 * u + q4);
+  }
   constexpr int kScales = (BR + BL) * kBK;  // offset in the stage
   const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)mine;
   auto load = [&](int k) __attribute__((always_inline)) {
     const uint8_t* const R = Rb + k * p.r_kb_stride;
     const uint8_t* const L = Lb + (int64_t)k * kBK;
-    if constexpr (WTL == 1) {
+    if constexpr (kQuantise) {
+#pragma unroll
+      for (int u = 0; u < kAhead; u++)
+        if (u == 0 || 4 * u < lvalid) request(raw[u], raw_at[u], k);
+      rs_next = rs[k * p.rs_blk_stride];
+    } else if constexpr (WTL == 1) {
       ls_next = sbase[0][k];
       rs_next = rs[k * p.rs_blk_stride];
     }
@@ -136,10 +182,10 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
     for (int n = 0; n < BR / 8; n++)
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(R_ROWS ? roff_t : roff[n & 1]), "s"(R + (int64_t)(n * (R_ROWS ? kRowsPer1K : 8)) * p.ldr), "s"(base + n * 1024) : "memory");
 #pragma unroll
-    for (int n = 0; n < 4 * WTL; n++)
+    for (int n = 0; n < (kQuantise ? 0 : 4 * WTL); n++)
       if (n < nl)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(loff[n]), "s"(L), "s"(base + BR * kBK + n * 1024) : "memory");
-    if constexpr (WTL > 1) {
+    if constexpr (WTL > 1 && !kQuantise) {
 #pragma unroll
       for (int n = 0; n < (WTL + 1) / 2; n++)
         asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(sbase[n] + k), "s"(base + kScales + n * 256) : "memory");
@@ -157,6 +203,29 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
   if (wave < nkb) load(wave);
   for (int kb = wave; kb < nkb; kb += W) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the block has landed
+    const float rs_now = rs_next;
+    if constexpr (kQuantise) {
+      auto quantise = [&](const Raw8<Elem>& from, int row) __attribute__((always_inline)) {
+        float v[8];
+        from.get(v);
+        const Divider d = make_scale(row16_max(amax8(v)), 0.f, false);
+        const v2i codes = quant8<false>(v, d);
+        if (row < lvalid) {
+          uint8_t* const to = mine + (BR + row) * kBK + (((q16 >> 1) ^ ((row & 7) ^ ((row >> 3) & 1))) << 4) + (q16 & 1) * 8;
+          *reinterpret_cast<v2i*>(to) = codes;
+          if (q16 == 0) *reinterpret_cast<float*>(mine + kScales + row * 4) = d.s;
+        }
+      };
+#pragma unroll
+      for (int u = 0; u < kAhead; u++)
+        if (u == 0 || 4 * u < lvalid) quantise(raw[u], 4 * u + q4);
+      for (int r = 4 * kAhead; r < lvalid; r += 4) {
+        Raw8<Elem> more;
+        request(more, raw_row(r + q4), kb);
+        quantise(more, r + q4);
+      }
+      __builtin_amdgcn_wave_barrier();  // same wave, in-order LDS: the reads below see the writes above
+    }
     v8i rf[WTR][2], lf[WTL][2];
     float sc[WTL];
     auto frag = [&](const uint8_t* row, int h) {
@@ -185,7 +254,7 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p) {
       }
     }
 #pragma unroll
-    for (int j = 0; j < WTL; j++) sc[j] = WTL == 1 ? ls_next * rs_next : S[j * 32 + l32] * S[BL];
+    for (int j = 0; j < WTL; j++) sc[j] = kQuantise ? S[j * 32 + l32] * rs_now : WTL == 1 ? ls_next * rs_next : S[j * 32 + l32] * S[BL];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and has been read: its place may be filled again
     if (kb + W < nkb) load(kb + W);
 #pragma unroll
@@ -247,13 +316,13 @@ static int64_t few_rows_tiles(int64_t M, int E, int rows) {
   return M / rows + groups < M ? M / rows + groups : M;
 }
 
-template <typename OUT, int W, int WTR, int WTL, bool R_ROWS>
-static int launch_few(GemmParams p, int64_t M, hipStream_t st) {
+template <typename OUT, int W, int WTR, int WTL, bool R_ROWS, typename IN = Codes>
+static int launch_few(GemmParams p, int64_t M, hipStream_t st, const FewSource& src = FewSource()) {
   p.nRt = (int)(p.Rrows / (32 * WTR));
   const int64_t lt = p.goff ? few_rows_tiles(M, p.E, 32 * WTL) : (M + 32 * WTL - 1) / (32 * WTL);
   const int64_t blocks = lt * p.nRt;
   AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
-  few_rows_kernel<OUT, W, WTR, WTL, R_ROWS><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p);
+  few_rows_kernel<OUT, W, WTR, WTL, R_ROWS, IN><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p, src);
   AAMD_LAUNCH_CHECK("grouped_gemm (few rows)");
   return AAMD_OK;
 }
@@ -267,6 +336,14 @@ static int launch_few_as(const GemmParams& p, int64_t M, bool split, bool r_rows
 }
 int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st) {
   return c_dtype == AAMD_BF16 ? launch_few_as<u16>(p, M, split, r_rows, st) : launch_few_as<float>(p, M, split, r_rows, st);
+}
+
+int launch_few_rows_quantising(const GemmParams& p, int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
+                               int64_t M, bool split, hipStream_t st) {
+  const FewSource src = {(const u16*)rows, ld, (int64_t)p.nkb * kTile, sorted_idx, (uint32_t)topk, (uint32_t)T};
+  if (what == AAMD_ROWS_PERMUTED) return split ? launch_few<u16, 8, 1, 1, false, BF16>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, BF16>(p, M, st, src);
+  if (what == AAMD_ROWS_SWIGLU) return split ? launch_few<u16, 8, 1, 1, false, GLU>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, GLU>(p, M, st, src);
+  return split ? launch_few<u16, 8, 1, 1, false, GELU>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, GELU>(p, M, st, src);
 }
 
 }  // namespace aamd

@@ -508,10 +508,23 @@ void check_mlp(const Tensor& x, const Tensor& q1, const Tensor& q2, const OptTen
   if (b1.has_value()) check_bias(*b1, E, n1);
   if (b2.has_value()) check_bias(*b2, E, q2.size(1));
 }
+// Quantiser and GEMM in one launch: the output, or nothing where the sizes or operands are not for it (most: rows a group can have).
+OptTensor quant_gemm(int what, const Tensor& rows, const OptTensor& sorted_idx, int64_t topk, int64_t M, int64_t most, const Tensor& q,
+                     const Tensor& s, const Tensor& goff, const OptTensor& bias) {
+  const int64_t E = q.size(0), N = q.size(1), K = q.size(2);
+  if (rows.scalar_type() != at::kBFloat16 || !rows.is_contiguous() || !q.is_contiguous() || !s.is_contiguous() || s.dim() != 3 ||
+      s.size(1) != N / kTile || !aamd_quant_grouped_gemm_fits(M, N, K, (int)E, most))
+    return {};
+  Tensor c = empty({M, N}, at::kBFloat16, rows);
+  check(aamd_quant_grouped_gemm_fp8_nt(what, ptr(rows), rows.size(1), ptr<int64_t>(sorted_idx), (int)topk, rows.size(0), ptr<uint8_t>(q),
+                                       ptr<float>(s), ptr<int64_t>(goff), (int)E, M, N, K, ptr(c), N, ptr(bias),
+                                       bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
+  return c;
+}
 using MlpResult = std::tuple<Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
-MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
-                      const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
-                      const OptTensor& b2, bool glu, bool train) {
+MlpResult mlp_rows(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
+                   const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
+                   const OptTensor& b2, bool glu, bool train, bool own_routing) {
   const int64_t E = q1.size(0);
   check_mlp(x, q1, q2, b1, b2, glu);
   check_offsets(goff, E);
@@ -524,22 +537,37 @@ MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sort
   const int64_t M = row_map.has_value() ? sorted_idx->numel() : x.size(0);  // (fewer than the map's entries where copies were dropped)
   Quantised qx;
   const int64_t ld_t = padded_bound(M, E);
-  if (train)
+  const int64_t most = own_routing ? std::min(M, x.size(0)) : M;  // (a token goes to an expert once)
+  OptTensor fused;
+  // (the indices of a routing made here name a row for every row of a group)
+  if (!train && own_routing) fused = quant_gemm(AAMD_ROWS_PERMUTED, x, sorted_idx, topk, M, most, q1, s1, goff, b1);
+  if (fused.has_value())
+    ;
+  else if (train)
     qx = row_map.has_value() ? permute_dual(x, *sorted_idx, topk, goff, E, 0.0, ld_t, true, true)
                              : dual(x, goff, E, 0.0, ld_t, true, true);
   else
     std::tie(qx.q, qx.s) = row_map.has_value() ? permute_tile_quant(x, *row_map, topk, M, 0.0) : tile_quant(x, 0.0);
-  Tensor fc1 = gemm_nt(qx.q, qx.s, q1, s1, goff, {}, at::kBFloat16, b1);
+  Tensor fc1 = fused.has_value() ? *fused : gemm_nt(qx.q, qx.s, q1, s1, goff, {}, at::kBFloat16, b1);
   Quantised qh;
   if (train) {
     qh = std::get<0>(act_dual(fc1, Tensor(), glu, goff, E, ld_t, true, true, false));
   } else {
+    if (x.scalar_type() == at::kBFloat16)
+      if (OptTensor out = quant_gemm(glu ? AAMD_ROWS_SWIGLU : AAMD_ROWS_GELU, fc1, {}, 0, M, most, q2, s2, goff, b2); out.has_value())
+        return {*out, {}, {}, {}, {}, {}};
     OptTensor none;
     std::tie(qh.q, qh.s, none) = act_quant(fc1, glu, false);
   }
   Tensor out = gemm_nt(qh.q, qh.s, q2, s2, goff, {}, x.scalar_type(), b2);
   if (!train) return {out, {}, {}, {}, {}, {}};
   return {out, fc1, qx.q_t, qx.s_t, qh.q_t, qh.s_t};
+}
+
+MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
+                      const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
+                      const OptTensor& b2, bool glu, bool train) {
+  return mlp_rows(x, goff, sorted_idx, row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, false);
 }
 
 // The same from the router's choices, routing and weighted combine included: (out, sorted_idx, row_map, goff) and, with
@@ -551,7 +579,7 @@ py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids,
               probs.is_contiguous() && q2.size(1) == x.size(1),
           "router weights and choices are [tokens, topk], and the experts return the hidden size");
   Routing r = route(ids, q1.size(0), true);
-  MlpResult m = mlp_forward(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train);
+  MlpResult m = mlp_rows(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, true);
   Tensor& y = std::get<0>(m);
   Tensor out = unpermute_combine(y, r.row_map, probs, x.size(0), topk);
   if (!train) return py::make_tuple(out, r.sorted_idx, r.row_map, r.goff);

@@ -257,6 +257,27 @@ int aamd_grouped_gemm_fp8_ws(const uint8_t *a, int64_t lda, const float *a_s, co
                              void *stream);
 
 /*
+ * Quantise and multiply in one launch, for the few rows of a decoding step: C = Q(rows) B_g^T (+ bias_g), where Q is the 1x128
+ * quantiser's result (its codes and scales, which are not written) of
+ *   AAMD_ROWS_PERMUTED  row j of the groups is row sorted_idx[j] / topk of `rows` [T, K] bf16, row stride ld elements
+ *   AAMD_ROWS_SWIGLU    SwiGLU of `rows` [M, 2 K] bf16 (as aamd_swiglu_quant_1x128)
+ *   AAMD_ROWS_GELU      GELU of `rows` [M, K] bf16 (as aamd_gelu_quant_1x128)
+ * c [M, N] bf16.  It takes up to 64 rows where the GEMM of codes would use its kernel for few rows; other sizes are
+ * AAMD_ERR_ARG.  _fits() says whether it does and is faster than the two launches, `most` being the most rows a group can have.
+ * The results are those of the two launches, bit for bit.
+ * Replaces tile_quant + grouped_qgemm, quantized_grouped_linear.py:90-101, 141-151 (and the permute in front of them,
+ * token_dispatcher.py:89-116).
+ */
+#define AAMD_ROWS_PERMUTED 0
+#define AAMD_ROWS_SWIGLU 1
+#define AAMD_ROWS_GELU 2
+int aamd_quant_grouped_gemm_fits(int64_t M, int64_t N, int64_t K, int E, int64_t most);
+int aamd_quant_grouped_gemm_fp8_nt(int what, const void *rows, int64_t ld, const int64_t *sorted_idx, int topk, int64_t T,
+                                   const uint8_t *b, const float *b_s, const int64_t *group_offsets, int E, int64_t M,
+                                   int64_t N, int64_t K, void *c, int64_t ldc, const void *bias, int bias_dtype,
+                                   void *stream);
+
+/*
  * aamd_grouped_gemm_fp8_nt for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): the same arguments without
  * tile_ws.  No counterpart in the reference.  The call allocates and
