@@ -1099,9 +1099,12 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   // blocks the split form is the faster one at any length (128 blocks, 16 steps 7.8 and 5.8 (5.3), 28 steps 12.7 and 8.6
   // (6.5); 176, 16: 7.8 and 6.9 (5.5); 256, 16: 10.4 and 9.6 (7.0)), from 512 on it is not (8 steps 10.2 and 10.5 (8.0), 16
   // steps 15.2 and 15.9 (11.7), 28 steps 23.4 and 24.1 (18.9)) unless the weights' stream bounds both (1024, 56: 79 and 76).
-  // Its estimate is 1 to 5 us too low in between, so that without a line it would be taken at 512 blocks too; the line at 128
-  // gives up what it gains between 128 and 256 blocks on short contractions, up to 2 us a launch.
-  const bool may_split = !b_rows && (blocks_f < 128.0 || nkb >= 28);
+  // Its estimate is 1 to 5 us too low in between, so that without a line it would be taken at 512 blocks too; from 128 on only
+  // groups of up to 32 rows take it, one token tile of either form.  (Around the line, on weights out of the caches, 64 x 64 blocks
+  // and their split form, us: 4 groups of a row, 2816 x 2048 (176 blocks) 13.0 and 11.7, 2048 x 1408 (128) 8.6 and 7.2; 16 rows in 8
+  // groups, 1536 x 1024 (192) 7.9 and 7.4; 100 in 4, 4096 x 512 (256) 7.5 and 6.5; 500 in 8, 1024 x 1024 (189) 8.8 and 6.8, but with
+  // the weights in the caches 6.5 and 7.3; 512 in 8, 2048 x 7168 (384) 48.6 and 56.5.)
+  const bool may_split = !b_rows && (blocks_f < 128.0 || nkb >= 28 || (blocks_f <= 256.0 && M <= 32 * groups));
   const double split = may_split ? std::max({2.2 + 1e-3 * blocks_p * (0.45 * n + 2.1), 4.0 + 0.63 * std::ceil(n / 8.0), weights / 6.2}) : 1e30;
   if (std::min(few, split) <= std::min(small, large)) return split < few ? kFewRowsSplit : kFewRows;
   return large < small ? kLargeTiles : kSmallTiles;
