@@ -90,6 +90,7 @@ SIGNATURES = {
     ),
     "aamd_group_sums": (_int, [_vp, _i64, _vp, _int, _vp, _int, _vp]),
     "aamd_transpose_scales": (_int, [_vp, _i64, _i64, _vp, _vp]),
+    "aamd_transpose_scales_pair": (_int, [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _vp]),
     "aamd_group_offsets": (_int, [_vp, _int, _int, _vp, _vp]),
     "aamd_moe_preprocess_ws_ints": (_i64, [_i64, _int]),
     "aamd_moe_preprocess": (_int, [_vp, _int, _i64, _int, _vp, _vp, _vp, _vp, _vp]),

@@ -132,6 +132,17 @@ Quantised dual(const Tensor& x, const OptTensor& goff, int64_t E, double eps, in
   return r;
 }
 
+// Rows [M, cols] of one group with both transposed results row-major, q_t [cols, ld_t] and s_t [cols, ld_t / 128].
+QuantTuple dual_rows(const Tensor& x, double eps) {
+  const int64_t M = x.size(0), cols = x.size(1), ld_t = (M + kTile - 1) / kTile * kTile;
+  Quantised r = alloc_dual(M, cols, ld_t, true, false, x);
+  r.s_t = r.s_t.view({cols, ld_t / kTile});
+  check(aamd_quant_1x128_dual_grouped(ptr(x), dtype_code(x.scalar_type(), true), M, cols, cols, nullptr, 1, nullptr, ptr<uint8_t>(r.q),
+                                      ptr<float>(r.s), ptr<uint8_t>(r.q_t), ptr<float>(r.s_t), ld_t, AAMD_QT_ROWS_SCALES, (float)eps,
+                                      stream()));
+  return {r.q, r.s, r.q_t, r.s_t};
+}
+
 Quantised permute_dual(const Tensor& x, const Tensor& sorted_idx, int64_t topk, const Tensor& goff, int64_t E, double eps,
                        int64_t ld_t, bool rowwise, bool blocked) {
   const int64_t T = x.size(0), cols = x.size(1), M = sorted_idx.numel();
@@ -272,7 +283,8 @@ Tensor fp8_gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tenso
   // 14336 x 4096 x 4096 327 -> 280, x 1024 117 -> 104, x 256 64 -> 58; 4096 x 4096 x 4096 95 -> 100; the results are equal).
   constexpr int64_t kDenseWgradTiles = 2048;  // 128 x 128 outputs
   if (b_tile_scaled && M % kTile == 0 && N % kTile == 0 && (M / kTile) * (N / kTile) >= kDenseWgradTiles) {
-    Tensor at = transpose_scales(a_s.view({M, blocks})), bt = transpose_scales(b_s);
+    Tensor at = empty({blocks, M}, at::kFloat, a), bt = empty({blocks, N}, at::kFloat, a);
+    check(aamd_transpose_scales_pair(ptr<float>(a_s), M, ptr<float>(at), ptr<float>(b_s), N, ptr<float>(bt), blocks, stream()));
     check(aamd_grouped_gemm_fp8_wgrad(ptr<uint8_t>(a), ptr<float>(at), ptr<uint8_t>(b), ptr<float>(bt), K, AAMD_QT_ROWS, nullptr,
                                       1, nullptr, M, N, ptr(c), dtype_code(dtype), M * N, 0, stream()));
     return c;
@@ -686,6 +698,7 @@ QuantTuple pack(const Quantised& r) { return {opt(r.q), opt(r.s), r.q_t, r.s_t};
 PYBIND11_MODULE(_host, m) {
   m.def("tile_quant", &tile_quant);
   m.def("permute_tile_quant", &permute_tile_quant);
+  m.def("dual_rows", &dual_rows);
   m.def("dual", [](const Tensor& x, const OptTensor& goff, int64_t E, double eps, int64_t ld_t, bool rowwise, bool blocked) {
     return pack(dual(x, goff, E, eps, ld_t, rowwise, blocked));
   });

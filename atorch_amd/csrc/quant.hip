@@ -190,8 +190,8 @@ __device__ __forceinline__ void store_staged_tile(const uint8_t* tile_t, uint8_t
 // token-block-major, so that a tile is 16 KB of consecutive bytes and the tiles of a token block follow each other:
 // the kernel then writes the transposed codes as one sequential sweep instead of 128-byte pieces ld_t apart.
 __device__ __forceinline__ uint8_t* qt_tile(uint8_t* q_t, int blocked, int64_t cols, uint32_t ld_t, int pt, int kc, uint32_t* ld) {
-  *ld = blocked ? (uint32_t)kTile : ld_t;
-  return blocked ? q_t + ((int64_t)pt * cols + (int64_t)kc * kTile) * kTile
+  *ld = blocked == AAMD_QT_BLOCKED ? (uint32_t)kTile : ld_t;
+  return blocked == AAMD_QT_BLOCKED ? q_t + ((int64_t)pt * cols + (int64_t)kc * kTile) * kTile
                  : q_t + (int64_t)kc * kTile * ld_t + (int64_t)pt * kTile;
 }
 
@@ -297,7 +297,8 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
     for (int i = 1; i < 16; i++) m = fmaxf(m, part[i][(int)threadIdx.x]);
     const Divider dv = make_scale(m, eps, plain_div);
     cdiv[((int)threadIdx.x & 7) * 16 + ((int)threadIdx.x >> 3)] = dv;  // [column % 8][column / 8]: lanes of a row read 16 neighbours
-    (s_t + (int64_t)pt * cols + (int64_t)kc * kTile)[(int)threadIdx.x] = dv.s;
+    if (blocked == AAMD_QT_ROWS_SCALES) s_t[((int64_t)kc * kTile + (int)threadIdx.x) * (int64_t)(ld_t / kTile) + pt] = dv.s;
+    else (s_t + (int64_t)pt * cols + (int64_t)kc * kTile)[(int)threadIdx.x] = dv.s;
   }
   __syncthreads();
   if constexpr (SUMS) {  // in the region of the maxima, which have been read
@@ -780,12 +781,21 @@ __global__ __launch_bounds__(256) void group_sums_kernel(const float* __restrict
   else out[(int64_t)g * cols + c] = (OUT)f32_to_bf16_bits(sum);
 }
 
-// [rows, blocks] scales to [blocks, rows], through 32 x 32 tiles in the LDS
-__global__ __launch_bounds__(256) void transpose_scales_kernel(const float* __restrict__ s, int rows, int blocks,
-                                                               float* __restrict__ s_t) {
+// [rows, blocks] scales to [blocks, rows], through 32 x 32 tiles in the LDS; two matrices one behind the other (a launch of its own
+// for either is 5.5 us of latency)
+struct ScaleMatrix {
+  const float* s;
+  float* s_t;
+  int rows;
+};
+__global__ __launch_bounds__(256) void transpose_scales_kernel(const ScaleMatrix a, const ScaleMatrix b, int blocks) {
   __shared__ float tile[32][33];
   const int c = (int)threadIdx.x & 31, r = (int)threadIdx.x >> 5;
-  const int row0 = (int)blockIdx.x * 32, blk0 = (int)blockIdx.y * 32;
+  const int tiles_a = (a.rows + 31) / 32, first = (int)blockIdx.x < tiles_a;
+  const float* __restrict__ s = first ? a.s : b.s;
+  float* __restrict__ s_t = first ? a.s_t : b.s_t;
+  const int rows = first ? a.rows : b.rows;
+  const int row0 = ((int)blockIdx.x - (first ? 0 : tiles_a)) * 32, blk0 = (int)blockIdx.y * 32;
 #pragma unroll
   for (int i = 0; i < 32; i += 8)
     if (row0 + r + i < rows && blk0 + c < blocks) tile[r + i][c] = s[(int64_t)(row0 + r + i) * blocks + blk0 + c];
@@ -933,7 +943,7 @@ static int quant_dual(const void* x, int x_dtype, int64_t M, int64_t cols, int64
                       uint8_t* q, float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout, float eps,
                       float* tile_sums, void* stream) {
   AAMD_REQUIRE(x_dtype == AAMD_BF16 || x_dtype == AAMD_F32 || x_dtype == AAMD_F16, "quant_dual: unsupported dtype %d", x_dtype);
-  AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "quant_dual: unknown q_t layout %d", q_t_layout);
+  AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED || q_t_layout == AAMD_QT_ROWS_SCALES, "quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(M >= 0 && cols >= 0 && cols % kTile == 0, "quant_dual: cols=%lld must be a multiple of 128",
                (long long)cols);
   AAMD_REQUIRE(ldx >= cols && ldx % 8 == 0 && ldx < kMaxTileLd, "quant_dual: bad ldx=%lld", (long long)ldx);
@@ -1246,8 +1256,18 @@ extern "C" int aamd_transpose_scales(const float* s, int64_t rows, int64_t block
   if (rows == 0 || blocks == 0) return AAMD_OK;
   AAMD_REQUIRE(s && s_t, "transpose_scales: null pointer");
   transpose_scales_kernel<<<dim3((unsigned)((rows + 31) / 32), (unsigned)((blocks + 31) / 32)), 256, 0, (hipStream_t)stream>>>(
-      s, (int)rows, (int)blocks, s_t);
+      ScaleMatrix{s, s_t, (int)rows}, ScaleMatrix{}, (int)blocks);
   AAMD_LAUNCH_CHECK("transpose_scales");
+  return AAMD_OK;
+}
+extern "C" int aamd_transpose_scales_pair(const float* a, int64_t rows_a, float* a_t, const float* b, int64_t rows_b, float* b_t,
+                                          int64_t blocks, void* stream) {
+  AAMD_REQUIRE(rows_a >= 1 && rows_b >= 1 && blocks >= 1 && rows_a < 0x3fffffffLL && rows_b < 0x3fffffffLL && (blocks + 31) / 32 <= 65535,
+               "transpose_scales_pair: bad sizes");
+  AAMD_REQUIRE(a && a_t && b && b_t, "transpose_scales_pair: null pointer");
+  transpose_scales_kernel<<<dim3((unsigned)((rows_a + 31) / 32 + (rows_b + 31) / 32), (unsigned)((blocks + 31) / 32)), 256, 0,
+                            (hipStream_t)stream>>>(ScaleMatrix{a, a_t, (int)rows_a}, ScaleMatrix{b, b_t, (int)rows_b}, (int)blocks);
+  AAMD_LAUNCH_CHECK("transpose_scales_pair");
   return AAMD_OK;
 }
 

@@ -48,7 +48,11 @@ def quantize_vector_blockwise(x, dtype=torch.float8_e4m3fn, block_size=TILE, ret
         q, s = kernels.tile_quant(x, eps=eps)
         return q, s, None, None
     x2 = x.view(-1, x.size(-1))
-    q, s, q_t, s_t = kernels.tile_quant(x2, eps=eps, return_transpose=True)
+    if x2.shape[0] == 0 or x2.shape[1] % TILE:
+        q, s, q_t, s_t = kernels.tile_quant(x2, eps=eps, return_transpose=True)
+    else:  # both transposed results come row-major
+        q, s, q_t, s_t = kernels.host().dual_rows(x2, eps)
+        q_t = q_t[:, : x2.shape[0]]
     return q.view(x.shape), s.view(*x.shape[:-1], -1), q_t.contiguous(), s_t.contiguous()
 
 

@@ -43,11 +43,13 @@ extern "C" {
 /* Layouts of the transposed 1x128 codes q_t of R rows (columns of the quantised tensor) and ld_t padded tokens:
  *   AAMD_QT_ROWS     q_t [R, ld_t]: one row of ld_t bytes per column of x;
  *   AAMD_QT_BLOCKED  q_t [ld_t / 128, R, 128]: token-block-major, byte (r, t) at ((t / 128) * R + r) * 128 + t % 128.
+ *   AAMD_QT_ROWS_SCALES  as AAMD_QT_ROWS with the scales row-major too, s_t [R, ld_t / 128] (aamd_quant_1x128_dual_grouped only).
  * The second is what the grouped kernels use among themselves: a 128 x 128 tile of codes is 16 KB of consecutive
  * bytes, which the quantisers write as one sequential sweep and the weight-gradient GEMM loads as whole slabs.
  * The scales s_t [ld_t / 128, R] are the same in both. */
 #define AAMD_QT_ROWS 0
 #define AAMD_QT_BLOCKED 1
+#define AAMD_QT_ROWS_SCALES 2
 
 #define AAMD_ABI_VERSION 4
 
@@ -366,6 +368,9 @@ int aamd_group_sums(const float *tile_sums, int64_t cols, const int64_t *group_o
  * [blocks, rows] that the weight-gradient GEMM reads.
  */
 int aamd_transpose_scales(const float *s, int64_t rows, int64_t blocks, float *s_t, void *stream);
+/* Two of them, with as many blocks, in one launch (triton_kernel.py:198-210 as above); no size is zero. */
+int aamd_transpose_scales_pair(const float *a, int64_t rows_a, float *a_t, const float *b, int64_t rows_b, float *b_t,
+                               int64_t blocks, void *stream);
 
 /*
  * Both gradients of the combine in one pass: drows[row_map[t*topk+j]] = dout[t] * probs[t, j] rounded to the rows'

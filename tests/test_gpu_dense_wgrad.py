@@ -30,3 +30,26 @@ def test_transpose_of_the_scales(dev, rows, blocks):
 
     s = torch.randn(rows, blocks, device=dev)
     assert torch.equal(kernels.host().transpose_scales(s), s.t().contiguous())
+
+
+@pytest.mark.parametrize("M,K", [(1, 128), (127, 256), (128, 1152), (300, 2048)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_transposed_scales_written_row_major(dev, M, K, dtype):
+    """The operator's transposed codes and scales, contiguous, against the quantiser that writes the scales block by block."""
+    from atorch_amd import kernels, ops
+
+    x = randn_bf16((M, K), 3).to(dev).to(dtype)
+    q, s, q_t, s_t = kernels.tile_quant(x, return_transpose=True)
+    got = ops.quantize_vector_blockwise(x, return_transpose=True)
+    for a, b in zip(got, (q, s, q_t, s_t)):
+        assert a.shape == b.shape and a.is_contiguous() and torch.equal(a.float(), b.float())
+
+
+@pytest.mark.parametrize("rows,other,blocks", [(1, 33, 1), (64, 32, 40), (129, 31, 7)])
+def test_two_transposes_in_one_launch(dev, rows, other, blocks):
+    from atorch_amd import _lib
+
+    a, b = torch.randn(rows, blocks, device=dev), torch.randn(other, blocks, device=dev)
+    at, bt = torch.empty(blocks, rows, device=dev), torch.empty(blocks, other, device=dev)
+    _lib.check(_lib.lib().aamd_transpose_scales_pair(a.data_ptr(), rows, at.data_ptr(), b.data_ptr(), other, bt.data_ptr(), blocks, _lib.stream()))
+    assert torch.equal(at, a.t()) and torch.equal(bt, b.t())
