@@ -89,6 +89,7 @@ SIGNATURES = {
         [_int, _vp, _vp, _i64, _i64, _vp, _int, _vp, _vp, _vp, _vp, _i64, _int, _f32, _vp, _vp],
     ),
     "aamd_group_sums": (_int, [_vp, _i64, _vp, _int, _vp, _int, _vp]),
+    "aamd_quant_1x128_with_offsets": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _int, _vp, _vp, _vp, _f32, _vp]),
     "aamd_transpose_scales": (_int, [_vp, _i64, _i64, _vp, _vp]),
     "aamd_transpose_scales_pair": (_int, [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _vp]),
     "aamd_group_offsets": (_int, [_vp, _int, _int, _vp, _vp]),

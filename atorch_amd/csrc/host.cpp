@@ -656,8 +656,16 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> linear_forward(const Tensor& x,
   require(goff_in.has_value() || (int64_t)splits.size() == E, "Number of splits should match number of GEMMs.");
   if (goff_in.has_value()) check_offsets(*goff_in, E);
   if (bias.has_value()) check_bias(*bias, E, qw.size(1));
-  Tensor goff = goff_in.has_value() ? *goff_in : offsets_from_list(splits, x.device());
   Quantised q;
+  if (!goff_in.has_value() && !train) {  // offsets and codes in one launch
+    Tensor goff = at::empty({E + 1}, at::TensorOptions().dtype(at::kLong).device(x.device()));
+    q.q = empty(x.sizes(), kFp8, x);
+    q.s = empty({x.size(0), x.size(1) / kTile}, at::kFloat, x);
+    check(aamd_quant_1x128_with_offsets(ptr(x), dtype_code(x.scalar_type(), true), x.size(0), x.size(1), x.size(1), splits.data(), (int)E,
+                                        ptr<int64_t>(goff), ptr<uint8_t>(q.q), ptr<float>(q.s), (float)eps, stream()));
+    return {gemm_nt(q.q, q.s, qw, sw, goff, {}, out_dtype, bias), goff, {}, {}};
+  }
+  Tensor goff = goff_in.has_value() ? *goff_in : offsets_from_list(splits, x.device());
   if (train) q = dual(x, goff, E, eps, padded_bound(x.size(0), E), true, true);
   else std::tie(q.q, q.s) = tile_quant(x, eps);
   return {gemm_nt(q.q, q.s, qw, sw, goff, {}, out_dtype, bias), goff, opt(q.q_t), opt(q.s_t)};

@@ -51,12 +51,12 @@ constexpr int64_t kMaxRowLd = (int64_t)1 << 24;  // row strides (elements) of th
 // byte 128 t of q; the input needs (row, column tile) only where its rows are strided.
 // (the launchers keep ldx below 2^24: 16 U rows of it stay within the 32-bit offset)
 template <typename IN, bool SCATTER, int U>
-__global__ __launch_bounds__(256) void quant_1x128_kernel(const typename IN::elem* __restrict__ x, int64_t ldx,
-                                                          int nt, FastDiv nt_div, int64_t total_tiles,
-                                                          const int32_t* __restrict__ row_map, int topk,
-                                                          int64_t M_out, uint8_t* __restrict__ q,
-                                                          float* __restrict__ s, float eps, int64_t gate_off,
-                                                          u16* __restrict__ h_out) {
+__device__ __forceinline__ void quant_1x128_tiles(const typename IN::elem* __restrict__ x, int64_t ldx,
+                                                  int nt, FastDiv nt_div, int64_t total_tiles,
+                                                  const int32_t* __restrict__ row_map, int topk,
+                                                  int64_t M_out, uint8_t* __restrict__ q,
+                                                  float* __restrict__ s, float eps, int64_t gate_off,
+                                                  u16* __restrict__ h_out) {
   // the short division is checked for bf16 values over scales of bf16 maxima only
   const bool plain_div = !kBf16Values<IN> || eps != 0.f;
   const int grp = threadIdx.x >> 4, l = threadIdx.x & 15;
@@ -122,6 +122,34 @@ __global__ __launch_bounds__(256) void quant_1x128_kernel(const typename IN::ele
       }
     }
   }
+}
+
+template <typename IN, bool SCATTER, int U>
+__global__ __launch_bounds__(256) void quant_1x128_kernel(const typename IN::elem* __restrict__ x, int64_t ldx,
+                                                          int nt, FastDiv nt_div, int64_t total_tiles,
+                                                          const int32_t* __restrict__ row_map, int topk,
+                                                          int64_t M_out, uint8_t* __restrict__ q,
+                                                          float* __restrict__ s, float eps, int64_t gate_off,
+                                                          u16* __restrict__ h_out) {
+  quant_1x128_tiles<IN, SCATTER, U>(x, ldx, nt, nt_div, total_tiles, row_map, topk, M_out, q, s, eps, gate_off, h_out);
+}
+// The rows of a grouped product whose groups' sizes are a host list: one workgroup more stores the offsets, which come as an
+// argument, for the launches behind this one (2048 rows in 4 groups, 512 x 1024: a launch of 1.4 us and its gap less).
+constexpr int kOffsetsHere = 64;
+struct OffsetsHere {
+  int32_t v[kOffsetsHere + 1];
+  int n;
+};
+template <typename IN, int U>
+__global__ __launch_bounds__(256) void quant_1x128_offsets_kernel(const typename IN::elem* __restrict__ x, int64_t ldx, int nt,
+                                                                  FastDiv nt_div, int64_t total_tiles, uint8_t* __restrict__ q,
+                                                                  float* __restrict__ s, float eps, int64_t rows,
+                                                                  const OffsetsHere off, int64_t* __restrict__ goff) {
+  if (blockIdx.x == gridDim.x - 1) {
+    if ((int)threadIdx.x < off.n) goff[threadIdx.x] = off.v[threadIdx.x];
+    return;
+  }
+  quant_1x128_tiles<IN, false, U>(x, ldx, nt, nt_div, total_tiles, nullptr, 1, rows, q, s, eps, 0, nullptr);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -897,6 +925,39 @@ using namespace aamd;
 extern "C" int aamd_quant_1x128(const void* x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx, uint8_t* q,
                                 float* s, float eps, void* stream) {
   return aamd_permute_quant_1x128(x, x_dtype, rows, cols, ldx, nullptr, 1, rows, q, s, eps, stream);
+}
+
+extern "C" int aamd_quant_1x128_with_offsets(const void* x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx, const int64_t* counts,
+                                             int E, int64_t* group_offsets, uint8_t* q, float* s, float eps, void* stream) {
+  AAMD_REQUIRE(x_dtype == AAMD_BF16 || x_dtype == AAMD_F32 || x_dtype == AAMD_F16, "quant_1x128: unsupported dtype %d", x_dtype);
+  AAMD_REQUIRE(rows >= 0 && cols >= 0 && cols % kTile == 0 && ldx >= cols && ldx % 8 == 0 && ldx < kMaxRowLd, "quant_1x128: bad sizes");
+  AAMD_REQUIRE(E >= 1 && counts && group_offsets, "quant_1x128_with_offsets: null pointer or no groups");
+  OffsetsHere off;
+  int64_t run = 0;
+  for (int e = 0; e <= E && e <= kOffsetsHere; e++) {
+    off.v[e] = (int32_t)run;
+    if (e < E) run += counts[e];
+    if (run < 0 || run >= 0x7fffffffLL) e = E;  // (left to the general form)
+  }
+  const int64_t total = rows * (cols / kTile), blocks = (total + 16 * kQuantU - 1) / (16 * kQuantU);
+  if (E > kOffsetsHere || total == 0 || total >= ((int64_t)1 << 31) || run < 0 || run >= 0x7fffffffLL) {
+    const int rc = aamd_group_offsets(counts, 1, E, group_offsets, stream);
+    return rc ? rc : aamd_quant_1x128(x, x_dtype, rows, cols, ldx, q, s, eps, stream);
+  }
+  AAMD_REQUIRE(x && q && s && aligned16(x) && aligned16(q), "quant_1x128: null or unaligned pointer");
+  off.n = E + 1;
+  hipStream_t st = (hipStream_t)stream;
+  const int nt = (int)(cols / kTile);
+  const FastDiv nd = make_fastdiv((uint32_t)nt);
+  const unsigned grid = (unsigned)blocks + 1;
+  if (x_dtype == AAMD_BF16)
+    quant_1x128_offsets_kernel<BF16, kQuantU><<<grid, 256, 0, st>>>((const u16*)x, ldx, nt, nd, total, q, s, eps, rows, off, group_offsets);
+  else if (x_dtype == AAMD_F16)
+    quant_1x128_offsets_kernel<F16, kQuantU><<<grid, 256, 0, st>>>((const u16*)x, ldx, nt, nd, total, q, s, eps, rows, off, group_offsets);
+  else
+    quant_1x128_offsets_kernel<F32, kQuantU><<<grid, 256, 0, st>>>((const float*)x, ldx, nt, nd, total, q, s, eps, rows, off, group_offsets);
+  AAMD_LAUNCH_CHECK("quant_1x128_with_offsets");
+  return AAMD_OK;
 }
 
 extern "C" int aamd_permute_quant_1x128(const void* x, int x_dtype, int64_t T, int64_t cols, int64_t ldx,

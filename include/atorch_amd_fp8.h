@@ -66,6 +66,10 @@ const char *aamd_last_error(void);
  */
 int aamd_quant_1x128(const void *x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx, uint8_t *q, float *s,
                      float eps, void *stream);
+/* aamd_group_offsets of `counts` [E] in host memory and aamd_quant_1x128, in one launch for up to 64 groups
+ * (triton_kernel.py:94-140, quantized_grouped_linear.py:90-101 as there). */
+int aamd_quant_1x128_with_offsets(const void *x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx, const int64_t *counts,
+                                  int E, int64_t *group_offsets, uint8_t *q, float *s, float eps, void *stream);
 
 /*
  * Token permute fused into the 1x128 quantisation: every token row is read and
