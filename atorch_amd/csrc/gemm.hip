@@ -21,8 +21,8 @@
 // matrix pipe busy.
 //
 // Data path: global -> LDS directly (global_load_lds, 16 bytes per lane, no register stop),
-// two stages, one workgroup barrier per step.  (Row-ragged launches on 256 x 256 tiles have a kernel of
-// their own, gemm_rows.hip.)  Rows are 128 bytes; the 16-byte chunks of a row
+// two stages, one workgroup barrier per step.  (Launches on 256 x 256 tiles have
+// kernels of their own, gemm_rows.hip and gemm_wgrad.hip.)  Rows are 128 bytes; the 16-byte chunks of a row
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
 #include <algorithm>

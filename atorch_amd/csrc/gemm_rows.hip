@@ -154,8 +154,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
 
   // ---- the tiles of this workgroup ------------------------------------------------------------
   // Workgroup ids go round-robin over the 8 XCDs; every XCD gets one contiguous range of tile ids, in which tiles that share
-  // operand panels are neighbours, and its workgroups take them side by side.  (Which one of them takes which tile of a round
-  // rotates, so that no workgroup gets the short last tile of every group.)
+  // operand panels are neighbours, and its workgroups take them side by side.
   GroupRanges gr = {};
   int total_lt = (int)((p.Lrows + BM - 1) / BM);
   if (p.goff != nullptr) {
@@ -172,6 +171,12 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
   const uint32_t xcd = blockIdx.x & 7u, nwg = gridDim.x >> 3;
   const RowTiles mine(ntot, xcd);
 
+  // Workgroups that share a panel should stay the same ones: then the first of them to reach a block waits for memory and the
+  // others catch up.  With short contractions, whose panels the L2 holds whole, a workgroup moves five places on with every round
+  // instead, so that none gets the short last tile of every group.  (Places moved by 5 and by none, us: 32768 rows in 8 groups, 28672
+  // x 4096 3425 and 3403, fetched beyond the L2 9.7 and 7.9 GB; 64 groups, 7168 x 2048 218 and 213; 4096 rows, 28672 x 4096 562 and
+  // 554; 60 uneven groups, 2048 x 2816 228 and 229, 1408 x 2048 130 and 132, 2048 x 1408 (11 blocks) 134 and 138.)
+  const uint32_t places = p.nkb >= 16 ? 0u : nwg > 5u ? 5u : 1u;
   uint32_t round_first = mine.first, turn = blockIdx.x >> 3;
   // the next tile of this workgroup, false if there is none; part and parts: of the contraction it takes, slot: where a part goes
   uint32_t part = 0, parts = 1;
@@ -189,7 +194,7 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
     }
     pid = round_first + at;
     round_first += nwg;
-    turn += nwg > 5u ? 5u : 1u;
+    turn += places;
     turn = turn >= nwg ? turn - nwg : turn;
     return at < left;
   };
