@@ -477,7 +477,7 @@ def run_gemm(args, kernels, dev, workload=None, steps=None, warmup=None, cpu_bas
     nt_med_ms = statistics.median(per_step)
     traffic, traffic_src = measured_traffic("grouped_gemm_" + workload)
     roofline = {
-        "kernel": "grouped_gemm_kernel<kRaggedRows> (forward and dgrad)",
+        "kernel": "row_tiles_kernel (forward and dgrad)",
         "bound": "mfma",
         "achieved": round(nt_tflops, 2),
         "peak": PEAK_FP8_TFLOPS,
