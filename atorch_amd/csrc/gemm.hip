@@ -21,8 +21,9 @@
 // matrix pipe busy.
 //
 // Data path: global -> LDS directly (global_load_lds, 16 bytes per lane, no register stop),
-// two stages, one workgroup barrier per step.  (Launches on 256 x 256 tiles have
-// kernels of their own, gemm_rows.hip and gemm_wgrad.hip.)  Rows are 128 bytes; the 16-byte chunks of a row
+// two stages, one workgroup barrier per step (two in the 256 x 256 configuration, whose L tile is
+// requested two steps ahead; it serves row-ragged launches of one round of tiles, longer ones and weight
+// gradients have kernels of their own, gemm_rows.hip and gemm_wgrad.hip).  Rows are 128 bytes; the 16-byte chunks of a row
 // are XOR-swizzled so that the linear 1 KB writes of the direct loads and the 32-row MFMA
 // operand reads are both bank-conflict free on the 64-bank LDS (measured: ~235 of 256 B/clk).
 #include <algorithm>
@@ -61,8 +62,9 @@ __device__ __forceinline__ void store4(OUT* dst, v4f o, bool accumulate) {
 }
 
 // Tile configuration: WR x WL waves, each computing (WTR*32) R rows x (WTL*32) L rows.
-template <int WR_, int WL_, int WTR_, int WTL_, int PRB_ = 2>
+template <int WR_, int WL_, int WTR_, int WTL_, int PRB_ = 2, bool LAHEAD_ = false>
 struct Cfg {
+  static constexpr bool LAHEAD = LAHEAD_;  // load the L tile two steps ahead (extra barrier per step)
   static constexpr int WR = WR_, WL = WL_, WTR = WTR_, WTL = WTL_;
   static constexpr int PRB = PRB_;  // raw-product buffers: 2 folds a sub-tile under the next one's MFMAs
   static constexpr int NT = 64 * WR * WL;   // threads
@@ -77,6 +79,7 @@ struct Cfg {
   static_assert((NT / 8) % 16 == 0, "the swizzle of a slab depends on the wave only");
 };
 typedef Cfg<2, 2, 2, 2, 3> CfgSmall;  // 256 threads, 128 (L) x 128 (R), two workgroups per CU
+typedef Cfg<2, 4, 4, 2, 1, true> CfgLarge;  // 512 threads, 256 (L) x 256 (R); one product buffer: 256 registers per lane
 typedef Cfg<2, 4, 2, 2> CfgWgrad;  // 512 threads, 256 (L) x 128 (R): room for the per-row R scales
 
 // ---- weight gradient of short groups -----------------------------------------------------------
@@ -600,7 +603,8 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   // are fetched every eighth step, 16 bytes per thread, into [row][8] floats.  The last batch is
   // shifted back so that it ends at the last block.
   const bool batch = MODE == kRaggedRows && p.ls_batch != 0;  // uniform; implies nkb >= 8
-  const bool step_scale = !(batch && l_side);  // this wave loads a scale every step
+  // this wave loads a scale every step (never in the configuration that takes all its scales in batches)
+  const bool step_scale = !C::LAHEAD && !(batch && l_side);
   const int brow = (tid >> 1) < lvalid ? (tid >> 1) : lvalid - 1;
   const uint32_t boff = ((uint32_t)brow * (uint32_t)p.ls_row_stride + (uint32_t)(tid & 1) * 4u) * 4u;
   auto batch_start = [&](int b) { return 8 * b + 8 <= nkb ? 8 * b : nkb - 8; };
@@ -638,8 +642,10 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
                  : "memory");
   };
   auto dmaR_scales = [&](int kb, float* Sd) {
-    if (!l_side) dma_scale(kb, Sd);
-    if (batch && (kb & 7) == 0) dma_scale_batch(kb >> 3);  // lands a step before its first use
+    if constexpr (!C::LAHEAD) {
+      if (!l_side) dma_scale(kb, Sd);
+      if (batch && (kb & 7) == 0) dma_scale_batch(kb >> 3);  // lands a step before its first use
+    }
   };
   auto dmaL_one = [&](int n, int kb, uint8_t* Ld, float* Sd) {
     dmaL_tile(n, kb, Ld);
@@ -750,7 +756,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
   // the workgroup barrier.  Branch free: waves outside a partial R tile compute on clamped
   // rows and skip only the final store.
   constexpr int NTILES = C::WTR * C::WTL;
-  auto compute = [&](int kb, int stage, const float* Sct) {
+  auto compute = [&](int kb, int stage, const float* Sct, auto&& after_l_reads, auto&& per_tile) {
     __builtin_amdgcn_sched_barrier(0);
     // L scale of tile row r: Lsc[r * lsc_stride]
     const int bsel = kb >> 3;
@@ -830,6 +836,10 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
       // the next R row overwrites the fragment and scale slot of row i - 1, whose last fold is done
       if (j == 0 && i + 1 < C::WTR) load_r(i + 1);
       __builtin_amdgcn_sched_barrier(0);
+      // every L fragment has been an MFMA operand by now, so it has left the LDS: the hook (a
+      // barrier and the next L loads) costs no extra wait here
+      per_tile(T);
+      if (t == C::WTL - 1) after_l_reads();
     });
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -845,28 +855,230 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  auto nothing = [] {};
+  auto no_feed = [](auto) {};
   // Two workgroups per CU: the loads of a step go out in one burst after the barrier (issued a few
   // at a time behind the sub-tiles they measured 6 % slower here: they have less time to arrive,
   // and the other workgroup already fills the issue gap).
-  if (nkb > 0) dma(0, Lbuf0, Rbuf0, Sc0);
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  // a wave without valid rows runs its own copy of the loop, loads and barriers only
-  auto loop = [&](auto W) {
-    constexpr bool kWork = decltype(W)::value;
-    int kb = 0;
-    for (; kb + 1 < nkb; kb += 2) {  // two steps per trip: the stage addresses are compile-time constants
-      dma(kb + 1, Lbuf1, Rbuf1, Sc1);
-      if constexpr (kWork) compute(kb, 0, Sc0);
-      dma_wait_and_sync();
-      dma(kb + 2 < nkb ? kb + 2 : kb + 1, Lbuf0, Rbuf0, Sc0);  // the last prefetch re-reads a valid block
-      if constexpr (kWork) compute(kb + 1, 1, Sc1);
-      dma_wait_and_sync();
+  if constexpr (!C::LAHEAD) {
+    if (nkb > 0) dma(0, Lbuf0, Rbuf0, Sc0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // a wave without valid rows runs its own copy of the loop, loads and barriers only
+    auto loop = [&](auto W) {
+      constexpr bool kWork = decltype(W)::value;
+      int kb = 0;
+      for (; kb + 1 < nkb; kb += 2) {  // two steps per trip: the stage addresses are compile-time constants
+        dma(kb + 1, Lbuf1, Rbuf1, Sc1);
+        if constexpr (kWork) compute(kb, 0, Sc0, nothing, no_feed);
+        dma_wait_and_sync();
+        dma(kb + 2 < nkb ? kb + 2 : kb + 1, Lbuf0, Rbuf0, Sc0);  // the last prefetch re-reads a valid block
+        if constexpr (kWork) compute(kb + 1, 1, Sc1, nothing, no_feed);
+        dma_wait_and_sync();
+      }
+      if constexpr (kWork)
+        if (kb < nkb) compute(kb, 0, Sc0, nothing, no_feed);  // odd number of steps
+    };
+    if (has_work) loop(std::true_type{});
+    else loop(std::false_type{});
+  } else {
+    // One workgroup per CU, eight waves, two per SIMD.  The matrix pipe of a SIMD idles whenever both
+    // of its waves are away from their MFMAs at the same time, which is what a workgroup barrier
+    // followed by LDS reads produces.  So the two barriers of a step stand where register-resident
+    // MFMA work follows them:
+    //   Q (start of step k): every wave holds the L fragments of step k, so the L half of stage k is
+    //     free and the L tile of step k+2 is requested behind the first sub-tiles;
+    //   P (before the last R row of sub-tiles): every wave has read the last fragments of stage k
+    //     and the tiles of step k+1 have landed; behind it the R tile of step k+2 is requested and
+    //     the first fragments of step k+1 are read from the LDS while the last R row, whose operands
+    //     are already in registers, runs on the matrix pipe.  The fragment registers of step k are
+    //     reused as they die, so the prefetch costs no registers.
+    // The fold of the sub-tile in front of a barrier is issued behind it: the wave that arrives last
+    // has just issued its MFMAs, and the one that waited folds while those still run.
+    // Loads complete in issue order, so "all but the newest L group" is one wait count.  Past the
+    // end the loads re-read the last block to keep the counts uniform.
+    static_assert(!R_PER_ROW && MODE == kRaggedRows, "the two-barrier pipeline is written for block-scaled R operands");
+    static_assert(C::PRB == 1 && C::WTR % 2 == 0 && C::RCH % C::WTL == 0 && C::LCH <= NTILES, "pipeline shape");
+    constexpr int PT = (C::WTR - 1) * C::WTL - 1;  // the sub-tile in front of barrier P
+    constexpr int RPER = C::RCH / C::WTL;
+    auto kclamp = [&](int k) { return k < nkb ? k : nkb - 1; };
+    // Scales of this pipeline come in batches of eight contraction blocks only (the launcher takes the other
+    // configuration when K has fewer than eight blocks), so a
+    // step issues no scale load and takes no branch: batch b (blocks 8 b .. 8 b + 7, the last one shifted
+    // back to end at the last block) is requested behind barrier P of step 8 (b - 1), eight steps before
+    // its first use.  L scales: every wave fetches 32 rows x 32 bytes into LsB[b & 1][row][8]; R block
+    // scales: wave 0 fetches the tile's two 128-row blocks x 32 bytes into RsB[b & 1][block][8] (lanes past
+    // the fourth repeat those addresses: the direct-to-LDS load always writes 1 KB).
+    // Scale rows that are not 16-byte aligned (a number of contraction blocks that is not a multiple of four, an
+    // unaligned base) take 4-byte loads instead: four per wave and batch for the L scales (lane l of load q fetches
+    // float 64 q + l of the wave's 32 rows x 8 floats), one for the R scales.
+    float* const RsB0 = Sc0;  // [2][NT] floats, the first 16 of each in use
+    const bool x4 = p.ls_batch == 1;
+    const int rblocks = rvalid / kTile;
+    const int rlane_blk = ((lane >> 1) & 1) < rblocks ? (lane >> 1) & 1 : rblocks - 1;
+    const uint32_t roff = ((uint32_t)rlane_blk * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 1) * 4u) * 4u;
+    const int rlane_blk1 = ((lane >> 3) & 1) < rblocks ? (lane >> 3) & 1 : rblocks - 1;
+    const uint32_t roff1 = ((uint32_t)rlane_blk1 * (uint32_t)p.rs_row_stride + (uint32_t)(lane & 7) * (uint32_t)p.rs_blk_stride) * 4u;
+    uint32_t boff1[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int row = wave * 32 + q * 8 + (lane >> 3);
+      boff1[q] = ((uint32_t)(row < lvalid ? row : lvalid - 1) * (uint32_t)p.ls_row_stride + (uint32_t)(lane & 7)) * 4u;
     }
-    if constexpr (kWork)
-      if (kb < nkb) compute(kb, 0, Sc0);  // odd number of steps
-  };
-  if (has_work) loop(std::true_type{});
-  else loop(std::false_type{});
+    auto dma_batches = [&](int b) {
+      const uint8_t* lsb = reinterpret_cast<const uint8_t*>(Lsg + uniform_i64(l0 * p.ls_row_stride + batch_start(b)));
+      const uint8_t* rsb = reinterpret_cast<const uint8_t*>(Rsg + uniform_i64((r0 / kTile) * p.rs_row_stride + batch_start(b) * p.rs_blk_stride));
+      const uint32_t ldst = lds_addr(LsB0 + (b & 1) * (BM * 8)) + (uint32_t)(wave * 1024);
+      const uint32_t rdst = lds_addr(RsB0 + (b & 1) * NT);
+      if (x4) {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(boff), "s"(lsb), "s"(ldst) : "memory");
+        if (!R_ROWS && wave == 0)
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(roff), "s"(rsb), "s"(rdst) : "memory");
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(boff1[q]), "s"(lsb), "s"(ldst + (uint32_t)(q * 256)) : "memory");
+        if (!R_ROWS && wave == 0)
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(roff1), "s"(rsb), "s"(rdst) : "memory");
+      }
+      if (R_ROWS && wave == 0)  // a row of scales per contraction block: never 16 bytes of one block
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(roff1), "s"(rsb), "s"(rdst) : "memory");
+    };
+    if (nkb > 0) {
+      dmaL(0, Lbuf0, Sc0);  // (the per-step scale hooks of these helpers are off: see step_scale)
+      dmaR(0, Rbuf0, Sc0);
+      dma_batches(0);
+      dmaL(kclamp(1), Lbuf1, Sc1);
+      dmaR(kclamp(1), Rbuf1, Sc1);
+      // the tiles of step 0 and the first scale batch have landed; those of step 1 may still be on their way
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::LCH + C::RCH) : "memory");
+      auto barrier_q = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+      // all but this step's L tile loads have landed (loads complete in issue order)
+      auto barrier_p = [&]() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::LCH) : "memory"); };
+      if (has_work) {
+        v8i lf[C::WTL][2], rf[2][2];
+        float cs[C::WTL], csn[C::WTL], rblkn;
+        float cs_last = 0.f;  // scale of the sub-tile whose fold is still owed (the last one of the step before)
+        v16f pr, zero;
+#pragma unroll
+        for (int r = 0; r < 16; r++) zero[r] = pr[r] = 0.f;
+        // scales of step kb: the lane's L row scales and the R block scale of the wave; their product is
+        // formed where it is first needed, not where the reads are issued
+        auto read_scales = [&](int kb, float (&dst)[C::WTL], float& rblk) {
+          const int b = kb >> 3, in_batch = kb - batch_start(b);
+          const float* Lsc = LsB0 + (b & 1) * (BM * 8) + in_batch;
+          rblk = RsB0[(b & 1) * NT + (wrow0 / kTile) * 8 + in_batch];
+#pragma unroll
+          for (int j = 0; j < C::WTL; j++) dst[j] = Lsc[(wlrow0 + j * 32 + l32) * 8];
+        };
+        // (the empty volatile statements pin MFMAs and folds between the memory instructions around
+        // them: plain arithmetic is otherwise free to drift past inline assembly)
+        auto fold = [&](int i, int j, float sc) {
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[i][j][r] = __builtin_fmaf(pr[r], sc, acc[i][j][r]);
+          asm volatile("" : "+v"(acc[i][j]));
+        };
+        // fragments and scales of step 0
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          lf[0][h] = frag(la, 0, BM, 0, h);
+          rf[0][h] = fragR(0, 0, h);
+        }
+#pragma unroll
+        for (int j = 1; j < C::WTL; j++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) lf[j][h] = frag(la, 0, BM, j, h);
+        read_scales(0, cs, rblkn);
+#pragma unroll
+        for (int j = 0; j < C::WTL; j++) cs[j] *= rblkn;
+        // FIRST: the first step of a run of eight, which requests the next scale batch behind barrier P
+        auto step = [&](int kb, auto S, auto FIRST) {
+          constexpr int s = decltype(S)::value;
+          constexpr bool kFirst = decltype(FIRST)::value;
+          uint8_t* const Lc = s ? Lbuf1 : Lbuf0;
+          uint8_t* const Rc = s ? Rbuf1 : Rbuf0;
+          const int k2 = kclamp(kb + 2);
+          __builtin_amdgcn_sched_barrier(0);
+          barrier_q();
+          __builtin_amdgcn_sched_barrier(0);
+          fold(C::WTR - 1, C::WTL - 1, cs_last);  // owed by the step before (adds zero in the first step)
+          static_for<NTILES>([&](auto T) {
+            constexpr int t = decltype(T)::value;
+            constexpr int i = t / C::WTL, j = t % C::WTL;
+            __builtin_amdgcn_sched_barrier(0);
+            pr = mfma_fp8_32x32x64(rf[i & 1][0], lf[j][0], zero);
+            pr = mfma_fp8_32x32x64(rf[i & 1][1], lf[j][1], pr);
+            asm volatile("" : "+v"(pr));
+            __builtin_amdgcn_sched_barrier(0);
+            // memory instructions go out while the MFMAs run, ahead of the fold that waits for them
+            if constexpr (t < C::LCH) dmaL_tile(t, k2, Lc);
+            if constexpr (j == 0 && i + 1 < C::WTR) {
+#pragma unroll
+              for (int h = 0; h < 2; h++) rf[(i + 1) & 1][h] = fragR(s, i + 1, h);
+            }
+            if constexpr (t == PT) {
+              __builtin_amdgcn_sched_barrier(0);
+              barrier_p();
+              __builtin_amdgcn_sched_barrier(0);
+              if constexpr (kFirst) {
+                if (kb + 8 < nkb) dma_batches((kb >> 3) + 1);
+              }
+              // row C::WTR - 2 has been consumed: its registers take the first R row of the next step
+#pragma unroll
+              for (int h = 0; h < 2; h++) rf[0][h] = fragR(s ^ 1, 0, h);
+              read_scales(kclamp(kb + 1), csn, rblkn);
+            }
+            if constexpr (t > PT) {
+              constexpr int jn = t - PT - 1;  // == j: this sub-tile was the last user of lf[j]
+              static_for<RPER>([&](auto N) { dmaR_tile(jn * RPER + decltype(N)::value, k2, Rc); });
+#pragma unroll
+              for (int h = 0; h < 2; h++) lf[jn][h] = frag(la, s ^ 1, BM, jn, h);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (t + 1 < NTILES) fold(i, j, cs[j]);
+          });
+          cs_last = cs[C::WTL - 1];
+#pragma unroll
+          for (int j = 0; j < C::WTL; j++) cs[j] = csn[j] * rblkn;
+        };
+        // runs of eight steps (the contraction has at least eight blocks; the last run may be shorter), two
+        // steps per trip so that the stage addresses are compile-time constants
+        constexpr std::integral_constant<int, 0> S0{};
+        constexpr std::integral_constant<int, 1> S1{};
+        for (int kb = 0; kb < nkb; kb += 8) {
+          const int n = nkb - kb < 8 ? nkb - kb : 8;
+          step(kb, S0, std::true_type{});
+          if (n > 1) step(kb + 1, S1, std::false_type{});
+          int kk = 2;
+          for (; kk + 1 < n; kk += 2) {
+            step(kb + kk, S0, std::false_type{});
+            step(kb + kk + 1, S1, std::false_type{});
+          }
+          if (kk < n) step(kb + kk, S0, std::false_type{});  // odd number of steps
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fold(C::WTR - 1, C::WTL - 1, cs_last);
+      } else {
+        // a wave without valid rows: loads and barriers only, in the order of the working waves
+        auto step = [&](int kb, uint8_t* Lc, uint8_t* Rc, bool first) {
+          const int k2 = kclamp(kb + 2);
+          barrier_q();
+#pragma unroll
+          for (int n = 0; n < C::LCH; n++) dmaL_tile(n, k2, Lc);
+          barrier_p();
+          if (first && kb + 8 < nkb) dma_batches((kb >> 3) + 1);
+#pragma unroll
+          for (int n = 0; n < C::RCH; n++) dmaR_tile(n, k2, Rc);
+        };
+        int kb = 0;
+        for (; kb + 1 < nkb; kb += 2) {
+          step(kb, Lbuf0, Rbuf0, (kb & 7) == 0);
+          step(kb + 1, Lbuf1, Rbuf1, false);
+        }
+        if (kb < nkb) step(kb, Lbuf0, Rbuf0, (kb & 7) == 0);
+      }
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the trailing loads must not land in the epilogue's staging
+    }
+  }
 
   // ---- epilogue ------------------------------------------------------------------------------
   // A lane holds, for one output row, groups of four consecutive columns; stored directly that
@@ -1003,7 +1215,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 // Launch choices a caller of the measurement build may pin per call (-1 = the library chooses, which is
 // all the product entry points ever pass).
 struct GemmOptions {
-  int tile = -1;      // 0: 128x128 tiles, 1: the large configuration, 2 / 3: the kernel for few rows, 3 in its split form
+  int tile = -1;      // 0: 128x128 tiles, 1: 256x256 tiles, 2 / 3: the kernel for few rows, 3 in its split form, 4: a workgroup per 256x256 tile
   int group_r = -1;   // tile order groups R tiles (1) or L tiles (0)
   int gl = -1;        // tiles that share a panel in the tile order
   int ls_batch = -1;  // 0: L scales fetched one contraction block at a time
@@ -1066,12 +1278,12 @@ static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8
 // 125 rows on the kernel for few rows 15.8 -> 25.5, on the small tiles 12.7 -> 19.0).  What they decide, us, the 256x256 tiles
 // or the kernel for few rows priced wrong -> this fit: one group of 14441 rows, 5504 x 640 200 -> 91; 64 groups, 8591 rows,
 // 16256 x 768 372 -> 195; 4 groups, 2498 rows, 8832 x 512 51 -> 30.
-enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3 };
+enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4 };
 // (weights read along their rows, b_rows: the same line but for the split form, which they do not have; 128 x 32 blocks of the
 // kernel for few rows are as many as 64 x 64 ones)
 // share_last: with a workspace for parts of the last round of 256 x 256 tiles.
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
-  if (g_opt.tile >= 0) return g_opt.tile == 1 && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
+  if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const int64_t groups = M < E ? M : E;
   const double n = (double)nkb;
   auto token_tiles = [&](int rows) -> double {
@@ -1107,7 +1319,16 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   const bool may_split = !b_rows && (blocks_f < 128.0 || nkb >= 28 || (blocks_f <= 256.0 && M <= 32 * groups));
   const double split = may_split ? std::max({2.2 + 1e-3 * blocks_p * (0.45 * n + 2.1), 4.0 + 0.63 * std::ceil(n / 8.0), weights / 6.2}) : 1e30;
   if (std::min(few, split) <= std::min(small, large)) return split < few ? kFewRowsSplit : kFewRows;
-  return large < small ? kLargeTiles : kSmallTiles;
+  if (small <= large) return kSmallTiles;
+  // A workgroup per tile where none would have a second one: the step of grouped_gemm_kernel has no bookkeeping of a stream of
+  // tiles (next tile, next scales; with an odd number of steps also the addresses of the stages) and is 1 to 3 % shorter, which
+  // counts while power does not bound the launch.  Persistent over this form, 486 launches of at most a round, mean ratio: up to 0.25
+  // rounds 1.01, 0.5 1.02, 0.75 1.04 (the most 1.11), 1 1.02; 1 to 1.5 0.99, 2 0.97, more 0.94 to 0.97.  Where the last round
+  // may share its contraction, up to half a round does (2599 rows, 2560 x 8576: 97 persistent, 89 this form, 79 shared); groups,
+  // whose tiles are only estimated, lose more past a round (8 groups, 1841 rows, 5248 x 7424, 0.92 expected and 1.07 rounds: 131
+  // shared, 163) than the launch that adds the parts costs below (2 to 6 us: 1667 rows, 6656 x 8832 116 -> 108).
+  const bool once = share_last ? rounds_l > 0.5 && rounds_l <= (grouped && E > 1 ? 0.8 : 1.0) : rounds_l <= 1.0;
+  return once ? kLargeOnce : kLargeTiles;
 }
 // Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
 static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
@@ -1189,7 +1410,8 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   const NtKernel kernel = b_tile_scaled ? (use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), g_opt) ? kLargeTiles : kSmallTiles)
                                         : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, ws != nullptr, g_opt);
   // (output rows of 8 M elements are out of reach of the large tiles' 32-bit offsets)
-  const bool large = kernel == kLargeTiles && (b_tile_scaled || ldc < (1LL << 23));
+  const bool once = kernel == kLargeOnce && !b_tile_scaled;
+  const bool large = once || (kernel == kLargeTiles && (b_tile_scaled || ldc < (1LL << 23)));
   const int BM = large ? kLargeTile : CfgSmall::BM;
   const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : kLargeTile) : CfgSmall::BN;
   static_assert(CfgWgrad::BM == kLargeTile, "L rows of a large tile");
@@ -1214,6 +1436,9 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   if (kernel == kFewRows || kernel == kFewRowsSplit) return launch_few_rows(p, c_dtype, M, kernel == kFewRowsSplit, b_rows, st);
   const int64_t max_lt = group_offsets ? M / BM + E : (M + BM - 1) / BM;
   const int64_t blocks = max_lt * p.nRt;
+  if (once)
+    return b_rows ? launch_gemm<kRaggedRows, false, CfgLarge, true>(p, c_dtype, blocks, st, g_opt)
+                  : launch_gemm<kRaggedRows, false, CfgLarge>(p, c_dtype, blocks, st, g_opt);
   if (large && !b_tile_scaled) {
     tile_order<kRaggedRows>(p, kLargeTile, g_opt);
     p.ws = ws;

@@ -23,10 +23,11 @@ const char *aamd_probes_last_error(void);
  * The grouped GEMMs of the product library (same kernels, same arguments as aamd_grouped_gemm_fp8_nt, _nn and
  * aamd_grouped_gemm_fp8_wgrad) with the launch choices the library otherwise makes by itself pinned for
  * this one call: opts = {tile, group_r, gl, ls_batch}, each -1 for the library's own choice.
- *   tile: 0 = 128x128 tiles, 1 = the large configuration (wgrad: 256x256 tiles), 2 / 3 = the kernel for few rows and its split form;
+ *   tile: 0 = 128x128 tiles, 1 = 256x256 tiles, 2 / 3 = the kernel for few rows and its split form, 4 = 256x256 tiles with a
+ *   workgroup each (1, 4: 128x128 tiles where the contraction has fewer than eight blocks; wgrad: 0 and 1 only);
  *   group_r: the tile order groups R tiles (1) or L tiles (0); gl: tiles sharing a panel in the tile order;
- *   ls_batch: 0 = scales fetched one contraction block at a time (which the 128x128 tiles do: the large
- *   configuration of the block-scaled GEMM takes its scales in batches only and is then not chosen).
+ *   ls_batch: 0 = the 128x128 tiles fetch their scales one contraction block at a time, the 256x256 tiles of the
+ *   block-scaled GEMM, which take theirs in batches only, by 4-byte loads.
  * Nothing is kept between calls.
  */
 int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t *a, int64_t lda, const float *a_s, const uint8_t *b,

@@ -36,6 +36,33 @@ def test_large_tiles_give_the_bits_of_small_ones(dev, splits, N, K, out_dtype, b
     assert torch.equal(got[0], got[1]) and torch.all(got[1][M:] == 7.0)
 
 
+@pytest.mark.parametrize("splits,N,K", [
+    ([1], 128, 1024), ([2047], 1152, 1152), ([300, 0, 257, 1, 700], 896, 1280), ([33] * 70 + [0, 1, 255], 384, 2176),
+])  # fmt: skip
+@pytest.mark.parametrize("out_dtype,bias", [(torch.bfloat16, None), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("turned", [False, True])
+def test_a_workgroup_per_tile_gives_the_same_bits(dev, splits, N, K, out_dtype, bias, turned):
+    """The form that launches of one round of tiles take."""
+    from atorch_amd import kernels
+
+    E, M = len(splits), sum(splits)
+    g = torch.Generator(device=dev).manual_seed(10)
+    qx, sx = kernels.tile_quant(torch.randn((M, K), generator=g, device=dev).bfloat16())
+    w = torch.randn((E, K, N) if turned else (E, N, K), generator=g, device=dev).bfloat16() * 0.05
+    q, s, q_t, s_t = kernels.block_quant_batched(w, return_transpose=True, written=kernels.STORED)
+    if turned:
+        q, s = q_t, s_t
+    b = torch.randn((E, N), generator=g, device=dev).to(bias) if bias is not None else None
+    goff = kernels.group_offsets_from_splits(splits, dev)
+    got = {}
+    for tile in (0, 4):
+        out = torch.full((M + 3, N), 7.0, dtype=out_dtype, device=dev)
+        with kernels.gemm_options(tile=tile):
+            kernels.grouped_gemm_nt(qx, sx, q, s, goff, out=out[:M], bias=b)
+        got[tile] = out
+    assert torch.equal(got[0], got[4]) and torch.all(got[4][M:] == 7.0)
+
+
 def test_output_rows_apart(dev):
     """Columns between the rows of a wider output are not touched."""
     from atorch_amd import kernels
