@@ -1,4 +1,5 @@
-// Row-ragged block-scaled FP8 GEMM on 256 x 256 tiles, one persistent workgroup per CU (forward, dgrad, dense).
+// Row-ragged block-scaled FP8 GEMM on 256 x 256 tiles, one persistent workgroup per CU (forward, dgrad, dense).  (Launches of
+// at most one round of tiles take the form with a workgroup per tile, see choose_nt in gemm.hip.)
 //
 // What a step does and why is the same as in gemm.hip: 128-deep blocks, two chained v_mfma_f32_32x32x64_f8f6f4 per 32 x 32
 // sub-tile, the raw product folded into fp32 accumulators with the block's scales, operands moved global -> LDS without a
@@ -19,7 +20,7 @@
 // until its first operands are there, 4.1 to turn the tile round through the LDS and store it.  So a workgroup stays and takes
 // one tile after the other, and the steps of its tiles are one stream: the last two steps of a tile request the first two
 // blocks of the next one, its last step reads the next one's first fragments, and the finished tile goes from the registers
-// to memory (lanes swap halves, so that four of them hold 64 consecutive bytes of a row) while those loads are in flight, as
+// to memory (lanes swap what they hold, so that eight of them have 128 consecutive bytes of a row) while those loads are in flight, as
 // the stage buffers hold them.  What a tile needs besides are scalars: rows past its end and columns past the weights' end
 // are left to the range check of buffer instructions, which neither reads nor writes them.
 //

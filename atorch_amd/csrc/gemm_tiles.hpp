@@ -37,13 +37,14 @@ __device__ __forceinline__ int lane_here() {
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
   return l;
 }
-// (the compiler does not see what is inside: five wait states in front, for scalar registers that the vector unit has just
-// written, and two behind, before the data registers are written again)
+// The kernel's arguments, fetched anew where they are used.
 __device__ __forceinline__ uint64_t args_here() {
   uint64_t a = (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(a));
   return (uint64_t)uniform_i64((int64_t)a);
 }
+// (the compiler does not see what is inside: five wait states in front, for scalar registers that the vector unit has just
+// written, and two behind, before the data registers are written again)
 template <int OFFSET, bool NT>
 __device__ __forceinline__ void store_x4(const v4i& v, uint32_t off, const v4i& buf) {
   if constexpr (NT)
