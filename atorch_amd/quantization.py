@@ -77,14 +77,26 @@ class QuantizeResult:
 
 class WeightCodeStack:
     """Codes of all weights of a module, stacked (data, scale, data_t | None, scale_t | None; the latter two may be views of
-    the former), and the per-weight caches that point into them.  ``whole`` while all of those still do."""
+    the former), and the per-weight caches that point into them.  ``whole`` while all of those still do.
 
-    __slots__ = ("codes", "members", "whole")
+    The fused path reads ``codes``.  Whoever asks a cache for one weight's codes gets them dense, as entries of one
+    buffer, so that the operator interface finds them equally spaced: a field whose stack is a view is made dense as a
+    whole the first time, and that second copy stays with the stack."""
+
+    __slots__ = ("codes", "dense", "members", "whole")
 
     def __init__(self, codes, caches):
-        self.codes, self.members, self.whole = codes, list(caches), True
+        self.codes, self.dense, self.members, self.whole = codes, [None] * 4, list(caches), True
         for i, c in enumerate(self.members):
             c.point_to(self, i)
+
+    def entry(self, k: int, index: int) -> Optional[torch.Tensor]:
+        """Field ``k`` of weight ``index``."""
+        if self.codes[k] is None:
+            return None
+        if self.dense[k] is None:
+            self.dense[k] = self.codes[k].contiguous()
+        return self.dense[k][index]
 
     def serves(self, caches) -> bool:
         return self.whole and len(caches) == len(self.members) and all(map(operator.is_, caches, self.members))
@@ -103,6 +115,9 @@ class _CodeField:
         cache._set(self.k, value)
 
 
+_FIELDS = ("data", "scale", "data_t", "scale_t")
+
+
 @dataclass
 class QuantizeResultCache:
     """Per-weight cache of the fp8 copies between microbatches
@@ -119,7 +134,7 @@ class QuantizeResultCache:
 
     def __new__(cls, *args, **kw):
         self = super().__new__(cls)
-        self._own = [None, None, None, None]
+        self._own, self._source = [None, None, None, None], None
         self.stack, self.index = None, 0
         return self
 
@@ -127,22 +142,27 @@ class QuantizeResultCache:
         """Use entry ``index`` of ``stack``."""
         if self.stack is not None:
             self.stack.whole = False
-        self._own = [None, None, None, None]
-        self.stack = stack
+        self._own = [..., ..., ..., ...]  # (not looked up yet)
+        self.stack = self._source = stack
         self.index = index
 
     def _get(self, k: int) -> Optional[torch.Tensor]:
-        if self._own[k] is None and self.stack is not None and self.stack.codes[k] is not None:
-            # (the stack may hold one orientation and a view of it)
-            self._own[k] = self.stack.codes[k][self.index].contiguous()
+        if self._own[k] is ...:
+            self._own[k] = self._source.entry(k, self.index)
         return self._own[k]
+
+    def holds(self, name: str) -> bool:
+        """Is field ``name`` there?  (Without looking it up.)"""
+        k = _FIELDS.index(name)
+        return (self._source.codes[k] if self._own[k] is ... else self._own[k]) is not None
 
     def _set(self, k: int, value: Optional[torch.Tensor]):
         if self.stack is not None:
-            self._own = [self._get(i) for i in range(4)]
             self.stack.whole = False
             self.stack = None
         self._own[k] = value
+        if all(t is not ... for t in self._own):
+            self._source = None
 
     def to_qresult(self) -> QuantizeResult:
         return QuantizeResult(self.data, self.scale, self.data_t, self.scale_t)

@@ -54,3 +54,33 @@ def test_places_in_a_stack_read_write_and_copy_as_fields():
     assert torch.equal(back.scale_t, c.scale_t)
     c.scale = torch.zeros(4)
     assert not stack.serves(caches) and c.stack is None and torch.equal(c.data, codes[0][1]) and torch.equal(c.scale, torch.zeros(4))
+
+
+def test_codes_of_one_weight_from_a_stack_that_holds_one_orientation():
+    """Dense, equally spaced and, for all weights together, one copy: what the operator interface runs in one launch."""
+    from atorch_amd.quantization import _base_of_stack
+
+    caches = [QuantizeResultCache() for _ in range(3)]
+    data, scale = torch.arange(3 * 4 * 6).view(3, 4, 6), torch.arange(3 * 2 * 3.0).view(3, 2, 3)
+    stack = WeightCodeStack((data, scale, data.transpose(1, 2), scale.transpose(1, 2)), caches)
+    assert caches[0].holds("data_t") and stack.dense == [None] * 4  # (asking whether does not make it)
+    for name, want in (("data", data), ("scale", scale), ("data_t", data.transpose(1, 2)), ("scale_t", scale.transpose(1, 2))):
+        got = [getattr(c, name) for c in caches]
+        assert all(torch.equal(g, w) and g.is_contiguous() for g, w in zip(got, want))
+        assert _base_of_stack(got) == (got[0].data_ptr(), want[0].numel())
+        assert len({g.untyped_storage().data_ptr() for g in got}) == 1
+    assert stack.serves(caches) and caches[1].data.data_ptr() == data[1].data_ptr()  # the stored orientation is not copied
+
+
+def test_replacing_fields_one_by_one_copies_nothing():
+    caches = [QuantizeResultCache() for _ in range(2)]
+    data = torch.arange(2 * 4 * 6).view(2, 4, 6)
+    stack = WeightCodeStack((data, data[:, :1], data.transpose(1, 2), None), caches)
+    for c in caches:
+        c.data = c.scale = torch.zeros(1)
+    assert not stack.serves(caches) and stack.dense == [None] * 4 and caches[0].scale_t is None
+    assert torch.equal(caches[1].data_t, data[1].t())
+    c = copy.deepcopy(caches[0])
+    assert torch.equal(c.data_t, data[0].t()) and torch.equal(pickle.loads(pickle.dumps(caches[0])).data_t, data[0].t())
+    c.data_t = c.scale_t = None
+    assert c.data_t is None and not c.holds("scale_t") and not c.holds("data_t") and c.holds("data")
