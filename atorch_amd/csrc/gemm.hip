@@ -1261,74 +1261,82 @@ constexpr int kSplitBlocks = 48;
 // The most parts of a contraction: eight blocks at least in each, see row_part.
 static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8); }
 
-// Which kernel a row-ragged launch with block-scaled R takes: the one whose estimated time is least.  The estimates (us)
-// are fits to 570 launches on MI355X of 64 to 40000 rows in 1 to 64 even or uneven groups, 512 to 18000 outputs and a
-// contraction of 512 to 14336, each with all of the kernels (n: its 128-deep steps):
-//   - a round of 512 tiles of the 128x128 configuration, two per CU, costs 2.4 us and 0.98 us per step, a launch of at most
-//     256 tiles 5.4 and 0.7;
-//   - a round of 256 tiles of the 256x256 configuration 5.9 us and 0.82 to 1.42 us per step, by how full its tiles are;
-//   - a 64 x 64 block of the kernel for few rows 2.1 ns and 1.06 ns per step, spread over the chip; a 32 x 32 block of its
-//     split form 2.1 and 0.45; and no less than a wave's own chain of every fourth (eighth) step;
-//   - and none can beat the weights' stream from memory, 5.2 to 6.2 TB/s.
-// Token tiles are counted as the groups' expected number (their sizes are known on the device only): one per group with
-// few rows, half a tile more than the rows fill with many.  Over those launches, the ones the fit was made from, the kernel
-// taken is 2.4 % slower than the best of the four (geometric mean).  They repeat one launch on the same operands, which then
-// come from a cache, so the estimates rank the kernels better than they give their times: in a pass over new operands the
-// launches of a few microseconds take longer (estimated -> traced: 4 groups of 512 rows, 1024 x 512 7.9 -> 11.3; 8 groups of
-// 125 rows on the kernel for few rows 15.8 -> 25.5, on the small tiles 12.7 -> 19.0).  What they decide, us, the 256x256 tiles
-// or the kernel for few rows priced wrong -> this fit: one group of 14441 rows, 5504 x 640 200 -> 91; 64 groups, 8591 rows,
-// 16256 x 768 372 -> 195; 4 groups, 2498 rows, 8832 x 512 51 -> 30.
-enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4 };
-// (weights read along their rows, b_rows: the same line but for the split form, which they do not have; 128 x 32 blocks of the
-// kernel for few rows are as many as 64 x 64 ones)
-// share_last: with a workspace for parts of the last round of 256 x 256 tiles.
+// Which kernel a row-ragged launch with block-scaled R takes: the one whose estimated time is least.  The estimates (us) were
+// fitted to 3280 timings on MI355X of launches of 1 to 40000 rows in 1 to 64 groups, even and uneven (Zipf) ones, 512 to 18000
+// outputs and a contraction of 512 to 14336, weights along either side and in a cache or in none, each with all of the kernels
+// (n: 128-deep steps):
+//   - 128 x 128 tiles, two of them per CU: up to a tile per CU 5.4 and 0.76 per step; else 2.9, and 3.3 and 1.045 per step for
+//     every round of 512 tiles; the last of few rounds up to 0.08 per step less where not every CU has two, 0.85 where none has;
+//   - 256 x 256 tiles 6.5, and 6.3 and 0.78 to 1.08 per step for every round of 256, by how full the tiles and the round are;
+//     with a last round in parts 20 and 10 times what it fills, for writing and adding them, and its steps by the number of
+//     parts; 4 more where a workspace is at hand and the last round turns out not to be shared;
+//   - a 64 x 64 block of the kernel for few rows 2.7 ns and 1.1 ns per step, spread over the chip; a 32 x 32 block of its split
+//     form 3.6 and 0.47; and no less than a wave's own chain of every fourth (eighth) step;
+//   - and none can beat the weights' stream from memory.
+// The groups' sizes are known on the device only.  Groups with rows are expected to be E (1 - exp(-0.6 M / E)), token tiles one
+// per such group with few rows and 0.56 of a tile per group more than the rows fill with many; what depends on rounds is the mean
+// over that many tiles and up to 16 % more and less, by what the groups' own tiles are of them.  The kernel taken is 1.2 % slower
+// than the best of them (geometric mean; more than 5 % slower in 7 %) over those timings, and 1.3 % over 4400 others; the lines these
+// replace, which priced the large tiles as they were with a workgroup per tile and took whole rounds of expected tiles, came to
+// 3.2 and 3.2 % (15 %).  Where the kernel changed it takes 0.90 of the time on average.  us: 83 rows in 64 groups, 768 x 768 9.6 ->
+// 3.9; 2965 in 60 (Zipf), 2048 x 11008 200 -> 97; 726 in 8, 6528 x 6656 141 -> 85; 1394 in 16, 5888 x 9216 186 -> 116.  Of the
+// others 2.9 % take 3 % or more longer than before, 11 % that much less; the worst are uneven groups, whose empty ones the host
+// does not know of (1776 in 60, 25856 x 512 63 -> 110; 3532 in 16, 1664 x 6144 53 -> 67).
+enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4, kLargeShared = 5 };
+// b_rows: weights read along their rows, which the split form cannot.  share_last: with a workspace for parts of the last round of
+// 256 x 256 tiles.
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
-  const int64_t groups = M < E ? M : E;
-  const double n = (double)nkb;
-  auto token_tiles = [&](int rows) -> double {
-    if (!grouped || E == 1) return (double)((M + rows - 1) / rows);
-    return std::max((double)M / rows + 0.5 * (double)groups, (double)groups);
+  const bool one = !grouped || E == 1;
+  const double n = (double)nkb, rows = (double)M;
+  const double groups = one ? 1.0 : std::min({rows, (double)E, (double)E * (1.0 - std::exp(-0.6 * rows / (double)E))});
+  auto token_tiles = [&](int64_t size) {
+    return one ? (double)((M + size - 1) / size) : std::max(rows / (double)size + 0.56 * groups, groups);
   };
-  // whole rounds where there are few; with many the tiles' times spread and half a round is lost at the end
-  auto rounds = [](double x) { return x <= 1.0 ? 1.0 : x < 3.0 ? std::ceil(x) : x + 0.5; };
-  const double weights = (double)groups * (double)N * n * (double)kBK * 1e-6;  // MB
-  const double tiles_s = token_tiles(128) * (double)(N / 128);
-  const double small = std::max(tiles_s <= 256.0 ? 5.4 + 0.7 * n : 2.5 + rounds(tiles_s / 512.0) * (2.4 + 0.98 * n), weights / 5.6);
-  // (the large configuration takes its scales in batches of eight contraction blocks)
-  const double rows_l = token_tiles(256), fill = std::min(1.0, (double)M / (256.0 * rows_l));
-  const double rounds_l = rows_l * (double)((N + 255) / 256) / 256.0, step_l = 0.82 + 0.6 * fill;
-  double loop_l = 2.3 + rounds(rounds_l) * (5.9 + step_l * n);
-  // (a last round in parts, after one or two whole ones: its steps, and 33 us for writing and adding the parts)
-  const double whole = std::floor(rounds_l), parts = std::min((double)row_max_split(nkb), std::floor(1.0 / (rounds_l - whole + 1e-9)));
-  if (share_last && whole >= 1.0 && whole < 3.0 && parts >= 2.0 && rounds_l > whole)
-    loop_l = std::min(loop_l, 2.3 + whole * (5.9 + step_l * n) + 33.0 + step_l * n / parts);
-  const double large = nkb < 8 ? 1e30 : std::max(loop_l, weights / 5.2);
-  const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_p = token_tiles(32) * (double)(N / 32);
-  const double few = std::max({4.5 + 1e-3 * blocks_f * (1.06 * n + 2.1), 1.5 + 1.1 * std::ceil(n / 4.0), weights / 6.2});
-  // The split form where the length of a wave's contraction is what counts: few workgroups, or a long contraction.  Traced on
-  // weights out of the caches and rows just quantised, us, 64 x 64 blocks and their split form (its estimate): up to 256
-  // blocks the split form is the faster one at any length (128 blocks, 16 steps 7.8 and 5.8 (5.3), 28 steps 12.7 and 8.6
-  // (6.5); 176, 16: 7.8 and 6.9 (5.5); 256, 16: 10.4 and 9.6 (7.0)), from 512 on it is not (8 steps 10.2 and 10.5 (8.0), 16
-  // steps 15.2 and 15.9 (11.7), 28 steps 23.4 and 24.1 (18.9)) unless the weights' stream bounds both (1024, 56: 79 and 76).
-  // Its estimate is 1 to 5 us too low in between, so that without a line it would be taken at 512 blocks too; from 128 on only
-  // groups of up to 32 rows take it, one token tile of either form.  (Around the line, on weights out of the caches, 64 x 64 blocks
-  // and their split form, us: 4 groups of a row, 2816 x 2048 (176 blocks) 13.0 and 11.7, 2048 x 1408 (128) 8.6 and 7.2; 16 rows in 8
-  // groups, 1536 x 1024 (192) 7.9 and 7.4; 100 in 4, 4096 x 512 (256) 7.5 and 6.5; 500 in 8, 1024 x 1024 (189) 8.8 and 6.8, but with
-  // the weights in the caches 6.5 and 7.3; 512 in 8, 2048 x 7168 (384) 48.6 and 56.5.)
-  const bool may_split = !b_rows && (blocks_f < 128.0 || nkb >= 28 || (blocks_f <= 256.0 && M <= 32 * groups));
-  const double split = may_split ? std::max({2.2 + 1e-3 * blocks_p * (0.45 * n + 2.1), 4.0 + 0.63 * std::ceil(n / 8.0), weights / 6.2}) : 1e30;
-  if (std::min(few, split) <= std::min(small, large)) return split < few ? kFewRowsSplit : kFewRows;
-  if (small <= large) return kSmallTiles;
+  // the time of a launch of about tiles x per rounds
+  auto mean = [&](double tiles, double per, auto&& time) {
+    const double x = tiles * per, d = std::min(0.16, 0.45 * groups / tiles);
+    return one ? time(x) : (time((1.0 - d) * x) + time(x) + time((1.0 + d) * x)) / 3.0;
+  };
+  const double weights = groups * (double)N * n * (double)kBK * 1e-6;  // MB
+
+  // (with many rounds the tiles' times spread and part of a round is lost at the end)
+  auto small_time = [&](double x) {
+    if (x <= 1.0) return 5.4 + 0.76 * n;
+    const double round = 3.3 + 1.045 * n;
+    if (x >= 6.0) return 2.9 + (0.5 * x + 0.6) * round;
+    const double whole = std::ceil(0.5 * x) - 1.0, left = x - 2.0 * whole;
+    return 2.9 + whole * round + (left <= 1.0 && whole > 0.0 ? 3.5 + 0.85 * n : round - 0.08 * (2.0 - left) * n);
+  };
+  const double small = std::max(mean(token_tiles(128), (double)(N / 128) / 256.0, small_time), weights / 5.1);
+
+  // (the 256 x 256 tiles take their scales in batches of eight contraction blocks)
+  const double tiles_l = token_tiles(256), fill = std::min(1.0, rows / (256.0 * tiles_l)), per_l = (double)((N + 255) / 256) / 256.0;
+  auto round_l = [&](double x) { return 6.3 + (0.78 + 0.16 * fill + 0.14 * std::min(x, 1.0)) * n; };
+  auto large_time = [&](double x) { return 6.5 + (x <= 1.0 ? 1.0 : x < 3.0 ? std::ceil(x) : x + 0.66) * round_l(x); };
+  auto shared_time = [&](double x) {
+    const double whole = std::floor(x), left = x - whole;
+    if (left > 0.5) return 4.0 + large_time(x);
+    if (whole >= 1.0 && left <= 1.0 / 32.0) return 4.0 + 6.5 + whole * round_l(x);
+    const double parts = std::min((double)row_max_split(nkb), std::floor(1.0 / left));
+    return 20.0 + 10.0 * left + 6.5 + whole * round_l(x) + (0.92 + 0.16 * fill) * n / parts;
+  };
+  const double large = nkb < 8 ? 1e30 : std::max(mean(tiles_l, per_l, large_time), weights / 6.7);
+  const double shared = nkb < 8 || !share_last ? 1e30 : std::max(mean(tiles_l, per_l, shared_time), weights / 6.7);
+
+  const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_s = token_tiles(32) * (double)(N / 32);
+  const double few = std::max({4.6 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
+  const double split = b_rows ? 1e30 : std::max({2.6 + 1e-3 * blocks_s * (0.47 * n + 3.6), 3.8 + 0.52 * std::ceil(n / 8.0), weights / 6.8});
+
+  const double tiles = std::min({small, large, shared});
+  if (std::min(few, split) <= tiles) return split < few ? kFewRowsSplit : kFewRows;
+  if (small <= tiles) return kSmallTiles;
+  if (shared <= tiles) return kLargeShared;
   // A workgroup per tile where none would have a second one: the step of grouped_gemm_kernel has no bookkeeping of a stream of
   // tiles (next tile, next scales; with an odd number of steps also the addresses of the stages) and is 1 to 3 % shorter, which
   // counts while power does not bound the launch.  Persistent over this form, 486 launches of at most a round, mean ratio: up to 0.25
-  // rounds 1.01, 0.5 1.02, 0.75 1.04 (the most 1.11), 1 1.02; 1 to 1.5 0.99, 2 0.97, more 0.94 to 0.97.  Where the last round
-  // may share its contraction, up to half a round does (2599 rows, 2560 x 8576: 97 persistent, 89 this form, 79 shared); groups,
-  // whose tiles are only estimated, lose more past a round (8 groups, 1841 rows, 5248 x 7424, 0.92 expected and 1.07 rounds: 131
-  // shared, 163) than the launch that adds the parts costs below (2 to 6 us: 1667 rows, 6656 x 8832 116 -> 108).
-  const bool once = share_last ? rounds_l > 0.5 && rounds_l <= (grouped && E > 1 ? 0.8 : 1.0) : rounds_l <= 1.0;
-  return once ? kLargeOnce : kLargeTiles;
+  // rounds 1.01, 0.5 1.02, 0.75 1.04 (the most 1.11), 1 1.02; 1 to 1.5 0.99, 2 0.97, more 0.94 to 0.97.
+  return tiles_l * per_l <= 1.0 ? kLargeOnce : kLargeTiles;
 }
 // Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
 static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
@@ -1411,7 +1419,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                                         : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, ws != nullptr, g_opt);
   // (output rows of 8 M elements are out of reach of the large tiles' 32-bit offsets)
   const bool once = kernel == kLargeOnce && !b_tile_scaled;
-  const bool large = once || (kernel == kLargeTiles && (b_tile_scaled || ldc < (1LL << 23)));
+  const bool large = once || ((kernel == kLargeTiles || kernel == kLargeShared) && (b_tile_scaled || ldc < (1LL << 23)));
   const int BM = large ? kLargeTile : CfgSmall::BM;
   const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : kLargeTile) : CfgSmall::BN;
   static_assert(CfgWgrad::BM == kLargeTile, "L rows of a large tile");
@@ -1527,7 +1535,7 @@ extern "C" int64_t aamd_grouped_gemm_fp8_ws_bytes(int64_t M, int64_t N, int64_t 
   // (the tiles of groups are counted on the device)
   const int64_t tiles = (M + kLargeTile - 1) / kLargeTile * ((N + kLargeTile - 1) / kLargeTile), left = (tiles + 7) / 8 % 32;
   if (!grouped && (left == 0 || left > 16)) return 0;
-  return choose_nt(M, N, nkb, E, grouped != 0, b_rows != 0, true, GemmOptions()) == kLargeTiles ? kRowPartsBytes : 0;
+  return choose_nt(M, N, nkb, E, grouped != 0, b_rows != 0, true, GemmOptions()) == kLargeShared ? kRowPartsBytes : 0;
 }
 extern "C" int aamd_grouped_gemm_fp8_ws(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
                                         int b_rows, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
