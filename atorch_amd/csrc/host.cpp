@@ -218,6 +218,8 @@ Tensor gemm_nt(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor
               (!b_rows || (b_s.dim() == 3 && b_s.size(1) == N / kTile)),
           "scales do not cover the codes");
   // (codes and scales come as views of one layout; who keeps tensors for a backward may have made one of them dense)
+  require(b_s.is_contiguous() || (!b_tile_scaled && b_s.dim() == 3 && b_s.transpose(1, 2).is_contiguous()),
+          "scales must be dense, in the order of either orientation");
   const Tensor bs = b_rows ? b_s.transpose(1, 2).contiguous() : b_s.contiguous();
   if (goff.has_value()) check_offsets(*goff, E);
   if (bias.has_value()) check_bias(*bias, E, N);

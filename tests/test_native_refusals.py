@@ -120,6 +120,25 @@ def test_linear_and_gemm_sizes_that_do_not_fit():
     _refused(h.offsets_from_tensor, torch.zeros(E, dtype=torch.int32), torch.device("cuda"))
 
 
+def test_gemm_scales_that_are_not_dense():
+    """Dense in either orientation, whichever the codes are in; any other strides are refused, not copied."""
+    h, M, N, K = _host(), 4, 384, 512
+    a, a_s = torch.zeros((M, K), dtype=torch.uint8).view(FP8), torch.ones(M, K // TILE)
+    codes, s = _codes(E, N, K)
+    view, s_view = _codes(E, K, N)[0].transpose(1, 2), torch.ones(E, K // TILE, N // TILE).transpose(1, 2)
+    nt = lambda b, b_s, x_s=a_s: h.gemm_nt(a, x_s, b, b_s, _offsets(), None, BF16, None)  # noqa: E731
+    for b in (codes, view):
+        _sound(nt, b, s)
+        _sound(nt, b, s_view)
+        _refused(nt, b, torch.ones(E, N // TILE, 2 * K // TILE)[..., ::2])
+        _refused(nt, b, torch.ones(2 * E, N // TILE, K // TILE)[::2])
+        _refused(nt, b, torch.ones(N // TILE, E, K // TILE).transpose(0, 1))
+        _refused(nt, b, s, torch.ones(K // TILE, M).t())
+    per_row = torch.ones(E, N, K // TILE)
+    _sound(nt, codes, per_row)
+    _refused(nt, codes, per_row.transpose(1, 2).contiguous().transpose(1, 2))
+
+
 def test_dual_quantisers_with_offsets_of_another_length():
     h, x = _host(), torch.zeros((T, H), dtype=BF16)
     si = torch.zeros(T, dtype=torch.int64)
