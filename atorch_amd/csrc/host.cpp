@@ -10,6 +10,7 @@
 #include <ATen/ops/empty_strided.h>
 #include <ATen/ops/stack.h>
 #include <ATen/ops/zeros.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -199,10 +200,28 @@ std::tuple<Quantised, Tensor> act_dual(const Tensor& fc1, const Tensor& dh, bool
 bool is_transposed_view(const Tensor& b) {
   return b.dim() == 3 && b.size(2) > 1 && b.stride(1) == 1 && b.stride(2) == b.size(1) && b.stride(0) == b.size(1) * b.size(2);
 }
+// Is there memory for `bytes` more without the allocator returning what it holds in reserve, which is what it tries before it
+// reports that there is none?  (A block at hand may be another stream's; an allocator that cannot say is asked.)
+bool memory_at_hand(int64_t bytes, const Tensor& like) {
+  namespace allocator = c10::hip::HIPCachingAllocator;
+  const c10::DeviceIndex device = like.device().index();
+  try {
+    size_t largest = 1;  // (0 would ask the driver too, which takes longer)
+    allocator::cacheInfo(device, &largest);
+    if ((int64_t)largest >= bytes) return true;
+    const auto [free, total] = allocator::get()->getMemoryInfo(device);
+    const int64_t held = allocator::getDeviceStats(device).reserved_bytes[0].current;
+    return (int64_t)free >= bytes && (double)(held + bytes) <= allocator::getMemoryFraction(device) * (double)total;
+  } catch (const c10::Error&) {
+    return true;
+  }
+}
 // Workspace of a GEMM with block-scaled weights; undefined where it has no use for one, or where there is no memory for it.
 Tensor gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t E, bool grouped, bool b_rows, const Tensor& like) {
   const int64_t bytes = aamd_grouped_gemm_fp8_ws_bytes(M, N, K, (int)E, grouped, b_rows);
   if (bytes == 0) return Tensor();
+  on_gpu(like);
+  if (!memory_at_hand(bytes, like)) return Tensor();
   try {
     return empty({bytes / 4}, at::kFloat, like);
   } catch (const c10::OutOfMemoryError&) {
