@@ -372,7 +372,8 @@ class Layer:
             dy = randn((M, N), dev, 1e-2, seed + 2)
             self.qdy, self.sdy, self.qdy_t, self.sdy_t = kernels.tile_quant_dual_grouped(dy, goff, E, blocked=True)
             del dy
-            self.qw, self.sw, self.qw_t, self.sw_t = kernels.block_quant_batched(w, return_transpose=True)
+            # one orientation of the codes, and the view of it that the modules' dgrad reads
+            self.qw, self.sw, self.qw_t, self.sw_t = kernels.block_quant_batched(w, return_transpose=True, written=kernels.STORED)
             self.dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
             self.dw = torch.empty((E, N, K), dtype=torch.float32, device=dev)
         else:

@@ -302,6 +302,8 @@ def test_grouped_gemm_mixtral_full_size(dev):
         ops = _layer_operands(K_, M, Kd, N, E, goff, dev, 10 * i, backward=True)
         _check_nt(K_, ops["qx"], ops["sx"], ops["qw"], ops["sw"], goff, dev, 1)
         _check_nt(K_, ops["qdy"], ops["sdy"], ops["qw_t"], ops["sw_t"], goff, dev, 2)
+        # (the modules keep one orientation of the codes and read its view)
+        _check_nt(K_, ops["qdy"], ops["sdy"], ops["qw"].transpose(1, 2), ops["sw"].transpose(1, 2), goff, dev, 2)
         _check_wgrad(K_, ops, goff, E, N, Kd, dev, 3)
         del ops
         torch.cuda.empty_cache()
@@ -340,6 +342,8 @@ def test_grouped_gemm_qwen_full_size(dev):
         ops = _layer_operands(K_, M, Kd, N, E, goff, dev, 40 + 10 * i, backward=True)
         _check_nt(K_, ops["qx"], ops["sx"], ops["qw"], ops["sw"], goff, dev, 5)
         _check_nt(K_, ops["qdy"], ops["sdy"], ops["qw_t"], ops["sw_t"], goff, dev, 6)
+        # (the modules keep one orientation of the codes and read its view)
+        _check_nt(K_, ops["qdy"], ops["sdy"], ops["qw"].transpose(1, 2), ops["sw"].transpose(1, 2), goff, dev, 6)
         _check_wgrad(K_, ops, goff, E, N, Kd, dev, 7)
         del ops
         torch.cuda.empty_cache()
