@@ -1228,8 +1228,11 @@ static void tile_order(GemmParams& p, int rows, const GemmOptions& g_opt) {
   // panels run over all tokens of an expert and are several times larger (measured: 5 % faster
   // at 4096 tokens per expert and 28672 x 4096 outputs, within 3 % either way elsewhere)
   p.gl = MODE == kRaggedK ? 4 : 8;
-  // group along the side with more tiles per expert (row-ragged launches: batches of 4 R tiles measured 1 % faster
-  // than the L grouping with many small groups, the same with few large ones)
+  // group along the side with more tiles per expert.  256 x 256 tiles, persistent, us, L tiles in groups of 4 / 8 and R tiles in
+  // batches of 2 / 4 / 8 / 16: 32768 rows in 8 groups, 28672 x 4096 3638 / 3592 and 3567 / 3505 / 3512 / 3622, 4096 x 14336 1805 /
+  // 1823 and 1867 / 1793 / 1807 / 1873; along the weights' rows, 4096 x 28672 3670 / 3681 and 3811 / 3666 / 3689 / 3900, 14336 x
+  // 4096 1870 / 1827 and 1835 / 1804 / 1818 / 1843; 65536 uneven rows in 64, 4096 x 7168 1947 / 1993 and 1918 / 1864 / 1877 / 1951;
+  // 131072 in 60, 2816 x 2048 and 2048 x 1408: within 4 %, the noise of the run.
   if (MODE == kRaggedK) p.group_r = p.nRt > p.nLt;
   else p.group_r = p.goff != nullptr && (int64_t)p.nRt * rows * p.E > p.Lrows;
   if (MODE == kRaggedRows && p.group_r) p.gl = 4;
@@ -1256,7 +1259,7 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
 // us, without and with, 4096 outputs, one round of 256 tiles and a last one of 1 / 4 / 8 / 12 / 16 tiles per XCD (in 8 / 8 / 4 / 2 /
 // 2 parts): 48 blocks 148 / 150 / 154 / 157 / 161 -> 123 / 128 / 138 / 149 / 159, 64 blocks 193 / 197 / 203 / 206 / 210 -> 155 /
 // 163 / 170 / 187 / 200, 112 blocks 327 / 337 / 345 / 349 / 354 -> 245 / 256 / 273 / 303 / 322; 32 blocks, 16 tiles 112 -> 122.
-// Where nothing is shared the second launch costs 2 to 4 us of at least 100.
+// Where nothing is shared the second launch costs 2 to 6 us of at least 100 (choose_nt).
 constexpr int kSplitBlocks = 48;
 // The most parts of a contraction: eight blocks at least in each, see row_part.
 static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8); }

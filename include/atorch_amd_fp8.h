@@ -250,9 +250,10 @@ int aamd_grouped_gemm_fp8_nn(const uint8_t *a, int64_t lda, const float *a_s, co
 /*
  * The two GEMMs above (b_rows == 0 as _nt with block scales, else as _nn) with a workspace that lets them share out the
  * contraction of the last output tiles, where fewer of those are left than the card has units.  ws_bytes() says what a
- * launch of this size can use (0: nothing); ws may be NULL, is 16-byte aligned and belongs to the call until it has run on
- * the stream.  The sum of a row in such a tile is made of up to eight partial sums, added in the order of the contraction;
- * which tiles those are depends on the sizes of the groups.
+ * launch of this size can use (0: nothing, or not expected to gain by it); ws may be NULL, is 16-byte aligned and belongs to the
+ * call until it has run on the stream.  The sum of a row in such a tile is made of up to eight partial sums, added in the order
+ * of the contraction.  Which tiles those are depends on the sizes of the groups, so that the last bits of a row may differ with
+ * the other rows of a launch, and between a call with a workspace and one without.
  * Replaces fp8_gemm / fp8_gemm_kernel, triton_kernel.py:143-210, and quantize_op.grouped_qgemm for fprop and dgrad,
  * quantized_grouped_linear.py:141-151, 214-223, as they do.
  */
