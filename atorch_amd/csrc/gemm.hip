@@ -1328,7 +1328,7 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   const double shared = nkb < 8 || !share_last ? 1e30 : std::max(mean(tiles_l, per_l, shared_time), weights / 6.7);
 
   const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_s = token_tiles(32) * (double)(N / 32);
-  const double few = std::max({4.6 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
+  const double few = std::max({4.5 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
   const double split = b_rows ? 1e30 : std::max({2.6 + 1e-3 * blocks_s * (0.47 * n + 3.6), 3.8 + 0.52 * std::ceil(n / 8.0), weights / 6.8});
 
   const double tiles = std::min({small, large, shared});
