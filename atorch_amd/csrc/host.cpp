@@ -484,9 +484,13 @@ struct BlockQuantised {
       s_t = empty({E, K / kTile, N / kTile}, at::kFloat, like);
     }
   }
-  void run(const void* w, at::ScalarType dtype, int64_t first, int64_t E, int64_t stride, double eps) {
+  // goff: only the codes of experts with rows are made
+  void run(const void* w, at::ScalarType dtype, int64_t first, int64_t E, int64_t stride, double eps, const int64_t* goff = nullptr) {
     const int64_t at = first * N * K, at_s = first * (N / kTile) * (K / kTile);
-    if (!q.defined())
+    if (goff != nullptr)
+      check(aamd_quant_128x128_grouped(w, dtype_code(dtype, true), E, N, K, stride, goff, raw<uint8_t>(q), raw<float>(s), raw<uint8_t>(q_t),
+                                       raw<float>(s_t), (float)eps, stream()));
+    else if (!q.defined())
       check(aamd_quant_128x128_t(w, dtype_code(dtype, true), E, N, K, stride, ptr<uint8_t>(q_t) + at, ptr<float>(s_t) + at_s,
                                  (float)eps, stream()));
     else
@@ -501,10 +505,11 @@ struct BlockQuantised {
     return {q, s, q_t, s_t};
   }
 };
-std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose, int one) {
+std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant(const Tensor& w, double eps, bool transpose, int one, const OptTensor& goff) {
   const int64_t E = w.size(0), N = w.size(1), K = w.size(2);
+  if (goff.has_value()) check_offsets(*goff, E);
   BlockQuantised r(E, N, K, transpose, one, w);
-  r.run(ptr(w), w.scalar_type(), 0, E, E > 1 ? w.stride(0) : N * K, eps);
+  r.run(ptr(w), w.scalar_type(), 0, E, E > 1 ? w.stride(0) : N * K, eps, ptr<int64_t>(goff));
   return r.get(transpose);
 }
 // The same from separate tensors of one shape: in one launch where they are equally far apart; else in one launch each or,
@@ -520,7 +525,7 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> block_quant_list(const std::vec
     direct = direct && w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
   }
   const auto at = spaced(ws, N * K);
-  if (!at.has_value() && !direct) return block_quant(at::stack(ws), eps, transpose, one);
+  if (!at.has_value() && !direct) return block_quant(at::stack(ws), eps, transpose, one, {});
   BlockQuantised r(E, N, K, transpose, one, ws[0]);
   if (at.has_value()) r.run(at->base, ws[0].scalar_type(), 0, E, at->stride, eps);
   else
@@ -750,7 +755,8 @@ PYBIND11_MODULE(_host, m) {
     const auto shape = qt_shape(rows, ld_t, blocked);
     return std::vector<int64_t>(shape.begin(), shape.end());
   });
-  m.def("block_quant", &block_quant, py::arg("w"), py::arg("eps"), py::arg("transpose"), py::arg("one") = (int)kBoth);
+  m.def("block_quant", &block_quant, py::arg("w"), py::arg("eps"), py::arg("transpose"), py::arg("one") = (int)kBoth,
+        py::arg("group_offsets") = OptTensor());
   m.def("block_quant_list", &block_quant_list, py::arg("ws"), py::arg("eps"), py::arg("transpose"), py::arg("one") = (int)kBoth);
   m.def("gemm_nt", &gemm_nt);
   m.def("gemm_wgrad", &gemm_wgrad);

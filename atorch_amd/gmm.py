@@ -40,9 +40,10 @@ class _Fp8Gmm(torch.autograd.Function):
         # Codes are written in one orientation: as stored where both products follow, else the forward's.
         both = need_grad or not trans_b
         written = kernels.STORED if need_grad or trans_b else kernels.TURNED
-        quantise = lambda t: kernels.block_quant_batched(b.detach().contiguous(), return_transpose=t, written=written)  # noqa: E731
-        if weight_cache is None:
-            qb, sb, qb_t, sb_t = quantise(both)
+        quantise = lambda t, rows=None: kernels.block_quant_batched(  # noqa: E731
+            b.detach().contiguous(), return_transpose=t, written=written, group_offsets=rows)
+        if weight_cache is None:  # codes for this call alone: experts without rows need none
+            qb, sb, qb_t, sb_t = quantise(both, goff)
         else:
             qb, sb, qb_t, sb_t = weight_cache.codes("b", (b,), is_first_microbatch, both, quantise)
         if trans_b:

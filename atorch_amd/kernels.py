@@ -340,13 +340,15 @@ def gradient_quant_with_sums(x: torch.Tensor, group_offsets: torch.Tensor, num_g
 BOTH, STORED, TURNED = 0, 1, 2
 
 
-def block_quant_batched(w: torch.Tensor, eps: float = 0.0, return_transpose: bool = False, written: int = BOTH):
-    """128x128 block quantisation of ``w [E, N, K]`` in one launch.
+def block_quant_batched(w: torch.Tensor, eps: float = 0.0, return_transpose: bool = False, written: int = BOTH,
+                        group_offsets: Optional[torch.Tensor] = None):
+    """128x128 block quantisation of ``w [E, N, K]`` in one launch; with ``group_offsets`` (int64 ``[E+1]``, on the device) that of
+    the experts that have rows, the others' codes are whatever the memory held.
     Returns ``(q [E,N,K], s [E,N/128,K/128], q_t [E,K,N] | None, s_t [E,K/128,N/128] | None)``.  With
     ``return_transpose``, ``written`` STORED (TURNED) writes only q and s (q_t and s_t), and the other two are their
     transposed views, which ``grouped_gemm_nt`` takes as well."""
     assert w.dim() == 3 and w.stride(2) == 1 and w.stride(1) == w.size(2), "rows of w must be dense"
-    return host().block_quant(w, eps, return_transpose, written if return_transpose else BOTH)
+    return host().block_quant(w, eps, return_transpose, written if return_transpose else BOTH, group_offsets)
 
 
 def grouped_gemm_nt(

@@ -154,6 +154,15 @@ int aamd_quant_128x128_t(const void *w, int w_dtype, int64_t E, int64_t N, int64
                          uint8_t *q_t, float *s_t, float eps, void *stream);
 
 /*
+ * The codes of aamd_quant_128x128 (q and s, q_t and s_t, or both) for the experts that have rows, group_offsets [E+1] int64 on the
+ * device; those of the others, which no product of these groups reads, are left as they are.  For weights that are new in every
+ * call, as in gmm (atorch/kernels/extensions/grouped_gemm_exts/grouped_gemm_gmm.py:10-52).
+ */
+int aamd_quant_128x128_grouped(const void *w, int w_dtype, int64_t E, int64_t N, int64_t K, int64_t expert_stride,
+                               const int64_t *group_offsets, uint8_t *q, float *s, uint8_t *q_t, float *s_t, float eps,
+                               void *stream);
+
+/*
  * Dequantisation y = code * scale.
  * Replaces dequant, triton_kernel.py:49-91.  tile_scale != 0: s [M, N/128]; else s [M/128, N/128].
  */
