@@ -308,6 +308,17 @@ __device__ __forceinline__ void wgrad_short_tiles(const GemmParams& p, uint8_t* 
   }
 }
 
+// Gradients of groups without rows are zeros: workgroup `part` of `parts` writes its share.
+template <typename OUT>
+__device__ __forceinline__ void zero_groups(const GemmParams& p, unsigned long long mask, int part, int parts) {
+  const int64_t bytes = p.Lrows * p.ldc * (int64_t)sizeof(OUT);
+  for (; mask != 0; mask &= mask - 1) {
+    uint8_t* const out = reinterpret_cast<uint8_t*>(reinterpret_cast<OUT*>(p.C) + (int64_t)__builtin_ctzll(mask) * p.c_group_stride);
+    for (int64_t at = ((int64_t)part * blockDim.x + threadIdx.x) * 16; at < bytes; at += (int64_t)parts * blockDim.x * 16)
+      __builtin_nontemporal_store(v4i{0, 0, 0, 0}, reinterpret_cast<v4i*>(out + at));
+  }
+}
+
 // R_ROWS: the R operand as it is stored where its contraction runs down the rows, [contraction, Rrows] (the codes of a
 // weight read for the product with its transpose: one scale per 128x128 block, so that the codes are the same bytes in
 // either orientation).  A step's R tile is then 128 rows of BN bytes, and the fragments are read with
@@ -362,7 +373,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     total_lt = (int)((p.Lrows + BM - 1) / BM);  // kRaggedRows without groups
   }
   const int64_t bid = blockIdx.x;
-  const int64_t xcd = bid % 8, idx = bid / 8;
+  const int64_t xcd = bid % 8, idx = bid / 8 - (MODE == kRaggedK ? p.zeroers / 8 : 0);  // (negative in zeroers, which have no tile)
   const int GL = p.gl;
   int g, lt, rt;
   int kb_lo = 0, kb_hi = 0;  // kRaggedK: the contraction blocks of group g
@@ -388,8 +399,12 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
       if constexpr (NT == 256) if (p.run > 0) {
         // the groups of few blocks leave the list of this loop: behind the long groups' tiles a workgroup takes a run of
         // theirs (and of the groups that the operand buffers do not hold, which are written as NaN)
-        const bool few = live && (gr.t_hi > p.max_kb || (n <= p.short_kb && (n > 0 || !p.accumulate)));
-        const bool none = n == 0 && p.accumulate;  // nothing to add
+        const bool few = live && (gr.t_hi > p.max_kb || (n <= p.short_kb && n > 0));
+        const bool none = n == 0 && gr.t_hi <= p.max_kb;  // nothing to add, or zeros to write
+        if (bid < p.zeroers) {
+          zero_groups<OUT>(p, __ballot(live && none), (int)bid, p.zeroers);
+          return;
+        }
         live = live && !few && !none;
         const int nlong = __popcll(__ballot(live));
         if (turn >= nlong) {
@@ -1360,6 +1375,15 @@ static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
 //   8 groups, 8192 rows, 4096 x 4096 bf16                  221 -> 238 / 227 / 226 / 250, 210     49
 // (the last is where the average rule ends it: from there on both forms are within the noise of each other)
 constexpr int kShortBlocks = 8, kShortAverage = 8, kShortUnits = 1024;
+// Gradients of groups without rows that are written and not added to are zeros, a stream of stores that leaves the matrix cores
+// alone: the launch's first kZeroers workgroups write them beside the tiles of the others, which came before them and left the
+// memory idle.  About 5 TB/s from 64 workgroups on; each takes half a CU from the tiles.  us, tiles of zeros as short ones -> zeroers
+// 32 / 64 / 96 / 128 / 256 / 512 (5 to 10 of the groups have rows):
+//   64 groups, 8192 rows (Zipf), 2048 x 7168 bf16   508 -> 468 / 386 / 355 / 369 / 441 / 484    stream of the outputs 342
+//   the same, all rows in one group                 510 -> 485 / 392 / 358 / 340 / 424 / 478
+//   60 groups, 16001 rows (Zipf), 2816 x 2048 fp32  326 -> 338 / 270 / 276 / 285 / 319 / 345
+// A launch whose groups all have rows sees its zeroers leave at once: 8 groups, 1000 rows, 4096 x 1024 19.4 -> 19.7.
+constexpr int kZeroers = 96;
 static bool use_short_runs(const GemmParams& p) {
   return p.goff != nullptr && p.E <= 64 && p.max_kb <= (int64_t)kShortAverage * p.E &&
          (int64_t)p.E * p.nLt * p.nRt < (1 << 27);
@@ -1593,10 +1617,11 @@ static int wgrad_impl(const uint8_t* dyt, const float* sdyt, const uint8_t* xt, 
   int64_t blocks = (int64_t)E * per_x * 8;
   if (g_opt.tile < 0 && use_short_runs(p)) {
     p.short_kb = kShortBlocks;
+    p.zeroers = accumulate ? 0 : kZeroers;
     p.run = (int)std::min<int64_t>(dw_dtype == AAMD_F32 && !accumulate ? 2 : 4, std::max<int64_t>(1, E * per_g / kShortUnits));
     // long groups have more than short_kb blocks each, so that the operand buffers bound their number
     const int64_t longs = std::min<int64_t>(E, p.max_kb / (p.short_kb + 1));
-    blocks = (longs * per_x + (E * per_g + 8 * p.run - 1) / (8 * p.run)) * 8;
+    blocks = (longs * per_x + (E * per_g + 8 * p.run - 1) / (8 * p.run)) * 8 + p.zeroers;
   }
   return launch_gemm<kRaggedK, true, CfgSmall>(p, dw_dtype, blocks, st, g_opt);
 }
