@@ -64,6 +64,8 @@ SIGNATURES = {
         [_vp, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int, _i64, _vp, _int, _vp],
     ),
     "aamd_quant_grouped_gemm_fits": (_int, [_i64, _i64, _i64, _int, _i64]),
+    "aamd_route_quant_grouped_gemm_fp8_nt": (
+        _int, [_vp, _int, _int, _i64, _vp, _i64, _vp, _vp, _int, _i64, _i64, _vp, _i64, _vp, _int, _vp, _vp, _vp, _vp]),
     "aamd_quant_grouped_gemm_fp8_nt": (
         _int,
         [_int, _vp, _i64, _vp, _int, _i64, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _int, _vp],

@@ -28,8 +28,14 @@ struct FewSource {
   int64_t ld, gate_off;        // elements
   const int64_t* sorted_idx;
   uint32_t topk, T;
+  // Choices: the router's choices of T tokens, at most 64 in all, and where the routing made of them is left
+  const void* ids;
+  int ids_are_i64;
+  int64_t *sorted_out, *goff_out;
+  int32_t* map_out;
 };
-struct Codes {};  // the token rows are codes
+struct Codes {};    // the token rows are codes
+struct Choices {};  // BF16 rows whose routing is made here
 
 // W waves, tiles of 32 WTR weight rows x 32 WTL token rows.  R_ROWS: the weights are stored [contraction, Rrows] and read
 // transposed from the LDS, as in gemm.hip; a block of them is 128 rows of BR bytes there.  That form takes whole cache lines
@@ -42,9 +48,14 @@ struct Codes {};  // the token rows are codes
 // one; here every wave quantises the 128-wide blocks of its own steps, four rows at a time, into its stage while its weights are on
 // their way (one token, four of 60 experts, 2048 wide: quantiser 3.4 + GEMM 7.0 us, activation 2.6 + GEMM 6.0).  The arithmetic is
 // that of quant_1x128_kernel: the same codes.
+//
+// Choices: with at most 64 (token, expert) pairs a lane holds one, and the counting sort of the router preprocess is a loop over them
+// in every wave, a fifth of a microsecond for 8 of them beside the weights' first load, in place of a launch (route_small_kernel 3.1 us).
+// The first workgroup leaves the tables for the launches that follow.
 template <typename OUT, int W, int WTR, int WTL, bool R_ROWS, typename IN = Codes>
 __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, const FewSource src) {
   constexpr bool kQuantise = !std::is_same<IN, Codes>::value;
+  constexpr bool kChoices = std::is_same<IN, Choices>::value, kPermuted = kChoices || std::is_same<IN, BF16>::value;
   constexpr int BL = 32 * WTL, BR = 32 * WTR;
   constexpr int kPitch = BR + 4;  // floats per row of a wave's partial result in the LDS
   constexpr int kStage = (BR + BL) * kBK + (WTL == 1 && !kQuantise ? 0 : BL * 4 + 256);  // weight rows, token rows, scales
@@ -60,10 +71,56 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, co
   // the weights), every XCD a contiguous range
   GroupRanges gr = {};
   int total = (int)((p.Lrows + BL - 1) / BL);
-  if (p.goff != nullptr) {
-    gr = group_ranges<BL>(p.goff, p.E, 0, 0);
+  int choice = -1, order = 0;  // (kChoices) lane i: the expert of pair i, -1 if there is none; the pair of row i
+  auto ranges = [&](int first, int carry) __attribute__((always_inline)) {
+    if constexpr (kChoices) {
+      GroupRanges r;
+      const int e = first + lane;
+      int lo = 0, n = 0;
+      for (int k = 0; k < (int)p.Lrows; k++) {
+        const int other = __builtin_amdgcn_readlane(choice, k);
+        lo += other >= 0 && other < e ? 1 : 0;
+        n += other == e ? 1 : 0;
+      }
+      r.r_lo = lo;
+      r.r_hi = lo + n;
+      n = (n + BL - 1) / BL;
+      r.t_hi = carry + wave_inclusive_sum(n);
+      r.t_lo = r.t_hi - n;
+      r.total = __builtin_amdgcn_readlane(r.t_hi, 63);
+      return r;
+    } else {
+      return group_ranges<BL>(p.goff, p.E, first, carry);
+    }
+  };
+  if constexpr (kChoices) {
+    if (lane < (int)p.Lrows) {
+      const int64_t e = src.ids_are_i64 ? ((const int64_t*)src.ids)[lane] : (int64_t)((const int32_t*)src.ids)[lane];
+      choice = e >= 0 && e < p.E ? (int)e : -1;
+    }
+    int at = 0;  // the row of this lane's pair: rows of an expert keep the order of the pairs
+    for (int k = 0; k < (int)p.Lrows; k++) {
+      const int other = __builtin_amdgcn_readlane(choice, k);
+      at += other >= 0 && (other < choice || (other == choice && k < lane)) ? 1 : 0;
+    }
+    const int rows = __popcll(__ballot(choice >= 0));
+    // (every lane takes part: one that is switched off would receive nothing.  Where lanes have no pair, row 63 is none.)
+    order = __builtin_amdgcn_ds_permute((choice >= 0 ? at : 63) * 4, lane);
+    if (blockIdx.x == 0 && wave == 0) {
+      if (lane < (int)p.Lrows) src.map_out[lane] = choice >= 0 ? at : -1;
+      if (choice >= 0) src.sorted_out[at] = lane;
+      for (int first = 0; first < p.E; first += 64) {
+        const int64_t lo = ranges(first, 0).r_lo;
+        if (first + lane < p.E) src.goff_out[first + lane] = lo;
+      }
+      if (lane == 0) src.goff_out[p.E] = rows;
+    }
+  }
+  const bool grouped = kChoices || p.goff != nullptr;
+  if (grouped) {
+    gr = ranges(0, 0);
     total = gr.total;
-    for (int base = 64; base < p.E; base += 64) total = group_ranges<BL>(p.goff, p.E, base, total).total;
+    for (int base = 64; base < p.E; base += 64) total = ranges(base, total).total;
   }
   const int64_t ntot = (int64_t)total * p.nRt, bid = blockIdx.x;
   if (bid >= ntot) return;
@@ -71,12 +128,12 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, co
   const int64_t pid = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
   int g = 0, rt, lvalid;
   int64_t l0;
-  if (p.goff != nullptr) {
+  if (grouped) {
     g = p.E;
     l0 = 0;
     rt = lvalid = 0;
     for (int base = 0; base < p.E; base += 64) {
-      if (base > 0) gr = group_ranges<BL>(p.goff, p.E, base, gr.total);
+      if (base > 0) gr = ranges(base, gr.total);
       const unsigned long long hit = __ballot(pid >= (int64_t)gr.t_lo * p.nRt && pid < (int64_t)gr.t_hi * p.nRt);
       if (hit != 0) {
         const int src = __builtin_ctzll(hit);
@@ -142,13 +199,16 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, co
   float ls_next = 0.f, rs_next = 0.f;  // (WTL == 1)
   // (kQuantise) the first eight rows are requested with the weights; 16 lanes per row
   constexpr int kAhead = 2;
-  typedef typename std::conditional<kQuantise, IN, BF16>::type Elem;
+  typedef typename std::conditional<kQuantise && !kPermuted, IN, BF16>::type Elem;
   Raw8<Elem> raw[kAhead];
   const int q4 = lane >> 4, q16 = lane & 15;
   auto raw_row = [&](int r) __attribute__((always_inline)) {  // clamped to the rows there are
     const int64_t row = l0 + (r < lvalid ? r : lvalid - 1);
-    if constexpr (std::is_same<IN, BF16>::value) {
-      const uint32_t token = (uint32_t)src.sorted_idx[row] / src.topk;
+    if constexpr (kPermuted) {
+      uint32_t pair;
+      if constexpr (kChoices) pair = (uint32_t)__builtin_amdgcn_ds_bpermute((int)row * 4, order);
+      else pair = (uint32_t)src.sorted_idx[row];
+      const uint32_t token = pair / src.topk;
       return src.rows + (int64_t)(token < src.T ? token : src.T - 1) * src.ld;
     } else {
       return src.rows + row * src.ld;
@@ -319,7 +379,7 @@ static int64_t few_rows_tiles(int64_t M, int E, int rows) {
 template <typename OUT, int W, int WTR, int WTL, bool R_ROWS, typename IN = Codes>
 static int launch_few(GemmParams p, int64_t M, hipStream_t st, const FewSource& src = FewSource()) {
   p.nRt = (int)(p.Rrows / (32 * WTR));
-  const int64_t lt = p.goff ? few_rows_tiles(M, p.E, 32 * WTL) : (M + 32 * WTL - 1) / (32 * WTL);
+  const int64_t lt = p.goff || src.ids ? few_rows_tiles(M, p.E, 32 * WTL) : (M + 32 * WTL - 1) / (32 * WTL);
   const int64_t blocks = lt * p.nRt;
   AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
   few_rows_kernel<OUT, W, WTR, WTL, R_ROWS, IN><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p, src);
@@ -340,10 +400,19 @@ int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, boo
 
 int launch_few_rows_quantising(const GemmParams& p, int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
                                int64_t M, bool split, hipStream_t st) {
-  const FewSource src = {(const u16*)rows, ld, (int64_t)p.nkb * kTile, sorted_idx, (uint32_t)topk, (uint32_t)T};
+  FewSource src = {};
+  src.rows = (const u16*)rows; src.ld = ld; src.gate_off = (int64_t)p.nkb * kTile;
+  src.sorted_idx = sorted_idx; src.topk = (uint32_t)topk; src.T = (uint32_t)T;
   if (what == AAMD_ROWS_PERMUTED) return split ? launch_few<u16, 8, 1, 1, false, BF16>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, BF16>(p, M, st, src);
   if (what == AAMD_ROWS_SWIGLU) return split ? launch_few<u16, 8, 1, 1, false, GLU>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, GLU>(p, M, st, src);
   return split ? launch_few<u16, 8, 1, 1, false, GELU>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, GELU>(p, M, st, src);
+}
+int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i64, const void* rows, int64_t ld, int topk, int64_t T,
+                            int64_t* sorted_idx, int32_t* row_map, int64_t* goff, bool split, hipStream_t st) {
+  FewSource src = {};
+  src.rows = (const u16*)rows; src.ld = ld; src.topk = (uint32_t)topk; src.T = (uint32_t)T;
+  src.ids = ids; src.ids_are_i64 = ids_are_i64; src.sorted_out = sorted_idx; src.map_out = row_map; src.goff_out = goff;
+  return split ? launch_few<u16, 8, 1, 1, false, Choices>(p, p.Lrows, st, src) : launch_few<u16, 4, 2, 2, false, Choices>(p, p.Lrows, st, src);
 }
 
 }  // namespace aamd

@@ -325,7 +325,7 @@ Tensor fp8_gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tenso
 struct Routing {
   Tensor sorted_idx, row_map, goff;
 };
-Routing route(const Tensor& ids, int64_t E, bool want_sorted) {
+Routing alloc_routing(const Tensor& ids, int64_t E, bool want_sorted) {
   // (the kernels read whole words of the ids)
   require((ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt) && ids.is_contiguous(),
           "expert ids must be int64 or int32 and contiguous");
@@ -334,14 +334,18 @@ Routing route(const Tensor& ids, int64_t E, bool want_sorted) {
   if (want_sorted) r.sorted_idx = empty({n}, at::kLong, ids);
   r.row_map = empty({n}, at::kInt, ids);
   r.goff = empty({E + 1}, at::kLong, ids);
+  return r;
+}
+void run_routing(const Routing& r, const Tensor& ids, int64_t E) {
+  const int64_t n = ids.numel();
   // (the one-workgroup form needs no scratch)
   Tensor ws = aamd_route_one_workgroup(n, E) ? Tensor() : empty({std::max<int64_t>(1, aamd_moe_preprocess_ws_ints(n, (int)E))}, at::kInt, ids);
   check(aamd_moe_preprocess(ptr(ids), ids.scalar_type() == at::kLong, n, (int)E, raw<int64_t>(r.sorted_idx), ptr<int32_t>(r.row_map),
                             ptr<int64_t>(r.goff), raw<int32_t>(ws), stream()));
-  return r;
 }
 std::tuple<OptTensor, Tensor, Tensor> moe_preprocess(const Tensor& ids, int64_t E, bool want_sorted) {
-  Routing r = route(ids, E, want_sorted);
+  const Routing r = alloc_routing(ids, E, want_sorted);
+  run_routing(r, ids, E);
   return {opt(r.sorted_idx), r.row_map, r.goff};
 }
 
@@ -547,22 +551,36 @@ void check_mlp(const Tensor& x, const Tensor& q1, const Tensor& q2, const OptTen
   if (b2.has_value()) check_bias(*b2, E, q2.size(1));
 }
 // Quantiser and GEMM in one launch: the output, or nothing where the sizes or operands are not for it (most: rows a group can have).
+bool quant_gemm_fits(const Tensor& rows, int64_t M, int64_t most, const Tensor& q, const Tensor& s) {
+  const int64_t E = q.size(0), N = q.size(1), K = q.size(2);
+  return rows.scalar_type() == at::kBFloat16 && rows.is_contiguous() && q.is_contiguous() && s.is_contiguous() && s.dim() == 3 &&
+         s.size(1) == N / kTile && aamd_quant_grouped_gemm_fits(M, N, K, (int)E, most);
+}
 OptTensor quant_gemm(int what, const Tensor& rows, const OptTensor& sorted_idx, int64_t topk, int64_t M, int64_t most, const Tensor& q,
                      const Tensor& s, const Tensor& goff, const OptTensor& bias) {
   const int64_t E = q.size(0), N = q.size(1), K = q.size(2);
-  if (rows.scalar_type() != at::kBFloat16 || !rows.is_contiguous() || !q.is_contiguous() || !s.is_contiguous() || s.dim() != 3 ||
-      s.size(1) != N / kTile || !aamd_quant_grouped_gemm_fits(M, N, K, (int)E, most))
-    return {};
+  if (!quant_gemm_fits(rows, M, most, q, s)) return {};
   Tensor c = empty({M, N}, at::kBFloat16, rows);
   check(aamd_quant_grouped_gemm_fp8_nt(what, ptr(rows), rows.size(1), ptr<int64_t>(sorted_idx), (int)topk, rows.size(0), ptr<uint8_t>(q),
                                        ptr<float>(s), ptr<int64_t>(goff), (int)E, M, N, K, ptr(c), N, ptr(bias),
                                        bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
   return c;
 }
+// The same of tokens through the router's choices, which makes the routing too.
+OptTensor route_quant_gemm(const Tensor& x, const Tensor& ids, int64_t topk, const Routing& r, const Tensor& q, const Tensor& s,
+                           const OptTensor& bias) {
+  const int64_t E = q.size(0), N = q.size(1), K = q.size(2), T = x.size(0), M = ids.numel();
+  if (E > 1024 || !quant_gemm_fits(x, M, std::min(M, T), q, s)) return {};  // (more experts than a routing takes)
+  Tensor c = empty({M, N}, at::kBFloat16, x);
+  check(aamd_route_quant_grouped_gemm_fp8_nt(ptr(ids), ids.scalar_type() == at::kLong, (int)topk, T, ptr(x), K, ptr<uint8_t>(q), ptr<float>(s),
+                                             (int)E, N, K, ptr(c), N, ptr(bias), bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE,
+                                             ptr<int64_t>(r.sorted_idx), ptr<int32_t>(r.row_map), ptr<int64_t>(r.goff), stream()));
+  return c;
+}
 using MlpResult = std::tuple<Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
 MlpResult mlp_rows(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
                    const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
-                   const OptTensor& b2, bool glu, bool train, bool own_routing) {
+                   const OptTensor& b2, bool glu, bool train, bool own_routing, OptTensor fused) {
   const int64_t E = q1.size(0);
   check_mlp(x, q1, q2, b1, b2, glu);
   check_offsets(goff, E);
@@ -576,9 +594,8 @@ MlpResult mlp_rows(const Tensor& x, const Tensor& goff, const OptTensor& sorted_
   Quantised qx;
   const int64_t ld_t = padded_bound(M, E);
   const int64_t most = own_routing ? std::min(M, x.size(0)) : M;  // (a token goes to an expert once)
-  OptTensor fused;
   // (the indices of a routing made here name a row for every row of a group)
-  if (!train && own_routing) fused = quant_gemm(AAMD_ROWS_PERMUTED, x, sorted_idx, topk, M, most, q1, s1, goff, b1);
+  if (!train && own_routing && !fused.has_value()) fused = quant_gemm(AAMD_ROWS_PERMUTED, x, sorted_idx, topk, M, most, q1, s1, goff, b1);
   if (fused.has_value())
     ;
   else if (train)
@@ -605,7 +622,7 @@ MlpResult mlp_rows(const Tensor& x, const Tensor& goff, const OptTensor& sorted_
 MlpResult mlp_forward(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
                       const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
                       const OptTensor& b2, bool glu, bool train) {
-  return mlp_rows(x, goff, sorted_idx, row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, false);
+  return mlp_rows(x, goff, sorted_idx, row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, false, {});
 }
 
 // The same from the router's choices, routing and weighted combine included: (out, sorted_idx, row_map, goff) and, with
@@ -616,8 +633,11 @@ py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids,
   require(ids.numel() == x.size(0) * topk && probs.dim() == 2 && probs.size(0) == x.size(0) && probs.size(1) == topk &&
               probs.is_contiguous() && q2.size(1) == x.size(1),
           "router weights and choices are [tokens, topk], and the experts return the hidden size");
-  Routing r = route(ids, q1.size(0), true);
-  MlpResult m = mlp_rows(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, true);
+  const Routing r = alloc_routing(ids, q1.size(0), true);
+  OptTensor fc1;
+  if (!train) fc1 = route_quant_gemm(x, ids, topk, r, q1, s1, b1);
+  if (!fc1.has_value()) run_routing(r, ids, q1.size(0));
+  MlpResult m = mlp_rows(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, true, fc1);
   Tensor& y = std::get<0>(m);
   Tensor out = unpermute_combine(y, r.row_map, probs, x.size(0), topk);
   if (!train) return py::make_tuple(out, r.sorted_idx, r.row_map, r.goff);

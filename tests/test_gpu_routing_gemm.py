@@ -1,0 +1,53 @@
+"""The GEMM of few rows that makes the routing itself: the tables of the router preprocess and the bits of the GEMM that reads them, for
+one pair to the most, dropped and repeated choices, more experts than lanes, both forms of the kernel and both id types."""
+import pytest
+import torch
+
+from helpers import randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,k,E,N,K", [(1, 1, 1, 128, 128), (1, 4, 60, 2816, 2048), (16, 4, 64, 256, 384), (64, 1, 3, 512, 640), (8, 8, 64, 2048, 1152),
+                                       (7, 9, 65, 128, 1024), (13, 2, 130, 384, 256), (2, 3, 1024, 128, 128)])  # fmt: skip
+@pytest.mark.parametrize("drop", ["none", "some", "all"])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_tables_and_bits(dev, T, k, E, N, K, drop, dtype):
+    from atorch_amd import _lib, kernels
+
+    M = T * k
+    g = torch.Generator().manual_seed(T + E)
+    ids = torch.randint(E, (T, k), generator=g)
+    if drop != "none":  # (out of range on either side)
+        out = torch.rand((T, k), generator=g) < (0.4 if drop == "some" else 2.0)
+        ids[out] = torch.where(torch.rand(int(out.sum()), generator=g) < 0.5, -1 - E, E)
+    ids = ids.to(dtype).to(dev)
+    q, s, _, _ = kernels.block_quant_batched(randn_bf16((E, N, K), 3, std=0.05).to(dev))
+    bias = torch.randn((E, N), generator=g).to(dev)
+    x = randn_bf16((T, K), 5).to(dev)
+    sorted_idx, row_map, goff = kernels.moe_preprocess(ids, E)
+    n = int(goff[-1])
+    want = torch.full((M + 2, N), 7.0, dtype=torch.bfloat16, device=dev)
+    got, tables = want.clone(), [torch.full_like(t, -9) for t in (sorted_idx, row_map, goff)]
+    args = (E, M, N, K)
+    if n:  # (a row for each index that is not there is not read)
+        sorted_idx[n:] = 0
+    _lib.check(_lib.lib().aamd_quant_grouped_gemm_fp8_nt(
+        0, x.data_ptr(), K, sorted_idx.data_ptr(), k, T, q.data_ptr(), s.data_ptr(), goff.data_ptr(), *args, want.data_ptr(), N,
+        bias.data_ptr(), kernels.dtype_code(bias.dtype), _lib.stream()))  # fmt: skip
+    _lib.check(_lib.lib().aamd_route_quant_grouped_gemm_fp8_nt(
+        ids.data_ptr(), int(dtype == torch.int64), k, T, x.data_ptr(), K, q.data_ptr(), s.data_ptr(), E, N, K, got.data_ptr(), N,
+        bias.data_ptr(), kernels.dtype_code(bias.dtype), *[t.data_ptr() for t in tables], _lib.stream()))  # fmt: skip
+    assert torch.equal(tables[0][:n], sorted_idx[:n]) and torch.all(tables[0][n:] == -9)
+    assert torch.equal(tables[1], row_map) and torch.equal(tables[2], goff)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.all(got[n:] == 7.0)
+
+
+def test_other_sizes_are_refused(dev):
+    from atorch_amd import _lib
+
+    t = torch.zeros(1 << 16, dtype=torch.uint8, device=dev)
+    call = lambda T, k, E: _lib.lib().aamd_route_quant_grouped_gemm_fp8_nt(  # noqa: E731
+        t.data_ptr(), 1, k, T, t.data_ptr(), 128, t.data_ptr(), t.data_ptr(), E, 128, 128, t.data_ptr(), 128, None, _lib.NONE,
+        t.data_ptr(), t.data_ptr(), t.data_ptr(), _lib.stream())  # fmt: skip
+    assert call(65, 1, 2) != 0 and call(13, 5, 2) != 0 and call(0, 1, 2) != 0 and call(1, 1, 1025) != 0 and call(1, 0, 2) != 0
