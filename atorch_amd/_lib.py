@@ -64,6 +64,8 @@ SIGNATURES = {
         [_vp, _i64, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int, _i64, _vp, _int, _vp],
     ),
     "aamd_quant_grouped_gemm_fits": (_int, [_i64, _i64, _i64, _int, _i64]),
+    "aamd_combine_grad_quant_1x128_dual_grouped": (
+        _int, [_vp, _int, _i64, _i64, _vp, _int, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _i64, _int, _vp, _vp]),
     "aamd_route_quant_grouped_gemm_fp8_nt": (
         _int, [_vp, _int, _int, _i64, _vp, _i64, _vp, _vp, _int, _i64, _i64, _vp, _i64, _vp, _int, _vp, _vp, _vp, _vp]),
     "aamd_quant_grouped_gemm_fp8_nt": (
@@ -86,6 +88,7 @@ SIGNATURES = {
     "aamd_unpermute_combine": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _int, _i64, _int, _vp, _vp]),
     "aamd_permute_rows_scaled": (_int, [_vp, _int, _i64, _i64, _vp, _int, _vp, _int, _i64, _vp, _int, _vp]),
     "aamd_unpermute_probs_grad": (_int, [_vp, _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, _vp]),
+    "aamd_unpermute_probs_grad_as": (_int, [_vp, _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, _int, _vp]),
     "aamd_unpermute_backward": (_int, [_vp, _int, _vp, _int, _i64, _i64, _vp, _vp, _int, _i64, _int, _vp, _vp, _vp]),
     "aamd_dual_grouped_with_sums": (
         _int,

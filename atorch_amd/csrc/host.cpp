@@ -658,21 +658,17 @@ std::tuple<Quantised, Tensor> dual_with_sums(int what, const Tensor& x, const Te
   return {r, sums};
 }
 
-// Gradients of the MLP: (dx, dw1, dw2, db1, db2), the last two where asked for.  With topk > 0 the rows were tokens
-// permuted through row_map, and dx goes back to token order as the sum over a token's copies.
-std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> mlp_backward(
-    const Tensor& dy, const Tensor& goff, const OptTensor& row_map, int64_t topk, const Tensor& fc1, const Tensor& qx_t,
-    const Tensor& sx_t, const Tensor& qh_t, const Tensor& sh_t, const Tensor& q1_t, const Tensor& s1_t, const Tensor& q2,
-    const Tensor& s2, bool glu, bool transpose_w1, bool want_b1, bool want_b2, at::ScalarType x_dtype, at::ScalarType w1_dtype,
-    at::ScalarType w2_dtype) {
+// Gradients of the MLP: (dx, dw1, dw2, db1, db2), the last two where asked for, from the codes of the gradient of its output rows (and
+// the sums of these, db2).  With topk > 0 the rows were tokens permuted through row_map, and dx goes back to token order as the sum over
+// a token's copies.
+using MlpGradients = std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor>;
+MlpGradients mlp_gradients(const Quantised& qdy, const Tensor& db2, const Tensor& goff, const OptTensor& row_map, int64_t topk, const Tensor& fc1,
+                           const Tensor& qx_t, const Tensor& sx_t, const Tensor& qh_t, const Tensor& sh_t, const Tensor& q1_t,
+                           const Tensor& s1_t, const Tensor& q2, const Tensor& s2, bool glu, bool transpose_w1, bool want_b1,
+                           at::ScalarType x_dtype, at::ScalarType w1_dtype, at::ScalarType w2_dtype) {
   const int64_t E = goff.numel() - 1, ld_t = qt_ld(qx_t);
-  check_offsets(goff, E);
-  require(dy.size(0) == fc1.size(0) && dy.is_contiguous() && fc1.size(1) == q1_t.size(2) && q2.size(1) * (glu ? 2 : 1) == fc1.size(1),
-          "the gradient, the saved activations and the weights do not fit each other");
-  Quantised qdy, qg;
-  Tensor db1, db2;
-  if (want_b2) std::tie(qdy, db2) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, ld_t, 0.0, at::kBFloat16);
-  else qdy = dual(dy, goff, E, 0.0, ld_t, true, true);
+  Quantised qg;
+  Tensor db1;
   // through the second linear: dh = dy @ w2^T ([M, F]); dw2[f, h] = sum_m h[m, f] dy[m, h]
   Tensor dh = gemm_nt(qdy.q, qdy.s, q2, s2, goff, {}, at::kBFloat16, {});
   Tensor dw2 = gemm_wgrad(qh_t, sh_t, qdy.q_t, qdy.s_t, goff, {}, w2_dtype, false);
@@ -688,6 +684,58 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> mlp_backward(
   Tensor dw1 = transpose_w1 ? gemm_wgrad(qg.q_t, qg.s_t, qx_t, sx_t, goff, {}, w1_dtype, false)
                             : gemm_wgrad(qx_t, sx_t, qg.q_t, qg.s_t, goff, {}, w1_dtype, false);
   return {dx, dw1, dw2, opt(db1), opt(db2)};
+}
+void check_gradients(int64_t M, const Tensor& goff, const Tensor& fc1, const Tensor& q1_t, const Tensor& q2, bool glu) {
+  check_offsets(goff, goff.numel() - 1);
+  require(M == fc1.size(0) && fc1.size(1) == q1_t.size(2) && q2.size(1) * (glu ? 2 : 1) == fc1.size(1),
+          "the gradient, the saved activations and the weights do not fit each other");
+}
+MlpGradients mlp_backward(const Tensor& dy, const Tensor& goff, const OptTensor& row_map, int64_t topk, const Tensor& fc1, const Tensor& qx_t,
+                          const Tensor& sx_t, const Tensor& qh_t, const Tensor& sh_t, const Tensor& q1_t, const Tensor& s1_t,
+                          const Tensor& q2, const Tensor& s2, bool glu, bool transpose_w1, bool want_b1, bool want_b2,
+                          at::ScalarType x_dtype, at::ScalarType w1_dtype, at::ScalarType w2_dtype) {
+  const int64_t E = goff.numel() - 1, ld_t = qt_ld(qx_t);
+  check_gradients(dy.size(0), goff, fc1, q1_t, q2, glu);
+  require(dy.is_contiguous(), "the gradient must be contiguous");
+  Quantised qdy;
+  Tensor db2;
+  if (want_b2) std::tie(qdy, db2) = dual_with_sums(AAMD_SUMS_PLAIN, dy, Tensor(), goff, E, ld_t, 0.0, at::kBFloat16);
+  else qdy = dual(dy, goff, E, 0.0, ld_t, true, true);
+  return mlp_gradients(qdy, db2, goff, row_map, topk, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, glu, transpose_w1, want_b1, x_dtype,
+                       w1_dtype, w2_dtype);
+}
+// From the gradient of the layer's output: (gradients of the MLP, d_probs in the weights' type where asked for).  y: the experts' rows.
+std::tuple<MlpGradients, OptTensor> layer_backward(const Tensor& dout, const Tensor& y, const Tensor& probs, const Tensor& sorted_idx,
+                                                   const Tensor& goff, const Tensor& row_map, int64_t topk, const Tensor& fc1,
+                                                   const Tensor& qx_t, const Tensor& sx_t, const Tensor& qh_t, const Tensor& sh_t,
+                                                   const Tensor& q1_t, const Tensor& s1_t, const Tensor& q2, const Tensor& s2, bool glu,
+                                                   bool transpose_w1, bool want_probs, bool want_b1, bool want_b2,
+                                                   at::ScalarType x_dtype, at::ScalarType w1_dtype, at::ScalarType w2_dtype) {
+  const int64_t E = goff.numel() - 1, ld_t = qt_ld(qx_t), T = dout.size(0), H = dout.size(1), M = T * topk;
+  check_gradients(M, goff, fc1, q1_t, q2, glu);
+  require(dout.is_contiguous() && y.is_contiguous() && y.size(0) == M && y.size(1) == H && probs.is_contiguous() && probs.numel() == M &&
+              row_map.scalar_type() == at::kInt && row_map.is_contiguous() && row_map.numel() == M && sorted_idx.scalar_type() == at::kLong &&
+              sorted_idx.is_contiguous() && sorted_idx.numel() == M,
+          "the gradient and the routing do not fit each other");
+  OptTensor d_probs;
+  if (want_probs) {
+    d_probs = empty(probs.sizes(), probs.scalar_type(), probs);
+    check(aamd_unpermute_probs_grad_as(ptr(dout), dtype_code(dout.scalar_type()), ptr(y), dtype_code(y.scalar_type()), M, H,
+                                       ptr<int32_t>(row_map), T, (int)topk, ptr(*d_probs), dtype_code(probs.scalar_type()), stream()));
+  }
+  Quantised qdy = alloc_dual(M, H, ld_t, true, true, dout);
+  Tensor tiles, db2;
+  if (want_b2) tiles = empty({ld_t / kTile, H}, at::kFloat, dout);
+  check(aamd_combine_grad_quant_1x128_dual_grouped(ptr(dout), dtype_code(dout.scalar_type()), T, H, ptr<int64_t>(sorted_idx), (int)topk, M,
+                                                   ptr(probs), dtype_code(probs.scalar_type()), ptr<int64_t>(goff), (int)E,
+                                                   ptr<uint8_t>(qdy.q), ptr<float>(qdy.s), ptr<uint8_t>(qdy.q_t), ptr<float>(qdy.s_t), ld_t,
+                                                   AAMD_QT_BLOCKED, raw<float>(tiles), stream()));
+  if (want_b2) {
+    db2 = empty({E, H}, at::kBFloat16, dout);
+    check(aamd_group_sums(ptr<float>(tiles), H, ptr<int64_t>(goff), (int)E, ptr(db2), AAMD_BF16, stream()));
+  }
+  return {mlp_gradients(qdy, db2, goff, row_map, topk, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, glu, transpose_w1, want_b1, x_dtype,
+                        w1_dtype, w2_dtype), d_probs};
 }
 
 // ---- the grouped linear ----------------------------------------------------------------------
@@ -801,4 +849,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("mlp_forward", &mlp_forward);
   m.def("mlp_backward", &mlp_backward);
   m.def("layer_forward", &layer_forward);
+  m.def("layer_backward", &layer_backward);
 }

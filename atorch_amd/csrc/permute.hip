@@ -183,7 +183,7 @@ template <typename DT, typename YT>
 __global__ __launch_bounds__(1024) void unpermute_probs_grad_kernel(const typename DT::elem* __restrict__ dout,
                                                                     const typename YT::elem* __restrict__ y, int64_t M,
                                                                     int H8, const int32_t* __restrict__ row_map,
-                                                                    int topk, float* __restrict__ dprobs) {
+                                                                    int topk, void* __restrict__ dprobs, int out_bf16) {
   constexpr bool kYF32 = std::is_same<YT, F32>::value;
   __shared__ int srow[kMaxTopk];
   __shared__ float red[16][kMaxTopk];
@@ -254,7 +254,8 @@ __global__ __launch_bounds__(1024) void unpermute_probs_grad_kernel(const typena
   if ((int)threadIdx.x < topk) {
     float sum = 0.f;
     for (int w = 0; w < nwaves; w++) sum += red[w][threadIdx.x];
-    dprobs[t * topk + threadIdx.x] = sum;
+    if (out_bf16) reinterpret_cast<u16*>(dprobs)[t * topk + threadIdx.x] = (u16)f32_to_bf16_bits(sum);
+    else reinterpret_cast<float*>(dprobs)[t * topk + threadIdx.x] = sum;
   }
 }
 
@@ -959,6 +960,11 @@ extern "C" int aamd_permute_rows_scaled(const void* x, int x_dtype, int64_t T, i
 
 extern "C" int aamd_unpermute_probs_grad(const void* dout, int dout_dtype, const void* y, int y_dtype, int64_t M, int64_t H,
                                          const int32_t* row_map, int64_t T, int topk, float* dprobs, void* stream) {
+  return aamd_unpermute_probs_grad_as(dout, dout_dtype, y, y_dtype, M, H, row_map, T, topk, dprobs, AAMD_F32, stream);
+}
+extern "C" int aamd_unpermute_probs_grad_as(const void* dout, int dout_dtype, const void* y, int y_dtype, int64_t M, int64_t H,
+                                            const int32_t* row_map, int64_t T, int topk, void* dprobs, int dprobs_dtype, void* stream) {
+  AAMD_REQUIRE(dprobs_dtype == AAMD_BF16 || dprobs_dtype == AAMD_F32, "unpermute_probs_grad: unsupported dtype %d of the weights", dprobs_dtype);
   AAMD_REQUIRE((dout_dtype == AAMD_BF16 || dout_dtype == AAMD_F32) && (y_dtype == AAMD_BF16 || y_dtype == AAMD_F32),
                "unpermute_probs_grad: unsupported dtype");
   AAMD_REQUIRE(M >= 0 && H >= 0 && T >= 0 && H % 8 == 0, "unpermute_probs_grad: H=%lld must be a multiple of 8", (long long)H);
@@ -970,20 +976,21 @@ extern "C" int aamd_unpermute_probs_grad(const void* dout, int dout_dtype, const
   if (M == 0) {  // every copy was dropped: no row to read (y may be null)
     const int64_t n = T * topk;
     AAMD_REQUIRE((n + 255) / 256 < 0x7fffffffLL, "unpermute_probs_grad: too large");
-    fill_zero_f32_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(dprobs, n);
+    AAMD_REQUIRE(dprobs_dtype == AAMD_F32, "unpermute_probs_grad: no rows");
+    fill_zero_f32_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>((float*)dprobs, n);
     AAMD_LAUNCH_CHECK("unpermute_probs_grad (clear)");
     return AAMD_OK;
   }
-  const int H8 = (int)(H / 8);
+  const int H8 = (int)(H / 8), out_bf16 = dprobs_dtype == AAMD_BF16;
   dim3 grid((unsigned)T), block((unsigned)threads_for_one_row(H8));
   if (dout_dtype == AAMD_BF16 && y_dtype == AAMD_BF16)
-    unpermute_probs_grad_kernel<BF16, BF16><<<grid, block, 0, st>>>((const u16*)dout, (const u16*)y, M, H8, row_map, topk, dprobs);
+    unpermute_probs_grad_kernel<BF16, BF16><<<grid, block, 0, st>>>((const u16*)dout, (const u16*)y, M, H8, row_map, topk, dprobs, out_bf16);
   else if (dout_dtype == AAMD_F32 && y_dtype == AAMD_BF16)
-    unpermute_probs_grad_kernel<F32, BF16><<<grid, block, 0, st>>>((const float*)dout, (const u16*)y, M, H8, row_map, topk, dprobs);
+    unpermute_probs_grad_kernel<F32, BF16><<<grid, block, 0, st>>>((const float*)dout, (const u16*)y, M, H8, row_map, topk, dprobs, out_bf16);
   else if (dout_dtype == AAMD_F32 && y_dtype == AAMD_F32)
-    unpermute_probs_grad_kernel<F32, F32><<<grid, block, 0, st>>>((const float*)dout, (const float*)y, M, H8, row_map, topk, dprobs);
+    unpermute_probs_grad_kernel<F32, F32><<<grid, block, 0, st>>>((const float*)dout, (const float*)y, M, H8, row_map, topk, dprobs, out_bf16);
   else
-    unpermute_probs_grad_kernel<BF16, F32><<<grid, block, 0, st>>>((const u16*)dout, (const float*)y, M, H8, row_map, topk, dprobs);
+    unpermute_probs_grad_kernel<BF16, F32><<<grid, block, 0, st>>>((const u16*)dout, (const float*)y, M, H8, row_map, topk, dprobs, out_bf16);
   AAMD_LAUNCH_CHECK("unpermute_probs_grad");
   return AAMD_OK;
 }

@@ -229,14 +229,15 @@ __device__ __forceinline__ uint8_t* qt_tile(uint8_t* q_t, int blocked, int64_t c
 // GATHER: row r of the tile is source row src_row[r] of x (the token permute fused in: x is in token order,
 // the outputs in expert-contiguous order); src_row lives in LDS and holds every valid row of the tile.
 // SUMS: the tile's column sums (a bias gradient's share of these 128 tokens) go to tile_sums[pt, column].
-template <typename IN, bool FULL, bool GATHER = false, bool SUMS = false>
+// WEIGHTED (with GATHER): row r is multiplied by row_w[r], which lives in LDS too, and rounded to bf16.
+template <typename IN, bool FULL, bool GATHER = false, bool SUMS = false, bool WEIGHTED = false>
 __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ x, uint32_t ldx, int nt, int64_t m0,
                                           int mvalid, int pt, int kc, uint8_t* __restrict__ q, float* __restrict__ s,
                                           uint8_t* __restrict__ q_t, float* __restrict__ s_t, uint32_t ld_t, int blocked,
                                           float eps, int64_t gate_off, u16* __restrict__ h_out, uint8_t* tile_t,
                                           Divider* cdiv, const uint32_t* src_row = nullptr, const void* lut = nullptr,
-                                          float* __restrict__ tile_sums = nullptr) {
-  const bool plain_div = !kBf16Values<IN> || eps != 0.f;  // see make_scale
+                                          float* __restrict__ tile_sums = nullptr, const float* row_w = nullptr) {
+  const bool plain_div = !(kBf16Values<IN> || WEIGHTED) || eps != 0.f;  // see make_scale
   float (*part)[kTile] = reinterpret_cast<float (*)[kTile]>(tile_t);
   const int64_t cols = (int64_t)nt * kTile;
   const int gr = (int)threadIdx.x >> 4, c = (int)threadIdx.x & 15;
@@ -285,6 +286,15 @@ __device__ __forceinline__ void dual_tile(const typename IN::elem* __restrict__ 
       }
     } else {
       raw[i].get(vi);
+      if constexpr (WEIGHTED) {
+        const float w = FULL || live ? row_w[r] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          const uint32_t pk = pack_bf16x2(vi[j] * w, vi[j + 1] * w);
+          vi[j] = __uint_as_float(pk << 16);
+          vi[j + 1] = __uint_as_float(pk & 0xffff0000u);
+        }
+      }
     }
     if constexpr (kPacked) {
       const v4i pk = pack8_bf16(vi);
@@ -415,15 +425,20 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
 // multiply and a shift: magic = floor(2^sh / topk) + 1 with 2^(sh - 31) >= topk, exact for indices below 2^31)
 // and then runs the tile of the grouped kernel on gathered rows.  Source rows are clamped to the token count,
 // so a corrupt index reads a wrong row, never beyond x.
-template <typename IN>
+// WEIGHTED: the row is bf16(token * probs[flat index]), the combine's gradient with respect to it.  Written by a kernel of its own and
+// read here those rows were a third of the two kernels' traffic (8191 tokens to 4 of 60 experts, 2048 wide, us: both gradients of the
+// combine 56 and the quantiser 59 took 25 more than this and the weights' gradient alone; the training step of that block 1774 -> 1739, of 500 tokens to 2 of 8 238 -> 233).
+template <typename IN, bool WEIGHTED = false, bool SUMS = false>
 __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ sorted_idx,
     uint32_t magic, int sh, uint32_t T, const int64_t* __restrict__ goff, int E, int64_t M,
     uint8_t* __restrict__ q, float* __restrict__ s, uint8_t* __restrict__ q_t, float* __restrict__ s_t, int64_t ld_t,
-    int blocked, float eps) {
+    int blocked, float eps, const void* __restrict__ probs = nullptr, int probs_f32 = 0, uint32_t n_flat = 0,
+    float* __restrict__ tile_sums = nullptr) {
   __shared__ __attribute__((aligned(16))) uint8_t tile_t[kTile * kTLd];
   __shared__ Divider cdiv[kTile];
   __shared__ uint32_t src_row[kTile];
+  __shared__ float row_w[WEIGHTED ? kTile : 1];
   uint32_t bx = blockIdx.x, by = blockIdx.y;  // eight column tiles of a token tile on one XCD: see quant_dual_grouped_kernel
   {
     const uint32_t ntx = gridDim.x, per_row = ntx >> 3;
@@ -444,12 +459,16 @@ __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     const uint32_t flat = (uint32_t)sorted_idx[m0 + (int)threadIdx.x];
     const uint32_t tok = (uint32_t)(((uint64_t)flat * magic) >> sh);
     src_row[threadIdx.x] = tok < T ? tok : T - 1;
+    if constexpr (WEIGHTED) {
+      const uint32_t at = flat < n_flat ? flat : n_flat - 1;
+      row_w[threadIdx.x] = probs_f32 ? reinterpret_cast<const float*>(probs)[at] : bf16_bits_to_f32(reinterpret_cast<const u16*>(probs)[at]);
+    }
   }
   __syncthreads();
   if (mvalid == kTile)
-    dual_tile<IN, true, true>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, 0, nullptr, tile_t, cdiv, src_row);
+    dual_tile<IN, true, true, SUMS, WEIGHTED>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, 0, nullptr, tile_t, cdiv, src_row, nullptr, tile_sums, row_w);
   else
-    dual_tile<IN, false, true>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, 0, nullptr, tile_t, cdiv, src_row);
+    dual_tile<IN, false, true, SUMS, WEIGHTED>(x, (uint32_t)ldx, nt, m0, mvalid, pt, kc, q, s, q_t, s_t, (uint32_t)ld_t, blocked, eps, 0, nullptr, tile_t, cdiv, src_row, nullptr, tile_sums, row_w);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1040,11 +1059,10 @@ static int quant_dual(const void* x, int x_dtype, int64_t M, int64_t cols, int64
   return AAMD_OK;
 }
 
-extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t T, int64_t cols, int64_t ldx,
-                                                     const int64_t* sorted_idx, int topk, int64_t M,
-                                                     const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, uint8_t* q,
-                                                     float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
-                                                     float eps, void* stream) {
+// probs: the rows are weighted
+static int permute_dual(const void* x, int x_dtype, int64_t T, int64_t cols, int64_t ldx, const int64_t* sorted_idx, int topk, int64_t M,
+                        const int64_t* group_offsets, int E, const void* probs, int probs_f32, uint8_t* q, float* s, uint8_t* q_t,
+                        float* s_t, int64_t ld_t, int q_t_layout, float eps, float* tile_sums, void* stream) {
   AAMD_REQUIRE(x_dtype == AAMD_BF16 || x_dtype == AAMD_F32 || x_dtype == AAMD_F16, "permute_quant_dual: unsupported dtype %d", x_dtype);
   AAMD_REQUIRE(q_t_layout == AAMD_QT_ROWS || q_t_layout == AAMD_QT_BLOCKED, "permute_quant_dual: unknown q_t layout %d", q_t_layout);
   AAMD_REQUIRE(T >= 0 && M >= 0 && cols >= 0 && cols % kTile == 0, "permute_quant_dual: cols=%lld must be a multiple of 128",
@@ -1072,14 +1090,43 @@ extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype,
   hipStream_t st = (hipStream_t)stream;
   dim3 grid((unsigned)(cols / kTile), (unsigned)grid_tiles), block(256);
   const int nt = (int)(cols / kTile);
-  if (x_dtype == AAMD_BF16)
-    quant_dual_gather_kernel<BF16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps);
-  else if (x_dtype == AAMD_F16)
-    quant_dual_gather_kernel<F16><<<grid, block, 0, st>>>((const u16*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps);
-  else
-    quant_dual_gather_kernel<F32><<<grid, block, 0, st>>>((const float*)x, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps);
+  auto launch = [&](auto kernel, auto* in) {
+    kernel<<<grid, block, 0, st>>>(in, ldx, nt, sorted_idx, magic, sh, (uint32_t)T, group_offsets, E, M, q, s, q_t, s_t, ld_t, q_t_layout, eps,
+                                   probs, probs_f32, (uint32_t)(T * topk), tile_sums);
+  };
+  if (probs && tile_sums) {
+    if (x_dtype == AAMD_BF16) launch(quant_dual_gather_kernel<BF16, true, true>, (const u16*)x);
+    else launch(quant_dual_gather_kernel<F32, true, true>, (const float*)x);
+  } else if (probs) {
+    if (x_dtype == AAMD_BF16) launch(quant_dual_gather_kernel<BF16, true>, (const u16*)x);
+    else launch(quant_dual_gather_kernel<F32, true>, (const float*)x);
+  } else if (x_dtype == AAMD_BF16) {
+    launch(quant_dual_gather_kernel<BF16>, (const u16*)x);
+  } else if (x_dtype == AAMD_F16) {
+    launch(quant_dual_gather_kernel<F16>, (const u16*)x);
+  } else {
+    launch(quant_dual_gather_kernel<F32>, (const float*)x);
+  }
   AAMD_LAUNCH_CHECK("permute_quant_dual_grouped");
   return AAMD_OK;
+}
+extern "C" int aamd_permute_quant_1x128_dual_grouped(const void* x, int x_dtype, int64_t T, int64_t cols, int64_t ldx,
+                                                     const int64_t* sorted_idx, int topk, int64_t M,
+                                                     const int64_t* group_offsets, int E, int32_t* /*tile_ws*/, uint8_t* q,
+                                                     float* s, uint8_t* q_t, float* s_t, int64_t ld_t, int q_t_layout,
+                                                     float eps, void* stream) {
+  return permute_dual(x, x_dtype, T, cols, ldx, sorted_idx, topk, M, group_offsets, E, nullptr, 0, q, s, q_t, s_t, ld_t, q_t_layout, eps,
+                      nullptr, stream);
+}
+extern "C" int aamd_combine_grad_quant_1x128_dual_grouped(const void* dout, int dtype, int64_t T, int64_t cols, const int64_t* sorted_idx,
+                                                          int topk, int64_t M, const void* probs, int probs_dtype,
+                                                          const int64_t* group_offsets, int E, uint8_t* q, float* s, uint8_t* q_t,
+                                                          float* s_t, int64_t ld_t, int q_t_layout, float* tile_sums, void* stream) {
+  AAMD_REQUIRE(dtype == AAMD_BF16 || dtype == AAMD_F32, "combine_grad_quant_dual: unsupported dtype %d", dtype);
+  AAMD_REQUIRE(probs_dtype == AAMD_BF16 || probs_dtype == AAMD_F32, "combine_grad_quant_dual: unsupported dtype %d of the weights", probs_dtype);
+  AAMD_REQUIRE(probs || T <= 0, "combine_grad_quant_dual: null weights");
+  return permute_dual(dout, dtype, T, cols, cols, sorted_idx, topk, M, group_offsets, E, probs, probs_dtype == AAMD_F32, q, s, q_t, s_t, ld_t,
+                      q_t_layout, 0.f, tile_sums, stream);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -89,11 +89,15 @@ def _mlp_backward(ctx, dy, goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2
         dy, goff, row_map, ctx.dispatch_topk, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, ctx.glu, ctx.transpose_w1,
         ctx.has_b1, ctx.has_b2, x_dtype, w1_dtype, w2_dtype,
     )  # fmt: skip
-    dv1 = None
-    if ctx.has_v1:  # the gate and the up half of the gradient go back to their own parameters
-        dim = 1 if ctx.transpose_w1 else 2
-        dw1, dv1 = (t.contiguous() for t in torch.chunk(dw1, 2, dim=dim))
+    dw1, dv1 = _gate_and_up(ctx, dw1)
     return dx, dw1, dw2, dv1, db1, db2
+
+
+def _gate_and_up(ctx, dw1):
+    """The gate and the up half of the gradient go back to their own parameters."""
+    if not ctx.has_v1:
+        return dw1, None
+    return tuple(t.contiguous() for t in torch.chunk(dw1, 2, dim=1 if ctx.transpose_w1 else 2))
 
 
 class _Fp8ExpertMlp(torch.autograd.Function):
@@ -147,20 +151,18 @@ class _Fp8MoeLayer(torch.autograd.Function):
             ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
             ctx.dtypes = (x.dtype, w1.dtype, w2.dtype)
             ctx.dispatch_topk = topk
-            ctx.save_for_backward(y, probs_c, goff, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2, row_map)
+            ctx.save_for_backward(y, probs_c, sorted_idx, goff, row_map, fc1, qx_t, sx_t, qh_t, sh_t, q1_t, s1_t, q2, s2)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        y, probs, *saved = ctx.saved_tensors
-        row_map = saved[-1]
-        dout = dout.contiguous()
-        d_probs = None
-        if ctx.needs_input_grad[1]:
-            dy, d_probs = kernels.unpermute_backward(dout, y, row_map, probs, ctx.dispatch_topk)
-        else:
-            dy = kernels.permute_rows_scaled(dout, row_map, ctx.dispatch_topk, y.shape[0], probs, y.dtype)
-        dx, dw1, dw2, dv1, db1, db2 = _mlp_backward(ctx, dy, *saved)
+        y, probs, sorted_idx, goff, row_map, *saved = ctx.saved_tensors
+        x_dtype, w1_dtype, w2_dtype = ctx.dtypes
+        (dx, dw1, dw2, db1, db2), d_probs = host().layer_backward(
+            dout.contiguous(), y, probs, sorted_idx, goff, row_map, ctx.dispatch_topk, *saved, ctx.glu, ctx.transpose_w1,
+            ctx.needs_input_grad[1], ctx.has_b1, ctx.has_b2, x_dtype, w1_dtype, w2_dtype,
+        )  # fmt: skip
+        dw1, dv1 = _gate_and_up(ctx, dw1)
         return dx, d_probs, dw1, dw2, dv1, db1, db2, None, None, None, None, None, None
 
 

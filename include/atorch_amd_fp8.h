@@ -134,6 +134,16 @@ int aamd_permute_quant_1x128_dual_grouped(const void *x, int x_dtype, int64_t T,
                                           void *stream);
 
 /*
+ * The same of the combine's gradient with respect to the permuted rows: row j is bf16(dout[sorted_idx[j] / topk] * probs[sorted_idx[j]]),
+ * what aamd_permute_rows_scaled writes for bf16 rows (autograd of token_dispatcher.py:155-159), quantised as aamd_quant_1x128_dual_grouped does (eps 0) without being written.
+ * dout [T, cols] bf16 or fp32, dense; probs [T, topk] bf16 or fp32; tile_sums as in aamd_dual_grouped_with_sums, or NULL.
+ */
+int aamd_combine_grad_quant_1x128_dual_grouped(const void *dout, int dtype, int64_t T, int64_t cols, const int64_t *sorted_idx,
+                                               int topk, int64_t M, const void *probs, int probs_dtype,
+                                               const int64_t *group_offsets, int E, uint8_t *q, float *s, uint8_t *q_t,
+                                               float *s_t, int64_t ld_t, int q_t_layout, float *tile_sums, void *stream);
+
+/*
  * 128x128 block quantisation of E weight matrices, optionally also emitting the
  * transposed codes and scale grid.
  * Replaces block_quant / block_quant_kernel, triton_kernel.py:21-46 (dispatch
@@ -296,7 +306,7 @@ int aamd_quant_grouped_gemm_fp8_nt(int what, const void *rows, int64_t ld, const
 /*
  * The same for permuted rows with the routing made in the launch: ids [T, topk] (int64 or int32, row-major) are the router's choices,
  * T topk at most 64 pairs; c has T topk rows, of which those of pairs with an expert in [0, E) are written.  sorted_idx [T topk],
- * row_map [T topk] and group_offsets [E+1] are outputs, what aamd_moe_preprocess gives.  Worth it where
+ * row_map [T topk] and group_offsets [E+1] are outputs, what aamd_moe_preprocess gives (token_dispatcher.py:89-116).  Worth it where
  * aamd_quant_grouped_gemm_fits(T topk, ...) says so.
  */
 int aamd_route_quant_grouped_gemm_fp8_nt(const void *ids, int ids_are_i64, int topk, int64_t T, const void *rows, int64_t ld,
@@ -365,6 +375,9 @@ int aamd_permute_rows_scaled(const void *x, int x_dtype, int64_t T, int64_t cols
                              void *stream);
 int aamd_unpermute_probs_grad(const void *dout, int dout_dtype, const void *y, int y_dtype, int64_t M, int64_t H,
                               const int32_t *row_map, int64_t T, int topk, float *dprobs, void *stream);
+/* The same in the weights' type (autograd of token_dispatcher.py:156), bf16 or fp32; bf16 needs M > 0. */
+int aamd_unpermute_probs_grad_as(const void *dout, int dout_dtype, const void *y, int y_dtype, int64_t M, int64_t H,
+                                 const int32_t *row_map, int64_t T, int topk, void *dprobs, int dprobs_dtype, void *stream);
 
 /*
  * The dual quantiser of a gradient that also leaves the column sums of its 128-token tiles, and the sums of those over
