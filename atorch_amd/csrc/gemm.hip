@@ -1580,6 +1580,34 @@ extern "C" int aamd_route_quant_grouped_gemm_fp8_nt(const void* ids, int ids_are
                                  (hipStream_t)stream);
 }
 
+// With the combine (few_rows_combine_kernel)?  It saves a launch and its gap, 2.5 us of a step that is queued launch by launch and
+// nothing of one that is replayed, and has a workgroup per token and 32 outputs where the GEMM alone has one per row: what it loses is
+// long chains of steps on few CUs, and weights that several tokens share are read for each.  SwiGLU, us, two launches -> one, both
+// replayed in a graph (E, N, K, topk; T tokens): 60, 2048, 1408, 4: T 1 8.3 -> 9.5, 2 10.7 -> 10.4, 4 15.4 -> 12.9, 8 20.2 -> 21.6;
+// 64, 7168, 2048, 8: T 1 27.7 -> 21.3; 8, 4096, 14336, 2 (14 steps a wave): T 1 23.3 -> 26.8; 8, 1024, 4096, 2: T 1 9.3 -> 9.6, 8 11.3
+// -> 12.3; 16, 4096, 4096, 1: T 1 10.7 -> 8.4, 2 12.2 -> 9.6, 4 17.2 -> 19.0, 8 (16 steps) 21.2 -> 31.0; 16, 7168, 1024, 4: T 1 13.7 ->
+// 9.6.  The block of 60 experts, one token, queued: 19.6 -> 16.6.
+constexpr int64_t kCombineSteps = 8;  // of a wave, over the rounds of workgroups, one per CU
+extern "C" int aamd_quant_grouped_gemm_combine_fits(int64_t T, int topk, int64_t N, int64_t K, int E) {
+  if (T < 1 || T > kQuantisingRows || topk < 1 || topk > 8 || T * topk > kQuantisingRows) return 0;
+  const int64_t per = topk <= 2 ? 8 : topk <= 4 ? 4 : 2, rounds = (T * (N / 32) + 255) / 256;  // (waves per slot: launch_combine)
+  return rounds * ((K / kBK + per - 1) / per) <= kCombineSteps && quantising_kernel(T * topk, N, K, E) == kFewRowsSplit;
+}
+extern "C" int aamd_quant_grouped_gemm_combine_fp8_nt(int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64,
+                                                      const int32_t* row_map, const void* probs, int probs_dtype, int topk, int64_t T,
+                                                      const uint8_t* b, const float* b_s, int E, int64_t N, int64_t K, void* out,
+                                                      const void* bias, int bias_dtype, void* stream) {
+  AAMD_REQUIRE(what == AAMD_ROWS_SWIGLU || what == AAMD_ROWS_GELU, "quant_grouped_gemm_combine: unknown source %d", what);
+  AAMD_REQUIRE(T >= 1 && T <= kQuantisingRows && topk >= 1 && topk <= 8 && T * topk <= kQuantisingRows, "quant_grouped_gemm_combine: bad routing");
+  AAMD_REQUIRE(E >= 1 && N >= kTile && N % kTile == 0 && K >= kBK && K % kBK == 0 && K < (1LL << 23), "quant_grouped_gemm_combine: bad sizes");
+  AAMD_REQUIRE(probs_dtype == AAMD_BF16 || probs_dtype == AAMD_F32, "quant_grouped_gemm_combine: bad type of the router weights");
+  AAMD_REQUIRE(bias == nullptr || bias_dtype == AAMD_BF16 || bias_dtype == AAMD_F32, "quant_grouped_gemm_combine: bad bias dtype");
+  AAMD_REQUIRE(rows && ids && row_map && probs && b && b_s && out, "quant_grouped_gemm_combine: null pointer");
+  AAMD_REQUIRE(ld >= (what == AAMD_ROWS_SWIGLU ? 2 * K : K) && ld % 8 == 0 && aligned16(rows) && aligned16(b), "quant_grouped_gemm_combine: operands must be 16-byte aligned");
+  const GemmParams p = quantising_params(b, b_s, nullptr, E, T * topk, N, K, out, N, bias, bias_dtype);
+  return launch_few_rows_combine(p, what, rows, ld, ids, ids_are_i64, row_map, probs, probs_dtype, topk, T, out, (hipStream_t)stream);
+}
+
 extern "C" int64_t aamd_grouped_gemm_fp8_ws_bytes(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows) {
   const int64_t nkb = K / kBK;
   if (M <= 0 || N <= 0 || E < 1 || nkb < kSplitBlocks) return 0;

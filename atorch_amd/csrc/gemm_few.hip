@@ -34,6 +34,7 @@ struct FewSource {
   int64_t *sorted_out, *goff_out;
   int32_t* map_out;
 };
+constexpr int kCombineWaves = 16, kCombineSlots = 8;  // of few_rows_combine_kernel: the most waves of a workgroup, and slots of a token
 struct Codes {};    // the token rows are codes
 struct Choices {};  // BF16 rows whose routing is made here
 
@@ -413,6 +414,174 @@ int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i6
   src.rows = (const u16*)rows; src.ld = ld; src.topk = (uint32_t)topk; src.T = (uint32_t)T;
   src.ids = ids; src.ids_are_i64 = ids_are_i64; src.sorted_out = sorted_idx; src.map_out = row_map; src.goff_out = goff;
   return split ? launch_few<u16, 8, 1, 1, false, Choices>(p, p.Lrows, st, src) : launch_few<u16, 4, 2, 2, false, Choices>(p, p.Lrows, st, src);
+}
+
+// The second GEMM of a decoding step with the weighted combine in it: out[t] = sum over the slots j of probs[t, j] (b[e_j] act(row_j)),
+// e_j the expert of slot j and row_j its row of `rows`.  A step of one token is a chain of launches of a few microseconds each, and
+// the combine, a gather of topk rows, was the last of them.  A workgroup takes 32 outputs of one token, eight, four or two waves
+// (`per`) for a slot; the blocks of the contraction are dealt to eight sums like those of the eight waves of few_rows_kernel's split
+// form, a wave makes some of these one after the other, two blocks in flight, and they are added in its order, the slots in that of
+// unpermute_combine_kernel: the same bits as of the two launches.  Bound by latency: a wave's steps behind each other, and the fetch of
+// the routing ahead.
+// With 8 or 16 outputs a workgroup, and a step more in flight, every workgroup still quantises all the rows: one token, four of 60
+// experts, 2048 x 1408 the same 9.5 us, two tokens 10.4 -> 16.1; 16 x 4096 x 4096, top-1 8.4 -> 10.5.
+// IN: GLU or GELU.  PD: type of the router weights, and of the output.
+template <typename IN, int PD>
+__global__ __launch_bounds__(1024) void few_rows_combine_kernel(const GemmParams p, const FewSource src, const int32_t* __restrict__ row_map,
+                                                                const void* __restrict__ probs, void* __restrict__ out, int per) {
+#pragma clang fp contract(off)
+  constexpr int BR = 32, kSums = 8, kStages = 2, kLoads = BR / 8, kRaws = std::is_same<IN, GLU>::value ? 2 : 1;
+  constexpr int kCodes = kStages * BR * kBK, kWave = kCodes + 256;  // stages of weight rows, the codes of the token row
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kCombineWaves * kWave];
+  __shared__ __attribute__((aligned(16))) float part[kCombineSlots][kSums][BR];
+  __shared__ float weight[kCombineSlots];
+  __shared__ int expert[kCombineSlots];  // -1: a dropped copy, which adds zeros
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hg = lane >> 5, r8 = lane >> 3, q16 = lane & 15;
+  const int topk = (int)src.topk, slot = wave / per, first = wave - slot * per;
+  const uint32_t t = blockIdx.x / (uint32_t)p.nRt;
+  const int r0 = (int)(blockIdx.x - t * (uint32_t)p.nRt) * BR;
+  const int64_t pair = (int64_t)t * topk + slot, id = src.ids_are_i64 ? ((const int64_t*)src.ids)[pair] : (int64_t)((const int32_t*)src.ids)[pair];
+  const int to = row_map[pair];
+  const float pv = PD == AAMD_BF16 ? bf16_bits_to_f32(reinterpret_cast<const u16*>(probs)[pair]) : reinterpret_cast<const float*>(probs)[pair];
+  const int row = __builtin_amdgcn_readfirstlane(to >= 0 && to < p.Lrows && id >= 0 && id < p.E ? to : -1);
+  const int e = __builtin_amdgcn_readfirstlane(row >= 0 ? (int)id : 0);
+
+  v16f zero;
+#pragma unroll
+  for (int r = 0; r < 16; r++) zero[r] = 0.f;
+  // a lane holds rows 8 q + 4 hg .. + 3 of 32, the same in every column
+  auto keep = [&](int i, const v16f& a) __attribute__((always_inline)) {
+    if (l32 != 0) return;
+#pragma unroll
+    for (int q = 0; q < BR / 8; q++)
+      *reinterpret_cast<v4f*>(&part[slot][i][8 * q + 4 * hg]) = v4f{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+  };
+  if (row >= 0) {
+    uint8_t* const mine = lds + wave * kWave;
+    uint8_t* const codes = mine + kCodes;
+    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)mine;
+    const uint8_t* const Rb = p.R + uniform_i64((int64_t)e * p.r_group_stride + (int64_t)r0 * p.ldr);
+    const float* const rs = p.Rs + (int64_t)e * p.rs_group_stride + (int64_t)(r0 / kTile) * p.rs_row_stride;
+    const u16* const from = src.rows + (int64_t)row * src.ld + q16 * 8;
+    // (16-byte chunks XOR-swizzled as in few_rows_kernel)
+    const uint32_t roff[2] = {(uint32_t)r8 * (uint32_t)p.ldr + (uint32_t)(((lane & 7) ^ r8) << 4),
+                              (uint32_t)r8 * (uint32_t)p.ldr + (uint32_t)(((lane & 7) ^ r8 ^ 1) << 4)};
+    const int r_row = l32 & (BR - 1), sw = (r_row & 7) ^ ((r_row >> 3) & 1);  // (the rows again in the other columns of 32)
+    const int nkb = p.nkb;
+    Raw8<IN> raw, raw_next;
+    float rs_now = 0.f, rs_next = 0.f;
+    uint32_t stage = 0;  // of the block under way
+    constexpr uint32_t kStage = BR * kBK, kRing = kStages * kStage - 1;
+    auto request = [&](int k, uint32_t at) __attribute__((always_inline)) {
+      raw_next.a = *reinterpret_cast<const v4i*>(from + k * kTile);
+      if constexpr (std::is_same<IN, GLU>::value) raw_next.b = *reinterpret_cast<const v4i*>(from + k * kTile + src.gate_off);
+      rs_next = rs[k];
+      const uint8_t* const R = Rb + (int64_t)k * kBK;
+#pragma unroll
+      for (int n = 0; n < BR / 8; n++)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(roff[n & 1]), "s"(R + (int64_t)(n * 8) * p.ldr), "s"(base + at + n * 1024) : "memory");
+    };
+    // the blocks of this wave: those of one sum after the other
+    auto after = [&](int k) __attribute__((always_inline)) {
+      const int next = k + kSums;
+      return next < nkb ? next : (k & (kSums - 1)) + per < kSums && (k & (kSums - 1)) + per < nkb ? (k & (kSums - 1)) + per : nkb;
+    };
+    auto step = [&](int k, v16f& sum) __attribute__((always_inline)) {
+      raw = raw_next;
+      rs_now = rs_next;
+      const int next = after(k);
+      if (next < nkb) {
+        request(next, (stage + kStage) & kRing);
+        // (what was requested behind this block may be on its way)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads + kRaws) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      float v[8];
+      raw.get(v);
+      const Divider d = make_scale(row16_max(amax8(v)), 0.f, false);
+      const v2i c8 = quant8<false>(v, d);
+      if (lane < 16) *reinterpret_cast<v2i*>(codes + q16 * 8) = c8;
+      __builtin_amdgcn_wave_barrier();  // same wave, in-order LDS: the reads below see the writes above
+      auto frag = [&](const uint8_t* at, int h, int x) __attribute__((always_inline)) {
+        const v4i lo = *reinterpret_cast<const v4i*>(at + (((4 * h + 2 * hg) ^ x) << 4));
+        const v4i hi = *reinterpret_cast<const v4i*>(at + (((4 * h + 2 * hg + 1) ^ x) << 4));
+        return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      };
+      v8i rf[2], lf[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        lf[h] = frag(codes, h, 0);  // (the token row in all 32 columns)
+        rf[h] = frag(mine + stage + r_row * kBK, h, sw);
+      }
+      const float sc = d.s * rs_now;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read and may be filled again
+      v16f pr = mfma_fp8_32x32x64(rf[0], lf[0], zero);
+      pr = mfma_fp8_32x32x64(rf[1], lf[1], pr);
+#pragma unroll
+      for (int r = 0; r < 16; r++) sum[r] = __builtin_fmaf(pr[r], sc, sum[r]);
+      stage = (stage + kStage) & kRing;
+    };
+    if (first < nkb) request(first, 0);
+    for (int i = first; i < kSums; i += per) {
+      v16f sum = zero;
+      for (int k = i; k < nkb; k += kSums) step(k, sum);
+      keep(i, sum);
+    }
+  }
+  if (first == 0 && lane == 0) {
+    expert[slot] = row >= 0 ? e : -1;
+    weight[slot] = pv;
+  }
+  __syncthreads();
+  if (tid >= BR) return;
+  float tot[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < kCombineSlots; j++) {
+    if (j >= topk) break;
+    float o = 0.f;
+    if (expert[j] >= 0) {
+      o = part[j][0][tid];
+#pragma unroll
+      for (int w = 1; w < kSums; w++) o += part[j][w][tid];
+      if (p.bias != nullptr) {
+        const int64_t at = (int64_t)expert[j] * p.bias_group_stride + r0 + tid;
+        o += p.bias_dtype == AAMD_F32 ? reinterpret_cast<const float*>(p.bias)[at] : bf16_bits_to_f32(reinterpret_cast<const u16*>(p.bias)[at]);
+      }
+      o = __uint_as_float(pack_bf16x2(o, 0.f) << 16);
+    }
+    float prod = o * weight[j];
+    if constexpr (PD == AAMD_BF16) prod = __uint_as_float(pack_bf16x2(prod, 0.f) << 16);
+    tot[j & 3] = tot[j & 3] + prod;
+  }
+  const float sum = ((tot[0] + tot[1]) + tot[2]) + tot[3];
+  const int64_t at = (int64_t)t * p.ldc + r0 + tid;
+  if constexpr (PD == AAMD_BF16) reinterpret_cast<u16*>(out)[at] = (u16)(pack_bf16x2(sum, 0.f) & 0xffffu);
+  else reinterpret_cast<float*>(out)[at] = sum;
+}
+template <typename IN, int PD>
+static void launch_combine(const GemmParams& p, const FewSource& src, const int32_t* row_map, const void* probs, void* out, hipStream_t st) {
+  const unsigned topk = src.topk, per = topk <= 2 ? 8 : topk <= 4 ? 4 : 2;
+  few_rows_combine_kernel<IN, PD><<<src.T * (unsigned)p.nRt, 64 * per * topk, 0, st>>>(p, src, row_map, probs, out, (int)per);
+}
+int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64, const int32_t* row_map,
+                            const void* probs, int probs_dtype, int topk, int64_t T, void* out, hipStream_t st) {
+  FewSource src = {};
+  src.rows = (const u16*)rows; src.ld = ld; src.gate_off = (int64_t)p.nkb * kTile;
+  src.topk = (uint32_t)topk; src.T = (uint32_t)T; src.ids = ids; src.ids_are_i64 = ids_are_i64;
+  p.nRt = (int)(p.Rrows / 32);
+  AAMD_REQUIRE(T * p.nRt < 0x7fffffffLL, "quant_grouped_gemm_combine: grid too large");
+  if (what == AAMD_ROWS_SWIGLU) {
+    if (probs_dtype == AAMD_BF16) launch_combine<GLU, AAMD_BF16>(p, src, row_map, probs, out, st);
+    else launch_combine<GLU, AAMD_F32>(p, src, row_map, probs, out, st);
+  } else {
+    if (probs_dtype == AAMD_BF16) launch_combine<GELU, AAMD_BF16>(p, src, row_map, probs, out, st);
+    else launch_combine<GELU, AAMD_F32>(p, src, row_map, probs, out, st);
+  }
+  AAMD_LAUNCH_CHECK("grouped_gemm (few rows, combined)");
+  return AAMD_OK;
 }
 
 }  // namespace aamd

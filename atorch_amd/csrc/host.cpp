@@ -577,6 +577,20 @@ OptTensor route_quant_gemm(const Tensor& x, const Tensor& ids, int64_t topk, con
                                              ptr<int64_t>(r.sorted_idx), ptr<int32_t>(r.row_map), ptr<int64_t>(r.goff), stream()));
   return c;
 }
+// Activation, second GEMM and weighted combine of such rows: the tokens, or nothing where it is not for them.
+OptTensor act_gemm_combine(const Tensor& fc1, const Tensor& ids, int64_t topk, const Routing& r, const Tensor& probs, const Tensor& q,
+                           const Tensor& s, const OptTensor& bias, bool glu) {
+  const int64_t E = q.size(0), N = q.size(1), K = q.size(2), M = ids.numel(), T = M / topk;
+  if ((probs.scalar_type() != at::kBFloat16 && probs.scalar_type() != at::kFloat) || !quant_gemm_fits(fc1, M, std::min(M, T), q, s) ||
+      !aamd_quant_grouped_gemm_combine_fits(T, (int)topk, N, K, (int)E))
+    return {};
+  Tensor out = empty({T, N}, probs.scalar_type(), fc1);
+  check(aamd_quant_grouped_gemm_combine_fp8_nt(glu ? AAMD_ROWS_SWIGLU : AAMD_ROWS_GELU, ptr(fc1), fc1.size(1), ptr(ids),
+                                               ids.scalar_type() == at::kLong, ptr<int32_t>(r.row_map), ptr(probs),
+                                               dtype_code(probs.scalar_type()), (int)topk, T, ptr<uint8_t>(q), ptr<float>(s), (int)E, N, K,
+                                               ptr(out), ptr(bias), bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE, stream()));
+  return out;
+}
 using MlpResult = std::tuple<Tensor, OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>;
 MlpResult mlp_rows(const Tensor& x, const Tensor& goff, const OptTensor& sorted_idx, const OptTensor& row_map, int64_t topk,
                    const Tensor& q1, const Tensor& s1, const Tensor& q2, const Tensor& s2, const OptTensor& b1,
@@ -637,6 +651,8 @@ py::tuple layer_forward(const Tensor& x, const Tensor& probs, const Tensor& ids,
   OptTensor fc1;
   if (!train) fc1 = route_quant_gemm(x, ids, topk, r, q1, s1, b1);
   if (!fc1.has_value()) run_routing(r, ids, q1.size(0));
+  else if (OptTensor out = act_gemm_combine(*fc1, ids, topk, r, probs, q2, s2, b2, glu); out.has_value())
+    return py::make_tuple(*out, r.sorted_idx, r.row_map, r.goff);
   MlpResult m = mlp_rows(x, r.goff, r.sorted_idx, r.row_map, topk, q1, s1, q2, s2, b1, b2, glu, train, true, fc1);
   Tensor& y = std::get<0>(m);
   Tensor out = unpermute_combine(y, r.row_map, probs, x.size(0), topk);

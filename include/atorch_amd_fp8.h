@@ -315,6 +315,19 @@ int aamd_route_quant_grouped_gemm_fp8_nt(const void *ids, int ids_are_i64, int t
                                          int32_t *row_map, int64_t *group_offsets, void *stream);
 
 /*
+ * The second GEMM of a decoding step with the weighted combine in it: out[t] = sum over j of probs[t, j] (b[ids[t, j]] act(row_map[t, j]-th
+ * of rows)), `what` AAMD_ROWS_SWIGLU or AAMD_ROWS_GELU of `rows` [T topk, 2K or K] bf16 with row stride ld; row_map [T topk] int32, negative
+ * for a copy that was dropped; probs [T, topk] bf16 or fp32; out [T, N] of the type of probs.  topk at most 8, T topk at most 64.
+ * The results are those of aamd_quant_grouped_gemm_fp8_nt and aamd_unpermute_combine (token_dispatcher.py:119-175), bit for bit, where
+ * _fits() says that it is faster than the two.
+ */
+int aamd_quant_grouped_gemm_combine_fits(int64_t T, int topk, int64_t N, int64_t K, int E);
+int aamd_quant_grouped_gemm_combine_fp8_nt(int what, const void *rows, int64_t ld, const void *ids, int ids_are_i64,
+                                           const int32_t *row_map, const void *probs, int probs_dtype, int topk, int64_t T,
+                                           const uint8_t *b, const float *b_s, int E, int64_t N, int64_t K, void *out,
+                                           const void *bias, int bias_dtype, void *stream);
+
+/*
  * aamd_grouped_gemm_fp8_nt for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): the same arguments without
  * tile_ws.  No counterpart in the reference.  The call allocates and
