@@ -1580,18 +1580,19 @@ extern "C" int aamd_route_quant_grouped_gemm_fp8_nt(const void* ids, int ids_are
                                  (hipStream_t)stream);
 }
 
-// With the combine (few_rows_combine_kernel)?  It saves a launch and its gap, 2.5 us of a step that is queued launch by launch and
-// nothing of one that is replayed, and has a workgroup per token and 32 outputs where the GEMM alone has one per row: what it loses is
-// long chains of steps on few CUs, and weights that several tokens share are read for each.  SwiGLU, us, two launches -> one, both
-// replayed in a graph (E, N, K, topk; T tokens): 60, 2048, 1408, 4: T 1 8.3 -> 9.5, 2 10.7 -> 10.4, 4 15.4 -> 12.9, 8 20.2 -> 21.6;
-// 64, 7168, 2048, 8: T 1 27.7 -> 21.3; 8, 4096, 14336, 2 (14 steps a wave): T 1 23.3 -> 26.8; 8, 1024, 4096, 2: T 1 9.3 -> 9.6, 8 11.3
-// -> 12.3; 16, 4096, 4096, 1: T 1 10.7 -> 8.4, 2 12.2 -> 9.6, 4 17.2 -> 19.0, 8 (16 steps) 21.2 -> 31.0; 16, 7168, 1024, 4: T 1 13.7 ->
-// 9.6.  The block of 60 experts, one token, queued: 19.6 -> 16.6.
-constexpr int64_t kCombineSteps = 8;  // of a wave, over the rounds of workgroups, one per CU
+// With the combine (few_rows_combine_kernel)?  It saves a launch and its gap, 2.5 us of a step that is queued launch by launch, and has a
+// workgroup per token and 32 outputs, one per CU, where the GEMM alone has one per row: what it loses is a second round of them that
+// has many steps, and weights that several tokens share, which are read for each.  SwiGLU, us, two launches -> one, both replayed in a
+// graph (E, N, K, topk; T tokens): 60, 2048, 1408, 4: T 1 8.4 -> 8.0, 2 10.6 -> 8.7, 4 15.3 -> 11.2, 8 (2 rounds of 3 steps) 22.0 ->
+// 19.4; 64, 7168, 2048, 8: T 1 (8 steps) 27.4 -> 22.0; 8, 4096, 14336, 2 (14 steps): T 1 23.7 -> 21.4, 2 40.8 -> 36.8; 8, 1024, 4096, 2:
+// T 1 9.2 -> 7.2, 8 11.5 -> 10.3; 16, 4096, 4096, 1: T 1 10.6 -> 7.4, 4 (2 rounds of 4) 17.1 -> 15.1; 4, 2048, 8192, 2 (8 steps): T 1
+// 14.3 -> 12.6, 4 16.6 -> 17.7, 8 (2 rounds) 21.2 -> 34.7; 8, 7168, 7168, 1 (7 steps): T 1 15.0 -> 11.9, 2 (2 rounds) 15.6 -> 20.0; 64,
+// 512, 512, 8: T 1 7.3 -> 7.7, 8 10.6 -> 8.7.  The block of 60 experts, one token, queued: 19.6 -> 16.5.
+constexpr int64_t kCombineSteps = 8, kCombineStepsOfOneRound = 16;  // of a wave, over the rounds
 extern "C" int aamd_quant_grouped_gemm_combine_fits(int64_t T, int topk, int64_t N, int64_t K, int E) {
   if (T < 1 || T > kQuantisingRows || topk < 1 || topk > 8 || T * topk > kQuantisingRows) return 0;
   const int64_t per = topk <= 2 ? 8 : topk <= 4 ? 4 : 2, rounds = (T * (N / 32) + 255) / 256;  // (waves per slot: launch_combine)
-  return rounds * ((K / kBK + per - 1) / per) <= kCombineSteps && quantising_kernel(T * topk, N, K, E) == kFewRowsSplit;
+  return rounds * ((K / kBK + per - 1) / per) <= (rounds == 1 ? kCombineStepsOfOneRound : kCombineSteps) && quantising_kernel(T * topk, N, K, E) == kFewRowsSplit;
 }
 extern "C" int aamd_quant_grouped_gemm_combine_fp8_nt(int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64,
                                                       const int32_t* row_map, const void* probs, int probs_dtype, int topk, int64_t T,

@@ -423,22 +423,23 @@ int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i6
 // form, a wave makes some of these one after the other, two blocks in flight, and they are added in its order, the slots in that of
 // unpermute_combine_kernel: the same bits as of the two launches.  Bound by latency: a wave's steps behind each other, and the fetch of
 // the routing ahead.
-// With 8 or 16 outputs a workgroup, and a step more in flight, every workgroup still quantises all the rows: one token, four of 60
-// experts, 2048 x 1408 the same 9.5 us, two tokens 10.4 -> 16.1; 16 x 4096 x 4096, top-1 8.4 -> 10.5.
+// A wave quantises four of its blocks at a time, 16 lanes each.  With one at a time, in all lanes alike, the vector unit bound it (us,
+// one token: four of 60 experts, 2048 x 1408 9.5 -> 8.0; two of 8, 1024 x 4096 9.6 -> 7.2), and 8 or 16 outputs per workgroup, which
+// quantise the same rows more often, took longer still.
 // IN: GLU or GELU.  PD: type of the router weights, and of the output.
 template <typename IN, int PD>
 __global__ __launch_bounds__(1024) void few_rows_combine_kernel(const GemmParams p, const FewSource src, const int32_t* __restrict__ row_map,
                                                                 const void* __restrict__ probs, void* __restrict__ out, int per) {
 #pragma clang fp contract(off)
-  constexpr int BR = 32, kSums = 8, kStages = 2, kLoads = BR / 8, kRaws = std::is_same<IN, GLU>::value ? 2 : 1;
-  constexpr int kCodes = kStages * BR * kBK, kWave = kCodes + 256;  // stages of weight rows, the codes of the token row
+  constexpr int BR = 32, kSums = 8, kStages = 2, kBatch = 4;
+  constexpr int kCodes = kStages * BR * kBK, kWave = kCodes + kBatch * kBK + 256;  // stages of weight rows, codes and scales of the token row
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kCombineWaves * kWave];
   __shared__ __attribute__((aligned(16))) float part[kCombineSlots][kSums][BR];
   __shared__ float weight[kCombineSlots];
   __shared__ int expert[kCombineSlots];  // -1: a dropped copy, which adds zeros
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, hg = lane >> 5, r8 = lane >> 3, q16 = lane & 15;
+  const int l32 = lane & 31, hg = lane >> 5, r8 = lane >> 3, q4 = lane >> 4, q16 = lane & 15;
   const int topk = (int)src.topk, slot = wave / per, first = wave - slot * per;
   const uint32_t t = blockIdx.x / (uint32_t)p.nRt;
   const int r0 = (int)(blockIdx.x - t * (uint32_t)p.nRt) * BR;
@@ -461,6 +462,7 @@ __global__ __launch_bounds__(1024) void few_rows_combine_kernel(const GemmParams
   if (row >= 0) {
     uint8_t* const mine = lds + wave * kWave;
     uint8_t* const codes = mine + kCodes;
+    float* const scales = reinterpret_cast<float*>(codes + kBatch * kBK);
     const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)mine;
     const uint8_t* const Rb = p.R + uniform_i64((int64_t)e * p.r_group_stride + (int64_t)r0 * p.ldr);
     const float* const rs = p.Rs + (int64_t)e * p.rs_group_stride + (int64_t)(r0 / kTile) * p.rs_row_stride;
@@ -468,15 +470,12 @@ __global__ __launch_bounds__(1024) void few_rows_combine_kernel(const GemmParams
     // (16-byte chunks XOR-swizzled as in few_rows_kernel)
     const uint32_t roff[2] = {(uint32_t)r8 * (uint32_t)p.ldr + (uint32_t)(((lane & 7) ^ r8) << 4),
                               (uint32_t)r8 * (uint32_t)p.ldr + (uint32_t)(((lane & 7) ^ r8 ^ 1) << 4)};
-    const int r_row = l32 & (BR - 1), sw = (r_row & 7) ^ ((r_row >> 3) & 1);  // (the rows again in the other columns of 32)
+    const int sw = (l32 & 7) ^ ((l32 >> 3) & 1);
     const int nkb = p.nkb;
-    Raw8<IN> raw, raw_next;
     float rs_now = 0.f, rs_next = 0.f;
     uint32_t stage = 0;  // of the block under way
     constexpr uint32_t kStage = BR * kBK, kRing = kStages * kStage - 1;
     auto request = [&](int k, uint32_t at) __attribute__((always_inline)) {
-      raw_next.a = *reinterpret_cast<const v4i*>(from + k * kTile);
-      if constexpr (std::is_same<IN, GLU>::value) raw_next.b = *reinterpret_cast<const v4i*>(from + k * kTile + src.gate_off);
       rs_next = rs[k];
       const uint8_t* const R = Rb + (int64_t)k * kBK;
 #pragma unroll
@@ -486,25 +485,32 @@ __global__ __launch_bounds__(1024) void few_rows_combine_kernel(const GemmParams
     // the blocks of this wave: those of one sum after the other
     auto after = [&](int k) __attribute__((always_inline)) {
       const int next = k + kSums;
-      return next < nkb ? next : (k & (kSums - 1)) + per < kSums && (k & (kSums - 1)) + per < nkb ? (k & (kSums - 1)) + per : nkb;
+      return k >= nkb ? nkb : next < nkb ? next : (k & (kSums - 1)) + per < kSums && (k & (kSums - 1)) + per < nkb ? (k & (kSums - 1)) + per : nkb;
     };
-    auto step = [&](int k, v16f& sum) __attribute__((always_inline)) {
-      raw = raw_next;
-      rs_now = rs_next;
-      const int next = after(k);
-      if (next < nkb) {
-        request(next, (stage + kStage) & kRing);
-        // (what was requested behind this block may be on its way)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads + kRaws) : "memory");
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
+    // the token row's codes of four blocks, 16 lanes each
+    auto quantise = [&](int k) __attribute__((always_inline)) {
+      const int k1 = after(k), k2 = after(k1), k3 = after(k2), theirs = q4 == 0 ? k : q4 == 1 ? k1 : q4 == 2 ? k2 : k3;
+      const u16* const at = from + (theirs < nkb ? theirs : k) * kTile;
+      Raw8<IN> raw;
+      raw.a = *reinterpret_cast<const v4i*>(at);
+      if constexpr (std::is_same<IN, GLU>::value) raw.b = *reinterpret_cast<const v4i*>(at + src.gate_off);
       float v[8];
       raw.get(v);
       const Divider d = make_scale(row16_max(amax8(v)), 0.f, false);
       const v2i c8 = quant8<false>(v, d);
-      if (lane < 16) *reinterpret_cast<v2i*>(codes + q16 * 8) = c8;
-      __builtin_amdgcn_wave_barrier();  // same wave, in-order LDS: the reads below see the writes above
+      *reinterpret_cast<v2i*>(codes + q4 * kBK + q16 * 8) = c8;
+      if (q16 == 0) scales[q4] = d.s;
+      __builtin_amdgcn_wave_barrier();  // same wave, in-order LDS: later reads see the writes
+    };
+    int in_batch = 0;
+    auto step = [&](int k, v16f& sum) __attribute__((always_inline)) {
+      rs_now = rs_next;
+      const int next = after(k);
+      if (next < nkb) request(next, (stage + kStage) & kRing);
+      if (in_batch == 0) quantise(k);
+      // (what was requested behind this block may be on its way)
+      if (next < nkb) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(BR / 8) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       auto frag = [&](const uint8_t* at, int h, int x) __attribute__((always_inline)) {
         const v4i lo = *reinterpret_cast<const v4i*>(at + (((4 * h + 2 * hg) ^ x) << 4));
         const v4i hi = *reinterpret_cast<const v4i*>(at + (((4 * h + 2 * hg + 1) ^ x) << 4));
@@ -513,10 +519,11 @@ __global__ __launch_bounds__(1024) void few_rows_combine_kernel(const GemmParams
       v8i rf[2], lf[2];
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        lf[h] = frag(codes, h, 0);  // (the token row in all 32 columns)
-        rf[h] = frag(mine + stage + r_row * kBK, h, sw);
+        lf[h] = frag(codes + in_batch * kBK, h, 0);  // (the token row in all 32 columns)
+        rf[h] = frag(mine + stage + l32 * kBK, h, sw);
       }
-      const float sc = d.s * rs_now;
+      const float sc = scales[in_batch] * rs_now;
+      in_batch = (in_batch + 1) & (kBatch - 1);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read and may be filled again
       v16f pr = mfma_fp8_32x32x64(rf[0], lf[0], zero);
       pr = mfma_fp8_32x32x64(rf[1], lf[1], pr);

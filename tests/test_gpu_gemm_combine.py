@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,k,E,N,K", [(1, 1, 1, 128, 128), (1, 4, 60, 2048, 1408), (3, 2, 8, 384, 1152), (8, 8, 64, 256, 640), (5, 3, 7, 128, 2176),
-                                       (64, 1, 3, 128, 256), (2, 5, 65, 512, 384), (9, 7, 1024, 128, 1280), (10, 6, 16, 256, 128)])  # fmt: skip
+                                       (64, 1, 3, 128, 256), (2, 5, 65, 512, 384), (9, 7, 1024, 128, 1280), (10, 6, 16, 256, 128), (1, 2, 4, 256, 15360)])  # fmt: skip
 @pytest.mark.parametrize("drop", ["none", "some", "all"])
 @pytest.mark.parametrize("glu", [True, False])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
