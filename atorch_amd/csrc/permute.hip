@@ -213,21 +213,22 @@ __global__ __launch_bounds__(1024) void unpermute_probs_grad_kernel(const typena
         unpack8(*reinterpret_cast<const v4i*>(dout + t * H + (int64_t)c * 8), a);
       }
       v4i raw[8][kYF32 ? 2 : 1];
+      int row[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) {
         // the row is the same in every lane (scalar base + lane offset); slots past topk and dropped copies are
         // skipped by a branch the whole wave takes
-        const int r = j0 + u < topk ? __builtin_amdgcn_readfirstlane(srow[j0 + u < topk ? j0 + u : 0]) : -1;
-        const v4i* src = reinterpret_cast<const v4i*>(y + (int64_t)(r < 0 ? 0 : r) * H + (int64_t)c * 8);
+        row[u] = j0 + u < topk ? __builtin_amdgcn_readfirstlane(srow[j0 + u < topk ? j0 + u : 0]) : -1;
+        const v4i* src = reinterpret_cast<const v4i*>(y + (int64_t)(row[u] < 0 ? 0 : row[u]) * H + (int64_t)c * 8);
 #pragma unroll
         for (int w = 0; w < (kYF32 ? 2 : 1); w++) {
-          if (r >= 0) raw[u][w] = __builtin_nontemporal_load(src + w);
+          if (row[u] >= 0) raw[u][w] = __builtin_nontemporal_load(src + w);
           else raw[u][w] = v4i{0, 0, 0, 0};
         }
       }
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        if (j0 + u >= topk) break;
+        if (row[u] < 0) continue;  // (not zeros times the gradient, which may be infinite)
         float b[8];
         if constexpr (kYF32) {
 #pragma unroll

@@ -48,3 +48,48 @@ def test_bits_of_the_separate_kernels(dev, T, k, E, H, dt, pd, drop):
         dout.data_ptr(), kernels.dtype_code(dt), y.data_ptr(), _lib.BF16, M, H, row_map.data_ptr(), T, k, d_probs.data_ptr(),
         kernels.dtype_code(pd), _lib.stream()))  # fmt: skip
     assert torch.equal(d_probs, want) or (torch.isnan(d_probs) == torch.isnan(want)).all()
+
+
+@pytest.mark.parametrize("dt,yt", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16), (torch.float32, torch.float32),
+                                   (torch.bfloat16, torch.float32)])  # fmt: skip
+@pytest.mark.parametrize("k", [1, 3, 8, 11])
+def test_a_dropped_copy_has_no_gradient(dev, dt, yt, k):
+    """Whatever its token's gradient holds: nothing is multiplied for a slot without a row."""
+    from atorch_amd import kernels
+
+    T, H, M = 9, 136, 9 * k
+    g = torch.Generator().manual_seed(k)
+    row_map = torch.randperm(M, generator=g).int()
+    row_map[torch.rand(M, generator=g) < 0.5] = -1
+    dout, y = torch.randn((T, H), generator=g).to(dt).to(dev), torch.randn((M, H), generator=g).to(yt).to(dev)
+    dout[2], dout[4, 7], dout[5, 130] = float("inf"), float("-inf"), float("nan")
+    row_map = row_map.to(dev)
+    got = kernels.unpermute_probs_grad(dout, y, row_map, k)
+    dropped = (row_map < 0).view(T, k)
+    assert dropped[[2, 4, 5]].any() and torch.all(got[dropped] == 0)
+    rows = y.float()[row_map.long().clamp(min=0)].view(T, k, H)
+    want = torch.where(dropped, 0.0, (rows * dout.float()[:, None]).sum(-1))
+    # (sums of 136 products of about 1 in two orders)
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4, equal_nan=True)
+
+
+@pytest.mark.parametrize("pd", [torch.bfloat16, torch.float32])
+def test_layer_with_dropped_copies_and_a_gradient_that_is_not_finite(dev, pd):
+    """Expert ids out of range: the router weights' gradient is 0 there, and the layer's own unfused path (a shared expert that adds
+    nothing) gives the same one."""
+    from atorch_amd.moe_layer import Grouped_GEMM_MoE
+
+    T, H, F, E, k = 96, 256, 128, 4, 2
+    torch.manual_seed(3)
+    layer = Grouped_GEMM_MoE(H, F, 0.0, E, k, use_swiglu=True, implementation_type="Megatron", device=dev, dtype=torch.bfloat16)
+    ids = torch.stack([torch.randperm(E)[:k] for _ in range(T)])
+    ids[::3, 1], ids[1::5, 0] = E, -1
+    x, dout = randn_bf16((T, H), 4).to(dev), torch.randn(T, H).to(pd).to(dev)
+    dout[0], dout[1, 3], dout[6, 9] = float("inf"), float("-inf"), float("nan")
+    grads = []
+    for kw in ({}, dict(se_fn1=lambda h: h, se_fn2=lambda h: torch.zeros_like(h))):
+        probs = torch.full((T, k), 0.5, dtype=pd, device=dev, requires_grad=True)
+        layer(x, probs, ids.to(dev), **kw).backward(dout)
+        grads.append(probs.grad)
+    assert torch.all(grads[0][(ids < 0) | (ids >= E)] == 0)
+    torch.testing.assert_close(grads[0], grads[1], rtol=0, atol=0, equal_nan=True)
