@@ -69,6 +69,7 @@ SIGNATURES = {
     "aamd_quant_grouped_gemm_fits": (_int, [_i64, _i64, _i64, _int, _i64]),
     "aamd_combine_grad_quant_1x128_dual_grouped": (
         _int, [_vp, _int, _i64, _i64, _vp, _int, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _i64, _int, _vp, _vp]),
+    "aamd_route_quant_grouped_gemm_fits": (_int, [_i64, _int, _i64, _i64, _int]),
     "aamd_route_quant_grouped_gemm_fp8_nt": (
         _int, [_vp, _int, _int, _i64, _vp, _i64, _vp, _vp, _int, _i64, _i64, _vp, _i64, _vp, _int, _vp, _vp, _vp, _vp]),
     "aamd_quant_grouped_gemm_fp8_nt": (

@@ -1518,6 +1518,10 @@ static NtKernel quantising_kernel(int64_t M, int64_t N, int64_t K, int E) {
   if (M < 1 || M > kQuantisingRows || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || K >= (1LL << 23)) return kSmallTiles;
   return choose_nt(M, N, K / kBK, E, true, false, false, GemmOptions());
 }
+// Workgroups of the few-rows kernel over their places, where every row may have its own group.
+static double few_rows_rounds(int64_t M, int64_t N, int E, NtKernel kernel) {
+  return std::max(1.0, (double)((M < E ? M : E) * (N / (kernel == kFewRows ? 64 : 32))) / 512.0);
+}
 // Worth it?  It saves a launch of 3 to 4 us and puts a tenth of a microsecond into every step of every round of workgroups, four
 // rows of a group at a time; from the ninth row on the rows of a step are fetched when their turn comes.  A block of experts,
 // SwiGLU, us, with both of its quantisers as launches -> in the GEMMs (E, H, F, k; T tokens): 60, 2048, 1408, 4: T 1 30.1 -> 22.3,
@@ -1527,10 +1531,9 @@ static NtKernel quantising_kernel(int64_t M, int64_t N, int64_t K, int E) {
 extern "C" int aamd_quant_grouped_gemm_fits(int64_t M, int64_t N, int64_t K, int E, int64_t most) {
   const NtKernel kernel = quantising_kernel(M, N, K, E);
   if (kernel != kFewRows && kernel != kFewRowsSplit) return 0;
-  const int64_t groups = M < E ? M : E, nkb = K / kBK;
-  const int waves = kernel == kFewRows ? 4 : 8, rows = kernel == kFewRows ? 64 : 32;
-  const double rounds = std::max(1.0, (double)(groups * (N / rows)) / 512.0);
-  return most <= 8 && rounds * (double)((nkb + waves - 1) / waves) <= 24.0;
+  const int64_t nkb = K / kBK;
+  const int waves = kernel == kFewRows ? 4 : 8;
+  return most <= 8 && few_rows_rounds(M, N, E, kernel) * (double)((nkb + waves - 1) / waves) <= 24.0;
 }
 static GemmParams quantising_params(const uint8_t* b, const float* b_s, const int64_t* group_offsets, int E, int64_t M, int64_t N,
                                     int64_t K, void* c, int64_t ldc, const void* bias, int bias_dtype) {
@@ -1560,8 +1563,20 @@ extern "C" int aamd_quant_grouped_gemm_fp8_nt(int what, const void* rows, int64_
   const GemmParams p = quantising_params(b, b_s, group_offsets, E, M, N, K, c, ldc, bias, bias_dtype);
   return launch_few_rows_quantising(p, what, rows, ld, sorted_idx, topk, T, M, kernel == kFewRowsSplit, (hipStream_t)stream);
 }
-// From the router's choices (aamd_quant_grouped_gemm_fits, with M = T topk).  One token through four of 60 experts of 2048 and 1408,
-// the whole block: routing as a launch 23.4 -> here 20.0 us.
+// From the router's choices.  It saves the routing's launch, 3 us and its gap, and puts 0.3 us into every round of workgroups, which look
+// among the choices for their pairs before they know their weights.  Routing and GEMM, replayed in a graph, us, two launches -> one
+// (E, N, K, topk; T tokens): 60, 2816, 2048, 4: T 1 9.1 -> 6.7, 8 29.2 -> 27.8; 64, 2816, 2048, 8: T 8 (5.5 rounds) 41.6 -> 39.9; 512,
+// 1024, 2048, 8: T 8 41.6 -> 24.7; 1024, 512, 1024, 8: T 8 29.0 -> 9.9; 60, 16384, 512, 6: T 2 (6) 27.8 -> 27.3; past the line 32, 16384,
+// 512, 4: T 4 (8) 31.2 -> 30.9; 16, 28672, 1024, 4: T 2 (7) 39.7 -> 40.3; 32, 28672, 512, 4: T 3 (10.5) 42.8 -> 44.2; 32, 16384, 512, 6: T
+// 8 (16) 51.3 -> 54.3.  (With a sort of the pairs in every wave, a loop over them for every 64 experts, 64 pairs took up to four times as
+// long as with the launch: the block of 1024 experts 54 -> 228.)
+constexpr double kRouteRounds = 6.0;
+extern "C" int aamd_route_quant_grouped_gemm_fits(int64_t T, int topk, int64_t N, int64_t K, int E) {
+  if (T < 1 || topk < 1 || T > kQuantisingRows || topk > kQuantisingRows || T * topk > kQuantisingRows || E > 1024) return 0;
+  const int64_t M = T * topk;
+  return aamd_quant_grouped_gemm_fits(M, N, K, E, T) &&  // (a token goes to an expert once)
+         few_rows_rounds(M, N, E, quantising_kernel(M, N, K, E)) <= kRouteRounds;
+}
 extern "C" int aamd_route_quant_grouped_gemm_fp8_nt(const void* ids, int ids_are_i64, int topk, int64_t T, const void* rows, int64_t ld,
                                                     const uint8_t* b, const float* b_s, int E, int64_t N, int64_t K, void* c, int64_t ldc,
                                                     const void* bias, int bias_dtype, int64_t* sorted_idx, int32_t* row_map,

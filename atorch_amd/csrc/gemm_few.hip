@@ -38,6 +38,27 @@ constexpr int kCombineWaves = 16, kCombineSlots = 8;  // of few_rows_combine_ker
 struct Codes {};    // the token rows are codes
 struct Choices {};  // BF16 rows whose routing is made here
 
+// The tables of the router preprocess from the experts of the pairs, one to a lane (-1: none), and their places inside an expert.
+template <int W>
+__device__ __forceinline__ void leave_routing(const GemmParams& p, const FewSource& src, int choice, int place, int wave, int lane) {
+  auto below = [&](uint32_t e) __attribute__((always_inline)) {  // pairs of experts below e
+    int n = 0;
+    for (int k = 0; k < (int)p.Lrows; k += 8)
+#pragma unroll
+      for (int u = 0; u < 8; u++) n += (uint32_t)__builtin_amdgcn_readlane(choice, k + u) < e ? 1 : 0;  // (no expert: above all)
+    return n;
+  };
+  if (wave == W - 1) {
+    const int row = below((uint32_t)choice) + place;
+    if (lane < (int)p.Lrows) src.map_out[lane] = choice >= 0 ? row : -1;
+    if (choice >= 0) src.sorted_out[row] = lane;
+  }
+  for (int first = wave * 64; first <= p.E; first += 64 * W) {
+    const int n = below((uint32_t)(first + lane));
+    if (first + lane <= p.E) src.goff_out[first + lane] = n;
+  }
+}
+
 // W waves, tiles of 32 WTR weight rows x 32 WTL token rows.  R_ROWS: the weights are stored [contraction, Rrows] and read
 // transposed from the LDS, as in gemm.hip; a block of them is 128 rows of BR bytes there.  That form takes whole cache lines
 // of a row, 128 weight rows x 32 token rows (us, 64 and 32 weight rows x 64 and 32 token rows, 128 x 32 with three waves, with
@@ -50,9 +71,10 @@ struct Choices {};  // BF16 rows whose routing is made here
 // their way (one token, four of 60 experts, 2048 wide: quantiser 3.4 + GEMM 7.0 us, activation 2.6 + GEMM 6.0).  The arithmetic is
 // that of quant_1x128_kernel: the same codes.
 //
-// Choices: with at most 64 (token, expert) pairs a lane holds one, and the counting sort of the router preprocess is a loop over them
-// in every wave, a fifth of a microsecond for 8 of them beside the weights' first load, in place of a launch (route_small_kernel 3.1 us).
-// The first workgroup leaves the tables for the launches that follow.
+// Choices: with at most 64 (token, expert) pairs a lane holds one, and a workgroup needs no sort to find its tile: a few ballots name
+// the pairs of every lane's expert, the first of which stands for the group, and count the rows before the group's.  They cost the same
+// for any number of pairs and a few instructions more for twice the experts, in every wave of every workgroup, in place of a launch
+// (route_small_kernel 3.1 us) and of a look at its tables.  The first workgroup leaves the tables for the launches that follow.
 template <typename OUT, int W, int WTR, int WTL, bool R_ROWS, typename IN = Codes>
 __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, const FewSource src) {
   constexpr bool kQuantise = !std::is_same<IN, Codes>::value;
@@ -72,81 +94,68 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, co
   // the weights), every XCD a contiguous range
   GroupRanges gr = {};
   int total = (int)((p.Lrows + BL - 1) / BL);
-  int choice = -1, order = 0;  // (kChoices) lane i: the expert of pair i, -1 if there is none; the pair of row i
-  auto ranges = [&](int first, int carry) __attribute__((always_inline)) {
-    if constexpr (kChoices) {
-      GroupRanges r;
-      const int e = first + lane;
-      int lo = 0, n = 0;
-      for (int k = 0; k < (int)p.Lrows; k++) {
-        const int other = __builtin_amdgcn_readlane(choice, k);
-        lo += other >= 0 && other < e ? 1 : 0;
-        n += other == e ? 1 : 0;
-      }
-      r.r_lo = lo;
-      r.r_hi = lo + n;
-      n = (n + BL - 1) / BL;
-      r.t_hi = carry + wave_inclusive_sum(n);
-      r.t_lo = r.t_hi - n;
-      r.total = __builtin_amdgcn_readlane(r.t_hi, 63);
-      return r;
-    } else {
-      return group_ranges<BL>(p.goff, p.E, first, carry);
-    }
-  };
+  int choice = -1, place = 0;  // (kChoices) lane i: the expert of pair i, -1 if there is none, and its place among the expert's pairs
   if constexpr (kChoices) {
     if (lane < (int)p.Lrows) {
       const int64_t e = src.ids_are_i64 ? ((const int64_t*)src.ids)[lane] : (int64_t)((const int32_t*)src.ids)[lane];
       choice = e >= 0 && e < p.E ? (int)e : -1;
     }
-    int at = 0;  // the row of this lane's pair: rows of an expert keep the order of the pairs
-    for (int k = 0; k < (int)p.Lrows; k++) {
-      const int other = __builtin_amdgcn_readlane(choice, k);
-      at += other >= 0 && (other < choice || (other == choice && k < lane)) ? 1 : 0;
+    unsigned long long same = __ballot(choice >= 0);  // the pairs of this lane's expert
+    for (int b = 0; (p.E - 1) >> b != 0; b++) {
+      const bool on = (choice >> b) & 1;
+      const unsigned long long with = __ballot(on);
+      same &= on ? with : ~with;
     }
-    const int rows = __popcll(__ballot(choice >= 0));
-    // (every lane takes part: one that is switched off would receive nothing.  Where lanes have no pair, row 63 is none.)
-    order = __builtin_amdgcn_ds_permute((choice >= 0 ? at : 63) * 4, lane);
-    if (blockIdx.x == 0 && wave == 0) {
-      if (lane < (int)p.Lrows) src.map_out[lane] = choice >= 0 ? at : -1;
-      if (choice >= 0) src.sorted_out[at] = lane;
-      for (int first = 0; first < p.E; first += 64) {
-        const int64_t lo = ranges(first, 0).r_lo;
-        if (first + lane < p.E) src.goff_out[first + lane] = lo;
-      }
-      if (lane == 0) src.goff_out[p.E] = rows;
+    place = __popcll(same & ((1ull << lane) - 1ull));
+    if (blockIdx.x == 0) {
+      leave_routing<W>(p, src, choice, place, wave, lane);
+      return;
     }
-  }
-  const bool grouped = kChoices || p.goff != nullptr;
-  if (grouped) {
-    gr = ranges(0, 0);
+    const int n = choice >= 0 && place == 0 ? (__popcll(same) + BL - 1) / BL : 0;
+    gr.t_hi = wave_inclusive_sum(n);
+    gr.t_lo = gr.t_hi - n;
+    total = __builtin_amdgcn_readlane(gr.t_hi, 63);
+  } else if (p.goff != nullptr) {
+    gr = group_ranges<BL>(p.goff, p.E, 0, 0);
     total = gr.total;
-    for (int base = 64; base < p.E; base += 64) total = ranges(base, total).total;
+    for (int base = 64; base < p.E; base += 64) total = group_ranges<BL>(p.goff, p.E, base, total).total;
   }
-  const int64_t ntot = (int64_t)total * p.nRt, bid = blockIdx.x;
+  const int64_t ntot = (int64_t)total * p.nRt, bid = (int64_t)blockIdx.x - (kChoices ? 1 : 0);
   if (bid >= ntot) return;
   const int64_t per = ntot / 8, rem = ntot % 8, xcd = bid % 8, idx = bid / 8;
   const int64_t pid = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
-  int g = 0, rt, lvalid;
+  int g = 0, rt, lvalid, order = 0, order_at = 0;  // (kChoices) lane i: the i-th pair of the group; that of the tile's first row
   int64_t l0;
-  if (grouped) {
+  if (kChoices || p.goff != nullptr) {
     g = p.E;
     l0 = 0;
     rt = lvalid = 0;
     for (int base = 0; base < p.E; base += 64) {
-      if (base > 0) gr = ranges(base, gr.total);
+      if constexpr (!kChoices) if (base > 0) gr = group_ranges<BL>(p.goff, p.E, base, gr.total);
       const unsigned long long hit = __ballot(pid >= (int64_t)gr.t_lo * p.nRt && pid < (int64_t)gr.t_hi * p.nRt);
       if (hit != 0) {
-        const int src = __builtin_ctzll(hit);
-        const int t_lo = __builtin_amdgcn_readlane(gr.t_lo, src), nl = __builtin_amdgcn_readlane(gr.t_hi, src) - t_lo;
-        const int64_t r_lo = readlane_i64(gr.r_lo, src), r_hi = readlane_i64(gr.r_hi, src);
+        const int at = __builtin_ctzll(hit);
+        const int t_lo = __builtin_amdgcn_readlane(gr.t_lo, at), nl = __builtin_amdgcn_readlane(gr.t_hi, at) - t_lo;
+        int64_t r_lo, r_hi;
+        if constexpr (kChoices) {
+          g = __builtin_amdgcn_readlane(choice, at);
+          r_lo = __popcll(__ballot(choice >= 0 && choice < g));
+          r_hi = r_lo + __popcll(__ballot(choice == g));
+          // (every lane takes part: one that is switched off would receive nothing.  Where lanes are not of the group, pair 63 is none.)
+          order = __builtin_amdgcn_ds_permute((choice == g ? place : 63) * 4, lane);
+        } else {
+          g = base + at;
+          r_lo = readlane_i64(gr.r_lo, at);
+          r_hi = readlane_i64(gr.r_hi, at);
+        }
         const uint32_t pe = (uint32_t)(pid - (int64_t)t_lo * p.nRt);
         rt = (int)(pe / (uint32_t)nl);
-        l0 = r_lo + (int64_t)(pe - (uint32_t)rt * (uint32_t)nl) * BL;
+        order_at = (int)(pe - (uint32_t)rt * (uint32_t)nl) * BL;
+        l0 = r_lo + order_at;
         lvalid = r_hi - l0 < BL ? (int)(r_hi - l0) : BL;
-        g = base + src;
         break;
       }
+      if constexpr (kChoices) break;
     }
     if (g >= p.E) return;
   } else {
@@ -204,10 +213,11 @@ __global__ __launch_bounds__(64 * W) void few_rows_kernel(const GemmParams p, co
   Raw8<Elem> raw[kAhead];
   const int q4 = lane >> 4, q16 = lane & 15;
   auto raw_row = [&](int r) __attribute__((always_inline)) {  // clamped to the rows there are
-    const int64_t row = l0 + (r < lvalid ? r : lvalid - 1);
+    const int in_tile = r < lvalid ? r : lvalid - 1;
+    const int64_t row = l0 + in_tile;
     if constexpr (kPermuted) {
       uint32_t pair;
-      if constexpr (kChoices) pair = (uint32_t)__builtin_amdgcn_ds_bpermute((int)row * 4, order);
+      if constexpr (kChoices) pair = (uint32_t)__builtin_amdgcn_ds_bpermute((order_at + in_tile) * 4, order);
       else pair = (uint32_t)src.sorted_idx[row];
       const uint32_t token = pair / src.topk;
       return src.rows + (int64_t)(token < src.T ? token : src.T - 1) * src.ld;
@@ -381,7 +391,7 @@ template <typename OUT, int W, int WTR, int WTL, bool R_ROWS, typename IN = Code
 static int launch_few(GemmParams p, int64_t M, hipStream_t st, const FewSource& src = FewSource()) {
   p.nRt = (int)(p.Rrows / (32 * WTR));
   const int64_t lt = p.goff || src.ids ? few_rows_tiles(M, p.E, 32 * WTL) : (M + 32 * WTL - 1) / (32 * WTL);
-  const int64_t blocks = lt * p.nRt;
+  const int64_t blocks = lt * p.nRt + (std::is_same<IN, Choices>::value ? 1 : 0);
   AAMD_REQUIRE(blocks < 0x7fffffffLL, "grouped_gemm: grid too large");
   few_rows_kernel<OUT, W, WTR, WTL, R_ROWS, IN><<<dim3((unsigned)blocks), dim3(64 * W), 0, st>>>(p, src);
   AAMD_LAUNCH_CHECK("grouped_gemm (few rows)");

@@ -570,7 +570,7 @@ OptTensor quant_gemm(int what, const Tensor& rows, const OptTensor& sorted_idx, 
 OptTensor route_quant_gemm(const Tensor& x, const Tensor& ids, int64_t topk, const Routing& r, const Tensor& q, const Tensor& s,
                            const OptTensor& bias) {
   const int64_t E = q.size(0), N = q.size(1), K = q.size(2), T = x.size(0), M = ids.numel();
-  if (E > 1024 || !quant_gemm_fits(x, M, std::min(M, T), q, s)) return {};  // (more experts than a routing takes)
+  if (!aamd_route_quant_grouped_gemm_fits(T, (int)topk, N, K, (int)E) || !quant_gemm_fits(x, M, std::min(M, T), q, s)) return {};
   Tensor c = empty({M, N}, at::kBFloat16, x);
   check(aamd_route_quant_grouped_gemm_fp8_nt(ptr(ids), ids.scalar_type() == at::kLong, (int)topk, T, ptr(x), K, ptr<uint8_t>(q), ptr<float>(s),
                                              (int)E, N, K, ptr(c), N, ptr(bias), bias.has_value() ? dtype_code(bias->scalar_type()) : AAMD_NONE,

@@ -307,8 +307,9 @@ int aamd_quant_grouped_gemm_fp8_nt(int what, const void *rows, int64_t ld, const
  * The same for permuted rows with the routing made in the launch: ids [T, topk] (int64 or int32, row-major) are the router's choices,
  * T topk at most 64 pairs; c has T topk rows, of which those of pairs with an expert in [0, E) are written.  sorted_idx [T topk],
  * row_map [T topk] and group_offsets [E+1] are outputs, what aamd_moe_preprocess gives (token_dispatcher.py:89-116).  Worth it where
- * aamd_quant_grouped_gemm_fits(T topk, ...) says so.
+ * _fits() says so.
  */
+int aamd_route_quant_grouped_gemm_fits(int64_t T, int topk, int64_t N, int64_t K, int E);
 int aamd_route_quant_grouped_gemm_fp8_nt(const void *ids, int ids_are_i64, int topk, int64_t T, const void *rows, int64_t ld,
                                          const uint8_t *b, const float *b_s, int E, int64_t N, int64_t K, void *c,
                                          int64_t ldc, const void *bias, int bias_dtype, int64_t *sorted_idx,

@@ -51,3 +51,52 @@ def test_other_sizes_are_refused(dev):
         t.data_ptr(), 1, k, T, t.data_ptr(), 128, t.data_ptr(), t.data_ptr(), E, 128, 128, t.data_ptr(), 128, None, _lib.NONE,
         t.data_ptr(), t.data_ptr(), t.data_ptr(), _lib.stream())  # fmt: skip
     assert call(65, 1, 2) != 0 and call(13, 5, 2) != 0 and call(0, 1, 2) != 0 and call(1, 1, 1025) != 0 and call(1, 0, 2) != 0
+
+
+@pytest.mark.parametrize("T,k,E,N,K", [(8, 8, 1024, 512, 1024), (8, 8, 256, 1024, 2048), (8, 4, 60, 2816, 2048)])
+def test_no_slower_than_the_routing_as_a_launch(dev, T, k, E, N, K):
+    """For many pairs and experts too (a sort in every wave took two to four times as long as both launches); the rule says yes here."""
+    from atorch_amd import _lib, kernels
+
+    M, lib = T * k, _lib.lib()
+    assert lib.aamd_route_quant_grouped_gemm_fits(T, k, N, K, E)
+    g = torch.Generator().manual_seed(1)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(dev)
+    x, c = randn_bf16((T, K), 5).to(dev), torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    q, s = torch.zeros((E, N, K), dtype=torch.uint8, device=dev), torch.ones((E, N // 128, K // 128), device=dev)
+    tables = [torch.empty_like(t) for t in kernels.moe_preprocess(ids, E)]
+
+    def two():
+        sorted_idx, _, goff = kernels.moe_preprocess(ids, E)
+        _lib.check(lib.aamd_quant_grouped_gemm_fp8_nt(0, x.data_ptr(), K, sorted_idx.data_ptr(), k, T, q.data_ptr(), s.data_ptr(), goff.data_ptr(), E,
+                                                      M, N, K, c.data_ptr(), N, None, _lib.NONE, _lib.stream()))  # fmt: skip
+
+    def one():
+        _lib.check(lib.aamd_route_quant_grouped_gemm_fp8_nt(ids.data_ptr(), 1, k, T, x.data_ptr(), K, q.data_ptr(), s.data_ptr(), E, N, K, c.data_ptr(),
+                                                            N, None, _lib.NONE, *[t.data_ptr() for t in tables], _lib.stream()))  # fmt: skip
+
+    def us(f):
+        f()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                f()
+        times = []
+        for _ in range(7):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return sorted(times)[3]
+
+    assert us(one) < 1.15 * us(two)  # (0.34 to 0.95 as measured)
+
+
+def test_many_rounds_keep_the_launch(dev):
+    from atorch_amd import _lib
+
+    fits = _lib.lib().aamd_route_quant_grouped_gemm_fits
+    assert not fits(8, 6, 16384, 512, 32) and not fits(65, 1, 256, 256, 4) and not fits(1, 1, 256, 256, 1025) and not fits(0, 1, 256, 256, 4)
