@@ -1565,12 +1565,13 @@ extern "C" int aamd_quant_grouped_gemm_fp8_nt(int what, const void* rows, int64_
 }
 // From the router's choices.  It saves the routing's launch, 3 us and its gap, and puts 0.3 us into every round of workgroups, which look
 // among the choices for their pairs before they know their weights.  Routing and GEMM, replayed in a graph, us, two launches -> one
-// (E, N, K, topk; T tokens): 60, 2816, 2048, 4: T 1 9.1 -> 6.7, 8 29.2 -> 27.8; 64, 2816, 2048, 8: T 8 (5.5 rounds) 41.6 -> 39.9; 512,
-// 1024, 2048, 8: T 8 41.6 -> 24.7; 1024, 512, 1024, 8: T 8 29.0 -> 9.9; 60, 16384, 512, 6: T 2 (6) 27.8 -> 27.3; past the line 32, 16384,
-// 512, 4: T 4 (8) 31.2 -> 30.9; 16, 28672, 1024, 4: T 2 (7) 39.7 -> 40.3; 32, 28672, 512, 4: T 3 (10.5) 42.8 -> 44.2; 32, 16384, 512, 6: T
-// 8 (16) 51.3 -> 54.3.  (With a sort of the pairs in every wave, a loop over them for every 64 experts, 64 pairs took up to four times as
+// (E, N, K, topk; T tokens): 60, 2816, 2048, 4: T 1 9.1 -> 6.7, 8 29.2 -> 27.8; 512, 1024, 2048, 8: T 8 41.6 -> 24.7; 1024, 512, 1024,
+// 8: T 8 29.0 -> 9.9; 60, 16384, 512, 6: T 2 (6 rounds) 27.8 -> 27.3; 16, 28672, 1024, 4: T 2 (7) 39.7 -> 40.3; 32, 28672, 512, 4: T 3
+// (10.5) 42.8 -> 44.2; 32, 16384, 512, 6: T 8 (16) 51.3 -> 54.3.  Other weights and choices in every launch (from memory): of 78 draws of
+// two to five rounds none slower by 0.3 us and half of them faster by 2; 64, 6144, 1536, 8: T 4 (6) 51.6 -> 52.8; 64, 28672, 1024, 2: T 4
+// (7) 49.0 -> 50.4.  (With a sort of the pairs in every wave, a loop over them for every 64 experts, 64 pairs took up to four times as
 // long as with the launch: the block of 1024 experts 54 -> 228.)
-constexpr double kRouteRounds = 6.0;
+constexpr double kRouteRounds = 5.0;
 extern "C" int aamd_route_quant_grouped_gemm_fits(int64_t T, int topk, int64_t N, int64_t K, int E) {
   if (T < 1 || topk < 1 || T > kQuantisingRows || topk > kQuantisingRows || T * topk > kQuantisingRows || E > 1024) return 0;
   const int64_t M = T * topk;
