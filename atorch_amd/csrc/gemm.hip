@@ -1518,9 +1518,9 @@ static NtKernel quantising_kernel(int64_t M, int64_t N, int64_t K, int E) {
   if (M < 1 || M > kQuantisingRows || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || K >= (1LL << 23)) return kSmallTiles;
   return choose_nt(M, N, K / kBK, E, true, false, false, GemmOptions());
 }
-// Workgroups of the few-rows kernel over their places, where every row may have its own group.
-static double few_rows_rounds(int64_t M, int64_t N, int E, NtKernel kernel) {
-  return std::max(1.0, (double)((M < E ? M : E) * (N / (kernel == kFewRows ? 64 : 32))) / 512.0);
+// Workgroups of `rows` weight rows over the places of 512, where every row may have its own group.
+static double few_rows_rounds(int64_t M, int64_t N, int E, int rows) {
+  return std::max(1.0, (double)((M < E ? M : E) * (N / rows)) / 512.0);
 }
 // Worth it?  It saves a launch of 3 to 4 us and puts a tenth of a microsecond into every step of every round of workgroups, four
 // rows of a group at a time; from the ninth row on the rows of a step are fetched when their turn comes.  A block of experts,
@@ -1532,8 +1532,8 @@ extern "C" int aamd_quant_grouped_gemm_fits(int64_t M, int64_t N, int64_t K, int
   const NtKernel kernel = quantising_kernel(M, N, K, E);
   if (kernel != kFewRows && kernel != kFewRowsSplit) return 0;
   const int64_t nkb = K / kBK;
-  const int waves = kernel == kFewRows ? 4 : 8;
-  return most <= 8 && few_rows_rounds(M, N, E, kernel) * (double)((nkb + waves - 1) / waves) <= 24.0;
+  const int waves = kernel == kFewRows ? 4 : 8, rows = kernel == kFewRows ? 64 : 32;
+  return most <= 8 && few_rows_rounds(M, N, E, rows) * (double)((nkb + waves - 1) / waves) <= 24.0;
 }
 static GemmParams quantising_params(const uint8_t* b, const float* b_s, const int64_t* group_offsets, int E, int64_t M, int64_t N,
                                     int64_t K, void* c, int64_t ldc, const void* bias, int bias_dtype) {
@@ -1571,12 +1571,12 @@ extern "C" int aamd_quant_grouped_gemm_fp8_nt(int what, const void* rows, int64_
 // two to five rounds none slower by 0.3 us and half of them faster by 2; 64, 6144, 1536, 8: T 4 (6) 51.6 -> 52.8; 64, 28672, 1024, 2: T 4
 // (7) 49.0 -> 50.4.  (With a sort of the pairs in every wave, a loop over them for every 64 experts, 64 pairs took up to four times as
 // long as with the launch: the block of 1024 experts 54 -> 228.)
-constexpr double kRouteRounds = 5.0;
+constexpr double kRouteRounds = 5.0;  // (of 64 weight rows to a workgroup, also where the form of 32 is taken)
 extern "C" int aamd_route_quant_grouped_gemm_fits(int64_t T, int topk, int64_t N, int64_t K, int E) {
   if (T < 1 || topk < 1 || T > kQuantisingRows || topk > kQuantisingRows || T * topk > kQuantisingRows || E > 1024) return 0;
   const int64_t M = T * topk;
   return aamd_quant_grouped_gemm_fits(M, N, K, E, T) &&  // (a token goes to an expert once)
-         few_rows_rounds(M, N, E, quantising_kernel(M, N, K, E)) <= kRouteRounds;
+         few_rows_rounds(M, N, E, 64) <= kRouteRounds;
 }
 extern "C" int aamd_route_quant_grouped_gemm_fp8_nt(const void* ids, int ids_are_i64, int topk, int64_t T, const void* rows, int64_t ld,
                                                     const uint8_t* b, const float* b_s, int E, int64_t N, int64_t K, void* c, int64_t ldc,
