@@ -1597,18 +1597,29 @@ extern "C" int aamd_route_quant_grouped_gemm_fp8_nt(const void* ids, int ids_are
 }
 
 // With the combine (few_rows_combine_kernel)?  It saves a launch and its gap, 2.5 us of a step that is queued launch by launch, and has a
-// workgroup per token and 32 outputs, one per CU, where the GEMM alone has one per row: what it loses is a second round of them that
-// has many steps, and weights that several tokens share, which are read for each.  SwiGLU, us, two launches -> one, both replayed in a
-// graph (E, N, K, topk; T tokens): 60, 2048, 1408, 4: T 1 8.4 -> 8.0, 2 10.6 -> 8.7, 4 15.3 -> 11.2, 8 (2 rounds of 3 steps) 22.0 ->
-// 19.4; 64, 7168, 2048, 8: T 1 (8 steps) 27.4 -> 22.0; 8, 4096, 14336, 2 (14 steps): T 1 23.7 -> 21.4, 2 40.8 -> 36.8; 8, 1024, 4096, 2:
-// T 1 9.2 -> 7.2, 8 11.5 -> 10.3; 16, 4096, 4096, 1: T 1 10.6 -> 7.4, 4 (2 rounds of 4) 17.1 -> 15.1; 4, 2048, 8192, 2 (8 steps): T 1
-// 14.3 -> 12.6, 4 16.6 -> 17.7, 8 (2 rounds) 21.2 -> 34.7; 8, 7168, 7168, 1 (7 steps): T 1 15.0 -> 11.9, 2 (2 rounds) 15.6 -> 20.0; 64,
-// 512, 512, 8: T 1 7.3 -> 7.7, 8 10.6 -> 8.7.  The block of 60 experts, one token, queued: 19.6 -> 16.5.
-constexpr int64_t kCombineSteps = 8, kCombineStepsOfOneRound = 16;  // of a wave, over the rounds
+// workgroup per token and 32 outputs, one per CU, where the GEMM alone has one per row and two per CU: what it loses is long chains of
+// steps on few CUs, further rounds, and weights that several tokens share, which are read for each.  A chain of a few steps in one round
+// is always taken: with two slots a wave has as many steps as in the GEMM alone, and else such a launch is hardly longer than its
+// latencies (at most 0.7 us lost in a graph, the saved launch won where it bounds).  The others by estimates of both, us, fitted to 890
+// launches of 4 to 256 experts, 512 x 256 to 7168 x 14336, that read their weights from the caches (11 and 9 % off), a microsecond apart.
+// What the rule takes of these is faster by 2.7 us on average, 14 of 710 are slower by 0.2 to 1.8; with other weights in every launch, from
+// memory, 2.8 of 223 and none is slower (up to sixteen steps were taken before: 58 of 329 slower there, 8, 4096, 14336, 2: T 1 28.3 ->
+// 32.9).  SwiGLU, replayed in a graph, two launches -> one (E, N, K, topk; T tokens): 60, 2048, 1408, 4: T 1 7.1 -> 6.8, 8 21.0 -> 18.2;
+// 8, 1024, 4096, 2: T 8 10.6 -> 8.4; 256, 512, 4096, 2: T 8 11.0 -> 8.0; 16, 512, 512, 8: T 1 7.0 -> 7.3; 4, 2048, 8192, 2: T 2 15.0 ->
+// 16.8; not taken: 16, 512, 4096, 8: T 4 (16 steps) 11.3 -> 19.6; 8, 7168, 768, 2: T 4 (4 rounds) 12.9 -> 16.0.  The block of 60
+// experts, one token, queued: 19.6 -> 16.5.
 extern "C" int aamd_quant_grouped_gemm_combine_fits(int64_t T, int topk, int64_t N, int64_t K, int E) {
   if (T < 1 || T > kQuantisingRows || topk < 1 || topk > 8 || T * topk > kQuantisingRows) return 0;
-  const int64_t per = topk <= 2 ? 8 : topk <= 4 ? 4 : 2, rounds = (T * (N / 32) + 255) / 256;  // (waves per slot: launch_combine)
-  return rounds * ((K / kBK + per - 1) / per) <= (rounds == 1 ? kCombineStepsOfOneRound : kCombineSteps) && quantising_kernel(T * topk, N, K, E) == kFewRowsSplit;
+  if (quantising_kernel(T * topk, N, K, E) != kFewRowsSplit) return 0;
+  const int64_t per = topk <= 2 ? 8 : topk <= 4 ? 4 : 2;  // waves per slot: launch_combine
+  const int64_t nkb = K / kBK, wgs = T * (N / 32), rounds = (wgs + 255) / 256, steps = (nkb + per - 1) / per;
+  if (rounds == 1 && (steps <= 5 || (topk <= 2 && steps * wgs < 1024))) return 1;
+  if (rounds > 2 || rounds * steps > 8) return 0;
+  const double groups = E * (1.0 - std::pow(1.0 - std::min(1.0, (double)topk / E), (double)T));  // that a random routing reaches
+  const double MB = (double)N * K * 1e-6, alone = groups * (N / 32) / 512.0, alone_rounds = std::ceil(alone), alone_steps = (double)((nkb + 7) / 8);
+  const double one = 1.9 + rounds * (1.6 + 0.83 * steps * (per * topk) / 16.0) + 0.061 * T * topk * MB;
+  const double two = 4.5 + alone_rounds * (0.95 + 0.55 * alone_steps) + 0.28 * alone * alone_steps + 0.096 * groups * MB + 20e-6 * T * topk * N;
+  return one + 1.0 < two;
 }
 extern "C" int aamd_quant_grouped_gemm_combine_fp8_nt(int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64,
                                                       const int32_t* row_map, const void* probs, int probs_dtype, int topk, int64_t T,

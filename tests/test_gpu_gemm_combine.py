@@ -55,3 +55,12 @@ def test_other_sizes_are_refused(dev):
         None, _lib.NONE, _lib.stream())  # fmt: skip
     assert call(0, 1) != 0 and call(65, 1) != 0 and call(9, 8) != 0 and call(1, 9) != 0 and call(1, 1, 0) != 0
     assert call(1, 1, 1, 64) != 0 and call(1, 1, 1, 128, 64) != 0
+
+
+# (measured, two launches -> one: 11.3 -> 19.6 us, 12.9 -> 16.0, 28.3 -> 32.9 from memory, 9.8 -> 15.6; 7.1 -> 6.8, 21.0 -> 18.2, 10.6 -> 8.4, 11.0 -> 8.0)
+@pytest.mark.parametrize("T,k,E,N,K,taken", [(4, 8, 16, 512, 4096, False), (4, 2, 8, 7168, 768, False), (1, 2, 8, 4096, 14336, False), (6, 3, 4, 5120, 512, False),
+                                             (1, 4, 60, 2048, 1408, True), (8, 4, 60, 2048, 1408, True), (8, 2, 8, 1024, 4096, True), (8, 2, 256, 512, 4096, True)])  # fmt: skip
+def test_taken_where_it_is_faster(T, k, E, N, K, taken):
+    from atorch_amd import _lib
+
+    assert bool(_lib.lib().aamd_quant_grouped_gemm_combine_fits(T, k, N, K, E)) == taken
