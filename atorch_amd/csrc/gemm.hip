@@ -308,7 +308,29 @@ __device__ __forceinline__ void wgrad_short_tiles(const GemmParams& p, uint8_t* 
   }
 }
 
-// Gradients of groups without rows are zeros: workgroup `part` of `parts` writes its share.
+// Gradients of groups without rows that are written and not added to are zeros, a stream of stores that leaves the matrix cores alone.
+// As tiles like the others they come at the end, at 3.7 TB/s; here the launch's first workgroups write them beside the tiles of the
+// others, at up to 5.  How many, 0 where it does not pay: each takes half a CU from the tiles, and what one workgroup computes, a long
+// contraction or a run of short ones, takes longer beside one.  So most groups have to be without rows, and their zeros a stream that
+// outlasts that (7 MB a block); more of them where there is much to compute besides.  us, as tiles -> by 48 / 64 / 96 / 128 workgroups:
+//   60 groups, 16001 rows (108 blocks and less), 2816 x 2048 fp32     325 -> 301 / 257 / 275 / 261    zeros 1223 MB
+//   64 groups, 8192 rows (56 blocks and less), 2048 x 7168 bf16       457 -> 399 / 377 / 361 / 359    1644 MB
+//   64 groups, 189 rows (2 blocks), 2816 x 2432 fp32                  337 -> 468 (32) / 256 / 300 / 305    1698 MB
+//   60 groups, 467 rows (4 blocks), 2688 x 1024 bf16                  86 -> 86 (32) / 49 / 56 / 58    314 MB
+//   not: 32 groups, 12000 rows (81 blocks), 3072 x 1024 fp32          84 -> 104 / 99 / 104 / 109    315 MB
+//   60 groups, 39191 rows (173 blocks), 640 x 3840 fp32               189 -> 193 (32) / 224 / 240 / 216    187 MB
+// Of 683 drawn launches with two thirds of the groups without rows (4 to 64 of 512 x 512 to 7168 x 7168, 64 to 46000 rows) the rule takes
+// 443: 0.83 of the time as tiles, two of them 3 and 4 % slower.  With 96 workgroups always, launches were up to 30 % slower.
+constexpr int kZeroers = 96, kZeroersOfShort = 64;  // (multiples of 8)
+template <typename OUT>
+__device__ __forceinline__ int zeroers_of(const GemmParams& p, unsigned long long empty, int n, int steps) {
+  const int groups = __popcll(empty);
+  const int64_t bytes = (int64_t)groups * p.Lrows * p.ldc * (int64_t)sizeof(OUT);
+  const int chain = n <= p.short_kb ? n * p.run : n;
+  if (3 * groups < 2 * p.E || __ballot((int64_t)chain * 7000000 > bytes) != 0) return 0;
+  return bytes >= 400000000 && steps >= 30 * 512 ? kZeroers : kZeroersOfShort;
+}
+// Workgroup `part` of `parts` writes its share.
 template <typename OUT>
 __device__ __forceinline__ void zero_groups(const GemmParams& p, unsigned long long mask, int part, int parts) {
   const int64_t bytes = p.Lrows * p.ldc * (int64_t)sizeof(OUT);
@@ -373,7 +395,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     total_lt = (int)((p.Lrows + BM - 1) / BM);  // kRaggedRows without groups
   }
   const int64_t bid = blockIdx.x;
-  const int64_t xcd = bid % 8, idx = bid / 8 - (MODE == kRaggedK ? p.zeroers / 8 : 0);  // (negative in zeroers, which have no tile)
+  const int64_t xcd = bid % 8, idx = bid / 8;
   const int GL = p.gl;
   int g, lt, rt;
   int kb_lo = 0, kb_hi = 0;  // kRaggedK: the contraction blocks of group g
@@ -386,8 +408,8 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
     // the groups that are longer than average go first, so that the launch ends on short tiles.
     const int per_g = p.nLt * p.nRt;  // tiles of a group
     const int per_x = (per_g + 7) >> 3;
-    const int turn = __builtin_amdgcn_readfirstlane((int)((uint32_t)idx / (uint32_t)per_x));
-    const int pos = (int)idx - turn * per_x;
+    int turn = __builtin_amdgcn_readfirstlane((int)((uint32_t)idx / (uint32_t)per_x));
+    int pos = (int)idx - turn * per_x;
     g = turn;
     if (turn >= p.E && p.run == 0) return;
     if (p.goff == nullptr) {  // one group over the whole contraction
@@ -399,12 +421,20 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
       if constexpr (NT == 256) if (p.run > 0) {
         // the groups of few blocks leave the list of this loop: behind the long groups' tiles a workgroup takes a run of
         // theirs (and of the groups that the operand buffers do not hold, which are written as NaN)
-        const bool few = live && (gr.t_hi > p.max_kb || (n <= p.short_kb && n > 0));
-        const bool none = n == 0 && gr.t_hi <= p.max_kb;  // nothing to add, or zeros to write
-        if (bid < p.zeroers) {
-          zero_groups<OUT>(p, __ballot(live && none), (int)bid, p.zeroers);
-          return;
+        const bool empty = live && n == 0 && gr.t_hi <= p.max_kb;
+        const int zeroers = p.zeroers > 0 ? zeroers_of<OUT>(p, __ballot(empty), live ? n : 0, gr.total * per_g) : 0;
+        int from = (int)idx;  // this workgroup's place among those that have tiles
+        if (zeroers > 0) {
+          if (bid < zeroers) {
+            zero_groups<OUT>(p, __ballot(empty), (int)bid, zeroers);
+            return;
+          }
+          from -= zeroers / 8;
+          turn = __builtin_amdgcn_readfirstlane((int)((uint32_t)from / (uint32_t)per_x));
+          pos = from - turn * per_x;
         }
+        const bool none = empty && (p.accumulate || zeroers > 0);  // nothing to add, or zeros that are being written
+        const bool few = live && !none && (gr.t_hi > p.max_kb || n <= p.short_kb);
         live = live && !few && !none;
         const int nlong = __popcll(__ballot(live));
         if (turn >= nlong) {
@@ -412,7 +442,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
           st.mask = __ballot(few);
           st.total = __popcll(st.mask) * per_g;
           st.gr = gr;
-          const int unit = ((int)idx - nlong * per_x) * 8 + (int)xcd;
+          const int unit = (from - nlong * per_x) * 8 + (int)xcd;
           if (p.accumulate) wgrad_short_tiles<OUT, true>(p, lds, Sc0, st, unit);
           else wgrad_short_tiles<OUT, false>(p, lds, Sc0, st, unit);
           return;
@@ -1375,15 +1405,6 @@ static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
 //   8 groups, 8192 rows, 4096 x 4096 bf16                  221 -> 238 / 227 / 226 / 250, 210     49
 // (the last is where the average rule ends it: from there on both forms are within the noise of each other)
 constexpr int kShortBlocks = 8, kShortAverage = 8, kShortUnits = 1024;
-// Gradients of groups without rows that are written and not added to are zeros, a stream of stores that leaves the matrix cores
-// alone: the launch's first kZeroers workgroups write them beside the tiles of the others, which came before them and left the
-// memory idle.  About 5 TB/s from 64 workgroups on; each takes half a CU from the tiles.  us, tiles of zeros as short ones -> zeroers
-// 32 / 64 / 96 / 128 / 256 / 512 (5 to 10 of the groups have rows):
-//   64 groups, 8192 rows (Zipf), 2048 x 7168 bf16   508 -> 468 / 386 / 355 / 369 / 441 / 484    stream of the outputs 342
-//   the same, all rows in one group                 510 -> 485 / 392 / 358 / 340 / 424 / 478
-//   60 groups, 16001 rows (Zipf), 2816 x 2048 fp32  326 -> 338 / 270 / 276 / 285 / 319 / 345
-// A launch whose groups all have rows sees its zeroers leave at once: 8 groups, 1000 rows, 4096 x 1024 19.4 -> 19.7.
-constexpr int kZeroers = 96;
 static bool use_short_runs(const GemmParams& p) {
   return p.goff != nullptr && p.E <= 64 && p.max_kb <= (int64_t)kShortAverage * p.E &&
          (int64_t)p.E * p.nLt * p.nRt < (1 << 27);

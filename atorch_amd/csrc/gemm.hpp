@@ -39,7 +39,7 @@ struct GemmParams {
   int gl;          // L tiles that share an R panel in the tile order
   int run;         // kRaggedK: tiles of short groups that a workgroup takes one after the other (0: none)
   int short_kb;    // kRaggedK: the most contraction blocks of a short group
-  int zeroers;     // kRaggedK with runs: the first workgroups, which write the gradients of groups without rows (a multiple of 8)
+  int zeroers;     // kRaggedK with runs: the most workgroups that write the gradients of groups without rows, ahead of the tiles' (0: none)
   int max_split;   // row_tiles_kernel: the most parts of a tile's contraction; more than one: ws holds kRowPartsBytes
   float* ws;
   int stream_out;  // row_tiles_kernel: the output is stored past the caches
