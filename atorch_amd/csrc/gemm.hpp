@@ -80,10 +80,11 @@ int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, boo
 int launch_few_rows_quantising(const GemmParams& p, int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
                                int64_t M, bool split, hipStream_t st);
 // The same of permuted rows from the router's choices, see aamd_route_quant_grouped_gemm_fp8_nt: p.Lrows of them, at most 64.
-int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64, const int32_t* row_map,
-                            const void* probs, int probs_dtype, int topk, int64_t T, void* out, hipStream_t st);
 int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i64, const void* rows, int64_t ld, int topk, int64_t T,
                             int64_t* sorted_idx, int32_t* row_map, int64_t* goff, bool split, hipStream_t st);
+// The second GEMM of a decoding step with the weighted combine in it, see aamd_quant_grouped_gemm_combine_fp8_nt: T tokens of topk slots.
+int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64, const int32_t* row_map,
+                            const void* probs, int probs_dtype, int topk, int64_t T, void* out, hipStream_t st);
 
 constexpr int64_t kRowPartsBytes = (int64_t)256 * kLargeTile * kLargeTile * 4;  // a tile of fp32 for each of 256 workgroups
 // Row-ragged GEMM with block-scaled R on 256 x 256 tiles (gemm_rows.hip): at least eight contraction blocks, p.ls_batch 1 where

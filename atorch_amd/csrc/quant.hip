@@ -426,8 +426,8 @@ __global__ __launch_bounds__(256) void quant_dual_grouped_kernel(
 // and then runs the tile of the grouped kernel on gathered rows.  Source rows are clamped to the token count,
 // so a corrupt index reads a wrong row, never beyond x.
 // WEIGHTED: the row is bf16(token * probs[flat index]), the combine's gradient with respect to it.  Written by a kernel of its own and
-// read here those rows were a third of the two kernels' traffic (8191 tokens to 4 of 60 experts, 2048 wide, us: both gradients of the
-// combine 56 and the quantiser 59 took 25 more than this and the weights' gradient alone; the training step of that block 1774 -> 1739, of 500 tokens to 2 of 8 238 -> 233).
+// read here those rows were a third of the two kernels' traffic (8191 tokens to 4 of 60 experts, 2048 wide, with the gradient of the
+// weights 107 us, this and a kernel for the weights' gradient alone 86; gathers_gradient in host.cpp says where it is taken).
 template <typename IN, bool WEIGHTED = false, bool SUMS = false>
 __global__ __launch_bounds__(256) void quant_dual_gather_kernel(
     const typename IN::elem* __restrict__ x, int64_t ldx, int nt, const int64_t* __restrict__ sorted_idx,
