@@ -1260,7 +1260,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 // Launch choices a caller of the measurement build may pin per call (-1 = the library chooses, which is
 // all the product entry points ever pass).
 struct GemmOptions {
-  int tile = -1;      // 0: 128x128 tiles, 1: 256x256 tiles, 2 / 3: the kernel for few rows, 3 in its split form, 4: a workgroup per 256x256 tile
+  int tile = -1;      // 0: 128x128 tiles, 1: 256x256 tiles, 2 / 3: the kernel for few rows, 3 in its split form, 4: a workgroup per 256x256 tile, 6: 256x256 tiles of up to 288 rows
   int group_r = -1;   // tile order groups R tiles (1) or L tiles (0)
   int gl = -1;        // tiles that share a panel in the tile order
   int ls_batch = -1;  // 0: L scales fetched one contraction block at a time
@@ -1330,11 +1330,11 @@ static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8
 // 3.9; 2965 in 60 (Zipf), 2048 x 11008 200 -> 97; 726 in 8, 6528 x 6656 141 -> 85; 1394 in 16, 5888 x 9216 186 -> 116.  Of the
 // others 2.9 % take 3 % or more longer than before, 11 % that much less; the worst are uneven groups, whose empty ones the host
 // does not know of (1776 in 60, 25856 x 512 63 -> 110; 3532 in 16, 1664 x 6144 53 -> 67).
-enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4, kLargeShared = 5 };
+enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4, kLargeShared = 5, kLargeMore = 6 };
 // b_rows: weights read along their rows, which the split form cannot.  share_last: with a workspace for parts of the last round of
 // 256 x 256 tiles.
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
-  if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
+  if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4 || g_opt.tile == 6) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const bool one = !grouped || E == 1;
   const double n = (double)nkb, rows = (double)M;
   const double groups = one ? 1.0 : std::min({rows, (double)E, (double)E * (1.0 - std::exp(-0.6 * rows / (double)E))});
@@ -1467,7 +1467,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                                         : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, ws != nullptr, g_opt);
   // (output rows of 8 M elements are out of reach of the large tiles' 32-bit offsets)
   const bool once = kernel == kLargeOnce && !b_tile_scaled;
-  const bool large = once || ((kernel == kLargeTiles || kernel == kLargeShared) && (b_tile_scaled || ldc < (1LL << 23)));
+  const bool large = once || ((kernel == kLargeTiles || kernel == kLargeShared || kernel == kLargeMore) && (b_tile_scaled || ldc < (1LL << 23)));
   const int BM = large ? kLargeTile : CfgSmall::BM;
   const int BN = large ? (b_tile_scaled ? CfgWgrad::BN : kLargeTile) : CfgSmall::BN;
   static_assert(CfgWgrad::BM == kLargeTile, "L rows of a large tile");
@@ -1497,6 +1497,17 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                   : launch_gemm<kRaggedRows, false, CfgLarge>(p, c_dtype, blocks, st, g_opt);
   if (large && !b_tile_scaled) {
     tile_order<kRaggedRows>(p, kLargeTile, g_opt);
+    // Tiles of up to 288 rows: the kernel decides by the groups' rows, where there can be enough remainders (32 rows more save a group at
+    // most 48 - 17 64ths of a tile, and every tile costs 4 to 7: not with more than seven a group; nor with much less than one) and
+    // the 1 to 2 us that deciding takes are little (launches of fewer R tiles, 60 uneven groups, 131 us: 1 to 2 % of them).
+    p.slices = p.group_r && E <= 64 && p.nRt >= 32;
+    p.higher_cost = (int)higher_tile_cost(p.nkb, p.slices);
+    if (g_opt.tile >= 0) p.higher = kernel == kLargeMore ? 1 : -1;
+    else if (group_offsets != nullptr) p.higher = E > 64 || M >= (int64_t)7 * kLargeTile * E || M < (int64_t)kLargeTile * 15 / 16 * E || p.nRt < 16 || p.nRt > 1024 ? -1 : 0;
+    else {
+      const uint32_t full = (uint32_t)std::min<int64_t>(M / kLargeTile, 8), over = (uint32_t)(M % kLargeTile), more = (over + 31) / 32;
+      p.higher = over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, (uint32_t)p.higher_cost, ws != nullptr, false) ? 1 : -1;
+    }
     p.ws = ws;
     p.max_split = ws != nullptr ? row_max_split(p.nkb) : 1;
     return launch_row_tiles(p, c_dtype, blocks, b_rows, st);

@@ -42,6 +42,9 @@ struct GemmParams {
   int zeroers;     // kRaggedK with runs: the most workgroups that write the gradients of groups without rows, ahead of the tiles' (0: none)
   int max_split;   // row_tiles_kernel: the most parts of a tile's contraction; more than one: ws holds kRowPartsBytes
   float* ws;
+  int higher;      // row_tiles_kernel: tiles of up to 288 rows (1), of 256 (-1), or as the groups' rows have it (0)
+  int higher_cost; // with these: of a tile, see higher_tiles_pay
+  int slices;      // row_tiles_kernel with these: every XCD takes an eighth of every group
   int stream_out;  // row_tiles_kernel: the output is stored past the caches
   int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
 };
@@ -85,6 +88,25 @@ int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i6
 // The second GEMM of a decoding step with the weighted combine in it, see aamd_quant_grouped_gemm_combine_fp8_nt: T tokens of topk slots.
 int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64, const int32_t* row_map,
                             const void* probs, int probs_dtype, int topk, int64_t T, void* out, hipStream_t st);
+
+// Are tiles of more rows worth it?  They save the tiles of remainders, which fetch their weights once more whatever few rows they have
+// (us, 28672 outputs x 4096, 8 groups of 512 rows 430, 513 to 576 548 to 560, 640 595, 768 640), and cost every step and every tile
+// something, more where addresses are made in the step.  In 64ths of a tile, fitted to 500 launches of 2 to 60 groups of 250 to 1700
+// rows on average with both.  With slices: a remainder's own tile 38, 32 rows more 13, a tile that may have them 68; else 48, 17, and
+// 71 and 64 a step; launches of up to three rounds by their rounds.  Taken for 112 of those, 0.94 of the time on average, three 2 % slower
+// or more.  28672 x 4096 in 8 groups, plain tiles -> these: 485 to 542 rows, five above 512 601 -> 497, three 552 -> 488; 264
+// 388 -> 310, 520 582 -> 494; 60 of about 270, 7168 x 4096, 702 -> 611; not: 512 449 -> 473, 640 595 -> 632, about 4096 3377 -> 3654.
+inline uint32_t higher_tile_cost(int nkb, bool slices) { return slices ? 68 : 71 + 64 / (uint32_t)nkb; }
+__host__ __device__ inline bool higher_tiles_pay(uint32_t full, uint32_t own0, uint32_t own1, uint32_t shared, uint32_t nRt, uint32_t cost, bool parts, bool slices) {
+  const uint32_t n0 = (full + own0) * nRt, n1 = (full + own1) * nRt;
+  if (n0 <= 3 * 256) {  // rounds, in tenths; one that is shared out counts for 6
+    const uint32_t l0 = n0 % 256, l1 = n1 % 256, shares = parts ? 128 : 0;
+    const uint32_t r0 = n0 / 256 * 10 + (l0 == 0 ? 0 : l0 <= shares ? 6 : 10), r1 = n1 / 256 * 10 + (l1 == 0 ? 0 : l1 <= shares ? 6 : 10);
+    return 64 * r0 > 74 * r1;
+  }
+  const uint32_t own = slices ? 38 : 48, more = slices ? 13 * 64 : 17 * 64;
+  return 64 * (64 * full + own * own0) > cost * (64 * full + own * own1) + more * shared;
+}
 
 constexpr int64_t kRowPartsBytes = (int64_t)256 * kLargeTile * kLargeTile * 4;  // a tile of fp32 for each of 256 workgroups
 // Row-ragged GEMM with block-scaled R on 256 x 256 tiles (gemm_rows.hip): at least eight contraction blocks, p.ls_batch 1 where

@@ -15,6 +15,11 @@ template <int OFFSET>
 __device__ __forceinline__ void load_lds_x4(uint32_t off, const v4i& buf, uint32_t lds) {
   asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(buf), "s"(lds), "i"(OFFSET) : "memory", "scc");
 }
+// The same for all lanes or none (-1 or 0); counted like a load either way.
+template <int OFFSET>
+__device__ __forceinline__ void load_lds_x4_for(int lanes, uint32_t off, const v4i& buf, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_mov_b32 exec_lo, %4\n\ts_mov_b32 exec_hi, %4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(buf), "s"(lds), "i"(OFFSET), "s"(lanes) : "memory", "scc");
+}
 __device__ __forceinline__ void advance_buffer(v4i& b, int64_t by) {
   const uint64_t a = (((uint64_t)(uint32_t)b[1] << 32) | (uint32_t)b[0]) + (uint64_t)by;
   b[0] = (int)(uint32_t)a;
@@ -31,11 +36,44 @@ __device__ __forceinline__ int opaque(int v) {
   asm volatile("" : "+s"(v));
   return __builtin_amdgcn_readfirstlane(v);
 }
+// The same of what lies in a scalar register (no copy of it in a vector register, which would be made in front of the loop).
+__device__ __forceinline__ int opaque_s(int v) {
+  asm volatile("" : "+s"(v));
+  return __builtin_amdgcn_readfirstlane(v);
+}
 // The lane, counted anew: what is computed from it lives where it is used, not in registers across the tile loop.
 __device__ __forceinline__ int lane_here() {
   int l;
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
   return l;
+}
+// v + s and v ^ s, made where they are used: what the compiler can move in front of the loop costs a register for the whole of it.
+__device__ __forceinline__ uint32_t add_here(uint32_t v, uint32_t s) {
+  uint32_t r;
+  asm volatile("v_add_u32 %0, %1, %2" : "=v"(r) : "s"(s), "v"(v));
+  return r;
+}
+__device__ __forceinline__ uint32_t xor_here(uint32_t v, uint32_t s) {
+  uint32_t r;
+  asm volatile("v_xor_b32 %0, %1, %2" : "=v"(r) : "s"(s), "v"(v));
+  return r;
+}
+// A word of the LDS that is the same for every lane, by one vector register and with its wait (five wait states behind it, for memory
+// instructions that take it as an operand), and 16 bytes of them.
+__device__ __forceinline__ int word_here(uint32_t at) {
+  int r, v;
+  asm volatile("v_mov_b32 %1, %2\n\tds_read_b32 %1, %1\n\ts_waitcnt lgkmcnt(0)\n\tv_readfirstlane_b32 %0, %1\n\ts_nop 4" : "=s"(r), "=&v"(v) : "s"(at) : "memory");
+  return __builtin_amdgcn_readfirstlane(r);
+}
+__device__ __forceinline__ v4i words_here(uint32_t at) {
+  asm volatile("" : "+s"(at));
+  const v4i v = *(const __attribute__((address_space(3))) v4i*)(uintptr_t)at;
+  return v4i{__builtin_amdgcn_readfirstlane(v[0]), __builtin_amdgcn_readfirstlane(v[1]), __builtin_amdgcn_readfirstlane(v[2]), __builtin_amdgcn_readfirstlane(v[3])};
+}
+__device__ __forceinline__ void put_words(uint32_t at, const v4i& w) { *(__attribute__((address_space(3))) v4i*)(uintptr_t)at = w; }
+__device__ __forceinline__ void copy_words(uint32_t to, uint32_t from) {
+  const v4i w = *(const __attribute__((address_space(3))) v4i*)(uintptr_t)from;
+  put_words(to, w);
 }
 // The kernel's arguments, fetched anew where they are used.
 __device__ __forceinline__ uint64_t args_here() {
@@ -141,6 +179,33 @@ __device__ __forceinline__ void store_sub_tiles(const v16f& a, const v16f& b, ui
     gather_bf16(b, xb, yb);
     store_lines<COL * 2, NT>(xa, xb, row, rows8, out);
     store_lines<COL * 2, NT>(ya, yb, row + 2 * rows8, rows8, out);
+  }
+}
+
+// One sub-tile alone, from the first byte of `out` on: 64 (bf16) or 128 bytes of a row.
+template <typename OUT>
+__device__ __forceinline__ void store_sub_tile(const v16f& o, int lane, uint32_t ldc, const v4i& out) {
+  if constexpr (sizeof(OUT) == 4) {
+    const uint32_t row = store_offset<float>(lane, ldc), rows8 = 8u * ldc * 4u;
+    v4i x[2], y[2];
+#pragma unroll
+    for (int qp = 0; qp < 2; qp++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float f = o[8 * qp + r], h = o[8 * qp + 4 + r];
+        int u = __builtin_bit_cast(int, f), v = __builtin_bit_cast(int, h);
+        swap16(u, v);
+        x[qp][r] = u;
+        y[qp][r] = v;
+      }
+    store_lines<0, false>(x[0], x[1], row, rows8, out);
+    store_lines<0, false>(y[0], y[1], row + 2 * rows8, rows8, out);
+  } else {
+    v4i x, y;
+    gather_bf16(o, x, y);
+    const uint32_t at = ((uint32_t)(lane & 15) * ldc + 8u * (2u * ((uint32_t)(lane >> 4) & 1u) + ((uint32_t)lane >> 5))) * 2u;
+    store_x4<0, false>(x, at, out);
+    store_x4<0, false>(y, at + 16u * ldc * 2u, out);
   }
 }
 
