@@ -235,6 +235,15 @@ __device__ __forceinline__ uint32_t row_split(uint32_t left, uint32_t nwg, uint3
   const uint32_t s = left > 0 ? nwg / left : 1;
   return s < 1 ? 1 : s < max_split ? s : max_split;
 }
+// Where the contraction is not shared and at most half the workgroups have a tile in the last round, two or four of them share the rows
+// of one, in pieces of 64.  The step of such a piece waits for its loads, which are asked for one step ahead: with 256 rows and half of the
+// chip idle 1.3 us, with 128 1.25, with 64 1.0 (a step of a whole round: 1.8).  us, 4096 rows, last round of 1 to 8 tiles per XCD:
+// 8704 x 1024 60 -> 57, x 4096 164 -> 157; 12800 x 2048 126 -> 121; 16640 x 4096 279 -> 271; of 16 tiles 14336 x 4096 229 -> 228; 16001 uneven
+// rows in 60 groups, 2048 x 2816 120 -> 114.  Parts of long contractions give more (1 tile per XCD, 56 blocks 150 -> 126, these 139), and
+// pieces of 128 rows x 128 columns no more than these.
+__device__ __forceinline__ uint32_t row_shares(uint32_t left, uint32_t nwg) { return left == 0 || 2 * left > nwg ? 1 : 4 * left > nwg ? 2 : 4; }
+// The last row that is loaded (a share may have none, and then loads one).
+__device__ __forceinline__ int last_row(int valid) { return valid > 0 ? valid - 1 : 0; }
 // First contraction block of a part: whole groups of four (16 bytes of scales) but for the end of the last part.  With
 // nkb >= 8 split every part has eight blocks or more.
 __device__ __forceinline__ uint32_t row_part(uint32_t nkb, uint32_t split, uint32_t part) {
@@ -294,6 +303,7 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
   const uint32_t places = p.nkb >= 16 ? 0u : nwg > 5u ? 5u : 1u;
   uint32_t round_first = mine.first, turn = blockIdx.x >> 3;
   // the next tile of this workgroup, false if there is none; part and parts: of the contraction it takes, slot: where a part goes
+  // (-1: of the tile's rows, see row_shares)
   uint32_t part = 0, parts = 1;
   int n_slot = -1;
   auto take = [&](uint32_t& pid) __attribute__((always_inline)) {
@@ -305,6 +315,13 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
         n_slot = turn < left * parts ? (int)(xcd * part_places(MORE) + turn) : -1;
         part = turn / left;
         at = n_slot >= 0 ? turn - part * left : left;
+      }
+    }
+    if (left < nwg && parts == 1) {
+      parts = row_shares(left, nwg);
+      if (parts > 1) {
+        part = turn / left;
+        at = turn < left * parts ? turn - part * left : left;
       }
     }
     pid = round_first + at;
@@ -323,17 +340,23 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
   int c_g, c_lvalid, c_r0, c_rvalid, c_kb0, c_steps, c_slot, n_g, n_lvalid, n_r0, n_rvalid, n_kb0, n_steps;
   auto take_tile = [&](uint32_t id, auto a) __attribute__((always_inline)) {
     const RowTile t = row_tile<MORE>(a, opaque(a->goff != nullptr && a->E <= 64) ? table : nullptr, id, nRt, total_lt, xcd);
-    int kb0 = 0, steps = t.steps;
+    int kb0 = 0, steps = t.steps, lvalid = t.lvalid;
+    int64_t l0 = t.l0;
     if (n_slot >= 0) {
       kb0 = (int)row_part((uint32_t)t.steps, parts, part);
       steps = (int)row_part((uint32_t)t.steps, parts, part + 1) - kb0;
+    } else if (parts > 1) {
+      // (without rows, where the tile has few: a workgroup that stores nothing)
+      const int size = (lvalid + 64 * (int)parts - 1) / (64 * (int)parts) * 64, from = (int)part * size, rest = lvalid - from;
+      l0 += rest > 0 ? from : 0;
+      lvalid = rest < 0 ? 0 : rest < size ? rest : size;
     }
     if constexpr (MORE) {
-      put_words(tile_words + kNext, v4i{(int)(uint32_t)(uint64_t)t.l0, (int)((uint64_t)t.l0 >> 32), t.g, t.lvalid});
+      put_words(tile_words + kNext, v4i{(int)(uint32_t)(uint64_t)l0, (int)((uint64_t)l0 >> 32), t.g, lvalid});
       put_words(tile_words + kNext + 16, v4i{t.r0, t.rvalid, kb0, steps});
       put_words(tile_words + kNext + 32, v4i{n_slot, 0, 0, 0});
     } else {
-      n_l0 = t.l0, n_g = t.g, n_lvalid = t.lvalid, n_r0 = t.r0, n_rvalid = t.rvalid, n_kb0 = kb0, n_steps = steps;
+      n_l0 = l0, n_g = t.g, n_lvalid = lvalid, n_r0 = t.r0, n_rvalid = t.rvalid, n_kb0 = kb0, n_steps = steps;
     }
   };
   auto no_more_tiles = [&]() __attribute__((always_inline)) {
@@ -402,7 +425,7 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
     const int block = t.kb0 + last;
     const int64_t l_at = t.l0 * a->ldl + block * kBK;
     const int64_t r_at = (int64_t)t.g * a->r_group_stride + (R_ROWS ? (int64_t)t.r0 : t.r0 * a->ldr) + block * a->r_kb_stride;
-    lbuf = buffer_at(a->L + uniform_i64(l_at), (uint32_t)__builtin_amdgcn_readfirstlane((t.lvalid - 1) * (int)a->ldl + kBK));
+    lbuf = buffer_at(a->L + uniform_i64(l_at), (uint32_t)__builtin_amdgcn_readfirstlane(last_row(t.lvalid) * (int)a->ldl + kBK));
     rbuf = buffer_at(a->R + uniform_i64(r_at), (uint32_t)__builtin_amdgcn_readfirstlane(
                                                    R_ROWS ? 127 * (int)a->ldr + t.rvalid : (t.rvalid - 1) * (int)a->ldr + kBK));
     to_load = t.steps - last;
@@ -449,7 +472,7 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
   const uint32_t lsr = (uint32_t)p.ls_row_stride, rsr = (uint32_t)p.rs_row_stride, rsb = (uint32_t)p.rs_blk_stride;
   auto ask_scales = [&](const RowTile t, int b, int parity, auto a) __attribute__((always_inline)) {
     const int at = t.kb0 + (8 * b + 8 <= t.steps ? 8 * b : t.steps - 8), ln = lane_here();
-    const v4i lb = buffer_at(a->Ls + uniform_i64(t.l0 * lsr + at), (uint32_t)__builtin_amdgcn_readfirstlane(((t.lvalid - 1) * (int)lsr + 8) * 4));
+    const v4i lb = buffer_at(a->Ls + uniform_i64(t.l0 * lsr + at), (uint32_t)__builtin_amdgcn_readfirstlane((last_row(t.lvalid) * (int)lsr + 8) * 4));
     const uint32_t ld = lds_offset(scales + parity * kScaleBatch) + (uint32_t)(wave * 1024);
     const int wide = opaque(x4);
     if (wide) {
