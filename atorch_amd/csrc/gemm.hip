@@ -1260,7 +1260,7 @@ __global__ __launch_bounds__(C::NT, C::NT == 256 ? 2 : 1) void grouped_gemm_kern
 // Launch choices a caller of the measurement build may pin per call (-1 = the library chooses, which is
 // all the product entry points ever pass).
 struct GemmOptions {
-  int tile = -1;      // 0: 128x128 tiles, 1: 256x256 tiles, 2 / 3: the kernel for few rows, 3 in its split form, 4: a workgroup per 256x256 tile, 6: 256x256 tiles of up to 288 rows
+  int tile = -1;      // 0: 128x128 tiles, 1: 256x256 tiles, 2 / 3: the kernel for few rows, 3 in its split form, 7 / 8 with two waves and one, 4: a workgroup per 256x256 tile, 6: 256x256 tiles of up to 288 rows
   int group_r = -1;   // tile order groups R tiles (1) or L tiles (0)
   int gl = -1;        // tiles that share a panel in the tile order
   int ls_batch = -1;  // 0: L scales fetched one contraction block at a time
@@ -1318,8 +1318,9 @@ static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8
 //   - 256 x 256 tiles 6.5, and 6.3 and 0.78 to 1.08 per step for every round of 256, by how full the tiles and the round are;
 //     with a last round in parts 20 and 10 times what it fills, for writing and adding them, and its steps by the number of
 //     parts; 4 more where a workspace is at hand and the last round turns out not to be shared;
-//   - a 64 x 64 block of the kernel for few rows 2.7 ns and 1.1 ns per step, spread over the chip; a 32 x 32 block of its split
-//     form 3.6 and 0.47; and no less than a wave's own chain of every fourth (eighth) step;
+//   - a 64 x 64 block of the kernel for few rows 2.7 ns and 1.1 ns per step, spread over the chip, with two waves 1.1 and 1.135, with
+//     one 0.26 and 1.135; a 32 x 32 block of its split form 3.6 and 0.47; and no less than a wave's own chain of every fourth (second,
+//     single, eighth) step;
 //   - and none can beat the weights' stream from memory.
 // The groups' sizes are known on the device only.  Groups with rows are expected to be E (1 - exp(-0.6 M / E)), token tiles one
 // per such group with few rows and 0.56 of a tile per group more than the rows fill with many; what depends on rounds is the mean
@@ -1330,9 +1331,21 @@ static int row_max_split(int64_t nkb) { return (int)std::min<int64_t>(8, nkb / 8
 // 3.9; 2965 in 60 (Zipf), 2048 x 11008 200 -> 97; 726 in 8, 6528 x 6656 141 -> 85; 1394 in 16, 5888 x 9216 186 -> 116.  Of the
 // others 2.9 % take 3 % or more longer than before, 11 % that much less; the worst are uneven groups, whose empty ones the host
 // does not know of (1776 in 60, 25856 x 512 63 -> 110; 3532 in 16, 1664 x 6144 53 -> 67).
-enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4, kLargeShared = 5, kLargeMore = 6 };
-// b_rows: weights read along their rows, which the split form cannot.  share_last: with a workspace for parts of the last round of
-// 256 x 256 tiles.
+enum NtKernel { kSmallTiles = 0, kLargeTiles = 1, kFewRows = 2, kFewRowsSplit = 3, kLargeOnce = 4, kLargeShared = 5, kLargeMore = 6, kFewRowsTwo = 7, kFewRowsOne = 8 };
+static bool is_few_rows(NtKernel k) { return k == kFewRows || k == kFewRowsSplit || k == kFewRowsTwo || k == kFewRowsOne; }
+static int few_rows_waves(NtKernel k) { return k == kFewRowsSplit ? 8 : k == kFewRowsTwo ? 2 : k == kFewRowsOne ? 1 : 4; }
+// b_rows: weights read along their rows, which the split form and those of one and two waves cannot.  share_last: with a workspace for
+// parts of the last round of 256 x 256 tiles.
+//
+// How many waves share the contraction of a 64 x 64 block: a CU holds two blocks of four waves, four of two or eight of one, with as
+// many loads in flight.  With fewer waves there is less to add up at the end, and 513 to 1024 (2048) blocks are no second round: 544
+// blocks of 4 steps 8.9 us with four, 7.3 with two, 512 blocks 6.5 and 6.9; 1440 blocks of few rows, of 1 / 2 / 4 / 8 / 16 steps,
+// four waves 11.1 / 11.6 / 15.2 / 20.5 / 31.8, one 5.6 / 6.4 / 11.2 / 17.5 / 30.0.  The lines lie where the mean of 12400 drawn launches
+// (1 to 64 groups, 8 to 6000 rows, 512 to 5120 outputs and a contraction of 256 to 5120, replayed in a graph) turns; past 20 steps, or
+// 14 with weights beyond the last-level cache, the weights' stream bounds such launches (64 groups of 6 rows, 7168 x 2048: 164 with four,
+// 168 with one).  With these forms and their estimates those launches take 0.964 of the time, 18 % of them 3 % or more less, 0.9 % more
+// (64 uneven groups, 335 rows, 2176 x 3072 74 -> 83).  The forms that quantise their rows take the same, and give the same bits: eight
+// tokens to 8 of 128 experts, 2048 x 768, layer 59 -> 53, 256, 1024 x 512 36 -> 33.
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4 || g_opt.tile == 6) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const bool one = !grouped || E == 1;
@@ -1373,11 +1386,15 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   const double shared = nkb < 8 || !share_last ? 1e30 : std::max(mean(tiles_l, per_l, shared_time), weights / 6.7);
 
   const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_s = token_tiles(32) * (double)(N / 32);
-  const double few = std::max({4.5 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
+  const bool fewer_waves = !b_rows && nkb < (weights <= 256.0 ? 20 : 14);
+  const bool one_wave = fewer_waves && blocks_f >= (nkb < 4 ? 724.0 : 1024.0), two_waves = fewer_waves && !one_wave && blocks_f >= 500.0;
+  const double few = one_wave    ? std::max({5.8 + 1e-3 * blocks_f * (1.135 * n + 0.26), 4.4 + 0.64 * n, weights / 6.8})
+                     : two_waves ? std::max({5.3 + 1e-3 * blocks_f * (1.135 * n + 1.1), 4.5 + 0.65 * std::ceil(n / 2.0), weights / 6.8})
+                                 : std::max({4.5 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
   const double split = b_rows ? 1e30 : std::max({2.6 + 1e-3 * blocks_s * (0.47 * n + 3.6), 3.8 + 0.52 * std::ceil(n / 8.0), weights / 6.8});
 
   const double tiles = std::min({small, large, shared});
-  if (std::min(few, split) <= tiles) return split < few ? kFewRowsSplit : kFewRows;
+  if (std::min(few, split) <= tiles) return split < few ? kFewRowsSplit : one_wave ? kFewRowsOne : two_waves ? kFewRowsTwo : kFewRows;
   if (small <= tiles) return kSmallTiles;
   if (shared <= tiles) return kLargeShared;
   // A workgroup per tile where none would have a second one: the step of grouped_gemm_kernel has no bookkeeping of a stream of
@@ -1489,7 +1506,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   p.goff = group_offsets;
   p.Lrows = M; p.Rrows = N; p.nkb = (int)(K / kBK); p.E = E; p.nRt = (int)((N + BN - 1) / BN); p.nLt = 0;
   p.accumulate = 0;
-  if (kernel == kFewRows || kernel == kFewRowsSplit) return launch_few_rows(p, c_dtype, M, kernel == kFewRowsSplit, b_rows, st);
+  if (is_few_rows(kernel)) return launch_few_rows(p, c_dtype, M, few_rows_waves(kernel), b_rows, st);
   const int64_t max_lt = group_offsets ? M / BM + E : (M + BM - 1) / BM;
   const int64_t blocks = max_lt * p.nRt;
   if (once)
@@ -1562,9 +1579,9 @@ static double few_rows_rounds(int64_t M, int64_t N, int E, int rows) {
 // 28.7 -> 49.2.
 extern "C" int aamd_quant_grouped_gemm_fits(int64_t M, int64_t N, int64_t K, int E, int64_t most) {
   const NtKernel kernel = quantising_kernel(M, N, K, E);
-  if (kernel != kFewRows && kernel != kFewRowsSplit) return 0;
+  if (!is_few_rows(kernel)) return 0;
   const int64_t nkb = K / kBK;
-  const int waves = kernel == kFewRows ? 4 : 8, rows = kernel == kFewRows ? 64 : 32;
+  const int waves = kernel == kFewRowsSplit ? 8 : 4, rows = kernel == kFewRowsSplit ? 32 : 64;  // (fewer waves: as many more places)
   return most <= 8 && few_rows_rounds(M, N, E, rows) * (double)((nkb + waves - 1) / waves) <= 24.0;
 }
 static GemmParams quantising_params(const uint8_t* b, const float* b_s, const int64_t* group_offsets, int E, int64_t M, int64_t N,
@@ -1585,7 +1602,7 @@ extern "C" int aamd_quant_grouped_gemm_fp8_nt(int what, const void* rows, int64_
                                               void* stream) {
   AAMD_REQUIRE(what >= AAMD_ROWS_PERMUTED && what <= AAMD_ROWS_GELU, "quant_grouped_gemm_nt: unknown source %d", what);
   const NtKernel kernel = quantising_kernel(M, N, K, E);
-  AAMD_REQUIRE(kernel == kFewRows || kernel == kFewRowsSplit, "quant_grouped_gemm_nt: not for M=%lld, N=%lld, K=%lld in %d groups", (long long)M,
+  AAMD_REQUIRE(is_few_rows(kernel), "quant_grouped_gemm_nt: not for M=%lld, N=%lld, K=%lld in %d groups", (long long)M,
                (long long)N, (long long)K, E);
   AAMD_REQUIRE(bias == nullptr || bias_dtype == AAMD_BF16 || bias_dtype == AAMD_F32, "quant_grouped_gemm_nt: bad bias dtype");
   AAMD_REQUIRE(rows && b && b_s && c && group_offsets && (what != AAMD_ROWS_PERMUTED || (sorted_idx && topk >= 1 && T >= 1 && T < (1LL << 31))),
@@ -1593,7 +1610,7 @@ extern "C" int aamd_quant_grouped_gemm_fp8_nt(int what, const void* rows, int64_
   AAMD_REQUIRE(ld >= (what == AAMD_ROWS_SWIGLU ? 2 * K : K) && ld % 8 == 0 && aligned16(rows) && aligned16(b), "quant_grouped_gemm_nt: operands must be 16-byte aligned");
   AAMD_REQUIRE(ldc >= N && ldc % 8 == 0 && aligned16(c), "quant_grouped_gemm_nt: output rows must be 16-byte aligned");
   const GemmParams p = quantising_params(b, b_s, group_offsets, E, M, N, K, c, ldc, bias, bias_dtype);
-  return launch_few_rows_quantising(p, what, rows, ld, sorted_idx, topk, T, M, kernel == kFewRowsSplit, (hipStream_t)stream);
+  return launch_few_rows_quantising(p, what, rows, ld, sorted_idx, topk, T, M, few_rows_waves(kernel), (hipStream_t)stream);
 }
 // From the router's choices.  It saves the routing's launch, 3 us and its gap, and puts 0.3 us into every round of workgroups, which look
 // among the choices for their pairs before they know their weights.  Routing and GEMM, replayed in a graph, us, two launches -> one
@@ -1617,14 +1634,14 @@ extern "C" int aamd_route_quant_grouped_gemm_fp8_nt(const void* ids, int ids_are
   AAMD_REQUIRE(topk >= 1 && T >= 1 && T <= kQuantisingRows && topk <= kQuantisingRows && E <= 1024, "route_quant_grouped_gemm_nt: bad routing");
   const int64_t M = T * topk;
   const NtKernel kernel = quantising_kernel(M, N, K, E);
-  AAMD_REQUIRE(kernel == kFewRows || kernel == kFewRowsSplit, "route_quant_grouped_gemm_nt: not for M=%lld, N=%lld, K=%lld in %d groups", (long long)M,
+  AAMD_REQUIRE(is_few_rows(kernel), "route_quant_grouped_gemm_nt: not for M=%lld, N=%lld, K=%lld in %d groups", (long long)M,
                (long long)N, (long long)K, E);
   AAMD_REQUIRE(bias == nullptr || bias_dtype == AAMD_BF16 || bias_dtype == AAMD_F32, "route_quant_grouped_gemm_nt: bad bias dtype");
   AAMD_REQUIRE(ids && rows && b && b_s && c && sorted_idx && row_map && group_offsets, "route_quant_grouped_gemm_nt: null pointer");
   AAMD_REQUIRE(ld >= K && ld % 8 == 0 && aligned16(rows) && aligned16(b), "route_quant_grouped_gemm_nt: operands must be 16-byte aligned");
   AAMD_REQUIRE(ldc >= N && ldc % 8 == 0 && aligned16(c), "route_quant_grouped_gemm_nt: output rows must be 16-byte aligned");
   const GemmParams p = quantising_params(b, b_s, nullptr, E, M, N, K, c, ldc, bias, bias_dtype);
-  return launch_few_rows_routing(p, ids, ids_are_i64, rows, ld, topk, T, sorted_idx, row_map, group_offsets, kernel == kFewRowsSplit,
+  return launch_few_rows_routing(p, ids, ids_are_i64, rows, ld, topk, T, sorted_idx, row_map, group_offsets, few_rows_waves(kernel),
                                  (hipStream_t)stream);
 }
 

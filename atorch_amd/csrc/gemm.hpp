@@ -78,13 +78,13 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // Row-ragged GEMM with block-scaled R for groups of few rows (gemm_few.hip); reads L, R, their scales and strides, C,
 // bias, goff, E, Lrows, Rrows and nkb of the parameters.  r_rows: R is stored [contraction, Rrows] (R_ROWS of gemm.hip).
-int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st);
+int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, int waves, bool r_rows, hipStream_t st);
 // The same from bf16 rows, see aamd_quant_grouped_gemm_fp8_nt.
 int launch_few_rows_quantising(const GemmParams& p, int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
-                               int64_t M, bool split, hipStream_t st);
+                               int64_t M, int waves, hipStream_t st);
 // The same of permuted rows from the router's choices, see aamd_route_quant_grouped_gemm_fp8_nt: p.Lrows of them, at most 64.
 int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i64, const void* rows, int64_t ld, int topk, int64_t T,
-                            int64_t* sorted_idx, int32_t* row_map, int64_t* goff, bool split, hipStream_t st);
+                            int64_t* sorted_idx, int32_t* row_map, int64_t* goff, int waves, hipStream_t st);
 // The second GEMM of a decoding step with the weighted combine in it, see aamd_quant_grouped_gemm_combine_fp8_nt: T tokens of topk slots.
 int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld, const void* ids, int ids_are_i64, const int32_t* row_map,
                             const void* probs, int probs_dtype, int topk, int64_t T, void* out, hipStream_t st);

@@ -398,32 +398,36 @@ static int launch_few(GemmParams p, int64_t M, hipStream_t st, const FewSource& 
   return AAMD_OK;
 }
 
-// `split`: the form for launches of few workgroups, which divides the contraction among eight waves and takes half the
-// weight rows and token rows per workgroup.
-template <typename OUT>
-static int launch_few_as(const GemmParams& p, int64_t M, bool split, bool r_rows, hipStream_t st) {
-  if (r_rows) return launch_few<OUT, 4, 4, 1, true>(p, M, st);
-  return split ? launch_few<OUT, 8, 1, 1, false>(p, M, st) : launch_few<OUT, 4, 2, 2, false>(p, M, st);
+// `waves`: eight in the split form for launches of few workgroups, which takes half the weight rows and token rows per workgroup; four;
+// two or one for many workgroups of a short contraction (see choose_nt).
+template <typename OUT, typename IN>
+static int launch_few_as(const GemmParams& p, int64_t M, int waves, hipStream_t st, const FewSource& src = FewSource()) {
+  switch (waves) {
+    case 8: return launch_few<OUT, 8, 1, 1, false, IN>(p, M, st, src);
+    case 2: return launch_few<OUT, 2, 2, 2, false, IN>(p, M, st, src);
+    case 1: return launch_few<OUT, 1, 2, 2, false, IN>(p, M, st, src);
+    default: return launch_few<OUT, 4, 2, 2, false, IN>(p, M, st, src);
+  }
 }
-int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, bool split, bool r_rows, hipStream_t st) {
-  return c_dtype == AAMD_BF16 ? launch_few_as<u16>(p, M, split, r_rows, st) : launch_few_as<float>(p, M, split, r_rows, st);
+int launch_few_rows(const GemmParams& p, int c_dtype, int64_t M, int waves, bool r_rows, hipStream_t st) {
+  if (r_rows) return c_dtype == AAMD_BF16 ? launch_few<u16, 4, 4, 1, true>(p, M, st) : launch_few<float, 4, 4, 1, true>(p, M, st);
+  return c_dtype == AAMD_BF16 ? launch_few_as<u16, Codes>(p, M, waves, st) : launch_few_as<float, Codes>(p, M, waves, st);
 }
 
 int launch_few_rows_quantising(const GemmParams& p, int what, const void* rows, int64_t ld, const int64_t* sorted_idx, int topk, int64_t T,
-                               int64_t M, bool split, hipStream_t st) {
+                               int64_t M, int waves, hipStream_t st) {
   FewSource src = {};
   src.rows = (const u16*)rows; src.ld = ld; src.gate_off = (int64_t)p.nkb * kTile;
   src.sorted_idx = sorted_idx; src.topk = (uint32_t)topk; src.T = (uint32_t)T;
-  if (what == AAMD_ROWS_PERMUTED) return split ? launch_few<u16, 8, 1, 1, false, BF16>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, BF16>(p, M, st, src);
-  if (what == AAMD_ROWS_SWIGLU) return split ? launch_few<u16, 8, 1, 1, false, GLU>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, GLU>(p, M, st, src);
-  return split ? launch_few<u16, 8, 1, 1, false, GELU>(p, M, st, src) : launch_few<u16, 4, 2, 2, false, GELU>(p, M, st, src);
+  if (what == AAMD_ROWS_PERMUTED) return launch_few_as<u16, BF16>(p, M, waves, st, src);
+  return what == AAMD_ROWS_SWIGLU ? launch_few_as<u16, GLU>(p, M, waves, st, src) : launch_few_as<u16, GELU>(p, M, waves, st, src);
 }
 int launch_few_rows_routing(const GemmParams& p, const void* ids, int ids_are_i64, const void* rows, int64_t ld, int topk, int64_t T,
-                            int64_t* sorted_idx, int32_t* row_map, int64_t* goff, bool split, hipStream_t st) {
+                            int64_t* sorted_idx, int32_t* row_map, int64_t* goff, int waves, hipStream_t st) {
   FewSource src = {};
   src.rows = (const u16*)rows; src.ld = ld; src.topk = (uint32_t)topk; src.T = (uint32_t)T;
   src.ids = ids; src.ids_are_i64 = ids_are_i64; src.sorted_out = sorted_idx; src.map_out = row_map; src.goff_out = goff;
-  return split ? launch_few<u16, 8, 1, 1, false, Choices>(p, p.Lrows, st, src) : launch_few<u16, 4, 2, 2, false, Choices>(p, p.Lrows, st, src);
+  return launch_few_as<u16, Choices>(p, p.Lrows, waves, st, src);
 }
 
 // The second GEMM of a decoding step with the weighted combine in it: out[t] = sum over the slots j of probs[t, j] (b[e_j] act(row_j)),
