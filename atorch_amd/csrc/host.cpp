@@ -338,8 +338,8 @@ Routing alloc_routing(const Tensor& ids, int64_t E, bool want_sorted) {
 }
 void run_routing(const Routing& r, const Tensor& ids, int64_t E) {
   const int64_t n = ids.numel();
-  // (the one-workgroup form needs no scratch)
-  Tensor ws = aamd_route_one_workgroup(n, E) ? Tensor() : empty({std::max<int64_t>(1, aamd_moe_preprocess_ws_ints(n, (int)E))}, at::kInt, ids);
+  // (one workgroup needs no scratch)
+  Tensor ws = !aamd_route_takes_scratch(n, E) ? Tensor() : empty({std::max<int64_t>(1, aamd_moe_preprocess_ws_ints(n, (int)E))}, at::kInt, ids);
   check(aamd_moe_preprocess(ptr(ids), ids.scalar_type() == at::kLong, n, (int)E, raw<int64_t>(r.sorted_idx), ptr<int32_t>(r.row_map),
                             ptr<int64_t>(r.goff), raw<int32_t>(ws), stream()));
 }

@@ -528,7 +528,7 @@ __global__ __launch_bounds__(256) void route_place_kernel(const ID* __restrict__
 
 // ---------------------------------------------------------------------------------------
 // The same sort for fewer ids, with fewer launches (each of the four above is latency: 2 to 5 us whatever n is).
-// Up to 8192 ids: one workgroup does it all, ids and ranks in registers, counts of every (64 ids, expert) in LDS.
+// Up to 3072 ids, or 8192 without scratch: one workgroup does it all, ids and ranks in registers, counts of every (64 ids, expert) in LDS.
 // ---------------------------------------------------------------------------------------
 // exclusive prefix of tot[0 .. E) into base[0 .. E), by one wave; returns the sum of all
 __device__ __forceinline__ int wave_exclusive_prefix(const int* tot, int* base, int E) {
@@ -1042,7 +1042,7 @@ extern "C" int aamd_moe_preprocess(const void* expert_ids, int ids_are_i64, int6
   AAMD_REQUIRE(group_offsets && (ws || aamd_route_one_workgroup(n, E)), "moe_preprocess: group_offsets / ws required");
   AAMD_REQUIRE(n == 0 || (expert_ids && row_map), "moe_preprocess: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  if (aamd_route_one_workgroup(n, E)) {
+  if (!aamd_route_takes_scratch(n, E) || ws == nullptr) {
     const int64_t small_lds = aamd_route_small_lds(n, E);
     if (ids_are_i64)
       route_small_kernel<int64_t><<<1, 1024, (size_t)small_lds, st>>>((const int64_t*)expert_ids, (int)n, E, sorted_idx, row_map, group_offsets);
