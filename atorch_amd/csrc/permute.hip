@@ -113,7 +113,7 @@ __global__ __launch_bounds__(1024) void unpermute_combine_kernel(const typename 
 // ---------------------------------------------------------------------------------------
 // plain row permute: 16-byte chunks, each source row read once and written topk times
 // ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void permute_rows_kernel(const v4i* __restrict__ x, int chunks,
+__global__ __launch_bounds__(1024) void permute_rows_kernel(const v4i* __restrict__ x, int chunks,
                                                            const int32_t* __restrict__ row_map, int topk,
                                                            int64_t M_out, v4i* __restrict__ out) {
   const int64_t t = blockIdx.x;
@@ -827,6 +827,19 @@ static int threads_for_one_row(int64_t chunks) {
   return (int)(((chunks + trips - 1) / trips + 63) / 64 * 64);
 }
 
+// The same for rows that are only copied (permute_rows_kernel), which 256 lanes took in as many trips as it needs, each of them a round
+// trip to memory.  Up to 256 chunks 256 lanes all the same (64 to 160 with eight copies up to 6 % slower with as many lanes as chunks);
+// else up to 1024 where the launch is few workgroups to a CU, and up to 512 beyond (13921 tokens, 544 chunks, 8 copies 1.06 of the time
+// with 512, 1.08 with 1024; this splits them 320 and 224).  us, 256 lanes -> this: 85 tokens, fp32 6784, two copies 6.5 -> 3.9; 570, fp32
+// 1152, four 4.7 -> 3.3; 978, fp32 1792, eight 14.1 -> 11.7; 8191, bf16 4096, two 40.0 -> 38.0 (5.3 TB/s of one read and two writes); 56
+// drawn launches 0.845 of the time, the slowest 1.03.  Reading the rows in the order of the copies instead, so that these are one
+// sweep: 39.3 -> 41 to 46, eight copies 54 -> 67.
+static unsigned threads_for_copies(int64_t chunks, int64_t T) {
+  if (chunks <= 256) return 256;
+  const int64_t most = T <= 2048 ? 1024 : 512, trips = (chunks + most - 1) / most;
+  return (unsigned)(((chunks + trips - 1) / trips + 63) / 64 * 64);
+}
+
 extern "C" int aamd_bias_gather_add(const void* inp, const void* bias, const void* bin_ids, int ids_are_i64, int64_t T,
                                     int64_t H, int E, int dtype, void* out, void* stream) {
   AAMD_REQUIRE(dtype == AAMD_BF16 || dtype == AAMD_F32, "bias_gather_add: unsupported dtype %d", dtype);
@@ -1005,8 +1018,8 @@ extern "C" int aamd_permute_rows(const void* x, int x_dtype, int64_t T, int64_t 
   if (T == 0 || cols == 0) return AAMD_OK;
   AAMD_REQUIRE(x && out && row_map, "permute_rows: null pointer");
   AAMD_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "permute_rows: pointers must be 16-byte aligned");
-  permute_rows_kernel<<<(unsigned)T, 256, 0, (hipStream_t)stream>>>((const v4i*)x, (int)(row_bytes / 16), row_map, topk,
-                                                                    M_out, (v4i*)out);
+  permute_rows_kernel<<<(unsigned)T, threads_for_copies(row_bytes / 16, T), 0, (hipStream_t)stream>>>(
+      (const v4i*)x, (int)(row_bytes / 16), row_map, topk, M_out, (v4i*)out);
   AAMD_LAUNCH_CHECK("permute_rows");
   return AAMD_OK;
 }
