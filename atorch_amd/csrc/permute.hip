@@ -132,7 +132,7 @@ __global__ __launch_bounds__(1024) void permute_rows_kernel(const v4i* __restric
 // multiply in token_dispatcher.py:156-158: the product in the promoted type, cast to the rows' type).
 // ---------------------------------------------------------------------------------------
 template <typename IN, typename OUT, int PD>
-__global__ __launch_bounds__(256) void permute_rows_scaled_kernel(const typename IN::elem* __restrict__ x, int64_t cols,
+__global__ __launch_bounds__(1024) void permute_rows_scaled_kernel(const typename IN::elem* __restrict__ x, int64_t cols,
                                                                   const int32_t* __restrict__ row_map, int topk,
                                                                   const void* __restrict__ probs, int64_t M_out,
                                                                   typename OUT::elem* __restrict__ out) {
@@ -827,7 +827,7 @@ static int threads_for_one_row(int64_t chunks) {
   return (int)(((chunks + trips - 1) / trips + 63) / 64 * 64);
 }
 
-// The same for rows that are only copied (permute_rows_kernel), which 256 lanes took in as many trips as it needs, each of them a round
+// The same for rows that are only copied (permute_rows_kernel; permute_rows_scaled_kernel takes it in part), which 256 lanes took in as many trips as it needs, each of them a round
 // trip to memory.  Up to 256 chunks 256 lanes all the same (64 to 160 with eight copies up to 6 % slower with as many lanes as chunks);
 // else up to 1024 where the launch is few workgroups to a CU, and up to 512 beyond (13921 tokens, 544 chunks, 8 copies 1.06 of the time
 // with 512, 1.08 with 1024; this splits them 320 and 224).  us, 256 lanes -> this: 85 tokens, fp32 6784, two copies 6.5 -> 3.9; 570, fp32
@@ -952,8 +952,11 @@ extern "C" int aamd_permute_rows_scaled(const void* x, int x_dtype, int64_t T, i
   AAMD_REQUIRE(x && out && row_map && (probs || probs_dtype == AAMD_NONE), "permute_rows_scaled: null pointer");
   AAMD_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "permute_rows_scaled: pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  // (write bound: 256 lanes and several trips over the row measured faster at top-8 than one trip of up to 1024)
-  dim3 grid((unsigned)T), block(256);
+  // 256 lanes where the launch fills the card, and with many fp32 copies, whose halves of a lane's 32 bytes are stored apart (226 tokens,
+  // 6400 fp32, eight copies 15.4 us, with 800 lanes 18.8); else a lane per eight columns, bf16 copies: 123 tokens, 6528, eight 11.7 ->
+  // 4.9; 1241, 2176, four 8.1 -> 5.7; 1307, 5760, eight 32.8 -> 29.0.  fp32 ones: 285, 2304, two 4.3 -> 3.6.
+  const bool few = T <= 2048 && (out_dtype == AAMD_BF16 || topk <= 2);
+  dim3 grid((unsigned)T), block(few ? threads_for_copies(cols / 8, T) : 256u);
 #define AAMD_PRS(IN_, OUT_, PD_)                                                                                          \
   permute_rows_scaled_kernel<IN_, OUT_, PD_><<<grid, block, 0, st>>>((const IN_::elem*)x, cols, row_map, topk, probs, M_out, \
                                                                      (OUT_::elem*)out)

@@ -1,4 +1,4 @@
-"""The plain row permute at the edges of its rule for lanes per row: 256 chunks of 16 bytes and one more, 512 and 1024 and one more, and
+"""The row permutes at the edges of their rules for lanes per row: 256 chunks of 16 bytes and one more, 512 and 1024 and one more, and
 2048 tokens and one more; with copies that are dropped or lie beyond the output, whose places stay as they are."""
 import pytest
 import torch
@@ -24,3 +24,19 @@ def test_permute_rows_copies_every_chunk(dev, T, chunks, dtype, topk):
     held, got, place = x.to(dev), torch.full((rows + 1, cols), 7.0, dtype=dtype, device=dev), place.to(dev)
     _lib.check(_lib.lib().aamd_permute_rows(held.data_ptr(), kernels.dtype_code(dtype), T, cols, place.data_ptr(), topk, rows, got.data_ptr(), _lib.stream()))
     assert torch.equal(got[:rows].cpu(), want) and torch.all(got[rows] == 7.0)
+
+
+@pytest.mark.parametrize("T", [1, 2048, 2049])
+@pytest.mark.parametrize("eights", [1, 256, 257, 1024, 1025])
+@pytest.mark.parametrize("dtype,out_dtype,topk", [(torch.bfloat16, torch.bfloat16, 3), (torch.float32, torch.bfloat16, 1), (torch.float32, torch.float32, 2), (torch.float32, torch.float32, 3)])
+def test_permute_rows_scaled_rounds_one_product(dev, T, eights, dtype, out_dtype, topk):
+    from atorch_amd import kernels
+
+    n, cols = T * topk, eights * 8
+    g = torch.Generator().manual_seed(T + eights)
+    place = torch.randperm(n, generator=g)
+    x, probs = torch.randn((T, cols), generator=g).to(dtype), torch.rand((T, topk), generator=g).to(dtype)
+    want = torch.empty((n, cols), dtype=out_dtype)
+    want[place] = (x.float().repeat_interleave(topk, 0) * probs.float().reshape(-1, 1)).to(out_dtype)
+    got = kernels.permute_rows_scaled(x.to(dev), place.to(torch.int32).to(dev), topk, n, probs.to(dev), out_dtype)
+    assert torch.equal(got.cpu(), want)
