@@ -1340,7 +1340,10 @@ static int few_rows_waves(NtKernel k) { return k == kFewRowsSplit ? 8 : k == kFe
 // How many waves share the contraction of a 64 x 64 block: a CU holds two blocks of four waves, four of two or eight of one, with as
 // many loads in flight.  With fewer waves there is less to add up at the end, and 513 to 1024 (2048) blocks are no second round: 544
 // blocks of 4 steps 8.9 us with four, 7.3 with two, 512 blocks 6.5 and 6.9; 1440 blocks of few rows, of 1 / 2 / 4 / 8 / 16 steps,
-// four waves 11.1 / 11.6 / 15.2 / 20.5 / 31.8, one 5.6 / 6.4 / 11.2 / 17.5 / 30.0.  The lines lie where the mean of 12400 drawn launches
+// four waves 11.1 / 11.6 / 15.2 / 20.5 / 31.8, one 5.6 / 6.4 / 11.2 / 17.5 / 30.0.  The blocks of a
+// launch without groups are known, and 512 (1024) are a round of four (two) waves yet: 512 blocks of 4 / 8 / 16 steps 6.2 / 7.5 / 10.6 with
+// four, 6.6 / 8.4 / 11.9 with two; 516 8.4 / 10.5 / 14.3 and 6.8 / 8.9 / 12.4; 1024 8.2 / 12.2 / 18.8 with two, 8.6 / 13.8 / 19.8 with one.
+// Of groups the lines lie where the mean of 12400 drawn launches
 // (1 to 64 groups, 8 to 6000 rows, 512 to 5120 outputs and a contraction of 256 to 5120, replayed in a graph) turns; past 20 steps, or
 // 14 with weights beyond the last-level cache, the weights' stream bounds such launches (64 groups of 6 rows, 7168 x 2048: 164 with four,
 // 168 with one).  With these forms and their estimates those launches take 0.964 of the time, 18 % of them 3 % or more less, 0.9 % more
@@ -1387,7 +1390,8 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
 
   const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_s = token_tiles(32) * (double)(N / 32);
   const bool fewer_waves = !b_rows && nkb < (weights <= 256.0 ? 20 : 14);
-  const bool one_wave = fewer_waves && blocks_f >= (nkb < 4 ? 724.0 : 1024.0), two_waves = fewer_waves && !one_wave && blocks_f >= 500.0;
+  const bool one_wave = fewer_waves && blocks_f >= (nkb < 4 ? 724.0 : one ? 1025.0 : 1024.0);
+  const bool two_waves = fewer_waves && !one_wave && blocks_f >= (one ? 513.0 : 500.0);
   const double few = one_wave    ? std::max({5.8 + 1e-3 * blocks_f * (1.135 * n + 0.26), 4.4 + 0.64 * n, weights / 6.8})
                      : two_waves ? std::max({5.3 + 1e-3 * blocks_f * (1.135 * n + 1.1), 4.5 + 0.65 * std::ceil(n / 2.0), weights / 6.8})
                                  : std::max({4.5 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
@@ -1402,6 +1406,15 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   // counts while power does not bound the launch.  Persistent over this form, 486 launches of at most a round, mean ratio: up to 0.25
   // rounds 1.01, 0.5 1.02, 0.75 1.04 (the most 1.11), 1 1.02; 1 to 1.5 0.99, 2 0.97, more 0.94 to 0.97.
   return tiles_l * per_l <= 1.0 ? kLargeOnce : kLargeTiles;
+}
+// Tiles of up to 288 rows: the kernel decides by the groups' rows (0), where there can be enough remainders (32 rows more save a group at
+// most 48 - 17 64ths of a tile, and every tile costs 4 to 7: not with more than seven a group; nor with much less than one) and
+// the 1 to 2 us that deciding takes are little (launches of fewer R tiles, 60 uneven groups, 131 us: 1 to 2 % of them).
+static int choose_higher(const GemmParams& p, bool parts) {
+  if (p.goff != nullptr)
+    return p.E > 64 || p.Lrows >= (int64_t)7 * kLargeTile * p.E || p.Lrows < (int64_t)kLargeTile * 15 / 16 * p.E || p.nRt < 16 || p.nRt > 1024 ? -1 : 0;
+  const uint32_t full = (uint32_t)std::min<int64_t>(p.Lrows / kLargeTile, 8), over = (uint32_t)(p.Lrows % kLargeTile), more = (over + 31) / 32;
+  return over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, (uint32_t)p.higher_cost, parts, false) ? 1 : -1;
 }
 // Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
 static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
@@ -1514,17 +1527,9 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                   : launch_gemm<kRaggedRows, false, CfgLarge>(p, c_dtype, blocks, st, g_opt);
   if (large && !b_tile_scaled) {
     tile_order<kRaggedRows>(p, kLargeTile, g_opt);
-    // Tiles of up to 288 rows: the kernel decides by the groups' rows, where there can be enough remainders (32 rows more save a group at
-    // most 48 - 17 64ths of a tile, and every tile costs 4 to 7: not with more than seven a group; nor with much less than one) and
-    // the 1 to 2 us that deciding takes are little (launches of fewer R tiles, 60 uneven groups, 131 us: 1 to 2 % of them).
     p.slices = p.group_r && E <= 64 && p.nRt >= 32;
     p.higher_cost = (int)higher_tile_cost(p.nkb, p.slices);
-    if (g_opt.tile >= 0) p.higher = kernel == kLargeMore ? 1 : -1;
-    else if (group_offsets != nullptr) p.higher = E > 64 || M >= (int64_t)7 * kLargeTile * E || M < (int64_t)kLargeTile * 15 / 16 * E || p.nRt < 16 || p.nRt > 1024 ? -1 : 0;
-    else {
-      const uint32_t full = (uint32_t)std::min<int64_t>(M / kLargeTile, 8), over = (uint32_t)(M % kLargeTile), more = (over + 31) / 32;
-      p.higher = over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, (uint32_t)p.higher_cost, ws != nullptr, false) ? 1 : -1;
-    }
+    p.higher = g_opt.tile >= 0 ? (kernel == kLargeMore ? 1 : -1) : choose_higher(p, ws != nullptr);
     p.ws = ws;
     p.max_split = ws != nullptr ? row_max_split(p.nkb) : 1;
     return launch_row_tiles(p, c_dtype, blocks, b_rows, st);
@@ -1777,6 +1782,10 @@ extern "C" int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, co
   o.tile = opts[0]; o.group_r = opts[1]; o.gl = opts[2]; o.ls_batch = opts[3];
   return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, false, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
                       stream, o);
+}
+extern "C" int aamd_tuning_grouped_gemm_choice(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows, int workspace) {
+  if (M < 1 || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || (E > 1 && !grouped)) return -1;
+  return choose_nt(M, N, K / kBK, E, grouped != 0, b_rows != 0, workspace != 0, GemmOptions());
 }
 extern "C" int aamd_tuning_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b,
                                                const float* b_s, const int64_t* group_offsets, int E, int64_t M, int64_t N,

@@ -23,8 +23,9 @@ const char *aamd_probes_last_error(void);
  * The grouped GEMMs of the product library (same kernels, same arguments as aamd_grouped_gemm_fp8_nt, _nn and
  * aamd_grouped_gemm_fp8_wgrad) with the launch choices the library otherwise makes by itself pinned for
  * this one call: opts = {tile, group_r, gl, ls_batch}, each -1 for the library's own choice.
- *   tile: 0 = 128x128 tiles, 1 = 256x256 tiles, 2 / 3 = the kernel for few rows and its split form, 4 = 256x256 tiles with a
- *   workgroup each (1, 4: 128x128 tiles where the contraction has fewer than eight blocks; wgrad: 0 and 1 only);
+ *   tile: 0 = 128x128 tiles, 1 = 256x256 tiles, 2 / 3 = the kernel for few rows and its split form, 7 / 8 = with two waves
+ *   and with one, 4 = 256x256 tiles with a workgroup each, 6 = 256x256 tiles of up to 288 rows (1, 4, 6: 128x128 tiles where the
+ *   contraction has fewer than eight blocks; wgrad: 0 and 1 only);
  *   group_r: the tile order groups R tiles (1) or L tiles (0); gl: tiles sharing a panel in the tile order;
  *   ls_batch: 0 = the 128x128 tiles fetch their scales one contraction block at a time, the 256x256 tiles of the
  *   block-scaled GEMM, which take theirs in batches only, by 4-byte loads.
@@ -42,6 +43,12 @@ int aamd_tuning_grouped_gemm_fp8_wgrad(const uint8_t *dyt, const float *sdyt, co
                                        int64_t ld_t, int q_t_layout, const int64_t *group_offsets, int E,
                                        int32_t *tile_ws, int64_t N, int64_t K, void *dw, int dw_dtype,
                                        int64_t expert_stride, int accumulate, const int *opts, void *stream);
+
+/*
+ * The kernel that the product library takes for a row-ragged launch with block scales, as `tile` above; 5 = 1 with the contraction of its
+ * last tiles shared out; -1 for sizes it refuses.  grouped: with group offsets; b_rows: the weights of _nn; workspace: with one.
+ */
+int aamd_tuning_grouped_gemm_choice(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows, int workspace);
 
 /*
  * Shader clock probe (no counterpart in the reference; the benchmark reports the clock the GEMMs
