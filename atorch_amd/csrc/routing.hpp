@@ -9,7 +9,8 @@ inline bool aamd_route_one_workgroup(int64_t n, int64_t E) {
   return n <= kRouteSmallRounds * 1024 && aamd_route_small_lds(n, E) <= kRouteSmallLds;
 }
 // Whether it should, where there is scratch for the other forms: one workgroup takes 2.2 us and 1.25 to 1.7 for every 1024 ids, two
-// launches of a workgroup per 1024 ids 6.5 to 8 in all.  One and two, us, replayed in a graph: 8 experts, 3072 ids 6.1 and 6.5, 4096
-// 7.3 and 6.5, 8192 12.4 and 7.0; 60 experts 6.8 and 7.3, 8.3 and 7.2, 14.6 and 7.7; 128 experts 7.4 and 8.1, 9.2 and 8.2.
-constexpr int64_t kRouteSmallIds = 3072;
-inline bool aamd_route_takes_scratch(int64_t n, int64_t E) { return n > kRouteSmallIds || !aamd_route_one_workgroup(n, E); }
+// launches of a workgroup per 1024 ids 6 to 8 in all, and 10 with hundreds of experts, whose counts each of them adds up.  One and two, us,
+// replayed in a graph: 8 experts, 3328 ids 6.2 and 6.2, 4096 7.0 and 6.2, 8192 12.1 and 6.7; 60, 3328 6.9 and 7.0, 4096 8.0 and 6.8, 8192
+// 14.2 and 7.4; 128, 3584 7.9 and 7.8, 4096 8.8 and 7.7; 192, 3584 8.4 and 8.6, 4096 9.4 and 8.6; 236, 3584 8.6 and 9.4, 4096 9.8 and 9.2;
+// 300, 3073 8.7 and 10.4.
+inline bool aamd_route_takes_scratch(int64_t n, int64_t E) { return n > 3200 + 3 * E || !aamd_route_one_workgroup(n, E); }

@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,E", [(3072, 60), (3073, 60), (4096, 8), (8192, 8), (8193, 8), (3073, 300)])
+@pytest.mark.parametrize("n,E", [(3072, 60), (3073, 60), (3380, 60), (3381, 60), (4096, 8), (8192, 8), (8193, 8), (3073, 300), (3788, 196), (3789, 196)])
 @pytest.mark.parametrize("scratch", [True, False])
 def test_routing_line(dev, n, E, scratch):
     from atorch_amd import _lib
@@ -20,7 +20,9 @@ def test_routing_line(dev, n, E, scratch):
     place[order[:kept]] = torch.arange(kept, dtype=torch.int32)
     goff = torch.cat([torch.zeros(1, dtype=torch.int64), torch.bincount(ids[ids >= 0], minlength=E).cumsum(0)])
     held, got_order, got_place, got_goff = (t.to(dev) for t in (ids, torch.zeros_like(order), torch.zeros_like(place), torch.zeros_like(goff)))
-    ws = torch.empty(_lib.lib().aamd_moe_preprocess_ws_ints(n, E), dtype=torch.int32, device=dev) if scratch else None
+    ws = torch.full((_lib.lib().aamd_moe_preprocess_ws_ints(n, E),), -9, dtype=torch.int32, device=dev) if scratch else None
     _lib.check(_lib.lib().aamd_moe_preprocess(held.data_ptr(), 1, n, E, got_order.data_ptr(), got_place.data_ptr(), got_goff.data_ptr(),
                                               ws.data_ptr() if scratch else None, _lib.stream()))  # fmt: skip
+    if scratch:  # one workgroup leaves it alone
+        assert bool((ws == -9).all()) == (n <= 3200 + 3 * E)
     assert torch.equal(got_goff.cpu(), goff) and torch.equal(got_place.cpu(), place) and torch.equal(got_order[:kept].cpu(), order[:kept])
