@@ -243,7 +243,10 @@ __device__ __forceinline__ uint32_t row_split(uint32_t left, uint32_t nwg, uint3
 // pieces of 128 rows x 128 columns no more than these.
 __device__ __forceinline__ uint32_t row_shares(uint32_t left, uint32_t nwg) { return left == 0 || 2 * left > nwg ? 1 : 4 * left > nwg ? 2 : 4; }
 // The last row that is loaded (a share may have none, and then loads one).
-__device__ __forceinline__ int last_row(int valid) { return valid > 0 ? valid - 1 : 0; }
+__host__ __device__ constexpr int last_row(int valid) { return valid > 0 ? valid - 1 : 0; }
+// Bytes to the end of its block: 288 rows that are 8 MB apart are more than an int holds.
+__host__ __device__ constexpr uint32_t rows_end(int valid, int64_t ld) { return (uint32_t)last_row(valid) * (uint32_t)ld + kBK; }
+static_assert(rows_end(rows::high_tile(true), (1 << 23) - 1) == (int64_t)(rows::high_tile(true) - 1) * ((1 << 23) - 1) + kBK, "the rows of a tile are in reach of 32 bits");
 // First contraction block of a part: whole groups of four (16 bytes of scales) but for the end of the last part.  With
 // nkb >= 8 split every part has eight blocks or more.
 __device__ __forceinline__ uint32_t row_part(uint32_t nkb, uint32_t split, uint32_t part) {
@@ -425,7 +428,7 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
     const int block = t.kb0 + last;
     const int64_t l_at = t.l0 * a->ldl + block * kBK;
     const int64_t r_at = (int64_t)t.g * a->r_group_stride + (R_ROWS ? (int64_t)t.r0 : t.r0 * a->ldr) + block * a->r_kb_stride;
-    lbuf = buffer_at(a->L + uniform_i64(l_at), (uint32_t)__builtin_amdgcn_readfirstlane(last_row(t.lvalid) * (int)a->ldl + kBK));
+    lbuf = buffer_at(a->L + uniform_i64(l_at), (uint32_t)__builtin_amdgcn_readfirstlane((int)rows_end(t.lvalid, a->ldl)));
     rbuf = buffer_at(a->R + uniform_i64(r_at), (uint32_t)__builtin_amdgcn_readfirstlane(
                                                    R_ROWS ? 127 * (int)a->ldr + t.rvalid : (t.rvalid - 1) * (int)a->ldr + kBK));
     to_load = t.steps - last;

@@ -76,3 +76,19 @@ def test_parts_of_higher_tiles(dev, splits, N, K, out_dtype, turned):
     # (sums of nkb products of like size: an addition rounds by at most 2^-24 of a partial sum, which stays below sqrt(nkb) of the
     # result's root mean square times 4; two sums on either side of a rounding give neighbours in bf16, up to 2^-7 apart)
     assert rel_err(out[:M], want) <= nkb * 2.0**-24 * 4 + (2.0**-7 if out_dtype == torch.bfloat16 else 0.0)
+
+
+@pytest.mark.parametrize("splits", [[288], [287, 0, 1]])
+def test_rows_as_far_apart_as_is_taken(dev, splits):
+    """288 rows of nearly 8 MB: their last byte lies beyond what a signed 32-bit offset reaches."""
+    from atorch_amd import kernels
+
+    N, K, M, lda = 384, 1024, sum(splits), (1 << 23) - 16
+    qx, *rest = operands(dev, splits, N, K, False)
+    goff = kernels.group_offsets_from_splits(splits, dev)
+    far = torch.empty((M - 1) * lda + K, dtype=torch.uint8, device=dev).view(qx.dtype).as_strided((M, K), (lda, 1))
+    far.view(torch.uint8).copy_(qx.view(torch.uint8))
+    with kernels.gemm_options(tile=0):
+        want = kernels.grouped_gemm_nt(qx, *rest, goff)
+    with kernels.gemm_options(tile=6):
+        assert torch.equal(kernels.grouped_gemm_nt(far, *rest, goff), want)
