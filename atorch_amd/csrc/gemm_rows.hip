@@ -921,7 +921,7 @@ __device__ __forceinline__ void row_tiles(ARGS& p, uint8_t* const lds) {
 }
 
 // EITHER: with tiles of up to 32 rows more where the groups' rows make them worth it.  (A kernel of its own: holding both forms and
-// deciding take 1 to 2 us.)
+// deciding take 0.2 to 0.5 us.)
 template <typename OUT, bool R_ROWS, bool PAIRS, bool EITHER>
 __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams p) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[rows::lds_bytes(EITHER)];
@@ -935,9 +935,11 @@ __global__ __launch_bounds__(rows::NT, 1) void row_tiles_kernel(const GemmParams
       table[0] = of_lane.lo;
       table[1] = of_lane.hi;
     }  // (every wave writes the same values, and reads what it wrote)
-    // (each fetches its arguments itself: what both used would be fetched in front, and held)
+    // (the form of more rows fetches its arguments itself: what both used would be fetched in front, and held.  The other takes them as they
+    // come, all at once: a launch that decides against more rows, 4096 rows in 8 groups, 4736 x 1024 31.9 us without the choice, 32.1 with
+    // it, 32.7 where this form too fetched them one by one)
     if (higher_tiles(&p, of_lane)) row_tiles<OUT, R_ROWS, PAIRS, true, true>(*(args_t)(uintptr_t)args_here(), lds);
-    else row_tiles<OUT, R_ROWS, PAIRS, false, true>(*(args_t)(uintptr_t)args_here(), lds);
+    else row_tiles<OUT, R_ROWS, PAIRS, false, true>(p, lds);
   } else {
     row_tiles<OUT, R_ROWS, PAIRS, false, false>(p, lds);
   }
