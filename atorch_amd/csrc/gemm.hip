@@ -1407,14 +1407,15 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
   // rounds 1.01, 0.5 1.02, 0.75 1.04 (the most 1.11), 1 1.02; 1 to 1.5 0.99, 2 0.97, more 0.94 to 0.97.
   return tiles_l * per_l <= 1.0 ? kLargeOnce : kLargeTiles;
 }
-// Tiles of up to 288 rows: the kernel decides by the groups' rows (0), where there can be enough remainders (32 rows more save a group at
-// most 48 - 17 64ths of a tile, and every tile costs 4 to 7: not with more than seven a group; nor with much less than one) and
-// the 1 to 2 us that deciding takes are little (launches of fewer R tiles, 60 uneven groups, 131 us: 1 to 2 % of them).
+static bool takes_slices(const GemmParams& p) { return p.group_r && p.E <= 64 && p.nRt >= 32; }
+// Tiles of up to 288 rows: the kernel decides by the groups' rows (0), where there can be enough remainders (a group's own tile costs two
+// thirds of one, and its full tiles a twentieth of one each: not with more than seven of them; nor with much less than one) and the 0.2 to 0.5
+// us that deciding takes are little.
 static int choose_higher(const GemmParams& p, bool parts) {
   if (p.goff != nullptr)
     return p.E > 64 || p.Lrows >= (int64_t)7 * kLargeTile * p.E || p.Lrows < (int64_t)kLargeTile * 15 / 16 * p.E || p.nRt < 16 || p.nRt > 1024 ? -1 : 0;
   const uint32_t full = (uint32_t)std::min<int64_t>(p.Lrows / kLargeTile, 8), over = (uint32_t)(p.Lrows % kLargeTile), more = (over + 31) / 32;
-  return over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, (uint32_t)p.higher_cost, parts, false) ? 1 : -1;
+  return over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, parts, false) ? 1 : -1;
 }
 // Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
 static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
@@ -1527,8 +1528,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
                   : launch_gemm<kRaggedRows, false, CfgLarge>(p, c_dtype, blocks, st, g_opt);
   if (large && !b_tile_scaled) {
     tile_order<kRaggedRows>(p, kLargeTile, g_opt);
-    p.slices = p.group_r && E <= 64 && p.nRt >= 32;
-    p.higher_cost = (int)higher_tile_cost(p.nkb, p.slices);
+    p.slices = takes_slices(p);
     p.higher = g_opt.tile >= 0 ? (kernel == kLargeMore ? 1 : -1) : choose_higher(p, ws != nullptr);
     p.ws = ws;
     p.max_split = ws != nullptr ? row_max_split(p.nkb) : 1;
@@ -1783,9 +1783,29 @@ extern "C" int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, co
   return gemm_nt_impl(a, lda, a_s, b, b_s, b_tile_scaled, false, group_offsets, E, M, N, K, c, c_dtype, ldc, bias, bias_dtype,
                       stream, o);
 }
-extern "C" int aamd_tuning_grouped_gemm_choice(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows, int workspace) {
+extern "C" int aamd_tuning_grouped_gemm_choice(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows, int workspace,
+                                               const int64_t* host_offsets) {
   if (M < 1 || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || (E > 1 && !grouped)) return -1;
-  return choose_nt(M, N, K / kBK, E, grouped != 0, b_rows != 0, workspace != 0, GemmOptions());
+  const NtKernel kernel = choose_nt(M, N, K / kBK, E, grouped != 0, b_rows != 0, workspace != 0, GemmOptions());
+  if (kernel != kLargeTiles && kernel != kLargeShared) return kernel;
+  GemmParams p = {};
+  const int64_t none = 0;
+  p.goff = grouped ? (host_offsets ? host_offsets : &none) : nullptr;
+  p.Lrows = M; p.E = E; p.nRt = (int)((N + kLargeTile - 1) / kLargeTile);
+  tile_order<kRaggedRows>(p, kLargeTile, GemmOptions());
+  int higher = choose_higher(p, workspace != 0);
+  if (higher == 0 && host_offsets != nullptr) {  // what higher_tiles of gemm_rows.hip counts
+    uint32_t full = 0, own0 = 0, own1 = 0, shared = 0;
+    for (int e = 0; e < E; e++) {
+      const uint32_t rows = (uint32_t)(host_offsets[e + 1] - host_offsets[e]), f = rows / kLargeTile, more = (rows % kLargeTile + 31) / 32;
+      full += f;
+      own0 += more > 0;
+      own1 += more > f;
+      shared += more > f ? 0 : more;
+    }
+    higher = own0 != own1 && higher_tiles_pay(full, own0, own1, shared, (uint32_t)p.nRt, workspace != 0 && row_max_split(K / kBK) > 1, takes_slices(p));
+  }
+  return higher > 0 ? kLargeMore : kernel;
 }
 extern "C" int aamd_tuning_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b,
                                                const float* b_s, const int64_t* group_offsets, int E, int64_t M, int64_t N,

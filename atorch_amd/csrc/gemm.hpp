@@ -43,7 +43,6 @@ struct GemmParams {
   int max_split;   // row_tiles_kernel: the most parts of a tile's contraction; more than one: ws holds kRowPartsBytes
   float* ws;
   int higher;      // row_tiles_kernel: tiles of up to 288 rows (1), of 256 (-1), or as the groups' rows have it (0)
-  int higher_cost; // with these: of a tile, see higher_tiles_pay
   int slices;      // row_tiles_kernel with these: every XCD takes an eighth of every group
   int stream_out;  // row_tiles_kernel: the output is stored past the caches
   int ls_batch;    // kRaggedRows: L scales are fetched eight contraction blocks at a time
@@ -90,22 +89,28 @@ int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld
                             const void* probs, int probs_dtype, int topk, int64_t T, void* out, hipStream_t st);
 
 // Are tiles of more rows worth it?  They save the tiles of remainders, which fetch their weights once more whatever few rows they have
-// (us, 28672 outputs x 4096, 8 groups of 512 rows 430, 513 to 576 548 to 560, 640 595, 768 640), and cost every step and every tile
-// something, more where addresses are made in the step.  In 64ths of a tile, fitted to 500 launches of 2 to 60 groups of 250 to 1700
-// rows on average with both.  With slices: a remainder's own tile 38, 32 rows more 13, a tile that may have them 68; else 48, 17, and
-// 71 and 64 a step; launches of up to three rounds by their rounds.  Taken for 112 of those, 0.94 of the time on average, three 2 % slower
-// or more.  28672 x 4096 in 8 groups, plain tiles -> these: 485 to 542 rows, five above 512 601 -> 497, three 552 -> 488; 264
-// 388 -> 310, 520 582 -> 494; 60 of about 270, 7168 x 4096, 702 -> 611; not: 512 449 -> 473, 640 595 -> 632, about 4096 3377 -> 3654.
-inline uint32_t higher_tile_cost(int nkb, bool slices) { return slices ? 68 : 71 + 64 / (uint32_t)nkb; }
-__host__ __device__ inline bool higher_tiles_pay(uint32_t full, uint32_t own0, uint32_t own1, uint32_t shared, uint32_t nRt, uint32_t cost, bool parts, bool slices) {
-  const uint32_t n0 = (full + own0) * nRt, n1 = (full + own1) * nRt;
-  if (n0 <= 3 * 256) {  // rounds, in tenths; one that is shared out counts for 6
-    const uint32_t l0 = n0 % 256, l1 = n1 % 256, shares = parts ? 128 : 0;
-    const uint32_t r0 = n0 / 256 * 10 + (l0 == 0 ? 0 : l0 <= shares ? 6 : 10), r1 = n1 / 256 * 10 + (l1 == 0 ? 0 : l1 <= shares ? 6 : 10);
-    return 64 * r0 > 74 * r1;
-  }
-  const uint32_t own = slices ? 38 : 48, more = slices ? 13 * 64 : 17 * 64;
-  return 64 * (64 * full + own * own0) > cost * (64 * full + own * own1) + more * shared;
+// (us, 28672 outputs x 4096, 8 groups of 512 rows 430, 513 to 576 548 to 560, 640 595, 768 640), and cost every step something, more
+// where addresses are made in the step.  In 256ths of a tile: 270 for one of theirs and 60 for 32 rows more in it, 171 and 181 for a
+// remainder's own.  With few rounds a launch is as long as the workgroup whose tiles are all full, or all higher; and a round counts
+// whole, but for a last one of few tiles, which is shared out (the slices of an XCD may be a tile longer than the mean, where that
+// begins another round).  Counts are of an R tile, all in whole numbers: the kernels of a launch have to come to the same.
+// Fitted to 1091 launches with remainders, of 1 to 64 groups of 240 to 1790 rows on average, 4096 to 32768 outputs and a contraction of 1024
+// to 14336.  Of 1400 others it takes these for 303, 0.892 of the time, 7 of them 1 % slower or more, the worst 1.06 (the lines that this
+// replaces, without rounds past the third: 68 of 513, the worst 1.21); of 400 without groups for 31, 0.845, the slowest 0.98.  Plain tiles ->
+// these: 28672 x 4096 in 8 groups of about 512 524 -> 474, of 264 373 -> 302, of 520 558 -> 489.  No longer taken: 2339 rows in 8, 16128 x
+// 11392 555 -> 625; 2546 in 2, 9344 x 7680 185 -> 225; 6599 in 8, 4096 x 7424 200 -> 237.  Taken, and should not be: 1285 and 1286 rows,
+// 25856 x 3456 227 -> 251.
+__host__ __device__ inline uint32_t higher_tile_rounds(uint32_t n, uint32_t shared_out, bool parts) {  // in tiles
+  const uint32_t left = n & 255u;
+  return n - left + (left == 0 ? 0 : left > shared_out ? 256 : parts ? 92 + (164 * left >> 8) : 143 + (113 * left >> 8));
+}
+__host__ __device__ inline bool higher_tiles_pay(uint32_t full, uint32_t own0, uint32_t own1, uint32_t shared, uint32_t nRt, bool parts, bool slices) {
+  const uint32_t t0 = full + own0, t1 = full + own1, n0 = t0 * nRt, n1 = t1 * nRt;
+  const uint32_t w0 = 256 * full + 171 * own0, w1 = 270 * full + 181 * own1 + 60 * shared;  // of an R tile, if all workgroups had the same
+  const uint32_t d0 = 256 * t0 - w0, d1 = (shared > 0 ? 330 : 270) * t1 - w1;               // and what the longest has beyond
+  const uint32_t l0 = w0 + (n0 <= 210 ? d0 : 210 * d0 / n0), l1 = w1 + (n1 <= 210 ? d1 : 210 * d1 / n1);
+  const uint32_t r0 = higher_tile_rounds(n0, 128, parts), r1 = higher_tile_rounds(n1 + (slices ? 8 : 0), parts ? 112 : 128, parts);
+  return 32 * (uint64_t)r1 * l1 * t0 < 31 * (uint64_t)r0 * l0 * t1;
 }
 
 constexpr int64_t kRowPartsBytes = (int64_t)256 * kLargeTile * kLargeTile * 4;  // a tile of fp32 for each of 256 workgroups

@@ -110,7 +110,7 @@ __device__ __forceinline__ bool higher_tiles(ARGS p, const GroupRows& of_lane) {
   const uint32_t own0 = (uint32_t)__popcll(__ballot(over > 0)), own1 = (uint32_t)__popcll(__ballot(more > f));
   if (own0 == own1) return false;
   const uint32_t sums = (uint32_t)__builtin_amdgcn_readlane(wave_inclusive_sum((int)(f << 16 | (more > f ? 0u : more))), 63);
-  return higher_tiles_pay(sums >> 16, own0, own1, sums & 0xffffu, (uint32_t)p->nRt, p->higher_cost, p->max_split > 1, p->slices);
+  return higher_tiles_pay(sums >> 16, own0, own1, sums & 0xffffu, (uint32_t)p->nRt, p->max_split > 1, p->slices != 0);
 }
 // With MORE every XCD may take an eighth of every group's tiles, R tile by R tile with all L tiles of it: tiles of more rows are then
 // spread over all of them (with one range of tiles for each XCD the one whose groups had the most of them took longest: 8 groups,

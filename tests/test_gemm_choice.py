@@ -1,13 +1,17 @@
 """Which kernel a row-ragged launch takes, where the choice has a line."""
+import ctypes
+from itertools import accumulate
+
 import pytest
 
-FOUR, TWO, ONE, SMALL_TILES = 2, 7, 8, 0
+FOUR, TWO, ONE, SMALL_TILES, LARGE_TILES, SHARED, HIGHER = 2, 7, 8, 0, 1, 5, 6
 
 
-def choice(M, N, steps, E=1, grouped=0, b_rows=0, workspace=0):
+def choice(M, N, steps, E=1, grouped=0, b_rows=0, workspace=0, splits=None):
     from atorch_amd import _probes
 
-    return _probes.lib().aamd_tuning_grouped_gemm_choice(M, N, 128 * steps, E, grouped, b_rows, workspace)
+    offsets = (ctypes.c_int64 * (E + 1))(0, *accumulate(splits)) if splits else None
+    return _probes.lib().aamd_tuning_grouped_gemm_choice(M, N, 128 * steps, E, grouped, b_rows, workspace, offsets)
 
 
 @pytest.mark.parametrize("grouped", [0, 1])
@@ -22,3 +26,23 @@ def test_blocks_that_are_known_and_fill_a_round(grouped, steps):
     if steps >= 4:
         assert choice(64, 65536, steps, grouped=grouped) in (TWO, SMALL_TILES)
         assert choice(64, 65664, steps, grouped=grouped) in (ONE, SMALL_TILES)
+
+
+# (us, tiles of 256 rows and of up to 288)
+@pytest.mark.parametrize("splits,N,K,workspace,higher", [
+    ([485, 505, 513, 520, 500, 516, 515, 542], 28672, 4096, 0, True),  # 524, 474
+    ([264] * 8, 28672, 4096, 0, True), ([520] * 8, 28672, 4096, 0, True), ([280, 277, 265], 15488, 3584, 0, True),  # 373, 302; 558, 489; 82, 62
+    ([285, 300, 276, 310, 292, 281, 302, 293], 16128, 11392, 1, False),  # 555, 625
+    ([1250, 1296], 9344, 7680, 1, False),  # 185, 225
+    ([1160, 1130, 1135], 9984, 4224, 0, False),  # 153, 179: 507 tiles, of which an XCD has 65
+    ([820] * 8, 4096, 7424, 1, False), ([512] * 8, 28672, 4096, 0, False), ([640] * 8, 28672, 4096, 0, False),  # 200, 237; 449, 473; 595, 632
+])  # fmt: skip
+def test_higher_tiles_where_they_are_faster(splits, N, K, workspace, higher):
+    got = choice(sum(splits), N, K // 128, len(splits), 1, 0, workspace, splits)
+    assert got == HIGHER if higher else got in (LARGE_TILES, SHARED)
+
+
+def test_higher_tiles_of_one_group_and_of_none():
+    for M, N, steps, workspace, higher in ((1288, 12032, 8, 0, True), (1032, 13312, 48, 1, True), (1280, 12032, 8, 0, False), (1300, 16384, 32, 0, False)):
+        assert (choice(M, N, steps, workspace=workspace) == HIGHER) == higher
+        assert (choice(M, N, steps, 1, 1, 0, workspace, [M]) == HIGHER) == higher
