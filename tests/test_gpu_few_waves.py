@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from helpers import rel_err
+from test_gemm_choice import ONE, choice
 
 pytestmark = pytest.mark.gpu
 
@@ -43,13 +44,20 @@ def test_fewer_waves(dev, splits, N, K, out_dtype, bias):
     assert rel_err(got[7][:M], got[0][:M]) <= tolerance(K, out_dtype)
 
 
-# 64 x 64 blocks the library expects: 480, 512, 720, 736, 1008, 1024 and 2400 of uneven groups
-@pytest.mark.parametrize("splits,N", [([1920], 1024), ([2048], 1024), ([2880], 1024), ([2944], 1024), ([4032], 1024), ([4096], 1024), ([3, 40, 0, 100] * 15, 2560)])
-@pytest.mark.parametrize("K", [256, 384, 512, 2432, 2560])
-def test_chosen_by_blocks(dev, splits, N, K):
+# 64 groups of six rows on average, 62 of which the library expects to have any: 498, 623, 747, 997, 1121, 1744 and 2243 blocks around its lines
+# at 500, 724 and 1024, with 2 to 20 steps around those at 4, 14 (weights of 256 MB and more) and 20; and one group of 512, 516, 1024 and 1032
+@pytest.mark.parametrize("splits,N", [([3, 0, 15, 2, 5, 8, 6, 9] * 8, n) for n in (512, 640, 768, 1024, 1152, 1792, 2304)]
+                         + [([64], n) for n in (32768, 33024, 65536, 66048)])  # fmt: skip
+@pytest.mark.parametrize("K", [256, 384, 512, 1664, 1792, 2432, 2560])
+@pytest.mark.parametrize("out_dtype", [torch.float32])
+def test_what_is_chosen_at_the_lines(dev, splits, N, K, out_dtype):
     from atorch_amd import kernels
 
+    kernel = choice(sum(splits), N, K // 128, len(splits), 1)
     ops = operands(dev, splits, N, K)
-    got = kernels.grouped_gemm_nt(*ops, out_dtype=torch.float32)
+    got = kernels.grouped_gemm_nt(*ops, out_dtype=out_dtype)
+    with kernels.gemm_options(tile=kernel):  # the library takes what it says
+        assert torch.equal(got, kernels.grouped_gemm_nt(*ops, out_dtype=out_dtype))
     with kernels.gemm_options(tile=0):
-        assert rel_err(got, kernels.grouped_gemm_nt(*ops, out_dtype=torch.float32)) <= tolerance(K, torch.float32)
+        want = kernels.grouped_gemm_nt(*ops, out_dtype=out_dtype)
+    assert torch.equal(got, want) if kernel == ONE else rel_err(got, want) <= tolerance(K, out_dtype)

@@ -5,8 +5,21 @@ import pytest
 import torch
 
 from helpers import randn_bf16
+from test_gemm_choice import FOUR, ONE, TWO, choice
 
 pytestmark = pytest.mark.gpu
+
+# (T, k, E, N, K) of 64 x 64 blocks with four waves, two and one: an odd number of steps, fewer steps than waves, groups of more rows than are
+# requested ahead, and more than 64 groups
+FEWER_WAVES = [((32, 2, 2, 8192, 1024), FOUR), ((8, 8, 32, 1408, 384), FOUR), ((8, 8, 64, 2048, 1408), TWO), ((8, 8, 256, 1024, 512), TWO), ((32, 2, 2, 16384, 1152), TWO),
+               ((1, 8, 64, 8192, 128), TWO), ((8, 8, 128, 2048, 768), ONE), ((8, 8, 64, 4096, 1024), ONE), ((32, 2, 8, 8192, 384), ONE),
+               ((40, 1, 3, 16384, 256), ONE)]  # fmt: skip
+
+
+@pytest.mark.parametrize("shape,kernel", FEWER_WAVES)
+def test_the_forms_of_these_sizes(shape, kernel):
+    T, k, E, N, K = shape
+    assert choice(T * k, N, K // 128, E, 1) == kernel
 
 
 def fused(what, rows, sorted_idx, topk, q, s, goff, bias, M):
@@ -24,6 +37,7 @@ def fused(what, rows, sorted_idx, topk, q, s, goff, bias, M):
 @pytest.mark.parametrize("T,k,E,N,K", [
     (1, 4, 60, 2816, 2048), (1, 1, 1, 128, 128), (16, 2, 2, 256, 1152), (32, 1, 1, 512, 640), (5, 3, 8, 4096, 1024), (8, 4, 64, 1024, 7168),
     (13, 2, 4, 1408, 384), (2, 8, 70, 2048, 1408),
+    *[shape for shape, _ in FEWER_WAVES],
 ])  # fmt: skip
 @pytest.mark.parametrize("what", [0, 1, 2], ids=["permuted", "swiglu", "gelu"])
 @pytest.mark.parametrize("bias", [None, torch.bfloat16, torch.float32])
@@ -34,7 +48,10 @@ def test_bits_of_the_two_launches(dev, T, k, E, N, K, what, bias):
     g = torch.Generator().manual_seed(T + 100 * what)
     ids = torch.stack([torch.randperm(E, generator=g)[:k] if E >= k else torch.randint(E, (k,), generator=g) for _ in range(T)]).to(dev)
     sorted_idx, row_map, goff = kernels.moe_preprocess(ids, E)
-    w = randn_bf16((E, N, K), 3, std=0.05).to(dev)
+    if (T, k, E, N, K) in dict(FEWER_WAVES):  # (many weights: made on the device)
+        w = torch.randn((E, N, K), generator=torch.Generator(device=dev).manual_seed(3), device=dev).bfloat16() * 0.05
+    else:
+        w = randn_bf16((E, N, K), 3, std=0.05).to(dev)
     q, s, _, _ = kernels.block_quant_batched(w)
     b = torch.randn((E, N), generator=g).to(dev).to(bias) if bias is not None else None
     x = randn_bf16((T if what == 0 else M, K * (2 if what == 1 else 1)), 5).to(dev)

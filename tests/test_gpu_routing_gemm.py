@@ -1,5 +1,5 @@
 """The GEMM of few rows that makes the routing itself: the tables of the router preprocess and the bits of the GEMM that reads them, for
-one pair to the most, dropped and repeated choices, more experts than lanes, both forms of the kernel and both id types."""
+one pair to the most, dropped and repeated choices, more experts than lanes, blocks of eight waves, two (8 of 64, 8 of 256) and one (8 of 128, 2 of 8), and both id types."""
 import pytest
 import torch
 
@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,k,E,N,K", [(1, 1, 1, 128, 128), (1, 4, 60, 2816, 2048), (16, 4, 64, 256, 384), (64, 1, 3, 512, 640), (8, 8, 64, 2048, 1152),
-                                       (7, 9, 65, 128, 1024), (13, 2, 130, 384, 256), (2, 3, 1024, 128, 128)])  # fmt: skip
+                                       (7, 9, 65, 128, 1024), (13, 2, 130, 384, 256), (2, 3, 1024, 128, 128),
+                                       (8, 8, 128, 2048, 768), (8, 8, 256, 1024, 512), (32, 2, 8, 8192, 384)])  # fmt: skip
 @pytest.mark.parametrize("drop", ["none", "some", "all"])
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
 def test_tables_and_bits(dev, T, k, E, N, K, drop, dtype):
@@ -22,7 +23,8 @@ def test_tables_and_bits(dev, T, k, E, N, K, drop, dtype):
         out = torch.rand((T, k), generator=g) < (0.4 if drop == "some" else 2.0)
         ids[out] = torch.where(torch.rand(int(out.sum()), generator=g) < 0.5, -1 - E, E)
     ids = ids.to(dtype).to(dev)
-    q, s, _, _ = kernels.block_quant_batched(randn_bf16((E, N, K), 3, std=0.05).to(dev))
+    w = torch.randn((E, N, K), generator=torch.Generator(device=dev).manual_seed(3), device=dev) * 0.05
+    q, s, _, _ = kernels.block_quant_batched(w.bfloat16())
     bias = torch.randn((E, N), generator=g).to(dev)
     x = randn_bf16((T, K), 5).to(dev)
     sorted_idx, row_map, goff = kernels.moe_preprocess(ids, E)
