@@ -1300,10 +1300,10 @@ static int launch_gemm(GemmParams p, int c_dtype, int64_t blocks, hipStream_t st
   return AAMD_OK;
 }
 
-// The 256 x 256 tiles' last round may share out its contraction (row_tiles_kernel) from this many blocks on.  Measured on MI355X,
-// us, without and with, 4096 outputs, one round of 256 tiles and a last one of 1 / 4 / 8 / 12 / 16 tiles per XCD (in 8 / 8 / 4 / 2 /
-// 2 parts): 48 blocks 148 / 150 / 154 / 157 / 161 -> 123 / 128 / 138 / 149 / 159, 64 blocks 193 / 197 / 203 / 206 / 210 -> 155 /
-// 163 / 170 / 187 / 200, 112 blocks 327 / 337 / 345 / 349 / 354 -> 245 / 256 / 273 / 303 / 322; 32 blocks, 16 tiles 112 -> 122.
+// The 256 x 256 tiles' last round may share out its contraction (row_tiles_kernel) from this many blocks on; shorter ones share rows (row_shares).
+// us, rows shared and contraction shared, 2048 outputs, one round of 256 tiles and a last one of 1 / 4 / 8 / 12 / 16 tiles per XCD (in 8 / 8 /
+// 4 / 2 / 2 parts): 40 blocks 113 / 113 / 115 / 125 / 130 and 103 / 107 / 119 / 125 / 134, 48 133 / 133 / 136 / 148 / 152 and 118 / 124 / 133 /
+// 142 / 153, 64 173 / 174 / 178 / 192 / 197 and 148 / 156 / 164 / 178 / 190, 112 295 / 296 / 301 / 317 / 325 and 234 / 250 / 267 / 293 / 312.
 // Where nothing is shared the second launch costs 2 to 6 us of at least 100 (choose_nt).
 constexpr int kSplitBlocks = 48;
 // The most parts of a contraction: eight blocks at least in each, see row_part.
@@ -1346,9 +1346,11 @@ static int few_rows_waves(NtKernel k) { return k == kFewRowsSplit ? 8 : k == kFe
 // Of groups the lines lie where the mean of 12400 drawn launches
 // (1 to 64 groups, 8 to 6000 rows, 512 to 5120 outputs and a contraction of 256 to 5120, replayed in a graph) turns; past 20 steps, or
 // 14 with weights beyond the last-level cache, the weights' stream bounds such launches (64 groups of 6 rows, 7168 x 2048: 164 with four,
-// 168 with one).  With these forms and their estimates those launches take 0.964 of the time, 18 % of them 3 % or more less, 0.9 % more
-// (64 uneven groups, 335 rows, 2176 x 3072 74 -> 83).  The forms that quantise their rows take the same, and give the same bits: eight
-// tokens to 8 of 128 experts, 2048 x 768, layer 59 -> 53, 256, 1024 x 512 36 -> 33.
+// 168 with one).  Of 14351 others, even and Zipf, 4000 take these forms, 0.819 of the time, 83 of them 3 % slower or more (2414 rows in 61,
+// 512 x 896 7.0 -> 8.3; 1742 in 23, 2560 x 1024 19.7 -> 23.3); with two thirds of the groups empty, which the host does not know, 0.853 and a
+// fifth of them (86 rows in 7 of 32, 2560 x 2048 9.4 -> 13.7).  A wave's chain of sums is as much longer, one wave's the tiles' own; against
+// 64-bit sums all are off by the same, 1.42e-5 in fp32 (19 steps).  The forms that quantise their rows take the same, and give the same bits:
+// eight tokens to 8 of 128 experts, 2048 x 768, layer 59 -> 53, 256, 1024 x 512 36 -> 33.
 static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4 || g_opt.tile == 6) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const bool one = !grouped || E == 1;
@@ -1415,7 +1417,7 @@ static int choose_higher(const GemmParams& p, bool parts) {
   if (p.goff != nullptr)
     return p.E > 64 || p.Lrows >= (int64_t)7 * kLargeTile * p.E || p.Lrows < (int64_t)kLargeTile * 15 / 16 * p.E || p.nRt < 16 || p.nRt > 1024 ? -1 : 0;
   const uint32_t full = (uint32_t)std::min<int64_t>(p.Lrows / kLargeTile, 8), over = (uint32_t)(p.Lrows % kLargeTile), more = (over + 31) / 32;
-  return over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, parts, false) ? 1 : -1;
+  return over > 0 && more <= full && full < 8 && p.nRt <= 1024 && higher_tiles_pay(full, 1, 0, more, (uint32_t)p.nRt, full * (uint32_t)p.nRt, parts) ? 1 : -1;
 }
 // Tile-scaled R (per-row scales, the dense weight gradient): 256 x 128 tiles when there are enough of them.
 static bool use_large_tiles(int64_t tiles_256, const GemmOptions& g_opt) {
@@ -1795,15 +1797,19 @@ extern "C" int aamd_tuning_grouped_gemm_choice(int64_t M, int64_t N, int64_t K, 
   tile_order<kRaggedRows>(p, kLargeTile, GemmOptions());
   int higher = choose_higher(p, workspace != 0);
   if (higher == 0 && host_offsets != nullptr) {  // what higher_tiles of gemm_rows.hip counts
-    uint32_t full = 0, own0 = 0, own1 = 0, shared = 0;
+    uint32_t full = 0, own0 = 0, own1 = 0, shared = 0, longest = 0, of_xcd[8] = {};
     for (int e = 0; e < E; e++) {
       const uint32_t rows = (uint32_t)(host_offsets[e + 1] - host_offsets[e]), f = rows / kLargeTile, more = (rows % kLargeTile + 31) / 32;
       full += f;
       own0 += more > 0;
       own1 += more > f;
       shared += more > f ? 0 : more;
+      const uint32_t tiles = (more > f ? f + 1 : f) * (uint32_t)p.nRt;
+      for (int x = 0; x < 8; x++) of_xcd[x] += tiles / 8 + (uint32_t)((x + e) % 8 < (int)(tiles % 8));
     }
-    higher = own0 != own1 && higher_tiles_pay(full, own0, own1, shared, (uint32_t)p.nRt, workspace != 0 && row_max_split(K / kBK) > 1, takes_slices(p));
+    for (uint32_t n : of_xcd) longest = std::max(longest, n);
+    const uint32_t n1 = takes_slices(p) ? 8 * longest : (full + own1) * (uint32_t)p.nRt;
+    higher = own0 != own1 && higher_tiles_pay(full, own0, own1, shared, (uint32_t)p.nRt, n1, workspace != 0 && row_max_split(K / kBK) > 1);
   }
   return higher > 0 ? kLargeMore : kernel;
 }

@@ -90,26 +90,26 @@ int launch_few_rows_combine(GemmParams p, int what, const void* rows, int64_t ld
 
 // Are tiles of more rows worth it?  They save the tiles of remainders, which fetch their weights once more whatever few rows they have
 // (us, 28672 outputs x 4096, 8 groups of 512 rows 430, 513 to 576 548 to 560, 640 595, 768 640), and cost every step something, more
-// where addresses are made in the step.  In 256ths of a tile: 270 for one of theirs and 60 for 32 rows more in it, 171 and 181 for a
+// where addresses are made in the step.  In 256ths of a tile: 270 for one of theirs and 60 for 32 rows more in it, 176 and 185 for a
 // remainder's own.  With few rounds a launch is as long as the workgroup whose tiles are all full, or all higher; and a round counts
-// whole, but for a last one of few tiles, which is shared out (the slices of an XCD may be a tile longer than the mean, where that
-// begins another round).  Counts are of an R tile, all in whole numbers: the kernels of a launch have to come to the same.
-// Fitted to 1091 launches with remainders, of 1 to 64 groups of 240 to 1790 rows on average, 4096 to 32768 outputs and a contraction of 1024
-// to 14336.  Of 1400 others it takes these for 303, 0.892 of the time, 7 of them 1 % slower or more, the worst 1.06 (the lines that this
-// replaces, without rounds past the third: 68 of 513, the worst 1.21); of 400 without groups for 31, 0.845, the slowest 0.98.  Plain tiles ->
-// these: 28672 x 4096 in 8 groups of about 512 524 -> 474, of 264 373 -> 302, of 520 558 -> 489.  No longer taken: 2339 rows in 8, 16128 x
-// 11392 555 -> 625; 2546 in 2, 9344 x 7680 185 -> 225; 6599 in 8, 4096 x 7424 200 -> 237.  Taken, and should not be: 1285 and 1286 rows,
-// 25856 x 3456 227 -> 251.
+// whole, but for a last one of few tiles, which is shared out.  Counts are of an R tile; n1: the tiles that the XCDs would have if all had
+// as many as the one with the most.  All in whole numbers: the kernels of a launch have to come to the same.
+// Fitted to 3000 launches of 1 to 64 groups of 240 to 1790 rows on average, 4096 to 32768 outputs and a contraction of 1024 to 14336.  Of 1800
+// others it takes these for 446, 0.894 of the time, 19 of them 1 % slower or more, the worst 1.09 (4210 rows in 4, 10240 x 1024 65 -> 71);
+// the lines that this replaces, without rounds past the third, for 506, 0.909, 59 and 1.18.  Of 300 without groups for 27, 0.863, the slowest
+// 0.99.  Plain tiles -> these: 28672 x 4096 in 8 groups of about 512 523 -> 502, of 264 373 -> 302, of 520 558 -> 489; 4096 x 14336 in 8 of
+// about 512 273 -> 251.  No longer taken: 2339 rows in 8, 16128 x 11392 555 -> 625; 2546 in 2, 9344 x 7680 185 -> 225; 6599 in 8, 4096 x
+// 7424 200 -> 237.
 __host__ __device__ inline uint32_t higher_tile_rounds(uint32_t n, uint32_t shared_out, bool parts) {  // in tiles
   const uint32_t left = n & 255u;
   return n - left + (left == 0 ? 0 : left > shared_out ? 256 : parts ? 92 + (164 * left >> 8) : 143 + (113 * left >> 8));
 }
-__host__ __device__ inline bool higher_tiles_pay(uint32_t full, uint32_t own0, uint32_t own1, uint32_t shared, uint32_t nRt, bool parts, bool slices) {
-  const uint32_t t0 = full + own0, t1 = full + own1, n0 = t0 * nRt, n1 = t1 * nRt;
-  const uint32_t w0 = 256 * full + 171 * own0, w1 = 270 * full + 181 * own1 + 60 * shared;  // of an R tile, if all workgroups had the same
+__host__ __device__ inline bool higher_tiles_pay(uint32_t full, uint32_t own0, uint32_t own1, uint32_t shared, uint32_t nRt, uint32_t n1, bool parts) {
+  const uint32_t t0 = full + own0, t1 = full + own1, n0 = t0 * nRt;
+  const uint32_t w0 = 256 * full + 176 * own0, w1 = 270 * full + 185 * own1 + 60 * shared;  // of an R tile, if all workgroups had the same
   const uint32_t d0 = 256 * t0 - w0, d1 = (shared > 0 ? 330 : 270) * t1 - w1;               // and what the longest has beyond
   const uint32_t l0 = w0 + (n0 <= 210 ? d0 : 210 * d0 / n0), l1 = w1 + (n1 <= 210 ? d1 : 210 * d1 / n1);
-  const uint32_t r0 = higher_tile_rounds(n0, 128, parts), r1 = higher_tile_rounds(n1 + (slices ? 8 : 0), parts ? 112 : 128, parts);
+  const uint32_t r0 = higher_tile_rounds(n0, 128, parts), r1 = higher_tile_rounds(n1, parts ? 112 : 128, parts);
   return 32 * (uint64_t)r1 * l1 * t0 < 31 * (uint64_t)r0 * l0 * t1;
 }
 

@@ -34,7 +34,7 @@
 // tiles of the group: a ninth load instruction of a wave and step, one sub-tile more for each of the eight waves (the 32 rows by 256
 // columns of all of them).  The registers for it come from addresses, which are made in the step, and from what a tile is, which lies in
 // the LDS; that costs 4 to 10 % of a step, so the kernel that holds both forms takes it where the rows of the groups save more (see
-// higher_tiles_pay).  8 groups of 485 to 542 rows, 28672 x 4096, 585 -> 500; 4096 x 14336, 250 on both.
+// higher_tiles_pay, and for what it gives).
 #include <algorithm>
 
 #include "gemm_tiles.hpp"
@@ -110,7 +110,18 @@ __device__ __forceinline__ bool higher_tiles(ARGS p, const GroupRows& of_lane) {
   const uint32_t own0 = (uint32_t)__popcll(__ballot(over > 0)), own1 = (uint32_t)__popcll(__ballot(more > f));
   if (own0 == own1) return false;
   const uint32_t sums = (uint32_t)__builtin_amdgcn_readlane(wave_inclusive_sum((int)(f << 16 | (more > f ? 0u : more))), 63);
-  return higher_tiles_pay(sums >> 16, own0, own1, sums & 0xffffu, (uint32_t)p->nRt, p->max_split > 1, p->slices != 0);
+  const uint32_t full = sums >> 16, tiles = (more > f ? f + 1 : f) * (uint32_t)p->nRt;
+  uint32_t n1 = (full + own1) * (uint32_t)p->nRt;
+  if (p->slices && p->nRt % 8 != 0) {  // the longest of the XCDs' slices
+    uint32_t most = 0;
+#pragma unroll 1
+    for (uint32_t xcd = 0; xcd < 8; xcd++) {
+      const uint32_t n = (uint32_t)__popcll(__ballot(((xcd + threadIdx.x) & 7u) < (tiles & 7u)));
+      most = n > most ? n : most;
+    }
+    n1 = 8 * ((uint32_t)__builtin_amdgcn_readlane(wave_inclusive_sum((int)(tiles >> 3)), 63) + most);
+  }
+  return higher_tiles_pay(full, own0, own1, sums & 0xffffu, (uint32_t)p->nRt, n1, p->max_split > 1);
 }
 // With MORE every XCD may take an eighth of every group's tiles, R tile by R tile with all L tiles of it: tiles of more rows are then
 // spread over all of them (with one range of tiles for each XCD the one whose groups had the most of them took longest: 8 groups,

@@ -31,6 +31,9 @@ def test_blocks_that_are_known_and_fill_a_round(grouped, steps):
 # (us, tiles of 256 rows and of up to 288)
 @pytest.mark.parametrize("splits,N,K,workspace,higher", [
     ([485, 505, 513, 520, 500, 516, 515, 542], 28672, 4096, 0, True),  # 524, 474
+    ([496, 493, 518, 511, 526, 505, 521, 526], 28672, 4096, 0, True), ([519, 512, 516, 485, 521, 506, 489, 548], 28672, 4096, 0, True),  # 510, 500; 523, 507
+    ([496, 493, 518, 511, 526, 505, 521, 526], 4096, 14336, 1, True),  # 266, 253
+    ([802], 21120, 2560, 0, True),  # 66, 52: 249 tiles, of which no XCD has more than 32
     ([264] * 8, 28672, 4096, 0, True), ([520] * 8, 28672, 4096, 0, True), ([280, 277, 265], 15488, 3584, 0, True),  # 373, 302; 558, 489; 82, 62
     ([285, 300, 276, 310, 292, 281, 302, 293], 16128, 11392, 1, False),  # 555, 625
     ([1250, 1296], 9344, 7680, 1, False),  # 185, 225
