@@ -25,7 +25,7 @@ SIGNATURES = {
         _int,
         [_vp, _vp, _vp, _vp, _i64, _int, _vp, _int, _vp, _i64, _i64, _vp, _int, _i64, _int, _opts, _vp],
     ),
-    "aamd_tuning_grouped_gemm_choice": (_int, [_i64, _i64, _i64, _int, _int, _int, _int, _vp]),
+    "aamd_tuning_grouped_gemm_choice": (_int, [_i64, _i64, _i64, _int, _int, _int, _int, _int, _vp]),
     "aamd_clock_probe": (_int, [_vp, _i64, _vp]),
     "aamd_stream_probe": (_int, [_vp, _vp, _int, _int, _i64, _i64, _vp]),
     "aamd_mfma_probe": (_int, [_vp, _int, _int, _int, _vp, _vp, _vp]),

@@ -1348,10 +1348,14 @@ static int few_rows_waves(NtKernel k) { return k == kFewRowsSplit ? 8 : k == kFe
 // 14 with weights beyond the last-level cache, the weights' stream bounds such launches (64 groups of 6 rows, 7168 x 2048: 164 with four,
 // 168 with one).  Of 14351 others, even and Zipf, 4000 take these forms, 0.819 of the time, 83 of them 3 % slower or more (2414 rows in 61,
 // 512 x 896 7.0 -> 8.3; 1742 in 23, 2560 x 1024 19.7 -> 23.3); with two thirds of the groups empty, which the host does not know, 0.853 and a
-// fifth of them (86 rows in 7 of 32, 2560 x 2048 9.4 -> 13.7).  A wave's chain of sums is as much longer, one wave's the tiles' own; against
+// fifth of them (86 rows in 7 of 32, 2560 x 2048 9.4 -> 13.7).  One wave not where the rows
+// of a group, which every 64 outputs read again, fill much of an XCD's L2, nor where the output and the weights pass the last-level cache, unless
+// most of that are weights: 128 x 128 tiles and one wave, us, 30000 rows, 4096 x 256 88 and 117; 8195 rows in 2, 21760 x 256 137 and 163; 9600
+// in 32, fp32 8192 x 256 78 and 118.  Of 2500 launches of 1 to 8 steps and 700 blocks or more these lines take it for 848, 0.815 of the time, 32
+// of them 3 % slower or more; without them for 1162, 0.910 and 314.  A wave's chain of sums is as much longer, one wave's the tiles' own; against
 // 64-bit sums all are off by the same, 1.42e-5 in fp32 (19 steps).  The forms that quantise their rows take the same, and give the same bits:
 // eight tokens to 8 of 128 experts, 2048 x 768, layer 59 -> 53, 256, 1024 x 512 36 -> 33.
-static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, const GemmOptions& g_opt) {
+static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool grouped, bool b_rows, bool share_last, int c_dtype, const GemmOptions& g_opt) {
   if (g_opt.tile >= 0) return (g_opt.tile == 1 || g_opt.tile == 4 || g_opt.tile == 6) && nkb < 8 ? kSmallTiles : (NtKernel)g_opt.tile;
   const bool one = !grouped || E == 1;
   const double n = (double)nkb, rows = (double)M;
@@ -1392,8 +1396,10 @@ static NtKernel choose_nt(int64_t M, int64_t N, int64_t nkb, int64_t E, bool gro
 
   const double blocks_f = token_tiles(64) * (double)(N / 64), blocks_s = token_tiles(32) * (double)(N / 32);
   const bool fewer_waves = !b_rows && nkb < (weights <= 256.0 ? 20 : 14);
-  const bool one_wave = fewer_waves && blocks_f >= (nkb < 4 ? 724.0 : one ? 1025.0 : 1024.0);
-  const bool two_waves = fewer_waves && !one_wave && blocks_f >= (one ? 513.0 : 500.0);
+  const bool many = blocks_f >= (nkb < 4 ? 724.0 : one ? 1025.0 : 1024.0);
+  const double written = rows * (double)N * (c_dtype == AAMD_BF16 ? 2e-6 : 4e-6), read_again = rows / groups * n * (double)kBK * 1e-6;
+  const bool one_wave = fewer_waves && many && read_again <= 1.5 && (0.8 * weights + written <= 240.0 || 3.0 * written <= 2.0 * weights);
+  const bool two_waves = fewer_waves && !many && blocks_f >= (one ? 513.0 : 500.0);
   const double few = one_wave    ? std::max({5.8 + 1e-3 * blocks_f * (1.135 * n + 0.26), 4.4 + 0.64 * n, weights / 6.8})
                      : two_waves ? std::max({5.3 + 1e-3 * blocks_f * (1.135 * n + 1.1), 4.5 + 0.65 * std::ceil(n / 2.0), weights / 6.8})
                                  : std::max({4.5 + 1e-3 * blocks_f * (1.1 * n + 2.7) * (b_rows ? 1.015 : 1.0), 3.2 + 1.12 * std::ceil(n / 4.0), weights / 6.8});
@@ -1497,7 +1503,7 @@ static int gemm_nt_impl(const uint8_t* a, int64_t lda, const float* a_s, const u
   const bool batches = (K / kBK) >= 8 && g_opt.ls_batch != 0;
   const bool batches16 = batches && (K / kBK) % 4 == 0 && aligned16(a_s);
   const NtKernel kernel = b_tile_scaled ? (use_large_tiles(((M + 255) / 256 + (group_offsets ? E : 0)) * ((N + 255) / 256), g_opt) ? kLargeTiles : kSmallTiles)
-                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, ws != nullptr, g_opt);
+                                        : choose_nt(M, N, K / kBK, E, group_offsets != nullptr, b_rows, ws != nullptr, c_dtype, g_opt);
   // (output rows of 8 M elements are out of reach of the large tiles' 32-bit offsets)
   const bool once = kernel == kLargeOnce && !b_tile_scaled;
   const bool large = once || ((kernel == kLargeTiles || kernel == kLargeShared || kernel == kLargeMore) && (b_tile_scaled || ldc < (1LL << 23)));
@@ -1572,7 +1578,7 @@ extern "C" int aamd_grouped_gemm_fp8_nn(const uint8_t* a, int64_t lda, const flo
 constexpr int64_t kQuantisingRows = 64;
 static NtKernel quantising_kernel(int64_t M, int64_t N, int64_t K, int E) {
   if (M < 1 || M > kQuantisingRows || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || K >= (1LL << 23)) return kSmallTiles;
-  return choose_nt(M, N, K / kBK, E, true, false, false, GemmOptions());
+  return choose_nt(M, N, K / kBK, E, true, false, false, AAMD_BF16, GemmOptions());
 }
 // Workgroups of `rows` weight rows over the places of 512, where every row may have its own group.
 static double few_rows_rounds(int64_t M, int64_t N, int E, int rows) {
@@ -1698,7 +1704,7 @@ extern "C" int64_t aamd_grouped_gemm_fp8_ws_bytes(int64_t M, int64_t N, int64_t 
   // (the tiles of groups are counted on the device)
   const int64_t tiles = (M + kLargeTile - 1) / kLargeTile * ((N + kLargeTile - 1) / kLargeTile), left = (tiles + 7) / 8 % 32;
   if (!grouped && (left == 0 || left > 16)) return 0;
-  return choose_nt(M, N, nkb, E, grouped != 0, b_rows != 0, true, GemmOptions()) == kLargeShared ? kRowPartsBytes : 0;
+  return choose_nt(M, N, nkb, E, grouped != 0, b_rows != 0, true, AAMD_BF16, GemmOptions()) == kLargeShared ? kRowPartsBytes : 0;
 }
 extern "C" int aamd_grouped_gemm_fp8_ws(const uint8_t* a, int64_t lda, const float* a_s, const uint8_t* b, const float* b_s,
                                         int b_rows, const int64_t* group_offsets, int E, int64_t M, int64_t N, int64_t K, void* c,
@@ -1786,9 +1792,9 @@ extern "C" int aamd_tuning_grouped_gemm_fp8_nt(const uint8_t* a, int64_t lda, co
                       stream, o);
 }
 extern "C" int aamd_tuning_grouped_gemm_choice(int64_t M, int64_t N, int64_t K, int E, int grouped, int b_rows, int workspace,
-                                               const int64_t* host_offsets) {
+                                               int c_dtype, const int64_t* host_offsets) {
   if (M < 1 || N < kTile || K < kBK || N % kTile != 0 || K % kBK != 0 || E < 1 || (E > 1 && !grouped)) return -1;
-  const NtKernel kernel = choose_nt(M, N, K / kBK, E, grouped != 0, b_rows != 0, workspace != 0, GemmOptions());
+  const NtKernel kernel = choose_nt(M, N, K / kBK, E, grouped != 0, b_rows != 0, workspace != 0, c_dtype, GemmOptions());
   if (kernel != kLargeTiles && kernel != kLargeShared) return kernel;
   GemmParams p = {};
   const int64_t none = 0;

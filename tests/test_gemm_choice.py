@@ -7,11 +7,11 @@ import pytest
 FOUR, TWO, ONE, SMALL_TILES, LARGE_TILES, SHARED, HIGHER = 2, 7, 8, 0, 1, 5, 6
 
 
-def choice(M, N, steps, E=1, grouped=0, b_rows=0, workspace=0, splits=None):
+def choice(M, N, steps, E=1, grouped=0, b_rows=0, workspace=0, splits=None, c_dtype=0):
     from atorch_amd import _probes
 
     offsets = (ctypes.c_int64 * (E + 1))(0, *accumulate(splits)) if splits else None
-    return _probes.lib().aamd_tuning_grouped_gemm_choice(M, N, 128 * steps, E, grouped, b_rows, workspace, offsets)
+    return _probes.lib().aamd_tuning_grouped_gemm_choice(M, N, 128 * steps, E, grouped, b_rows, workspace, c_dtype, offsets)
 
 
 @pytest.mark.parametrize("grouped", [0, 1])
@@ -26,6 +26,18 @@ def test_blocks_that_are_known_and_fill_a_round(grouped, steps):
     if steps >= 4:
         assert choice(64, 65536, steps, grouped=grouped) in (TWO, SMALL_TILES)
         assert choice(64, 65664, steps, grouped=grouped) in (ONE, SMALL_TILES)
+
+
+# (us, 128 x 128 tiles and one wave to a block)
+@pytest.mark.parametrize("M,N,steps,E,c_dtype,one_wave", [
+    (8195, 21760, 2, 2, 0, False), (8192, 14336, 2, 16, 0, False), (94295, 2048, 2, 55, 0, False), (8907, 13312, 2, 44, 0, False),  # 137, 163; 94, 117; 163, 194; 116, 131
+    (9600, 8192, 2, 32, 1, False), (24000, 5120, 1, 4, 1, False),  # 78, 118; 101, 104: outputs of 315 and 492 MB
+    (9600, 8192, 2, 32, 0, True), (8192, 4096, 2, 8, 1, True), (3072, 27776, 2, 1, 0, True), (410, 25728, 4, 56, 0, True),  # 76, 59; 34, 31; 73, 62; 193, 142
+    (30000, 4096, 2, 1, 0, False), (11718, 1024, 2, 1, 0, False), (40000, 1024, 2, 4, 0, False), (20000, 4096, 2, 4, 0, True),  # 85, 112, rows of 7.7 MB in a group; of 3 and 2.6 MB; of 1.3
+])  # fmt: skip
+def test_one_wave_where_the_caches_hold_what_it_needs(M, N, steps, E, c_dtype, one_wave):
+    got = choice(M, N, steps, E, 1, c_dtype=c_dtype)
+    assert got == (ONE if one_wave else SMALL_TILES)
 
 
 # (us, tiles of 256 rows and of up to 288)
