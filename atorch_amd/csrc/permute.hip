@@ -528,7 +528,7 @@ __global__ __launch_bounds__(256) void route_place_kernel(const ID* __restrict__
 
 // ---------------------------------------------------------------------------------------
 // The same sort for fewer ids, with fewer launches (each of the four above is latency: 2 to 5 us whatever n is).
-// Up to 3200 ids and three per expert, or 8192 without scratch: one workgroup does it all, ids and ranks in registers, counts of every (64 ids, expert) in LDS.
+// Up to aamd_route_takes_scratch's line, 3300 to 4600 ids, or 8192 without scratch: one workgroup does it all, ids and ranks in registers, counts of every (64 ids, expert) in LDS.
 // ---------------------------------------------------------------------------------------
 // exclusive prefix of tot[0 .. E) into base[0 .. E), by one wave; returns the sum of all
 __device__ __forceinline__ int wave_exclusive_prefix(const int* tot, int* base, int E) {
