@@ -16,8 +16,8 @@ import sys
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ["capi.hip", "quant.hip", "permute.hip", "gemm.hip", "gemm_rows.hip", "gemm_wgrad.hip", "gemm_few.hip"]
-PROBE_SOURCES = ["capi.hip", "gemm.hip", "gemm_rows.hip", "gemm_wgrad.hip", "gemm_few.hip", "probe.hip"]  # compiled with -DAAMD_TUNING
+SOURCES = ["capi.hip", "quant.hip", "permute.hip", "gemm.hip", "gemm_rows.hip", "gemm_rows_higher.hip", "gemm_wgrad.hip", "gemm_few.hip"]
+PROBE_SOURCES = ["capi.hip", "gemm.hip", "gemm_rows.hip", "gemm_rows_higher.hip", "gemm_wgrad.hip", "gemm_few.hip", "probe.hip"]  # compiled with -DAAMD_TUNING
 LIB = os.path.join(HERE, "libatorch_amd_fp8.so")
 HOST = os.path.join(os.path.dirname(HERE), "_host.so")
 PROBES_LIB = os.path.join(HERE, "libatorch_amd_probes.so")
@@ -31,6 +31,7 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]  # fmt: skip
+SOURCE_FLAGS = {"gemm_rows_higher.hip": ["-falign-loops=64"]}  # (what it is for stands there)
 LINK = ["--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-Bsymbolic"]
 
 
@@ -55,7 +56,7 @@ def _build_host() -> None:
 def _compile(job) -> str:
     src, suffix, extra = job
     obj = os.path.join(HERE, src.replace(".hip", suffix + ".o"))
-    subprocess.check_call([HIPCC, *FLAGS, *extra, "-c", os.path.join(HERE, src), "-o", obj])
+    subprocess.check_call([HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), *extra, "-c", os.path.join(HERE, src), "-o", obj])
     return obj
 
 

@@ -1036,11 +1036,18 @@ static void launch_row_tiles_as(const GemmParams& p, unsigned blocks, hipStream_
     row_parts_kernel<OUT, EITHER><<<sums, 256, 0, st>>>(p);
   }
 }
-template <typename OUT>
-static void launch_row_tiles_of(const GemmParams& p, unsigned blocks, bool r_rows, hipStream_t st) {
-  if (p.higher >= 0) r_rows ? launch_row_tiles_as<OUT, true, true>(p, blocks, st) : launch_row_tiles_as<OUT, false, true>(p, blocks, st);
-  else r_rows ? launch_row_tiles_as<OUT, true, false>(p, blocks, st) : launch_row_tiles_as<OUT, false, false>(p, blocks, st);
+template <bool EITHER>
+static void launch_row_tiles_of(const GemmParams& p, int c_dtype, unsigned blocks, bool r_rows, hipStream_t st) {
+  if (c_dtype == AAMD_BF16) r_rows ? launch_row_tiles_as<u16, true, EITHER>(p, blocks, st) : launch_row_tiles_as<u16, false, EITHER>(p, blocks, st);
+  else r_rows ? launch_row_tiles_as<float, true, EITHER>(p, blocks, st) : launch_row_tiles_as<float, false, EITHER>(p, blocks, st);
 }
+// Both halves of the launches, one in each unit that is made of this file (gemm_rows_higher.hip).
+void launch_row_tiles_higher(const GemmParams& p, int c_dtype, unsigned blocks, bool r_rows, hipStream_t st);
+#ifdef AAMD_ROW_TILES_HIGHER
+void launch_row_tiles_higher(const GemmParams& p, int c_dtype, unsigned blocks, bool r_rows, hipStream_t st) {
+  launch_row_tiles_of<true>(p, c_dtype, blocks, r_rows, st);
+}
+#else
 int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipStream_t st) {
   AAMD_REQUIRE(tiles < 0x7fffffffLL, "grouped_gemm: grid too large");
   unsigned blocks = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, rows::kWorkgroups);
@@ -1049,9 +1056,11 @@ int launch_row_tiles(GemmParams p, int c_dtype, int64_t tiles, bool r_rows, hipS
   // 1024 160 -> 175; 32768 x 28672 (1.9 GB), 4096 3449 -> 3414; 4096 x 14336 (117 MB), 4096 222 both).
   p.stream_out = p.nkb >= 32 && p.Lrows * p.Rrows * (c_dtype == AAMD_BF16 ? 2 : 4) >= (int64_t)1 << 28;
   if (p.max_split > 1) blocks = rows::kWorkgroups;
-  c_dtype == AAMD_BF16 ? launch_row_tiles_of<u16>(p, blocks, r_rows, st) : launch_row_tiles_of<float>(p, blocks, r_rows, st);
+  if (p.higher >= 0) launch_row_tiles_higher(p, c_dtype, blocks, r_rows, st);
+  else launch_row_tiles_of<false>(p, c_dtype, blocks, r_rows, st);
   AAMD_LAUNCH_CHECK("grouped_gemm (256 x 256 tiles)");
   return AAMD_OK;
 }
+#endif
 
 }  // namespace aamd
